@@ -6,14 +6,20 @@
 //     epilogue  none:   y = bf16(s)                                                                     (kernels.py:153-160)
 //               add:    y = bf16(BF(s) + res)                                                           (kernels.py:161-169)
 //               swiglu: y[m][p] = bf16(silu_bf16(BF(s[m][2p])) * BF(s[m][2p+1]))   interleaved rows     (kernels.py:170-182)
-// The batch is small, so the product is bound by streaming W once from HBM.  General form: one workgroup owns 16 output
-// features and all rows (64 per pass); its wavefronts split K, each feeding 16x16x32 bf16 MFMAs straight from global memory (a
-// W fragment is 16 features x 32 k, an x fragment 16 rows x 32 k: both are 16-byte row-contiguous loads per lane), and the
-// partial sums meet in LDS.  The wide projections of a decode batch (K = 1024, 4 to 64 rows) keep the rows in LDS instead and
-// give every wavefront a feature block with all of its K (xlds_gemm_kernel): what bounds such a launch is the bytes one CU
-// has to pull in, its share of W plus ALL of x.  Arithmetic contract of rms_rows: sum of squares exact, rounded to float once; inv = correctly
-// rounded 1/sqrt(ss / K + eps); t = x * inv and w * t rounded to float separately, then to bf16.
+// The batch is small, so the product is bound by what ONE CU has to pull in (its share of W and of x) and by the launch itself.
+// Three kernels by shape:
+//   rows_gemm_kernel  the wide projections of a decode / verify batch (K = 1024, N >= 4096): the rows live in LDS, the rms
+//                     prologue is applied on the way there, a workgroup owns 32 or 64 output features
+//   quad_gemm_kernel  narrow outputs: small tiles (4 x 4 .. 16 x 16 outputs) so that every CU has one
+//   skinny_gemm_kernel  everything else: 16 features x up to 64 rows per workgroup
+// What decides the first two is how a load maps to lanes.  An MFMA operand wants 16 different rows in 16 neighbouring lanes; a
+// load shaped like that asks for 16 bytes of 16 different rows per quarter-wavefront, and the CU takes in 16 bytes per clock
+// (measured: 33 GB/s and less per CU).  Four neighbouring lanes that read 64 contiguous bytes get four times that.  The two
+// kernels load in that shape and put the lanes right afterwards, each in its own way.
+// Arithmetic contract of rms_rows: sum of squares exact, rounded to float once; inv = correctly rounded 1/sqrt(ss / K + eps);
+// t = x * inv and w * t rounded to float separately, then to bf16.
 #include "qt_common.h"
+#include <type_traits>
 
 using namespace qt;
 
@@ -146,220 +152,392 @@ __global__ __launch_bounds__(64 * NWV, 16 / NWV) void skinny_gemm_kernel(const b
     }
 }
 
-// Wide outputs (N in the thousands): the rows are the expensive operand, because every workgroup reads all of x from L2.  Here
-// a wavefront keeps its K range of x in registers (KCW chunks x four 16-row blocks) and walks NT feature blocks with it, so
-// x is fetched once per 16 NT features and only W streams.  grid = (ceil(N / 16 NT), ceil(M / 64)), K = 32 KCW NWV.
-template <int NWV, int KCW, int NT, int MS, int EPI>
-__global__ __launch_bounds__(64 * NWV) void wide_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
-                                                             const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N, int K) {
-    __shared__ float red[NWV][16][MT + 1];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MS);
-    const int k_base = w * KCW * 32 + 8 * g;
-    u32x4 a[NT][KCW], b[KCW][MS];
+// barrier for data that goes through LDS only: global loads stay in flight across it (__syncthreads() would drain them)
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// a + b over lane pairs (l, l + 32) / (l, l + 16): one v_permlane swap per dword serves two values at once, so that two rows'
+// sums are folded together and land in different lanes
+__device__ __forceinline__ double swap_add32(double a, double b) {
+    const auto l = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+    const auto l = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+constexpr int XK = 1024;
+// inv[r] = 1 / sqrt(sum / 1024 + eps) of NR = 2, 4 or 6 rows whose exact (double) sums of squares lie spread over the 64 lanes of
+// ss[r].  The first two folding steps halve the number of values (row r ends in 16-lane row (r & 1) * 2 + (r >> 1 & 1) of value
+// r / 4), so the reduction costs about a third of NR separate ones, and the double-precision root is taken once.
+template <int NR>
+__device__ __forceinline__ void rows_inv(const double (&ss)[NR], float eps, int lane, float (&inv)[NR]) {
+    constexpr int NT = NR / 2, NU = (NT + 1) / 2;
+    double t[NT], u[NU];
 #pragma unroll
-    for (int c = 0; c < KCW; c++)                                 // the first feature block's W rides ahead of x
-        a[0][c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(W + (size_t)min(n0 + n, N - 1) * K + k_base + c * 32));
+    for (int i = 0; i < NT; i++) t[i] = swap_add32(ss[2 * i], ss[2 * i + 1]);
 #pragma unroll
-    for (int ms = 0; ms < MS; ms++) {
-        const bf16_t* xp = x + (size_t)min(m0 + 16 * ms + n, M - 1) * K + k_base;
+    for (int i = 0; i < NU; i++) u[i] = row16_sum_d(swap_add16(t[2 * i], t[2 * i + 1 < NT ? 2 * i + 1 : 2 * i]));
+    const float mine = NU > 1 && (lane & 1) ? (float)u[NU - 1] : (float)u[0];
+    const float rv = rsqrt_rn(mine / (float)XK + eps);
 #pragma unroll
-        for (int c = 0; c < KCW; c++) b[c][ms] = *reinterpret_cast<const u32x4*>(xp + c * 32);
-    }
+    for (int r = 0; r < NR; r++)
+        inv[r] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(rv), (r & 1) * 32 + (r & 2) * 8 + r / 4));
+}
+
+// 4 x 4 transpose of 16-byte items between four registers and the four lanes of a quad: 48 vector instructions
+__device__ __forceinline__ void quad_transpose(u32x4& a, u32x4& b, u32x4& c, u32x4& d, bool odd, bool high) {
+    auto swz = [](unsigned v, auto ctrl) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl.value, 0xF, 0xF, true); };
+    constexpr std::integral_constant<int, 0xB1> by1{};            // quad_perm [1,0,3,2]
+    constexpr std::integral_constant<int, 0x4E> by2{};            // quad_perm [2,3,0,1]
 #pragma unroll
-    for (int nt = 1; nt < NT; nt++)
-#pragma unroll
-        for (int c = 0; c < KCW; c++)
-            a[nt][c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(W + (size_t)min(n0 + 16 * nt + n, N - 1) * K + k_base + c * 32));
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        f32x4 acc[MS];
-#pragma unroll
-        for (int ms = 0; ms < MS; ms++) acc[ms] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < KCW; c++)
-#pragma unroll
-            for (int ms = 0; ms < MS; ms++)
-                acc[ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[nt][c]),
-                                                                 __builtin_bit_cast(bf16x8, b[c][ms]), acc[ms], 0, 0, 0);
-        if (nt) __syncthreads();                                  // the previous block's sums have been read
-#pragma unroll
-        for (int ms = 0; ms < MS; ms++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) red[w][4 * g + i][16 * ms + n] = acc[ms][i];
-        __syncthreads();
-        auto total = [&](int f, int m) {                          // fixed order: pairs, then pairs of pairs, ...
-            float t[NWV];
-#pragma unroll
-            for (int i = 0; i < NWV; i++) t[i] = red[i][f][m];
-#pragma unroll
-            for (int st = 1; st < NWV; st *= 2)
-#pragma unroll
-                for (int i = 0; i < NWV; i += 2 * st) t[i] += t[i + st];
-            return t[0];
-        };
-        const int nb = n0 + 16 * nt;
-        if (EPI == EPI_SWIGLU) {
-            for (int idx = threadIdx.x; idx < 8 * 16 * MS; idx += 64 * NWV) {
-                const int p = idx % 8, m = idx / 8;
-                if (m0 + m < M && nb + 2 * p + 1 < N) {
-                    const float gt = BF(total(2 * p, m)), up = BF(total(2 * p + 1, m));
-                    y[(size_t)(m0 + m) * (N / 2) + nb / 2 + p] = f2bf(silu_bf16(gt) * up);
-                }
-            }
-        } else {
-            for (int idx = threadIdx.x; idx < 16 * 16 * MS; idx += 64 * NWV) {
-                const int f = idx % 16, m = idx / 16;
-                if (m0 + m < M && nb + f < N) {
-                    const size_t o = (size_t)(m0 + m) * N + nb + f;
-                    const float s = total(f, m);
-                    y[o] = EPI == EPI_ADD ? f2bf(BF(s) + bf2f(res[o])) : f2bf(s);
-                }
-            }
-        }
+    for (int i = 0; i < 4; i++) {
+        unsigned x0 = a[i], x1 = b[i], x2 = c[i], x3 = d[i];
+        unsigned t = swz(odd ? x0 : x1, by1), u = swz(odd ? x2 : x3, by1);
+        x0 = odd ? t : x0, x1 = odd ? x1 : t, x2 = odd ? u : x2, x3 = odd ? x3 : u;
+        t = swz(high ? x0 : x2, by2), u = swz(high ? x1 : x3, by2);
+        a[i] = high ? t : x0, c[i] = high ? x2 : t, b[i] = high ? u : x1, d[i] = high ? x3 : u;
     }
 }
 
-// K = 1024, wide outputs: the rows live in LDS, shared by the whole workgroup, and a wavefront owns a feature block with all
-// of its K, so nothing is summed across wavefronts.  x [16 MS rows][1024] goes HBM / L2 -> LDS directly (global_load_lds: one
-// instruction lands half a row, 1 KiB, contiguously), its 16-byte chunks XOR-swizzled by the row number (the loading lane
-// fetches the chunk that belongs at its position) so that the fragment reads of 16 rows fall on distinct banks.  The
-// wavefront's W block [16 features][1024] is 32 loads, all issued up front (128 registers); every W fragment then meets MS
-// x fragments read from LDS.  Accumulator element i of lane (n, g) is feature 4 g + i of row 16 ms + n: four adjacent
-// features, stored as 8 bytes.  grid = ceil(N / (16 WPB)), block = 64 WPB.
-// With `full` > 0 the launch is one workgroup for every CU whatever N: wavefronts 0 .. WPB - 2 of workgroup i take feature
-// blocks (WPB - 1) i + w, and the last wavefront takes block `full` + i, which exists in the first few workgroups only (the
-// 514 blocks of N = 8224 are 2 x 256 + 2: with three blocks per workgroup 84 of 256 CUs would have none, and what bounds the
-// launch is the bytes one CU has to pull in).  A wavefront without a block still helps to bring in the rows.
-constexpr int XK = 1024;
-template <int MS, int WPB, int EPI>
-__global__ __launch_bounds__(64 * WPB) void xlds_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
-                                                        const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N, int full) {
-    __shared__ __align__(1024) bf16_t x_s[16 * MS * XK];
+// K = 1024, wide outputs.  A workgroup of eight wavefronts owns NB = 2 FB blocks of 16 features and 16 RB rows; wavefront (half,
+// q) multiplies FB of the blocks over the quarter q of K (two of the eight 128-wide steps of a row), and the quarters meet in
+// LDS in a fixed order.
+// Rows: every wavefront brings in 2 RB of them, a row per two loads of 1 KiB, asks for its W right after, and applies the rms
+// prologue (RMS) while W is on its way from HBM; the rows then go to LDS, their 16-byte chunks XOR-swizzled by the row number
+// so that the fragment reads of 16 rows fall on distinct banks.  Every workgroup normalises its rows itself: 0.1 us (16 rows)
+// to 1.2 us (32 rows x 64 features) instead of a launch of its own at 2.6 us.
+// W: a load takes 256 contiguous bytes of four features, 64 of them in each quad of lanes (register j of lane (g, h, c): feature
+// 4 h + j, elements 32 g + 8 c ..), and quad_transpose turns four such loads into the MFMA layout: feature n in lane (n, g),
+// elements 32 g + 8 r .. in register r.  The x fragments are read from LDS in the same enumeration of k.  Workgroups start at
+// different steps of the row (rot), so that they do not all ask the same memory channels first.
+// Two of the launch's shapes do not divide: with `extra` > 0 the first `extra` tiles take one block more, from the end of
+// N (the 514 blocks of N = 8224 are 256 x 2 + 2; a 257th workgroup would take a CU twice as long as the others).
+// Tile sizes (us in a HIP graph, rms prologue included, N = 8224 / 7168 swiglu / 5120; before: rms_rows and the product as two
+// launches, x fragments and W loaded in MFMA shape): 1 row 6.2 / 5.7 / 4.9 (8.5 / 7.9 / 6.9), 16 rows 6.3 / 5.7 / 4.9 (9.1 / 8.5 /
+// 7.9), 32 rows 7.5 / 7.1 / 6.2 (9.9 / 9.8 / 9.0), 64 rows 8.9 / 8.6 / 7.8 (11.9 / 13.0 / 11.3), 80 rows 10.1 / 9.8 / 9.1 (20.2 /
+// 19.5 / 14.2).  An empty kernel takes 1.9 us there; what is left at 64 rows is the 64 KiB of rows and 128 KiB of W a CU pulls.
+template <int RB, int FB, bool RMS, int EPI>
+__global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
+                                                                         const bf16_t* __restrict__ nw, float eps,
+                                                                         const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N,
+                                                                         int groups, int tiles, int extra) {
+    constexpr int NB = 2 * FB, R = 16 * RB, RW = R / 8;
+    __shared__ __align__(1024) bf16_t x_s[R * XK];                // later: the partial sums [NB + 1][4 quarters][R][16 features]
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-    // this wavefront's feature block (may lie past N: then it multiplies a copy of the last row block and stores nothing)
-    const int n0 = 16 * (full <= 0 ? blockIdx.x * WPB + w : w < WPB - 1 ? blockIdx.x * (WPB - 1) + w : full + blockIdx.x);
-    // W first (it comes from HBM): the wavefront's block is 32 loads, all in flight at once
-    u32x4 a[XK / 32];
-    const bool has_block = n0 < N;                                // (the same for the whole wavefront)
-    if (has_block) {
-        const bf16_t* wp = W + (size_t)min(n0 + n, N - 1) * XK + 8 * g;
+    // the row groups of a tile sit on one XCD (workgroups are dealt to the eight XCDs in turn) and share its W through the L2
+    const int s = blockIdx.x >> 3, grp = s % groups, tile = (s / groups) * 8 + (blockIdx.x & 7);
+    if (tile >= tiles) return;
+    const int q = w & 3, half = w >> 2, m0 = grp * R, nb0 = tile * 16 * NB, nx = 16 * (tiles * NB + tile), rot = s & 7;
+    const bool has_x = tile < extra && half == 0;
+    u32x4 xr[RW][2], wn[2];
 #pragma unroll
-        for (int c = 0; c < XK / 32; c++) a[c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp + 32 * c));
+    for (int i = 0; i < RW; i++) {
+        const bf16_t* src = x + (size_t)min(m0 + w + 8 * i, M - 1) * XK + 8 * lane;      // (rows past M repeat the last one)
+        xr[i][0] = *reinterpret_cast<const u32x4*>(src);
+        xr[i][1] = *reinterpret_cast<const u32x4*>(src + 512);
     }
-    // x -> LDS: half-row h (of 2 * 16 MS) by wavefront h % WPB; lane l lands at chunk position 64 (h & 1) + l of row h >> 1
-    // (every workgroup reads the same rows at the same time; starting each at another half-row changed nothing)
-    for (int h = w; h < 32 * MS; h += WPB) {
-        const int r = h >> 1, cp = 64 * (h & 1) + lane;
-        const bf16_t* src = x + (size_t)min(r, M - 1) * XK + 8 * (cp ^ (r & 15));
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                         (__attribute__((address_space(3))) void*)(x_s + h * 512), 16, 0, 0);
+    if (RMS) {
+        wn[0] = *reinterpret_cast<const u32x4*>(nw + 8 * lane);
+        wn[1] = *reinterpret_cast<const u32x4*>(nw + 512 + 8 * lane);
     }
-    // (a direct-to-LDS load in flight makes the compiler wait for every outstanding load before the first use of any, so the
-    // products cannot start under the tail of the W stream; both streams are drained here)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (!has_block) return;                                       // it has done its share of the rows
-    f32x4 acc[MS];
+    u32x4 a[FB + 1][8];
+    auto w_load = [&](u32x4 (&d)[8], int f0) {
 #pragma unroll
-    for (int ms = 0; ms < MS; ms++) acc[ms] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // x fragments are read two chunks ahead of their MFMAs (a ring of three), the scheduler pinned
-    auto x_frag = [&](int c, int ms) {
-        return *reinterpret_cast<const u32x4*>(x_s + (16 * ms + n) * XK + 8 * ((4 * c + g) ^ n));
+        for (int i = 0; i < 8; i++)
+            d[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+                W + (size_t)min(f0 + (n & 12) + (i & 3), N - 1) * XK + 128 * ((q + (i & 4) + rot) & 7) + 32 * g + 8 * (n & 3)));
     };
-    u32x4 b[3][MS];
 #pragma unroll
-    for (int ms = 0; ms < MS; ms++) b[0][ms] = x_frag(0, ms), b[1][ms] = x_frag(1, ms);
+    for (int f = 0; f < FB; f++) w_load(a[f], nb0 + 16 * (half * FB + f));
+    if (has_x) w_load(a[FB], nx);
+    __builtin_amdgcn_sched_barrier(0);                            // everything is in flight before the first row is looked at
+    if (RMS) {
+        double ss[RW];
 #pragma unroll
-    for (int c = 0; c < XK / 32; c++) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (c + 2 < XK / 32) {
+        for (int i = 0; i < RW; i++) {
+            ss[i] = 0.0;
 #pragma unroll
-            for (int ms = 0; ms < MS; ms++) b[(c + 2) % 3][ms] = x_frag(c + 2, ms);
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const double lo = (double)lo_bf(xr[i][c][j]), hi = (double)hi_bf(xr[i][c][j]);
+                    ss[i] = fma(hi, hi, fma(lo, lo, ss[i]));
+                }
         }
-        __builtin_amdgcn_sched_barrier(0);
+        float inv[RW];
+        rows_inv<RW>(ss, eps, lane, inv);
 #pragma unroll
-        for (int ms = 0; ms < MS; ms++)
-            acc[ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[c]), __builtin_bit_cast(bf16x8, b[c % 3][ms]),
-                                                             acc[ms], 0, 0, 0);
+        for (int i = 0; i < RW; i++)
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    xr[i][c][j] = pack_bf(lo_bf(wn[c][j]) * (lo_bf(xr[i][c][j]) * inv[i]), hi_bf(wn[c][j]) * (hi_bf(xr[i][c][j]) * inv[i]));
     }
-    __builtin_amdgcn_sched_barrier(0);
-    const int f0 = n0 + 4 * g;                                    // first of this lane's four features (N is a multiple of 4)
-    if (f0 >= N) return;                                          // (also a wavefront whose whole block lies past N)
 #pragma unroll
-    for (int ms = 0; ms < MS; ms++) {
-        const int m = 16 * ms + n;
-        if (m >= M) continue;
+    for (int i = 0; i < RW; i++) {
+        const int r = w + 8 * i;
+#pragma unroll
+        for (int c = 0; c < 2; c++) *reinterpret_cast<u32x4*>(x_s + r * XK + 8 * ((lane + 64 * c) ^ (r & 15))) = xr[i][c];
+    }
+    lds_barrier();
+    f32x4 acc[FB + 1][RB];
+#pragma unroll
+    for (int f = 0; f <= FB; f++)
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++) acc[f][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bool odd = n & 1, high = n & 2;
+    auto x_frag = [&](int i, int rb) {
+        return *reinterpret_cast<const u32x4*>(x_s + (16 * rb + n) * XK + 8 * ((16 * ((q + (i & 4) + rot) & 7) + 4 * g + (i & 3)) ^ n));
+    };
+    auto mma = [](const u32x4& av, const u32x4& bv, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv), c, 0, 0, 0);
+    };
+#pragma unroll
+    for (int f = 0; f < FB; f++)
+#pragma unroll
+        for (int t = 0; t < 8; t += 4) quad_transpose(a[f][t], a[f][t + 1], a[f][t + 2], a[f][t + 3], odd, high);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        u32x4 b[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++) b[rb] = x_frag(i, rb);
+#pragma unroll
+        for (int f = 0; f < FB; f++)
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) acc[f][rb] = mma(a[f][i], b[rb], acc[f][rb]);
+    }
+    if (has_x) {
+#pragma unroll
+        for (int t = 0; t < 8; t += 4) quad_transpose(a[FB][t], a[FB][t + 1], a[FB][t + 2], a[FB][t + 3], odd, high);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) acc[FB][rb] = mma(a[FB][i], x_frag(i, rb), acc[FB][rb]);
+    }
+    lds_barrier();                                                // the rows have been read: their memory takes the partial sums
+    // accumulator element i of lane (n, g) is feature 4 g + i of row 16 rb + n
+    float* red = reinterpret_cast<float*>(x_s);
+    auto put = [&](int blk, const f32x4 (&v)[RB]) {
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++) *reinterpret_cast<f32x4*>(red + ((blk * 4 + q) * R + 16 * rb + n) * 16 + 4 * g) = v[rb];
+    };
+#pragma unroll
+    for (int f = 0; f < FB; f++) put(half * FB + f, acc[f]);
+    if (has_x) put(NB, acc[FB]);
+    lds_barrier();
+    const int items = (NB + (tile < extra ? 1 : 0)) * R * 4;
+    for (int idx = threadIdx.x; idx < items; idx += 512) {        // four adjacent features of a row each (N is a multiple of 4)
+        const int blk = idx / (R * 4), r = (idx / 4) % R, f4 = idx & 3;
+        const int m = m0 + r, f0 = (blk < NB ? nb0 + 16 * blk : nx) + 4 * f4;
+        if (m >= M || f0 >= N) continue;
+        f32x4 t[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) t[k] = *reinterpret_cast<const f32x4*>(red + ((blk * 4 + k) * R + r) * 16 + 4 * f4);
+        f32x4 v = (t[0] + t[1]) + (t[2] + t[3]);
         if (EPI == EPI_SWIGLU) {
-            const float g0 = BF(acc[ms][0]), u0 = BF(acc[ms][1]), g1 = BF(acc[ms][2]), u1 = BF(acc[ms][3]);
-            *reinterpret_cast<uint32_t*>(y + (size_t)m * (N / 2) + f0 / 2) = pack_bf(silu_bf16(g0) * u0, silu_bf16(g1) * u1);
+            *reinterpret_cast<uint32_t*>(y + (size_t)m * (N / 2) + f0 / 2) = pack_bf(silu_bf16(BF(v[0])) * BF(v[1]), silu_bf16(BF(v[2])) * BF(v[3]));
         } else {
             const size_t o = (size_t)m * N + f0;
-            float v[4] = {acc[ms][0], acc[ms][1], acc[ms][2], acc[ms][3]};
             if (EPI == EPI_ADD) {
                 const uint2 rr = *reinterpret_cast<const uint2*>(res + o);
-                v[0] = BF(v[0]) + lo_bf(rr.x), v[1] = BF(v[1]) + hi_bf(rr.x), v[2] = BF(v[2]) + lo_bf(rr.y), v[3] = BF(v[3]) + hi_bf(rr.y);
+                v = f32x4{BF(v[0]) + lo_bf(rr.x), BF(v[1]) + hi_bf(rr.x), BF(v[2]) + lo_bf(rr.y), BF(v[3]) + hi_bf(rr.y)};
             }
             *reinterpret_cast<uint2*>(y + o) = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
         }
     }
 }
 
-template <int MS, int WPB>
-void launch_xlds_wpb(int epi, const bf16_t* W, const bf16_t* x, const bf16_t* res, bf16_t* y, int M, int N, hipStream_t stream, int grid_x,
-                     int full) {
-    const dim3 grid(grid_x), block(64 * WPB);
-    if (epi == EPI_NONE)
-        hipLaunchKernelGGL((xlds_gemm_kernel<MS, WPB, EPI_NONE>), grid, block, 0, stream, W, x, res, y, M, N, full);
-    else if (epi == EPI_ADD)
-        hipLaunchKernelGGL((xlds_gemm_kernel<MS, WPB, EPI_ADD>), grid, block, 0, stream, W, x, res, y, M, N, full);
-    else
-        hipLaunchKernelGGL((xlds_gemm_kernel<MS, WPB, EPI_SWIGLU>), grid, block, 0, stream, W, x, res, y, M, N, full);
-}
-template <int MS>
-void launch_xlds_ms(int epi, const bf16_t* W, const bf16_t* x, const bf16_t* res, bf16_t* y, int M, int N, hipStream_t stream, int cus) {
-    // as few wavefronts per workgroup as keep the launch within one workgroup per CU (the rows take most of a CU's LDS)
-    const int blocks = (N + 15) / 16, wpb = (blocks + cus - 1) / cus;
-    // a few blocks more than a whole number per CU: every CU gets that number, the first few workgroups one more
-    const int base = blocks / cus, rest = blocks - base * cus;
-    if (base >= 1 && base <= 3 && rest > 0 && rest <= cus / 16) {
-        const int full = base * cus;
-        if (base == 1)
-            launch_xlds_wpb<MS, 2>(epi, W, x, res, y, M, N, stream, cus, full);
-        else if (base == 2)
-            launch_xlds_wpb<MS, 3>(epi, W, x, res, y, M, N, stream, cus, full);
-        else
-            launch_xlds_wpb<MS, 4>(epi, W, x, res, y, M, N, stream, cus, full);
-        return;
+// Narrow outputs (N = 1024: out_proj, o_proj, down_proj): a workgroup owns 4 FG features x 4 MG rows, its NWV wavefronts deal the
+// 128-wide steps of K among themselves, KS at a time with all their loads in flight, and meet in LDS in a fixed order.  The
+// point of the small tile is that every CU has one: at 1 to 16 rows a 16-feature tile leaves 192 of 256 CUs idle, and one CU
+// pulls its 115 KiB of W no faster than ~33 GB/s.
+// Operand layout: lane (n, g) of a load holds elements 32 g + 8 (n & 3) .. of row 4 i + (n >> 2), so a quad of lanes reads 64 and the
+// wavefront 256 contiguous bytes of four rows; W and x alike.  Taken as it is by a 16 x 16 x 32 MFMA, "row" n of the operand is
+// (row n >> 2, k slice n & 3), and of the 16 x 16 results those whose k slices agree are partial sums: element i of lane (n, g)
+// belongs to feature g and row n >> 2 if i = n & 3.  Three of four MFMA results are thrown away; the matrix cores have nothing
+// else to do here (8 x 8 tile, K = 3584: 28 steps x 4 MFMAs per CU).
+// Measured in a HIP graph with the residual epilogue, K = 2048 / 3584 (before: skinny_gemm_kernel): 1 row 3.0 / 3.6 us (4.5 / 6.8),
+// 16 rows 3.6 / 4.5 (6.0 / 9.5), 32 rows 4.1 / 5.9 (6.0 / 9.2), 64 rows 5.3 / 7.2 (6.0 / 9.1).
+template <int NWV, int KS, int FG, int MG, int EPI>
+__global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
+                                                             const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N, int K,
+                                                             int groups) {
+    constexpr int F = 4 * FG, R = 4 * MG;
+    __shared__ __align__(16) float red[NWV][R][F];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int s = blockIdx.x >> 3, grp = s % groups, tile = (s / groups) * 8 + (blockIdx.x & 7);      // row groups of a tile: one XCD
+    const int n0 = tile * F, m0 = grp * R, steps = K / 128;
+    if (n0 >= N) return;
+    const bf16_t *wp[FG], *xp[MG];
+#pragma unroll
+    for (int f = 0; f < FG; f++) wp[f] = W + (size_t)min(n0 + 4 * f + (n >> 2), N - 1) * K + 32 * g + 8 * (n & 3);
+#pragma unroll
+    for (int m = 0; m < MG; m++) xp[m] = x + (size_t)min(m0 + 4 * m + (n >> 2), M - 1) * K + 32 * g + 8 * (n & 3);
+    f32x4 acc[FG][MG];
+#pragma unroll
+    for (int f = 0; f < FG; f++)
+#pragma unroll
+        for (int m = 0; m < MG; m++) acc[f][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int base = w; base < steps; base += NWV * KS) {
+        u32x4 a[KS][FG], b[KS][MG];
+#pragma unroll
+        for (int c = 0; c < KS; c++) {
+            const int k0 = min(base + c * NWV, steps - 1) * 128;  // (a step past the end loads the last one and is not multiplied)
+#pragma unroll
+            for (int f = 0; f < FG; f++) a[c][f] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp[f] + k0));
+#pragma unroll
+            for (int m = 0; m < MG; m++) b[c][m] = *reinterpret_cast<const u32x4*>(xp[m] + k0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < KS; c++)
+            if (base + c * NWV < steps)
+#pragma unroll
+                for (int f = 0; f < FG; f++)
+#pragma unroll
+                    for (int m = 0; m < MG; m++)
+                        acc[f][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[c][f]),
+                                                                           __builtin_bit_cast(bf16x8, b[c][m]), acc[f][m], 0, 0, 0);
     }
-    if (wpb <= 2)
-        launch_xlds_wpb<MS, 2>(epi, W, x, res, y, M, N, stream, (blocks + 1) / 2, 0);
-    else if (wpb == 3)
-        launch_xlds_wpb<MS, 3>(epi, W, x, res, y, M, N, stream, (blocks + 2) / 3, 0);
+    const int c = n & 3;                                          // of the quad's four sums lane c keeps the one of row block c
+#pragma unroll
+    for (int f = 0; f < FG; f++) {
+        float keep = 0.f;
+#pragma unroll
+        for (int m = 0; m < MG; m++) {
+            float v = c == 0 ? acc[f][m][0] : c == 1 ? acc[f][m][1] : c == 2 ? acc[f][m][2] : acc[f][m][3];
+            v += dpp_mov<0xB1>(v);
+            v += dpp_mov<0x4E>(v);
+            keep = (m == 0 || c == m) ? v : keep;
+        }
+        if (c < MG) red[w][4 * c + (n >> 2)][4 * f + g] = keep;
+    }
+    lds_barrier();
+    auto total = [&](int r, int f) {                              // fixed order: pairs, then pairs of pairs, ...
+        float t[NWV];
+#pragma unroll
+        for (int k = 0; k < NWV; k++) t[k] = red[k][r][f];
+#pragma unroll
+        for (int st = 1; st < NWV; st *= 2)
+#pragma unroll
+            for (int k = 0; k < NWV; k += 2 * st) t[k] += t[k + st];
+        return t[0];
+    };
+    if (EPI == EPI_SWIGLU) {
+        const int r = threadIdx.x / (F / 2), p = threadIdx.x % (F / 2), m = m0 + r;
+        if (r < R && m < M && n0 + 2 * p + 1 < N)
+            y[(size_t)m * (N / 2) + n0 / 2 + p] = f2bf(silu_bf16(BF(total(r, 2 * p))) * BF(total(r, 2 * p + 1)));
+    } else {
+        const int r = threadIdx.x / F, f = threadIdx.x % F, m = m0 + r;
+        if (r < R && m < M && n0 + f < N) {
+            const size_t o = (size_t)m * N + n0 + f;
+            const float v = total(r, f);
+            y[o] = EPI == EPI_ADD ? f2bf(BF(v) + bf2f(res[o])) : f2bf(v);
+        }
+    }
+}
+
+struct gemv_args {
+    const bf16_t *W, *x, *nw, *res;
+    bf16_t* y;
+    int M, N, K, epi;
+    float eps;
+    hipStream_t stream;
+};
+
+template <int RB, int FB, bool RMS>
+void launch_rows(const gemv_args& p, int cus) {
+    const int groups = (p.M + 16 * RB - 1) / (16 * RB), blocks = (p.N + 15) / 16, per_cu = cus / groups > 0 ? cus / groups : 1;
+    int tiles = (blocks + 2 * FB - 1) / (2 * FB), extra = 0;
+    // a few blocks more than a whole tile per CU: the first tiles take one each instead of a workgroup of their own
+    if (blocks > per_cu * 2 * FB && blocks - per_cu * 2 * FB <= per_cu / 16) tiles = per_cu, extra = blocks - per_cu * 2 * FB;
+    const dim3 grid((tiles + 7) / 8 * 8 * groups), block(512);
+    if (p.epi == EPI_NONE)
+        hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_NONE>), grid, block, 0, p.stream, p.W, p.x, p.nw, p.eps, p.res, p.y, p.M, p.N, groups, tiles, extra);
+    else if (p.epi == EPI_ADD)
+        hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_ADD>), grid, block, 0, p.stream, p.W, p.x, p.nw, p.eps, p.res, p.y, p.M, p.N, groups, tiles, extra);
     else
-        launch_xlds_wpb<MS, 4>(epi, W, x, res, y, M, N, stream, (blocks + 3) / 4, 0);
+        hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_SWIGLU>), grid, block, 0, p.stream, p.W, p.x, p.nw, p.eps, p.res, p.y, p.M, p.N, groups, tiles, extra);
+}
+// the shapes rows_gemm_kernel takes (its 8-byte stores and residual loads want y and res aligned to 8 bytes)
+inline bool rows_shape(const gemv_args& p) {
+    return p.K == XK && p.N >= 4096 && (p.N & 3) == 0 && ((reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.res)) & 7u) == 0;
+}
+constexpr int RMS_ROWS_MAX = 96;       // most rows with the prologue fused in: beyond, the rows are normalised too often
+// Tile by rows.  Up to 96 rows: the smallest tile that leaves at most one workgroup per CU (32 features as long as one row
+// group holds the batch, then 64).  Beyond 96 rows there is no such tile; 64 x 64 up to 128 rows, then 32 x 32 (N = 8224 /
+// 7168 / 5120 at 128 rows 9.9 / 9.6 / 8.6 us against 20.8 / 19.7 / 11.7 before, at 256 rows 19.6 / 18.4 / 13.0 against 30.8 / 28.3 /
+// 21.5).
+template <bool RMS>
+void launch_rows_any(const gemv_args& p, int cus) {
+    if (p.M <= 16)
+        launch_rows<1, 1, RMS>(p, cus);
+    else if (p.M <= 32)
+        launch_rows<2, 1, RMS>(p, cus);
+    else if (p.M <= 48)
+        launch_rows<3, 1, RMS>(p, cus);
+    else if (p.M <= 64 || (p.M <= 96 && ((p.N + 63) / 64) * 3 <= cus))
+        launch_rows<2, 2, RMS>(p, cus);
+    else if (p.M <= 96)
+        launch_rows<3, 2, RMS>(p, cus);
+    else if constexpr (!RMS) {
+        if (p.M <= 128)
+            launch_rows<4, 2, false>(p, cus);
+        else
+            launch_rows<2, 1, false>(p, cus);
+    }
+}
+
+template <int NWV, int KS, int FG, int MG>
+void launch_quad_tile(const gemv_args& p) {
+    const int groups = (p.M + 4 * MG - 1) / (4 * MG), tiles = (p.N + 4 * FG - 1) / (4 * FG);
+    const dim3 grid((tiles + 7) / 8 * 8 * groups), block(64 * NWV);
+    if (p.epi == EPI_NONE)
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_NONE>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+    else if (p.epi == EPI_ADD)
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_ADD>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+    else
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_SWIGLU>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+}
+template <int FG, int MG>
+void launch_quad(const gemv_args& p) {       // wavefronts and steps at a time by K: all of K in flight at once up to 4096
+    if (p.K <= 1024)
+        launch_quad_tile<4, 2, FG, MG>(p);
+    else if (p.K <= 2048)
+        launch_quad_tile<8, 2, FG, MG>(p);
+    else
+        launch_quad_tile<8, 4, FG, MG>(p);
+}
+// The smallest tile that leaves at most one workgroup per CU; some shapes still gain with two or four workgroups per CU
+// (measured against skinny_gemm_kernel over N = 264 .. 8192, K = 512 .. 3584, 1 .. 128 rows: N = 1024, K = 2048, 64 rows, two
+// workgroups of 8 x 16 per CU 5.3 against 6.0 us; N = 8192, K = 2048, 8 rows, four of 8 x 8 8.3 against 9.4; but N = 4096, K = 2048,
+// 32 rows 9.7 against 8.4).  Returns false where the skinny kernel is the better one.
+inline bool launch_quad_any(const gemv_args& p, int cus) {
+    auto wgs = [&](int f, int r) { return (long)((p.N + f - 1) / f) * ((p.M + r - 1) / r); };
+    if (wgs(4, 4) <= cus || (p.M <= 4 && wgs(4, 4) <= 2 * cus))
+        launch_quad<1, 1>(p);
+    else if (wgs(8, 8) <= cus || (p.M <= 8 && wgs(8, 8) <= 4 * cus))
+        launch_quad<2, 2>(p);
+    else if (wgs(8, 16) <= cus)
+        launch_quad<2, 4>(p);
+    else if (p.K > 2048 && wgs(16, 16) <= cus)
+        launch_quad<4, 4>(p);
+    else if (p.K > 1024 && p.K <= 2048 && wgs(8, 16) <= 2 * cus)
+        launch_quad<2, 4>(p);
+    else
+        return false;
+    return true;
 }
 
 // row blocks per pass: 1, 2 or 4 (3 rounds up)
 inline int row_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
-
-template <int NWV, int KCW, int NT, int MS>
-void launch_wide_ms(int epi, const bf16_t* W, const bf16_t* x, const bf16_t* res, bf16_t* y, int M, int N, int K, hipStream_t stream) {
-    const dim3 grid((N + 16 * NT - 1) / (16 * NT), (M + 16 * MS - 1) / (16 * MS)), block(64 * NWV);
-    if (epi == EPI_NONE)
-        hipLaunchKernelGGL((wide_gemm_kernel<NWV, KCW, NT, MS, EPI_NONE>), grid, block, 0, stream, W, x, res, y, M, N, K);
-    else if (epi == EPI_ADD)
-        hipLaunchKernelGGL((wide_gemm_kernel<NWV, KCW, NT, MS, EPI_ADD>), grid, block, 0, stream, W, x, res, y, M, N, K);
-    else
-        hipLaunchKernelGGL((wide_gemm_kernel<NWV, KCW, NT, MS, EPI_SWIGLU>), grid, block, 0, stream, W, x, res, y, M, N, K);
-}
-template <int NWV, int KCW, int NT>
-void launch_wide(int epi, const bf16_t* W, const bf16_t* x, const bf16_t* res, bf16_t* y, int M, int N, int K, hipStream_t stream) {
-    if (row_blocks(M) == 2)
-        launch_wide_ms<NWV, KCW, NT, 2>(epi, W, x, res, y, M, N, K, stream);
-    else
-        launch_wide_ms<NWV, KCW, NT, 4>(epi, W, x, res, y, M, N, K, stream);
-}
 
 template <int NWV, int MS>
 void launch_gemm_ms(int epi, const bf16_t* W, const bf16_t* x, const bf16_t* res, bf16_t* y, int M, int N, int K, hipStream_t stream) {
@@ -401,47 +579,55 @@ int qt_rms_rows(const void* x, const void* nw, void* y, int M, int K, float eps,
     return QT_OK;
 }
 
+static int check_gemv(const gemv_args& p) {
+    if (p.epi < 0 || p.epi > 2) return QT_ERR_UNSUPPORTED;
+    if (p.M < 0 || p.N < 1 || p.K < 256 || (p.K % 256) || (p.epi == EPI_SWIGLU && (p.N & 1))) return QT_ERR_DIM;
+    if (p.M == 0) return QT_OK;                                   // nothing to do: empty buffers may be null
+    if (!p.W || !p.x || !p.y || (p.epi == EPI_ADD && !p.res)) return QT_ERR_NULL;
+    for (const void* v : {p.W, p.x, p.nw})
+        if (reinterpret_cast<uintptr_t>(v) & 15u) return QT_ERR_ALIGN;
+    return QT_OK;
+}
+
 // y = epilogue(W [N, K] . x [M, K]^T): epilogue 0 none (y [M, N]), 1 add (res [M, N], y [M, N]), 2 swiglu (y [M, N / 2], N even).
 // K a multiple of 256.
 int qt_fused_gemv(const void* W, const void* x, const void* res, void* y, int M, int N, int K, int epilogue, hipStream_t stream) {
-    if (epilogue < 0 || epilogue > 2) return QT_ERR_UNSUPPORTED;
-    if (M < 0 || N < 1 || K < 256 || (K % 256) || (epilogue == EPI_SWIGLU && (N & 1))) return QT_ERR_DIM;
-    if (M == 0) return QT_OK;                                     // nothing to do: empty buffers may be null
-    if (!W || !x || !y || (epilogue == EPI_ADD && !res)) return QT_ERR_NULL;
-    for (const void* p : {W, x})
-        if (reinterpret_cast<uintptr_t>(p) & 15u) return QT_ERR_ALIGN;
+    const gemv_args p{(const bf16_t*)W, (const bf16_t*)x, nullptr, (const bf16_t*)res, (bf16_t*)y, M, N, K, epilogue, 0.f, stream};
+    const int rc = check_gemv(p);
+    if (rc != QT_OK || M == 0) return rc;
+    const int cus = cu_count();
+    if (rows_shape(p)) {
+        launch_rows_any<false>(p, cus);
+        QT_CHECK_LAUNCH();
+        return QT_OK;
+    }
+    if (launch_quad_any(p, cus)) {
+        QT_CHECK_LAUNCH();
+        return QT_OK;
+    }
     // wavefronts per workgroup: 4 when the output is wide enough to fill the chip with workgroups; 16 or 8 (as K divides) for
     // the narrow outputs, whose few workgroups would otherwise walk long K chains
     const int kc = K / 32;
-    // the wide projections of a decode batch: rows in LDS.  From four rows on (in_proj, one row 6.6 us either way; 4 / 16 /
-    // 64 rows: 6.9 / 7.0 / 9.7 us against 7.0 / 8.4 / 11.9 us for the kernels below)
-    // (its 8-byte stores and residual loads want y and res aligned to 8 bytes; anything else takes the general kernels)
-    if (K == XK && N >= 4096 && (N & 3) == 0 && M >= 4 && M <= 64 &&
-        ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(res)) & 7u) == 0) {
-        const int cus = cu_count();
-        if (M <= 16)
-            launch_xlds_ms<1>(epilogue, (const bf16_t*)W, (const bf16_t*)x, (const bf16_t*)res, (bf16_t*)y, M, N, stream, cus);
-        else if (M <= 32)
-            launch_xlds_ms<2>(epilogue, (const bf16_t*)W, (const bf16_t*)x, (const bf16_t*)res, (bf16_t*)y, M, N, stream, cus);
-        else
-            launch_xlds_ms<4>(epilogue, (const bf16_t*)W, (const bf16_t*)x, (const bf16_t*)res, (bf16_t*)y, M, N, stream, cus);
-        QT_CHECK_LAUNCH();
-        return QT_OK;
-    }
-    if (K == 1024 && N >= 4096 && M > 16) {                       // ... of more than 64 rows: x stays in registers
-        // three feature blocks per workgroup (172 workgroups for 8224 features): four leave half the CUs without one, two
-        // double what the workgroups pull of x from L2; measured 13.2 / 11.7 / 16.3 us for 4 / 3 / 2 at 64 rows
-        launch_wide<8, 4, 3>(epilogue, (const bf16_t*)W, (const bf16_t*)x, (const bf16_t*)res, (bf16_t*)y, M, N, K, stream);
-        QT_CHECK_LAUNCH();
-        return QT_OK;
-    }
     const bool wide = (long)((N + 15) / 16) * ((M + MT - 1) / MT) >= 512;
     if (!wide && kc % (2 * 16) == 0)
-        launch_gemm<16>(epilogue, (const bf16_t*)W, (const bf16_t*)x, (const bf16_t*)res, (bf16_t*)y, M, N, K, stream, true);
+        launch_gemm<16>(epilogue, p.W, p.x, p.res, p.y, M, N, K, stream, true);
     else if (!wide && kc % (2 * 8) == 0)
-        launch_gemm<8>(epilogue, (const bf16_t*)W, (const bf16_t*)x, (const bf16_t*)res, (bf16_t*)y, M, N, K, stream, true);
+        launch_gemm<8>(epilogue, p.W, p.x, p.res, p.y, M, N, K, stream, true);
     else
-        launch_gemm<4>(epilogue, (const bf16_t*)W, (const bf16_t*)x, (const bf16_t*)res, (bf16_t*)y, M, N, K, stream, !wide);
+        launch_gemm<4>(epilogue, p.W, p.x, p.res, p.y, M, N, K, stream, !wide);
+    QT_CHECK_LAUNCH();
+    return QT_OK;
+}
+
+// qt_rms_rows and qt_fused_gemv in one launch, for the shapes where that is the faster form; -4 for the others (nothing launched).
+int qt_fused_gemv_rms(const void* W, const void* x, const void* nw, float eps, const void* res, void* y, int M, int N, int K, int epilogue,
+                      hipStream_t stream) {
+    const gemv_args p{(const bf16_t*)W, (const bf16_t*)x, (const bf16_t*)nw, (const bf16_t*)res, (bf16_t*)y, M, N, K, epilogue, eps, stream};
+    const int rc = check_gemv(p);
+    if (rc != QT_OK || M == 0) return rc;
+    if (!nw) return QT_ERR_NULL;
+    if (!rows_shape(p) || M > RMS_ROWS_MAX) return QT_ERR_UNSUPPORTED;
+    launch_rows_any<true>(p, cu_count());
     QT_CHECK_LAUNCH();
     return QT_OK;
 }

@@ -77,8 +77,6 @@ def fused_gemv(W, x, *, nw=None, eps=1e-6, res=None, swiglu=False, gnorm=None, T
         raise ValueError("nw and gnorm are exclusive")
     if swiglu and res is not None:
         raise ValueError("swiglu and res are exclusive")
-    if nw is not None:
-        x = rms_rows(x, nw, eps)
     if gnorm is not None:
         from .batch import gnorm_rows
         x = gnorm_rows(x, gnorm[0].reshape(M, PW), gnorm[1], eps)
@@ -87,5 +85,14 @@ def fused_gemv(W, x, *, nw=None, eps=1e-6, res=None, swiglu=False, gnorm=None, T
     if res is not None:
         res = L.dev(res.reshape(-1, N), BF16, "res", (M, N))
     y = torch.empty((M, n_out), dtype=BF16, device=x.device)
+    if nw is not None:
+        nw = L.dev(nw, BF16, "nw", (K,))
+        # one launch for the shapes that have it (the C side decides), otherwise the prologue as its own kernel
+        rc = L.lib().qt_fused_gemv_rms(L.ptr(W), L.ptr(x), L.ptr(nw), float(eps), L.ptr(res), L.ptr(y), M, N, K, epi, L.stream())
+        if rc == 0:
+            return y.reshape(*lead, n_out)
+        if rc != -4:
+            raise RuntimeError(f"qt_fused_gemv_rms failed: {L.ERRORS.get(rc, rc)}")
+        x = rms_rows(x, nw, eps)
     L.call("qt_fused_gemv", L.ptr(W), L.ptr(x), L.ptr(res), L.ptr(y), M, N, K, epi, L.stream())
     return y.reshape(*lead, n_out)

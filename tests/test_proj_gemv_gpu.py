@@ -108,6 +108,52 @@ def test_wide_projection_exact_and_any_output_alignment(qt, dev, M, N, epi):
     assert torch.equal(ybuf[1:1 + M * NO].reshape(M, NO), got), "outputs off an 8-byte boundary differ"
 
 
+# edges of the row blocks (16, 32, 48, 64, 96, 128 rows) and of the feature tiles (32 or 64 features; 8224 = 514 blocks of 16, more
+# than two per CU by two; 4100 = a last block of 4 features; 5132 = 64 x 80 + 12)
+@pytest.mark.parametrize("M,N,epi", [
+    (1, 4096, 0), (1, 8224, 2), (15, 4100, 0), (16, 8224, 1), (17, 5132, 0), (32, 8224, 2), (33, 4100, 1), (48, 8224, 0), (49, 8224, 1),
+    (64, 5132, 2), (65, 4100, 0), (80, 8224, 1), (96, 7168, 2), (97, 8224, 0), (128, 5132, 1), (129, 4096, 0), (257, 4100, 2)])
+def test_wide_projection_tiles_and_fused_rms_prologue(qt, dev, M, N, epi):
+    """exact on small integers (every order of summation gives the same bits); with the rms prologue, in one launch up to 96 rows,
+    the bits of the two calls"""
+    g = torch.Generator().manual_seed(M * 5 + N + epi)
+    K = 1024
+    W = to_dev(torch.randint(-3, 4, (N, K), generator=g).float().numpy(), dev, BF16)
+    x = torch.randint(-2, 3, (M, K), generator=g).float().numpy()
+    res = torch.randint(-9, 10, (M, N), generator=g).float().numpy() if epi == 1 else None
+    dres = None if res is None else to_dev(res, dev, BF16)
+    got = qt.kernels.fused_gemv(W, to_dev(x, dev, BF16), res=dres, swiglu=epi == 2)
+    want = O.fused_gemv(to_np(W), x, res=res, swiglu=epi == 2)
+    if epi == 2:
+        _close("integer swiglu", to_np(got), want, 1)
+    else:
+        check_equal("integer product", to_np(got), want)
+    r = to_dev(rand_bf(g, (M, K), 1.3), dev, BF16)
+    nw = to_dev(bf(1.0 + 0.2 * torch.randn(K, generator=g).numpy()), dev, BF16)
+    one = qt.kernels.fused_gemv(W, r, nw=nw, res=dres, swiglu=epi == 2)
+    two = qt.kernels.fused_gemv(W, qt.kernels.rms_rows(r, nw), res=dres, swiglu=epi == 2)
+    assert torch.equal(one, two), "rms prologue in the launch and on its own differ"
+
+
+# edges of the 4 x 4, 8 x 8, 8 x 16 and 16 x 16 tiles, outputs and rows that end inside a tile, K shorter than one batch of every
+# wavefront (256, 512), not a multiple of the wavefronts' steps (1280, 3584) and longer than one batch (4352)
+@pytest.mark.parametrize("M,N,K,epi", [
+    (1, 1024, 2048, 1), (1, 50, 256, 2), (3, 1027, 1280, 0), (4, 2048, 3584, 1), (5, 1024, 3584, 1), (8, 4090, 2048, 2), (9, 1030, 2048, 0),
+    (16, 1024, 4352, 1), (17, 1024, 2048, 1), (31, 1021, 3584, 0), (33, 1000, 2048, 2), (64, 1024, 3584, 1), (63, 1023, 3584, 0),
+    (64, 1024, 2048, 1), (5, 16, 512, 0), (40, 40, 256, 1)])
+def test_narrow_projection_tiles_exact_on_small_integers(qt, dev, M, N, K, epi):
+    g = torch.Generator().manual_seed(M * 3 + N + K + epi)
+    W = torch.randint(-3, 4, (N, K), generator=g).float().numpy()
+    x = torch.randint(-2, 3, (M, K), generator=g).float().numpy()
+    res = torch.randint(-9, 10, (M, N), generator=g).float().numpy() if epi == 1 else None
+    got = qt.kernels.fused_gemv(to_dev(W, dev, BF16), to_dev(x, dev, BF16), res=None if res is None else to_dev(res, dev, BF16), swiglu=epi == 2)
+    want = O.fused_gemv(W, x, res=res, swiglu=epi == 2)
+    if epi == 2:
+        _close("integer swiglu", to_np(got), want, 1)
+    else:
+        check_equal("integer product", to_np(got), want)
+
+
 def test_fused_gemv_prologues_and_leading_dims(qt, dev):
     """nw = rms_rows first; gnorm = gated norm first (same bits as the stand-alone kernels, qwen35/batch.py:241-248);
     leading dimensions are flattened and restored; float32 x holding bf16 values is taken as is"""
