@@ -173,6 +173,11 @@ long qt_gqa_prefill_workspace_bytes(int L);
 long qt_gqa_prefill_workspace_bytes_for(int S, int L, int q_pos0);
 int qt_gqa_prefill_causal(const void* q, const void* K, const void* V, void* out, void* workspace, long workspace_bytes, int S,
                           int L, int q_pos0, long q_head_stride, long kv_head_stride, qt_stream_t stream);
+/* The same with a row stride for q and out (elements, a multiple of 8): q_row_stride = 256 is the call above; rows as a projection
+ * leaves them, [S][8][256], have q_head_stride = 256 and q_row_stride = 2048. */
+int qt_gqa_prefill_causal_strided(const void* q, const void* K, const void* V, void* out, void* workspace, long workspace_bytes,
+                                  int S, int L, int q_pos0, long q_head_stride, int q_row_stride, long kv_head_stride,
+                                  qt_stream_t stream);
 
 /* The elementwise steps either side of the attention kernels in a full-attention layer (qwen35/batch.py:505-513,
  * qwen35/model.py:154-169).  qkv [R,5120] bf16 = [(q_h[256] | gate_h[256]) for 8 heads | k[2][256] | v[2][256]].

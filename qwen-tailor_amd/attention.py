@@ -12,7 +12,8 @@ BF16 = torch.bfloat16
 
 def scaled_dot_product_attention(q, k, v, *, scale: float, mask="causal"):
     """q [1, 8, S, 256], k / v [1, 2, L, 256] bf16 (k, v may be length-slices of a longer cache).  mask = "causal": query i
-    sits at position L - S + i and sees keys 0 .. L - S + i.  Returns [1, 8, S, 256] bf16."""
+    sits at position L - S + i and sees keys 0 .. L - S + i.  Returns [1, 8, S, 256] bf16 in q's memory layout: head-major, or
+    token-major if q is the transposed view of [S, 8, 256] rows (what qkv_prep returns and out_gate takes); neither is copied."""
     if mask != "causal":
         raise ValueError("only mask='causal' is built (decode / verify rows go through batch.attn_b)")
     if abs(scale - 256 ** -0.5) > 1e-9:
@@ -30,13 +31,18 @@ def scaled_dot_product_attention(q, k, v, *, scale: float, mask="causal"):
     Lk = k.shape[2]
     if Lk < S:
         raise ValueError("fewer keys than queries")
-    q = q.contiguous()
-    out = torch.empty_like(q)
+    if q.stride() == (q.stride(0), 256, 2048, 1) and S > 1 and not q.data_ptr() & 15:      # a transposed view of token-major rows
+        out = torch.empty((1, S, 8, 256), dtype=BF16, device=q.device).transpose(1, 2)
+        head_stride, row_stride = 256, 2048
+    else:
+        q = q.contiguous()
+        out = torch.empty_like(q)
+        head_stride, row_stride = S * 256, 256
     # launches that would leave half of the CUs idle are split along the keys; their parts meet in a workspace
     nws = L.lib().qt_gqa_prefill_workspace_bytes_for(S, Lk, Lk - S)
     ws = L.workspace("prefill_attention", q.device, nws) if nws > 0 else None      # cached per (device, stream)
-    L.call("qt_gqa_prefill_causal", L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), L.ptr(ws), max(nws, 0),
-           S, Lk, Lk - S, S * 256, k.stride(1), L.stream())
+    L.call("qt_gqa_prefill_causal_strided", L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), L.ptr(ws), max(nws, 0),
+           S, Lk, Lk - S, head_stride, row_stride, k.stride(1), L.stream())
     return out
 
 

@@ -25,78 +25,104 @@ __constant__ float rope_freq[ROPE_DIM / 2] = {
     2.54829683e-05f, 1.5399266e-05f, 9.3057206e-06f, 5.62341347e-06f, 3.39820826e-06f, 2.05352512e-06f,
     1.24093776e-06f, 7.49894184e-07f, 4.5315835e-07f, 2.73841977e-07f, 1.65481708e-07f};
 
-// One workgroup per row r = b * M + j (position pos[b] + j): threads 0..31 bring the row's 32 (cos, sin) pairs into LDS, from
-// the table of rope_table_kernel where it covers the position, else evaluated here (double-precision libm, the expensive part:
-// the same expression, so the same bits); then a wavefront takes one 256-wide vector at a time (lane l holds elements
-// 4l .. 4l+3) out of the row's 12: 0..7 = q heads, 8..9 = k heads, 10..11 = v heads.
+// One wavefront per row r = b * M + j (position pos[b] + j), four rows per workgroup.  The row's twelve 256-wide vectors (8 q heads, 2
+// k heads, 2 v heads) are taken four at a time, one per 16-lane group: lane c of a group holds elements 8 c .. + 7 and 128 + 8 c ..
+// + 7, so every load and store is 16 bytes per lane and all six loads of a row are in flight at once; a sum of squares needs
+// four DPP steps, and no exchange leaves the wavefront.  The row's 32 (cos, sin) pairs come from the table of rope_table_kernel
+// where it covers the position, else lanes 0..31 evaluate one each (double-precision libm, the expensive part: the same
+// expression, so the same bits).
+// Bound by the bytes it moves (12 KiB in and out per row).  With the table, 1024 / 2048 / 4096 / 8192 rows 7.6 / 11.1 / 17.8 / 29.3
+// us with a workgroup per row, 8 bytes per lane and the sums over 64 lanes through LDS; now 5.4 / 8.6 / 13.9 / 25.0 us (4 TB/s).
+// Nontemporal stores would take another 1 us off this kernel at 2048 rows, and cost the attention kernel that reads q next 18 us
+// at 8192.
 __global__ __launch_bounds__(256) void attn_qkv_prep_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ q_norm,
                                                             const bf16_t* __restrict__ k_norm, const int* __restrict__ pos,
                                                             bf16_t* __restrict__ q, bf16_t* __restrict__ k, bf16_t* __restrict__ v,
                                                             long R, int M, float eps, const float2* __restrict__ table,
                                                             int table_positions) {
-    __shared__ float cs_s[2][ROPE_DIM / 2];
-    const long r = blockIdx.x;
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const bf16_t* row = qkv + r * QKV_W;
-    // all loads of this wavefront's three vectors first
-    uint2 xw[3];
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4), aligned(8)));      // the entry points ask for 8-byte alignment only
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) float2 cs_s[4][ROPE_DIM / 2];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, rr = lane >> 4, c = lane & 15;
+    const long r = (long)blockIdx.x * 4 + w;
+    if (r >= R) return;
+    // vector t of the group: q heads rr and 4 + rr, then (k0, k1, v0, v1)[rr]
+    const bf16_t* row = qkv + r * QKV_W + 8 * c;
+    u32x4 x[3][2], wn[2][2];
 #pragma unroll
-    for (int t = 0; t < 3; t++) {
-        const int part = w + 4 * t;
-        xw[t] = reinterpret_cast<const uint2*>(part < 8 ? row + part * 2 * AD : row + AH * 2 * AD + (part - 8) * AD)[lane];
+    for (int hf = 0; hf < 2; hf++) {
+        x[0][hf] = *reinterpret_cast<const u32x4*>(row + rr * 2 * AD + 128 * hf);
+        x[1][hf] = *reinterpret_cast<const u32x4*>(row + (4 + rr) * 2 * AD + 128 * hf);
+        x[2][hf] = *reinterpret_cast<const u32x4*>(row + AH * 2 * AD + rr * AD + 128 * hf);
+        wn[0][hf] = *reinterpret_cast<const u32x4*>(q_norm + 8 * c + 128 * hf);
+        wn[1][hf] = *reinterpret_cast<const u32x4*>(k_norm + 8 * c + 128 * hf);
     }
-    const uint2 wq = reinterpret_cast<const uint2*>(q_norm)[lane], wk = reinterpret_cast<const uint2*>(k_norm)[lane];
-    if (threadIdx.x < ROPE_DIM / 2) {
-        const int ip = pos[r / M] + (int)(r % M);
+    const int ip = pos[(unsigned)r / (unsigned)M] + (int)((unsigned)r % (unsigned)M);
+    if (lane < ROPE_DIM / 2) {
         if (ip >= 0 && ip < table_positions) {                   // (table_positions = 0 without a table)
-            const float2 cs = table[(size_t)ip * (ROPE_DIM / 2) + threadIdx.x];
-            cs_s[0][threadIdx.x] = cs.x;
-            cs_s[1][threadIdx.x] = cs.y;
+            cs_s[w][lane] = table[(size_t)ip * (ROPE_DIM / 2) + lane];
         } else {
-            const float th = __fmul_rn((float)ip, rope_freq[threadIdx.x]);
-            cs_s[0][threadIdx.x] = (float)cos((double)th);
-            cs_s[1][threadIdx.x] = (float)sin((double)th);
+            const float th = __fmul_rn((float)ip, rope_freq[lane]);
+            cs_s[w][lane] = make_float2((float)cos((double)th), (float)sin((double)th));
         }
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    f32x4 cs[4];                                                  // pairs 8 (c & 3) .. + 7: (cos, sin, cos, sin) each (lanes c < 8 use them)
+#pragma unroll
+    for (int i = 0; i < 4; i++) cs[i] = reinterpret_cast<const f32x4*>(&cs_s[w][8 * (c & 3)])[i];
+    // v is a plain copy into the contiguous [R,2,256] layout
+    if (rr >= 2) {
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++) *reinterpret_cast<u32x4*>(v + (r * AKV + rr - 2) * AD + 8 * c + 128 * hf) = x[2][hf];
+    }
 #pragma unroll
     for (int t = 0; t < 3; t++) {
-        const int part = w + 4 * t;                              // wavefront-uniform
-        if (part >= 10) {                                        // v: a plain copy into the contiguous [R,2,256] layout
-            reinterpret_cast<uint2*>(v + (r * AKV + (part - 10)) * AD)[lane] = xw[t];
-            continue;
-        }
-        const bool is_q = part < 8;
-        const uint2 ww = is_q ? wq : wk;
-        float x[4] = {lo_bf(xw[t].x), hi_bf(xw[t].x), lo_bf(xw[t].y), hi_bf(xw[t].y)};
-        const float wt[4] = {lo_bf(ww.x), hi_bf(ww.x), lo_bf(ww.y), hi_bf(ww.y)};
+        const u32x4(&wt)[2] = wn[t == 2 ? 1 : 0];
         double ss = 0.0;
 #pragma unroll
-        for (int e = 0; e < 4; e++) ss += (double)x[e] * x[e];
-        const float inv = rsqrt_rn((float)wave_sum_d(ss) / (float)AD + eps);
-        float y[4];
+        for (int hf = 0; hf < 2; hf++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = BF(wt[e] * BF(x[e] * inv));
-        // rotary embedding of features 0..63: lanes 0..7 hold x1 = features 0..31, lanes 8..15 their partners 32..63
-        float o4[4];
+            for (int j = 0; j < 4; j++) {
+                const double lo = (double)lo_bf(x[t][hf][j]), hi = (double)hi_bf(x[t][hf][j]);
+                ss = fma(hi, hi, fma(lo, lo, ss));
+            }
+        const float inv = rsqrt_rn((float)row16_sum_d(ss) / (float)AD + eps);
+        u32x4 y[2];
 #pragma unroll
-        for (int e = 0; e < 4; e++) o4[e] = __shfl_xor(y[e], 8, 64);
-        if (lane < 16) {
+        for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t n2 = pack2_bf(lo_bf(x[t][hf][j]) * inv, hi_bf(x[t][hf][j]) * inv);
+                y[hf][j] = pack2_bf(lo_bf(wt[hf][j]) * lo_bf(n2), hi_bf(wt[hf][j]) * hi_bf(n2));
+            }
+        // rotary embedding of features 0..63: lanes 0..3 of a group hold x1 = features 0..31, lanes 4..7 their partners 32..63 (lane
+        // c ^ 4 = the half row mirrored, then every quad reversed)
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int m = __builtin_amdgcn_update_dpp(0, (int)y[0][j], 0x141, 0xF, 0xF, true);
+            o[j] = (unsigned)__builtin_amdgcn_update_dpp(0, m, 0x1B, 0xF, 0xF, true);
+        }
+        if (c < 8) {
             // The two products and their sum are rounded one by one.  Plain operators inside a contract(off) block: the
             // __fmul_rn / __fadd_rn helpers are ordinary operators compiled elsewhere, which the compiler contracts into one
             // fused multiply-add after inlining (a bf16 value in ~10^5 then rounds the other way).
 #pragma clang fp contract(off)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int i = (lane & 7) * 4 + e;
-                const float c = cs_s[0][i], sn = cs_s[1][i];
-                const float own = y[e] * c, other = o4[e] * sn;
-                y[e] = BF(lane < 8 ? own - other                 // y1 c - y2 s
-                                   : other + own);               // y1 s + y2 c
+            for (int j = 0; j < 4; j++) {
+                const float a0 = lo_bf(y[0][j]) * cs[j][0], b0 = lo_bf(o[j]) * cs[j][1];
+                const float a1 = hi_bf(y[0][j]) * cs[j][2], b1 = hi_bf(o[j]) * cs[j][3];
+                y[0][j] = c < 4 ? pack2_bf(a0 - b0, a1 - b1)     // y1 c - y2 s
+                                : pack2_bf(b0 + a0, b1 + a1);    // y1 s + y2 c
             }
         }
-        bf16_t* dst = is_q ? q + (r * AH + part) * AD : k + (r * AKV + (part - 8)) * AD;
-        reinterpret_cast<uint2*>(dst)[lane] = make_uint2(pack_bf(y[0], y[1]), pack_bf(y[2], y[3]));
+        bf16_t* dst = t < 2 ? q + (r * AH + 4 * t + rr) * AD : k + (r * AKV + rr) * AD;
+        if (t < 2 || rr < 2) {
+#pragma unroll
+            for (int hf = 0; hf < 2; hf++) *reinterpret_cast<u32x4*>(dst + 8 * c + 128 * hf) = y[hf];
+        }
     }
 }
 
@@ -141,7 +167,7 @@ int qt_attn_qkv_prep_table(const void* qkv, const void* q_norm, const void* k_no
     if (R == 0) return QT_OK;
     for (const void* p : {qkv, q_norm, k_norm, rope_table, (const void*)q, (const void*)k, (const void*)v})
         if (reinterpret_cast<uintptr_t>(p) & 7u) return QT_ERR_ALIGN;
-    hipLaunchKernelGGL(attn_qkv_prep_kernel, dim3((unsigned)R), dim3(256), 0, stream, (const bf16_t*)qkv, (const bf16_t*)q_norm,
+    hipLaunchKernelGGL(attn_qkv_prep_kernel, dim3((unsigned)((R + 3) / 4)), dim3(256), 0, stream, (const bf16_t*)qkv, (const bf16_t*)q_norm,
                        (const bf16_t*)k_norm, pos, (bf16_t*)q, (bf16_t*)k, (bf16_t*)v, R, M, eps, (const float2*)rope_table,
                        rope_table ? table_positions : 0);
     QT_CHECK_LAUNCH();

@@ -137,7 +137,7 @@ __device__ __forceinline__ volatile __attribute__((address_space(3))) int* lds_w
 template <int NH>
 __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ K,
                                                               const bf16_t* __restrict__ V, bf16_t* __restrict__ out, int S, int L,
-                                                              int q_pos0, long q_head_stride, long kv_head_stride, int tmax,
+                                                              int q_pos0, long q_head_stride, int q_row_stride, long kv_head_stride, int tmax,
                                                               _Float16* __restrict__ part_o, float* __restrict__ part_ml) {
     __shared__ __align__(1024) bf16_t kv_s[4 * TILE];            // K tiles of even / odd iterations, then the V tiles
     __shared__ __align__(16) u32x4 p_s[4][NH][2][64];             // [pair][head][32-key half][lane]: P as the lanes hold it
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         bf16x8 bq[NH][8];
 #pragma unroll
         for (int hh = 0; hh < NH; hh++) {
-            const u32x4* qr = reinterpret_cast<const u32x4*>(q + (size_t)(h0 + hh) * q_head_stride + (size_t)(row_ok ? row : 0) * AD);
+            const u32x4* qr = reinterpret_cast<const u32x4*>(q + (size_t)(h0 + hh) * q_head_stride + (size_t)(row_ok ? row : 0) * q_row_stride);
 #pragma unroll
             for (int kb = 0; kb < 8; kb++) {
                 u32x4 v = qr[kb * 4 + g];
@@ -563,7 +563,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
             const int orow = r0 + 4 * g + r;
             if (orow < S) {
                 const float inv = 1.0f / Lsum[hh][r];
-                bf16_t* dst = out + (size_t)(h0 + hh) * q_head_stride + (size_t)orow * AD + n;
+                bf16_t* dst = out + (size_t)(h0 + hh) * q_head_stride + (size_t)orow * q_row_stride + n;
 #pragma unroll
                 for (int j = 0; j < 16; j++) dst[16 * j] = f2bf(O[hh][j][r] * inv);
             }
@@ -577,7 +577,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
 template <int RB>
 __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                  bf16_t* __restrict__ out, int S, int q_pos0, int tmax, long slots_per_kv,
-                                                                 long q_head_stride) {
+                                                                 long q_head_stride, int q_row_stride) {
     constexpr int PO = part_o_floats(RB), PML = part_ml_floats(RB);
     const int c = (KT / RB) * tmax, p = (q_pos0 + RB - 1) / RB;
     const int rb = max(0, c - p) + blockIdx.x;                   // the first block with two parts is c - p
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16*
             pk[2 * i] = pack_bf(acc[i][0] * inv, acc[i][1] * inv);
             pk[2 * i + 1] = pack_bf(acc[i][2] * inv, acc[i][3] * inv);
         }
-        u32x4* dst = reinterpret_cast<u32x4*>(out + (size_t)(blockIdx.y * (AH / AKV) + hq) * q_head_stride + (size_t)(rb * RB + lr) * AD + cg * 16);
+        u32x4* dst = reinterpret_cast<u32x4*>(out + (size_t)(blockIdx.y * (AH / AKV) + hq) * q_head_stride + (size_t)(rb * RB + lr) * q_row_stride + cg * 16);
         dst[0] = u32x4{pk[0], pk[1], pk[2], pk[3]};
         dst[1] = u32x4{pk[4], pk[5], pk[6], pk[7]};
     }
@@ -708,17 +708,21 @@ long qt_gqa_prefill_workspace_bytes(int L) {
     return std::max(b16, b32);
 }
 
-// q, out [8][S][256] bf16 (head stride q_head_stride elements), K, V [2][>=L][256] bf16 (head stride kv_head_stride):
+// q, out [8 heads][S rows][256] bf16 with head stride q_head_stride and row stride q_row_stride (elements; head-major rows have row
+// stride 256, the token-major rows of a projection head stride 256 and row stride 2048, so neither has to be copied into the other),
+// K, V [2][>=L][256] bf16 (head stride kv_head_stride):
 // query i sits at absolute position q_pos0 + i and sees keys 0 .. q_pos0 + i (< L).  workspace: see above; may be null.
-int qt_gqa_prefill_causal(const void* q, const void* K, const void* V, void* out, void* workspace, long workspace_bytes, int S,
-                          int L, int q_pos0, long q_head_stride, long kv_head_stride, hipStream_t stream) {
+int qt_gqa_prefill_causal_strided(const void* q, const void* K, const void* V, void* out, void* workspace, long workspace_bytes, int S,
+                          int L, int q_pos0, long q_head_stride, int q_row_stride, long kv_head_stride, hipStream_t stream) {
     if (!q || !K || !V || !out) return QT_ERR_NULL;
-    if (S < 0 || L < 1 || q_pos0 < 0 || (long)q_pos0 + S > L || q_head_stride < (long)S * AD || kv_head_stride < (long)L * AD)
+    if (S < 0 || L < 1 || q_pos0 < 0 || (long)q_pos0 + S > L || kv_head_stride < (long)L * AD || q_row_stride < AD)
         return QT_ERR_DIM;
+    // the rows of different heads must not overlap: heads apart by whole row ranges, or side by side within a row
+    if (q_head_stride < (long)S * q_row_stride && (q_head_stride < AD || q_row_stride < (AH - 1) * q_head_stride + AD)) return QT_ERR_DIM;
     if (S == 0) return QT_OK;
     for (const void* p : {q, K, V, (const void*)out, (const void*)workspace})
         if (reinterpret_cast<uintptr_t>(p) & 15u) return QT_ERR_ALIGN;
-    if ((q_head_stride | kv_head_stride) & 7) return QT_ERR_ALIGN;
+    if ((q_head_stride | q_row_stride | kv_head_stride) & 7) return QT_ERR_ALIGN;
     KeySplit ks = plan_split(S, L, q_pos0);
     if (ks.tmax && (!workspace || workspace_bytes < ks.bytes())) {          // no room for the parts: the unsplit form
         ks = KeySplit();
@@ -730,21 +734,26 @@ int qt_gqa_prefill_causal(const void* q, const void* K, const void* V, void* out
     float* part_ml = ks.tmax ? reinterpret_cast<float*>(part_o + (size_t)ks.parts * AKV * part_o_floats(RB)) : nullptr;
     if (ks.nh == 2)
         hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(512), 0, stream, (const bf16_t*)q, (const bf16_t*)K, (const bf16_t*)V,
-                           (bf16_t*)out, S, L, q_pos0, q_head_stride, kv_head_stride, ks.tmax, part_o, part_ml);
+                           (bf16_t*)out, S, L, q_pos0, q_head_stride, q_row_stride, kv_head_stride, ks.tmax, part_o, part_ml);
     else
         hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, dim3(512), 0, stream, (const bf16_t*)q, (const bf16_t*)K, (const bf16_t*)V,
-                           (bf16_t*)out, S, L, q_pos0, q_head_stride, kv_head_stride, ks.tmax, part_o, part_ml);
+                           (bf16_t*)out, S, L, q_pos0, q_head_stride, q_row_stride, kv_head_stride, ks.tmax, part_o, part_ml);
     if (ks.tmax) {
         const dim3 mgrid((unsigned)ks.split_blocks, AKV, (AH / AKV) * ks.nh);
         if (ks.nh == 2)
             hipLaunchKernelGGL(attn_prefill_merge_kernel<32>, mgrid, dim3(256), 0, stream, part_o, part_ml, (bf16_t*)out, S, q_pos0,
-                               ks.tmax, ks.parts, q_head_stride);
+                               ks.tmax, ks.parts, q_head_stride, q_row_stride);
         else
             hipLaunchKernelGGL(attn_prefill_merge_kernel<16>, mgrid, dim3(256), 0, stream, part_o, part_ml, (bf16_t*)out, S, q_pos0,
-                               ks.tmax, ks.parts, q_head_stride);
+                               ks.tmax, ks.parts, q_head_stride, q_row_stride);
     }
     QT_CHECK_LAUNCH();
     return QT_OK;
+}
+int qt_gqa_prefill_causal(const void* q, const void* K, const void* V, void* out, void* workspace, long workspace_bytes, int S,
+                          int L, int q_pos0, long q_head_stride, long kv_head_stride, hipStream_t stream) {
+    if (q_head_stride < (long)S * AD) return !q || !K || !V || !out ? QT_ERR_NULL : QT_ERR_DIM;
+    return qt_gqa_prefill_causal_strided(q, K, V, out, workspace, workspace_bytes, S, L, q_pos0, q_head_stride, AD, kv_head_stride, stream);
 }
 
 }  // extern "C"

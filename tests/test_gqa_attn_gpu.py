@@ -404,6 +404,20 @@ def test_prefill_causal_split_equals_unsplit_on_random_shapes(qt, dev):
     assert nsplit >= 10, nsplit                                   # the sample does exercise the split
 
 
+# unsplit and split launches of both forms (16- and 32-row blocks), one row, a partial last block
+@pytest.mark.parametrize("S,L", [(2, 2), (37, 200), (300, 3300), (1000, 1000), (2048, 2048), (4801, 4801)])
+def test_prefill_causal_token_major_rows_are_not_copied(qt, dev, S, L):
+    """q as the transposed view of [S, 8, 256] rows: the same bits as from head-major rows, in the same token-major layout"""
+    g = torch.Generator().manual_seed(S + L)
+    q = torch.randn((S, 8, 256), generator=g).bfloat16().to(dev)
+    K = torch.randn((1, 2, L, 256), generator=g).bfloat16().to(dev)
+    V = torch.randn((1, 2, L, 256), generator=g).bfloat16().to(dev)
+    f = lambda x: qt.attention.scaled_dot_product_attention(x, K, V, scale=256 ** -0.5, mask="causal")
+    a, b = f(q.transpose(0, 1)[None]), f(q.transpose(0, 1)[None].contiguous())
+    assert a.shape == b.shape and a[0].transpose(0, 1).is_contiguous() and b.is_contiguous()
+    check_tensors_equal("token-major against head-major", a.contiguous(), b)
+
+
 def test_prefill_causal_rejects_queries_past_the_keys(qt, dev):
     from qwen_tailor_amd import _lib as QL
     t = torch.zeros((1, 8, 32, 256), dtype=BF16, device=dev)
