@@ -161,6 +161,12 @@ int qt_gdn_phase_b(const void* ops, const void* U, const float* gC, void* snap, 
                    void* y, int S, qt_stream_t stream);
 int qt_gdn_phase_b_norm(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out,
                         const void* proj, const float* gw, float eps, void* out, int S, qt_stream_t stream);
+/* qt_gdn_phase_b (proj and gw null: out is y) or qt_gdn_phase_b_norm (both given) with a report to the host: host_words points at two
+ * int32 in pinned host memory that the GPU can write; word 0 / 1 is set to 1 where bit 0 / 1 of the status word is set (the
+ * status word in `snap` is set as well).  No launch clears them.  They can be read without synchronising (a launch still in
+ * flight has not reported yet) and need no copy behind the launch. */
+int qt_gdn_phase_b_report(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out,
+                          const void* proj, const float* gw, float eps, void* out, int S, int32_t* host_words, qt_stream_t stream);
 
 /* Causal prefill attention: the mx.fast.scaled_dot_product_attention(..., mask="causal") call of the full-attention layers
  * (qwen35/model.py:160-167, qwen35/prefill.py:468).  q, out [8][S][256] bf16 with head stride q_head_stride (elements);

@@ -4,7 +4,8 @@ There is no CPU fallback: every operator of this package runs a HIP kernel or ra
 from __future__ import annotations
 
 import ctypes
-import os
+import importlib.machinery
+import importlib.util
 
 import torch
 
@@ -32,6 +33,7 @@ _SIGS = {
     "qt_gqa_attn_layer_decode": [_vp] * 4 + [_i] + [_vp] * 6 + [_l, _i, _i, _i, _i, _i, _f, _vp],
     "qt_rope_table_build": [_vp, _i, _vp],
     "qt_gdn_phase_b": [_vp] * 7 + [_i, _vp],
+    "qt_gdn_phase_b_report": [_vp] * 8 + [_f, _vp, _i, _vp, _vp],
     "qt_gdn_phase_b_poll_limit": [_i],
     "qt_gdn_phase_b_norm": [_vp] * 8 + [_f, _vp, _i, _vp],
     "qt_gqa_prefill_causal": [_vp] * 5 + [_l, _i, _i, _i, _l, _l, _vp],
@@ -85,57 +87,32 @@ def call(name, *args):
         raise RuntimeError(f"{name} failed: {ERRORS.get(rc, rc)}")
 
 
-_SILU_TABLES = {}
+class _Host:
+    """The functions of csrc/_qt_host (host.cpp): argument checks, output allocation and launch of one operator in a native call.
+    The module is loaded (and built, if it is missing or out of date) when the first of them is asked for."""
+
+    def __getattr__(self, name):
+        lib()                                                    # libqwen_tailor_hip.so: current, and loaded first
+        loader = importlib.machinery.ExtensionFileLoader("_qt_host", _build.HOST_SO)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_qt_host", loader))
+        loader.exec_module(module)
+        for hook in _on_host_load:
+            hook(module)
+        self.__dict__.update({k: v for k, v in vars(module).items() if not k.startswith("_")})
+        return self.__dict__[name]
 
 
-def silu_table(dev):
-    """The 11 KiB silu_bf16 table of `dev` (built once per device by the library, owned here: the C ABI keeps no state)."""
-    t = _SILU_TABLES.get(dev)
-    if t is None:
-        t = torch.empty(lib().qt_silu_table_bytes() // 2, dtype=torch.bfloat16, device=dev)
-        call("qt_silu_table_build", ptr(t), stream())
-        _SILU_TABLES[dev] = t
-    return t
+host = _Host()
+_on_host_load = []
 
 
-_ROPE_TABLES = {}        # device -> float32 [positions, 32, 2]
-_ROPE_RETIRED = []       # outgrown tables stay alive: a captured HIP graph may hold their address
-
-
-def rope_table(dev, n_pos):
-    """The (cos, sin) pairs of the rotary embedding for positions 0 .. n_pos - 1 on `dev` (built by the library, owned here;
-    grown in steps of 16384 positions).  Returns (tensor, positions it covers)."""
-    t = _ROPE_TABLES.get(dev)
-    if t is None or t.shape[0] < n_pos:
-        if t is not None:
-            _ROPE_RETIRED.append(t)
-        n = -(-max(n_pos, 1) // 16384) * 16384
-        t = torch.empty((n, 32, 2), dtype=torch.float32, device=dev)
-        call("qt_rope_table_build", ptr(t), n, stream())
-        _ROPE_TABLES[dev] = t
-    return t, t.shape[0]
+def on_host_load(hook):
+    """hook(module) is called once the host module is loaded."""
+    _on_host_load.append(hook)
 
 
 def stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
-_WORKSPACES = {}         # (purpose, device index, stream handle) -> uint8 tensor
-_RETIRED = []            # outgrown buffers: kept for the life of the process, a captured HIP graph may still hold their address
-
-
-def workspace(purpose, dev, nbytes, first_bytes=0):
-    """Scratch memory for a kernel's partial results (the C ABI never allocates): one uint8 buffer per (purpose, device, stream),
-    because launches on different streams may overlap.  A buffer that is outgrown is replaced but never freed: a HIP graph
-    captured earlier replays with the old address.  first_bytes: size of the first allocation, so that growth is rare."""
-    key = (purpose, dev.index if dev.index is not None else torch.cuda.current_device(), torch.cuda.current_stream(dev).cuda_stream)
-    buf = _WORKSPACES.get(key)
-    if buf is None or buf.numel() < nbytes:
-        if buf is not None:
-            _RETIRED.append(buf)
-        buf = torch.empty(max(nbytes, first_bytes), dtype=torch.uint8, device=dev)
-        _WORKSPACES[key] = buf
-    return buf
 
 
 def ptr(t):

@@ -4,7 +4,6 @@ from __future__ import annotations
 import torch
 
 from . import _lib as L
-from .kernels import flat_conv_w
 from .model import Cfg
 
 BF16 = torch.bfloat16
@@ -15,19 +14,7 @@ def deltanet_bm(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, sslots, sels,
     """proj [B*M, 8224] bf16 (row b*M+j = token j of sequence b); sslots / sels / pars int32 [B]: the sequence's entry in the
     snapshot pools, the snapshot it starts from, and the conv buffer it reads.  Returns y [B*M, 2048] bf16; writes snapshots
     0..M-1 of ssm_pool[sslot] and conv buffer par^1 IN PLACE (qwen35/batch_spec.py:142-150)."""
-    sslots = L.i32(sslots, "sslots")
-    B = sslots.shape[0]
-    proj = L.dev(proj, BF16, "proj", (B * M, PW))
-    ssm_pool = L.dev(ssm_pool, torch.float32, "ssm_pool", (None, M, HV, DV, DK))
-    n_entries = ssm_pool.shape[0]
-    conv_pool = L.dev(conv_pool, BF16, "conv_pool", (n_entries * 2, M, 3, CD))
-    sels, pars = L.i32(sels, "sels", B), L.i32(pars, "pars", B)
-    w = flat_conv_w(conv_w)
-    A, dtb = L.f32(A_log, "A_log", (HV,)), L.f32(dt_bias, "dt_bias", (HV,))
-    y = torch.empty((B * M, HV * DV), dtype=BF16, device=proj.device)
-    L.call("qt_gdn_verify_step", L.ptr(proj), L.ptr(conv_pool), L.ptr(w), L.ptr(A), L.ptr(dtb), L.ptr(ssm_pool), L.ptr(sslots),
-           L.ptr(sels), L.ptr(pars), L.ptr(y), B, M, n_entries, rows_per_wg, L.stream())
-    return y
+    return L.host.verify_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, sslots, sels, pars, M, rows_per_wg)
 
 
 class SpecPools:

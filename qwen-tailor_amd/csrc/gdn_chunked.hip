@@ -140,7 +140,7 @@ struct ChainLds {
 // wavefronts share their SIMDs with output wavefronts and have 168 registers each)
 template <bool PUBLISH, int PB_DEP>
 __device__ __forceinline__ void chain_role(ChainLds& L, int blk, const _Float16* ops, const _Float16* U, const float* gates,
-                                           const float* st_in, float* st_out, _Float16* snaps, int* flags, int NC) {
+                                           const float* st_in, float* st_out, _Float16* snaps, int* flags, int* host_words, int NC) {
     // heads that share an XCD's L2 keep their 8 slices there: workgroup id = xcd + 8 k, head = xcd + 8 (k / 8), slice = k % 8
     const int xcd = blk & 7, kq = blk >> 3;
     const int h = xcd + 8 * (kq >> 3), sl = kq & 7;
@@ -345,7 +345,10 @@ __device__ __forceinline__ void chain_role(ChainLds& L, int blk, const _Float16*
         bool bad = false;
 #pragma unroll
         for (int i = 0; i < 4; i++) bad |= !(fabsf(ST[0][i]) <= 3.0e38f) | !(fabsf(ST[1][i]) <= 3.0e38f);
-        if (__any(bad) && lane == 0) atomicOr(flags + FLAG_ERR, ERR_NOT_FINITE);
+        if (__any(bad) && lane == 0) {
+            atomicOr(flags + FLAG_ERR, ERR_NOT_FINITE);
+            if (host_words) host_words[1] = 1;
+        }
     }
 }
 
@@ -424,7 +427,7 @@ __device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c,
 // With WAIT the item's snapshots come from a chain that runs in the same launch: `seq` counts the items of this workgroup.
 template <bool NORM, bool WAIT>
 __device__ __forceinline__ void output_item(bf16_t* ys, volatile int* ready, int seq, int spin_limit, int c, int h, const _Float16* __restrict__ ops,
-                                            const _Float16* snaps, int* flags, const float* __restrict__ gates,
+                                            const _Float16* snaps, int* flags, int* host_words, const float* __restrict__ gates,
                                             bf16_t* __restrict__ y, const bf16_t* __restrict__ proj, const float* __restrict__ gw,
                                             float eps, int S) {
     const int tid = threadIdx.x & 255, w = tid >> 6, lane = tid & 63, n = lane & 15, g = lane >> 4;
@@ -463,7 +466,10 @@ __device__ __forceinline__ void output_item(bf16_t* ys, volatile int* ready, int
                     __builtin_amdgcn_s_sleep(32);
                 }
                 if (lane == 0) {
-                    if (gave_up) atomicOr(flags + FLAG_ERR, ERR_GAVE_UP);
+                    if (gave_up) {
+                        atomicOr(flags + FLAG_ERR, ERR_GAVE_UP);
+                        if (host_words) host_words[0] = 1;
+                    }
                     *ready = 2 * (seq + 1) + (gave_up ? 1 : 0);
                 }
                 if (gave_up) return;                                            // (all four wavefronts leave here: no barrier is skipped by some only)
@@ -526,9 +532,9 @@ __device__ __forceinline__ void output_item(bf16_t* ys, volatile int* ready, int
 
 // the two-launch form: 128 chain workgroups of 320 threads, then one output workgroup of 256 threads per (chunk, head)
 __global__ __launch_bounds__(384) void gdn_chain_kernel(const _Float16* ops, const _Float16* U, const float* gates, const float* st_in,
-                                                        float* st_out, _Float16* snap, int NC) {
+                                                        float* st_out, _Float16* snap, int* host_words, int NC) {
     __shared__ ChainLds chain_lds;
-    chain_role<false, 4>(chain_lds, blockIdx.x, ops, U, gates, st_in, st_out, snap + FLAG_HALVES, reinterpret_cast<int*>(snap), NC);
+    chain_role<false, 4>(chain_lds, blockIdx.x, ops, U, gates, st_in, st_out, snap + FLAG_HALVES, reinterpret_cast<int*>(snap), host_words, NC);
 }
 template <bool NORM>
 __global__ __launch_bounds__(256) void gdn_output_kernel(const _Float16* __restrict__ ops, const _Float16* __restrict__ snap,
@@ -536,7 +542,7 @@ __global__ __launch_bounds__(256) void gdn_output_kernel(const _Float16* __restr
                                                          const bf16_t* __restrict__ proj, const float* __restrict__ gw, float eps,
                                                          int S, int NC) {
     __shared__ __align__(16) bf16_t ys[C * YS_LD];
-    output_item<NORM, false>(ys, nullptr, 0, 0, blockIdx.x / HV, blockIdx.x % HV, ops, snap + FLAG_HALVES, nullptr, gates, y, proj, gw, eps, S);
+    output_item<NORM, false>(ys, nullptr, 0, 0, blockIdx.x / HV, blockIdx.x % HV, ops, snap + FLAG_HALVES, nullptr, nullptr, gates, y, proj, gw, eps, S);
 }
 
 // the one-launch form: N_CHAIN chain workgroups, then output workgroups (4 wavefronts at work) that take (chunk, head) items
@@ -549,14 +555,14 @@ __global__ __launch_bounds__(256) void gdn_output_kernel(const _Float16* __restr
 template <bool NORM>
 __global__ __launch_bounds__(384, 3) void gdn_phase_b_kernel(const _Float16* ops, const _Float16* U, const float* gates, const float* st_in,
                                                              float* st_out, _Float16* snap, bf16_t* y, const bf16_t* proj,
-                                                             const float* gw, float eps, int S, int NC, int spin_limit) {
+                                                             const float* gw, float eps, int S, int NC, int spin_limit, int* host_words) {
     __shared__ ChainLds chain_lds;
     __shared__ __align__(16) bf16_t ys[C * YS_LD];
     __shared__ int ready, item_s, last;
     int* flags = reinterpret_cast<int*>(snap);
     _Float16* snaps = snap + FLAG_HALVES;
     if (blockIdx.x < N_CHAIN) {
-        chain_role<true, 3>(chain_lds, blockIdx.x, ops, U, gates, st_in, st_out, snaps, flags, NC);
+        chain_role<true, 3>(chain_lds, blockIdx.x, ops, U, gates, st_in, st_out, snaps, flags, host_words, NC);
         return;
     }
     if (threadIdx.x >= 256) return;                                             // (a wavefront that has ended is no party to the barriers)
@@ -567,7 +573,7 @@ __global__ __launch_bounds__(384, 3) void gdn_phase_b_kernel(const _Float16* ops
         __syncthreads();
         const int item = item_s;
         if (item >= total) break;
-        output_item<NORM, true>(ys, &ready, seq, spin_limit, item / HV, item % HV, ops, snaps, flags, gates, y, proj, gw, eps, S);
+        output_item<NORM, true>(ys, &ready, seq, spin_limit, item / HV, item % HV, ops, snaps, flags, host_words, gates, y, proj, gw, eps, S);
     }
     // a workgroup counts itself done when it has taken its last item; the last workgroup of the launch (of either role)
     // leaves the flag area zero for the next launch
@@ -1062,7 +1068,8 @@ long qt_gdn_chunk_gc_bytes(int S) { return S < 0 ? -1 : (long)((S + C - 1) / C) 
 static std::atomic<int> poll_limit{0};
 
 static int phase_b_launch(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out,
-                          void* y, const void* proj, const float* gw, float eps, bool norm, int S, hipStream_t stream) {
+                          void* y, const void* proj, const float* gw, float eps, bool norm, int S, int32_t* host_words,
+                          hipStream_t stream) {
     if (!ops || !U || !gC || !snap || !state_in || !state_out || !y) return QT_ERR_NULL;
     if (norm && (!proj || !gw)) return QT_ERR_NULL;
     if (S < 0) return QT_ERR_DIM;
@@ -1080,13 +1087,13 @@ static int phase_b_launch(const void* ops, const void* U, const float* gC, void*
         const int pl = poll_limit.load(std::memory_order_relaxed), spin = pl > 0 ? pl : SPIN_LIMIT;
         if (norm)
             hipLaunchKernelGGL(gdn_phase_b_kernel<true>, grid, block, 0, stream, (const _Float16*)ops, (const _Float16*)U, gC, state_in,
-                               state_out, (_Float16*)snap, (bf16_t*)y, (const bf16_t*)proj, gw, eps, S, NC, spin);
+                               state_out, (_Float16*)snap, (bf16_t*)y, (const bf16_t*)proj, gw, eps, S, NC, spin, (int*)host_words);
         else
             hipLaunchKernelGGL(gdn_phase_b_kernel<false>, grid, block, 0, stream, (const _Float16*)ops, (const _Float16*)U, gC, state_in,
-                               state_out, (_Float16*)snap, (bf16_t*)y, (const bf16_t*)nullptr, (const float*)nullptr, 0.f, S, NC, spin);
+                               state_out, (_Float16*)snap, (bf16_t*)y, (const bf16_t*)nullptr, (const float*)nullptr, 0.f, S, NC, spin, (int*)host_words);
     } else {
         hipLaunchKernelGGL(gdn_chain_kernel, dim3(N_CHAIN), dim3(384), 0, stream, (const _Float16*)ops, (const _Float16*)U, gC, state_in,
-                           state_out, (_Float16*)snap, NC);
+                           state_out, (_Float16*)snap, (int*)host_words, NC);
         QT_CHECK_LAUNCH();
         if (norm)
             hipLaunchKernelGGL(gdn_output_kernel<true>, dim3(NC * HV), dim3(256), 0, stream, (const _Float16*)ops, (const _Float16*)snap,
@@ -1110,12 +1117,21 @@ long qt_gdn_chunk_snap_bytes(int S) { return S < 0 ? -1 : (long)FLAG_WORDS * 4 +
 
 int qt_gdn_phase_b(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out, void* y,
                    int S, hipStream_t stream) {
-    return phase_b_launch(ops, U, gC, snap, state_in, state_out, y, nullptr, nullptr, 0.f, false, S, stream);
+    return phase_b_launch(ops, U, gC, snap, state_in, state_out, y, nullptr, nullptr, 0.f, false, S, nullptr, stream);
 }
 
 int qt_gdn_phase_b_norm(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out,
                         const void* proj, const float* gw, float eps, void* out, int S, hipStream_t stream) {
-    return phase_b_launch(ops, U, gC, snap, state_in, state_out, out, proj, gw, eps, true, S, stream);
+    return phase_b_launch(ops, U, gC, snap, state_in, state_out, out, proj, gw, eps, true, S, nullptr, stream);
+}
+
+// qt_gdn_phase_b (proj and gw null) or qt_gdn_phase_b_norm with a report to the host: host_words[0] / [1] (pinned host memory the GPU can
+// write) are set to 1 where bit 0 / bit 1 of the status word is set.  Nothing is written there in the ordinary case, and the
+// caller needs no copy of the status word behind every launch (2 - 5 us on the stream and 8 us of host time per prefill).
+int qt_gdn_phase_b_report(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out,
+                          const void* proj, const float* gw, float eps, void* out, int S, int32_t* host_words, hipStream_t stream) {
+    if (!host_words) return QT_ERR_NULL;
+    return phase_b_launch(ops, U, gC, snap, state_in, state_out, out, proj, gw, eps, proj != nullptr || gw != nullptr, S, host_words, stream);
 }
 
 int qt_gdn_phase_a(const void* proj, const void* q, const void* k, const void* v, const float* A_log, const float* dt_bias,

@@ -1,0 +1,710 @@
+// The host side of the operators as a Python extension module: argument checks, output allocation and the C-ABI call of each hot
+// operator in one native call.  At decode sizes a launch takes the GPU 2 - 7 us, and the same steps in Python (a dozen tensor
+// checks, torch.empty, the current stream, a ctypes call) took 10 - 22 us, so that a program that launches eagerly waited for
+// its host; here they take 3 - 5 us.
+//
+// Every function takes its arguments by position (the Python modules of the package hold the signatures and their defaults) and
+// raises what the checks of _lib.py raise: TypeError for something that is not a GPU tensor of the expected type, ValueError for
+// a wrong shape or layout, RuntimeError for an error code of the C ABI.  The module keeps scratch buffers and tables per device
+// (and stream); they are touched with the GIL held only.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/empty.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <climits>
+#include <map>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include "../../include/qwen_tailor_hip.h"
+
+namespace {
+
+using at::Tensor;
+using at::ScalarType;
+
+constexpr ScalarType BF16 = at::kBFloat16, F32 = at::kFloat, I32 = at::kInt, F16 = at::kHalf, U8 = at::kByte;
+constexpr int64_t HV = 16, DK = 128, DV = 128, CD = 6144, PW = 8224, QKV_W = 5120, ANY = -1;
+
+struct Error {                              // a Python exception to be raised
+    PyObject* type;
+    std::string text;
+};
+struct Raised {};                           // ... that is already set
+[[noreturn]] void type_error(const std::string& s) { throw Error{PyExc_TypeError, s}; }
+[[noreturn]] void value_error(const std::string& s) { throw Error{PyExc_ValueError, s}; }
+
+template <typename V>
+std::string shape_text(const V& v) {        // as Python prints a tuple (None for a free entry)
+    std::string r = "(";
+    for (size_t i = 0; i < v.size(); i++) r += (i ? ", " : "") + (v[i] == ANY ? std::string("None") : std::to_string(v[i]));
+    return r + (v.size() == 1 ? ",)" : ")");
+}
+const char* dtype_text(ScalarType t) {
+    switch (t) {
+        case BF16: return "torch.bfloat16";
+        case F32: return "torch.float32";
+        case I32: return "torch.int32";
+        case F16: return "torch.float16";
+        case U8: return "torch.uint8";
+        case at::kDouble: return "torch.float64";
+        case at::kLong: return "torch.int64";
+        default: return at::toString(t);
+    }
+}
+
+const Tensor& gpu_tensor(PyObject* o, const char* name) {
+    if (!THPVariable_Check(o) || !THPVariable_Unpack(o).is_cuda()) type_error(std::string(name) + ": expected a tensor on the GPU");
+    return THPVariable_Unpack(o);
+}
+void check_shape(const Tensor& t, const char* name, std::initializer_list<int64_t> shape) {
+    const auto have = t.sizes();
+    bool ok = have.size() == shape.size();
+    size_t i = 0;
+    for (int64_t s : shape) ok = ok && (s == ANY || have[i] == s), i++;
+    if (!ok) value_error(std::string(name) + ": expected shape " + shape_text(std::vector<int64_t>(shape)) + ", got " + shape_text(have.vec()));
+}
+void check_layout(const Tensor& t, ScalarType dtype, const char* name) {
+    if (t.scalar_type() != dtype)
+        type_error(std::string(name) + ": expected " + dtype_text(dtype) + ", got " + dtype_text(t.scalar_type()));
+    if (!t.is_contiguous()) value_error(std::string(name) + ": must be contiguous");
+}
+// a contiguous GPU tensor of `dtype` (and of `shape`, where given; ANY entries are free)
+const Tensor& dev(PyObject* o, ScalarType dtype, const char* name) {
+    const Tensor& t = gpu_tensor(o, name);
+    check_layout(t, dtype, name);
+    return t;
+}
+const Tensor& dev(PyObject* o, ScalarType dtype, const char* name, std::initializer_list<int64_t> shape) {
+    const Tensor& t = dev(o, dtype, name);
+    check_shape(t, name, shape);
+    return t;
+}
+// per-head parameter vectors are consumed as float32: anything else is converted
+Tensor f32(PyObject* o, const char* name, int64_t n) {
+    Tensor t = gpu_tensor(o, name);
+    if (t.scalar_type() != F32 || !t.is_contiguous()) t = t.to(F32).contiguous();
+    check_shape(t, name, {n});
+    return t;
+}
+const Tensor& flat_conv_w(PyObject* o) {
+    const Tensor& w = dev(o, BF16, "conv_w");
+    if (w.numel() != CD * 4) value_error("conv_w: expected " + std::to_string(CD * 4) + " elements, got " + std::to_string(w.numel()));
+    return w;
+}
+
+long integer(PyObject* o) {                 // int(o)
+    long v = PyLong_AsLong(o);
+    if (v == -1 && PyErr_Occurred()) {
+        PyErr_Clear();
+        PyObject* i = PyNumber_Long(o);
+        if (!i) throw Raised{};
+        v = PyLong_AsLong(i);
+        Py_DECREF(i);
+        if (v == -1 && PyErr_Occurred()) throw Raised{};
+    }
+    return v;
+}
+float real(PyObject* o) {                   // float(o)
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) throw Raised{};
+    return (float)v;
+}
+bool truth(PyObject* o) {
+    const int v = PyObject_IsTrue(o);
+    if (v < 0) throw Raised{};
+    return v != 0;
+}
+
+Tensor empty(at::IntArrayRef size, ScalarType dtype, const Tensor& like) {
+    return Tensor(at::detail::empty_cuda(size, dtype, like.device(), std::nullopt));
+}
+void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+const char* code_text(int rc) {
+    switch (rc) {
+        case -1: return "bad dimension";
+        case -2: return "misaligned pointer";
+        case -3: return "null pointer";
+        case -4: return "unsupported shape";
+        case -5: return "kernel launch failed";
+        case -6: return "workspace too small";
+        case -7: return "size beyond the maximum of the allocation-free entry point";
+        default: return "unknown error";
+    }
+}
+void check(int rc, const char* name) {
+    if (rc) throw Error{PyExc_RuntimeError, std::string(name) + " failed: " + code_text(rc)};
+}
+int dim32(int64_t v) { return v > INT_MAX ? INT_MAX : (int)v; }
+
+PyObject* wrap(const Tensor& t) { return THPVariable_Wrap(t); }
+PyObject* wrap(std::initializer_list<Tensor> ts) {
+    PyObject* r = PyTuple_New(ts.size());
+    Py_ssize_t i = 0;
+    for (const Tensor& t : ts) PyTuple_SET_ITEM(r, i++, THPVariable_Wrap(t));
+    return r;
+}
+
+// ---- buffers that outlive a call ----------------------------------------------------------------------------------------
+// Never destroyed: at interpreter exit the allocator that owns their memory may be gone already.  A buffer that is outgrown is
+// kept: a HIP graph captured earlier replays with its address.
+std::vector<Tensor>& retired() {
+    static auto* v = new std::vector<Tensor>;
+    return *v;
+}
+// Scratch memory for a kernel's partial results (the C ABI never allocates): one buffer per (purpose, device, stream), because
+// launches on different streams may overlap.  `first`: size of the first allocation, so that growth is rare.
+enum Purpose { ATTN_B, PREFILL_ATTENTION };
+const Tensor& workspace(int purpose, const Tensor& like, long bytes, long first) {
+    static auto* m = new std::map<std::tuple<int, int, void*>, Tensor>;
+    Tensor& buf = (*m)[{purpose, (int)like.device().index(), stream()}];
+    if (!buf.defined() || buf.numel() < bytes) {
+        if (buf.defined()) retired().push_back(buf);
+        buf = empty({std::max(bytes, first)}, U8, like);
+    }
+    return buf;
+}
+constexpr long WS_FIRST = 32 << 20;         // attn_b: enough for 256 sequences x 4 rows
+
+const Tensor& silu_table(const Tensor& like) {
+    static auto* m = new std::map<int, Tensor>;
+    Tensor& t = (*m)[(int)like.device().index()];
+    if (!t.defined()) {
+        Tensor n = empty({qt_silu_table_bytes() / 2}, BF16, like);
+        check(qt_silu_table_build(n.data_ptr(), stream()), "qt_silu_table_build");
+        t = n;
+    }
+    return t;
+}
+// the (cos, sin) pairs of the rotary embedding for positions 0 .. n_pos - 1; grown in steps of 16384 positions
+const Tensor& rope_table(const Tensor& like, int64_t n_pos) {
+    static auto* m = new std::map<int, Tensor>;
+    Tensor& t = (*m)[(int)like.device().index()];
+    if (!t.defined() || t.size(0) < n_pos) {
+        const int64_t n = (std::max<int64_t>(n_pos, 1) + 16383) / 16384 * 16384;
+        Tensor grown = empty({n, 32, 2}, F32, like);
+        check(qt_rope_table_build(grown.data_ptr(), dim32(n), stream()), "qt_rope_table_build");
+        if (t.defined()) retired().push_back(t);
+        t = grown;
+    }
+    return t;
+}
+
+// ---- projections ----------------------------------------------------------------------------------------------------------
+Tensor do_rms_rows(const Tensor& x, const Tensor& nw, float eps) {
+    Tensor y = empty(x.sizes(), BF16, x);
+    check(qt_rms_rows(x.data_ptr(), nw.data_ptr(), y.data_ptr(), dim32(x.size(0)), dim32(x.size(1)), eps, stream()), "qt_rms_rows");
+    return y;
+}
+Tensor do_gated_norm(const Tensor& y, const Tensor& proj, const Tensor& gw, float eps) {
+    Tensor out = empty({y.size(0), HV * DV}, BF16, y);
+    check(qt_gated_rmsnorm(y.data_ptr(), proj.data_ptr(), gw.data_ptr<float>(), out.data_ptr(), y.size(0), eps, stream()), "qt_gated_rmsnorm");
+    return out;
+}
+
+// rms_rows(x, nw, eps, f32)
+PyObject* rms_rows(PyObject* const* a) {
+    const Tensor& x = dev(a[0], BF16, "x", {ANY, ANY});
+    Tensor y = do_rms_rows(x, dev(a[1], BF16, "nw", {x.size(1)}), real(a[2]));
+    return wrap(truth(a[3]) ? y.to(F32) : y);
+}
+
+// fused_gemv(W, x, nw, eps, res, swiglu, gnorm)
+PyObject* fused_gemv(PyObject* const* a) {
+    if (PyTuple_Check(a[0]) || PyList_Check(a[0])) type_error("W: compressed weight pairs are not supported, pass the plain bf16 [N, K] matrix");
+    const Tensor& W = dev(a[0], BF16, "W", {ANY, ANY});
+    const int64_t N = W.size(0), K = W.size(1);
+    const Tensor& xin = gpu_tensor(a[1], "x");
+    if (xin.dim() < 1 || xin.size(-1) != K) value_error("x: last dimension must be " + std::to_string(K) + ", got " + shape_text(xin.sizes().vec()));
+    const bool has_nw = a[2] != Py_None, has_res = a[4] != Py_None, swiglu = truth(a[5]), has_gnorm = a[6] != Py_None;
+    Tensor x = xin;
+    if (x.scalar_type() == F32) {
+        if (has_nw || has_gnorm) value_error("float32 x carries already normalised values: no prologue may follow");
+        x = x.to(BF16);                                          // exact: the values are bf16 values
+    }
+    if (x.dim() != 2) x = x.reshape({-1, K});
+    if (!x.is_contiguous() && xin.dim() != 2) x = x.contiguous();
+    check_layout(x, BF16, "x");
+    const int64_t M = x.size(0);
+    if (has_nw && has_gnorm) value_error("nw and gnorm are exclusive");
+    if (swiglu && has_res) value_error("swiglu and res are exclusive");
+    const float eps = real(a[3]);
+    if (has_gnorm) {
+        PyObject* pair = PySequence_Fast(a[6], "gnorm: expected (proj, gw)");
+        if (!pair) throw Raised{};
+        PyObject *pp = PySequence_Fast_GET_ITEM(pair, 0), *pg = PySequence_Fast_GET_ITEM(pair, 1);
+        Py_DECREF(pair);                                         // (a[6] keeps its items)
+        check_shape(x, "y", {ANY, HV * DV});
+        const Tensor proj = gpu_tensor(pp, "proj").reshape({M, PW});
+        check_layout(proj, BF16, "proj");
+        x = do_gated_norm(x, proj, f32(pg, "gw", DV), eps);
+    }
+    const int epi = swiglu ? 2 : has_res ? 1 : 0;
+    const int64_t n_out = swiglu ? N / 2 : N;
+    Tensor res;
+    if (has_res) {
+        res = gpu_tensor(a[4], "res");
+        if (res.dim() != 2) res = res.reshape({-1, N});
+        check_layout(res, BF16, "res");
+        check_shape(res, "res", {M, N});
+    }
+    std::vector<int64_t> shape = xin.sizes().vec();
+    shape.back() = n_out;
+    Tensor y = empty(shape, BF16, x);
+    const void* rp = has_res ? res.data_ptr() : nullptr;
+    if (has_nw) {
+        const Tensor& nw = dev(a[2], BF16, "nw", {K});
+        // one launch for the shapes that have it, otherwise the prologue as its own kernel
+        const int rc = qt_fused_gemv_rms(W.data_ptr(), x.data_ptr(), nw.data_ptr(), eps, rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream());
+        if (rc == 0) return wrap(y);
+        if (rc != -4) check(rc, "qt_fused_gemv_rms");
+        x = do_rms_rows(x, nw, eps);
+    }
+    check(qt_fused_gemv(W.data_ptr(), x.data_ptr(), rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream()), "qt_fused_gemv");
+    return wrap(y);
+}
+
+// gated_norm(y [rows, 2048], proj, gw, eps)
+PyObject* gated_norm(PyObject* const* a) {
+    const Tensor& y = dev(a[0], BF16, "y", {ANY, HV * DV});
+    return wrap(do_gated_norm(y, dev(a[1], BF16, "proj", {y.size(0), PW}), f32(a[2], "gw", DV), real(a[3])));
+}
+
+// ---- recurrent steps ------------------------------------------------------------------------------------------------------
+// decode_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, gw or None, eps, rows_per_wg)
+PyObject* decode_step(PyObject* const* a) {
+    const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
+    const int64_t B = proj.size(0);
+    const Tensor& ssm = dev(a[5], F32, "ssm_pool", {ANY, HV, DV, DK});
+    const int64_t n_slots = ssm.size(0);
+    const Tensor& conv = dev(a[1], BF16, "conv_pool", {n_slots * 2, 3, CD});
+    const Tensor &slots = dev(a[6], I32, "slots", {B}), &pos = dev(a[7], I32, "pos", {B}), &w = flat_conv_w(a[2]);
+    const Tensor A = f32(a[3], "A_log", HV), dtb = f32(a[4], "dt_bias", HV);
+    const bool norm = a[8] != Py_None;
+    const Tensor gw = norm ? f32(a[8], "gw", DV) : Tensor();
+    Tensor out = empty({B, HV * DV}, BF16, proj);
+    if (norm)
+        check(qt_gdn_decode_step_gnorm(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
+                                       slots.data_ptr<int>(), pos.data_ptr<int>(), gw.data_ptr<float>(), real(a[9]), out.data_ptr(), dim32(B),
+                                       dim32(n_slots), stream()), "qt_gdn_decode_step_gnorm");
+    else
+        check(qt_gdn_decode_step(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
+                                 slots.data_ptr<int>(), pos.data_ptr<int>(), out.data_ptr(), dim32(B), dim32(n_slots), (int)integer(a[10]), stream()),
+              "qt_gdn_decode_step");
+    return wrap(out);
+}
+
+// verify_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, sslots, sels, pars, M, rows_per_wg)
+PyObject* verify_step(PyObject* const* a) {
+    const Tensor& ss = dev(a[6], I32, "sslots");
+    if (ss.dim() < 1) value_error("sslots: expected one entry per sequence");
+    const int64_t B = ss.size(0), M = integer(a[9]);
+    const Tensor& proj = dev(a[0], BF16, "proj", {B * M, PW});
+    const Tensor& ssm = dev(a[5], F32, "ssm_pool", {ANY, M, HV, DV, DK});
+    const int64_t n = ssm.size(0);
+    const Tensor& conv = dev(a[1], BF16, "conv_pool", {n * 2, M, 3, CD});
+    const Tensor &sels = dev(a[7], I32, "sels", {B}), &pars = dev(a[8], I32, "pars", {B}), &w = flat_conv_w(a[2]);
+    const Tensor A = f32(a[3], "A_log", HV), dtb = f32(a[4], "dt_bias", HV);
+    Tensor y = empty({B * M, HV * DV}, BF16, proj);
+    check(qt_gdn_verify_step(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
+                             ss.data_ptr<int>(), sels.data_ptr<int>(), pars.data_ptr<int>(), y.data_ptr(), dim32(B), dim32(M), dim32(n),
+                             (int)integer(a[10]), stream()), "qt_gdn_verify_step");
+    return wrap(y);
+}
+
+// deltanet(proj, conv_snap, conv_w, A_log, dt_bias, ssm_snap, sel, rows_per_wg)
+PyObject* deltanet(PyObject* const* a) {
+    const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
+    const int64_t M = proj.size(0);
+    const Tensor &conv = dev(a[1], BF16, "conv_snap", {ANY, 3, CD}), &ssm = dev(a[5], F32, "ssm_snap", {ANY, HV, DV, DK});
+    const int64_t S = ssm.size(0);
+    if (conv.size(0) != S) value_error("conv_snap and ssm_snap must hold the same number of snapshots");
+    const Tensor &sel = dev(a[6], I32, "sel", {1}), &w = flat_conv_w(a[2]);
+    const Tensor A = f32(a[3], "A_log", HV), dtb = f32(a[4], "dt_bias", HV);
+    Tensor y = empty({M, HV * DV}, BF16, proj), cs = empty({M, 3, CD}, BF16, proj), st = empty({M, HV, DV, DK}, F32, proj);
+    check(qt_gdn_deltanet(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
+                          sel.data_ptr<int>(), y.data_ptr(), cs.data_ptr(), st.data_ptr<float>(), dim32(M), dim32(S), (int)integer(a[7]), stream()),
+          "qt_gdn_deltanet");
+    return wrap({y, cs, st});
+}
+
+// ---- decode / verify attention --------------------------------------------------------------------------------------------
+struct Pool {
+    const Tensor &K, &V, &slots, &pos;
+    int64_t n_slots, Lmax;
+};
+Pool kv_pool(PyObject* kp, PyObject* vp, PyObject* slots, PyObject* pos, int64_t B) {
+    const Tensor& K = dev(kp, BF16, "Kp", {ANY, 2, ANY, 256});
+    const Tensor& V = dev(vp, BF16, "Vp", {K.size(0), K.size(1), K.size(2), K.size(3)});
+    return {K, V, dev(slots, I32, "slots", {B}), dev(pos, I32, "pos", {B}), K.size(0), K.size(2)};
+}
+Tensor attn_scratch(PyObject* given, const Tensor& like, int64_t B, int64_t M, int64_t Lmax, long CH, const char* who) {
+    const long bytes = qt_gqa_attn_workspace_bytes(dim32(B), dim32(M), dim32(Lmax), (int)CH);
+    if (bytes < 0) value_error(std::string(who) + ": bad split size");
+    if (given == Py_None) return workspace(ATTN_B, like, bytes, WS_FIRST);
+    const Tensor& ws = dev(given, U8, "workspace");
+    if (ws.numel() < bytes)
+        value_error(std::string(who) + ": workspace of " + std::to_string(ws.numel()) + " bytes, " + std::to_string(bytes) + " needed");
+    return ws;
+}
+int64_t sequences(int64_t R, int64_t M, const char* who, const char* limit) {
+    if (M < 1 || M > 16 || R % M)
+        value_error(std::string(who) + ": M = " + std::to_string(M) + " (" + limit + ") must divide the number of rows (" + std::to_string(R) + ")");
+    return R / M;
+}
+
+// attn_b(q, k, v, Kp, Vp, slots, pos, M, split, workspace or None)
+PyObject* attn_b(PyObject* const* a) {
+    const Tensor& q = dev(a[0], BF16, "q", {ANY, 8, 256});
+    const int64_t R = q.size(0), M = integer(a[7]), B = sequences(R, M, "attn_b", "1..16, as deltanet_bm");
+    const Tensor &k = dev(a[1], BF16, "k", {R, 2, 256}), &v = dev(a[2], BF16, "v", {R, 2, 256});
+    const Pool p = kv_pool(a[3], a[4], a[5], a[6], B);
+    const long CH = integer(a[8]);
+    const Tensor ws = attn_scratch(a[9], q, B, M, p.Lmax, CH, "attn_b");
+    Tensor o = empty({R, 8, 256}, BF16, q);
+    check(qt_gqa_attn_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), p.K.data_ptr(), p.V.data_ptr(), p.slots.data_ptr<int>(), p.pos.data_ptr<int>(),
+                             o.data_ptr(), ws.data_ptr(), ws.numel(), dim32(B), dim32(M), dim32(p.Lmax), dim32(p.n_slots), (int)CH, stream()),
+          "qt_gqa_attn_decode");
+    return wrap(o);
+}
+
+// attn_layer_b(qkv, q_norm, k_norm, Kp, Vp, slots, pos, M, eps, split, workspace or None)
+PyObject* attn_layer_b(PyObject* const* a) {
+    const Tensor& qkv = dev(a[0], BF16, "qkv", {ANY, QKV_W});
+    const int64_t R = qkv.size(0), M = integer(a[7]), B = sequences(R, M, "attn_layer_b", "1..16");
+    const Tensor &qn = dev(a[1], BF16, "q_norm", {256}), &kn = dev(a[2], BF16, "k_norm", {256});
+    const Pool p = kv_pool(a[3], a[4], a[5], a[6], B);
+    const long CH = integer(a[9]);
+    const Tensor ws = attn_scratch(a[10], qkv, B, M, p.Lmax, CH, "attn_layer_b");
+    const Tensor& table = rope_table(qkv, p.Lmax);
+    Tensor out = empty({R, 2048}, BF16, qkv);
+    check(qt_gqa_attn_layer_decode(qkv.data_ptr(), qn.data_ptr(), kn.data_ptr(), table.data_ptr(), dim32(table.size(0)), p.K.data_ptr(), p.V.data_ptr(),
+                                   p.slots.data_ptr<int>(), p.pos.data_ptr<int>(), out.data_ptr(), ws.data_ptr(), ws.numel(), dim32(B), dim32(M),
+                                   dim32(p.Lmax), dim32(p.n_slots), (int)CH, real(a[8]), stream()), "qt_gqa_attn_layer_decode");
+    return wrap(out);
+}
+
+// ---- prefill attention ----------------------------------------------------------------------------------------------------
+// sdpa(q, k, v): the checks that need no arithmetic on floats; causal, scale 256^-0.5
+PyObject* sdpa(PyObject* const* a) {
+    const auto& qin = THPVariable_Check(a[0]) ? THPVariable_Unpack(a[0]) : Tensor();
+    if (!qin.defined() || qin.dim() != 4 || qin.size(0) != 1 || qin.size(1) != 8 || qin.size(3) != 256 || qin.scalar_type() != BF16 || !qin.is_cuda())
+        value_error("q: expected [1, 8, S, 256] bf16 on the GPU" + (qin.defined() ? ", got " + shape_text(qin.sizes().vec()) + " " + dtype_text(qin.scalar_type()) : std::string()));
+    Tensor q = qin;
+    const int64_t S = q.size(2);
+    for (int i = 1; i < 3; i++) {
+        const std::string name = i == 1 ? "k" : "v";
+        if (!THPVariable_Check(a[i])) value_error(name + ": expected [1, 2, L, 256] bf16 on the GPU");
+        const Tensor& t = THPVariable_Unpack(a[i]);
+        if (t.dim() != 4 || t.size(0) != 1 || t.size(1) != 2 || t.size(3) != 256 || t.scalar_type() != BF16 || !t.is_cuda())
+            value_error(name + ": expected [1, 2, L, 256] bf16 on the GPU");
+        if (t.stride(3) != 1 || t.stride(2) != 256) value_error(name + ": rows must be contiguous");
+    }
+    const Tensor &k = THPVariable_Unpack(a[1]), &v = THPVariable_Unpack(a[2]);
+    if (k.sizes() != v.sizes() || k.stride(1) != v.stride(1)) value_error("k and v must have the same shape and head stride");
+    const int64_t L = k.size(2);
+    if (L < S) value_error("fewer keys than queries");
+    Tensor out;
+    long head_stride = S * 256;
+    int row_stride = 256;
+    if (S > 1 && q.stride(1) == 256 && q.stride(2) == 2048 && q.stride(3) == 1 && !((uintptr_t)q.data_ptr() & 15)) {
+        out = empty({1, S, 8, 256}, BF16, q).transpose(1, 2);    // a transposed view of token-major rows: neither side is copied
+        head_stride = 256, row_stride = 2048;
+    } else {
+        q = q.contiguous();
+        out = empty(q.sizes(), BF16, q);
+    }
+    // launches that would leave half of the CUs idle are split along the keys; their parts meet in a workspace
+    const long bytes = qt_gqa_prefill_workspace_bytes_for(dim32(S), dim32(L), dim32(L - S));
+    void* ws = bytes > 0 ? workspace(PREFILL_ATTENTION, q, bytes, 0).data_ptr() : nullptr;
+    check(qt_gqa_prefill_causal_strided(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), ws, bytes > 0 ? bytes : 0, dim32(S), dim32(L),
+                                        dim32(L - S), head_stride, row_stride, k.stride(1), stream()), "qt_gqa_prefill_causal");
+    return wrap(out);
+}
+
+// qkv_prep(qkv, q_norm, k_norm, pos, M, eps, max_pos or None)
+PyObject* qkv_prep(PyObject* const* a) {
+    const Tensor& qkv = dev(a[0], BF16, "qkv", {ANY, QKV_W});
+    const int64_t R = qkv.size(0), M = integer(a[4]);
+    if (M < 1 || R % M) value_error("qkv_prep: M = " + std::to_string(M) + " must divide the number of rows (" + std::to_string(R) + ")");
+    const Tensor &pos = dev(a[3], I32, "pos", {R / M}), &qn = dev(a[1], BF16, "q_norm", {256}), &kn = dev(a[2], BF16, "k_norm", {256});
+    Tensor q = empty({R, 8, 256}, BF16, qkv), k = empty({R, 2, 256}, BF16, qkv), v = empty({R, 2, 256}, BF16, qkv);
+    const Tensor table = a[6] != Py_None ? rope_table(qkv, integer(a[6]) + 1) : Tensor();
+    check(qt_attn_qkv_prep_table(qkv.data_ptr(), qn.data_ptr(), kn.data_ptr(), pos.data_ptr<int>(), table.defined() ? table.data_ptr() : nullptr,
+                                 table.defined() ? dim32(table.size(0)) : 0, q.data_ptr(), k.data_ptr(), v.data_ptr(), R, dim32(M), real(a[5]), stream()),
+          "qt_attn_qkv_prep");
+    return wrap({q, k, v});
+}
+
+// out_gate(o, qkv)
+PyObject* out_gate(PyObject* const* a) {
+    const Tensor& qkv = dev(a[1], BF16, "qkv", {ANY, QKV_W});
+    const int64_t R = qkv.size(0);
+    const Tensor& o = dev(a[0], BF16, "o", {R, 8, 256});
+    Tensor out = empty({R, 2048}, BF16, qkv);
+    check(qt_attn_out_gate(o.data_ptr(), qkv.data_ptr(), out.data_ptr(), R, stream()), "qt_attn_out_gate");
+    return wrap(out);
+}
+
+// ---- chunked prefill ------------------------------------------------------------------------------------------------------
+// conv_prep(proj, conv_state, conv_w)
+PyObject* conv_prep(PyObject* const* a) {
+    const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
+    const int64_t S = proj.size(0);
+    const Tensor &cs = dev(a[1], BF16, "conv_state", {3, CD}), &w = flat_conv_w(a[2]);
+    Tensor q = empty({S, HV, DK}, BF16, proj), k = empty({S, HV, DK}, BF16, proj), v = empty({S, HV, DK}, BF16, proj);
+    check(qt_gdn_conv_prep(proj.data_ptr(), cs.data_ptr(), w.data_ptr(), silu_table(proj).data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), dim32(S),
+                           stream()), "qt_gdn_conv_prep");
+    return wrap({q, k, v});
+}
+
+struct Records {
+    Tensor ops, U, gC;
+};
+Records new_records(const Tensor& proj) {
+    const int S = dim32(proj.size(0));
+    return {empty({qt_gdn_chunk_ops_bytes(S) / 2}, F16, proj), empty({qt_gdn_chunk_u_bytes(S) / 2}, F16, proj), empty({qt_gdn_chunk_gc_bytes(S) / 4}, F32, proj)};
+}
+void phase_a_conv(const Tensor& proj, const Tensor& cs, const Tensor& w, const Tensor& A, const Tensor& dtb, const Tensor* qkv, void* conv_out,
+                  const Records& r) {
+    check(qt_gdn_phase_a_conv(proj.data_ptr(), cs.data_ptr(), w.data_ptr(), silu_table(proj).data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(),
+                              qkv ? qkv[0].data_ptr() : nullptr, qkv ? qkv[1].data_ptr() : nullptr, qkv ? qkv[2].data_ptr() : nullptr, conv_out,
+                              r.ops.data_ptr(), r.U.data_ptr(), r.gC.data_ptr<float>(), dim32(proj.size(0)), stream()), "qt_gdn_phase_a_conv");
+}
+
+// phase_a(proj, conv_state, conv_w, A_log, dt_bias, (q, k, v) or None, want_qkv, conv_out or None) -> (q, k, v, ops, U, gC)
+PyObject* phase_a(PyObject* const* a) {
+    const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
+    const int64_t S = proj.size(0);
+    const Tensor A = f32(a[3], "A_log", HV), dtb = f32(a[4], "dt_bias", HV);
+    const Records r = new_records(proj);
+    if (a[5] != Py_None) {
+        PyObject* seq = PySequence_Fast(a[5], "qkv: expected (q, k, v)");
+        if (!seq) throw Raised{};
+        static const char* names[3] = {"q", "k", "v"};
+        Tensor t[3];
+        try {
+            if (PySequence_Fast_GET_SIZE(seq) != 3) value_error("qkv: expected (q, k, v)");
+            for (int i = 0; i < 3; i++) t[i] = dev(PySequence_Fast_GET_ITEM(seq, i), BF16, names[i], {S, HV, DK});
+        } catch (...) {
+            Py_DECREF(seq);
+            throw;
+        }
+        Py_DECREF(seq);
+        check(qt_gdn_phase_a(proj.data_ptr(), t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(),
+                             r.ops.data_ptr(), r.U.data_ptr(), r.gC.data_ptr<float>(), dim32(S), stream()), "qt_gdn_phase_a");
+        return wrap({t[0], t[1], t[2], r.ops, r.U, r.gC});
+    }
+    const Tensor &cs = dev(a[1], BF16, "conv_state", {3, CD}), &w = flat_conv_w(a[2]);
+    Tensor qkv[3];
+    const bool want = truth(a[6]);
+    if (want)
+        for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
+    phase_a_conv(proj, cs, w, A, dtb, want ? qkv : nullptr, a[7] != Py_None ? dev(a[7], BF16, "conv_out", {3, CD}).data_ptr() : nullptr, r);
+    PyObject* out = PyTuple_New(6);
+    for (int i = 0; i < 3; i++) PyTuple_SET_ITEM(out, i, want ? wrap(qkv[i]) : (Py_INCREF(Py_None), Py_None));
+    PyTuple_SET_ITEM(out, 3, wrap(r.ops));
+    PyTuple_SET_ITEM(out, 4, wrap(r.U));
+    PyTuple_SET_ITEM(out, 5, wrap(r.gC));
+    return out;
+}
+
+// The buffer between phase B's chain and output workgroups and the host words its failures are reported in, per (device,
+// stream).  gdn_nax makes them (it owns the caches that a caller can look at): snap_provider(device index, bytes) -> (buffer,
+// pinned int32 tensor); failed(device index) raises what the words say and resets them.
+PyObject *snap_provider = nullptr, *snap_failed = nullptr;
+struct Snap {
+    Tensor buf, words;
+};
+const Snap& snap_buffer(const Tensor& like, long bytes) {
+    static auto* m = new std::map<std::pair<int, void*>, Snap>;
+    Snap& s = (*m)[{(int)like.device().index(), stream()}];
+    if (!s.buf.defined() || s.buf.numel() * 2 < bytes) {
+        if (!snap_provider) throw Error{PyExc_RuntimeError, "gdn_nax is not imported"};
+        PyObject* r = PyObject_CallFunction(snap_provider, "il", (int)like.device().index(), bytes);
+        if (!r) throw Raised{};
+        s = {THPVariable_Unpack(PyTuple_GET_ITEM(r, 0)), THPVariable_Unpack(PyTuple_GET_ITEM(r, 1))};
+        Py_DECREF(r);
+    }
+    const int* w = s.words.data_ptr<int>();
+    if (w[0] | w[1]) {                                           // an earlier launch with this buffer has failed
+        PyObject* r = PyObject_CallFunction(snap_failed, "i", (int)like.device().index());
+        if (!r) throw Raised{};
+        Py_DECREF(r);
+    }
+    return s;
+}
+// set_hooks(snap_provider, failed)
+PyObject* set_hooks(PyObject* const* a) {
+    Py_INCREF(a[0]);
+    Py_INCREF(a[1]);
+    Py_XSETREF(snap_provider, a[0]);
+    Py_XSETREF(snap_failed, a[1]);
+    Py_RETURN_NONE;
+}
+void phase_b_launch(const Records& r, const Snap& s, const Tensor& st, const Tensor& st_out, const Tensor* proj, const Tensor* gw, float eps,
+                    const Tensor& out, int64_t S) {
+    check(qt_gdn_phase_b_report(r.ops.data_ptr(), r.U.data_ptr(), r.gC.data_ptr<float>(), s.buf.data_ptr(), st.data_ptr<float>(), st_out.data_ptr<float>(),
+                                proj ? proj->data_ptr() : nullptr, gw ? gw->data_ptr<float>() : nullptr, eps, out.data_ptr(), dim32(S),
+                                s.words.data_ptr<int>(), stream()), "qt_gdn_phase_b");
+}
+
+// phase_b(S or proj, ops, U, gC, state, gw or None, eps): with gw (and proj) the gated norm follows in the same pass
+PyObject* phase_b(PyObject* const* a) {
+    const bool norm = a[5] != Py_None;
+    const Tensor proj = norm ? dev(a[0], BF16, "proj", {ANY, PW}) : Tensor();
+    const int64_t S = norm ? proj.size(0) : integer(a[0]);
+    const Records r{dev(a[1], F16, "Tb"), dev(a[2], F16, "Am"), dev(a[3], F32, "gv")};
+    const int s32 = dim32(S);
+    if (r.ops.numel() * 2 < qt_gdn_chunk_ops_bytes(s32) || r.U.numel() * 2 < qt_gdn_chunk_u_bytes(s32) || r.gC.numel() * 4 < qt_gdn_chunk_gc_bytes(s32))
+        value_error("phase_b: the phase A records are too small for this many tokens");
+    const Tensor state = dev(a[4], F32, "state").reshape({1, HV, DV, DK});
+    const Snap& s = snap_buffer(state, qt_gdn_chunk_snap_bytes(s32));
+    Tensor st_out = empty({1, HV, DV, DK}, F32, state), out;
+    if (norm) {
+        const Tensor gw = f32(a[5], "gw", DV);
+        out = empty({S, HV * DV}, BF16, state);
+        phase_b_launch(r, s, state, st_out, &proj, &gw, real(a[6]), out, S);
+    } else {
+        out = empty({S, HV, DV}, BF16, state);
+        phase_b_launch(r, s, state, st_out, nullptr, nullptr, 0.f, out, S);
+    }
+    return wrap({out, st_out});
+}
+
+// gdn_core(proj, conv_state, ssm_state, conv_w, A_log, dt_bias, gw, want_qkv): both phases with the gated norm
+PyObject* gdn_core(PyObject* const* a) {
+    const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
+    const int64_t S = proj.size(0);
+    const Tensor cs = gpu_tensor(a[1], "conv_state").reshape({3, CD});
+    check_layout(cs, BF16, "conv_state");
+    const Tensor& w = flat_conv_w(a[3]);
+    const Tensor A = f32(a[4], "A_log", HV), dtb = f32(a[5], "dt_bias", HV), gw = f32(a[6], "gw", DV);
+    const Tensor state = dev(a[2], F32, "state").reshape({1, HV, DV, DK});
+    Tensor qkv[3];
+    const bool want = truth(a[7]);
+    if (want)
+        for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
+    const Snap& s = snap_buffer(proj, qt_gdn_chunk_snap_bytes(dim32(S)));
+    const Records r = new_records(proj);
+    Tensor conv_out = empty({1, 3, CD}, BF16, proj), st_out = empty({1, HV, DV, DK}, F32, proj), out = empty({S, HV * DV}, BF16, proj);
+    phase_a_conv(proj, cs, w, A, dtb, want ? qkv : nullptr, conv_out.data_ptr(), r);
+    phase_b_launch(r, s, state, st_out, &proj, &gw, 1e-6f, out, S);
+    return wrap({out, conv_out, st_out});
+}
+
+// ---- copies ---------------------------------------------------------------------------------------------------------------
+struct Jobs {
+    std::vector<void*> dst;
+    std::vector<const void*> src;
+    std::vector<long> meta;
+    void add(const Tensor& d, const Tensor& s, long n, long d0, long s0, long ny, long ds, long ss) {
+        const std::string who = "blit_batch: job " + std::to_string(dst.size());
+        if (d.scalar_type() != s.scalar_type() || (d.scalar_type() != BF16 && d.scalar_type() != F32))
+            type_error(who + ": bf16 or float32 tensors of one dtype expected");
+        check_layout(d, d.scalar_type(), "dst");
+        check_layout(s, s.scalar_type(), "src");
+        if (n < 0 || ny < 0 || d0 < 0 || s0 < 0 || ds < 0 || ss < 0) value_error(who + ": negative size, offset or stride");
+        if (n && ny && (d0 + (ny - 1) * ds + n > d.numel() || s0 + (ny - 1) * ss + n > s.numel()))
+            value_error(who + ": the copy leaves the source or the destination");
+        dst.push_back(d.data_ptr());
+        src.push_back(s.data_ptr());
+        for (long v : {(long)d.element_size(), n, d0, s0, ny, ds, ss}) meta.push_back(v);
+    }
+    void run() const {
+        if (dst.empty()) return;
+        const int rc = qt_blit_batch(dst.data(), src.data(), meta.data(), (int)dst.size(), stream());
+        if (rc == -2) value_error("blit_batch: every copy must be 16-byte granular (base pointers, sizes, offsets, strides)");
+        check(rc, "qt_blit_batch");
+    }
+};
+struct Items {                                                   // the items of a list or tuple
+    PyObject* seq;
+    explicit Items(PyObject* o) : seq(PySequence_Fast(o, "expected a sequence")) {
+        if (!seq) throw Raised{};
+    }
+    ~Items() { Py_DECREF(seq); }
+    Py_ssize_t size() const { return PySequence_Fast_GET_SIZE(seq); }
+    PyObject* operator[](Py_ssize_t i) const {
+        if (i >= size()) value_error("a sequence is shorter than expected");
+        return PySequence_Fast_GET_ITEM(seq, i);
+    }
+};
+
+// blit_batch(jobs): a sequence of (dst, src, n, d0, s0, ny, dstride, sstride)
+PyObject* blit_batch(PyObject* const* a) {
+    const Items jobs(a[0]);
+    Jobs j;
+    for (Py_ssize_t i = 0; i < jobs.size(); i++) {
+        const Items t(jobs[i]);
+        if (t.size() != 8) value_error("blit_batch: job " + std::to_string(i) + ": expected eight values");
+        j.add(gpu_tensor(t[0], "dst"), gpu_tensor(t[1], "src"), integer(t[2]), integer(t[3]), integer(t[4]), integer(t[5]), integer(t[6]), integer(t[7]));
+    }
+    j.run();
+    Py_RETURN_NONE;
+}
+
+// pools_load(conv pools, ssm pools, K pools, V pools, state conv, state ssm, state kv, slot, pos, Lmax, heads, width)
+PyObject* pools_load(PyObject* const* a) {
+    const Items pc(a[0]), ps(a[1]), pk(a[2]), pv(a[3]), sc(a[4]), sm(a[5]), kv(a[6]);
+    const long slot = integer(a[7]), pos = integer(a[8]), Lmax = integer(a[9]), nkv = integer(a[10]), D = integer(a[11]), par = pos & 1;
+    const long C = 3 * CD, N = HV * DV * DK;
+    Jobs j;
+    for (Py_ssize_t i = 0; i < std::min(sc.size(), sm.size()); i++) {
+        j.add(gpu_tensor(pc[i], "dst"), gpu_tensor(sc[i], "src"), C, (slot * 2 + par) * C, 0, 1, 0, 0);
+        j.add(gpu_tensor(ps[i], "dst"), gpu_tensor(sm[i], "src"), N, slot * N, 0, 1, 0, 0);
+    }
+    for (Py_ssize_t i = 0; i < kv.size(); i++) {
+        const Items pair(kv[i]);
+        const Tensor& K = gpu_tensor(pair[0], "src");
+        if (K.dim() != 4) value_error("state: K / V are expected as [1, heads, rows, width]");
+        const long smax = K.size(2);
+        j.add(gpu_tensor(pk[i], "dst"), K, pos * D, slot * nkv * Lmax * D, 0, nkv, Lmax * D, smax * D);
+        j.add(gpu_tensor(pv[i], "dst"), gpu_tensor(pair[1], "src"), pos * D, slot * nkv * Lmax * D, 0, nkv, Lmax * D, smax * D);
+    }
+    j.run();
+    Py_RETURN_NONE;
+}
+
+// ---- the module -----------------------------------------------------------------------------------------------------------
+template <PyObject* (*F)(PyObject* const*), int N>
+PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != N) {
+        PyErr_Format(PyExc_TypeError, "expected %d arguments, got %zd", N, n);
+        return nullptr;
+    }
+    try {
+        return F(args);
+    } catch (const Error& e) {
+        PyErr_SetString(e.type, e.text.c_str());
+    } catch (const Raised&) {
+    } catch (const c10::OutOfMemoryError& e) {
+        PyObject *torch = PyImport_ImportModule("torch"), *type = torch ? PyObject_GetAttrString(torch, "OutOfMemoryError") : nullptr;
+        if (type) PyErr_SetString(type, e.what_without_backtrace());
+        Py_XDECREF(type);
+        Py_XDECREF(torch);
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+}
+#define QT_FN(name, fn, n) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(entry<fn, n>)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    QT_FN("rms_rows", rms_rows, 4),       QT_FN("fused_gemv", fused_gemv, 7),     QT_FN("gated_norm", gated_norm, 4),
+    QT_FN("decode_step", decode_step, 11), QT_FN("verify_step", verify_step, 11), QT_FN("deltanet", deltanet, 8),
+    QT_FN("attn_b", attn_b, 10),          QT_FN("attn_layer_b", attn_layer_b, 11), QT_FN("sdpa", sdpa, 3),
+    QT_FN("qkv_prep", qkv_prep, 7),       QT_FN("out_gate", out_gate, 2),         QT_FN("conv_prep", conv_prep, 3),
+    QT_FN("phase_a", phase_a, 8),         QT_FN("phase_b", phase_b, 7),           QT_FN("gdn_core", gdn_core, 8),
+    QT_FN("set_hooks", set_hooks, 2),     QT_FN("blit_batch", blit_batch, 1),     QT_FN("pools_load", pools_load, 12),
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_qt_host", "argument checks, allocation and launch of the operators", -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__qt_host() { return PyModule_Create(&module); }

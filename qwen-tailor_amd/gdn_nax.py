@@ -8,7 +8,6 @@ from __future__ import annotations
 import torch
 
 from . import _lib as L
-from .kernels import flat_conv_w
 
 BF16 = torch.bfloat16
 HV, DK, DV, CD, PW = 16, 128, 128, 6144, 8224
@@ -20,37 +19,11 @@ DEFAULT_FLAGS = frozenset()
 TG = 64
 
 
-def _alloc_records(S, dev):
-    lib = L.lib()
-    ops = torch.empty(lib.qt_gdn_chunk_ops_bytes(S) // 2, dtype=torch.float16, device=dev)
-    U = torch.empty(lib.qt_gdn_chunk_u_bytes(S) // 2, dtype=torch.float16, device=dev)
-    gC = torch.empty(lib.qt_gdn_chunk_gc_bytes(S) // 4, dtype=torch.float32, device=dev)
-    return ops, U, gC
-
-
 def _phase_a(proj, conv_state, conv_w, A_log, dt_bias, qkv=None, want_qkv=True, conv_out=None):
     """Phase A.  With q, k, v given: the kernel that consumes them.  Otherwise one kernel that convolves and normalizes the
     projection rows itself (returning q, k, v only if want_qkv) and, if conv_out [3,6144] is given, writes the new conv
     window there.  Returns (q, k, v, ops, U, gC)."""
-    proj = L.dev(proj, BF16, "proj", (None, PW))
-    S = proj.shape[0]
-    A, dtb = L.f32(A_log, "A_log", (HV,)), L.f32(dt_bias, "dt_bias", (HV,))
-    ops, U, gC = _alloc_records(S, proj.device)
-    if qkv is not None:
-        q, k, v = (L.dev(t, BF16, name, (S, HV, DK)) for t, name in zip(qkv, "qkv"))
-        L.call("qt_gdn_phase_a", L.ptr(proj), L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(A), L.ptr(dtb), L.ptr(ops), L.ptr(U), L.ptr(gC), S,
-               L.stream())
-        return q, k, v, ops, U, gC
-    cs = L.dev(conv_state, BF16, "conv_state", (3, CD))
-    w = flat_conv_w(conv_w)
-    q = k = v = None
-    if want_qkv:
-        q, k, v = (torch.empty((S, HV, DK), dtype=BF16, device=proj.device) for _ in range(3))
-    if conv_out is not None:
-        conv_out = L.dev(conv_out, BF16, "conv_out", (3, CD))
-    L.call("qt_gdn_phase_a_conv", L.ptr(proj), L.ptr(cs), L.ptr(w), L.ptr(L.silu_table(proj.device)), L.ptr(A), L.ptr(dtb), L.ptr(q),
-           L.ptr(k), L.ptr(v), L.ptr(conv_out), L.ptr(ops), L.ptr(U), L.ptr(gC), S, L.stream())
-    return q, k, v, ops, U, gC
+    return L.host.phase_a(proj, conv_state, conv_w, A_log, dt_bias, qkv, want_qkv, conv_out)
 
 
 def prep_a(proj, conv_state, conv_w, A_log, dt_bias, relaxed=True):
@@ -68,7 +41,7 @@ def gdn_chunked(q, k, v, proj, A_log, dt_bias, state, relaxed=True, flags=DEFAUL
 
 _SNAP = {}            # (device index, stream handle) -> float16 tensor: flag area + chain snapshots
 _SNAP_RETIRED = []    # outgrown buffers stay alive: a captured HIP graph may hold their address
-_STATUS = {}          # (device index, stream handle) -> pinned int32[1]: the last copy of the buffer's status word
+_STATUS = {}          # (device index, stream handle) -> pinned int32[2]: set to 1 by a launch that gave up / whose state is not finite
 
 GAVE_UP, NOT_FINITE = 1, 2        # bits of the status word
 
@@ -92,7 +65,7 @@ def _snap_buffer(dev, nbytes):
             _SNAP_RETIRED.append(buf)
         buf = torch.zeros(max(nbytes // 2, 8), dtype=torch.float16, device=dev)
         _SNAP[key] = buf
-        _STATUS[key] = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        _STATUS[key] = torch.zeros(2, dtype=torch.int32, pin_memory=True)
     return buf
 
 
@@ -111,25 +84,33 @@ def _describe(v):
 
 
 def _raise_if_failed(key, buf, sync=False):
-    """Looks at the status word of the launches made so far with `buf`.  Without `sync` it reads the host copy that the last
-    launch's asynchronous read-back has left (no wait: a launch still in flight is judged at the next call); with `sync` it
-    waits for the stream first.  A set word is cleared on the device and raised as ChunkedPrefillError."""
+    """Looks at what the launches made so far with `buf` have reported into pinned host memory.  Without `sync` it does not wait
+    (a launch still in flight is judged at the next call); with `sync` it waits for the stream first.  A report is cleared, here
+    and in the buffer's status word, and raised as ChunkedPrefillError."""
     pin = _STATUS[key]
     if sync and not torch.cuda.is_current_stream_capturing():
         torch.cuda.current_stream(buf.device).synchronize()
-        pin.copy_(_status_word(buf))
-    v = int(pin[0])
+    v = (GAVE_UP if pin[0] else 0) | (NOT_FINITE if pin[1] else 0)
     if v:
-        torch.cuda.current_stream(buf.device).synchronize()     # error path only: no read-back may land after the reset
+        torch.cuda.current_stream(buf.device).synchronize()     # error path only: no launch may report after the reset
         _status_word(buf).zero_()
         pin.zero_()
         raise ChunkedPrefillError("chunked prefill: " + _describe(v))
 
 
-def _read_back_status(key, buf):
-    """Enqueues the copy of the status word to pinned host memory behind the launch (skipped under graph capture)."""
-    if not torch.cuda.is_current_stream_capturing():
-        _STATUS[key].copy_(_status_word(buf), non_blocking=True)
+def _provide_snap(index, nbytes):
+    """The buffer of the current stream of device `index` and its report words, for the native launch path (which keeps them until
+    it needs a larger one)."""
+    dev = torch.device("cuda", index)
+    return _snap_buffer(dev, nbytes), _STATUS[_key(dev)]
+
+
+def _report_found(index):
+    key = _key(torch.device("cuda", index))
+    _raise_if_failed(key, _SNAP[key])
+
+
+L.on_host_load(lambda host: host.set_hooks(_provide_snap, _report_found))
 
 
 def check_status(device=None, sync=True):
@@ -142,38 +123,13 @@ def check_status(device=None, sync=True):
         _raise_if_failed(key, _SNAP[key], sync=sync)
 
 
-def _phase_b_args(S, Tb, Am, gv, state):
-    ops, U, gC = L.dev(Tb, torch.float16, "Tb"), L.dev(Am, torch.float16, "Am"), L.dev(gv, torch.float32, "gv")
-    lib = L.lib()
-    if ops.numel() * 2 < lib.qt_gdn_chunk_ops_bytes(S) or U.numel() * 2 < lib.qt_gdn_chunk_u_bytes(S) or \
-            gC.numel() * 4 < lib.qt_gdn_chunk_gc_bytes(S):
-        raise ValueError("phase_b: the phase A records are too small for this many tokens")
-    state = L.dev(state, torch.float32, "state").reshape(1, HV, DV, DK)
-    snap = _snap_buffer(state.device, lib.qt_gdn_chunk_snap_bytes(S))
-    _raise_if_failed(_key(state.device), snap)              # the previous launch with this buffer, if its word has arrived
-    return ops, U, gC, snap, state, torch.empty_like(state)
-
-
 def phase_b(q, k, v, Tb, Am, gv, state, relaxed=True, flags=DEFAULT_FLAGS, tg=None):
     """The serial state recurrence on the outputs of phase A -> y [S,16,128] bf16, new state [1,16,128,128] f32
     (qwen35/gdn_nax.py:404-410).  Tb / Am / gv are the records prep_a (or gdn_chunked's phase A) produced."""
-    S = q.shape[0]
-    ops, U, gC, snap, state, out = _phase_b_args(S, Tb, Am, gv, state)
-    y = torch.empty((S, HV, DV), dtype=BF16, device=state.device)
-    L.call("qt_gdn_phase_b", L.ptr(ops), L.ptr(U), L.ptr(gC), L.ptr(snap), L.ptr(state), L.ptr(out), L.ptr(y), S, L.stream())
-    _read_back_status(_key(state.device), snap)
-    return y, out
+    return L.host.phase_b(q.shape[0], Tb, Am, gv, state, None, 0.0)
 
 
 def phase_b_norm(proj, Tb, Am, gv, state, gw, eps=1e-6):
     """phase_b followed by prefill.gated_norm (qwen35/prefill.py:241-244) in one pass: the outputs never leave the chip
     un-normalised.  proj [S,8224] bf16 supplies z; gw [128].  -> out [S,2048] bf16, new state [1,16,128,128] f32."""
-    proj = L.dev(proj, BF16, "proj", (None, PW))
-    S = proj.shape[0]
-    ops, U, gC, snap, state, new_state = _phase_b_args(S, Tb, Am, gv, state)
-    gw = L.f32(gw, "gw", (DV,))
-    out = torch.empty((S, HV * DV), dtype=BF16, device=state.device)
-    L.call("qt_gdn_phase_b_norm", L.ptr(ops), L.ptr(U), L.ptr(gC), L.ptr(snap), L.ptr(state), L.ptr(new_state), L.ptr(proj),
-           L.ptr(gw), float(eps), L.ptr(out), S, L.stream())
-    _read_back_status(_key(state.device), snap)
-    return out, new_state
+    return L.host.phase_b(proj, Tb, Am, gv, state, gw, eps)
