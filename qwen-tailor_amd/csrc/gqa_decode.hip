@@ -25,6 +25,7 @@
 // to 16) run as passes of up to four: pass j0 = 0, 4, 8, 12 takes rows j0 .. j0+3 of every sequence at position pos[b] + j0 and
 // finds the rows that the earlier passes appended among its pool keys (the passes are launches on one stream, in order).
 #include "qt_common.h"
+#include <type_traits>
 
 using namespace qt;
 
@@ -39,23 +40,47 @@ constexpr int GQA = AH / AKV;          // 4 query heads per KV head
 constexpr float SCALE = 0.0625f;       // 256^-0.5, batch.py:177
 constexpr float NEG = -3.0e38f;
 constexpr int VL_LD = AD + 16;         // row stride (elements) of the V tile in LDS: 544 bytes spread the 16 rows over the banks
+constexpr int MO_LD = AD + 4;           // row stride (floats) of the O tiles in LDS: the 16 rows of a store start 4 banks apart
 constexpr int KL_LD = AD + 8;          // row stride of the K tile: 528 bytes, the 16 rows of a fragment read start 4 banks apart
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
+// workgroup barrier for data that goes through LDS: loads and stores of global memory stay in flight across it (__syncthreads()
+// would wait for all of them)
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// a copy the compiler cannot see through: what is derived from it is computed again where it is used instead of living in
+// registers across the whole visit loop (about 30 lane-dependent addresses: they were spilled)
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // ---- the layer form: q / k RMSNorm and rotary embedding inside the attention kernel (qwen35/batch.py:505-512) ----------------
 constexpr int QKV_W = AH * 2 * AD + 2 * AKV * AD;      // 5120: [(q_h | gate_h) x 8 | k x 2 | v x 2]
 constexpr int ROPE_PAIRS = 32;                         // rotary pairs (i, i + 32), i < 32, of the first 64 features
 
+// max over the four lanes n, n + 16, n + 32, n + 48 with the vector-ALU lane swaps (v_permlane32_swap exchanges the upper half of one
+// register with the lower half of the other, v_permlane16_swap the odd 16-lane rows of one with the even rows of the other)
+__device__ __forceinline__ float max_over_groups(float x) {
+    const unsigned xi = __float_as_uint(x);
+    const auto a = __builtin_amdgcn_permlane32_swap(xi, xi, false, false);
+    const unsigned mi = __float_as_uint(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+    const auto b = __builtin_amdgcn_permlane16_swap(mi, mi, false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 // Online-softmax update of one tile of 16 keys from its transposed scores: lane (row n, group g) holds keys 4g .. 4g+3.
-// Leaves the probabilities of those keys in p (fp32) and writes the row's rescale factor to c_lds[row].
-__device__ __forceinline__ void softmax_tile(const f32x4& acc, int nvalid, bool causal, float& m_run, float& l_run, float (&p)[4],
-                                             float* c_lds, int lane) {
+// Leaves the probabilities of those keys in p (fp32) and returns the row's rescale factor (the same in the row's four lanes).
+__device__ __forceinline__ float softmax_tile(const f32x4& acc, int nvalid, bool causal, float& m_run, float& l_run, float (&p)[4], int lane) {
     const int n = lane & 15, g = lane >> 4;
     const int jq = n / GQA;                                      // query token of this row (rows >= 4*M are padding)
     float s[4], mx = NEG;
@@ -66,8 +91,7 @@ __device__ __forceinline__ void softmax_tile(const f32x4& acc, int nvalid, bool 
         s[i] = vis ? acc[i] * SCALE : NEG;
         mx = fmaxf(mx, s[i]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_over_groups(mx);
     const float m_new = fmaxf(m_run, mx);
     const float corr = __expf(m_run - m_new);                    // m_run = NEG initially: exp(-huge) = 0
     float ps = 0.f;
@@ -78,12 +102,14 @@ __device__ __forceinline__ void softmax_tile(const f32x4& acc, int nvalid, bool 
     }
     l_run = l_run * corr + ps;                                   // this lane's share; summed over g at the end
     m_run = m_new;
-    if (g == 0) c_lds[n] = corr;
+    return corr;
 }
 
-// O (16 rows x 256, accumulator layout: block j, lane (column 16 j + n, group g), rows 4g .. 4g+3) = c * O + P . V for the
-// V tile in v_lds ([16 keys][VL_LD]).  p: this lane's probabilities (row n, keys 4g .. 4g+3).
-__device__ __forceinline__ void pv_tile(f32x4 (&O)[16], const float (&p)[4], const bf16_t* v_lds, const float* c_lds, int lane) {
+// O^T (256 x 16 rows, accumulator layout: block j, lane (row n, group g), columns 16 j + 4 g .. + 3) = c * O^T + V^T . P^T for the
+// V tile in v_lds ([16 keys][VL_LD]).  p: this lane's probabilities (row n, keys 4g .. 4g+3), c: the row's rescale factor.  Taken in
+// this order a row's factor and its output columns belong to the lane that holds its probabilities, so the factor goes through
+// no LDS and a lane stores four adjacent columns.
+__device__ __forceinline__ void pv_tile(f32x4 (&O)[16], const float (&p)[4], float c, const bf16_t* v_lds, int lane) {
     const int n = lane & 15, g = lane >> 4;
     s16x4 ph, pl;
 #pragma unroll
@@ -92,19 +118,32 @@ __device__ __forceinline__ void pv_tile(f32x4 (&O)[16], const float (&p)[4], con
         ph[i] = (short)h;
         pl[i] = (short)f2bf(p[i] - bf2f(h));
     }
-    const f32x4 c4 = *reinterpret_cast<const f32x4*>(c_lds + 4 * g);
+    if (__any(c != 1.0f)) {                                      // some row's maximum moved
+#pragma unroll
+        for (int j = 0; j < 16; j++) O[j] *= c;
+    }
     // transposing load: within a group of 16 lanes, lane 4q + i receives element i of the 8-byte chunks addressed by lanes
     // q, q+4, q+8, q+12.  Lane j' = n of group g points at key 4g + n/4, columns 4 (n%4) .. + 3 of the block: lane n then
-    // receives keys 4g .. 4g+3 of column n, the B operand.
+    // receives keys 4g .. 4g+3 of column n, the A operand.
     const bf16_t* vrow = v_lds + (4 * g + (n >> 2)) * VL_LD + 4 * (n & 3);
 #pragma unroll
     for (int j = 0; j < 16; j++) {
-        const s16x4 B = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        if (j % 8 == 0) __builtin_amdgcn_sched_barrier(0);       // (at most eight fragments in registers at a time)
+        const s16x4 A = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (__attribute__((address_space(3))) s16x4*)(const_cast<bf16_t*>(vrow + 16 * j)));
-        O[j] *= c4;
-        O[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ph, B, O[j], 0, 0, 0);
-        O[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pl, B, O[j], 0, 0, 0);
+        O[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A, ph, O[j], 0, 0, 0);
+        O[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A, pl, O[j], 0, 0, 0);
     }
+}
+
+// inclusive prefix sum over the wavefront's lanes: four shifts within each 16-lane row, then the rows' totals as scalars
+__device__ __forceinline__ int wave_prefix_sum(int v, int lane) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);           // row_shr:1, 2, 4, 8 (zeros shifted in)
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+    const int r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31), r2 = __builtin_amdgcn_readlane(v, 47);
+    return v + (lane < 16 ? 0 : lane < 32 ? r0 : lane < 48 ? r0 + r1 : r0 + r1 + r2);
 }
 
 constexpr int MAX_SEG = 2048;          // segments (2 per sequence) a launch can hold
@@ -114,35 +153,35 @@ constexpr int MAX_SEG = 2048;          // segments (2 per sequence) a launch can
 constexpr int VISIT_TILES = 5;
 
 
-// Exclusive prefix of the segments' tile counts -> seg_start[0 .. nseg] (LDS); returns the total.  Rows whose slot or position
-// is out of range own no tiles (they are skipped by both kernels).  Every thread of the workgroup must call it.
-template <int M, int VISIT>
+// tiles of a segment in the flat tile space; a row whose slot or position is out of range owns none (it is skipped by both kernels)
+__device__ __forceinline__ int segment_tiles(int slot, int p0, int Lmax, int n_slots, int Mtot, int j0) {
+    const bool ok = (unsigned)slot < (unsigned)n_slots && p0 >= 0 && p0 + Mtot <= Lmax;    // all of the sequence's rows fit, or none is taken
+    return ok ? max(1, (p0 + j0 + 15) >> 4) + VISIT_TILES : 0;
+}
+// Prefix sums of the segments' tile counts -> seg_start[0 .. nseg] (LDS); returns the total.  Every thread of the workgroup (256)
+// must call it; 256 segments per round.
 __device__ __forceinline__ int build_segments(int* seg_start, const int* __restrict__ slots, const int* __restrict__ pos, int nseg,
                                               int Lmax, int n_slots, int Mtot, int j0) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    for (int sg = tid; sg < nseg; sg += 256) {
-        const int b = sg / AKV, slot = slots[b], p0 = pos[b];
-        const bool ok = (unsigned)slot < (unsigned)n_slots && p0 >= 0 && p0 + Mtot <= Lmax;    // all of the sequence's rows fit, or none is taken
-        seg_start[sg + 1] = ok ? max(1, (p0 + j0 + 15) >> 4) + VISIT : 0;
-    }
+    __shared__ int wave_total[2][4];
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    int carry = 0;
     if (tid == 0) seg_start[0] = 0;
-    __syncthreads();
-    if (tid < 64) {
-        int carry = 0;
-        for (int base = 1; base <= nseg; base += 64) {
-            const int i = base + lane;
-            int v = i <= nseg ? seg_start[i] : 0;
+    for (int base = 0, r = 0; base < nseg; base += 256, r ^= 1) {
+        const int sg = base + tid;
+        const int end = wave_prefix_sum(sg < nseg ? segment_tiles(slots[sg / AKV], pos[sg / AKV], Lmax, n_slots, Mtot, j0) : 0, lane);
+        if (lane == 63) wave_total[r][w] = end;
+        lds_barrier();
+        int before = carry;
 #pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int o = __shfl_up(v, d, 64);
-                if (lane >= d) v += o;
-            }
-            if (i <= nseg) seg_start[i] = v + carry;
-            carry += __shfl(v, 63, 64);
+        for (int i = 0; i < 4; i++) {
+            const int t = wave_total[r][i];
+            before += i < w ? t : 0;
+            carry += t;
         }
+        if (sg < nseg) seg_start[sg + 1] = end + before;
     }
-    __syncthreads();
-    return seg_start[nseg];
+    lds_barrier();
+    return carry;
 }
 // tiles per workgroup for `total` tiles spread over nwg workgroups, at least min_tiles
 __device__ __forceinline__ int tiles_per_wg(int total, int nwg, int min_tiles) { return max(min_tiles, (total + nwg - 1) / nwg); }
@@ -166,55 +205,101 @@ __global__ __launch_bounds__(256, 2) void attn_partial_kernel(const bf16_t* __re
     // one V tile and one K tile per wavefront, in one array: at the end the same memory holds the four wavefronts' scaled O
     // ([4][R rows][256] f32) for the merge
     __shared__ __align__(16) bf16_t tile_s[4 * 16 * (VL_LD + KL_LD)];
-    __shared__ __align__(16) float c_s[4][16];
     __shared__ float m_s[4][16], l_s[4][16];
-    static_assert(sizeof(bf16_t) * 4 * 16 * (VL_LD + KL_LD) >= sizeof(float) * 4 * 16 * AD, "the four O tiles must fit into the K / V tiles");
+    static_assert(sizeof(bf16_t) * 4 * 16 * (VL_LD + KL_LD) >= sizeof(float) * 4 * 16 * MO_LD, "the four O tiles must fit into the K / V tiles");
     float* const mo = reinterpret_cast<float*>(tile_s);
 
     const int nseg = B * AKV;
-    // (both forms cut the tile space alike, so that the layer form sums its partial results in the order of the plain one: same bits)
-    constexpr int VISIT = VISIT_TILES;
-    const int total = build_segments<M, VISIT>(seg_start, slots, pos, nseg, Lmax, n_slots, Mtot, j0);
-    if (blockIdx.x == 0)                                         // the merge kernel reads the table instead of building it again
-        for (int i = threadIdx.x; i <= nseg; i += 256) seg_tab[i] = seg_start[i];
-    const int per = tiles_per_wg(total, gridDim.x, min_tiles);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    // Every wavefront holds a window of 64 segments in its lanes: lane i has the end, the slot and the position of segment win + i (ends
+    // count in the flat tile space).  With up to 64 segments (32 sequences) the window is the whole table and comes from a prefix
+    // sum over the lanes: nothing goes through LDS and no barrier is met.  With more, the ends are built in LDS and the window is
+    // read where the workgroup's range begins.
+    // (both forms of the kernel cut the tile space alike, so that the layer form sums its partial results in the order of the
+    // plain one: same bits)
+    int win = 0, lane_end = 0, lane_slot = 0, lane_pos = 0, total;
+    auto load_rows = [&](int base) {
+        if (base + lane < nseg) lane_slot = slots[(base + lane) / AKV], lane_pos = pos[(base + lane) / AKV];
+    };
+    if (nseg <= 64) {
+        load_rows(0);
+        lane_end = wave_prefix_sum(segment_tiles(lane < nseg ? lane_slot : -1, lane_pos, Lmax, n_slots, Mtot, j0), lane);
+        total = __builtin_amdgcn_readlane(lane_end, 63);
+        if (blockIdx.x == 0 && w == 0) {                         // the merge kernel reads the table instead of building it again
+            if (lane == 0) seg_tab[0] = 0;
+            if (lane < nseg) seg_tab[lane + 1] = lane_end;
+        }
+    } else {
+        total = build_segments(seg_start, slots, pos, nseg, Lmax, n_slots, Mtot, j0);
+        if (blockIdx.x == 0)
+            for (int i = threadIdx.x; i <= nseg; i += 256) seg_tab[i] = seg_start[i];
+    }
+    const int per = tiles_per_wg(__builtin_amdgcn_readfirstlane(total), gridDim.x, min_tiles);
     const int wt0 = blockIdx.x * per, wt1 = min(wt0 + per, total);
     if (wt0 >= wt1) return;
-    int sg0 = 0;                                                 // the segment that holds tile wt0 (uniform binary search)
-    for (int lo_ = 0, hi_ = nseg; lo_ < hi_;) {
-        const int mid = (lo_ + hi_) >> 1;
-        if (seg_start[mid + 1] <= wt0) lo_ = mid + 1; else hi_ = mid;
-        sg0 = lo_;
+    int sg0 = 0;                                                 // the segment that holds tile wt0
+    if (nseg <= 64) {
+        sg0 = __popcll(__ballot(lane < nseg && lane_end <= wt0));
+    } else {
+        for (int hi_ = nseg; sg0 < hi_;) {                       // (uniform binary search)
+            const int mid = (sg0 + hi_) >> 1;
+            if (__builtin_amdgcn_readfirstlane(seg_start[mid + 1]) <= wt0) sg0 = mid + 1; else hi_ = mid;
+        }
     }
-    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 15, g = lane >> 4;
-    const int hw = lane >> 5, cl = lane & 31;
-
-  for (int sg = sg0; sg < nseg && seg_start[sg] < wt1; sg++) {
-    const int ss = seg_start[sg], se = seg_start[sg + 1];
-    if (se == ss) continue;                                      // a skipped row
-    const int kvh = sg % AKV, b = sg / AKV;
-    const int slot = slots[b], p0 = pos[b] + j0;                 // the pass's rows start at p0; the keys below it are in the pool
-    const bool first = wt0 <= ss;                                // this workgroup holds the segment's first tile
-    const int lo = max(0, max(wt0, ss) - ss - VISIT) * 16, hi = min(max(0, min(wt1, se) - ss - VISIT) * 16, p0);
-    const size_t pslot = (size_t)blockIdx.x + sg;
-
-    const size_t pbase = ((size_t)slot * AKV + kvh) * Lmax * AD;
-    const bf16_t* kbase = Kp + pbase;
-    const bf16_t* vbase = Vp + pbase;
-    bf16_t* vl = tile_s + w * (16 * VL_LD);
-    bf16_t* kl = tile_s + 4 * (16 * VL_LD) + w * (16 * KL_LD);
-    const int ntiles = hi > lo ? (hi - lo + 15) / 16 : 0;
-    // Row addresses of a tile: key 2i (lower half wavefront) / 2i + 1 (upper half), 8 columns per lane, so one load covers
-    // two whole 512-byte rows (a wavefront-wide load of 16 rows x 64 bytes streams about 15 % slower from HBM).  Keys past
-    // `hi` re-read the tile's first key (they are masked / weighted by 0).
-    auto row_ptr = [&](const bf16_t* base, int t, int i) {
-        const int key0 = lo + t * 16, key = key0 + 2 * i + hw;
-        return reinterpret_cast<const u32x4*>(base + (size_t)(key < hi ? key : key0) * AD) + cl;
+    auto move_window = [&](int base) {
+        win = base;
+        load_rows(base);
+        lane_end = seg_start[min(base + lane, nseg - 1) + 1];
     };
-    u32x4 a[8], vv[8];
+    // A visit is the part of one segment that lies in this workgroup's range: its number (-1: there is none), slot, position of the
+    // pass's first row, pool keys [lo, hi), and whether the range holds the segment's first tile.  All of it is scalar.
+    auto find_visit = [&](int sg, int begin, int& v_sg, int& v_slot, int& v_p0, int& v_lo, int& v_hi, int& v_first) {
+        // the first one at or after segment sg, which begins at `begin`
+        int end = 0;
+        for (; sg < nseg && begin < wt1; sg++) {
+            if (sg - win >= 64) move_window(sg);
+            end = __builtin_amdgcn_readlane(lane_end, sg - win);
+            if (end != begin) break;                             // (otherwise a skipped row)
+        }
+        const bool found = sg < nseg && begin < wt1;
+        const int at = found ? sg - win : 0;
+        v_sg = __builtin_amdgcn_readfirstlane(found ? sg : -1);
+        v_slot = __builtin_amdgcn_readlane(lane_slot, at);
+        v_p0 = __builtin_amdgcn_readlane(lane_pos, at) + j0;
+        v_first = __builtin_amdgcn_readfirstlane(wt0 <= begin);
+        v_lo = __builtin_amdgcn_readfirstlane(max(0, max(wt0, begin) - begin - VISIT_TILES) * 16);
+        v_hi = __builtin_amdgcn_readfirstlane(min(max(0, min(wt1, end) - begin - VISIT_TILES) * 16, v_p0));
+    };
+    auto end_of = [&](int sg) { return __builtin_amdgcn_readlane(lane_end, sg - win); };
+    if (nseg > 64) move_window(sg0);
+    int v_sg, v_slot, v_p0, v_lo, v_hi;
+    int v_first;
+    find_visit(sg0, nseg <= 64 ? (sg0 ? end_of(sg0 - 1) : 0) : __builtin_amdgcn_readfirstlane(seg_start[sg0]), v_sg, v_slot, v_p0, v_lo, v_hi, v_first);
+    auto rows_of = [&](int sg, int slot) { return ((size_t)slot * AKV + sg % AKV) * Lmax * AD; };      // the (slot, head)'s rows in the pools
+    auto tiles_in = [](int lo, int hi) { return hi > lo ? (hi - lo + 15) / 16 : 0; };
 
-    // Q^T as the MFMA B operand: lane (row n, group g) holds q[row n][32 kb + 8 g .. + 8]; row n = token (n / 4), head n % 4
-    bf16x8 bq[8];
+    bf16_t* const vl = tile_s + w * (16 * VL_LD);
+    bf16_t* const kl = tile_s + 4 * (16 * VL_LD) + w * (16 * KL_LD);
+    u32x4 a[8], vv[8];
+    // Rows of a tile: key 2i (lower half wavefront) / 2i + 1 (upper half), 8 columns per lane, so one load covers two whole
+    // 512-byte rows (a wavefront-wide load of 16 rows x 64 bytes streams about 15 % slower from HBM).  Keys past `hi` re-read the
+    // tile's first key (they are masked / weighted by 0).  The tile's address is a scalar; a lane adds 32 bits.
+    auto load_row = [](int ln, const bf16_t* tile0, int nkeys, int i) {
+        const unsigned key = 2 * i + (ln >> 5);
+        const unsigned off = ((int)key < nkeys ? key * (AD * 2) : 0u) + (ln & 31) * 16u;
+        return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(tile0) + off));
+    };
+    auto load_first_tile = [&](int sg, int slot, int lo, int hi) {             // in the order of their use
+        if (sg < 0 || w >= tiles_in(lo, hi)) return;
+        const size_t at = rows_of(sg, slot) + (size_t)(lo + w * 16) * AD;
+        const int nkeys = hi - (lo + w * 16), ln = opaque(lane);
+#pragma unroll
+        for (int i = 0; i < 8; i++) a[i] = load_row(ln, Kp + at, nkeys, i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) vv[i] = load_row(ln, Vp + at, nkeys, i);
+        __builtin_amdgcn_sched_barrier(0);
+    };
     // layer form: the staged query rows lie in wavefront 0's V tile (the tiles are not in use yet), the staged new keys in an
     // array of their own (they are read after the tile loop).  With the query rows in an array of their own the workgroup's LDS
     // would pass half of a CU's: the compiler then plans for one workgroup per CU and all 512 registers, puts O into the
@@ -222,29 +307,67 @@ __global__ __launch_bounds__(256, 2) void attn_partial_kernel(const bf16_t* __re
     __shared__ __align__(16) bf16_t k_s[LAYER ? 4 * KL_LD : 8];
     bf16_t* const q_s = tile_s;
     static_assert(16 * KL_LD <= 16 * VL_LD, "the staged query rows must fit into one V tile");
+
+  if (v_sg < 0) return;                                          // (a range that lies in empty positions)
+  // What a visit needs besides its tiles: the new values, and Q^T as the MFMA B operand: lane (row n, group g) holds q[row n][32 kb +
+  // 8 g .. + 8]; row n = token (n / 4), head n % 4.  The first visit's first tile is requested in here.
+  constexpr int NEW_REGS = (M + 1) / 2;
+  u32x4 nv[NEW_REGS];
+  bf16x8 bq[8];
+  auto prepare = [&](auto first_visit) {
+    const int v_b = v_sg / AKV, v_kvh = v_sg % AKV, v_ntiles = tiles_in(v_lo, v_hi);
+    const size_t v_base = rows_of(v_sg, v_slot);
+    // The wavefront with the fewest tiles also takes the M new keys of the sequence, where this workgroup holds the segment's first
+    // tile; it asks for the new values now (keys 2 i and 2 i + 1 in the lower and upper half of the lanes; they are used after its tiles) and appends what it holds.
+    const bool takes_new = v_first && w == (v_ntiles & 3);
+#pragma unroll
+    for (u32x4& x : nv) x = u32x4{0, 0, 0, 0};
+    if (takes_new) {
+        const bf16_t* vn = LAYER ? q + (size_t)(v_b * Mtot + j0) * QKV_W + AH * 2 * AD + AKV * AD + v_kvh * AD
+                                 : v_new + ((size_t)(v_b * Mtot + j0) * AKV + v_kvh) * AD;
+        const size_t stride = LAYER ? (size_t)QKV_W : (size_t)AKV * AD;
+        const int ln = opaque(lane);
+#pragma unroll
+        for (int i = 0; i < NEW_REGS; i++)
+            if (2 * i + (ln >> 5) < M) nv[i] = reinterpret_cast<const u32x4*>(vn + (size_t)(2 * i + (ln >> 5)) * stride)[ln & 31];
+    }
+
     if constexpr (LAYER) {
-        // The wavefront's first tile is requested before anything else: the norm and the rotary embedding below run while it
-        // is on its way from HBM.
-        if (w < ntiles) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) a[i] = __builtin_nontemporal_load(row_ptr(kbase, w, i));
-#pragma unroll
-            for (int i = 0; i < 8; i++) vv[i] = __builtin_nontemporal_load(row_ptr(vbase, w, i));
-        }
-        __builtin_amdgcn_sched_barrier(0);
         // The 4 M query rows are normed and roped once per workgroup: wavefront w takes token w (its four heads, a row per
         // 16-lane group, 16 consecutive elements per lane) and leaves the rows in LDS, where every wavefront picks up its
-        // B operand.  The workgroup that holds the segment's first tile does the same for the M new keys (wavefront 0, a key
-        // per 16-lane group), which it also appends to the pool (batch.py:196-201).  Same arithmetic, value for value, as
+        // B operand.  The workgroup that holds the segment's first tile does the same for the M new keys (a key per 16-lane
+        // group), which it also appends to the pool (batch.py:196-201).  Same arithmetic, value for value, as
         // attn_qkv_prep_kernel: sum of squares exact in double and rounded once, correctly rounded 1 / sqrt,
         // BF(w * BF(x * inv)), rotary products and sums rounded one by one; (cos, sin) from the table qt_rope_table_build wrote.
-        const int rr = lane >> 4, c = lane & 15;
-        auto glue16 = [&](const bf16_t* x, const bf16_t* wgt, const float2* cs, u32x4& o0, u32x4& o1) {
-            const u32x4 x0 = reinterpret_cast<const u32x4*>(x)[0], x1 = reinterpret_cast<const u32x4*>(x)[1];
-            const u32x4 w0 = reinterpret_cast<const u32x4*>(wgt)[0], w1 = reinterpret_cast<const u32x4*>(wgt)[1];
+        // A wavefront's loads return in the order in which they were issued, so the first visit's rows are requested before
+        // its first tile and the arithmetic runs while the tile is on its way from HBM; a later visit's tile was requested
+        // while the visit before it was still at work.
+        const int ln = opaque(lane), rr = ln >> 4, c = ln & 15;
+        if (w >= M) {                                             // rows past 4 M: zeros
+            *reinterpret_cast<u32x4*>(q_s + (4 * w + rr) * KL_LD + 16 * c) = u32x4{0, 0, 0, 0};
+            *reinterpret_cast<u32x4*>(q_s + (4 * w + rr) * KL_LD + 16 * c + 8) = u32x4{0, 0, 0, 0};
+        }
+        // item it: the query rows of token it, or (it = M, on an idle wavefront if there is one) the new keys; one copy of the code
+        const int items = M + (v_first ? 1 : 0);
+        int it = w;
+#pragma unroll 1
+        do {
+            const bool is_q = it < M, real = it < items;          // (a wavefront without an item goes along once: it has a tile to request)
+            const int tok = is_q ? it : rr < M ? rr : 0;          // (of the keys' four groups the idle ones work on a copy of key 0)
+            const u32x4* x = reinterpret_cast<const u32x4*>(q + (size_t)(v_b * Mtot + j0 + tok) * QKV_W +
+                                                            (is_q ? (v_kvh * GQA + rr) * 2 * AD : AH * 2 * AD + v_kvh * AD) + 16 * c);
+            const u32x4* wgt = reinterpret_cast<const u32x4*>((is_q ? q_norm : k_norm) + 16 * c);
+            const f32x4* cs = reinterpret_cast<const f32x4*>(rope_tab + (size_t)(v_p0 + tok) * ROPE_PAIRS + 16 * (c & 1));
+            u32x4 x0, x1, w0, w1;
             f32x4 cv[8];                                          // rotary pairs 16 (c & 1) .. + 15 (used by lanes c < 4 only)
+            if (real) {
+                x0 = x[0], x1 = x[1], w0 = wgt[0], w1 = wgt[1];
 #pragma unroll
-            for (int e = 0; e < 8; e++) cv[e] = reinterpret_cast<const f32x4*>(cs)[e];
+                for (int e = 0; e < 8; e++) cv[e] = cs[e];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (decltype(first_visit)::value && it == w) load_first_tile(v_sg, v_slot, v_lo, v_hi);
+            if (!real) break;
             float y[16], wt[16];
             unpack8(make_uint4(x0[0], x0[1], x0[2], x0[3]), reinterpret_cast<float(&)[8]>(y[0]));
             unpack8(make_uint4(x1[0], x1[1], x1[2], x1[3]), reinterpret_cast<float(&)[8]>(y[8]));
@@ -259,7 +382,7 @@ __global__ __launch_bounds__(256, 2) void attn_partial_kernel(const bf16_t* __re
             // rotary pairs (i, i + 32), i < 32: lanes 0, 1 of a row hold the first halves, lanes 2, 3 their partners
             float other[16];
 #pragma unroll
-            for (int e = 0; e < 16; e++) other[e] = __shfl_xor(y[e], 2, 64);
+            for (int e = 0; e < 16; e++) other[e] = dpp_mov<0x4E>(y[e]);              // lane c ^ 2
             if (c < 4) {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -270,167 +393,154 @@ __global__ __launch_bounds__(256, 2) void attn_partial_kernel(const bf16_t* __re
                                     : oth + own);                 // y1 s + y2 c
                 }
             }
-            o0 = u32x4{pack2_bf(y[0], y[1]), pack2_bf(y[2], y[3]), pack2_bf(y[4], y[5]), pack2_bf(y[6], y[7])};
-            o1 = u32x4{pack2_bf(y[8], y[9]), pack2_bf(y[10], y[11]), pack2_bf(y[12], y[13]), pack2_bf(y[14], y[15])};
-        };
-        {
-            u32x4 o0 = {0, 0, 0, 0}, o1 = {0, 0, 0, 0};           // (rows past 4 M: zeros)
-            if (w < M)
-                glue16(q + (size_t)(b * Mtot + j0 + w) * QKV_W + (kvh * GQA + rr) * 2 * AD + 16 * c, q_norm + 16 * c,
-                       rope_tab + (size_t)(p0 + w) * ROPE_PAIRS + 16 * (c & 1), o0, o1);
-            *reinterpret_cast<u32x4*>(q_s + (4 * w + rr) * KL_LD + 16 * c) = o0;
-            *reinterpret_cast<u32x4*>(q_s + (4 * w + rr) * KL_LD + 16 * c + 8) = o1;
-        }
-        if (first && w == 0) {
-            const int key = rr < M ? rr : 0;                      // (idle groups work on a copy of key 0 and store nothing)
-            u32x4 o0, o1;
-            glue16(q + (size_t)(b * Mtot + j0 + key) * QKV_W + AH * 2 * AD + kvh * AD + 16 * c, k_norm + 16 * c,
-                   rope_tab + (size_t)(p0 + key) * ROPE_PAIRS + 16 * (c & 1), o0, o1);
-            if (rr < M) {
+            const u32x4 o0 = u32x4{pack2_bf(y[0], y[1]), pack2_bf(y[2], y[3]), pack2_bf(y[4], y[5]), pack2_bf(y[6], y[7])};
+            const u32x4 o1 = u32x4{pack2_bf(y[8], y[9]), pack2_bf(y[10], y[11]), pack2_bf(y[12], y[13]), pack2_bf(y[14], y[15])};
+            if (is_q) {                                           // (a pointer that may mean either array would be a flat access)
+                *reinterpret_cast<u32x4*>(q_s + (4 * it + rr) * KL_LD + 16 * c) = o0;
+                *reinterpret_cast<u32x4*>(q_s + (4 * it + rr) * KL_LD + 16 * c + 8) = o1;
+            } else if (rr < M) {
                 *reinterpret_cast<u32x4*>(k_s + rr * KL_LD + 16 * c) = o0;
                 *reinterpret_cast<u32x4*>(k_s + rr * KL_LD + 16 * c + 8) = o1;
-                *reinterpret_cast<u32x4*>(Kp + pbase + (size_t)(p0 + rr) * AD + 16 * c) = o0;
-                *reinterpret_cast<u32x4*>(Kp + pbase + (size_t)(p0 + rr) * AD + 16 * c + 8) = o1;
+                *reinterpret_cast<u32x4*>(Kp + v_base + (size_t)(v_p0 + rr) * AD + 16 * c) = o0;
+                *reinterpret_cast<u32x4*>(Kp + v_base + (size_t)(v_p0 + rr) * AD + 16 * c + 8) = o1;
             }
-        }
-        __syncthreads();
+            it += 4;
+        } while (it < items);
+        lds_barrier();
+        const int n = ln & 15, g = ln >> 4;
 #pragma unroll
         for (int kb = 0; kb < 8; kb++) bq[kb] = as_bf16x8(*reinterpret_cast<const u32x4*>(q_s + n * KL_LD + 32 * kb + 8 * g));
-        __syncthreads();                                          // every wavefront has its rows: wavefront 0 may park its first tile there
+        lds_barrier();                                            // every wavefront has its rows: wavefront 0 may park its first tile there
     } else {
+        const int ln = opaque(lane), n = ln & 15, g = ln >> 4;
         const bool real = n < R;
-        const bf16_t* qr = q + ((size_t)(b * Mtot + j0 + (real ? n / GQA : 0)) * AH + kvh * GQA + (n % GQA)) * AD;
+        const bf16_t* qr = q + ((size_t)(v_b * Mtot + j0 + (real ? n / GQA : 0)) * AH + v_kvh * GQA + (n % GQA)) * AD;
 #pragma unroll
         for (int kb = 0; kb < 8; kb++) {
-            u32x4 v = reinterpret_cast<const u32x4*>(qr)[kb * 4 + g];
-            if (!real) v = u32x4{0, 0, 0, 0};
-            bq[kb] = as_bf16x8(v);
+            u32x4 x = reinterpret_cast<const u32x4*>(qr)[kb * 4 + g];
+            if (!real) x = u32x4{0, 0, 0, 0};
+            bq[kb] = as_bf16x8(x);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        if (decltype(first_visit)::value) load_first_tile(v_sg, v_slot, v_lo, v_hi);
     }
+  };
+  prepare(std::true_type{});
+  while (true) {
+    const int v_b = v_sg / AKV, v_kvh = v_sg % AKV, v_ntiles = tiles_in(v_lo, v_hi);
+    const size_t v_base = rows_of(v_sg, v_slot);
+    const bool takes_new = v_first && w == (v_ntiles & 3);
     float m_run = NEG, l_run = 0.f;
     f32x4 O[16];
 #pragma unroll
     for (int j = 0; j < 16; j++) O[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    if (w < ntiles) {
-        if constexpr (!LAYER) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) a[i] = __builtin_nontemporal_load(row_ptr(kbase, w, i));
-#pragma unroll
-            for (int i = 0; i < 8; i++) vv[i] = __builtin_nontemporal_load(row_ptr(vbase, w, i));
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        for (int t = w; t < ntiles; t += 4) {
-            const int tn = t + 4 < ntiles ? t + 4 : t;           // the last step re-reads its own tile
-            const int nvalid = min(16, hi - (lo + t * 16));
+    // the tile registers of the last step take the first tile of the next visit: its latency passes while this one is finished
+    int n_sg, n_slot, n_p0, n_lo, n_hi;
+    int n_first;
+    find_visit(v_sg + 1, end_of(v_sg), n_sg, n_slot, n_p0, n_lo, n_hi, n_first);
+    if (w < v_ntiles) {
+        const int ln = opaque(lane), n = ln & 15, g = ln >> 4, hw = ln >> 5, cl = ln & 31;
+        auto tile = [&](int t, auto refill) {
+            const int nvalid = min(16, v_hi - (v_lo + t * 16)), nnext = v_hi - (v_lo + (t + 4) * 16);
+            const size_t at = v_base + (size_t)(v_lo + (t + 4) * 16) * AD;
             // park both tiles row-major in LDS; every register is refilled with the next tile's row right after its store
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 *reinterpret_cast<u32x4*>(kl + (2 * i + hw) * KL_LD + 8 * cl) = a[i];
-                a[i] = __builtin_nontemporal_load(row_ptr(kbase, tn, i));
+                if constexpr (decltype(refill)::value) a[i] = load_row(ln, Kp + at, nnext, i);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 *reinterpret_cast<u32x4*>(vl + (2 * i + hw) * VL_LD + 8 * cl) = vv[i];
-                vv[i] = __builtin_nontemporal_load(row_ptr(vbase, tn, i));
+                if constexpr (decltype(refill)::value) vv[i] = load_row(ln, Vp + at, nnext, i);
                 __builtin_amdgcn_sched_barrier(0);
             }
+            if constexpr (!decltype(refill)::value) load_first_tile(n_sg, n_slot, n_lo, n_hi);
             wave_lds_sync();
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};      // (two chains: half the dependent latency)
 #pragma unroll
             for (int kb = 0; kb < 8; kb++) {                     // A operand: lane (key n, group g) holds k[key n][32 kb + 8 g .. + 8]
                 const u32x4 ka = *reinterpret_cast<const u32x4*>(kl + n * KL_LD + 32 * kb + 8 * g);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka), bq[kb], acc, 0, 0, 0);
+                acc[kb & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka), bq[kb], acc[kb & 1], 0, 0, 0);
             }
             float p[4];
-            softmax_tile(acc, nvalid, false, m_run, l_run, p, c_s[w], lane);
+            const float c = softmax_tile(acc[0] + acc[1], nvalid, false, m_run, l_run, p, ln);
+            pv_tile(O, p, c, vl, ln);
             wave_lds_sync();
-            pv_tile(O, p, vl, c_s[w], lane);
-            wave_lds_sync();
-        }
+        };
+        // the last tile is taken outside the loop: inside, its refill would read some tile again (64 KiB per visited segment, 17 %
+        // of the bytes of 64 sequences of 1100 keys)
+        int t = w;
+        for (; t + 4 < v_ntiles; t += 4) tile(t, std::true_type{});
+        tile(t, std::false_type{});
+    } else {
+        load_first_tile(n_sg, n_slot, n_lo, n_hi);
     }
-    if (first && w == 3) {
+    const int ln = opaque(lane), n = ln & 15, g = ln >> 4;
+    if (takes_new) {
+        const int hw = ln >> 5, cl = ln & 31;
         // The M new keys of this sequence, straight from the inputs (batch.py:143-145), with the causal rule among them:
-        // key i is visible to query token j only if i <= j.  Not pipelined: it runs once per sequence.
-        const bf16_t* kn = LAYER ? q + (size_t)(b * Mtot + j0) * QKV_W + AH * 2 * AD + kvh * AD
-                                 : k_new + ((size_t)(b * Mtot + j0) * AKV + kvh) * AD;
-        const bf16_t* vn = LAYER ? q + (size_t)(b * Mtot + j0) * QKV_W + AH * 2 * AD + AKV * AD + kvh * AD
-                                 : v_new + ((size_t)(b * Mtot + j0) * AKV + kvh) * AD;
-        const size_t stride = LAYER ? (size_t)QKV_W : (size_t)AKV * AD;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (LAYER) {                                    // the new keys as wavefront 0 left them in LDS
+        // key i is visible to query token j only if i <= j.  Not pipelined: it runs once per sequence.  The rows are appended to the
+        // pool here (batch.py:196-201): row j of the sequence goes to position p0 + j.
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        if constexpr (LAYER) {                                    // the new keys as they were left in LDS (and appended)
 #pragma unroll
             for (int kb = 0; kb < 8; kb++) {
-                u32x4 v = *reinterpret_cast<const u32x4*>(k_s + (n & 3) * KL_LD + 32 * kb + 8 * g);
-                if (n >= M) v = u32x4{0, 0, 0, 0};
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v), bq[kb], acc, 0, 0, 0);
+                u32x4 x = *reinterpret_cast<const u32x4*>(k_s + (n & 3) * KL_LD + 32 * kb + 8 * g);
+                if (n >= M) x = u32x4{0, 0, 0, 0};
+                acc[kb & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x), bq[kb], acc[kb & 1], 0, 0, 0);
             }
         } else {
-            const u32x4* kr = reinterpret_cast<const u32x4*>(kn + (size_t)(n < M ? n : 0) * stride);
-            u32x4 a[8];
+            const u32x4* kr = reinterpret_cast<const u32x4*>(k_new + ((size_t)(v_b * Mtot + j0 + (n < M ? n : 0)) * AKV + v_kvh) * AD);
+            u32x4 ka[8];
 #pragma unroll
-            for (int kb = 0; kb < 8; kb++) a[kb] = kr[kb * 4 + g];
+            for (int kb = 0; kb < 8; kb++) ka[kb] = kr[kb * 4 + g];
 #pragma unroll
-            for (int kb = 0; kb < 8; kb++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[kb]), bq[kb], acc, 0, 0, 0);
-        }
-        float p[4];
-        softmax_tile(acc, M, true, m_run, l_run, p, c_s[w], lane);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int key = 2 * i + hw;                          // rows past the M new keys are zero: their weight is 0
-            u32x4 v = u32x4{0, 0, 0, 0};
-            if (key < M) v = reinterpret_cast<const u32x4*>(vn + (size_t)key * stride)[cl];
-            *reinterpret_cast<u32x4*>(vl + key * VL_LD + 8 * cl) = v;
-        }
-        wave_lds_sync();
-        pv_tile(O, p, vl, c_s[w], lane);
-        wave_lds_sync();
-    }
-    if (first && w == 0) {
-        // append (batch.py:196-201): row j of this sequence goes to pool position p0 + j
-        for (int j = 0; j < M; j++) {
-            if constexpr (LAYER) {                               // (the keys are appended by the wavefront that norms them)
-                const uint2 vv2 = reinterpret_cast<const uint2*>(q + (size_t)(b * Mtot + j0 + j) * QKV_W + AH * 2 * AD + AKV * AD + kvh * AD)[lane];
-                reinterpret_cast<uint2*>(Vp + pbase + (size_t)(p0 + j) * AD)[lane] = vv2;
-            } else {
-                const uint2 kk = reinterpret_cast<const uint2*>(k_new + ((size_t)(b * Mtot + j0 + j) * AKV + kvh) * AD)[lane];
-                const uint2 vv2 = reinterpret_cast<const uint2*>(v_new + ((size_t)(b * Mtot + j0 + j) * AKV + kvh) * AD)[lane];
-                reinterpret_cast<uint2*>(Kp + pbase + (size_t)(p0 + j) * AD)[lane] = kk;
-                reinterpret_cast<uint2*>(Vp + pbase + (size_t)(p0 + j) * AD)[lane] = vv2;
+            for (int kb = 0; kb < 8; kb++) {
+                if (n < M) reinterpret_cast<u32x4*>(Kp + v_base + (size_t)(v_p0 + n) * AD)[kb * 4 + g] = ka[kb];
+                const u32x4 x = n < M ? ka[kb] : u32x4{0, 0, 0, 0};
+                acc[kb & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x), bq[kb], acc[kb & 1], 0, 0, 0);
             }
         }
+#pragma unroll
+        for (int i = 0; i < NEW_REGS; i++)
+            if (2 * i + hw < M) reinterpret_cast<u32x4*>(Vp + v_base + (size_t)(v_p0 + 2 * i + hw) * AD)[cl] = nv[i];
+        float p[4];
+        const float c = softmax_tile(acc[0] + acc[1], M, true, m_run, l_run, p, ln);
+#pragma unroll
+        for (int i = 0; i < 8; i++)                               // rows past the M new keys are zero: their weight is 0
+            *reinterpret_cast<u32x4*>(vl + (2 * i + hw) * VL_LD + 8 * cl) = i < NEW_REGS ? nv[i < NEW_REGS ? i : 0] : u32x4{0, 0, 0, 0};
+        wave_lds_sync();
+        pv_tile(O, p, c, vl, ln);
+        wave_lds_sync();
     }
 
-    // ---- merge the 4 wavefronts (deterministic order); lane (n, g) holds rows 4g .. 4g+3 of column 16 j + n
+    // ---- merge the 4 wavefronts (deterministic order); lane (n, g) holds columns 16 j + 4 g .. + 3 of row n
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
     if (g == 0) {
         m_s[w][n] = m_run;
         l_s[w][n] = l_run;
     }
-    __syncthreads();                                             // also: every wavefront is done with its V tile
-    float f[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int row = 4 * g + r;
-        const float mm = fmaxf(fmaxf(m_s[0][row], m_s[1][row]), fmaxf(m_s[2][row], m_s[3][row]));
-        f[r] = __expf(m_s[w][row] - mm);
-    }
+    lds_barrier();                                               // also: every wavefront is done with its V tile
+    const float f = __expf(m_run - fmaxf(fmaxf(m_s[0][n], m_s[1][n]), fmaxf(m_s[2][n], m_s[3][n])));
     // every wavefront leaves its scaled O in its own part of LDS; then each thread adds the four for R / 4 groups of four
     // columns, in a fixed order, and writes the partial result
-    if (4 * g < R) {
+    if (n < R) {
 #pragma unroll
-        for (int j = 0; j < 16; j++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) mo[(w * R + 4 * g + r) * AD + 16 * j + n] = O[j][r] * f[r];
+        for (int j = 0; j < 16; j++) *reinterpret_cast<f32x4*>(&mo[(w * R + n) * MO_LD + 16 * j + 4 * g]) = O[j] * f;
     }
-    __syncthreads();
+    lds_barrier();
+    const size_t pslot = (size_t)blockIdx.x + v_sg;
     float* po = part_o + pslot * R * AD;
+    const int tid = 64 * w + ln;
 #pragma unroll
     for (int i = tid; i < R * AD / 4; i += 256) {
-        const f32x4* src = reinterpret_cast<const f32x4*>(mo) + i;
-        reinterpret_cast<f32x4*>(po)[i] = (src[0] + src[R * AD / 4]) + (src[2 * (R * AD / 4)] + src[3 * (R * AD / 4)]);
+        const float* src = mo + (i / (AD / 4)) * MO_LD + 4 * (i % (AD / 4));
+        const auto part = [&](int ww) { return *reinterpret_cast<const f32x4*>(src + ww * (R * MO_LD)); };
+        reinterpret_cast<f32x4*>(po)[i] = (part(0) + part(1)) + (part(2) + part(3));
     }
     if (tid < R) {
         const float mm = fmaxf(fmaxf(m_s[0][tid], m_s[1][tid]), fmaxf(m_s[2][tid], m_s[3][tid]));
@@ -439,7 +549,10 @@ __global__ __launch_bounds__(256, 2) void attn_partial_kernel(const bf16_t* __re
         part_ml[(pslot * R + tid) * 2] = mm;
         part_ml[(pslot * R + tid) * 2 + 1] = ll;
     }
-    __syncthreads();                                             // the LDS tiles are reused by the next segment
+    lds_barrier();                                               // the LDS tiles are reused by the next visit
+    if (n_sg < 0) break;
+    v_sg = n_sg, v_slot = n_slot, v_p0 = n_p0, v_lo = n_lo, v_hi = n_hi, v_first = n_first;
+    prepare(std::false_type{});
   }
 }
 
