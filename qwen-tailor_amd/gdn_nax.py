@@ -65,7 +65,8 @@ def _snap_buffer(dev, nbytes):
             _SNAP_RETIRED.append(buf)
         buf = torch.zeros(max(nbytes // 2, 8), dtype=torch.float16, device=dev)
         _SNAP[key] = buf
-        _STATUS[key] = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+        if key not in _STATUS:                             # (kept when the buffer is outgrown: a captured HIP graph reports into it)
+            _STATUS[key] = torch.zeros(2, dtype=torch.int32, pin_memory=True)
     return buf
 
 

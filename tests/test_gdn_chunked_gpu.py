@@ -286,6 +286,21 @@ def test_give_up_path_ends_the_launch_and_leaves_the_flags_clean(qt, dev):
     check_tensors_equal("state of the launch after a give-up", s_got, s_want)
 
 
+def test_report_words_outlive_an_outgrown_buffer(qt, dev):
+    """launches (those of a captured HIP graph among them) keep the address of their stream's report words: a longer prompt that
+    outgrows the snapshot buffer must not replace the words"""
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        for T in (70, 700):
+            proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(77 + T, T)
+            _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0)
+            key = qt.gdn_nax._key(torch.device("cuda", torch.cuda.current_device()))
+            words = qt.gdn_nax._STATUS[key].data_ptr() if T == 70 else words
+        stream.synchronize()
+        assert qt.gdn_nax._STATUS[key].data_ptr() == words
+        qt.gdn_nax.check_status(dev, sync=True)
+
+
 @pytest.mark.parametrize("T", [4096, 4100])
 def test_phase_b_through_the_c_abi_with_a_caller_owned_snap(qt, dev, T):
     """qt_gdn_phase_b_norm called directly (ctypes) with a snap buffer the caller allocated and zeroed once: two launches in a row
