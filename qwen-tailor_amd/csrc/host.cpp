@@ -37,6 +37,14 @@ struct Error {                              // a Python exception to be raised
     std::string text;
 };
 struct Raised {};                           // ... that is already set
+struct Ref {                                // an owned reference (a null one is an exception that is already set)
+    PyObject* o;
+    explicit Ref(PyObject* p) : o(p) {
+        if (!o) throw Raised{};
+    }
+    Ref(const Ref&) = delete;
+    ~Ref() { Py_DECREF(o); }
+};
 [[noreturn]] void type_error(const std::string& s) { throw Error{PyExc_TypeError, s}; }
 [[noreturn]] void value_error(const std::string& s) { throw Error{PyExc_ValueError, s}; }
 
@@ -229,28 +237,24 @@ PyObject* fused_gemv(PyObject* const* a) {
         x = x.to(BF16);                                          // exact: the values are bf16 values
     }
     if (x.dim() != 2) x = x.reshape({-1, K});
-    if (!x.is_contiguous() && xin.dim() != 2) x = x.contiguous();
     check_layout(x, BF16, "x");
     const int64_t M = x.size(0);
     if (has_nw && has_gnorm) value_error("nw and gnorm are exclusive");
     if (swiglu && has_res) value_error("swiglu and res are exclusive");
     const float eps = real(a[3]);
     if (has_gnorm) {
-        PyObject* pair = PySequence_Fast(a[6], "gnorm: expected (proj, gw)");
-        if (!pair) throw Raised{};
-        PyObject *pp = PySequence_Fast_GET_ITEM(pair, 0), *pg = PySequence_Fast_GET_ITEM(pair, 1);
-        Py_DECREF(pair);                                         // (a[6] keeps its items)
+        const Ref pp(PySequence_GetItem(a[6], 0)), pg(PySequence_GetItem(a[6], 1));
         check_shape(x, "y", {ANY, HV * DV});
-        const Tensor proj = gpu_tensor(pp, "proj").reshape({M, PW});
+        const Tensor proj = gpu_tensor(pp.o, "proj").reshape({M, PW});
         check_layout(proj, BF16, "proj");
-        x = do_gated_norm(x, proj, f32(pg, "gw", DV), eps);
+        x = do_gated_norm(x, proj, f32(pg.o, "gw", DV), eps);
     }
     const int epi = swiglu ? 2 : has_res ? 1 : 0;
     const int64_t n_out = swiglu ? N / 2 : N;
     Tensor res;
     if (has_res) {
         res = gpu_tensor(a[4], "res");
-        if (res.dim() != 2) res = res.reshape({-1, N});
+        if (res.dim() != 2 || res.size(1) != N) res = res.reshape({-1, N});
         check_layout(res, BF16, "res");
         check_shape(res, "res", {M, N});
     }

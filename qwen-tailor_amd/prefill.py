@@ -43,4 +43,5 @@ def conv_prep(proj, conv_state, conv_w):
 
 def gated_norm(y, proj, gw):
     """Gated RMSNorm for S tokens (qwen35/prefill.py:241-244): y [S,16,128] or [S,2048] bf16 -> [S,2048] bf16."""
-    return L.host.gated_norm(y.reshape(-1, HV * DV) if y.dim() != 2 else y, proj, gw, 1e-6)
+    proj = L.dev(proj, BF16, "proj", (None, PW))
+    return L.host.gated_norm(L.dev(y, BF16, "y").reshape(proj.shape[0], HV * DV), proj, gw, 1e-6)

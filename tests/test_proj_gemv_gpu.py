@@ -195,3 +195,21 @@ def test_fused_gemv_rejects_bad_arguments(qt, dev):
         qt.kernels.fused_gemv(torch.zeros((64, 1000), dtype=BF16, device=dev), torch.zeros((2, 1000), dtype=BF16, device=dev))
     with pytest.raises(TypeError):
         qt.kernels.fused_gemv(W.cpu(), x)
+    with pytest.raises(IndexError):
+        qt.kernels.fused_gemv(torch.zeros((64, 2048), dtype=BF16, device=dev), torch.zeros((2, 2048), dtype=BF16, device=dev),
+                              gnorm=(torch.zeros((2, PW), dtype=BF16, device=dev),))
+    with pytest.raises(ValueError):                               # rows that are not contiguous are refused in any number of dimensions
+        qt.kernels.fused_gemv(W, torch.zeros((1, 2, 2048), dtype=BF16, device=dev)[..., :1024])
+
+
+def test_row_blocks_are_taken_in_any_shape(qt, dev):
+    """a residual and the rows of gated_norm count by their elements: [2 M, N / 2] is [M, N], [S * 16, 128] is [S, 2048]"""
+    g = torch.Generator().manual_seed(13)
+    W, x = to_dev(rand_bf(g, (64, 1024), 0.03), dev, BF16), to_dev(rand_bf(g, (3, 1024), 1.0), dev, BF16)
+    res = to_dev(rand_bf(g, (3, 64), 1.0), dev, BF16)
+    assert torch.equal(qt.kernels.fused_gemv(W, x, res=res.reshape(6, 32)), qt.kernels.fused_gemv(W, x, res=res))
+    y, proj = to_dev(rand_bf(g, (3, 2048), 1.0), dev, BF16), to_dev(rand_bf(g, (3, PW), 1.0), dev, BF16)
+    gw = torch.ones(128, device=dev)
+    want = qt.prefill.gated_norm(y, proj, gw)
+    assert torch.equal(qt.prefill.gated_norm(y.reshape(48, 128), proj, gw), want)
+    assert torch.equal(qt.prefill.gated_norm(y.reshape(3, 16, 128), proj, gw), want)
