@@ -228,6 +228,9 @@ int qt_blit(void* dst, const void* src, int elem_size, long n, long d0, long s0,
  * n, d0, s0, dstride, sstride in bytes), otherwise -2 and nothing is launched. */
 int qt_blit_batch(void* const* dst, const void* const* src, const long* meta, int count, qt_stream_t stream);
 
+/* qt_blit_batch with jobs that fill: where src[k] is null the rows of job k become zeros (its s0 and sstride are not used). */
+int qt_blit_fill_batch(void* const* dst, const void* const* src, const long* meta, int count, qt_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -85,7 +85,7 @@ def blit(dst, src, n, d0, s0, ny=1, dstride=0, sstride=0):
 def blit_batch(jobs):
     """Several blits in one launch: jobs = [(dst, src, n, d0, s0, ny, dstride, sstride), ...] with the arguments of blit.
     Every copy must be 16-byte granular (a ValueError says which one is not)."""
-    L.host.blit_batch(jobs)
+    L.host.blit_batch(jobs, ())
 
 
 class Pools:

@@ -621,9 +621,15 @@ struct Jobs {
         src.push_back(s.data_ptr());
         for (long v : {(long)d.element_size(), n, d0, s0, ny, ds, ss}) meta.push_back(v);
     }
+    void add_zeros(const Tensor& d, long n, long d0, long ny, long ds) {       // `ny` rows of `n` zeros
+        add(d, d, n, d0, d0, ny, ds, ds);                        // (the checks of the destination range)
+        src.back() = nullptr;
+        fills = true;
+    }
+    bool fills = false;
     void run() const {
         if (dst.empty()) return;
-        const int rc = qt_blit_batch(dst.data(), src.data(), meta.data(), (int)dst.size(), stream());
+        const int rc = (fills ? qt_blit_fill_batch : qt_blit_batch)(dst.data(), src.data(), meta.data(), (int)dst.size(), stream());
         if (rc == -2) value_error("blit_batch: every copy must be 16-byte granular (base pointers, sizes, offsets, strides)");
         check(rc, "qt_blit_batch");
     }
@@ -641,14 +647,19 @@ struct Items {                                                   // the items of
     }
 };
 
-// blit_batch(jobs): a sequence of (dst, src, n, d0, s0, ny, dstride, sstride)
+// blit_batch(jobs, zeros): sequences of (dst, src, n, d0, s0, ny, dstride, sstride) and of (dst, n, d0, ny, dstride)
 PyObject* blit_batch(PyObject* const* a) {
-    const Items jobs(a[0]);
+    const Items jobs(a[0]), zeros(a[1]);
     Jobs j;
     for (Py_ssize_t i = 0; i < jobs.size(); i++) {
         const Items t(jobs[i]);
         if (t.size() != 8) value_error("blit_batch: job " + std::to_string(i) + ": expected eight values");
         j.add(gpu_tensor(t[0], "dst"), gpu_tensor(t[1], "src"), integer(t[2]), integer(t[3]), integer(t[4]), integer(t[5]), integer(t[6]), integer(t[7]));
+    }
+    for (Py_ssize_t i = 0; i < zeros.size(); i++) {
+        const Items t(zeros[i]);
+        if (t.size() != 5) value_error("blit_batch: zeros " + std::to_string(i) + ": expected five values");
+        j.add_zeros(gpu_tensor(t[0], "dst"), integer(t[1]), integer(t[2]), integer(t[3]), integer(t[4]));
     }
     j.run();
     Py_RETURN_NONE;
@@ -705,7 +716,7 @@ PyMethodDef methods[] = {
     QT_FN("attn_b", attn_b, 10),          QT_FN("attn_layer_b", attn_layer_b, 11), QT_FN("sdpa", sdpa, 3),
     QT_FN("qkv_prep", qkv_prep, 7),       QT_FN("out_gate", out_gate, 2),         QT_FN("conv_prep", conv_prep, 3),
     QT_FN("phase_a", phase_a, 8),         QT_FN("phase_b", phase_b, 7),           QT_FN("gdn_core", gdn_core, 8),
-    QT_FN("set_hooks", set_hooks, 2),     QT_FN("blit_batch", blit_batch, 1),     QT_FN("pools_load", pools_load, 12),
+    QT_FN("set_hooks", set_hooks, 2),     QT_FN("blit_batch", blit_batch, 2),     QT_FN("pools_load", pools_load, 12),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_qt_host", "argument checks, allocation and launch of the operators", -1, methods};
 

@@ -149,3 +149,22 @@ def test_blit_batch_with_empty_jobs_and_more_units_than_workgroups(qt, dev):
         check_equal(f"job {k}", to_np(j[0]), w)
     qt.batch.blit_batch([jobs[0], jobs[2]])                                  # nothing to move at all
     check_equal("empty launch", to_np(jobs[0][0]), want[0])
+
+
+@pytest.mark.parametrize("n,d0,ny,ds", [(8, 8, 5, 64), (8192 + 8, 16, 3, 16384), (12 << 20, 0, 1, 0), (16, 0, 0, 16)])
+def test_fill_jobs_between_copies(qt, dev, n, d0, ny, ds):
+    """rows of zeros in one launch with copies, at the edges of a 16 KiB unit (8192 bf16 elements): only their rows change; a null
+    source is an error where copies only are asked for, and a range past the destination's end is refused"""
+    src = to_dev(bf(np.random.default_rng(5).standard_normal(4096)), dev, BF16)
+    a, b = torch.ones(4096 + 32, dtype=BF16, device=dev), torch.ones(d0 + max(ny - 1, 0) * ds + n + 24, dtype=BF16, device=dev)
+    qt._lib.host.blit_batch([(a, src, 4096, 16, 0, 1, 0, 0)], [(b, n, d0, ny, ds)])
+    want = torch.ones_like(b)
+    for y in range(ny):
+        want[d0 + y * ds:d0 + y * ds + n] = 0
+    assert torch.equal(a[16:4112], src) and bool((a[:16] == 1).all()) and bool((a[4112:] == 1).all())
+    assert torch.equal(b, want)
+    with pytest.raises(TypeError):
+        qt.batch.blit_batch([(b, None, 8, 0, 0, 1, 0, 0)])
+    if ny:
+        with pytest.raises(ValueError):
+            qt._lib.host.blit_batch([], [(b, n + 32, d0, ny, ds)])
