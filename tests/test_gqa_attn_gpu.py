@@ -456,6 +456,23 @@ def test_qkv_prep_and_out_gate_bit_exact(qt, dev, R, M):
     check_equal("gated output", to_np(qt.attention.out_gate(to_dev(o, dev, BF16), dq)), O.attn_out_gate(o, qkv))
 
 
+def test_out_gate_every_gate_value(qt, dev):
+    """out_gate takes the sigmoid two values at a time and without the tests of the general helper: every bf16 gate, in either half
+    of a pair and beside a gate that needs the general form, infinities and NaN among them"""
+    x = (np.arange(65536, dtype=np.uint32) << 16).view(np.float32)
+    g = np.concatenate([x, np.roll(x, 1), np.stack([x, np.full_like(x, 1000.0)], 1).ravel(), np.full(2048 - 1, 0.5, np.float32), x[:1]])
+    g = g[:len(g) // 2048 * 2048].reshape(-1, 8, 256)
+    qkv = np.zeros((len(g), O.QKV_W), np.float32)
+    qkv[:, :4096].reshape(-1, 8, 512)[:, :, 256:] = g
+    o = np.ones((len(g), 8, 256), np.float32)
+    with np.errstate(all="ignore"):
+        want = O.attn_out_gate(o, qkv)
+    got = to_np(qt.attention.out_gate(to_dev(o, dev, BF16), to_dev(qkv, dev, BF16)))
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    check_equal("gate", np.where(nan, 0, got), np.where(nan, 0, want))
+
+
 def test_attention_layer_core_decode_rows(qt, dev):
     """qkv_prep -> attn_b -> out_gate on 5 decode rows against the same chain of oracle functions (a full-attention layer between
     its qkv and o_proj projections, batch.py:504-514)"""
