@@ -66,7 +66,8 @@ int qt_normalize_qk(const void* q, const void* k, void* q_out, void* k_out, long
 
 /* prefill.conv_prep (qwen35/prefill.py:228-238): proj [S,8224], conv_state [3,6144] -> q, k, v [S,16,128] bf16.
  * silu_table: the qt_silu_table_bytes() byte table written once by qt_silu_table_build (the bf16 -> bf16 map of
- * mslib.py:21-22 on 2^-9 <= |x| < 2^5), owned by the caller; null = every workgroup computes its own copy. */
+ * mslib.py:21-22 on 2^-17 <= |x| < 2^7, in the order that this build of the library reads it in), owned by the caller; null = every
+ * workgroup computes its own copy. */
 int qt_silu_table_bytes(void);
 int qt_silu_table_build(void* table, qt_stream_t stream);
 int qt_gdn_conv_prep(const void* proj, const void* conv_state, const void* conv_w, const void* silu_table, void* q, void* k,

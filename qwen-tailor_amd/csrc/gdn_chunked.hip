@@ -382,7 +382,8 @@ __device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c,
     for (int j = 0; j < 8; j++) gwv[j] = gw[cc * 8 + j];
     // the four rows of this 16-lane group: all sums of squares first, then one reciprocal square root per lane
     uint4 yv4[4];
-    float ss4[4], inv4[4];
+    double ss4[4];
+    float inv4[4];
 #pragma unroll
     for (int it = 0; it < 4; it++) {
         const int row = it * 16 + (tid >> 4);
@@ -393,7 +394,7 @@ __device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c,
         double ss = 0.0;
 #pragma unroll
         for (int j = 0; j < 4; j++) ss += (double)yy[2 * j] * yy[2 * j] + (double)yy[2 * j + 1] * yy[2 * j + 1];
-        ss4[it] = (float)row16_sum_d(ss);
+        ss4[it] = ss;
     }
     // every z row is requested before the first result is stored: a wavefront's loads and stores share one counter, so a load
     // issued behind a store is waited for together with it, and a store takes microseconds to complete
@@ -404,7 +405,7 @@ __device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c,
         const u32x4 zw = load_once<STREAM>(reinterpret_cast<const u32x4*>(proj + (size_t)t * PW + CD + h * DV) + cc);
         zv4[it] = make_uint4(zw[0], zw[1], zw[2], zw[3]);
     }
-    rsqrt_rows<4>(ss4, eps, inv4, cc);
+    rsqrt_rows4(ss4, eps, inv4, cc);
 #pragma unroll
     for (int it = 0; it < 4; it++) {
         const int row = it * 16 + (tid >> 4);
@@ -583,12 +584,14 @@ __global__ __launch_bounds__(384, 3) void gdn_phase_b_kernel(const _Float16* ops
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Phase A: one workgroup of 512 threads per (chunk, head), two workgroups per CU.
+// Phase A: one workgroup of 512 threads per (chunk, head), two workgroups per CU.  Bound by its vector-ALU instructions (half of the time)
+// and by the latencies at either end of a workgroup.  Whole prefill at 61 / 2048 / 8192 tokens 20.5 / 51.5 / 170.1 us with row addresses
+// chosen per row, the table behind the rows and the gates ahead of the barrier; 19.7 / 50.0 / 166.9 us now.
 //
 // A (chunk, head) costs about 10^5 vector-ALU instructions of conv + SiLU + normalisation and a chain of dependent matrix
 // steps (K K^T, the 64 x 64 triangular inverse, the products with it) that keeps no unit busy.  The two run side by side:
 // wavefronts 0..3 (group M) convolve k, then walk the matrix chain while wavefronts 4..7 (group V) convolve q and v and
-// form A = lower(G * Q K^T).  One workgroup barrier (table, taps and gates ready); after it a consumer of k, q or v waits for
+// form A = lower(G * Q K^T).  One workgroup barrier (table and taps ready); after it a consumer of k, q or v waits for
 // that part's four producers through a counter in LDS.
 //
 // q, k and v are converted to half precision ONCE, when they are staged into LDS, and every MFMA operand is then a plain
@@ -614,15 +617,16 @@ constexpr int ND_BLK = 16 * ND_LD + 4;   // floats between diagonal blocks: the 
 constexpr float LOG2E = 1.4426950408889634f;
 
 struct PhaseALds {                       // 73 KiB: two workgroups per CU
+    __align__(16) bf16_t tab[SILU_TAB_SIZE];     // fused conv only: the silu_bf16 table.  First: an offset of 16 bits stays in this struct
     __align__(16) _Float16 Ks[C * QS_LD];
     __align__(16) _Float16 Qs[C * QS_LD];
     __align__(16) _Float16 Vs[C * VS_LD];
-    __align__(16) bf16_t tab[SILU_TAB_SIZE];     // fused conv only: the silu_bf16 table and this head's conv taps
-    __align__(16) bf16_t taps[3 * DK * 4];
+    __align__(16) bf16_t taps[3 * DK * 4];       // fused conv only: this head's conv taps
     __align__(16) float Td[4 * ND_BLK];          // their inverses: [block][column][row]
-    float Lc2[C], beta[C], gam[C], dec[C];       // Lc2 = log2(e) * cumsum(log g)
+    float Lc2[C], beta[C], gam[C];               // Lc2 = log2(e) * cumsum(log g)
     int staged[4];                               // wavefronts that have staged their part of k, q, v (PA_K, PA_Q, PA_V)
 };
+static_assert(sizeof(PhaseALds) >= 65536 && __builtin_offsetof(PhaseALds, tab) == 0, "an unclamped lookup reads up to 64 KiB from tab on");
 constexpr int PA_K = 0, PA_Q = 1, PA_V = 2;
 
 // A wavefront announces that its LDS stores of a part are done; a consumer waits until all four producers have.  (The parts
@@ -837,11 +841,44 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
     // one register array per part for both forms.  !from_proj: rw[rr] = token rr * 16 + gi, a lane 8 consecutive columns;
     // from_proj: rw[d] = input row 4 gi - 3 + d of 8 channels of the part
     uint4 rwA[7], rwB[7];
-    // (wavefront 0 asks for its gate inputs first: loads return in order, so the gates are computed while the rows are in flight)
-    bf16_t ga_raw = 0, gb_raw = 0;
-    if (wv == 0 && t0 + lane < S) {
-        ga_raw = proj[(size_t)(t0 + lane) * PW + CD + KD + HV + h];
-        gb_raw = proj[(size_t)(t0 + lane) * PW + CD + KD + h];
+    // input rows 4 gi - 3 .. + 3 of this thread's channels of a part; rows before the sequence come from the conv state (first chunk
+    // only), rows past the end repeat the last.  Elsewhere an address is one multiply-add on a scalar base: with the choice
+    // made row by row the 21 addresses of a thread were 200 instructions, and the first loads left that much later.
+    auto conv_rows = [&](uint4 (&rw)[7], int part) {
+        const int ch = part * KD + h * DK;
+        if (c > 0) {
+            const char* base = reinterpret_cast<const char*>(proj + (size_t)(t0 - 3) * PW + ch);
+            const unsigned last = (unsigned)(S + 2 - t0);
+#pragma unroll
+            for (int d = 0; d < 7; d++)
+                rw[d] = *reinterpret_cast<const uint4*>(base + (__umul24(min((unsigned)(4 * gi + d), last), PW * 2) + 16u * (unsigned)cc));
+        } else {
+#pragma unroll
+            for (int d = 0; d < 7; d++) {
+                const int tt = min(4 * gi - 3 + d, S - 1);
+                rw[d] = *reinterpret_cast<const uint4*>((tt < 0 ? cs + (tt + 3) * CD : proj + tt * PW) + ch + 8 * cc);
+            }
+        }
+    };
+    // (wavefront 0 asks for its gate inputs first: loads return in order)
+    unsigned ga_raw = 0, gb_raw = 0;
+    if (wv == 0) {
+        const bf16_t* row = proj + (size_t)min(t0 + lane, S - 1) * PW + CD + KD + h;
+        ga_raw = row[HV];
+        gb_raw = row[0];
+    }
+    // the SiLU table and the head's conv taps (3 x 128 channels x 4 taps: every token group needs the same 3 KiB) go to LDS.  Both
+    // are asked for ahead of the rows: a load behind them returns behind them, and a copy loop waits once per trip.
+    constexpr int TAB_VECS = SILU_TAB_SIZE / 8, TAP0 = 512 - 3 * 64;
+    uint4 tab0 = make_uint4(0, 0, 0, 0), tab1 = tab0, tap = tab0;
+    if (from_proj) {
+        const int i3 = max(tid - TAP0, 0);
+        if (silu_tab) {
+            tab0 = reinterpret_cast<const uint4*>(silu_tab)[tid];
+            tab1 = reinterpret_cast<const uint4*>(silu_tab)[min(tid + 512, TAB_VECS - 1)];
+        }
+        tap = reinterpret_cast<const uint4*>(cw + (size_t)((i3 >> 6) * KD + h * DK) * 4)[i3 & 63];
+        __builtin_amdgcn_sched_barrier(0);
     }
     if (!from_proj) {
 #pragma unroll
@@ -852,17 +889,7 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
             if (t >= S) rwA[rr] = make_uint4(0, 0, 0, 0);
         }
     } else {
-        const int chA = partA * KD + h * DK + cc * 8;
-#pragma unroll
-        for (int d = 0; d < 7; d++) {
-            const int tt = min(t0 + 4 * gi - 3 + d, S - 1);
-            rwA[d] = *reinterpret_cast<const uint4*>(tt < 0 ? cs + (tt + 3) * CD + chA : proj + (size_t)tt * PW + chA);
-        }
-        // the head's conv taps (3 x 128 channels x 4 taps) go through LDS: every token group needs the same 3 KiB
-        if (wv >= 5) {
-            const int i3 = tid - 320, part = i3 >> 6, i = i3 & 63;
-            reinterpret_cast<uint4*>(L.taps)[i3] = reinterpret_cast<const uint4*>(cw + (size_t)(part * KD + h * DK) * 4)[i];
-        }
+        conv_rows(rwA, partA);
         if (conv_out && c == (S - 1) / C && tid >= 64 && tid < 64 + 3 * 48) {   // new conv window: input rows S-3 .. S-1 of this head's channels
             const int i3 = tid - 64;
             const int r = i3 / 48, part = (i3 % 48) >> 4, ch0 = part * KD + h * DK + (i3 & 15) * 8, tt = S - 3 + r;
@@ -871,13 +898,29 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
         }
     }
 
-    // ---- gates of the chunk's tokens (gdn_nax.py:80-104): wavefront 0, one token per lane
+    if (from_proj) {
+        static_assert(TAB_VECS > 512 && TAB_VECS <= 1024, "two vectors of the table per thread");
+        if (silu_tab) {
+            reinterpret_cast<uint4*>(L.tab)[tid] = tab0;
+            if (tid + 512 < TAB_VECS) reinterpret_cast<uint4*>(L.tab)[tid + 512] = tab1;
+        } else {
+            silu_table_fill(L.tab, nullptr, tid, 512);
+        }
+        if (tid >= TAP0) reinterpret_cast<uint4*>(L.taps)[tid - TAP0] = tap;
+    }
+
+    if (tid >= 508) L.staged[tid - 508] = 0;
+    __syncthreads();
+
+    // ---- gates of the chunk's tokens (gdn_nax.py:80-104): wavefront 0, one token per lane.  Behind the barrier: nobody needs them before
+    // k is staged, which wavefront 0 announces after them, and group M has the time (it waits for v in the end).
     if (wv == 0) {
         const int t = t0 + lane;
         float lg = 0.f, be = 0.f;
+        asm volatile("" : "+v"(ga_raw), "+v"(gb_raw));          // (first used here: moved up to the loads, the use would wait for them there)
         if (t < S) {
-            lg = log_decay(A_log[h], BF(bf2f(ga_raw) + dt_bias[h]));
-            be = sigmoid_bf16(bf2f(gb_raw));
+            lg = log_decay(A_log[h], BF(bf2f((bf16_t)ga_raw) + dt_bias[h]));
+            be = sigmoid_bf16(bf2f((bf16_t)gb_raw));
         }
         float lc = lg;
 #pragma unroll
@@ -897,15 +940,11 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
         L.Lc2[lane] = lc * LOG2E;
         L.beta[lane] = be;
         L.gam[lane] = gm;
-        L.dec[lane] = dc;
         float* gp = gates + rec * GATE_FLOATS;
         gp[G_GAM + lane] = gm;
         gp[G_DEC + lane] = dc;
         if (lane >= 60) gp[G_GC + lane - 60] = lane == 60 ? expf(tot) : 0.f;
     }
-    if (from_proj) silu_table_fill(L.tab, silu_tab, tid, 512);
-    if (tid >= 508) L.staged[tid - 508] = 0;
-    __syncthreads();
 
     // ---- k (group M) and q (group V): conv + SiLU + L2 norm, staged as half precision
     {
@@ -924,21 +963,17 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
         } else {
             const float sc = grpV ? BF(INV_SCALE * INV_SCALE) : BF(INV_SCALE);
             uint4 wt[4], pk[4];
-            float ss[4], rr[4];
+            double ss[4];
+            float rr[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) wt[e] = *reinterpret_cast<const uint4*>(&L.taps[(partA * DK + cc * 8 + 2 * e) * 4]);
 #pragma unroll
-            for (int j = 0; j < 4; j++) ss[j] = (float)row16_sum_d(conv8_silu_packed(L.tab, rwA[j], rwA[j + 1], rwA[j + 2], rwA[j + 3], wt, pk[j]));
+            for (int j = 0; j < 4; j++) ss[j] = conv8_silu_packed<true>(L.tab, rwA[j], rwA[j + 1], rwA[j + 2], rwA[j + 3], wt, pk[j]);
             __builtin_amdgcn_sched_barrier(0);           // (the loads below must not be moved up: there is no room for them before)
             if (grpV) {                                  // v's rows: requested once q's are consumed (the register file holds one set)
-                const int chB = 2 * KD + h * DK + cc * 8;
-#pragma unroll
-                for (int d = 0; d < 7; d++) {
-                    const int tt = min(t0 + 4 * gi - 3 + d, S - 1);
-                    rwB[d] = *reinterpret_cast<const uint4*>(tt < 0 ? cs + (tt + 3) * CD + chB : proj + (size_t)tt * PW + chB);
-                }
+                conv_rows(rwB, 2);
             }
-            rsqrt_rows<4>(ss, qk_eps(), rr, cc);
+            rsqrt_rows4(ss, qk_eps(), rr, cc);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int tl = 4 * gi + j, t = t0 + tl;
@@ -964,7 +999,7 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
             for (int j = 0; j < 4; j++) {
                 const int tl = 4 * gi + j, t = t0 + tl;
                 uint4 p;
-                (void)conv8_silu_packed(L.tab, rwB[j], rwB[j + 1], rwB[j + 2], rwB[j + 3], wt, p);
+                (void)conv8_silu_packed<true>(L.tab, rwB[j], rwB[j + 1], rwB[j + 2], rwB[j + 3], wt, p);
                 if (t >= S) p = make_uint4(0, 0, 0, 0);
                 if (write_qkv && t < S) *reinterpret_cast<uint4*>(vi + ((size_t)t * HV + h) * DK + cc * 8) = p;
                 *reinterpret_cast<half8*>(&L.Vs[tl * VS_LD + cc * 8]) = bf8_to_half8(p);

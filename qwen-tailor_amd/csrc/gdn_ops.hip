@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void silu_table_kernel(bf16_t* __restrict__ ta
 // workgroup takes GN_ROWS rows (all loads first), and the GN_ROWS double-precision reciprocal square roots of a 16-lane group
 // are evaluated one per lane instead of all by every lane.  GN_ROWS = 4 for many rows (the kernel is then bound by those
 // evaluations), 1 for few (bound by the latency of one workgroup).
-template <int GN_ROWS>
+template <int GN_ROWS>                                           // 4 or 1
 __global__ __launch_bounds__(256) void gated_norm_kernel(const bf16_t* __restrict__ y, const bf16_t* __restrict__ proj,
                                                          const float* __restrict__ gw, bf16_t* __restrict__ out, long rows,
                                                          float eps) {
@@ -115,7 +115,8 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(const bf16_t* __restric
     float gwv[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) gwv[j] = gw[c * 8 + j];
-    float ss[GN_ROWS], inv[GN_ROWS];
+    double ss[GN_ROWS];
+    float inv[GN_ROWS];
 #pragma unroll
     for (int it = 0; it < GN_ROWS; it++) {
         float yy[8];
@@ -123,9 +124,12 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(const bf16_t* __restric
         double s2 = 0.0;
 #pragma unroll
         for (int j = 0; j < 4; j++) s2 += (double)yy[2 * j] * yy[2 * j] + (double)yy[2 * j + 1] * yy[2 * j + 1];
-        ss[it] = (float)row16_sum_d(s2);
+        ss[it] = s2;
     }
-    rsqrt_rows<GN_ROWS>(ss, eps, inv, c);
+    if constexpr (GN_ROWS == 4)
+        rsqrt_rows4(ss, eps, inv, c);
+    else
+        inv[0] = rsqrt_rn((float)row16_sum_d(ss[0]) / 128.0f + eps);
 #pragma unroll
     for (int it = 0; it < GN_ROWS; it++) {
         if (row0 + it >= rows) break;

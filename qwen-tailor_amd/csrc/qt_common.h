@@ -136,13 +136,15 @@ __device__ __forceinline__ float conv_silu(float w0, float w1, float w2, float x
 }
 
 // silu_bf16 is a bf16 -> bf16 map, so kernels that evaluate it many times per thread read it from a table in LDS:
-// 24 exponents (bf16 exponent fields 110..133, 2^-17 <= |x| < 2^7) x 128 mantissas x 2 signs = 6144 entries (12 KiB), the two
-// signs of a magnitude side by side: entry index = rotl16(x, 1) - 2 * (110 << 7).  Outside that range the map needs no
-// exponential (silu_out_of_table).  The table array has 8 more entries: index SILU_TAB_N2 is where out-of-range lookups land.
-constexpr int SILU_TAB_LO = 110, SILU_TAB_N2 = 2 * 24 * 128, SILU_TAB_SIZE = SILU_TAB_N2 + 8;
+// 24 exponents (bf16 exponent fields 110..133, 2^-17 <= |x| < 2^7) x 128 mantissas x 2 signs = 6144 entries (12 KiB), positive
+// values first: the byte offset of |x| is 2 (|x| - (110 << 7)), and a 16-bit product 2 x drops the sign by itself; negative values
+// lie SILU_TAB_HALF bytes behind (silu_offset2).  Outside that range the map needs no exponential (silu_out_of_table).  The table array
+// has 8 more entries: offset 2 SILU_TAB_HALF is where negative lookups outside the range land.
+constexpr int SILU_TAB_LO = 110, SILU_TAB_HALF = 2 * 24 * 128, SILU_TAB_SIZE = SILU_TAB_HALF + 8;
 __device__ __forceinline__ bf16_t silu_table_entry(int i) {
-    if (i >= SILU_TAB_N2) return 0;
-    const bf16_t xb = (bf16_t)(((i & 1) << 15) | (SILU_TAB_LO * 128 + (i >> 1)));
+    if (i >= SILU_TAB_HALF) return 0;
+    const bool neg = i >= SILU_TAB_HALF / 2;
+    const bf16_t xb = (bf16_t)((neg ? 0x8000 - SILU_TAB_HALF / 2 : 0) + SILU_TAB_LO * 128 + i);
     return f2bf(silu_bf16(bf2f(xb)));
 }
 // fills `tab` (LDS) from a prebuilt copy in global memory, or computes it when there is none
@@ -186,14 +188,25 @@ __device__ __forceinline__ uint32_t sigmoid_bf16_small2(uint32_t w) {
     const uint32_t neg = __builtin_bit_cast(uint32_t, (i16x2)(sw >> 15));          // (-0 counts as negative: both results are 1/2)
     return (y & neg) | (m & ~neg);
 }
-// table index of both halves of a bf16 pair (packed 16-bit arithmetic): rotl16(x, 1) - 2 * (LO << 7), wrapping for small |x|
-__device__ __forceinline__ u16x2 silu_index2(uint32_t w) {
-    const u16x2 x = __builtin_bit_cast(u16x2, w);
-    return x * (unsigned short)2 + (x >> 15) - (unsigned short)(SILU_TAB_LO * 256);
+// byte offset of the magnitude of both halves of a bf16 pair: 2 |x| - (LO << 8) in 16 bits, SILU_TAB_HALF or more outside the table.
+// (Packed multiply-adds, here and below; plain code becomes shifts, masks and permutations.)
+__device__ __forceinline__ u16x2 silu_offset2(uint32_t w) {
+    uint32_t r;
+    asm("v_pk_mad_u16 %0, %1, 2, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "s"(0x10000 - SILU_TAB_LO * 256));
+    return __builtin_bit_cast(u16x2, r);
+}
+// ... and with the sign: `mag`, for negative values SILU_TAB_HALF more
+__device__ __forceinline__ u16x2 silu_signed2(uint32_t w, u16x2 mag) {
+    uint32_t r;
+    asm("v_pk_lshrrev_b16 %0, 15, %1 op_sel_hi:[0,1]\n\tv_pk_mad_u16 %0, %0, %2, %3 op_sel_hi:[1,0,1]"
+        : "=&v"(r) : "v"(w), "s"(SILU_TAB_HALF), "v"(__builtin_bit_cast(uint32_t, mag)));
+    return __builtin_bit_cast(u16x2, r);
 }
 // conv4 + silu of 8 consecutive channels of one token: rows x0..x3 (oldest first, 8 bf16 each), taps wt (4 bf16 per channel);
-// the results as four bf16 pairs (their values are what silu_bf16 returns).  An input outside the table reads the spare entry
-// and is re-evaluated in one unlikely block per 8 channels.
+// the results as four bf16 pairs (their values are what silu_bf16 returns).  An input outside the table reads something else
+// and is re-evaluated in one unlikely block per 8 channels.  FREE: any offset below 64 KiB from `tab` may be read, so the offsets of such
+// inputs need not be clamped.
+template <bool FREE = false>
 __device__ __forceinline__ void conv8_silu_pairs(const bf16_t* tab, const uint4& x0, const uint4& x1, const uint4& x2,
                                                  const uint4& x3, const uint4 (&wt)[4], uint32_t (&r)[4]) {
     float a[8], b[8], c[8], d[8];
@@ -216,30 +229,32 @@ __device__ __forceinline__ void conv8_silu_pairs(const bf16_t* tab, const uint4&
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         xb[i] = pack2_bf(s[2 * i], s[2 * i + 1]);
-        const u16x2 idx = silu_index2(xb[i]);
-        worst = __builtin_elementwise_max(worst, idx);
-        const u16x2 off = __builtin_elementwise_min(idx, (u16x2){SILU_TAB_N2, SILU_TAB_N2}) << 1;     // byte offsets into the table
+        const u16x2 mag = silu_offset2(xb[i]);
+        worst = __builtin_elementwise_max(worst, mag);
+        const u16x2 in = FREE ? mag : __builtin_elementwise_min(mag, (u16x2){SILU_TAB_HALF, SILU_TAB_HALF});
+        const u16x2 off = silu_signed2(xb[i], in);
         const char* tb = reinterpret_cast<const char*>(tab);
         u16x2 v;
         v.x = *reinterpret_cast<const bf16_t*>(tb + off.x);
         v.y = *reinterpret_cast<const bf16_t*>(tb + off.y);
         r[i] = __builtin_bit_cast(uint32_t, v);
     }
-    if (__builtin_expect(max(worst.x, worst.y) >= SILU_TAB_N2, 0)) {
+    if (__builtin_expect(max(worst.x, worst.y) >= SILU_TAB_HALF, 0)) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const u16x2 idx = silu_index2(xb[i]);
-            if (idx.x >= SILU_TAB_N2) r[i] = (r[i] & 0xffff0000u) | f2bf(silu_out_of_table(lo_bf(xb[i])));
-            if (idx.y >= SILU_TAB_N2) r[i] = (r[i] & 0x0000ffffu) | ((uint32_t)f2bf(silu_out_of_table(hi_bf(xb[i]))) << 16);
+            const u16x2 mag = silu_offset2(xb[i]);
+            if (mag.x >= SILU_TAB_HALF) r[i] = (r[i] & 0xffff0000u) | f2bf(silu_out_of_table(lo_bf(xb[i])));
+            if (mag.y >= SILU_TAB_HALF) r[i] = (r[i] & 0x0000ffffu) | ((uint32_t)f2bf(silu_out_of_table(hi_bf(xb[i]))) << 16);
         }
     }
 }
 
 // conv4 + silu of 8 channels of one token, packed as bf16 pairs, and their exact sum of squares
+template <bool FREE = false>
 __device__ __forceinline__ double conv8_silu_packed(const bf16_t* tab, const uint4& x0, const uint4& x1, const uint4& x2,
                                                     const uint4& x3, const uint4 (&wt)[4], uint4& packed) {
     uint32_t r[4];
-    conv8_silu_pairs(tab, x0, x1, x2, x3, wt, r);
+    conv8_silu_pairs<FREE>(tab, x0, x1, x2, x3, wt, r);
     packed = make_uint4(r[0], r[1], r[2], r[3]);
     float u[8];
     unpack8(packed, u);
@@ -315,6 +330,19 @@ __device__ __forceinline__ void rsqrt_rows(const float (&ss)[N], float eps, floa
     }
     const float rv = rsqrt_rn(mine / 128.0f + eps);
     row16_bcast_all<N>(rv, r);
+}
+// r[i] = rsqrt_rn(sum / 128 + eps) of four rows whose exact sums of squares lie spread over the 16 lanes (c) of ss[i].  Each of the first
+// two steps halves the number of values (a lane keeps the row that it will hold and hands over the other), so four sums take 27
+// instructions instead of 48 and end where they are evaluated: lane c holds row c % 4.  The tree is row16_sum_d's, the same bits.
+__device__ __forceinline__ void rsqrt_rows4(const double (&ss)[4], float eps, float (&r)[4], int c) {
+    const bool odd = c & 1, high = c & 2;
+    const double p = (odd ? ss[1] : ss[0]) + dpp_mov_d<0xB1>(odd ? ss[0] : ss[1]);
+    const double q = (odd ? ss[3] : ss[2]) + dpp_mov_d<0xB1>(odd ? ss[2] : ss[3]);
+    double t = (high ? q : p) + dpp_mov_d<0x4E>(high ? p : q);
+    t += dpp_mov_d<0x124>(t);  // row_ror:4
+    t += dpp_mov_d<0x128>(t);  // row_ror:8
+    const float rv = rsqrt_rn((float)t / 128.0f + eps);
+    r[0] = row16_bcast<4>(rv), r[1] = row16_bcast<5>(rv), r[2] = row16_bcast<6>(rv), r[3] = row16_bcast<7>(rv);
 }
 // total over the whole 64-lane wavefront (every lane gets it)
 __device__ __forceinline__ double wave_sum_d(double v) {

@@ -189,6 +189,23 @@ def test_fused_conv_phase_a_equals_separate_kernels(qt, dev, T):
     check_equal("conv tail", to_np(tail), np.concatenate([cs, proj[:, :CD]], axis=0)[-3:])
 
 
+@pytest.mark.parametrize("T", [2, 66, 129])
+def test_phase_a_without_a_silu_table(qt, dev, T):
+    """qt_gdn_phase_a_conv with a null table (every workgroup computes its own) gives the bits of the wrapper's call, in the first
+    chunk (rows from the conv state) and in a last one of one or two rows"""
+    import ctypes
+    proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(700 + T, T)
+    ins = [to_dev(proj, dev, BF16), to_dev(cs, dev, BF16), to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev)]
+    want = qt.gdn_nax._phase_a(*ins)
+    got = [torch.empty_like(t) for t in want]
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = qt._lib.lib().qt_gdn_phase_a_conv(p(ins[0]), p(ins[1]), p(ins[2]), None, p(ins[3]), p(ins[4]), p(got[0]), p(got[1]), p(got[2]), None,
+                                           p(got[3]), p(got[4]), p(got[5]), T, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    for name, a, b in zip(("q", "k", "v", "ops", "U", "gC"), got, want):
+        check_tensors_equal(name, a, b)
+
+
 def test_fused_conv_silu_exhaustive(qt, dev):
     """every finite bf16 value as a conv sum (taps 0, 0, 0, 1) through the fused conv of phase A: the SiLU table and what
     lies outside it, against the restatement of silu_bf16 (mslib.py:21-22)"""
