@@ -119,6 +119,15 @@ long integer(PyObject* o) {                 // int(o)
     }
     return v;
 }
+// a size, offset or stride of a copy: int(o), held at the ends of the range (no tensor is that large, so the range check refuses it)
+long extent(PyObject* o) {
+    PyObject* i = PyNumber_Long(o);
+    if (!i) throw Raised{};
+    int beyond = 0;
+    const long v = PyLong_AsLongAndOverflow(i, &beyond);
+    Py_DECREF(i);
+    return beyond > 0 ? LONG_MAX : beyond < 0 ? LONG_MIN : v;
+}
 float real(PyObject* o) {                   // float(o)
     const double v = PyFloat_AsDouble(o);
     if (v == -1.0 && PyErr_Occurred()) throw Raised{};
@@ -615,8 +624,13 @@ struct Jobs {
         check_layout(d, d.scalar_type(), "dst");
         check_layout(s, s.scalar_type(), "src");
         if (n < 0 || ny < 0 || d0 < 0 || s0 < 0 || ds < 0 || ss < 0) value_error(who + ": negative size, offset or stride");
-        if (n && ny && (d0 + (ny - 1) * ds + n > d.numel() || s0 + (ny - 1) * ss + n > s.numel()))
-            value_error(who + ": the copy leaves the source or the destination");
+        // `ny` rows of n elements from `first` on, `stride` apart, end inside t.  By subtraction and division: the sum
+        // first + (ny - 1) * stride + n of sizes that no tensor has can pass 2^63
+        auto fits = [n, ny](const Tensor& t, long first, long stride) {
+            const long numel = t.numel();
+            return n <= numel && first <= numel - n && (stride == 0 || ny - 1 <= (numel - n - first) / stride);
+        };
+        if (n && ny && !(fits(d, d0, ds) && fits(s, s0, ss))) value_error(who + ": the copy leaves the source or the destination");
         dst.push_back(d.data_ptr());
         src.push_back(s.data_ptr());
         for (long v : {(long)d.element_size(), n, d0, s0, ny, ds, ss}) meta.push_back(v);
@@ -654,12 +668,12 @@ PyObject* blit_batch(PyObject* const* a) {
     for (Py_ssize_t i = 0; i < jobs.size(); i++) {
         const Items t(jobs[i]);
         if (t.size() != 8) value_error("blit_batch: job " + std::to_string(i) + ": expected eight values");
-        j.add(gpu_tensor(t[0], "dst"), gpu_tensor(t[1], "src"), integer(t[2]), integer(t[3]), integer(t[4]), integer(t[5]), integer(t[6]), integer(t[7]));
+        j.add(gpu_tensor(t[0], "dst"), gpu_tensor(t[1], "src"), extent(t[2]), extent(t[3]), extent(t[4]), extent(t[5]), extent(t[6]), extent(t[7]));
     }
     for (Py_ssize_t i = 0; i < zeros.size(); i++) {
         const Items t(zeros[i]);
         if (t.size() != 5) value_error("blit_batch: zeros " + std::to_string(i) + ": expected five values");
-        j.add_zeros(gpu_tensor(t[0], "dst"), integer(t[1]), integer(t[2]), integer(t[3]), integer(t[4]));
+        j.add_zeros(gpu_tensor(t[0], "dst"), extent(t[1]), extent(t[2]), extent(t[3]), extent(t[4]));
     }
     j.run();
     Py_RETURN_NONE;

@@ -135,6 +135,13 @@ int qt_blit(void* dst, const void* src, int elem_size, long n, long d0, long s0,
     return QT_OK;
 }
 
+// the last byte of `ny` rows of n elements of size e, `stride` apart from `first` on, has an offset that fits a long
+static bool ends_in_range(long e, long n, long first, long ny, long stride) {
+    long end;
+    return !__builtin_mul_overflow(ny - 1, stride, &end) && !__builtin_add_overflow(end, first, &end) && !__builtin_add_overflow(end, n, &end) &&
+           !__builtin_mul_overflow(end, e, &end);
+}
+
 // fill: a null source stands for zeros
 static int blit_batch(void* const* dst, const void* const* src, const long* meta, int count, bool fill, hipStream_t stream) {
     if (!dst || !src || !meta) return QT_ERR_NULL;
@@ -147,8 +154,9 @@ static int blit_batch(void* const* dst, const void* const* src, const long* meta
         for (int i = 1; i < 7; i++)
             if (m[i] < 0) return QT_ERR_DIM;
         if (((reinterpret_cast<uintptr_t>(dst[k]) | reinterpret_cast<uintptr_t>(src[k])) & 15u) ||
-            ((m[1] * e) | (m[2] * e) | (m[3] * e) | (m[5] * e) | (m[6] * e)) % 16)
+            (m[1] | m[2] | m[3] | m[5] | m[6]) % (16 / e))
             return QT_ERR_ALIGN;
+        if (m[1] && m[4] && (!ends_in_range(e, m[1], m[2], m[4], m[5]) || (src[k] && !ends_in_range(e, m[1], m[3], m[4], m[6])))) return QT_ERR_DIM;
     }
     for (int k0 = 0; k0 < count; k0 += MAX_JOBS) {
         BlitJobs jobs;
@@ -165,8 +173,9 @@ static int blit_batch(void* const* dst, const void* const* src, const long* meta
             j.dstride = m[5] / per;
             j.sstride = m[6] / per;
             jobs.first_block[k] = (int)total;
-            total += (j.nvec + 1023) / 1024 * j.ny;
-            if (total > 0x7fffffffL) return QT_ERR_DIM;                  // (32 TiB in one call)
+            long units;                                                  // (32 TiB in one call)
+            if (__builtin_mul_overflow((j.nvec + 1023) / 1024, j.ny, &units) || units > 0x7fffffffL - total) return QT_ERR_DIM;
+            total += units;
         }
         for (int k = nj; k < MAX_JOBS; k++) jobs.job[k] = BlitJob{nullptr, nullptr, 0, 0, 0, 0};
         for (int k = nj; k <= MAX_JOBS; k++) jobs.first_block[k] = (int)total;

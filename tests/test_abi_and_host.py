@@ -81,6 +81,19 @@ def test_null_and_dimension_errors_from_the_c_abi():
     assert lib.qt_fused_gemv(ctypes.c_void_p(8), p16, z, p16, 4, 64, 1024, 0, z) == -2
 
 
+@pytest.mark.parametrize("e,n,d0,s0,ny,ds,ss", [
+    (2, 8, 2 ** 63 - 8, 0, 1, 0, 0), (4, 8, 0, 2 ** 61, 1, 0, 0),              # the last byte's offset does not fit 64 bits
+    (2, 8, 0, 0, 65537, 2 ** 48, 0), (2, 8, 0, 0, 65537, 0, 2 ** 48),          # ... nor does the last row's start
+    (4, 2 ** 60, 0, 0, 2 ** 20, 0, 0), (4, 4, 0, 0, 2 ** 31, 0, 0)])           # ... nor does the number of units fit a launch
+def test_batched_copy_refuses_sizes_that_overflow(e, n, d0, s0, ny, ds, ss):
+    import qwen_tailor_amd as qt
+    lib = qt._lib.lib()
+    p = (ctypes.c_void_p * 1)(16)
+    meta = (ctypes.c_long * 7)(e, n, d0, s0, ny, ds, ss)
+    assert lib.qt_blit_batch(p, p, meta, 1, ctypes.c_void_p(0)) == -1
+    assert lib.qt_blit_fill_batch(p, p, meta, 1, ctypes.c_void_p(0)) == -1
+
+
 def test_prefill_attention_split_plan_on_the_host():
     """The key split of the causal prefill attention is planned on the host (no GPU call computes anything here): which launches
     are split, how much workspace they use, and that the bound for a key count covers every launch below it."""

@@ -168,3 +168,29 @@ def test_fill_jobs_between_copies(qt, dev, n, d0, ny, ds):
     if ny:
         with pytest.raises(ValueError):
             qt._lib.host.blit_batch([], [(b, n + 32, d0, ny, ds)])
+
+
+@pytest.mark.parametrize("n,d0,s0,ny,ds,ss", [
+    (8, 2 ** 63 - 8, 0, 1, 0, 0),            # d0 + n passes 2^63: as a 64-bit sum it is negative
+    (8, 0, 2 ** 63 - 8, 1, 0, 0),
+    (8, 0, 0, 65537, 2 ** 48, 0),            # (ny - 1) * dstride is 2^64: as a 64-bit product it is 0
+    (8, 0, 0, 65537, 0, 2 ** 48),
+    (8, 8, 0, 2 ** 62, 4, 0), (2 ** 63 - 8, 0, 0, 1, 0, 0), (2 ** 64, 0, 0, 1, 0, 0), (8, 2 ** 64, 0, 1, 0, 0),
+    (8, 0, 0, 2, 2 ** 64, 0), (8, 64 - 8 + 8, 0, 1, 0, 0), (8, 0, 0, 8, 16, 0)])
+def test_copies_that_leave_their_tensors_are_refused_at_any_size(qt, dev, n, d0, s0, ny, ds, ss):
+    """nothing is launched: every range that ends past its tensor is a ValueError, also one whose end does not fit 64 bits"""
+    dst, src = torch.zeros(64, dtype=BF16, device=dev), torch.ones(64, dtype=BF16, device=dev)
+    with pytest.raises(ValueError, match="leaves"):
+        qt.batch.blit_batch([(dst, src, n, d0, s0, ny, ds, ss)])
+    if not s0 and not ss:
+        with pytest.raises(ValueError, match="leaves"):
+            qt._lib.host.blit_batch([], [(dst, n, d0, ny, ds)])
+    assert not bool(dst.any())
+
+
+def test_copies_that_end_with_their_tensors_are_taken(qt, dev):
+    dst, src = torch.zeros(64, dtype=BF16, device=dev), torch.ones(64, dtype=BF16, device=dev)
+    qt.batch.blit_batch([(dst, src, 8, 8, 0, 4, 16, 0), (dst, src, 0, 2 ** 40, 0, 1, 0, 0), (dst, src, 8, 0, 56, 1, 2 ** 40, 2 ** 40)])
+    want = torch.zeros(8, 8)
+    want[1::2], want[0] = 1, 1
+    assert torch.equal(dst.float().cpu().view(8, 8), want)
