@@ -20,14 +20,14 @@ HV, DK, DV, CD, PW = 16, 128, 128, 6144, 8224
 def deltanet_b(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, rows_per_wg: int = 0):
     """proj [B, 8224] bf16; slots / pos int32 [B] (pos = tokens already in the slot's state).  Returns y [B, 2048] bf16 and
     updates ssm_pool[slot] and the conv buffer (pos&1)^1 of the slot IN PLACE (qwen35/batch.py:128-135)."""
-    return L.host.decode_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, None, 0.0, rows_per_wg)
+    return L.host.decode_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, rows_per_wg)
 
 
 def deltanet_b_gnorm(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, gw, eps=1e-6):
     """deltanet_b followed by gnorm_rows (qwen35/batch.py:128-135, 338-343; the two calls of the reference's decode step,
     batch.py:497-499) in one launch.  Returns the gated-norm output [B, 2048] bf16 (the same bits as the two calls); pools are
     updated in place as by deltanet_b."""
-    return L.host.decode_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, gw, eps, 0)
+    return L.host.decode_step_gnorm(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, gw, eps)
 
 
 def split_size(Lmax: int, B: int = 16) -> int:

@@ -290,26 +290,40 @@ PyObject* gated_norm(PyObject* const* a) {
 }
 
 // ---- recurrent steps ------------------------------------------------------------------------------------------------------
-// decode_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, gw or None, eps, rows_per_wg)
-PyObject* decode_step(PyObject* const* a) {
+struct Step {                               // the operands of a decode step
+    const Tensor &proj, &ssm, &conv, &slots, &pos, &w;
+    Tensor A, dtb;
+    int B, n_slots;
+};
+// (proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos)
+Step step_operands(PyObject* const* a) {
     const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
     const int64_t B = proj.size(0);
     const Tensor& ssm = dev(a[5], F32, "ssm_pool", {ANY, HV, DV, DK});
     const int64_t n_slots = ssm.size(0);
     const Tensor& conv = dev(a[1], BF16, "conv_pool", {n_slots * 2, 3, CD});
     const Tensor &slots = dev(a[6], I32, "slots", {B}), &pos = dev(a[7], I32, "pos", {B}), &w = flat_conv_w(a[2]);
-    const Tensor A = f32(a[3], "A_log", HV), dtb = f32(a[4], "dt_bias", HV);
-    const bool norm = a[8] != Py_None;
-    const Tensor gw = norm ? f32(a[8], "gw", DV) : Tensor();
-    Tensor out = empty({B, HV * DV}, BF16, proj);
-    if (norm)
-        check(qt_gdn_decode_step_gnorm(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
-                                       slots.data_ptr<int>(), pos.data_ptr<int>(), gw.data_ptr<float>(), real(a[9]), out.data_ptr(), dim32(B),
-                                       dim32(n_slots), stream()), "qt_gdn_decode_step_gnorm");
-    else
-        check(qt_gdn_decode_step(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
-                                 slots.data_ptr<int>(), pos.data_ptr<int>(), out.data_ptr(), dim32(B), dim32(n_slots), (int)integer(a[10]), stream()),
-              "qt_gdn_decode_step");
+    return {proj, ssm, conv, slots, pos, w, f32(a[3], "A_log", HV), f32(a[4], "dt_bias", HV), dim32(B), dim32(n_slots)};
+}
+// decode_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, rows_per_wg)
+PyObject* decode_step(PyObject* const* a) {
+    const Step s = step_operands(a);
+    const int rows_per_wg = (int)integer(a[8]);
+    Tensor y = empty({s.proj.size(0), HV * DV}, BF16, s.proj);
+    check(qt_gdn_decode_step(s.proj.data_ptr(), s.conv.data_ptr(), s.w.data_ptr(), s.A.data_ptr<float>(), s.dtb.data_ptr<float>(),
+                             s.ssm.data_ptr<float>(), s.slots.data_ptr<int>(), s.pos.data_ptr<int>(), y.data_ptr(), s.B, s.n_slots, rows_per_wg,
+                             stream()), "qt_gdn_decode_step");
+    return wrap(y);
+}
+// decode_step_gnorm(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, gw, eps)
+PyObject* decode_step_gnorm(PyObject* const* a) {
+    const Step s = step_operands(a);
+    const Tensor gw = f32(a[8], "gw", DV);
+    const float eps = real(a[9]);
+    Tensor out = empty({s.proj.size(0), HV * DV}, BF16, s.proj);
+    check(qt_gdn_decode_step_gnorm(s.proj.data_ptr(), s.conv.data_ptr(), s.w.data_ptr(), s.A.data_ptr<float>(), s.dtb.data_ptr<float>(),
+                                   s.ssm.data_ptr<float>(), s.slots.data_ptr<int>(), s.pos.data_ptr<int>(), gw.data_ptr<float>(), eps,
+                                   out.data_ptr(), s.B, s.n_slots, stream()), "qt_gdn_decode_step_gnorm");
     return wrap(out);
 }
 
@@ -568,26 +582,32 @@ void phase_b_launch(const Records& r, const Snap& s, const Tensor& st, const Ten
                                 s.words.data_ptr<int>(), stream()), "qt_gdn_phase_b");
 }
 
-// phase_b(S or proj, ops, U, gC, state, gw or None, eps): with gw (and proj) the gated norm follows in the same pass
-PyObject* phase_b(PyObject* const* a) {
-    const bool norm = a[5] != Py_None;
-    const Tensor proj = norm ? dev(a[0], BF16, "proj", {ANY, PW}) : Tensor();
-    const int64_t S = norm ? proj.size(0) : integer(a[0]);
-    const Records r{dev(a[1], F16, "Tb"), dev(a[2], F16, "Am"), dev(a[3], F32, "gv")};
-    const int s32 = dim32(S);
-    if (r.ops.numel() * 2 < qt_gdn_chunk_ops_bytes(s32) || r.U.numel() * 2 < qt_gdn_chunk_u_bytes(s32) || r.gC.numel() * 4 < qt_gdn_chunk_gc_bytes(s32))
+Records given_records(PyObject* const* a, int S) {              // (ops, U, gC), of at least S tokens
+    const Records r{dev(a[0], F16, "Tb"), dev(a[1], F16, "Am"), dev(a[2], F32, "gv")};
+    if (r.ops.numel() * 2 < qt_gdn_chunk_ops_bytes(S) || r.U.numel() * 2 < qt_gdn_chunk_u_bytes(S) || r.gC.numel() * 4 < qt_gdn_chunk_gc_bytes(S))
         value_error("phase_b: the phase A records are too small for this many tokens");
+    return r;
+}
+// phase_b(S, ops, U, gC, state)
+PyObject* phase_b(PyObject* const* a) {
+    const int64_t S = integer(a[0]);
+    const Records r = given_records(a + 1, dim32(S));
     const Tensor state = dev(a[4], F32, "state").reshape({1, HV, DV, DK});
-    const Snap& s = snap_buffer(state, qt_gdn_chunk_snap_bytes(s32));
-    Tensor st_out = empty({1, HV, DV, DK}, F32, state), out;
-    if (norm) {
-        const Tensor gw = f32(a[5], "gw", DV);
-        out = empty({S, HV * DV}, BF16, state);
-        phase_b_launch(r, s, state, st_out, &proj, &gw, real(a[6]), out, S);
-    } else {
-        out = empty({S, HV, DV}, BF16, state);
-        phase_b_launch(r, s, state, st_out, nullptr, nullptr, 0.f, out, S);
-    }
+    const Snap& s = snap_buffer(state, qt_gdn_chunk_snap_bytes(dim32(S)));
+    Tensor st_out = empty({1, HV, DV, DK}, F32, state), out = empty({S, HV, DV}, BF16, state);
+    phase_b_launch(r, s, state, st_out, nullptr, nullptr, 0.f, out, S);
+    return wrap({out, st_out});
+}
+// phase_b_norm(proj, ops, U, gC, state, gw, eps): the gated norm follows in the same pass
+PyObject* phase_b_norm(PyObject* const* a) {
+    const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
+    const int64_t S = proj.size(0);
+    const Records r = given_records(a + 1, dim32(S));
+    const Tensor state = dev(a[4], F32, "state").reshape({1, HV, DV, DK}), gw = f32(a[5], "gw", DV);
+    const float eps = real(a[6]);
+    const Snap& s = snap_buffer(state, qt_gdn_chunk_snap_bytes(dim32(S)));
+    Tensor st_out = empty({1, HV, DV, DK}, F32, state), out = empty({S, HV * DV}, BF16, state);
+    phase_b_launch(r, s, state, st_out, &proj, &gw, eps, out, S);
     return wrap({out, st_out});
 }
 
@@ -726,10 +746,12 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define QT_FN(name, fn, n) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(entry<fn, n>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     QT_FN("rms_rows", rms_rows, 4),       QT_FN("fused_gemv", fused_gemv, 7),     QT_FN("gated_norm", gated_norm, 4),
-    QT_FN("decode_step", decode_step, 11), QT_FN("verify_step", verify_step, 11), QT_FN("deltanet", deltanet, 8),
+    QT_FN("decode_step", decode_step, 9), QT_FN("decode_step_gnorm", decode_step_gnorm, 10), QT_FN("verify_step", verify_step, 11),
+    QT_FN("deltanet", deltanet, 8),
     QT_FN("attn_b", attn_b, 10),          QT_FN("attn_layer_b", attn_layer_b, 11), QT_FN("sdpa", sdpa, 3),
     QT_FN("qkv_prep", qkv_prep, 7),       QT_FN("out_gate", out_gate, 2),         QT_FN("conv_prep", conv_prep, 3),
-    QT_FN("phase_a", phase_a, 8),         QT_FN("phase_b", phase_b, 7),           QT_FN("gdn_core", gdn_core, 8),
+    QT_FN("phase_a", phase_a, 8),         QT_FN("phase_b", phase_b, 5),           QT_FN("phase_b_norm", phase_b_norm, 7),
+    QT_FN("gdn_core", gdn_core, 8),
     QT_FN("set_hooks", set_hooks, 2),     QT_FN("blit_batch", blit_batch, 2),     QT_FN("pools_load", pools_load, 12),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_qt_host", "argument checks, allocation and launch of the operators", -1, methods};

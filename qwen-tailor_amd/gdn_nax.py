@@ -127,10 +127,10 @@ def check_status(device=None, sync=True):
 def phase_b(q, k, v, Tb, Am, gv, state, relaxed=True, flags=DEFAULT_FLAGS, tg=None):
     """The serial state recurrence on the outputs of phase A -> y [S,16,128] bf16, new state [1,16,128,128] f32
     (qwen35/gdn_nax.py:404-410).  Tb / Am / gv are the records prep_a (or gdn_chunked's phase A) produced."""
-    return L.host.phase_b(q.shape[0], Tb, Am, gv, state, None, 0.0)
+    return L.host.phase_b(q.shape[0], Tb, Am, gv, state)
 
 
 def phase_b_norm(proj, Tb, Am, gv, state, gw, eps=1e-6):
     """phase_b followed by prefill.gated_norm (qwen35/prefill.py:241-244) in one pass: the outputs never leave the chip
     un-normalised.  proj [S,8224] bf16 supplies z; gw [128].  -> out [S,2048] bf16, new state [1,16,128,128] f32."""
-    return L.host.phase_b(proj, Tb, Am, gv, state, gw, eps)
+    return L.host.phase_b_norm(proj, Tb, Am, gv, state, gw, eps)

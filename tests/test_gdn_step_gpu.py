@@ -443,3 +443,18 @@ def test_deltanet_b_gnorm_equals_two_launches(qt, dev, B):
     check_tensors_equal("conv pool", c2, c1)
     check_tensors_equal("ssm pool", s2, s1)
     check_equal("against the oracle", to_np(got), O.gated_norm(to_np(y), to_np(proj), gw))
+
+
+def test_a_missing_norm_weight_is_refused(qt, dev):
+    """the fused forms without their norm weight: TypeError, nothing launched (not the step without its norm)"""
+    proj, ssm = torch.zeros((2, PW), dtype=BF16, device=dev), torch.ones((3, 16, 128, 128), device=dev)
+    conv, cw = torch.ones((6, 3, CD), dtype=BF16, device=dev), torch.ones((CD, 4), dtype=BF16, device=dev)
+    A, idx = torch.zeros(16, device=dev), torch.tensor([0, 1], dtype=torch.int32, device=dev)
+    with pytest.raises(TypeError, match="gw"):
+        qt.batch.deltanet_b_gnorm(proj, conv, cw, A, A, ssm, idx, idx, None)
+    assert bool((conv == 1).all()) and bool((ssm == 1).all())
+    records = qt.gdn_nax._phase_a(proj, conv[0], cw, A, A, want_qkv=False)[3:]
+    with pytest.raises(TypeError, match="gw"):
+        qt.gdn_nax.phase_b_norm(proj, *records, ssm[:1], None)
+    with pytest.raises(TypeError, match="gw"):
+        qt.prefill.gdn_core(proj, conv[:1], ssm[:1], cw, A, A, None)
