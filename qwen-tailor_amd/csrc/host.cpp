@@ -16,6 +16,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <climits>
 #include <map>
 #include <string>
@@ -107,31 +108,22 @@ const Tensor& flat_conv_w(PyObject* o) {
     return w;
 }
 
-long integer(PyObject* o) {                 // int(o)
-    long v = PyLong_AsLong(o);
-    if (v == -1 && PyErr_Occurred()) {
-        PyErr_Clear();
-        PyObject* i = PyNumber_Long(o);
-        if (!i) throw Raised{};
-        v = PyLong_AsLong(i);
-        Py_DECREF(i);
-        if (v == -1 && PyErr_Occurred()) throw Raised{};
-    }
+long integer(PyObject* o) {                 // an int, or what stands for one (__index__): a float or a string does not
+    const Ref i(PyNumber_Index(o));
+    const long v = PyLong_AsLong(i.o);
+    if (v == -1 && PyErr_Occurred()) throw Raised{};
     return v;
 }
 // a size, offset or stride of a copy: int(o), held at the ends of the range (no tensor is that large, so the range check refuses it)
 long extent(PyObject* o) {
-    PyObject* i = PyNumber_Long(o);
-    if (!i) throw Raised{};
+    const Ref i(PyNumber_Long(o));
     int beyond = 0;
-    const long v = PyLong_AsLongAndOverflow(i, &beyond);
-    Py_DECREF(i);
+    const long v = PyLong_AsLongAndOverflow(i.o, &beyond);
     return beyond > 0 ? LONG_MAX : beyond < 0 ? LONG_MIN : v;
 }
 float real(PyObject* o) {                   // float(o)
-    const double v = PyFloat_AsDouble(o);
-    if (v == -1.0 && PyErr_Occurred()) throw Raised{};
-    return (float)v;
+    const Ref f(PyNumber_Float(o));
+    return (float)PyFloat_AS_DOUBLE(f.o);
 }
 bool truth(PyObject* o) {
     const int v = PyObject_IsTrue(o);
@@ -250,7 +242,7 @@ PyObject* fused_gemv(PyObject* const* a) {
     const int64_t M = x.size(0);
     if (has_nw && has_gnorm) value_error("nw and gnorm are exclusive");
     if (swiglu && has_res) value_error("swiglu and res are exclusive");
-    const float eps = real(a[3]);
+    const float eps = has_nw || has_gnorm ? real(a[3]) : 0.f;    // (without a prologue nothing looks at it)
     if (has_gnorm) {
         const Ref pp(PySequence_GetItem(a[6], 0)), pg(PySequence_GetItem(a[6], 1));
         check_shape(x, "y", {ANY, HV * DV});
@@ -462,7 +454,7 @@ PyObject* qkv_prep(PyObject* const* a) {
     if (M < 1 || R % M) value_error("qkv_prep: M = " + std::to_string(M) + " must divide the number of rows (" + std::to_string(R) + ")");
     const Tensor &pos = dev(a[3], I32, "pos", {R / M}), &qn = dev(a[1], BF16, "q_norm", {256}), &kn = dev(a[2], BF16, "k_norm", {256});
     Tensor q = empty({R, 8, 256}, BF16, qkv), k = empty({R, 2, 256}, BF16, qkv), v = empty({R, 2, 256}, BF16, qkv);
-    const Tensor table = a[6] != Py_None ? rope_table(qkv, integer(a[6]) + 1) : Tensor();
+    const Tensor table = a[6] != Py_None ? rope_table(qkv, std::min(extent(a[6]), 1L << 40) + 1) : Tensor();
     check(qt_attn_qkv_prep_table(qkv.data_ptr(), qn.data_ptr(), kn.data_ptr(), pos.data_ptr<int>(), table.defined() ? table.data_ptr() : nullptr,
                                  table.defined() ? dim32(table.size(0)) : 0, q.data_ptr(), k.data_ptr(), v.data_ptr(), R, dim32(M), real(a[5]), stream()),
           "qt_attn_qkv_prep");
@@ -676,7 +668,7 @@ struct Items {                                                   // the items of
     ~Items() { Py_DECREF(seq); }
     Py_ssize_t size() const { return PySequence_Fast_GET_SIZE(seq); }
     PyObject* operator[](Py_ssize_t i) const {
-        if (i >= size()) value_error("a sequence is shorter than expected");
+        if (i >= size()) throw Error{PyExc_IndexError, "list index out of range"};
         return PySequence_Fast_GET_ITEM(seq, i);
     }
 };
@@ -711,6 +703,7 @@ PyObject* pools_load(PyObject* const* a) {
     }
     for (Py_ssize_t i = 0; i < kv.size(); i++) {
         const Items pair(kv[i]);
+        if (pair.size() != 2) value_error("state: (K, V) pairs expected");
         const Tensor& K = gpu_tensor(pair[0], "src");
         if (K.dim() != 4) value_error("state: K / V are expected as [1, heads, rows, width]");
         const long smax = K.size(2);

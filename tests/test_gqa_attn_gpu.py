@@ -541,3 +541,21 @@ def test_attention_layer_two_launches_equal_the_three_calls(qt, dev, B, M, Lmax,
 def test_attention_layer_config4_two_launches(qt, dev):
     """benchmark config 4's attention half (B = 16 x M = 4, ragged lengths in [1024, 8192]) through the layer form"""
     _layer_case(qt, dev, 1004, 16, 4, 8192 + 8, 1024, 8192)
+
+
+@pytest.mark.parametrize("bad", [2.0, "2", None])
+def test_counts_are_integers(qt, dev, bad):
+    """a number of tokens, a split size or a slot that is no integer is a TypeError, not cut to one; integers of any kind are taken"""
+    q, k = torch.ones((4, 8, 256), dtype=BF16, device=dev), torch.ones((4, 2, 256), dtype=BF16, device=dev)
+    K, idx = torch.ones((3, 2, 32, 256), dtype=BF16, device=dev), torch.tensor([0, 1], dtype=torch.int32, device=dev)
+    qkv, w = torch.ones((4, 5120), dtype=BF16, device=dev), torch.ones(256, dtype=BF16, device=dev)
+    for M in (2, np.int64(2), torch.tensor(2)):
+        qt.batch.attn_b(q, k, k, K, K.clone(), idx, idx, M)
+        qt.attention.qkv_prep(qkv, w, w, idx, M, max_pos="7")
+    for call in (lambda: qt.batch.attn_b(q, k, k, K, K.clone(), idx, idx, bad), lambda: qt.attention.qkv_prep(qkv, w, w, idx, bad),
+                 lambda: qt.batch.attn_layer_b(qkv, w, w, K, K.clone(), idx, idx, bad)):
+        with pytest.raises(TypeError):
+            call()
+    if bad is not None:                                          # (None: the default split)
+        with pytest.raises(TypeError):
+            qt.batch.attn_b(q, k, k, K, K.clone(), idx, idx, 2, split=bad)

@@ -213,3 +213,12 @@ def test_row_blocks_are_taken_in_any_shape(qt, dev):
     want = qt.prefill.gated_norm(y, proj, gw)
     assert torch.equal(qt.prefill.gated_norm(y.reshape(48, 128), proj, gw), want)
     assert torch.equal(qt.prefill.gated_norm(y.reshape(3, 16, 128), proj, gw), want)
+
+
+def test_eps_is_what_float_takes_and_only_where_it_is_used(qt, dev):
+    W, x = torch.ones((64, 1024), dtype=BF16, device=dev), torch.ones((2, 1024), dtype=BF16, device=dev)
+    want = qt.kernels.fused_gemv(W, x, nw=x[0], eps=0.5)
+    check_tensors_equal("eps as text", qt.kernels.fused_gemv(W, x, nw=x[0], eps="0.5"), want)
+    check_tensors_equal("no prologue", qt.kernels.fused_gemv(W, x, eps=None), qt.kernels.fused_gemv(W, x))
+    with pytest.raises(TypeError):
+        qt.kernels.fused_gemv(W, x, nw=x[0], eps=None)

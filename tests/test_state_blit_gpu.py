@@ -194,3 +194,18 @@ def test_copies_that_end_with_their_tensors_are_taken(qt, dev):
     want = torch.zeros(8, 8)
     want[1::2], want[0] = 1, 1
     assert torch.equal(dst.float().cpu().view(8, 8), want)
+
+
+def test_states_that_do_not_fit_the_pools_are_refused(qt, dev):
+    cfg = _small_cfg(qt)
+    P = qt.batch.Pools(cfg, 2, 16, device=dev)
+    st = {"conv": [torch.ones((1, 3, CD), dtype=BF16, device=dev) for _ in P.conv], "ssm": [torch.ones((1, HV, DV, DK), device=dev) for _ in P.ssm],
+          "kv": [(torch.ones((1, 2, 8, 256), dtype=BF16, device=dev),) * 2 for _ in P.K]}
+    for error, change, slot, pos in ((TypeError, {}, 1, 5.0), (IndexError, {"conv": st["conv"] * 2, "ssm": st["ssm"] * 2}, 1, 5),
+                                     (IndexError, {"kv": st["kv"] * 2}, 1, 5), (ValueError, {"kv": [(st["kv"][0][0],)]}, 1, 5),
+                                     (ValueError, {}, 1, 9), (AssertionError, {}, 1, 17), (AssertionError, {}, 2, 5)):
+        with pytest.raises(error):
+            P.load(slot, dict(st, **change), pos)
+    assert not any(bool(t.any()) for t in P.conv + P.ssm + P.K + P.V)
+    P.load(np.int32(1), st, np.int64(5))
+    assert all(bool((t[1, :, :5] == 1).all()) for t in P.K + P.V)
