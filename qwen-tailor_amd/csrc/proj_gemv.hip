@@ -214,13 +214,16 @@ __device__ __forceinline__ void quad_transpose(u32x4& a, u32x4& b, u32x4& c, u32
 // to 1.2 us (32 rows x 64 features) instead of a launch of its own at 2.6 us.
 // W: a load takes 256 contiguous bytes of four features, 64 of them in each quad of lanes (register j of lane (g, h, c): feature
 // 4 h + j, elements 32 g + 8 c ..), and quad_transpose turns four such loads into the MFMA layout: feature n in lane (n, g),
-// elements 32 g + 8 r .. in register r.  The x fragments are read from LDS in the same enumeration of k.  Workgroups start at
-// different steps of the row (rot), so that they do not all ask the same memory channels first.
+// elements 32 g + 8 r .. in register r.  The x fragments are read from LDS in the same enumeration of k.  Which wavefront takes
+// which quarter differs from workgroup to workgroup, so that they do not all ask the same memory channels first; a quarter's
+// product and the sum of the four do not depend on it, so a row has the same bits in every place of a batch of any size.  (Letting
+// half of the workgroups begin with their quarter's second step would take another 3 % off 16 rows at N = 5120 and 7168, but the order of
+// summation would follow; with the order kept by exchanging registers, in a branch, or by summing the steps apart it costs as much or more.)
 // Two of the launch's shapes do not divide: with `extra` > 0 the first `extra` tiles take one block more, from the end of
 // N (the 514 blocks of N = 8224 are 256 x 2 + 2; a 257th workgroup would take a CU twice as long as the others).
 // Tile sizes (us in a HIP graph, rms prologue included, N = 8224 / 7168 swiglu / 5120; before: rms_rows and the product as two
-// launches, x fragments and W loaded in MFMA shape): 1 row 6.2 / 5.7 / 4.9 (8.5 / 7.9 / 6.9), 16 rows 6.3 / 5.7 / 4.9 (9.1 / 8.5 /
-// 7.9), 32 rows 7.5 / 7.1 / 6.2 (9.9 / 9.8 / 9.0), 64 rows 8.9 / 8.6 / 7.8 (11.9 / 13.0 / 11.3), 80 rows 10.1 / 9.8 / 9.1 (20.2 /
+// launches, x fragments and W loaded in MFMA shape): 1 row 6.3 / 5.7 / 5.1 (8.5 / 7.9 / 6.9), 16 rows 6.4 / 5.9 / 5.3 (9.1 / 8.5 /
+// 7.9), 32 rows 7.2 / 6.7 / 6.1 (9.9 / 9.8 / 9.0), 64 rows 9.0 / 8.4 / 7.9 (11.9 / 13.0 / 11.3), 80 rows 10.6 / 9.8 / 7.9 (20.2 /
 // 19.5 / 14.2).  An empty kernel takes 1.9 us there; what is left at 64 rows is the 64 KiB of rows and 128 KiB of W a CU pulls.
 template <int RB, int FB, bool RMS, int EPI>
 __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
@@ -233,7 +236,7 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
     // the row groups of a tile sit on one XCD (workgroups are dealt to the eight XCDs in turn) and share its W through the L2
     const int s = blockIdx.x >> 3, grp = s % groups, tile = (s / groups) * 8 + (blockIdx.x & 7);
     if (tile >= tiles) return;
-    const int q = w & 3, half = w >> 2, m0 = grp * R, nb0 = tile * 16 * NB, nx = 16 * (tiles * NB + tile), rot = s & 7;
+    const int q = (w + s) & 3, half = w >> 2, m0 = grp * R, nb0 = tile * 16 * NB, nx = 16 * (tiles * NB + tile);
     const bool has_x = tile < extra && half == 0;
     u32x4 xr[RW][2], wn[2];
 #pragma unroll
@@ -251,7 +254,7 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
 #pragma unroll
         for (int i = 0; i < 8; i++)
             d[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
-                W + (size_t)min(f0 + (n & 12) + (i & 3), N - 1) * XK + 128 * ((q + (i & 4) + rot) & 7) + 32 * g + 8 * (n & 3)));
+                W + (size_t)min(f0 + (n & 12) + (i & 3), N - 1) * XK + 128 * (2 * q + (i >> 2)) + 32 * g + 8 * (n & 3)));
     };
 #pragma unroll
     for (int f = 0; f < FB; f++) w_load(a[f], nb0 + 16 * (half * FB + f));
@@ -294,7 +297,7 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
         for (int rb = 0; rb < RB; rb++) acc[f][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
     const bool odd = n & 1, high = n & 2;
     auto x_frag = [&](int i, int rb) {
-        return *reinterpret_cast<const u32x4*>(x_s + (16 * rb + n) * XK + 8 * ((16 * ((q + (i & 4) + rot) & 7) + 4 * g + (i & 3)) ^ n));
+        return *reinterpret_cast<const u32x4*>(x_s + (16 * rb + n) * XK + 8 * ((16 * (2 * q + (i >> 2)) + 4 * g + (i & 3)) ^ n));
     };
     auto mma = [](const u32x4& av, const u32x4& bv, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv), c, 0, 0, 0);

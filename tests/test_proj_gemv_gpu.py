@@ -222,3 +222,21 @@ def test_eps_is_what_float_takes_and_only_where_it_is_used(qt, dev):
     check_tensors_equal("no prologue", qt.kernels.fused_gemv(W, x, eps=None), qt.kernels.fused_gemv(W, x))
     with pytest.raises(TypeError):
         qt.kernels.fused_gemv(W, x, nw=x[0], eps=None)
+
+
+# the model's projections; row counts at the edges of every row block and of the rules that choose a kernel or a tile
+@pytest.mark.parametrize("N,K,kind", [(8224, 1024, "rms"), (7168, 1024, "swiglu"), (5120, 1024, "rms"), (1024, 2048, "add"), (1024, 3584, "add")])
+def test_a_row_has_the_same_bits_wherever_it_stands(qt, dev, N, K, kind):
+    """real-valued rows, so that another order of summation shows: a row's product depends neither on its place in the batch nor (up
+    to 64 rows, the wide projections at any number) on how many rows there are"""
+    g = torch.Generator().manual_seed(N + K)
+    M = 264 if K == 1024 else 64
+    W = (torch.randn((N, K), generator=g) * K ** -0.5).to(BF16).to(dev)
+    x, nw = torch.randn((M, K), generator=g).to(BF16).to(dev), (1 + 0.1 * torch.randn(K, generator=g)).to(BF16).to(dev)
+    res = torch.randn((M, N), generator=g).to(BF16).to(dev)
+    f = lambda i: qt.kernels.fused_gemv(W, x[i], nw=nw if kind != "add" else None, res=res[i] if kind == "add" else None, swiglu=kind == "swiglu")
+    want = f(torch.arange(M, device=dev))
+    for m in (1, 3, 5, 16, 17, 32, 33, 48, 49, 64, 65, 80, 96, 97, 128, 129, 200):
+        if m <= M:
+            i = torch.randperm(M, generator=g)[:m].to(dev)
+            check_tensors_equal(f"{m} rows", f(i), want[i])
