@@ -211,7 +211,8 @@ int qt_attn_out_gate(const void* o, const void* qkv, void* out, long R, qt_strea
 int qt_rms_rows(const void* x, const void* nw, void* y, int M, int K, float eps, qt_stream_t stream);
 int qt_fused_gemv(const void* W, const void* x, const void* res, void* y, int M, int N, int K, int epilogue, qt_stream_t stream);
 /* qt_rms_rows followed by qt_fused_gemv in one launch, for the shapes where that is the faster form (K = 1024, N >= 4096 and a
- * multiple of 4, at most 96 rows, y and res aligned to 8 bytes); any other shape returns -4 with nothing launched, and the caller
+ * multiple of 4, at most 96 rows, from 17 rows on no more features than a workgroup per CU takes, y and res aligned to 8 bytes);
+ * any other shape returns -4 with nothing launched, and the caller
  * makes the two calls.  The normalised rows have the same bits as qt_rms_rows' and are not stored. */
 int qt_fused_gemv_rms(const void* W, const void* x, const void* nw, float eps, const void* res, void* y, int M, int N, int K,
                       int epilogue, qt_stream_t stream);

@@ -455,12 +455,22 @@ struct gemv_args {
     hipStream_t stream;
 };
 
+// the workgroups of a launch: `tiles` of 32 FB features, of which the first `extra` take one block of 16 more, times `groups` of 16 RB rows
+struct RowsGrid {
+    int groups, tiles, extra;
+    RowsGrid(const gemv_args& p, int cus, int RB, int FB) {
+        groups = (p.M + 16 * RB - 1) / (16 * RB), extra = 0;
+        const int blocks = (p.N + 15) / 16, per_cu = cus / groups > 0 ? cus / groups : 1;
+        tiles = (blocks + 2 * FB - 1) / (2 * FB);
+        // a few blocks more than a whole tile per CU: the first tiles take one each instead of a workgroup of their own
+        if (blocks > per_cu * 2 * FB && blocks - per_cu * 2 * FB <= per_cu / 16) tiles = per_cu, extra = blocks - per_cu * 2 * FB;
+    }
+    bool one_round(int cus) const { return (long)tiles * groups <= cus; }        // a workgroup per CU at most
+};
 template <int RB, int FB, bool RMS>
 void launch_rows(const gemv_args& p, int cus) {
-    const int groups = (p.M + 16 * RB - 1) / (16 * RB), blocks = (p.N + 15) / 16, per_cu = cus / groups > 0 ? cus / groups : 1;
-    int tiles = (blocks + 2 * FB - 1) / (2 * FB), extra = 0;
-    // a few blocks more than a whole tile per CU: the first tiles take one each instead of a workgroup of their own
-    if (blocks > per_cu * 2 * FB && blocks - per_cu * 2 * FB <= per_cu / 16) tiles = per_cu, extra = blocks - per_cu * 2 * FB;
+    const RowsGrid r(p, cus, RB, FB);
+    const int groups = r.groups, tiles = r.tiles, extra = r.extra;
     const dim3 grid((tiles + 7) / 8 * 8 * groups), block(512);
     if (p.epi == EPI_NONE)
         hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_NONE>), grid, block, 0, p.stream, p.W, p.x, p.nw, p.eps, p.res, p.y, p.M, p.N, groups, tiles, extra);
@@ -475,27 +485,50 @@ inline bool rows_shape(const gemv_args& p) {
 }
 constexpr int RMS_ROWS_MAX = 96;       // most rows with the prologue fused in: beyond, the rows are normalised too often
 // Tile by rows.  Up to 96 rows: the smallest tile that leaves at most one workgroup per CU (32 features as long as one row
-// group holds the batch, then 64).  Beyond 96 rows there is no such tile; 64 x 64 up to 128 rows, then 32 x 32 (N = 8224 /
-// 7168 / 5120 at 128 rows 9.9 / 9.6 / 8.6 us against 20.8 / 19.7 / 11.7 before, at 256 rows 19.6 / 18.4 / 13.0 against 30.8 / 28.3 /
-// 21.5).
+// group holds the batch, then 64).  Where none does, W is what costs, and one row group is better than two that read it twice:
+// 64 features x 48 or 64 rows (N = 9216 / 32768 / 151936 at 48 rows 8.5 / 19.2 / 82 us, 11.3 / 24.4 / 102 with 32 features; at 64 rows 9.1 /
+// 20.8 / 88, 11.9 / 25.7 / 108 with two groups of 32 rows); up to 32 rows 32 features again, whose two workgroups per CU overlap (N =
+// 32768 / 151936 16 / 61 us at 17 rows, 17.3 / 68 with 64).  Beyond 96 rows 64 x 64 up to 128 rows, then 32 x 32 (N = 8224 / 7168 / 5120 at
+// 128 rows 13.1 / 12.5 / 11.6 us with the rms launch, 256 23 / 21.4 / 16.8, 4096 351 / 301 / 221; 23.7 / 22.6 / 14.7, 33.8 / 31.5 / 24.7 and 429 / 325 / 274
+// with the 64-row tiles of general loads before).
+// The rms prologue: false (nothing launched) where more than one workgroup per CU would normalise the same rows, which then cost
+// more than the launch they save (from 17 rows on; N = 32768 / 151936 at 64 rows 29 / 124 us fused, 24 / 91 in two launches).
 template <bool RMS>
-void launch_rows_any(const gemv_args& p, int cus) {
-    if (p.M <= 16)
+bool launch_rows_any(const gemv_args& p, int cus) {
+    auto one_round = [&](int RB, int FB) { return RowsGrid(p, cus, RB, FB).one_round(cus); };
+    if (p.M <= 16) {
         launch_rows<1, 1, RMS>(p, cus);
-    else if (p.M <= 32)
-        launch_rows<2, 1, RMS>(p, cus);
-    else if (p.M <= 48)
+        return true;
+    }
+    if (p.M <= 32) {
+        if (!one_round(2, 1) && one_round(2, 2))
+            launch_rows<2, 2, RMS>(p, cus);
+        else if (!RMS || one_round(2, 1))
+            launch_rows<2, 1, RMS>(p, cus);
+        else
+            return false;
+        return true;
+    }
+    if (p.M <= 48 && one_round(3, 1)) {
         launch_rows<3, 1, RMS>(p, cus);
-    else if (p.M <= 64 || (p.M <= 96 && ((p.N + 63) / 64) * 3 <= cus))
+        return true;
+    }
+    if (p.M > 48 && p.M <= 96 && one_round(2, 2)) {
         launch_rows<2, 2, RMS>(p, cus);
-    else if (p.M <= 96)
+        return true;
+    }
+    if ((p.M <= 48 || (p.M > 64 && p.M <= 96)) && (!RMS || one_round(3, 2))) {
         launch_rows<3, 2, RMS>(p, cus);
-    else if constexpr (!RMS) {
+        return true;
+    }
+    if constexpr (!RMS) {
         if (p.M <= 128)
             launch_rows<4, 2, false>(p, cus);
         else
             launch_rows<2, 1, false>(p, cus);
+        return true;
     }
+    return false;
 }
 
 template <int NWV, int KS, int FG, int MG>
@@ -630,7 +663,7 @@ int qt_fused_gemv_rms(const void* W, const void* x, const void* nw, float eps, c
     if (rc != QT_OK || M == 0) return rc;
     if (!nw) return QT_ERR_NULL;
     if (!rows_shape(p) || M > RMS_ROWS_MAX) return QT_ERR_UNSUPPORTED;
-    launch_rows_any<true>(p, cu_count());
+    if (!launch_rows_any<true>(p, cu_count())) return QT_ERR_UNSUPPORTED;
     QT_CHECK_LAUNCH();
     return QT_OK;
 }

@@ -114,6 +114,19 @@ def test_wide_projection_exact_and_any_output_alignment(qt, dev, M, N, epi):
     (1, 4096, 0), (1, 8224, 2), (15, 4100, 0), (16, 8224, 1), (17, 5132, 0), (32, 8224, 2), (33, 4100, 1), (48, 8224, 0), (49, 8224, 1),
     (64, 5132, 2), (65, 4100, 0), (80, 8224, 1), (96, 7168, 2), (97, 8224, 0), (128, 5132, 1), (129, 4096, 0), (257, 4100, 2)])
 def test_wide_projection_tiles_and_fused_rms_prologue(qt, dev, M, N, epi):
+    _check_wide(qt, dev, M, N, epi)
+
+
+# the last N of a tile that leaves a workgroup per CU and the first beyond it (256 CUs x 32 or 64 features + one more block for a
+# sixteenth of the CUs), by rows; beyond it the rms prologue is a launch of its own from 17 rows on
+@pytest.mark.parametrize("M,N,epi", [
+    (16, 8452, 0), (17, 8448, 0), (17, 8452, 1), (32, 16384, 2), (32, 16640, 0), (32, 16644, 1), (33, 8448, 2), (48, 8452, 0), (40, 16640, 1),
+    (48, 16644, 2), (49, 8320, 0), (64, 8324, 2), (50, 16644, 1), (65, 5520, 0), (96, 5524, 2), (96, 8320, 1), (66, 8324, 0)])
+def test_wide_projection_beyond_a_workgroup_per_cu(qt, dev, M, N, epi):
+    _check_wide(qt, dev, M, N, epi)
+
+
+def _check_wide(qt, dev, M, N, epi):
     """exact on small integers (every order of summation gives the same bits); with the rms prologue, in one launch up to 96 rows,
     the bits of the two calls"""
     g = torch.Generator().manual_seed(M * 5 + N + epi)
