@@ -42,11 +42,12 @@ struct BlitJobs {
 };
 // One flat space of (job, row, 1024-vector block) units of 16 KiB, walked with a grid stride: every workgroup moves the same
 // number of units whatever the mix of job sizes, and asks for its next unit's vectors before it stores the current one's.
-// What bounds it: HBM.  Loads are nontemporal (a source is read once), stores are not: the lines collect in the L2s and leave
-// in larger bursts, and the copy that follows (an admission copies cache -> fresh state -> slot) reads what is still on the chip.
-// Rows of zeros are a job of their own: copied from a block of zeros they cost the reads.  The two copies of an admission, us, all
-// nontemporal and zeros copied -> now: 300 rows into 512 23.5 -> 20.5, 300 into 4096 35.2 -> 24.9, 2048 into 4096 39.8 -> 34.6
-// (5.9 TB/s of reads and writes), 4000 into 4096 53.4 -> 45.4; plain loads 20 / 29 / 42 / 53, 16 workgroups per CU 20 / 25 / 37 / 47.
+// What bounds it: HBM; loads and stores are nontemporal (everything is touched once).  Rows of zeros are a job of their own: copied from a
+// block of zeros they cost the reads.  Plain stores leave lines in the L2s for a copy that follows, which pays only where it follows at
+// once and both are large, and costs every other copy a quarter of its rate: a checkpoint / a slot load of 2048 rows 17.0 / 17.5 us
+// nontemporal, 18.6 / 19.1 plain; a restore into as many rows and its load 33.3 (17.8 at 64 rows into 512) both nontemporal, 30.7 (20.9)
+// both plain, 35.4 (22.2) the restore alone plain.  The two copies of an admission, us, zeros copied -> filled: 300 rows into 512 25.0 ->
+// 19.9, 300 into 4096 36.8 -> 26.8, 2048 into 4096 40.1 -> 37.3, 4000 into 4096 55.5 -> 50.0.
 __global__ __launch_bounds__(256) void blit_batch_kernel(const BlitJobs jobs, int njobs) {
     const int total = jobs.first_block[njobs];
     auto locate = [&](int b, const u32x4*& s, u32x4*& d, long& left) {
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(256) void blit_batch_kernel(const BlitJobs jobs, in
         }
 #pragma unroll
         for (int k = 0; k < 4; k++)
-            if (k * 256 < left) d[k * 256] = v[k];
+            if (k * 256 < left) __builtin_nontemporal_store(v[k], d + k * 256);
         if (nb >= total) break;
         b = nb, d = d2, left = left2;
         v[0] = v2[0], v[1] = v2[1], v[2] = v2[2], v[3] = v2[3];
