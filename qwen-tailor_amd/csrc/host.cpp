@@ -13,6 +13,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -135,6 +136,7 @@ Tensor empty(at::IntArrayRef size, ScalarType dtype, const Tensor& like) {
     return Tensor(at::detail::empty_cuda(size, dtype, like.device(), std::nullopt));
 }
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 const char* code_text(int rc) {
     switch (rc) {
         case -1: return "bad dimension";
@@ -181,28 +183,32 @@ const Tensor& workspace(int purpose, const Tensor& like, long bytes, long first)
 }
 constexpr long WS_FIRST = 32 << 20;         // attn_b: enough for 256 sequences x 4 rows
 
-const Tensor& silu_table(const Tensor& like) {
+// A table of constants per device, written by a kernel on whichever stream asks first.  It is handed to other streams and kept only
+// once it has been written: the first use waits for its stream (once per device, and when a table grows).  While a HIP graph is
+// being captured nothing has run, and nothing may be waited for: the table then belongs to the graph, whose replays write it, and
+// is not kept.  need: the rows that the caller asks for.
+template <typename Build>
+Tensor table(std::map<int, Tensor>& m, const Tensor& like, int64_t need, std::initializer_list<int64_t> shape, ScalarType dtype, Build build) {
+    const int device = like.device().index();
+    if (const auto it = m.find(device); it != m.end() && it->second.size(0) >= need) return it->second;
+    Tensor t = empty(shape, dtype, like);
+    build(t);
+    if (capturing()) return t;
+    c10::hip::getCurrentHIPStream().synchronize();
+    Tensor& kept = m[device];
+    if (kept.defined()) retired().push_back(kept);
+    return kept = t;
+}
+Tensor silu_table(const Tensor& like) {
     static auto* m = new std::map<int, Tensor>;
-    Tensor& t = (*m)[(int)like.device().index()];
-    if (!t.defined()) {
-        Tensor n = empty({qt_silu_table_bytes() / 2}, BF16, like);
-        check(qt_silu_table_build(n.data_ptr(), stream()), "qt_silu_table_build");
-        t = n;
-    }
-    return t;
+    return table(*m, like, 0, {qt_silu_table_bytes() / 2}, BF16,
+                 [](const Tensor& t) { check(qt_silu_table_build(t.data_ptr(), stream()), "qt_silu_table_build"); });
 }
 // the (cos, sin) pairs of the rotary embedding for positions 0 .. n_pos - 1; grown in steps of 16384 positions
-const Tensor& rope_table(const Tensor& like, int64_t n_pos) {
+Tensor rope_table(const Tensor& like, int64_t n_pos) {
     static auto* m = new std::map<int, Tensor>;
-    Tensor& t = (*m)[(int)like.device().index()];
-    if (!t.defined() || t.size(0) < n_pos) {
-        const int64_t n = (std::max<int64_t>(n_pos, 1) + 16383) / 16384 * 16384;
-        Tensor grown = empty({n, 32, 2}, F32, like);
-        check(qt_rope_table_build(grown.data_ptr(), dim32(n), stream()), "qt_rope_table_build");
-        if (t.defined()) retired().push_back(t);
-        t = grown;
-    }
-    return t;
+    return table(*m, like, n_pos, {(std::max<int64_t>(n_pos, 1) + 16383) / 16384 * 16384, 32, 2}, F32,
+                 [](const Tensor& t) { check(qt_rope_table_build(t.data_ptr(), dim32(t.size(0)), stream()), "qt_rope_table_build"); });
 }
 
 // ---- projections ----------------------------------------------------------------------------------------------------------
@@ -401,7 +407,7 @@ PyObject* attn_layer_b(PyObject* const* a) {
     const Pool p = kv_pool(a[3], a[4], a[5], a[6], B);
     const long CH = integer(a[9]);
     const Tensor ws = attn_scratch(a[10], qkv, B, M, p.Lmax, CH, "attn_layer_b");
-    const Tensor& table = rope_table(qkv, p.Lmax);
+    const Tensor table = rope_table(qkv, p.Lmax);
     Tensor out = empty({R, 2048}, BF16, qkv);
     check(qt_gqa_attn_layer_decode(qkv.data_ptr(), qn.data_ptr(), kn.data_ptr(), table.data_ptr(), dim32(table.size(0)), p.K.data_ptr(), p.V.data_ptr(),
                                    p.slots.data_ptr<int>(), p.pos.data_ptr<int>(), out.data_ptr(), ws.data_ptr(), ws.numel(), dim32(B), dim32(M),

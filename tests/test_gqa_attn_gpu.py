@@ -559,3 +559,54 @@ def test_counts_are_integers(qt, dev, bad):
     if bad is not None:                                          # (None: the default split)
         with pytest.raises(TypeError):
             qt.batch.attn_b(q, k, k, K, K.clone(), idx, idx, 2, split=bad)
+
+
+def _prep_at(qt, dev, top, seed=7):
+    """qkv rows at positions top - 3 .. top and the call on them, with a given bound of the positions (None: no table)"""
+    rng = np.random.default_rng(seed)
+    qkv, w = to_dev(bf(rng.standard_normal((4, 5120))), dev, BF16), to_dev(bf(1 + 0.1 * rng.standard_normal(256)), dev, BF16)
+    pos = torch.tensor([top - 3], dtype=torch.int32, device=dev)
+    return lambda max_pos: qt.attention.qkv_prep(qkv, w, w, pos, 4, max_pos=max_pos)
+
+
+def test_a_grown_rotary_table_is_ready_for_every_stream(qt, dev):
+    """the table grows on a stream that is busy for a while and is used on another one at once: the second call must not read it
+    before it has been written"""
+    top = 400_000                                                 # (longer than any other test's table)
+    f = _prep_at(qt, dev, top)
+    want = f(None)
+    a = torch.randn((4096, 4096), device=dev)
+    busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        for _ in range(40):
+            a = (a @ a).clamp_(-1, 1)
+        first = f(top)
+    with torch.cuda.stream(other):
+        second = f(top)
+    torch.cuda.synchronize()
+    for got in (first, second):
+        for name, x, y in zip("qkv", got, want):
+            check_tensors_equal(name, x, y)
+
+
+def test_a_rotary_table_that_grows_under_capture_belongs_to_the_graph(qt, dev):
+    """the call is captured before any table is that long: an eager call ahead of the first replay finds a written table, and every
+    replay gives the eager bits"""
+    top = 600_000
+    f = _prep_at(qt, dev, top, 8)
+    want = f(None)
+    side, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=side):
+        got = f(top)
+    eager = f(top)
+    for i in range(3):
+        torch.cuda.synchronize()
+        for t in got:
+            t.fill_(0)
+        g.replay()
+        torch.cuda.synchronize()
+        for name, x, y, z in zip("qkv", got, want, eager):
+            check_tensors_equal(f"{name}, replay {i}", x, y)
+            check_tensors_equal(f"{name}, eager", z, y)
