@@ -170,9 +170,12 @@ std::vector<Tensor>& retired() {
     return *v;
 }
 // Scratch memory for a kernel's partial results (the C ABI never allocates): one buffer per (purpose, device, stream), because
-// launches on different streams may overlap.  `first`: size of the first allocation, so that growth is rare.
+// launches on different streams may overlap.  `first`: size of the first allocation, so that growth is rare.  Under HIP graph capture
+// it is memory of the graph, free for the next call once this one has been recorded: graphs captured on one stream may be replayed
+// side by side, and beside eager calls.
 enum Purpose { ATTN_B, PREFILL_ATTENTION };
-const Tensor& workspace(int purpose, const Tensor& like, long bytes, long first) {
+Tensor workspace(int purpose, const Tensor& like, long bytes, long first) {
+    if (capturing()) return empty({bytes}, U8, like);
     static auto* m = new std::map<std::tuple<int, int, void*>, Tensor>;
     Tensor& buf = (*m)[{purpose, (int)like.device().index(), stream()}];
     if (!buf.defined() || buf.numel() < bytes) {
@@ -447,8 +450,8 @@ PyObject* sdpa(PyObject* const* a) {
     }
     // launches that would leave half of the CUs idle are split along the keys; their parts meet in a workspace
     const long bytes = qt_gqa_prefill_workspace_bytes_for(dim32(S), dim32(L), dim32(L - S));
-    void* ws = bytes > 0 ? workspace(PREFILL_ATTENTION, q, bytes, 0).data_ptr() : nullptr;
-    check(qt_gqa_prefill_causal_strided(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), ws, bytes > 0 ? bytes : 0, dim32(S), dim32(L),
+    const Tensor ws = bytes > 0 ? workspace(PREFILL_ATTENTION, q, bytes, 0) : Tensor();
+    check(qt_gqa_prefill_causal_strided(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), bytes > 0 ? ws.data_ptr() : nullptr, std::max(bytes, 0L), dim32(S), dim32(L),
                                         dim32(L - S), head_stride, row_stride, k.stride(1), stream()), "qt_gqa_prefill_causal");
     return wrap(out);
 }
@@ -542,35 +545,39 @@ PyObject* phase_a(PyObject* const* a) {
 
 // The buffer between phase B's chain and output workgroups and the host words its failures are reported in, per (device,
 // stream).  gdn_nax makes them (it owns the caches that a caller can look at): snap_provider(device index, bytes) -> (buffer,
-// pinned int32 tensor); failed(device index) raises what the words say and resets them.
-PyObject *snap_provider = nullptr, *snap_failed = nullptr;
+// pinned int32 tensor); words_provider(device index) -> the words alone; failed(device index) raises what the words say and
+// resets them.
+PyObject *snap_provider = nullptr, *words_provider = nullptr, *snap_failed = nullptr;
 struct Snap {
     Tensor buf, words;
 };
-const Snap& snap_buffer(const Tensor& like, long bytes) {
+constexpr int64_t ONE_LAUNCH_TOKENS = 64 * 64 - 63;              // (FUSED_MIN_CHUNKS of gdn_chunked.hip) from here on the flag area is read
+Snap snap_buffer(const Tensor& like, int64_t S) {
+    const long bytes = qt_gdn_chunk_snap_bytes(dim32(S));
+    const int device = like.device().index();
+    if (!snap_provider) throw Error{PyExc_RuntimeError, "gdn_nax is not imported"};
+    if (capturing()) {                                           // memory of the graph, see workspace(); its replays clear the flag area
+        const Ref words(PyObject_CallFunction(words_provider, "i", device));
+        Snap s{empty({bytes / 2}, F16, like), THPVariable_Unpack(words.o)};
+        if (S >= ONE_LAUNCH_TOKENS) s.buf.narrow(0, 0, qt_gdn_chunk_snap_bytes(0) / 2).zero_();
+        return s;
+    }
     static auto* m = new std::map<std::pair<int, void*>, Snap>;
-    Snap& s = (*m)[{(int)like.device().index(), stream()}];
+    Snap& s = (*m)[{device, stream()}];
     if (!s.buf.defined() || s.buf.numel() * 2 < bytes) {
-        if (!snap_provider) throw Error{PyExc_RuntimeError, "gdn_nax is not imported"};
-        PyObject* r = PyObject_CallFunction(snap_provider, "il", (int)like.device().index(), bytes);
-        if (!r) throw Raised{};
-        s = {THPVariable_Unpack(PyTuple_GET_ITEM(r, 0)), THPVariable_Unpack(PyTuple_GET_ITEM(r, 1))};
-        Py_DECREF(r);
+        const Ref r(PyObject_CallFunction(snap_provider, "il", device, bytes));
+        s = {THPVariable_Unpack(PyTuple_GET_ITEM(r.o, 0)), THPVariable_Unpack(PyTuple_GET_ITEM(r.o, 1))};
     }
     const int* w = s.words.data_ptr<int>();
-    if (w[0] | w[1]) {                                           // an earlier launch with this buffer has failed
-        PyObject* r = PyObject_CallFunction(snap_failed, "i", (int)like.device().index());
-        if (!r) throw Raised{};
-        Py_DECREF(r);
-    }
+    if (w[0] | w[1]) const Ref r(PyObject_CallFunction(snap_failed, "i", device));      // an earlier launch with these words has failed
     return s;
 }
-// set_hooks(snap_provider, failed)
+// set_hooks(snap_provider, words_provider, failed)
 PyObject* set_hooks(PyObject* const* a) {
-    Py_INCREF(a[0]);
-    Py_INCREF(a[1]);
+    for (int i = 0; i < 3; i++) Py_INCREF(a[i]);
     Py_XSETREF(snap_provider, a[0]);
-    Py_XSETREF(snap_failed, a[1]);
+    Py_XSETREF(words_provider, a[1]);
+    Py_XSETREF(snap_failed, a[2]);
     Py_RETURN_NONE;
 }
 void phase_b_launch(const Records& r, const Snap& s, const Tensor& st, const Tensor& st_out, const Tensor* proj, const Tensor* gw, float eps,
@@ -591,7 +598,7 @@ PyObject* phase_b(PyObject* const* a) {
     const int64_t S = integer(a[0]);
     const Records r = given_records(a + 1, dim32(S));
     const Tensor state = dev(a[4], F32, "state").reshape({1, HV, DV, DK});
-    const Snap& s = snap_buffer(state, qt_gdn_chunk_snap_bytes(dim32(S)));
+    const Snap s = snap_buffer(state, S);
     Tensor st_out = empty({1, HV, DV, DK}, F32, state), out = empty({S, HV, DV}, BF16, state);
     phase_b_launch(r, s, state, st_out, nullptr, nullptr, 0.f, out, S);
     return wrap({out, st_out});
@@ -603,7 +610,7 @@ PyObject* phase_b_norm(PyObject* const* a) {
     const Records r = given_records(a + 1, dim32(S));
     const Tensor state = dev(a[4], F32, "state").reshape({1, HV, DV, DK}), gw = f32(a[5], "gw", DV);
     const float eps = real(a[6]);
-    const Snap& s = snap_buffer(state, qt_gdn_chunk_snap_bytes(dim32(S)));
+    const Snap s = snap_buffer(state, S);
     Tensor st_out = empty({1, HV, DV, DK}, F32, state), out = empty({S, HV * DV}, BF16, state);
     phase_b_launch(r, s, state, st_out, &proj, &gw, eps, out, S);
     return wrap({out, st_out});
@@ -622,7 +629,7 @@ PyObject* gdn_core(PyObject* const* a) {
     const bool want = truth(a[7]);
     if (want)
         for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
-    const Snap& s = snap_buffer(proj, qt_gdn_chunk_snap_bytes(dim32(S)));
+    const Snap s = snap_buffer(proj, S);
     const Records r = new_records(proj);
     Tensor conv_out = empty({1, 3, CD}, BF16, proj), st_out = empty({1, HV, DV, DK}, F32, proj), out = empty({S, HV * DV}, BF16, proj);
     phase_a_conv(proj, cs, w, A, dtb, want ? qkv : nullptr, conv_out.data_ptr(), r);
@@ -751,7 +758,7 @@ PyMethodDef methods[] = {
     QT_FN("qkv_prep", qkv_prep, 7),       QT_FN("out_gate", out_gate, 2),         QT_FN("conv_prep", conv_prep, 3),
     QT_FN("phase_a", phase_a, 8),         QT_FN("phase_b", phase_b, 5),           QT_FN("phase_b_norm", phase_b_norm, 7),
     QT_FN("gdn_core", gdn_core, 8),
-    QT_FN("set_hooks", set_hooks, 2),     QT_FN("blit_batch", blit_batch, 2),     QT_FN("pools_load", pools_load, 12),
+    QT_FN("set_hooks", set_hooks, 3),     QT_FN("blit_batch", blit_batch, 2),     QT_FN("pools_load", pools_load, 12),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_qt_host", "argument checks, allocation and launch of the operators", -1, methods};
 

@@ -61,13 +61,26 @@ def _snap_buffer(dev, nbytes):
     buf = _SNAP.get(key)
     if buf is None or buf.numel() * 2 < nbytes:
         if buf is not None:
-            _raise_if_failed(key, buf, sync=True)          # the old buffer's word is looked at one last time
+            torch.cuda.current_stream(dev).synchronize()
+            _raise_if_failed([key])                        # what the launches with the old buffer have reported
             _SNAP_RETIRED.append(buf)
         buf = torch.zeros(max(nbytes // 2, 8), dtype=torch.float16, device=dev)
         _SNAP[key] = buf
-        if key not in _STATUS:                             # (kept when the buffer is outgrown: a captured HIP graph reports into it)
-            _STATUS[key] = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+        _words(dev)
     return buf
+
+
+def _words(dev, captured=False):
+    """The words that launches on the current stream of `dev` report into (kept when the buffer is outgrown: launches in flight and
+    captured HIP graphs hold their address).  captured: for a launch that is being recorded any words of the device will do, it is
+    not known where the graph will be replayed, and nothing should be allocated."""
+    key = _key(dev)
+    if key not in _STATUS:
+        for other, words in _STATUS.items():
+            if captured and other[0] == key[0]:
+                return words
+        _STATUS[key] = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+    return _STATUS[key]
 
 
 def _status_word(buf):
@@ -84,18 +97,19 @@ def _describe(v):
     return "; ".join(what) or f"status {v}"
 
 
-def _raise_if_failed(key, buf, sync=False):
-    """Looks at what the launches made so far with `buf` have reported into pinned host memory.  Without `sync` it does not wait
-    (a launch still in flight is judged at the next call); with `sync` it waits for the stream first.  A report is cleared, here
-    and in the buffer's status word, and raised as ChunkedPrefillError."""
-    pin = _STATUS[key]
-    if sync and not torch.cuda.is_current_stream_capturing():
-        torch.cuda.current_stream(buf.device).synchronize()
-    v = (GAVE_UP if pin[0] else 0) | (NOT_FINITE if pin[1] else 0)
+def _raise_if_failed(keys):
+    """Looks at what launches have reported into the pinned host words of `keys`, without waiting (a launch still in flight is judged
+    at the next call).  A report is cleared, here and in the buffer's status word, and raised as ChunkedPrefillError."""
+    v = 0
+    for key in keys:
+        pin = _STATUS[key]
+        if pin[0] or pin[1]:
+            torch.cuda.current_stream(key[0]).synchronize()      # error path only: no launch of this stream may report after the reset
+            v |= (GAVE_UP if pin[0] else 0) | (NOT_FINITE if pin[1] else 0)
+            if key in _SNAP:
+                _status_word(_SNAP[key]).zero_()
+            pin.zero_()
     if v:
-        torch.cuda.current_stream(buf.device).synchronize()     # error path only: no launch may report after the reset
-        _status_word(buf).zero_()
-        pin.zero_()
         raise ChunkedPrefillError("chunked prefill: " + _describe(v))
 
 
@@ -103,25 +117,32 @@ def _provide_snap(index, nbytes):
     """The buffer of the current stream of device `index` and its report words, for the native launch path (which keeps them until
     it needs a larger one)."""
     dev = torch.device("cuda", index)
-    return _snap_buffer(dev, nbytes), _STATUS[_key(dev)]
+    return _snap_buffer(dev, nbytes), _words(dev)
+
+
+def _provide_words(index):
+    return _words(torch.device("cuda", index), captured=True)
 
 
 def _report_found(index):
-    key = _key(torch.device("cuda", index))
-    _raise_if_failed(key, _SNAP[key])
+    _raise_if_failed([_key(torch.device("cuda", index))])
 
 
-L.on_host_load(lambda host: host.set_hooks(_provide_snap, _report_found))
+L.on_host_load(lambda host: host.set_hooks(_provide_snap, _provide_words, _report_found))
 
 
 def check_status(device=None, sync=True):
-    """Raises ChunkedPrefillError if a chunked-prefill launch on the current stream of `device` has failed (see
-    _raise_if_failed).  phase_b / phase_b_norm call this without waiting before every launch, so a failure surfaces at the
-    next call at the latest; a caller that needs the answer for the launches already made calls it with sync=True."""
+    """Raises ChunkedPrefillError if a chunked-prefill launch on `device` has reported a failure, whichever stream it ran on: a
+    launch in a replayed HIP graph reports into the words of the stream that it was captured on (or of another one of the device).
+    sync: wait for the current stream first.  phase_b / phase_b_norm look at the words of their own stream, without waiting, before
+    every launch; a caller that needs the answer for the launches and replays already made calls this on their stream with
+    sync=True.  While the current stream is being captured nothing is looked at."""
     dev = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
-    key = _key(dev)
-    if key in _SNAP:
-        _raise_if_failed(key, _SNAP[key], sync=sync)
+    if torch.cuda.is_current_stream_capturing():
+        return
+    if sync:
+        torch.cuda.current_stream(dev).synchronize()
+    _raise_if_failed([key for key in _STATUS if key[0] == _key(dev)[0]])
 
 
 def phase_b(q, k, v, Tb, Am, gv, state, relaxed=True, flags=DEFAULT_FLAGS, tg=None):

@@ -142,3 +142,77 @@ def test_prefill_attention_under_graph(qt, dev):
     def run():
         o.copy_(qt.attention.scaled_dot_product_attention(q, K, V, scale=256 ** -0.5, mask="causal"))
     _replays(dev, run, lambda: [o])
+
+
+def _prefill_inputs(dev, T, seed):
+    gen = torch.Generator().manual_seed(seed)
+    cw, A_log, dtb, gw = layer_params(seed)
+    S0 = to_dev((torch.randn((1, 16, 128, 128), generator=gen) * 0.02).numpy(), dev)
+    return [to_dev(rand_bf(gen, (T, PW)), dev, BF16), to_dev(rand_bf(gen, (1, 3, CD)), dev, BF16), S0, to_dev(cw, dev, BF16), to_dev(A_log, dev),
+            to_dev(dtb, dev), to_dev(gw, dev)]
+
+
+@pytest.mark.parametrize("T", [300, 4033, 4100])
+def test_a_replayed_prefill_reports_to_the_stream_it_is_replayed_on(qt, dev, T):
+    """captured on a side stream that has seen no prefill, replayed on the current one: its failure (a state beyond the half-precision
+    range) is found by check_status there, and the next replay, with a good state, has the eager bits (4033 tokens are the first
+    that read the flag area, which the replays have to clear)"""
+    ins = _prefill_inputs(dev, T, 70 + T)
+    good = ins[2].clone()
+    want = qt.prefill.gdn_core(*ins)
+    qt.gdn_nax.check_status(dev)
+    side, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=side):
+        got = qt.prefill.gdn_core(*ins)
+    for _ in range(2):
+        ins[2].copy_(good * 1e8)
+        g.replay()
+        with pytest.raises(qt.gdn_nax.ChunkedPrefillError, match="not finite"):
+            qt.gdn_nax.check_status(dev, sync=True)
+        ins[2].copy_(good)
+        g.replay()
+        qt.gdn_nax.check_status(dev, sync=True)
+        for k, (a, b) in enumerate(zip(got, want)):
+            check_tensors_equal(f"output {k}", a, b)
+
+
+def test_graphs_captured_on_one_stream_may_overlap(qt, dev):
+    """two graphs of the operators that need scratch memory, captured one after the other on one stream and replayed side by side on two
+    others, with eager calls on the stream of the capture: every result has the bits of the call by itself"""
+    rng = np.random.default_rng(60)
+    B, M, Lmax, S, L = 6, 2, 700, 320, 1500
+    rb = lambda *s: to_dev(bf(rng.standard_normal(s)), dev, BF16)
+    qn, kn = rb(256), rb(256)
+
+    def work(seed):
+        ins = _prefill_inputs(dev, 300, seed)
+        q, K, V = rb(1, 8, S, 256), rb(1, 2, L, 256), rb(1, 2, L, 256)
+        qkv, Kp, Vp = rb(B * M, 5120), rb(B, 2, Lmax, 256), rb(B, 2, Lmax, 256)
+        slots = to_dev(rng.permutation(B).astype(np.int32), dev)
+        pos = to_dev(rng.integers(0, Lmax - M, B).astype(np.int32), dev)
+
+        def run():                                    # (the rows that attn_layer_b appends are the same each time)
+            return [qt.batch.attn_layer_b(qkv, qn, kn, Kp, Vp, slots, pos, M),
+                    qt.attention.scaled_dot_product_attention(q, K, V, scale=256 ** -0.5), *qt.prefill.gdn_core(*ins)]
+        return run
+    runs = [work(61), work(62), work(63)]
+    want = [[t.clone() for t in f()] for f in runs]
+    torch.cuda.synchronize()
+    side, a, b = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.Stream()
+    graphs, outs = [torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()], []
+    for g, f in zip(graphs, runs):
+        with torch.cuda.graph(g, stream=side):
+            outs.append(f())
+    for _ in range(20):
+        with torch.cuda.stream(a):
+            graphs[0].replay()
+        with torch.cuda.stream(b):
+            graphs[1].replay()
+        with torch.cuda.stream(side):
+            eager = runs[2]()
+    torch.cuda.synchronize()
+    for k, (got, w) in enumerate(zip([*outs, eager], want)):
+        for i, (x, y) in enumerate(zip(got, w)):
+            check_tensors_equal(f"program {k}, result {i}", x, y)
+    qt.gdn_nax.check_status(dev, sync=True)
