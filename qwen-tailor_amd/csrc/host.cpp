@@ -6,7 +6,8 @@
 // Every function takes its arguments by position (the Python modules of the package hold the signatures and their defaults) and
 // raises what the checks of _lib.py raise: TypeError for something that is not a GPU tensor of the expected type, ValueError for
 // a wrong shape or layout, RuntimeError for an error code of the C ABI.  The module keeps scratch buffers and tables per device
-// (and stream); they are touched with the GIL held only.
+// (and stream); they are touched with the GIL held only.  It is released while memory is allocated and kernels are launched: either may
+// wait for the GPU, and other threads of the program go on meanwhile.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -20,6 +21,7 @@
 #include <algorithm>
 #include <climits>
 #include <map>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -132,6 +134,18 @@ bool truth(PyObject* o) {
     return v != 0;
 }
 
+struct Unlocked {                           // the GIL released; nothing of Python's may be touched meanwhile
+    PyThreadState* state = PyEval_SaveThread();
+    Unlocked() = default;
+    Unlocked(const Unlocked&) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <typename F>
+auto unlocked(F f) {
+    const Unlocked u;
+    return f();
+}
+
 Tensor empty(at::IntArrayRef size, ScalarType dtype, const Tensor& like) {
     return Tensor(at::detail::empty_cuda(size, dtype, like.device(), std::nullopt));
 }
@@ -173,16 +187,37 @@ std::vector<Tensor>& retired() {
 // launches on different streams may overlap.  `first`: size of the first allocation, so that growth is rare.  Under HIP graph capture
 // it is memory of the graph, free for the next call once this one has been recorded: graphs captured on one stream may be replayed
 // side by side, and beside eager calls.
-enum Purpose { ATTN_B, PREFILL_ATTENTION };
-Tensor workspace(int purpose, const Tensor& like, long bytes, long first) {
-    if (capturing()) return empty({bytes}, U8, like);
-    static auto* m = new std::map<std::tuple<int, int, void*>, Tensor>;
-    Tensor& buf = (*m)[{purpose, (int)like.device().index(), stream()}];
-    if (!buf.defined() || buf.numel() < bytes) {
-        if (buf.defined()) retired().push_back(buf);
-        buf = empty({std::max(bytes, first)}, U8, like);
+// The launches of one call must follow each other on their stream: a call holds `busy` over them, so that another thread that uses the
+// same stream (its buffer, then) does not come in between.  It is taken without the GIL.
+struct Scratch {
+    Tensor buf;
+    std::mutex* busy;                       // null: the buffer is not shared
+};
+struct Busy {
+    std::mutex* m;
+    explicit Busy(std::mutex* busy) : m(busy) {
+        if (m) m->lock();
     }
-    return buf;
+    Busy(const Busy&) = delete;
+    ~Busy() {
+        if (m) m->unlock();
+    }
+};
+enum Purpose { ATTN_B, PREFILL_ATTENTION };
+Scratch workspace(int purpose, const Tensor& like, long bytes, long first) {
+    if (capturing()) return {unlocked([&] { return empty({bytes}, U8, like); }), nullptr};
+    struct Kept {
+        Tensor buf;
+        std::mutex busy;
+    };
+    static auto* m = new std::map<std::tuple<int, int, void*>, Kept>;
+    Kept& k = (*m)[{purpose, (int)like.device().index(), stream()}];
+    if (!k.buf.defined() || k.buf.numel() < bytes) {
+        Tensor larger = unlocked([&] { return empty({std::max(bytes, first)}, U8, like); });
+        if (k.buf.defined()) retired().push_back(k.buf);         // (also one that another thread has made meanwhile)
+        k.buf = larger;
+    }
+    return {k.buf, &k.busy};
 }
 constexpr long WS_FIRST = 32 << 20;         // attn_b: enough for 256 sequences x 4 rows
 
@@ -194,12 +229,15 @@ template <typename Build>
 Tensor table(std::map<int, Tensor>& m, const Tensor& like, int64_t need, std::initializer_list<int64_t> shape, ScalarType dtype, Build build) {
     const int device = like.device().index();
     if (const auto it = m.find(device); it != m.end() && it->second.size(0) >= need) return it->second;
-    Tensor t = empty(shape, dtype, like);
-    build(t);
+    Tensor t = unlocked([&] {
+        Tensor n = empty(shape, dtype, like);
+        build(n);
+        if (!capturing()) c10::hip::getCurrentHIPStream().synchronize();
+        return n;
+    });
     if (capturing()) return t;
-    c10::hip::getCurrentHIPStream().synchronize();
     Tensor& kept = m[device];
-    if (kept.defined()) retired().push_back(kept);
+    if (kept.defined()) retired().push_back(kept);               // (also one that another thread has made meanwhile)
     return kept = t;
 }
 Tensor silu_table(const Tensor& like) {
@@ -229,8 +267,13 @@ Tensor do_gated_norm(const Tensor& y, const Tensor& proj, const Tensor& gw, floa
 // rms_rows(x, nw, eps, f32)
 PyObject* rms_rows(PyObject* const* a) {
     const Tensor& x = dev(a[0], BF16, "x", {ANY, ANY});
-    Tensor y = do_rms_rows(x, dev(a[1], BF16, "nw", {x.size(1)}), real(a[2]));
-    return wrap(truth(a[3]) ? y.to(F32) : y);
+    const Tensor& nw = dev(a[1], BF16, "nw", {x.size(1)});
+    const float eps = real(a[2]);
+    const bool wide = truth(a[3]);
+    return wrap(unlocked([&] {
+        Tensor y = do_rms_rows(x, nw, eps);
+        return wide ? y.to(F32) : y;
+    }));
 }
 
 // fused_gemv(W, x, nw, eps, res, swiglu, gnorm)
@@ -252,12 +295,13 @@ PyObject* fused_gemv(PyObject* const* a) {
     if (has_nw && has_gnorm) value_error("nw and gnorm are exclusive");
     if (swiglu && has_res) value_error("swiglu and res are exclusive");
     const float eps = has_nw || has_gnorm ? real(a[3]) : 0.f;    // (without a prologue nothing looks at it)
+    Tensor proj, gw;
     if (has_gnorm) {
         const Ref pp(PySequence_GetItem(a[6], 0)), pg(PySequence_GetItem(a[6], 1));
         check_shape(x, "y", {ANY, HV * DV});
-        const Tensor proj = gpu_tensor(pp.o, "proj").reshape({M, PW});
+        proj = gpu_tensor(pp.o, "proj").reshape({M, PW});
         check_layout(proj, BF16, "proj");
-        x = do_gated_norm(x, proj, f32(pg.o, "gw", DV), eps);
+        gw = f32(pg.o, "gw", DV);
     }
     const int epi = swiglu ? 2 : has_res ? 1 : 0;
     const int64_t n_out = swiglu ? N / 2 : N;
@@ -268,26 +312,32 @@ PyObject* fused_gemv(PyObject* const* a) {
         check_layout(res, BF16, "res");
         check_shape(res, "res", {M, N});
     }
+    Tensor nw;
+    if (has_nw) nw = dev(a[2], BF16, "nw", {K});
     std::vector<int64_t> shape = xin.sizes().vec();
     shape.back() = n_out;
-    Tensor y = empty(shape, BF16, x);
-    const void* rp = has_res ? res.data_ptr() : nullptr;
-    if (has_nw) {
-        const Tensor& nw = dev(a[2], BF16, "nw", {K});
-        // one launch for the shapes that have it, otherwise the prologue as its own kernel
-        const int rc = qt_fused_gemv_rms(W.data_ptr(), x.data_ptr(), nw.data_ptr(), eps, rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream());
-        if (rc == 0) return wrap(y);
-        if (rc != -4) check(rc, "qt_fused_gemv_rms");
-        x = do_rms_rows(x, nw, eps);
-    }
-    check(qt_fused_gemv(W.data_ptr(), x.data_ptr(), rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream()), "qt_fused_gemv");
-    return wrap(y);
+    return wrap(unlocked([&] {
+        if (has_gnorm) x = do_gated_norm(x, proj, gw, eps);
+        Tensor y = empty(shape, BF16, x);
+        const void* rp = has_res ? res.data_ptr() : nullptr;
+        if (has_nw) {
+            // one launch for the shapes that have it, otherwise the prologue as its own kernel
+            const int rc = qt_fused_gemv_rms(W.data_ptr(), x.data_ptr(), nw.data_ptr(), eps, rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream());
+            if (rc == 0) return y;
+            if (rc != -4) check(rc, "qt_fused_gemv_rms");
+            x = do_rms_rows(x, nw, eps);
+        }
+        check(qt_fused_gemv(W.data_ptr(), x.data_ptr(), rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream()), "qt_fused_gemv");
+        return y;
+    }));
 }
 
 // gated_norm(y [rows, 2048], proj, gw, eps)
 PyObject* gated_norm(PyObject* const* a) {
     const Tensor& y = dev(a[0], BF16, "y", {ANY, HV * DV});
-    return wrap(do_gated_norm(y, dev(a[1], BF16, "proj", {y.size(0), PW}), f32(a[2], "gw", DV), real(a[3])));
+    const Tensor &proj = dev(a[1], BF16, "proj", {y.size(0), PW}), gw = f32(a[2], "gw", DV);
+    const float eps = real(a[3]);
+    return wrap(unlocked([&] { return do_gated_norm(y, proj, gw, eps); }));
 }
 
 // ---- recurrent steps ------------------------------------------------------------------------------------------------------
@@ -310,22 +360,26 @@ Step step_operands(PyObject* const* a) {
 PyObject* decode_step(PyObject* const* a) {
     const Step s = step_operands(a);
     const int rows_per_wg = (int)integer(a[8]);
-    Tensor y = empty({s.proj.size(0), HV * DV}, BF16, s.proj);
-    check(qt_gdn_decode_step(s.proj.data_ptr(), s.conv.data_ptr(), s.w.data_ptr(), s.A.data_ptr<float>(), s.dtb.data_ptr<float>(),
-                             s.ssm.data_ptr<float>(), s.slots.data_ptr<int>(), s.pos.data_ptr<int>(), y.data_ptr(), s.B, s.n_slots, rows_per_wg,
-                             stream()), "qt_gdn_decode_step");
-    return wrap(y);
+    return wrap(unlocked([&] {
+        Tensor y = empty({s.proj.size(0), HV * DV}, BF16, s.proj);
+        check(qt_gdn_decode_step(s.proj.data_ptr(), s.conv.data_ptr(), s.w.data_ptr(), s.A.data_ptr<float>(), s.dtb.data_ptr<float>(),
+                                 s.ssm.data_ptr<float>(), s.slots.data_ptr<int>(), s.pos.data_ptr<int>(), y.data_ptr(), s.B, s.n_slots, rows_per_wg,
+                                 stream()), "qt_gdn_decode_step");
+        return y;
+    }));
 }
 // decode_step_gnorm(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, pos, gw, eps)
 PyObject* decode_step_gnorm(PyObject* const* a) {
     const Step s = step_operands(a);
     const Tensor gw = f32(a[8], "gw", DV);
     const float eps = real(a[9]);
-    Tensor out = empty({s.proj.size(0), HV * DV}, BF16, s.proj);
-    check(qt_gdn_decode_step_gnorm(s.proj.data_ptr(), s.conv.data_ptr(), s.w.data_ptr(), s.A.data_ptr<float>(), s.dtb.data_ptr<float>(),
-                                   s.ssm.data_ptr<float>(), s.slots.data_ptr<int>(), s.pos.data_ptr<int>(), gw.data_ptr<float>(), eps,
-                                   out.data_ptr(), s.B, s.n_slots, stream()), "qt_gdn_decode_step_gnorm");
-    return wrap(out);
+    return wrap(unlocked([&] {
+        Tensor out = empty({s.proj.size(0), HV * DV}, BF16, s.proj);
+        check(qt_gdn_decode_step_gnorm(s.proj.data_ptr(), s.conv.data_ptr(), s.w.data_ptr(), s.A.data_ptr<float>(), s.dtb.data_ptr<float>(),
+                                       s.ssm.data_ptr<float>(), s.slots.data_ptr<int>(), s.pos.data_ptr<int>(), gw.data_ptr<float>(), eps,
+                                       out.data_ptr(), s.B, s.n_slots, stream()), "qt_gdn_decode_step_gnorm");
+        return out;
+    }));
 }
 
 // verify_step(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, sslots, sels, pars, M, rows_per_wg)
@@ -339,11 +393,14 @@ PyObject* verify_step(PyObject* const* a) {
     const Tensor& conv = dev(a[1], BF16, "conv_pool", {n * 2, M, 3, CD});
     const Tensor &sels = dev(a[7], I32, "sels", {B}), &pars = dev(a[8], I32, "pars", {B}), &w = flat_conv_w(a[2]);
     const Tensor A = f32(a[3], "A_log", HV), dtb = f32(a[4], "dt_bias", HV);
-    Tensor y = empty({B * M, HV * DV}, BF16, proj);
-    check(qt_gdn_verify_step(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
-                             ss.data_ptr<int>(), sels.data_ptr<int>(), pars.data_ptr<int>(), y.data_ptr(), dim32(B), dim32(M), dim32(n),
-                             (int)integer(a[10]), stream()), "qt_gdn_verify_step");
-    return wrap(y);
+    const int rows_per_wg = (int)integer(a[10]);
+    return wrap(unlocked([&] {
+        Tensor y = empty({B * M, HV * DV}, BF16, proj);
+        check(qt_gdn_verify_step(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
+                                 ss.data_ptr<int>(), sels.data_ptr<int>(), pars.data_ptr<int>(), y.data_ptr(), dim32(B), dim32(M), dim32(n),
+                                 rows_per_wg, stream()), "qt_gdn_verify_step");
+        return y;
+    }));
 }
 
 // deltanet(proj, conv_snap, conv_w, A_log, dt_bias, ssm_snap, sel, rows_per_wg)
@@ -355,10 +412,14 @@ PyObject* deltanet(PyObject* const* a) {
     if (conv.size(0) != S) value_error("conv_snap and ssm_snap must hold the same number of snapshots");
     const Tensor &sel = dev(a[6], I32, "sel", {1}), &w = flat_conv_w(a[2]);
     const Tensor A = f32(a[3], "A_log", HV), dtb = f32(a[4], "dt_bias", HV);
-    Tensor y = empty({M, HV * DV}, BF16, proj), cs = empty({M, 3, CD}, BF16, proj), st = empty({M, HV, DV, DK}, F32, proj);
-    check(qt_gdn_deltanet(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
-                          sel.data_ptr<int>(), y.data_ptr(), cs.data_ptr(), st.data_ptr<float>(), dim32(M), dim32(S), (int)integer(a[7]), stream()),
-          "qt_gdn_deltanet");
+    const int rows_per_wg = (int)integer(a[7]);
+    Tensor y, cs, st;
+    unlocked([&] {
+        y = empty({M, HV * DV}, BF16, proj), cs = empty({M, 3, CD}, BF16, proj), st = empty({M, HV, DV, DK}, F32, proj);
+        check(qt_gdn_deltanet(proj.data_ptr(), conv.data_ptr(), w.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(), ssm.data_ptr<float>(),
+                              sel.data_ptr<int>(), y.data_ptr(), cs.data_ptr(), st.data_ptr<float>(), dim32(M), dim32(S), rows_per_wg, stream()),
+              "qt_gdn_deltanet");
+    });
     return wrap({y, cs, st});
 }
 
@@ -372,14 +433,14 @@ Pool kv_pool(PyObject* kp, PyObject* vp, PyObject* slots, PyObject* pos, int64_t
     const Tensor& V = dev(vp, BF16, "Vp", {K.size(0), K.size(1), K.size(2), K.size(3)});
     return {K, V, dev(slots, I32, "slots", {B}), dev(pos, I32, "pos", {B}), K.size(0), K.size(2)};
 }
-Tensor attn_scratch(PyObject* given, const Tensor& like, int64_t B, int64_t M, int64_t Lmax, long CH, const char* who) {
+Scratch attn_scratch(PyObject* given, const Tensor& like, int64_t B, int64_t M, int64_t Lmax, long CH, const char* who) {
     const long bytes = qt_gqa_attn_workspace_bytes(dim32(B), dim32(M), dim32(Lmax), (int)CH);
     if (bytes < 0) value_error(std::string(who) + ": bad split size");
     if (given == Py_None) return workspace(ATTN_B, like, bytes, WS_FIRST);
     const Tensor& ws = dev(given, U8, "workspace");
     if (ws.numel() < bytes)
         value_error(std::string(who) + ": workspace of " + std::to_string(ws.numel()) + " bytes, " + std::to_string(bytes) + " needed");
-    return ws;
+    return {ws, nullptr};
 }
 int64_t sequences(int64_t R, int64_t M, const char* who, const char* limit) {
     if (M < 1 || M > 16 || R % M)
@@ -394,12 +455,15 @@ PyObject* attn_b(PyObject* const* a) {
     const Tensor &k = dev(a[1], BF16, "k", {R, 2, 256}), &v = dev(a[2], BF16, "v", {R, 2, 256});
     const Pool p = kv_pool(a[3], a[4], a[5], a[6], B);
     const long CH = integer(a[8]);
-    const Tensor ws = attn_scratch(a[9], q, B, M, p.Lmax, CH, "attn_b");
-    Tensor o = empty({R, 8, 256}, BF16, q);
-    check(qt_gqa_attn_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), p.K.data_ptr(), p.V.data_ptr(), p.slots.data_ptr<int>(), p.pos.data_ptr<int>(),
-                             o.data_ptr(), ws.data_ptr(), ws.numel(), dim32(B), dim32(M), dim32(p.Lmax), dim32(p.n_slots), (int)CH, stream()),
-          "qt_gqa_attn_decode");
-    return wrap(o);
+    const Scratch ws = attn_scratch(a[9], q, B, M, p.Lmax, CH, "attn_b");
+    return wrap(unlocked([&] {
+        Tensor o = empty({R, 8, 256}, BF16, q);
+        const Busy busy(ws.busy);
+        check(qt_gqa_attn_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), p.K.data_ptr(), p.V.data_ptr(), p.slots.data_ptr<int>(), p.pos.data_ptr<int>(),
+                                 o.data_ptr(), ws.buf.data_ptr(), ws.buf.numel(), dim32(B), dim32(M), dim32(p.Lmax), dim32(p.n_slots), (int)CH, stream()),
+              "qt_gqa_attn_decode");
+        return o;
+    }));
 }
 
 // attn_layer_b(qkv, q_norm, k_norm, Kp, Vp, slots, pos, M, eps, split, workspace or None)
@@ -409,13 +473,17 @@ PyObject* attn_layer_b(PyObject* const* a) {
     const Tensor &qn = dev(a[1], BF16, "q_norm", {256}), &kn = dev(a[2], BF16, "k_norm", {256});
     const Pool p = kv_pool(a[3], a[4], a[5], a[6], B);
     const long CH = integer(a[9]);
-    const Tensor ws = attn_scratch(a[10], qkv, B, M, p.Lmax, CH, "attn_layer_b");
+    const Scratch ws = attn_scratch(a[10], qkv, B, M, p.Lmax, CH, "attn_layer_b");
     const Tensor table = rope_table(qkv, p.Lmax);
-    Tensor out = empty({R, 2048}, BF16, qkv);
-    check(qt_gqa_attn_layer_decode(qkv.data_ptr(), qn.data_ptr(), kn.data_ptr(), table.data_ptr(), dim32(table.size(0)), p.K.data_ptr(), p.V.data_ptr(),
-                                   p.slots.data_ptr<int>(), p.pos.data_ptr<int>(), out.data_ptr(), ws.data_ptr(), ws.numel(), dim32(B), dim32(M),
-                                   dim32(p.Lmax), dim32(p.n_slots), (int)CH, real(a[8]), stream()), "qt_gqa_attn_layer_decode");
-    return wrap(out);
+    const float eps = real(a[8]);
+    return wrap(unlocked([&] {
+        Tensor out = empty({R, 2048}, BF16, qkv);
+        const Busy busy(ws.busy);
+        check(qt_gqa_attn_layer_decode(qkv.data_ptr(), qn.data_ptr(), kn.data_ptr(), table.data_ptr(), dim32(table.size(0)), p.K.data_ptr(), p.V.data_ptr(),
+                                       p.slots.data_ptr<int>(), p.pos.data_ptr<int>(), out.data_ptr(), ws.buf.data_ptr(), ws.buf.numel(), dim32(B), dim32(M),
+                                       dim32(p.Lmax), dim32(p.n_slots), (int)CH, eps, stream()), "qt_gqa_attn_layer_decode");
+        return out;
+    }));
 }
 
 // ---- prefill attention ----------------------------------------------------------------------------------------------------
@@ -438,22 +506,24 @@ PyObject* sdpa(PyObject* const* a) {
     if (k.sizes() != v.sizes() || k.stride(1) != v.stride(1)) value_error("k and v must have the same shape and head stride");
     const int64_t L = k.size(2);
     if (L < S) value_error("fewer keys than queries");
-    Tensor out;
-    long head_stride = S * 256;
-    int row_stride = 256;
-    if (S > 1 && q.stride(1) == 256 && q.stride(2) == 2048 && q.stride(3) == 1 && !((uintptr_t)q.data_ptr() & 15)) {
-        out = empty({1, S, 8, 256}, BF16, q).transpose(1, 2);    // a transposed view of token-major rows: neither side is copied
-        head_stride = 256, row_stride = 2048;
-    } else {
-        q = q.contiguous();
-        out = empty(q.sizes(), BF16, q);
-    }
+    const bool token_major = S > 1 && q.stride(1) == 256 && q.stride(2) == 2048 && q.stride(3) == 1 && !((uintptr_t)q.data_ptr() & 15);
     // launches that would leave half of the CUs idle are split along the keys; their parts meet in a workspace
     const long bytes = qt_gqa_prefill_workspace_bytes_for(dim32(S), dim32(L), dim32(L - S));
-    const Tensor ws = bytes > 0 ? workspace(PREFILL_ATTENTION, q, bytes, 0) : Tensor();
-    check(qt_gqa_prefill_causal_strided(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), bytes > 0 ? ws.data_ptr() : nullptr, std::max(bytes, 0L), dim32(S), dim32(L),
-                                        dim32(L - S), head_stride, row_stride, k.stride(1), stream()), "qt_gqa_prefill_causal");
-    return wrap(out);
+    const Scratch ws = bytes > 0 ? workspace(PREFILL_ATTENTION, q, bytes, 0) : Scratch{Tensor(), nullptr};
+    return wrap(unlocked([&] {
+        Tensor out;
+        if (token_major) {
+            out = empty({1, S, 8, 256}, BF16, q).transpose(1, 2);    // a transposed view of token-major rows: neither side is copied
+        } else {
+            q = q.contiguous();
+            out = empty(q.sizes(), BF16, q);
+        }
+        const Busy busy(ws.busy);
+        check(qt_gqa_prefill_causal_strided(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), bytes > 0 ? ws.buf.data_ptr() : nullptr,
+                                            std::max(bytes, 0L), dim32(S), dim32(L), dim32(L - S), token_major ? 256 : S * 256, token_major ? 2048 : 256,
+                                            k.stride(1), stream()), "qt_gqa_prefill_causal");
+        return out;
+    }));
 }
 
 // qkv_prep(qkv, q_norm, k_norm, pos, M, eps, max_pos or None)
@@ -462,11 +532,15 @@ PyObject* qkv_prep(PyObject* const* a) {
     const int64_t R = qkv.size(0), M = integer(a[4]);
     if (M < 1 || R % M) value_error("qkv_prep: M = " + std::to_string(M) + " must divide the number of rows (" + std::to_string(R) + ")");
     const Tensor &pos = dev(a[3], I32, "pos", {R / M}), &qn = dev(a[1], BF16, "q_norm", {256}), &kn = dev(a[2], BF16, "k_norm", {256});
-    Tensor q = empty({R, 8, 256}, BF16, qkv), k = empty({R, 2, 256}, BF16, qkv), v = empty({R, 2, 256}, BF16, qkv);
+    const float eps = real(a[5]);
     const Tensor table = a[6] != Py_None ? rope_table(qkv, std::min(extent(a[6]), 1L << 40) + 1) : Tensor();
-    check(qt_attn_qkv_prep_table(qkv.data_ptr(), qn.data_ptr(), kn.data_ptr(), pos.data_ptr<int>(), table.defined() ? table.data_ptr() : nullptr,
-                                 table.defined() ? dim32(table.size(0)) : 0, q.data_ptr(), k.data_ptr(), v.data_ptr(), R, dim32(M), real(a[5]), stream()),
-          "qt_attn_qkv_prep");
+    Tensor q, k, v;
+    unlocked([&] {
+        q = empty({R, 8, 256}, BF16, qkv), k = empty({R, 2, 256}, BF16, qkv), v = empty({R, 2, 256}, BF16, qkv);
+        check(qt_attn_qkv_prep_table(qkv.data_ptr(), qn.data_ptr(), kn.data_ptr(), pos.data_ptr<int>(), table.defined() ? table.data_ptr() : nullptr,
+                                     table.defined() ? dim32(table.size(0)) : 0, q.data_ptr(), k.data_ptr(), v.data_ptr(), R, dim32(M), eps, stream()),
+              "qt_attn_qkv_prep");
+    });
     return wrap({q, k, v});
 }
 
@@ -475,9 +549,11 @@ PyObject* out_gate(PyObject* const* a) {
     const Tensor& qkv = dev(a[1], BF16, "qkv", {ANY, QKV_W});
     const int64_t R = qkv.size(0);
     const Tensor& o = dev(a[0], BF16, "o", {R, 8, 256});
-    Tensor out = empty({R, 2048}, BF16, qkv);
-    check(qt_attn_out_gate(o.data_ptr(), qkv.data_ptr(), out.data_ptr(), R, stream()), "qt_attn_out_gate");
-    return wrap(out);
+    return wrap(unlocked([&] {
+        Tensor out = empty({R, 2048}, BF16, qkv);
+        check(qt_attn_out_gate(o.data_ptr(), qkv.data_ptr(), out.data_ptr(), R, stream()), "qt_attn_out_gate");
+        return out;
+    }));
 }
 
 // ---- chunked prefill ------------------------------------------------------------------------------------------------------
@@ -486,9 +562,13 @@ PyObject* conv_prep(PyObject* const* a) {
     const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
     const int64_t S = proj.size(0);
     const Tensor &cs = dev(a[1], BF16, "conv_state", {3, CD}), &w = flat_conv_w(a[2]);
-    Tensor q = empty({S, HV, DK}, BF16, proj), k = empty({S, HV, DK}, BF16, proj), v = empty({S, HV, DK}, BF16, proj);
-    check(qt_gdn_conv_prep(proj.data_ptr(), cs.data_ptr(), w.data_ptr(), silu_table(proj).data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), dim32(S),
-                           stream()), "qt_gdn_conv_prep");
+    const Tensor silu = silu_table(proj);
+    Tensor q, k, v;
+    unlocked([&] {
+        q = empty({S, HV, DK}, BF16, proj), k = empty({S, HV, DK}, BF16, proj), v = empty({S, HV, DK}, BF16, proj);
+        check(qt_gdn_conv_prep(proj.data_ptr(), cs.data_ptr(), w.data_ptr(), silu.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), dim32(S), stream()),
+              "qt_gdn_conv_prep");
+    });
     return wrap({q, k, v});
 }
 
@@ -499,9 +579,9 @@ Records new_records(const Tensor& proj) {
     const int S = dim32(proj.size(0));
     return {empty({qt_gdn_chunk_ops_bytes(S) / 2}, F16, proj), empty({qt_gdn_chunk_u_bytes(S) / 2}, F16, proj), empty({qt_gdn_chunk_gc_bytes(S) / 4}, F32, proj)};
 }
-void phase_a_conv(const Tensor& proj, const Tensor& cs, const Tensor& w, const Tensor& A, const Tensor& dtb, const Tensor* qkv, void* conv_out,
-                  const Records& r) {
-    check(qt_gdn_phase_a_conv(proj.data_ptr(), cs.data_ptr(), w.data_ptr(), silu_table(proj).data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(),
+void phase_a_conv(const Tensor& proj, const Tensor& cs, const Tensor& w, const Tensor& silu, const Tensor& A, const Tensor& dtb, const Tensor* qkv,
+                  void* conv_out, const Records& r) {
+    check(qt_gdn_phase_a_conv(proj.data_ptr(), cs.data_ptr(), w.data_ptr(), silu.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(),
                               qkv ? qkv[0].data_ptr() : nullptr, qkv ? qkv[1].data_ptr() : nullptr, qkv ? qkv[2].data_ptr() : nullptr, conv_out,
                               r.ops.data_ptr(), r.U.data_ptr(), r.gC.data_ptr<float>(), dim32(proj.size(0)), stream()), "qt_gdn_phase_a_conv");
 }
@@ -511,7 +591,7 @@ PyObject* phase_a(PyObject* const* a) {
     const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
     const int64_t S = proj.size(0);
     const Tensor A = f32(a[3], "A_log", HV), dtb = f32(a[4], "dt_bias", HV);
-    const Records r = new_records(proj);
+    Records r;
     if (a[5] != Py_None) {
         PyObject* seq = PySequence_Fast(a[5], "qkv: expected (q, k, v)");
         if (!seq) throw Raised{};
@@ -525,16 +605,24 @@ PyObject* phase_a(PyObject* const* a) {
             throw;
         }
         Py_DECREF(seq);
-        check(qt_gdn_phase_a(proj.data_ptr(), t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(),
-                             r.ops.data_ptr(), r.U.data_ptr(), r.gC.data_ptr<float>(), dim32(S), stream()), "qt_gdn_phase_a");
+        unlocked([&] {
+            r = new_records(proj);
+            check(qt_gdn_phase_a(proj.data_ptr(), t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(),
+                                 r.ops.data_ptr(), r.U.data_ptr(), r.gC.data_ptr<float>(), dim32(S), stream()), "qt_gdn_phase_a");
+        });
         return wrap({t[0], t[1], t[2], r.ops, r.U, r.gC});
     }
     const Tensor &cs = dev(a[1], BF16, "conv_state", {3, CD}), &w = flat_conv_w(a[2]);
     Tensor qkv[3];
     const bool want = truth(a[6]);
-    if (want)
-        for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
-    phase_a_conv(proj, cs, w, A, dtb, want ? qkv : nullptr, a[7] != Py_None ? dev(a[7], BF16, "conv_out", {3, CD}).data_ptr() : nullptr, r);
+    void* conv_out = a[7] != Py_None ? dev(a[7], BF16, "conv_out", {3, CD}).data_ptr() : nullptr;
+    const Tensor silu = silu_table(proj);
+    unlocked([&] {
+        r = new_records(proj);
+        if (want)
+            for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
+        phase_a_conv(proj, cs, w, silu, A, dtb, want ? qkv : nullptr, conv_out, r);
+    });
     PyObject* out = PyTuple_New(6);
     for (int i = 0; i < 3; i++) PyTuple_SET_ITEM(out, i, want ? wrap(qkv[i]) : (Py_INCREF(Py_None), Py_None));
     PyTuple_SET_ITEM(out, 3, wrap(r.ops));
@@ -550,6 +638,7 @@ PyObject* phase_a(PyObject* const* a) {
 PyObject *snap_provider = nullptr, *words_provider = nullptr, *snap_failed = nullptr;
 struct Snap {
     Tensor buf, words;
+    std::mutex* busy;                                            // see Scratch
 };
 constexpr int64_t ONE_LAUNCH_TOKENS = 64 * 64 - 63;              // (FUSED_MIN_CHUNKS of gdn_chunked.hip) from here on the flag area is read
 Snap snap_buffer(const Tensor& like, int64_t S) {
@@ -558,16 +647,23 @@ Snap snap_buffer(const Tensor& like, int64_t S) {
     if (!snap_provider) throw Error{PyExc_RuntimeError, "gdn_nax is not imported"};
     if (capturing()) {                                           // memory of the graph, see workspace(); its replays clear the flag area
         const Ref words(PyObject_CallFunction(words_provider, "i", device));
-        Snap s{empty({bytes / 2}, F16, like), THPVariable_Unpack(words.o)};
-        if (S >= ONE_LAUNCH_TOKENS) s.buf.narrow(0, 0, qt_gdn_chunk_snap_bytes(0) / 2).zero_();
-        return s;
+        return {unlocked([&] {
+                    Tensor buf = empty({bytes / 2}, F16, like);
+                    if (S >= ONE_LAUNCH_TOKENS) buf.narrow(0, 0, qt_gdn_chunk_snap_bytes(0) / 2).zero_();
+                    return buf;
+                }), THPVariable_Unpack(words.o), nullptr};
     }
-    static auto* m = new std::map<std::pair<int, void*>, Snap>;
-    Snap& s = (*m)[{device, stream()}];
-    if (!s.buf.defined() || s.buf.numel() * 2 < bytes) {
+    struct Kept {
+        Tensor buf, words;
+        std::mutex busy;
+    };
+    static auto* m = new std::map<std::pair<int, void*>, Kept>;
+    Kept& k = (*m)[{device, stream()}];
+    if (!k.buf.defined() || k.buf.numel() * 2 < bytes) {
         const Ref r(PyObject_CallFunction(snap_provider, "il", device, bytes));
-        s = {THPVariable_Unpack(PyTuple_GET_ITEM(r.o, 0)), THPVariable_Unpack(PyTuple_GET_ITEM(r.o, 1))};
+        k.buf = THPVariable_Unpack(PyTuple_GET_ITEM(r.o, 0)), k.words = THPVariable_Unpack(PyTuple_GET_ITEM(r.o, 1));
     }
+    const Snap s{k.buf, k.words, &k.busy};
     const int* w = s.words.data_ptr<int>();
     if (w[0] | w[1]) const Ref r(PyObject_CallFunction(snap_failed, "i", device));      // an earlier launch with these words has failed
     return s;
@@ -582,6 +678,7 @@ PyObject* set_hooks(PyObject* const* a) {
 }
 void phase_b_launch(const Records& r, const Snap& s, const Tensor& st, const Tensor& st_out, const Tensor* proj, const Tensor* gw, float eps,
                     const Tensor& out, int64_t S) {
+    const Busy busy(s.busy);
     check(qt_gdn_phase_b_report(r.ops.data_ptr(), r.U.data_ptr(), r.gC.data_ptr<float>(), s.buf.data_ptr(), st.data_ptr<float>(), st_out.data_ptr<float>(),
                                 proj ? proj->data_ptr() : nullptr, gw ? gw->data_ptr<float>() : nullptr, eps, out.data_ptr(), dim32(S),
                                 s.words.data_ptr<int>(), stream()), "qt_gdn_phase_b");
@@ -599,8 +696,11 @@ PyObject* phase_b(PyObject* const* a) {
     const Records r = given_records(a + 1, dim32(S));
     const Tensor state = dev(a[4], F32, "state").reshape({1, HV, DV, DK});
     const Snap s = snap_buffer(state, S);
-    Tensor st_out = empty({1, HV, DV, DK}, F32, state), out = empty({S, HV, DV}, BF16, state);
-    phase_b_launch(r, s, state, st_out, nullptr, nullptr, 0.f, out, S);
+    Tensor st_out, out;
+    unlocked([&] {
+        st_out = empty({1, HV, DV, DK}, F32, state), out = empty({S, HV, DV}, BF16, state);
+        phase_b_launch(r, s, state, st_out, nullptr, nullptr, 0.f, out, S);
+    });
     return wrap({out, st_out});
 }
 // phase_b_norm(proj, ops, U, gC, state, gw, eps): the gated norm follows in the same pass
@@ -611,8 +711,11 @@ PyObject* phase_b_norm(PyObject* const* a) {
     const Tensor state = dev(a[4], F32, "state").reshape({1, HV, DV, DK}), gw = f32(a[5], "gw", DV);
     const float eps = real(a[6]);
     const Snap s = snap_buffer(state, S);
-    Tensor st_out = empty({1, HV, DV, DK}, F32, state), out = empty({S, HV * DV}, BF16, state);
-    phase_b_launch(r, s, state, st_out, &proj, &gw, eps, out, S);
+    Tensor st_out, out;
+    unlocked([&] {
+        st_out = empty({1, HV, DV, DK}, F32, state), out = empty({S, HV * DV}, BF16, state);
+        phase_b_launch(r, s, state, st_out, &proj, &gw, eps, out, S);
+    });
     return wrap({out, st_out});
 }
 
@@ -627,18 +730,23 @@ PyObject* gdn_core(PyObject* const* a) {
     const Tensor state = dev(a[2], F32, "state").reshape({1, HV, DV, DK});
     Tensor qkv[3];
     const bool want = truth(a[7]);
-    if (want)
-        for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
     const Snap s = snap_buffer(proj, S);
-    const Records r = new_records(proj);
-    Tensor conv_out = empty({1, 3, CD}, BF16, proj), st_out = empty({1, HV, DV, DK}, F32, proj), out = empty({S, HV * DV}, BF16, proj);
-    phase_a_conv(proj, cs, w, A, dtb, want ? qkv : nullptr, conv_out.data_ptr(), r);
-    phase_b_launch(r, s, state, st_out, &proj, &gw, 1e-6f, out, S);
+    const Tensor silu = silu_table(proj);
+    Tensor conv_out, st_out, out;
+    unlocked([&] {
+        if (want)
+            for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
+        const Records r = new_records(proj);
+        conv_out = empty({1, 3, CD}, BF16, proj), st_out = empty({1, HV, DV, DK}, F32, proj), out = empty({S, HV * DV}, BF16, proj);
+        phase_a_conv(proj, cs, w, silu, A, dtb, want ? qkv : nullptr, conv_out.data_ptr(), r);
+        phase_b_launch(r, s, state, st_out, &proj, &gw, 1e-6f, out, S);
+    });
     return wrap({out, conv_out, st_out});
 }
 
 // ---- copies ---------------------------------------------------------------------------------------------------------------
 struct Jobs {
+    std::vector<Tensor> held;                                    // (the caller's lists may change while the GIL is released)
     std::vector<void*> dst;
     std::vector<const void*> src;
     std::vector<long> meta;
@@ -656,6 +764,8 @@ struct Jobs {
             return n <= numel && first <= numel - n && (stride == 0 || ny - 1 <= (numel - n - first) / stride);
         };
         if (n && ny && !(fits(d, d0, ds) && fits(s, s0, ss))) value_error(who + ": the copy leaves the source or the destination");
+        held.push_back(d);
+        held.push_back(s);
         dst.push_back(d.data_ptr());
         src.push_back(s.data_ptr());
         for (long v : {(long)d.element_size(), n, d0, s0, ny, ds, ss}) meta.push_back(v);
@@ -668,7 +778,7 @@ struct Jobs {
     bool fills = false;
     void run() const {
         if (dst.empty()) return;
-        const int rc = (fills ? qt_blit_fill_batch : qt_blit_batch)(dst.data(), src.data(), meta.data(), (int)dst.size(), stream());
+        const int rc = unlocked([&] { return (fills ? qt_blit_fill_batch : qt_blit_batch)(dst.data(), src.data(), meta.data(), (int)dst.size(), stream()); });
         if (rc == -2) value_error("blit_batch: every copy must be 16-byte granular (base pointers, sizes, offsets, strides)");
         check(rc, "qt_blit_batch");
     }
