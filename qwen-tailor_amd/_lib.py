@@ -92,14 +92,19 @@ class _Host:
     """The functions of csrc/_qt_host (host.cpp): argument checks, output allocation and launch of one operator in a native call.
     The module is loaded (and built, if it is missing or out of date) when the first of them is asked for."""
 
+    FUNCTIONS = ("rms_rows", "fused_gemv", "gated_norm", "decode_step", "decode_step_gnorm", "verify_step", "deltanet", "attn_b", "attn_layer_b",
+                 "sdpa", "qkv_prep", "out_gate", "conv_prep", "phase_a", "phase_b", "phase_b_norm", "gdn_core", "blit_batch", "pools_load")
+
     def __getattr__(self, name):
+        if name not in self.FUNCTIONS:
+            raise AttributeError(f"the host module has no function {name!r}")
         lib()                                                    # libqwen_tailor_hip.so: current, and loaded first
         loader = importlib.machinery.ExtensionFileLoader("_qt_host", _build.HOST_SO)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_qt_host", loader))
         loader.exec_module(module)
         for hook in _on_host_load:
             hook(module)
-        self.__dict__.update({k: v for k, v in vars(module).items() if not k.startswith("_")})
+        self.__dict__.update({f: getattr(module, f) for f in self.FUNCTIONS})
         return self.__dict__[name]
 
 
@@ -108,7 +113,7 @@ _on_host_load = []
 
 
 def on_host_load(hook):
-    """hook(module) is called once the host module is loaded."""
+    """hook(module) is called once the host module is loaded (before its first function is handed out)."""
     _on_host_load.append(hook)
 
 

@@ -81,6 +81,17 @@ def test_null_and_dimension_errors_from_the_c_abi():
     assert lib.qt_fused_gemv(ctypes.c_void_p(8), p16, z, p16, 4, 64, 1024, 0, z) == -2
 
 
+def test_host_functions_are_the_modules_and_nothing_else_is_looked_up(monkeypatch):
+    """every function the module's method table holds can be asked for; any other name is an AttributeError, without a build or a load"""
+    import qwen_tailor_amd as qt
+    table = re.findall(r'QT_FN\("(\w+)"', open(os.path.join(ROOT, "qwen-tailor_amd", "csrc", "host.cpp")).read())
+    assert sorted(qt._lib._Host.FUNCTIONS) == sorted(set(table) - {"set_hooks"})
+    probe = qt._lib._Host()
+    monkeypatch.setattr(qt._lib, "lib", lambda: pytest.fail("a probe of an attribute loaded the library"))
+    for name in ("nope", "__wrapped__", "_ipython_display_", "set_hooks"):
+        assert not hasattr(probe, name)
+
+
 @pytest.mark.parametrize("e,n,d0,s0,ny,ds,ss", [
     (2, 8, 2 ** 63 - 8, 0, 1, 0, 0), (4, 8, 0, 2 ** 61, 1, 0, 0),              # the last byte's offset does not fit 64 bits
     (2, 8, 0, 0, 65537, 2 ** 48, 0), (2, 8, 0, 0, 65537, 0, 2 ** 48),          # ... nor does the last row's start
