@@ -21,10 +21,16 @@ HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1
 HASH = SO + ".srchash"
 
 
+def host_abi() -> str:
+    """what the host module is compiled against besides its source: torch's version and its C++ ABI, HIP's version, CPython's ABI"""
+    import torch
+    return " ".join(map(str, (torch.__version__, torch.version.hip, torch._C._GLIBCXX_USE_CXX11_ABI, sysconfig.get_config_var("SOABI"))))
+
+
 def source_hash() -> str:
-    """sha256 over the names and contents of every source the libraries are built from (csrc/*.hip, *.h, *.cpp and the C header) and
-    the flags"""
-    h = hashlib.sha256(" ".join(FLAGS + HOST_FLAGS).encode())
+    """sha256 over the names and contents of every source the libraries are built from (csrc/*.hip, *.h, *.cpp and the C header), the
+    flags and what the host module is compiled against"""
+    h = hashlib.sha256(" ".join([*FLAGS, *HOST_FLAGS, host_abi()]).encode())
     for path in sorted(p for kind in ("*.hip", "*.h", "*.cpp") for p in glob.glob(os.path.join(CSRC, kind))) + [HEADER]:
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as f:
@@ -33,7 +39,7 @@ def source_hash() -> str:
 
 
 def is_current() -> bool:
-    """True if the built libraries exist and were built from the sources as they are now."""
+    """True if the built libraries exist and were built from the sources, and for the torch and the Python, as they are now."""
     try:
         with open(HASH) as f:
             return os.path.exists(SO) and os.path.exists(HOST_SO) and f.read().strip() == source_hash()

@@ -92,6 +92,20 @@ def test_host_functions_are_the_modules_and_nothing_else_is_looked_up(monkeypatc
         assert not hasattr(probe, name)
 
 
+@pytest.mark.parametrize("what", ["torch", "abi", "python"])
+def test_a_change_of_torch_or_python_makes_the_built_libraries_stale(monkeypatch, what):
+    import qwen_tailor_amd as qt
+    qt._lib.lib()
+    assert qt._build.is_current()
+    if what == "torch":
+        monkeypatch.setattr(torch, "__version__", "0.0.0")
+    elif what == "abi":
+        monkeypatch.setattr(torch._C, "_GLIBCXX_USE_CXX11_ABI", not torch._C._GLIBCXX_USE_CXX11_ABI)
+    else:
+        monkeypatch.setattr(qt._build.sysconfig, "get_config_var", lambda name: "cpython-0")
+    assert not qt._build.is_current()
+
+
 @pytest.mark.parametrize("e,n,d0,s0,ny,ds,ss", [
     (2, 8, 2 ** 63 - 8, 0, 1, 0, 0), (4, 8, 0, 2 ** 61, 1, 0, 0),              # the last byte's offset does not fit 64 bits
     (2, 8, 0, 0, 65537, 2 ** 48, 0), (2, 8, 0, 0, 65537, 0, 2 ** 48),          # ... nor does the last row's start
