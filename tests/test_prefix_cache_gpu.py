@@ -84,6 +84,22 @@ def test_restore_then_admission_into_slot_pools(qt, dev):
         assert torch.equal(back["conv"][i], st["conv"][i]) and torch.equal(back["ssm"][i], st["ssm"][i])
 
 
+def test_restored_tensors_are_contiguous_and_disjoint(qt, dev):
+    """the tensors of a restored state share three blocks, and no bytes with each other or with the cache"""
+    cfg, st = make_state(qt, dev, 64, 3)
+    pc = qt.prefix_cache.PrefixCache(budget_mb=512)
+    ids = np.arange(64, dtype=np.int32)
+    node = pc.insert(pc.insert(None, ids, 20, st), ids, 51, st)
+    for max_len in (51, 80):
+        got, chain = pc.restore(node, max_len)
+        groups = [[t for pair in got["kv"] for t in pair], got["conv"], got["ssm"]]
+        for group in groups:
+            assert all(t.is_contiguous() for t in group) and len({t.untyped_storage().data_ptr() for t in group}) == 1
+        spans = sorted((t.data_ptr(), t.data_ptr() + t.numel() * t.element_size())
+                       for t in [*groups[0], *groups[1], *groups[2], *(x for n in chain for x in (n.kv, n.conv, n.ssm))])
+        assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
+
+
 def test_cat_rows_pads_with_zeros(qt, dev):
     pc = qt.prefix_cache.PrefixCache
     a, b = torch.ones((1, 3, 4), device=dev), 2 * torch.ones((1, 5, 4), device=dev)
