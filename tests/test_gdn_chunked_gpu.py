@@ -306,16 +306,20 @@ def test_give_up_path_ends_the_launch_and_leaves_the_flags_clean(qt, dev):
 def test_report_words_outlive_an_outgrown_buffer(qt, dev):
     """launches (those of a captured HIP graph among them) keep the address of their stream's report words: a longer prompt that
     outgrows the snapshot buffer must not replace the words"""
-    stream = torch.cuda.Stream()
+    stream, nax = torch.cuda.Stream(), qt.gdn_nax
+    snap_bytes = qt._lib.lib().qt_gdn_chunk_snap_bytes
     with torch.cuda.stream(stream):
-        for T in (70, 700):
-            proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(77 + T, T)
-            _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0)
-            key = qt.gdn_nax._key(torch.device("cuda", torch.cuda.current_device()))
-            words = qt.gdn_nax._STATUS[key].data_ptr() if T == 70 else words
+        def core(T):
+            _core(qt, dev, *proj_inputs(77 + T, T))
+        core(70)
+        key = nax._key(torch.device("cuda", torch.cuda.current_device()))
+        words, buf = nax._STATUS[key].data_ptr(), nax._SNAP[key]
+        # (streams are reused: an earlier test may have left a buffer for longer prompts under this one's handle)
+        core(next(T for T in range(700, 100000, 640) if snap_bytes(T) > buf.numel() * 2))
         stream.synchronize()
-        assert qt.gdn_nax._STATUS[key].data_ptr() == words
-        qt.gdn_nax.check_status(dev, sync=True)
+        assert nax._SNAP[key].data_ptr() != buf.data_ptr(), "the buffer was not outgrown"
+        assert nax._STATUS[key].data_ptr() == words
+        nax.check_status(dev, sync=True)
 
 
 @pytest.mark.parametrize("T", [4096, 4100])

@@ -418,6 +418,29 @@ def test_prefill_causal_token_major_rows_are_not_copied(qt, dev, S, L):
     check_tensors_equal("token-major against head-major", a.contiguous(), b)
 
 
+@pytest.mark.parametrize("B,holes", [(100, [(10, 50)]), (130, [(0, 40), (70, 110)]), (120, [(3, 36), (37, 69), (70, 120)])])
+def test_attn_b_steps_over_long_runs_of_skipped_sequences(qt, dev, B, holes):
+    """more than 64 segments (32 sequences) in a row that own no tiles, between short ones: the workgroup whose range reaches across such a
+    hole moves its window of 64 segments over it, at the front, in the middle and up to the end of the table"""
+    rng = np.random.default_rng(B)
+    S, Lmax = B + 2, 64
+    slots, pos = rng.permutation(S)[:B].astype(np.int32), rng.integers(0, 40, B).astype(np.int32)
+    bad = np.zeros(B, bool)
+    for a, b in holes:
+        bad[a:b] = True
+    slots[bad] = np.where(rng.random(bad.sum()) < 0.5, -1, S + 7)
+    Kp, Vp = bf(rng.standard_normal((S + 1, 2, Lmax, 256))), bf(rng.standard_normal((S + 1, 2, Lmax, 256)))
+    q, kn, vn = bf(rng.standard_normal((B, 8, 256))), bf(rng.standard_normal((B, 2, 256))), bf(rng.standard_normal((B, 2, 256)))
+    dK, dV = to_dev(Kp, dev, BF16), to_dev(Vp, dev, BF16)
+    o = to_np(qt.batch.attn_b(to_dev(q, dev, BF16), to_dev(kn, dev, BF16), to_dev(vn, dev, BF16), dK, dV, to_dev(slots, dev), to_dev(pos, dev)))
+    oK, oV, good = Kp.copy(), Vp.copy(), ~bad
+    ref = O.attn_b(q[good], kn[good], vn[good], oK, oV, slots[good], pos[good], 1)
+    for r, got, want in zip(np.flatnonzero(good), o[good], ref):
+        check_attn(f"o row {r}", got, want)
+    check_equal("K pool", to_np(dK), oK)
+    check_equal("V pool", to_np(dV), oV)
+
+
 def test_prefill_causal_rejects_queries_past_the_keys(qt, dev):
     from qwen_tailor_amd import _lib as QL
     t = torch.zeros((1, 8, 32, 256), dtype=BF16, device=dev)
