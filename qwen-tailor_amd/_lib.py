@@ -146,7 +146,3 @@ def f32(t, name, shape=None):
     if t.dtype != torch.float32 or not t.is_contiguous():
         t = t.float().contiguous()
     return dev(t, torch.float32, name, shape)
-
-
-def i32(t, name, n=None):
-    return dev(t, torch.int32, name, None if n is None else (n,))

@@ -13,9 +13,10 @@
 //   quad_gemm_kernel  narrow outputs: small tiles (4 x 4 .. 16 x 16 outputs) so that every CU has one
 //   skinny_gemm_kernel  everything else: 16 features x up to 64 rows per workgroup
 // What decides the first two is how a load maps to lanes.  An MFMA operand wants 16 different rows in 16 neighbouring lanes; a
-// load shaped like that asks for 16 bytes of 16 different rows per quarter-wavefront, and the CU takes in 16 bytes per clock
-// (measured: 33 GB/s and less per CU).  Four neighbouring lanes that read 64 contiguous bytes get four times that.  The two
-// kernels load in that shape and put the lanes right afterwards, each in its own way.
+// load shaped like that asks for 16 bytes of 16 different rows per quarter-wavefront, and a CU then takes in 16 bytes per clock
+// (512 threads a CU that read rows 2 KiB apart from the L2: 38 GB/s per CU).  Where four neighbouring lanes read 64 contiguous bytes it
+// is 63 GB/s, and 78 with 256 bytes per 16 lanes.  The two kernels load in the second shape and put the lanes right afterwards,
+// each in its own way.
 // Arithmetic contract of rms_rows: sum of squares exact, rounded to float once; inv = correctly rounded 1/sqrt(ss / K + eps);
 // t = x * inv and w * t rounded to float separately, then to bf16.
 #include "qt_common.h"
@@ -174,7 +175,7 @@ __device__ __forceinline__ double swap_add16(double a, double b) {
 constexpr int XK = 1024;
 // inv[r] = 1 / sqrt(sum / 1024 + eps) of NR = 2, 4 or 6 rows whose exact (double) sums of squares lie spread over the 64 lanes of
 // ss[r].  The first two folding steps halve the number of values (row r ends in 16-lane row (r & 1) * 2 + (r >> 1 & 1) of value
-// r / 4), so the reduction costs about a third of NR separate ones, and the double-precision root is taken once.
+// r / 4), so the reduction costs about a third of NR separate ones, and the root is taken once.
 template <int NR>
 __device__ __forceinline__ void rows_inv(const double (&ss)[NR], float eps, int lane, float (&inv)[NR]) {
     constexpr int NT = NR / 2, NU = (NT + 1) / 2;
@@ -233,7 +234,8 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
     constexpr int NB = 2 * FB, R = 16 * RB, RW = R / 8;
     __shared__ __align__(1024) bf16_t x_s[R * XK];                // later: the partial sums [NB + 1][4 quarters][R][16 features]
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-    // the row groups of a tile sit on one XCD (workgroups are dealt to the eight XCDs in turn) and share its W through the L2
+    // the row groups of a tile sit on one XCD (workgroups are dealt to the eight XCDs in turn) and share its W through the L2, also though
+    // it is loaded nontemporally (N = 8224, two groups: 18.1 MB fetched, W is 16.8 and the rows on eight XCDs 1.0)
     const int s = blockIdx.x >> 3, grp = s % groups, tile = (s / groups) * 8 + (blockIdx.x & 7);
     if (tile >= tiles) return;
     const int q = (w + s) & 3, half = w >> 2, m0 = grp * R, nb0 = tile * 16 * NB, nx = 16 * (tiles * NB + tile);
@@ -360,7 +362,7 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
 // Narrow outputs (N = 1024: out_proj, o_proj, down_proj): a workgroup owns 4 FG features x 4 MG rows, its NWV wavefronts deal the
 // 128-wide steps of K among themselves, KS at a time with all their loads in flight, and meet in LDS in a fixed order.  The
 // point of the small tile is that every CU has one: at 1 to 16 rows a 16-feature tile leaves 192 of 256 CUs idle, and one CU
-// pulls its 115 KiB of W no faster than ~33 GB/s.
+// takes its 115 KiB of W in at 38 - 63 GB/s at best.
 // Operand layout: lane (n, g) of a load holds elements 32 g + 8 (n & 3) .. of row 4 i + (n >> 2), so a quad of lanes reads 64 and the
 // wavefront 256 contiguous bytes of four rows; W and x alike.  Taken as it is by a 16 x 16 x 32 MFMA, "row" n of the operand is
 // (row n >> 2, k slice n & 3), and of the 16 x 16 results those whose k slices agree are partial sums: element i of lane (n, g)

@@ -5,7 +5,7 @@
 // behaviour so that a CPU restatement reproduces every bf16 value bit for bit:
 //   exp32 / log32 : double-precision libm result rounded to float
 //   sum of squares: exact (double), rounded to float once
-//   rsqrt         : 1 / sqrt evaluated in double precision and rounded to float once
+//   rsqrt         : 1 / sqrt, correctly rounded (rsqrt_rn)
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -316,7 +316,7 @@ __device__ __forceinline__ void row16_bcast_all(float v, float (&r)[N]) {
     }
 }
 // N <= 16 sums of squares of 128-wide rows (every lane of a 16-lane row holds all N) -> r[i] = rsqrt_rn(ss[i] / 128 + eps).
-// Lane c of the row evaluates entry c % N only and the results are broadcast, so the double-precision rsqrt runs once per lane.
+// Lane c of the row evaluates entry c % N only and the results are broadcast, so rsqrt_rn runs once per lane.
 template <int N>
 __device__ __forceinline__ void rsqrt_rows(const float (&ss)[N], float eps, float (&r)[N], int c) {
     // (each candidate passes through an empty asm: a bare chain of selects is turned into an indexed read of a stack array,
