@@ -119,9 +119,14 @@ long integer(PyObject* o) {                 // an int, or what stands for one (_
 }
 // a size, offset or stride of a copy: int(o), held at the ends of the range (no tensor is that large, so the range check refuses it)
 long extent(PyObject* o) {
-    const Ref i(PyNumber_Long(o));
     int beyond = 0;
-    const long v = PyLong_AsLongAndOverflow(i.o, &beyond);
+    long v;
+    if (PyLong_CheckExact(o)) {
+        v = PyLong_AsLongAndOverflow(o, &beyond);
+    } else {
+        const Ref i(PyNumber_Long(o));
+        v = PyLong_AsLongAndOverflow(i.o, &beyond);
+    }
     return beyond > 0 ? LONG_MAX : beyond < 0 ? LONG_MIN : v;
 }
 float real(PyObject* o) {                   // float(o)
@@ -312,8 +317,7 @@ PyObject* fused_gemv(PyObject* const* a) {
         check_layout(res, BF16, "res");
         check_shape(res, "res", {M, N});
     }
-    Tensor nw;
-    if (has_nw) nw = dev(a[2], BF16, "nw", {K});
+    const Tensor* nw = has_nw ? &dev(a[2], BF16, "nw", {K}) : nullptr;
     std::vector<int64_t> shape = xin.sizes().vec();
     shape.back() = n_out;
     return wrap(unlocked([&] {
@@ -322,10 +326,10 @@ PyObject* fused_gemv(PyObject* const* a) {
         const void* rp = has_res ? res.data_ptr() : nullptr;
         if (has_nw) {
             // one launch for the shapes that have it, otherwise the prologue as its own kernel
-            const int rc = qt_fused_gemv_rms(W.data_ptr(), x.data_ptr(), nw.data_ptr(), eps, rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream());
+            const int rc = qt_fused_gemv_rms(W.data_ptr(), x.data_ptr(), nw->data_ptr(), eps, rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream());
             if (rc == 0) return y;
             if (rc != -4) check(rc, "qt_fused_gemv_rms");
-            x = do_rms_rows(x, nw, eps);
+            x = do_rms_rows(x, *nw, eps);
         }
         check(qt_fused_gemv(W.data_ptr(), x.data_ptr(), rp, y.data_ptr(), dim32(M), dim32(N), dim32(K), epi, stream()), "qt_fused_gemv");
         return y;
@@ -746,11 +750,18 @@ PyObject* gdn_core(PyObject* const* a) {
 
 // ---- copies ---------------------------------------------------------------------------------------------------------------
 struct Jobs {
-    std::vector<Tensor> held;                                    // (the caller's lists may change while the GIL is released)
+    std::vector<PyObject*> held;                                 // (the caller's lists may change while the GIL is released)
     std::vector<void*> dst;
     std::vector<const void*> src;
     std::vector<long> meta;
-    void add(const Tensor& d, const Tensor& s, long n, long d0, long s0, long ny, long ds, long ss) {
+    Jobs() = default;
+    Jobs(const Jobs&) = delete;
+    ~Jobs() {
+        for (PyObject* o : held) Py_DECREF(o);
+    }
+    void reserve(size_t n) { held.reserve(2 * n), dst.reserve(n), src.reserve(n), meta.reserve(7 * n); }
+    void add(PyObject* dest, PyObject* source, long n, long d0, long s0, long ny, long ds, long ss) {
+        const Tensor &d = gpu_tensor(dest, "dst"), &s = gpu_tensor(source, "src");
         const std::string who = "blit_batch: job " + std::to_string(dst.size());
         if (d.scalar_type() != s.scalar_type() || (d.scalar_type() != BF16 && d.scalar_type() != F32))
             type_error(who + ": bf16 or float32 tensors of one dtype expected");
@@ -764,13 +775,15 @@ struct Jobs {
             return n <= numel && first <= numel - n && (stride == 0 || ny - 1 <= (numel - n - first) / stride);
         };
         if (n && ny && !(fits(d, d0, ds) && fits(s, s0, ss))) value_error(who + ": the copy leaves the source or the destination");
-        held.push_back(d);
-        held.push_back(s);
+        for (PyObject* o : {dest, source}) {
+            Py_INCREF(o);
+            held.push_back(o);
+        }
         dst.push_back(d.data_ptr());
         src.push_back(s.data_ptr());
         for (long v : {(long)d.element_size(), n, d0, s0, ny, ds, ss}) meta.push_back(v);
     }
-    void add_zeros(const Tensor& d, long n, long d0, long ny, long ds) {       // `ny` rows of `n` zeros
+    void add_zeros(PyObject* d, long n, long d0, long ny, long ds) {       // `ny` rows of `n` zeros
         add(d, d, n, d0, d0, ny, ds, ds);                        // (the checks of the destination range)
         src.back() = nullptr;
         fills = true;
@@ -800,15 +813,16 @@ struct Items {                                                   // the items of
 PyObject* blit_batch(PyObject* const* a) {
     const Items jobs(a[0]), zeros(a[1]);
     Jobs j;
+    j.reserve(jobs.size() + zeros.size());
     for (Py_ssize_t i = 0; i < jobs.size(); i++) {
         const Items t(jobs[i]);
         if (t.size() != 8) value_error("blit_batch: job " + std::to_string(i) + ": expected eight values");
-        j.add(gpu_tensor(t[0], "dst"), gpu_tensor(t[1], "src"), extent(t[2]), extent(t[3]), extent(t[4]), extent(t[5]), extent(t[6]), extent(t[7]));
+        j.add(t[0], t[1], extent(t[2]), extent(t[3]), extent(t[4]), extent(t[5]), extent(t[6]), extent(t[7]));
     }
     for (Py_ssize_t i = 0; i < zeros.size(); i++) {
         const Items t(zeros[i]);
         if (t.size() != 5) value_error("blit_batch: zeros " + std::to_string(i) + ": expected five values");
-        j.add_zeros(gpu_tensor(t[0], "dst"), extent(t[1]), extent(t[2]), extent(t[3]), extent(t[4]));
+        j.add_zeros(t[0], extent(t[1]), extent(t[2]), extent(t[3]), extent(t[4]));
     }
     j.run();
     Py_RETURN_NONE;
@@ -820,9 +834,10 @@ PyObject* pools_load(PyObject* const* a) {
     const long slot = integer(a[7]), pos = integer(a[8]), Lmax = integer(a[9]), nkv = integer(a[10]), D = integer(a[11]), par = pos & 1;
     const long C = 3 * CD, N = HV * DV * DK;
     Jobs j;
+    j.reserve(2 * sc.size() + 2 * kv.size());
     for (Py_ssize_t i = 0; i < std::min(sc.size(), sm.size()); i++) {
-        j.add(gpu_tensor(pc[i], "dst"), gpu_tensor(sc[i], "src"), C, (slot * 2 + par) * C, 0, 1, 0, 0);
-        j.add(gpu_tensor(ps[i], "dst"), gpu_tensor(sm[i], "src"), N, slot * N, 0, 1, 0, 0);
+        j.add(pc[i], sc[i], C, (slot * 2 + par) * C, 0, 1, 0, 0);
+        j.add(ps[i], sm[i], N, slot * N, 0, 1, 0, 0);
     }
     for (Py_ssize_t i = 0; i < kv.size(); i++) {
         const Items pair(kv[i]);
@@ -830,8 +845,8 @@ PyObject* pools_load(PyObject* const* a) {
         const Tensor& K = gpu_tensor(pair[0], "src");
         if (K.dim() != 4) value_error("state: K / V are expected as [1, heads, rows, width]");
         const long smax = K.size(2);
-        j.add(gpu_tensor(pk[i], "dst"), K, pos * D, slot * nkv * Lmax * D, 0, nkv, Lmax * D, smax * D);
-        j.add(gpu_tensor(pv[i], "dst"), gpu_tensor(pair[1], "src"), pos * D, slot * nkv * Lmax * D, 0, nkv, Lmax * D, smax * D);
+        j.add(pk[i], pair[0], pos * D, slot * nkv * Lmax * D, 0, nkv, Lmax * D, smax * D);
+        j.add(pv[i], pair[1], pos * D, slot * nkv * Lmax * D, 0, nkv, Lmax * D, smax * D);
     }
     j.run();
     Py_RETURN_NONE;
