@@ -41,7 +41,7 @@ def attn_b(q, k, v, Kp, Vp, slots, pos, M=1, split=None, workspace=None):
     slots[b]; slots / pos int32 [B]).  Returns o [R,H,D] bf16 and appends k / v at pos[b]+j (in place)
     (qwen35/batch.py:230-237).  M up to 16 (the limit of batch_spec.deltanet_bm); more than four tokens per sequence run as
     passes of four, each reading the pool once.  workspace: optional uint8 device tensor of at least qt_gqa_attn_workspace_bytes(B, M, Lmax, split)
-    bytes for the split-K partial results (default: a buffer cached per device and stream)."""
+    bytes for the split-K partial results (default: a buffer cached per device and stream; under HIP graph capture, memory of the graph)."""
     return L.host.attn_b(q, k, v, Kp, Vp, slots, pos, M, split or split_size(0), workspace)
 
 
