@@ -9,7 +9,7 @@
 // The batch is small, so the product is bound by what ONE CU has to pull in (its share of W and of x) and by the launch itself.
 // Three kernels by shape:
 //   rows_gemm_kernel  the wide projections of a decode / verify batch (K = 1024, N >= 4096): the rows live in LDS, the rms
-//                     prologue is applied on the way there, a workgroup owns 32 or 64 output features
+//                     prologue is applied on the way there, a workgroup owns 32 or 64 output features (and up to four more)
 //   quad_gemm_kernel  narrow outputs: small tiles (4 x 4 .. 16 x 16 outputs) so that every CU has one
 //   skinny_gemm_kernel  everything else: 16 features x up to 64 rows per workgroup
 // What decides the first two is how a load maps to lanes.  An MFMA operand wants 16 different rows in 16 neighbouring lanes; a
@@ -220,25 +220,30 @@ __device__ __forceinline__ void quad_transpose(u32x4& a, u32x4& b, u32x4& c, u32
 // product and the sum of the four do not depend on it, so a row has the same bits in every place of a batch of any size.  (Letting
 // half of the workgroups begin with their quarter's second step would take another 3 % off 16 rows at N = 5120 and 7168, but the order of
 // summation would follow; with the order kept by exchanging registers, in a branch, or by summing the steps apart it costs as much or more.)
-// Two of the launch's shapes do not divide: with `extra` > 0 the first `extra` tiles take one block more, from the end of
-// N (the 514 blocks of N = 8224 are 256 x 2 + 2; a 257th workgroup would take a CU twice as long as the others).
-// Tile sizes (us in a HIP graph, rms prologue included, N = 8224 / 7168 swiglu / 5120; before: rms_rows and the product as two
-// launches, x fragments and W loaded in MFMA shape): 1 row 6.3 / 5.7 / 5.1 (8.5 / 7.9 / 6.9), 16 rows 6.4 / 5.9 / 5.3 (9.1 / 8.5 /
-// 7.9), 32 rows 7.2 / 6.7 / 6.1 (9.9 / 9.8 / 9.0), 64 rows 9.0 / 8.4 / 7.9 (11.9 / 13.0 / 11.3), 80 rows 10.6 / 9.8 / 7.9 (20.2 /
-// 19.5 / 14.2).  An empty kernel takes 1.9 us there; what is left at 64 rows is the 64 KiB of rows and 128 KiB of W a CU pulls.
+// N need not divide: with `extra` > 0 the first `extra` tiles take four features more each, from the end of N (N = 8224 is 256 tiles of 32
+// and eight times four; a 257th workgroup would take a CU twice as long as the others).  They come in MFMA layout, four lanes to an
+// address, and need no transpose; with a whole block of 16 more for two workgroups those two ended the launch 0.5 us late.
+// A workgroup's time at one row (in-kernel time stamps): rows in LDS after 1.9 us, W there after 3.0, product 0.65, the quarters' sum and
+// the store 0.6.  Hence the order: the rows' loads ahead of all W (0.2 us from 16 rows on), the row fragments read before W is waited
+// for and the partial sums beside the rows in LDS, without a barrier between (0.4 us; 16 rows only: beyond, registers and LDS are short).
+// Tile sizes (us in a HIP graph, rms prologue included, N = 8224 / 7168 swiglu / 5120; before these: 6.2 / 5.7 / 5.0 at one row, 6.2 / 5.9 / 5.1
+// at 16, 7.1 / 6.7 / 5.9, 8.9 / 8.3 / 7.6, 10.4 / 9.6 / 7.6): 1 row 5.5 / 5.2 / 4.6, 16 rows 5.8 / 5.2 / 4.6, 32 rows 7.1 / 6.3 / 5.7, 64 rows 8.6 / 7.9 /
+// 7.3, 80 rows 10.1 / 9.5 / 7.4.  An empty kernel takes 1.8 us there, a bare read of the 16.8 MB 4.1; what is left at 64 rows is the 64 KiB of rows
+// and 128 KiB of W a CU pulls and the vector instructions of the prologue and the transposes.
 template <int RB, int FB, bool RMS, int EPI>
 __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
                                                                          const bf16_t* __restrict__ nw, float eps,
                                                                          const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N,
-                                                                         int groups, int tiles, int extra) {
+                                                                         int tiles, int extra) {
     constexpr int NB = 2 * FB, R = 16 * RB, RW = R / 8;
-    __shared__ __align__(1024) bf16_t x_s[R * XK];                // later: the partial sums [NB + 1][4 quarters][R][16 features]
+    __shared__ __align__(1024) bf16_t x_s[R * XK];                // later (16 rows: beside them): the partial sums [NB + 1][4 quarters][R][16 features]
+    __shared__ __align__(16) float red_s[RB == 1 ? (NB + 1) * 4 * R * 16 : 4];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
     // the row groups of a tile sit on one XCD (workgroups are dealt to the eight XCDs in turn) and share its W through the L2, also though
     // it is loaded nontemporally (N = 8224, two groups: 18.1 MB fetched, W is 16.8 and the rows on eight XCDs 1.0)
-    const int s = blockIdx.x >> 3, grp = s % groups, tile = (s / groups) * 8 + (blockIdx.x & 7);
+    const int grp = blockIdx.y, tile = blockIdx.z * 8 + blockIdx.x;
     if (tile >= tiles) return;
-    const int q = (w + s) & 3, half = w >> 2, m0 = grp * R, nb0 = tile * 16 * NB, nx = 16 * (tiles * NB + tile);
+    const int q = (w + grp + blockIdx.z) & 3, half = w >> 2, m0 = grp * R, nb0 = tile * 16 * NB, nx = 16 * NB * tiles + 4 * tile;
     const bool has_x = tile < extra && half == 0;
     u32x4 xr[RW][2], wn[2];
 #pragma unroll
@@ -251,16 +256,21 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
         wn[0] = *reinterpret_cast<const u32x4*>(nw + 8 * lane);
         wn[1] = *reinterpret_cast<const u32x4*>(nw + 512 + 8 * lane);
     }
-    u32x4 a[FB + 1][8];
-    auto w_load = [&](u32x4 (&d)[8], int f0) {
+    // a CU's loads return in the order in which they were issued, whichever wavefront asked: no W before the last row has been requested
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 a[FB][8], ax[8];
+#pragma unroll
+    for (int f = 0; f < FB; f++)
 #pragma unroll
         for (int i = 0; i < 8; i++)
-            d[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
-                W + (size_t)min(f0 + (n & 12) + (i & 3), N - 1) * XK + 128 * (2 * q + (i >> 2)) + 32 * g + 8 * (n & 3)));
-    };
+            a[f][i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+                W + (size_t)min(nb0 + 16 * (half * FB + f) + (n & 12) + (i & 3), N - 1) * XK + 128 * (2 * q + (i >> 2)) + 32 * g + 8 * (n & 3)));
+    if (has_x)
 #pragma unroll
-    for (int f = 0; f < FB; f++) w_load(a[f], nb0 + 16 * (half * FB + f));
-    if (has_x) w_load(a[FB], nx);
+        for (int i = 0; i < 8; i++)
+            ax[i] = *reinterpret_cast<const u32x4*>(W + (size_t)(nx + (n & 3)) * XK + 128 * (2 * q + (i >> 2)) + 32 * g + 8 * (i & 3));
     __builtin_amdgcn_sched_barrier(0);                            // everything is in flight before the first row is looked at
     if (RMS) {
         double ss[RW];
@@ -292,9 +302,11 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
         for (int c = 0; c < 2; c++) *reinterpret_cast<u32x4*>(x_s + r * XK + 8 * ((lane + 64 * c) ^ (r & 15))) = xr[i][c];
     }
     lds_barrier();
-    f32x4 acc[FB + 1][RB];
+    f32x4 acc[FB][RB], acc_x[RB];
 #pragma unroll
-    for (int f = 0; f <= FB; f++)
+    for (int rb = 0; rb < RB; rb++) acc_x[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int f = 0; f < FB; f++)
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) acc[f][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
     const bool odd = n & 1, high = n & 2;
@@ -304,6 +316,12 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
     auto mma = [](const u32x4& av, const u32x4& bv, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv), c, 0, 0, 0);
     };
+    u32x4 xf[RB == 1 ? 8 : 1];                                    // (one row block: read while the last of W is still on its way)
+    if constexpr (RB == 1) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) xf[i] = x_frag(i, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int f = 0; f < FB; f++)
 #pragma unroll
@@ -312,7 +330,7 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
     for (int i = 0; i < 8; i++) {
         u32x4 b[RB];
 #pragma unroll
-        for (int rb = 0; rb < RB; rb++) b[rb] = x_frag(i, rb);
+        for (int rb = 0; rb < RB; rb++) b[rb] = RB == 1 ? xf[RB == 1 ? i : 0] : x_frag(i, rb);
 #pragma unroll
         for (int f = 0; f < FB; f++)
 #pragma unroll
@@ -320,27 +338,26 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
     }
     if (has_x) {
 #pragma unroll
-        for (int t = 0; t < 8; t += 4) quad_transpose(a[FB][t], a[FB][t + 1], a[FB][t + 2], a[FB][t + 3], odd, high);
-#pragma unroll
         for (int i = 0; i < 8; i++)
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++) acc[FB][rb] = mma(a[FB][i], x_frag(i, rb), acc[FB][rb]);
+            for (int rb = 0; rb < RB; rb++) acc_x[rb] = mma(ax[i], RB == 1 ? xf[RB == 1 ? i : 0] : x_frag(i, rb), acc_x[rb]);
     }
-    lds_barrier();                                                // the rows have been read: their memory takes the partial sums
+    if (RB > 1) lds_barrier();                                    // the rows have been read: their memory takes the partial sums
     // accumulator element i of lane (n, g) is feature 4 g + i of row 16 rb + n
-    float* red = reinterpret_cast<float*>(x_s);
+    float* red = RB == 1 ? red_s : reinterpret_cast<float*>(x_s);
     auto put = [&](int blk, const f32x4 (&v)[RB]) {
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) *reinterpret_cast<f32x4*>(red + ((blk * 4 + q) * R + 16 * rb + n) * 16 + 4 * g) = v[rb];
     };
 #pragma unroll
     for (int f = 0; f < FB; f++) put(half * FB + f, acc[f]);
-    if (has_x) put(NB, acc[FB]);
+    if (has_x && g == 0) put(NB, acc_x);
     lds_barrier();
-    const int items = (NB + (tile < extra ? 1 : 0)) * R * 4;
+    const int items = NB * R * 4 + (tile < extra ? R : 0);
     for (int idx = threadIdx.x; idx < items; idx += 512) {        // four adjacent features of a row each (N is a multiple of 4)
-        const int blk = idx / (R * 4), r = (idx / 4) % R, f4 = idx & 3;
-        const int m = m0 + r, f0 = (blk < NB ? nb0 + 16 * blk : nx) + 4 * f4;
+        const bool own = idx < NB * R * 4;
+        const int blk = idx / (R * 4), r = own ? (idx / 4) % R : idx - NB * R * 4, f4 = own ? idx & 3 : 0;
+        const int m = m0 + r, f0 = own ? nb0 + 16 * blk + 4 * f4 : nx;
         if (m >= M || f0 >= N) continue;
         f32x4 t[4];
 #pragma unroll
@@ -368,9 +385,11 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
 // (row n >> 2, k slice n & 3), and of the 16 x 16 results those whose k slices agree are partial sums: element i of lane (n, g)
 // belongs to feature g and row n >> 2 if i = n & 3.  Three of four MFMA results are thrown away; the matrix cores have nothing
 // else to do here (8 x 8 tile, K = 3584: 28 steps x 4 MFMAs per CU).
-// Measured in a HIP graph with the residual epilogue, K = 2048 / 3584 (before: skinny_gemm_kernel): 1 row 3.0 / 3.6 us (4.5 / 6.8),
-// 16 rows 3.6 / 4.5 (6.0 / 9.5), 32 rows 4.1 / 5.9 (6.0 / 9.2), 64 rows 5.3 / 7.2 (6.0 / 9.1).
-template <int NWV, int KS, int FG, int MG, int EPI>
+// PEEL: the first trip is taken out of the loop (by the residual's load, which only that trip makes): 0.2 - 0.6 us less, for a tenth more
+// registers, which costs where several workgroups share a CU (80 rows 7.2 / 10.8 us against 6.4 / 10.3).
+// Measured in a HIP graph with the residual epilogue, K = 2048 / 3584 (before: residual loaded behind the last barrier, no trip peeled): 1 row
+// 3.0 / 3.5 us (3.3 / 3.8), 16 rows 3.4 / 4.4 (3.7 / 4.8), 32 rows 3.8 / 5.2 (4.2 / 5.6), 64 rows 5.2 / 6.2 (5.4 / 6.9).
+template <int NWV, int KS, int FG, int MG, int EPI, bool PEEL>
 __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
                                                              const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N, int K,
                                                              int groups) {
@@ -385,6 +404,12 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
     for (int f = 0; f < FG; f++) wp[f] = W + (size_t)min(n0 + 4 * f + (n >> 2), N - 1) * K + 32 * g + 8 * (n & 3);
 #pragma unroll
     for (int m = 0; m < MG; m++) xp[m] = x + (size_t)min(m0 + 4 * m + (n >> 2), M - 1) * K + 32 * g + 8 * (n & 3);
+    // the thread's output in the epilogue; its residual is requested with the operands, not behind their last barrier
+    const int er = threadIdx.x / F, ef = threadIdx.x % F;
+    const bool e_mine = er < R && m0 + er < M && n0 + ef < N;
+    const size_t eo = (size_t)(m0 + er) * N + n0 + ef;
+    unsigned res_raw = 0;
+    if (EPI == EPI_ADD && !PEEL && e_mine) res_raw = res[eo];
     f32x4 acc[FG][MG];
 #pragma unroll
     for (int f = 0; f < FG; f++)
@@ -400,6 +425,8 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
 #pragma unroll
             for (int m = 0; m < MG; m++) b[c][m] = *reinterpret_cast<const u32x4*>(xp[m] + k0);
         }
+        // (what only the first trip does makes the compiler take that trip out of the loop)
+        if (EPI == EPI_ADD && PEEL && base == w && e_mine) res_raw = res[eo];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c = 0; c < KS; c++)
@@ -440,11 +467,9 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
         if (r < R && m < M && n0 + 2 * p + 1 < N)
             y[(size_t)m * (N / 2) + n0 / 2 + p] = f2bf(silu_bf16(BF(total(r, 2 * p))) * BF(total(r, 2 * p + 1)));
     } else {
-        const int r = threadIdx.x / F, f = threadIdx.x % F, m = m0 + r;
-        if (r < R && m < M && n0 + f < N) {
-            const size_t o = (size_t)m * N + n0 + f;
-            const float v = total(r, f);
-            y[o] = EPI == EPI_ADD ? f2bf(BF(v) + bf2f(res[o])) : f2bf(v);
+        if (e_mine) {
+            const float v = total(er, ef);
+            y[eo] = EPI == EPI_ADD ? f2bf(BF(v) + bf2f((bf16_t)res_raw)) : f2bf(v);
         }
     }
 }
@@ -457,29 +482,36 @@ struct gemv_args {
     hipStream_t stream;
 };
 
-// the workgroups of a launch: `tiles` of 32 FB features, of which the first `extra` take one block of 16 more, times `groups` of 16 RB rows
+// the workgroups of a launch: `tiles` of 32 FB features, of which the first `extra` take four features more, times `groups` of 16 RB rows
 struct RowsGrid {
     int groups, tiles, extra;
     RowsGrid(const gemv_args& p, int cus, int RB, int FB) {
         groups = (p.M + 16 * RB - 1) / (16 * RB), extra = 0;
         const int blocks = (p.N + 15) / 16, per_cu = cus / groups > 0 ? cus / groups : 1;
         tiles = (blocks + 2 * FB - 1) / (2 * FB);
-        // a few blocks more than a whole tile per CU: the first tiles take one each instead of a workgroup of their own
-        if (blocks > per_cu * 2 * FB && blocks - per_cu * 2 * FB <= per_cu / 16) tiles = per_cu, extra = blocks - per_cu * 2 * FB;
+        // a few features more than a whole tile per CU: the first tiles take four each instead of a workgroup of their own
+        if (blocks > per_cu * 2 * FB && blocks - per_cu * 2 * FB <= per_cu / 16) tiles = per_cu, extra = (p.N - per_cu * 32 * FB) / 4;
     }
     bool one_round(int cus) const { return (long)tiles * groups <= cus; }        // a workgroup per CU at most
 };
+constexpr int MAX_GROUPS = 65535;      // of a launch (second dimension of a grid)
 template <int RB, int FB, bool RMS>
 void launch_rows(const gemv_args& p, int cus) {
     const RowsGrid r(p, cus, RB, FB);
-    const int groups = r.groups, tiles = r.tiles, extra = r.extra;
-    const dim3 grid((tiles + 7) / 8 * 8 * groups), block(512);
-    if (p.epi == EPI_NONE)
-        hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_NONE>), grid, block, 0, p.stream, p.W, p.x, p.nw, p.eps, p.res, p.y, p.M, p.N, groups, tiles, extra);
-    else if (p.epi == EPI_ADD)
-        hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_ADD>), grid, block, 0, p.stream, p.W, p.x, p.nw, p.eps, p.res, p.y, p.M, p.N, groups, tiles, extra);
-    else
-        hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_SWIGLU>), grid, block, 0, p.stream, p.W, p.x, p.nw, p.eps, p.res, p.y, p.M, p.N, groups, tiles, extra);
+    const dim3 block(512);
+    for (int g0 = 0; g0 < r.groups; g0 += MAX_GROUPS) {          // (one launch up to 65535 row groups)
+        const size_t row0 = (size_t)g0 * 16 * RB;
+        const dim3 grid(8, r.groups - g0 < MAX_GROUPS ? r.groups - g0 : MAX_GROUPS, (r.tiles + 7) / 8);
+        const bf16_t *x = p.x + row0 * p.K, *res = p.res ? p.res + row0 * p.N : nullptr;
+        bf16_t* y = p.y + row0 * (p.epi == EPI_SWIGLU ? p.N / 2 : p.N);
+        const int M = p.M - (int)row0;
+        if (p.epi == EPI_NONE)
+            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_NONE>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
+        else if (p.epi == EPI_ADD)
+            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_ADD>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
+        else
+            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_SWIGLU>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
+    }
 }
 // the shapes rows_gemm_kernel takes (its 8-byte stores and residual loads want y and res aligned to 8 bytes)
 inline bool rows_shape(const gemv_args& p) {
@@ -533,30 +565,32 @@ bool launch_rows_any(const gemv_args& p, int cus) {
     return false;
 }
 
-template <int NWV, int KS, int FG, int MG>
+template <int NWV, int KS, int FG, int MG, bool PEEL>
 void launch_quad_tile(const gemv_args& p) {
     const int groups = (p.M + 4 * MG - 1) / (4 * MG), tiles = (p.N + 4 * FG - 1) / (4 * FG);
     const dim3 grid((tiles + 7) / 8 * 8 * groups), block(64 * NWV);
     if (p.epi == EPI_NONE)
-        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_NONE>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_NONE, PEEL>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
     else if (p.epi == EPI_ADD)
-        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_ADD>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_ADD, PEEL>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
     else
-        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_SWIGLU>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_SWIGLU, PEEL>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
 }
-template <int FG, int MG>
-void launch_quad(const gemv_args& p) {       // wavefronts and steps at a time by K: all of K in flight at once up to 4096
+// wavefronts and steps at a time by K: all of K in flight at once up to 4096.  PEEL_: the first trip taken out of the loop
+template <int FG, int MG, bool PEEL_ = true>
+void launch_quad(const gemv_args& p) {
     if (p.K <= 1024)
-        launch_quad_tile<4, 2, FG, MG>(p);
+        launch_quad_tile<4, 2, FG, MG, false>(p);
     else if (p.K <= 2048)
-        launch_quad_tile<8, 2, FG, MG>(p);
+        launch_quad_tile<8, 2, FG, MG, PEEL_>(p);
     else
-        launch_quad_tile<8, 4, FG, MG>(p);
+        launch_quad_tile<8, 4, FG, MG, PEEL_>(p);
 }
-// The smallest tile that leaves at most one workgroup per CU; some shapes still gain with two or four workgroups per CU
-// (measured against skinny_gemm_kernel over N = 264 .. 8192, K = 512 .. 3584, 1 .. 128 rows: N = 1024, K = 2048, 64 rows, two
-// workgroups of 8 x 16 per CU 5.3 against 6.0 us; N = 8192, K = 2048, 8 rows, four of 8 x 8 8.3 against 9.4; but N = 4096, K = 2048,
-// 32 rows 9.7 against 8.4).  Returns false where the skinny kernel is the better one.
+// The smallest tile that leaves at most one workgroup per CU; beyond, small tiles still win with several workgroups per CU (measured
+// against skinny_gemm_kernel over N = 264 .. 3072, K = 512 .. 4096, 16 .. 192 rows, us: three workgroups of 8 x 16 per CU N = 1024, K = 2048 / 3584 at 80
+// rows 6.4 / 10.3 against 9.5 / 16.1, N = 3072, K = 2048 at 32 rows 7.3 against 10.1; N = 8192, K = 2048, 8 rows, four of 8 x 8 8.3 against 9.4; two
+// of 16 x 16 N = 1024, K = 2048 at 128 rows 7.3 against 7.9, but K = 3584 12.2 against 11.9, K = 1024 and N = 2048 at 64 rows 5.4 against 5.2; four of 8 x
+// 16 at 128 rows 8.3 / 12.6 against 7.9 / 11.9).  Returns false where the skinny kernel is the better one.
 inline bool launch_quad_any(const gemv_args& p, int cus) {
     auto wgs = [&](int f, int r) { return (long)((p.N + f - 1) / f) * ((p.M + r - 1) / r); };
     if (wgs(4, 4) <= cus || (p.M <= 4 && wgs(4, 4) <= 2 * cus))
@@ -567,8 +601,10 @@ inline bool launch_quad_any(const gemv_args& p, int cus) {
         launch_quad<2, 4>(p);
     else if (p.K > 2048 && wgs(16, 16) <= cus)
         launch_quad<4, 4>(p);
-    else if (p.K > 1024 && p.K <= 2048 && wgs(8, 16) <= 2 * cus)
-        launch_quad<2, 4>(p);
+    else if (wgs(8, 16) <= 3 * cus)
+        launch_quad<2, 4, false>(p);
+    else if (p.K > 1024 && p.K <= 2048 && wgs(16, 16) <= 2 * cus)
+        launch_quad<4, 4>(p);
     else
         return false;
     return true;

@@ -148,12 +148,20 @@ def _check_wide(qt, dev, M, N, epi):
     assert torch.equal(one, two), "rms prologue in the launch and on its own differ"
 
 
+# a few features more than whole tiles: one group of four, several, the most that the first tiles take; one and two row groups, 32 and 64
+# features a tile
+@pytest.mark.parametrize("M,N,epi", [(1, 8196, 0), (7, 8204, 2), (16, 8448, 1), (30, 8196, 1), (45, 8220, 0), (64, 8196, 2), (64, 8320, 1), (16, 8444, 2)])
+def test_wide_projection_with_a_few_features_more(qt, dev, M, N, epi):
+    _check_wide(qt, dev, M, N, epi)
+
+
 # edges of the 4 x 4, 8 x 8, 8 x 16 and 16 x 16 tiles, outputs and rows that end inside a tile, K shorter than one batch of every
 # wavefront (256, 512), not a multiple of the wavefronts' steps (1280, 3584) and longer than one batch (4352)
 @pytest.mark.parametrize("M,N,K,epi", [
     (1, 1024, 2048, 1), (1, 50, 256, 2), (3, 1027, 1280, 0), (4, 2048, 3584, 1), (5, 1024, 3584, 1), (8, 4090, 2048, 2), (9, 1030, 2048, 0),
     (16, 1024, 4352, 1), (17, 1024, 2048, 1), (31, 1021, 3584, 0), (33, 1000, 2048, 2), (64, 1024, 3584, 1), (63, 1023, 3584, 0),
-    (64, 1024, 2048, 1), (5, 16, 512, 0), (40, 40, 256, 1)])
+    (64, 1024, 2048, 1), (5, 16, 512, 0), (40, 40, 256, 1), (65, 1024, 3584, 1), (96, 1026, 2048, 2), (81, 1000, 512, 0), (128, 1020, 1280, 1),
+    (97, 1024, 2048, 0), (30, 3070, 4352, 1)])
 def test_narrow_projection_tiles_exact_on_small_integers(qt, dev, M, N, K, epi):
     g = torch.Generator().manual_seed(M * 3 + N + K + epi)
     W = torch.randint(-3, 4, (N, K), generator=g).float().numpy()
