@@ -1,6 +1,6 @@
 // Fused GatedDeltaNet decode / speculative-verify step for gfx950.
 //
-// One workgroup (256 threads = 4 wavefronts of 64) owns ROWS = RS*16 value rows of one (sequence, head) and streams them
+// One group of WPH wavefronts (4; 8 for a few whole heads) owns ROWS = 4 RS WPH value rows of one (sequence, head) and streams them
 // HBM -> registers -> HBM exactly once: conv4 + SiLU, q/k L2 norm, gates, then for every value row r
 //     s = S[r,:] * g;  kv = s.k;  delta = (v_r - kv) * beta;  s += k * delta;  y_r = s.q
 // (qwen35/kernels.py:518-530).  Replaces the Metal kernels deltanet_b (qwen35/batch.py:36-135), deltanet_bm
@@ -19,128 +19,166 @@ namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));   // native vector: nontemporal loads / stores take it
 
-struct RawIn {          // the un-convolved inputs one prologue thread needs for one token
-    float w0, w1, w2, x;
+struct RawIn {          // the un-convolved inputs one prologue thread needs for one token: raw bf16 bits
+    unsigned w0, w1, w2, x;
     uint2 c;
 };
 
 // input row t of channel ch for the chained tokens of one sequence: t < 0 reads the stored window (kernels.py:477-479)
-__device__ __forceinline__ float inp(const bf16_t* __restrict__ cs_in, const bf16_t* __restrict__ proj, int t, int ch) {
-    return t < 0 ? bf2f(cs_in[(t + 3) * CD + ch]) : bf2f(proj[(size_t)t * PW + ch]);
+__device__ __forceinline__ unsigned inp(const bf16_t* __restrict__ cs_in, const bf16_t* __restrict__ proj, int t, int ch) {
+    return t < 0 ? cs_in[(t + 3) * CD + ch] : proj[(size_t)t * PW + ch];
 }
-__device__ __forceinline__ RawIn load_raw(const bf16_t* __restrict__ cs_in, const bf16_t* __restrict__ proj,
-                                          const bf16_t* __restrict__ cw, int j, int ch) {
-    RawIn r;
+// what does not depend on the sequence's slot ...
+__device__ __forceinline__ void load_raw_proj(RawIn& r, const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cw, int j, int ch) {
+    r.x = proj[(size_t)j * PW + ch];
+    r.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch * 4);
+}
+// ... and what does
+__device__ __forceinline__ void load_raw_window(RawIn& r, const bf16_t* __restrict__ cs_in, const bf16_t* __restrict__ proj, int j, int ch) {
     r.w0 = inp(cs_in, proj, j - 3, ch);
     r.w1 = inp(cs_in, proj, j - 2, ch);
     r.w2 = inp(cs_in, proj, j - 1, ch);
-    r.x = inp(cs_in, proj, j, ch);
-    r.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch * 4);
-    return r;
+}
+// (a value that is converted in the block that loads it is waited for there: what is read again behind this is converted behind it)
+__device__ __forceinline__ void pin(RawIn& r) { asm volatile("" : "+v"(r.w0), "+v"(r.w1), "+v"(r.w2), "+v"(r.x)); }
+__device__ __forceinline__ float conv_raw(const RawIn& r) {
+    return conv_silu(bf2f((bf16_t)r.w0), bf2f((bf16_t)r.w1), bf2f((bf16_t)r.w2), bf2f((bf16_t)r.x), r.c);
 }
 __device__ __forceinline__ void store_window(bf16_t* __restrict__ cs_out, const RawIn& r, int ch) {
-    cs_out[ch] = f2bf(r.w1);            // kernels.py:531: the new window is the last three input rows
-    cs_out[CD + ch] = f2bf(r.w2);
-    cs_out[2 * CD + ch] = f2bf(r.x);
+    cs_out[ch] = (bf16_t)r.w1;          // kernels.py:531: the new window is the last three input rows
+    cs_out[CD + ch] = (bf16_t)r.w2;
+    cs_out[2 * CD + ch] = (bf16_t)r.x;
 }
+// where a sequence's window and state lie; snapshot j of the state goes to st_out + j*st_stride and of the conv window to cs_out +
+// j*cs_stride (strides 0 = update in place).  ok = false: the row is skipped; its places are then others inside the pools, from which
+// is read but nothing is written
+struct Place {
+    bool ok;
+    const bf16_t* cs_in;
+    bf16_t* cs_out;
+    size_t cs_stride;
+    const float* st_in;
+    float* st_out;
+    size_t st_stride;
+};
+// the value of lane I of the wavefront, which is the same for all of them
+__device__ __forceinline__ float lane_value(float v, int i) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), i)); }
 
-// M chained tokens of one (sequence, head, row split).  Snapshot j of the state goes to st_out + j*st_stride and of the
-// conv window to cs_out + j*cs_stride (strides 0 = update in place).
-// NORM (whole heads only, RS = 8): y receives the gated RMSNorm of the head's 128 outputs, BF(z sigmoid(z) gw (y inv)) with
+// M chained tokens of one (sequence, head, row split), by WPH wavefronts; place() tells where they lie.
+// NORM (whole heads only): y receives the gated RMSNorm of the head's 128 outputs, BF(z sigmoid(z) gw (y inv)) with
 // z = proj[6144 + h*128 + row] (qwen35/batch.py:321-331), instead of the outputs themselves: same bits as the stand-alone
 // norm kernel applied to the stored outputs.
-template <int RS, int HPW = 1, bool NORM = false>
-__device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cs_in,
-                                           bf16_t* __restrict__ cs_out, size_t cs_stride,
-                                           const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
-                                           const float* __restrict__ dt_bias, const float* st_in,
-                                           float* st_out, size_t st_stride, bf16_t* __restrict__ y, int M, int h,
-                                           int split, const float* __restrict__ gw = nullptr, float eps = 0.f) {
-    static_assert(!NORM || RS == 8, "the fused norm needs the whole head in one group of 256 threads");
-    constexpr int ROWS = RS * 16;
-    __shared__ double red_a[HPW][4];
+// Order of the loads: what depends on neither slot nor position first, while those two are looked up, then the window, then the state;
+// nothing is waited for before the state has been requested.  (Slot, position and the inputs one after the other, and the inputs
+// converted where they are loaded, the state's requests left about two memory latencies late.  Fused norm, us in a HIP graph at 1 / 8 / 16 /
+// 20 / 64 rows 4.7 / 5.8 / 7.6 / 9.2 / 24.6, now 4.4 / 5.4 / 7.2 / 8.9 / 24.4; verify of 16 x 4 17.9, now 17.5.)
+// WPH: four wavefronts share q, k, v and the gates; with more, q and k, v, and the gates have wavefronts of their own, and the state is in
+// more hands: a little faster while most CUs have nothing to do.
+template <int RS, int HPW = 1, bool NORM = false, int WPH = 4, class PlaceFn>
+__device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
+                                           const float* __restrict__ dt_bias, bf16_t* __restrict__ y, int M, int h, int split,
+                                           PlaceFn place, const float* __restrict__ gw = nullptr, float eps = 0.f) {
+    constexpr int GRPS = 4 * WPH, ROWS = RS * GRPS;
+    static_assert(!NORM || ROWS == DV, "the fused norm needs the whole head in one group of wavefronts");
+    static_assert(WPH == 4 || (WPH >= 8 && ROWS == DV), "more wavefronts take whole heads");
+    __shared__ double red_a[HPW][WPH];
     __shared__ __align__(16) float qk_a[HPW][2][DK];
     __shared__ float v_a[HPW][ROWS];
     __shared__ float gb_a[HPW][2];
-    // HPW heads per workgroup: each group of 256 threads runs one head, only the barriers are shared
-    const int sub = HPW > 1 ? (int)(threadIdx.x >> 8) : 0;
+    // HPW heads per workgroup: each group of WPH wavefronts runs one head, only the barriers are shared
+    const int wg_w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sub = HPW > 1 ? wg_w / WPH : 0, w = HPW > 1 ? wg_w % WPH : wg_w;
     double* red = red_a[sub];
     float (*qk_s)[DK] = qk_a[sub];
     float* v_s = v_a[sub];
     float* gb_s = gb_a[sub];
 
-    const int tid = threadIdx.x & 255, w = tid >> 6, lane = tid & 63, grp = lane >> 4, c = lane & 15;
+    const int lane = threadIdx.x & 63, tid = 64 * w + lane, grp = lane >> 4, c = lane & 15;
     const int row0 = split * ROWS;
-    const int which = tid >> 7;                                  // 0: a q channel, 1: a k channel
+    // wavefronts 0, 1: q channels, 2, 3: k channels; v channels: the first ROWS threads, or wavefronts 4 and 5; gates: wavefront GW
+    constexpr int V0 = WPH > 4 ? 256 : 0, GW = WPH > 4 ? 6 : 3;
+    const bool is_qk = WPH == 4 || w < 4, has_v = WPH == 4 ? tid < ROWS : (w == 4 || w == 5), is_g = w == GW;
+    const int which = w >> 1;                                    // 0: a q channel, 1: a k channel
     const int ch_qk = which * KD + h * DK + (tid & 127);
-    const bool has_v = tid < ROWS;
-    const int ch_v = 2 * KD + h * DV + row0 + tid;
+    const int ch_v = 2 * KD + h * DV + row0 + tid - V0;
+    const int ch_v_ld = has_v ? ch_v : ch_qk;                    // (four wavefronts: every load is unconditional)
 
-    // ---- token 0's prologue inputs first, then the state: the prologue runs while the state is in flight.  Every load
-    // below is unconditional (threads without a v channel re-read their q/k channel) so that nothing has to be waited
-    // for before the state loads are issued.
-    const int ch_v_ld = has_v ? ch_v : ch_qk;
-    RawIn rq = load_raw(cs_in, proj, cw, 0, ch_qk);
-    RawIn rv = load_raw(cs_in, proj, cw, 0, ch_v_ld);
-    // gates are evaluated by wave 3: lane 1 the decay gate (reads a), lane 2 beta (reads b)
-    const int gl = lane < 3 ? lane : 0;
-    float gx = bf2f(proj[CD + KD + HV * (gl == 1 ? 1 : 0) + h]);       // lane 1: a;  lanes 0, 2: b
+    RawIn rq = {0, 0, 0, 0, {0, 0}}, rv = {0, 0, 0, 0, {0, 0}};
+    if (is_qk) load_raw_proj(rq, proj, cw, 0, ch_qk);
+    if (WPH == 4 || has_v) load_raw_proj(rv, proj, cw, 0, ch_v_ld);
+    // gates: lane 1 the decay gate (reads a), lane 2 beta (reads b)
+    const int g_at = CD + KD + HV * (lane == 1 ? 1 : 0) + h;
+    unsigned gx = 0;
+    if (WPH == 4 || is_g) gx = proj[g_at];
     const float gA = A_log[h], gdt = dt_bias[h];
-    // fused norm: lane c < 8 of a 16-lane group finishes the group's row i = c (row c*16 + w*4 + grp of the head)
-    const int nrow = (c & 7) * 16 + w * 4 + grp;
-    float nz = 0.f, ngw = 0.f;
+    // fused norm: lane c < RS of a 16-lane group finishes the group's row i = c (row c*GRPS + w*4 + grp of the head)
+    const int nrow = (c % RS) * GRPS + w * 4 + grp;
+    unsigned nz = 0;
+    float ngw = 0.f;
     if (NORM) {
-        nz = bf2f(proj[CD + h * DV + nrow]);
+        nz = proj[CD + h * DV + nrow];
         ngw = gw[nrow];
     }
+    __builtin_amdgcn_sched_barrier(0);
+    const Place at = place();
+    if (is_qk) load_raw_window(rq, at.cs_in, proj, 0, ch_qk);
+    if (WPH == 4 || has_v) load_raw_window(rv, at.cs_in, proj, 0, ch_v_ld);
     __builtin_amdgcn_sched_barrier(0);           // keep the small loads ahead of the state loads in issue order
 
     f4 s[RS][2];
     {
-        const f4* sin4 = reinterpret_cast<const f4*>(st_in + ((size_t)h * DV + row0) * DK);
+        const f4* sin4 = reinterpret_cast<const f4*>(at.st_in + ((size_t)h * DV + row0) * DK);
 #pragma unroll
         for (int i = 0; i < RS; i++) {
-            const int row = i * 16 + w * 4 + grp;
+            const int row = i * GRPS + w * 4 + grp;
             s[i][0] = __builtin_nontemporal_load(sin4 + row * (DK / 4) + c);
             s[i][1] = __builtin_nontemporal_load(sin4 + row * (DK / 4) + 16 + c);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
+    pin(rq);
+    pin(rv);
+    asm volatile("" : "+v"(gx), "+v"(nz));
 
     const float sc = which == 0 ? BF(INV_SCALE * INV_SCALE) : BF(INV_SCALE);       // kernels.py:492
     for (int j = 0; j < M; j++) {
         if (j > 0) {
-            rq = load_raw(cs_in, proj, cw, j, ch_qk);
-            rv = load_raw(cs_in, proj, cw, j, ch_v_ld);
-            gx = bf2f(proj[(size_t)j * PW + CD + KD + HV * (gl == 1 ? 1 : 0) + h]);
+            if (is_qk) load_raw_proj(rq, proj, cw, j, ch_qk), load_raw_window(rq, at.cs_in, proj, j, ch_qk);
+            if (WPH == 4 || has_v) load_raw_proj(rv, proj, cw, j, ch_v_ld), load_raw_window(rv, at.cs_in, proj, j, ch_v_ld);
+            if (WPH == 4 || is_g) gx = proj[(size_t)j * PW + g_at];
         }
-        bf16_t* cso = cs_out + (size_t)j * cs_stride;
+        bf16_t* cso = at.cs_out + (size_t)j * at.cs_stride;
         // conv + silu, exact sum of squares over the head's 128 q (waves 0,1) / k (waves 2,3) channels
-        const float u = conv_silu(rq.w0, rq.w1, rq.w2, rq.x, rq.c);
-        const double tot = wave_sum_d((double)u * (double)u);
-        if (lane == 0) red[w] = tot;
-        if (split == 0) store_window(cso, rq, ch_qk);
+        float u = 0.f;
+        if (is_qk) {
+            u = conv_raw(rq);
+            const double tot = wave_sum_d((double)u * (double)u);
+            if (lane == 0) red[w] = tot;
+        }
         float vv = 0.f;
         if (has_v) {
-            vv = conv_silu(rv.w0, rv.w1, rv.w2, rv.x, rv.c);
-            store_window(cso, rv, ch_v);
+            vv = conv_raw(rv);
         }
         float g = 0.f, beta = 0.f;
-        if (w == 3) {                                                            // kernels.py:511-515
-            // lane 1: decay gate from a; lane 2: beta from b
-            g = __shfl(decay_gate(gA, BF(gx + gdt)), 1, 64);
-            beta = __shfl(sigmoid_bf16(gx), 2, 64);
+        if (is_g) {                                                              // kernels.py:511-515
+            const float gv = bf2f((bf16_t)gx);
+            g = lane_value(decay_gate(gA, BF(gv + gdt)), 1);
+            beta = lane_value(sigmoid_bf16(gv), 2);
         }
         __syncthreads();
-        {
+        if (!at.ok) return;                                      // (before the first barrier the loads would be sunk below this branch, and wait for it)
+        if (is_qk) {
+            if (split == 0) store_window(cso, rq, ch_qk);
             const float ss = (float)(red[which * 2] + red[which * 2 + 1]);
             const float r = rsqrt_rn(ss / (float)DK + qk_eps());
             qk_s[which][tid & 127] = BF(BF(u * r) * sc);                         // kernels.py:507-510
-            if (has_v) v_s[tid] = vv;
-            if (tid == 192) {
-                gb_s[0] = g;
-                gb_s[1] = beta;
-            }
+        }
+        if (has_v) {
+            v_s[tid - V0] = vv;
+            store_window(cso, rv, ch_v);
+        }
+        if (is_g && lane == 0) {
+            gb_s[0] = g;
+            gb_s[1] = beta;
         }
         __syncthreads();
 
@@ -155,12 +193,12 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
         const float gg = gb_s[0], bb = gb_s[1];
         const float kq = dot8_row16(k8, q8);
 
-        f4* so4 = reinterpret_cast<f4*>(st_out + (size_t)j * st_stride + ((size_t)h * DV + row0) * DK);
+        f4* so4 = reinterpret_cast<f4*>(at.st_out + (size_t)j * at.st_stride + ((size_t)h * DV + row0) * DK);
         bf16_t* yo = y + (size_t)j * KD + h * DV + row0;
         float yb[RS];
 #pragma unroll
         for (int i = 0; i < RS; i++) {
-            const int row = i * 16 + w * 4 + grp;
+            const int row = i * GRPS + w * 4 + grp;
             float sv[8] = {s[i][0].x, s[i][0].y, s[i][0].z, s[i][0].w, s[i][1].x, s[i][1].y, s[i][1].z, s[i][1].w};
             const float yv = gdn_row_step(sv, k8, q8, v_s[row], gg, bb, kq);
             s[i][0] = f4{sv[0], sv[1], sv[2], sv[3]};
@@ -174,20 +212,23 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
             }
         }
         if (NORM) {
-            // sum of squares of the head's 128 stored outputs: this lane's 8 rows, the wavefront's 4 groups, the 4 wavefronts
+            // sum of squares of the head's 128 stored outputs: this lane's RS rows, the wavefront's 4 groups, the WPH wavefronts
             double ss = 0.0;
 #pragma unroll
             for (int i = 0; i < RS; i++) ss += (double)yb[i] * yb[i];
-            ss += __shfl_xor(ss, 16, 64);
-            ss += __shfl_xor(ss, 32, 64);
-            __syncthreads();                                     // `red` was last read in the prologue
-            if (lane == 0) red[w] = ss;
+            ss = groups_sum_d(ss);
+            __shared__ double red_y[HPW][WPH];
+            if (lane == 0) red_y[sub][w] = ss;
             __syncthreads();
-            const float inv = rsqrt_rn((float)((red[0] + red[1]) + (red[2] + red[3])) / 128.f + eps);
+            double tot = 0.0;
+#pragma unroll
+            for (int i = 0; i < WPH; i += 4)
+                tot += (red_y[sub][i] + red_y[sub][i + 1]) + (red_y[sub][i + 2] + red_y[sub][i + 3]);
+            const float inv = rsqrt_rn((float)tot / 128.f + eps);
             float mine = yb[0];
 #pragma unroll
-            for (int i = 1; i < RS; i++) mine = ((c & 7) == i) ? yb[i] : mine;
-            if (c < 8) yo[nrow] = gated_out(nz, ngw * (mine * inv));
+            for (int i = 1; i < RS; i++) mine = ((c % RS) == i) ? yb[i] : mine;
+            if (c < RS) yo[nrow] = gated_out(bf2f((bf16_t)nz), ngw * (mine * inv));
         }
     }
 }
@@ -202,6 +243,14 @@ __device__ __forceinline__ void split_id(int& b, int& h, int& split) {
     split = rem % NSPLIT;
 }
 
+__device__ __forceinline__ Place decode_place(bf16_t* conv_pool, float* ssm_pool, int slot, int p, int n_slots) {
+    const int par = p & 1;                                       // batch.py:49-52: read buffer pos&1, write the other
+    const bool ok = (unsigned)slot < (unsigned)n_slots;
+    slot = ok ? slot : 0;
+    float* st = ssm_pool + (size_t)slot * HV * DV * DK;
+    return {ok, conv_pool + (size_t)(slot * 2 + par) * 3 * CD, conv_pool + (size_t)(slot * 2 + (par ^ 1)) * 3 * CD, 0, st, st, 0};
+}
+
 // batch.deltanet_b (qwen35/batch.py:128-135): one token per row, pools updated in place
 template <int RS>
 __global__ __launch_bounds__(256) void gdn_decode_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
@@ -211,35 +260,25 @@ __global__ __launch_bounds__(256) void gdn_decode_kernel(const bf16_t* __restric
                                                          bf16_t* __restrict__ y, int n_slots) {
     int b, h, split;
     split_id<RS>(b, h, split);
-    const int slot = slots[b];
-    if ((unsigned)slot >= (unsigned)n_slots) return;             // never touch memory outside the pools
-    const int par = pos[b] & 1;                                  // batch.py:49-52: read buffer pos&1, write the other
-    float* st = ssm_pool + (size_t)slot * HV * DV * DK;
-    gdn_tokens<RS>(proj + (size_t)b * PW, conv_pool + (size_t)(slot * 2 + par) * 3 * CD,
-                   conv_pool + (size_t)(slot * 2 + (par ^ 1)) * 3 * CD, 0, cw, A_log, dt_bias, st, st, 0,
-                   y + (size_t)b * KD, 1, h, split);
+    const int slot = slots[b], p = pos[b];
+    gdn_tokens<RS>(proj + (size_t)b * PW, cw, A_log, dt_bias, y + (size_t)b * KD, 1, h, split,
+                   [&] { return decode_place(conv_pool, ssm_pool, slot, p, n_slots); });
 }
 
-// the same step with HPW heads of one row per workgroup (256 threads per head, whole heads only): the workgroup streams
+// the same step with HPW heads of one row per workgroup (WPH wavefronts per head, whole heads only): the workgroup streams
 // HPW * 64 KiB of contiguous state
-template <int HPW, bool NORM = false>
-__global__ __launch_bounds__(256 * HPW) void gdn_decode_wide_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
-                                                                    const bf16_t* __restrict__ cw,
-                                                                    const float* __restrict__ A_log,
-                                                                    const float* __restrict__ dt_bias, float* ssm_pool,
-                                                                    const int* __restrict__ slots,
-                                                                    const int* __restrict__ pos, bf16_t* __restrict__ y,
-                                                                    int n_slots, const float* __restrict__ gw = nullptr,
-                                                                    float eps = 0.f) {
+template <int HPW, bool NORM = false, int WPH = 4>
+__global__ __launch_bounds__(64 * WPH * HPW) void gdn_decode_wide_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
+                                                                         const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
+                                                                         const float* __restrict__ dt_bias, float* ssm_pool,
+                                                                         const int* __restrict__ slots, const int* __restrict__ pos,
+                                                                         bf16_t* __restrict__ y, int n_slots,
+                                                                         const float* __restrict__ gw = nullptr, float eps = 0.f) {
     const unsigned id = xcd_remap(blockIdx.x, gridDim.x);
-    const int b = id / (HV / HPW), h = (id % (HV / HPW)) * HPW + (threadIdx.x >> 8);
-    const int slot = slots[b];
-    if ((unsigned)slot >= (unsigned)n_slots) return;
-    const int par = pos[b] & 1;
-    float* st = ssm_pool + (size_t)slot * HV * DV * DK;
-    gdn_tokens<8, HPW, NORM>(proj + (size_t)b * PW, conv_pool + (size_t)(slot * 2 + par) * 3 * CD,
-                             conv_pool + (size_t)(slot * 2 + (par ^ 1)) * 3 * CD, 0, cw, A_log, dt_bias, st, st, 0,
-                             y + (size_t)b * KD, 1, h, 0, gw, eps);
+    const int b = id / (HV / HPW), h = (id % (HV / HPW)) * HPW + (HPW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * WPH)) : 0);
+    const int slot = slots[b], p = pos[b];
+    gdn_tokens<32 / WPH, HPW, NORM, WPH>(proj + (size_t)b * PW, cw, A_log, dt_bias, y + (size_t)b * KD, 1, h, 0,
+                                         [&] { return decode_place(conv_pool, ssm_pool, slot, p, n_slots); }, gw, eps);
 }
 
 // batch_spec.deltanet_bm (qwen35/batch_spec.py:142-150): M chained tokens per sequence, snapshot pools in place
@@ -252,14 +291,16 @@ __global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restric
                                                          int n_entries) {
     int b, h, split;
     split_id<RS>(b, h, split);
-    const int ss = sslots[b], sl = sels[b];
-    if ((unsigned)ss >= (unsigned)n_entries || (unsigned)sl >= (unsigned)M) return;
-    const int par = pars[b] & 1;
-    const size_t hs = (size_t)HV * DV * DK;
-    gdn_tokens<RS>(proj + (size_t)b * M * PW, conv_pool + ((size_t)(ss * 2 + par) * M + sl) * 3 * CD,
-                   conv_pool + (size_t)(ss * 2 + (par ^ 1)) * M * 3 * CD, (size_t)3 * CD, cw, A_log, dt_bias,
-                   ssm_pool + ((size_t)ss * M + sl) * hs, ssm_pool + (size_t)ss * M * hs, hs, y + (size_t)b * M * KD, M,
-                   h, split);
+    const int s_in = sslots[b], sl_in = sels[b], pr = pars[b];
+    gdn_tokens<RS>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, [&] {
+        const int par = pr & 1;
+        const size_t hs = (size_t)HV * DV * DK;
+        const bool ok = (unsigned)s_in < (unsigned)n_entries && (unsigned)sl_in < (unsigned)M;
+        const int ss = ok ? s_in : 0, sl = ok ? sl_in : 0;
+        return Place{ok, conv_pool + ((size_t)(ss * 2 + par) * M + sl) * 3 * CD,
+                     conv_pool + (size_t)(ss * 2 + (par ^ 1)) * M * 3 * CD, (size_t)3 * CD, ssm_pool + ((size_t)ss * M + sl) * hs,
+                     ssm_pool + (size_t)ss * M * hs, hs};
+    });
 }
 
 // kernels.deltanet (qwen35/kernels.py:555-567): one sequence, starts from snapshot sel[0], writes M fresh snapshots
@@ -272,11 +313,13 @@ __global__ __launch_bounds__(256) void gdn_solo_kernel(const bf16_t* __restrict_
                                                        int n_snap) {
     int b, h, split;
     split_id<RS>(b, h, split);
-    const int sl = sel[0];
-    if ((unsigned)sl >= (unsigned)n_snap) return;
-    const size_t hs = (size_t)HV * DV * DK;
-    gdn_tokens<RS>(proj, cs_snap + (size_t)sl * 3 * CD, cs_out, (size_t)3 * CD, cw, A_log, dt_bias, st_snap + sl * hs,
-                   st_out, hs, y, M, h, split);
+    const int sl_in = sel[0];
+    gdn_tokens<RS>(proj, cw, A_log, dt_bias, y, M, h, split, [&] {
+        const size_t hs = (size_t)HV * DV * DK;
+        const bool ok = (unsigned)sl_in < (unsigned)n_snap;
+        const int sl = ok ? sl_in : 0;
+        return Place{ok, cs_snap + (size_t)sl * 3 * CD, cs_out, (size_t)3 * CD, st_snap + sl * hs, st_out, hs};
+    });
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -354,13 +397,14 @@ int qt_gdn_decode_step_gnorm(const void* proj, void* conv_pool, const void* conv
     if (B < 0 || n_slots <= 0) return QT_ERR_DIM;
     if (B == 0) return QT_OK;
     if (!aligned16(ssm_pool) || (reinterpret_cast<uintptr_t>(conv_w) & 7u)) return QT_ERR_ALIGN;
-#define QT_GNORM_LAUNCH(HPW_)                                                                                                  \
-    hipLaunchKernelGGL((gdn_decode_wide_kernel<HPW_, true>), dim3(B * (HV / HPW_)), dim3(256 * HPW_), 0, stream, (const bf16_t*)proj, \
+#define QT_GNORM_LAUNCH(HPW_, WPH_)                                                                                                  \
+    hipLaunchKernelGGL((gdn_decode_wide_kernel<HPW_, true, WPH_>), dim3(B * (HV / HPW_)), dim3(64 * WPH_ * HPW_), 0, stream, (const bf16_t*)proj, \
                        (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log, dt_bias, ssm_pool, slots, pos, (bf16_t*)out, n_slots, gw, eps)
     const int hpw = decode_heads_per_wg(B);
-    if (hpw == 4) QT_GNORM_LAUNCH(4);
-    else if (hpw == 2) QT_GNORM_LAUNCH(2);
-    else QT_GNORM_LAUNCH(1);
+    if (hpw == 4) QT_GNORM_LAUNCH(4, 4);
+    else if (hpw == 2) QT_GNORM_LAUNCH(2, 4);
+    else if (4L * B * HV <= cu_count()) QT_GNORM_LAUNCH(1, 8);   // (8 against 4 wavefronts a head, us: 1 row 4.4 / 4.7, 4 rows 4.9 / 5.0, 8 rows 5.9 / 5.4)
+    else QT_GNORM_LAUNCH(1, 4);
     QT_CHECK_LAUNCH();
     return QT_OK;
 }

@@ -344,13 +344,17 @@ __device__ __forceinline__ void rsqrt_rows4(const double (&ss)[4], float eps, fl
     const float rv = rsqrt_rn((float)t / 128.0f + eps);
     r[0] = row16_bcast<4>(rv), r[1] = row16_bcast<5>(rv), r[2] = row16_bcast<6>(rv), r[3] = row16_bcast<7>(rv);
 }
-// total over the whole 64-lane wavefront (every lane gets it)
-__device__ __forceinline__ double wave_sum_d(double v) {
-    v = row16_sum_d(v);
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    return v;
+// sum over the four lanes n, n + 16, n + 32, n + 48 with the vector-ALU lane swaps (a shuffle goes through the LDS pipeline)
+__device__ __forceinline__ double groups_sum_d(double v) {
+    auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
+    auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
+    v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
+    hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
 }
+// total over the whole 64-lane wavefront (every lane gets it)
+__device__ __forceinline__ double wave_sum_d(double v) { return groups_sum_d(row16_sum_d(v)); }
 __device__ __forceinline__ float wave_sum(float v) {
     v = row16_sum(v);
     v += __shfl_xor(v, 16, 64);

@@ -421,7 +421,7 @@ def test_deltanet_bm_config4_size(qt, dev):
     check_equal("trash entry", got[NS], sp[NS])
 
 
-@pytest.mark.parametrize("B", [1, 5, 24, 32, 48, 64, 80])
+@pytest.mark.parametrize("B", [1, 4, 5, 24, 32, 48, 64, 80])
 def test_deltanet_b_gnorm_equals_two_launches(qt, dev, B):
     """the decode step with the gated RMSNorm fused in == deltanet_b followed by gnorm_rows (batch.py:497-499), bit for bit,
     for each workgroup shape the batch size selects (1, 2 or 4 heads per workgroup)"""
@@ -443,6 +443,43 @@ def test_deltanet_b_gnorm_equals_two_launches(qt, dev, B):
     check_tensors_equal("conv pool", c2, c1)
     check_tensors_equal("ssm pool", s2, s1)
     check_equal("against the oracle", to_np(got), O.gated_norm(to_np(y), to_np(proj), gw))
+
+
+@pytest.mark.parametrize("B", [3, 6, 20, 36])
+def test_skipped_rows_between_others(qt, dev, B):
+    """a row whose slot lies outside the pools reads, but writes nothing, whichever workgroup shape takes it: the other rows get what they
+    get without it, and slot 0, which no row names, keeps its bits"""
+    gen = torch.Generator().manual_seed(300 + B)
+    cw, A_log, dtb, gw = layer_params(30 + B)
+    args = [to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev)]
+    dgw = to_dev(gw, dev)
+    proj = to_dev(rand_bf(gen, (B, PW), 1.0), dev, BF16)
+    ssm = to_dev((torch.randn((B + 1, 16, 128, 128), generator=gen) * 0.05).numpy(), dev)
+    conv = to_dev(rand_bf(gen, ((B + 1) * 2, 3, CD)), dev, BF16)
+    slots, pos = torch.arange(1, B + 1, dtype=torch.int32), torch.randint(0, 9, (B,), generator=gen, dtype=torch.int32)
+    slots[1], slots[B - 1] = -1, B + 1
+    good = [b for b in range(B) if 0 <= slots[b] <= B]
+    i = torch.tensor(good, device=dev)
+    c1, s1, c2, s2 = conv.clone(), ssm.clone(), conv.clone(), ssm.clone()
+    want = qt.batch.deltanet_b_gnorm(proj[i], c1, *args, s1, slots[good].to(dev), pos[good].to(dev), dgw)
+    got = qt.batch.deltanet_b_gnorm(proj, c2, *args, s2, slots.to(dev), pos.to(dev), dgw)
+    check_tensors_equal("rows", got[i], want)
+    check_tensors_equal("conv pool", c2, c1)
+    check_tensors_equal("ssm pool", s2, s1)
+    M, n = 2, B + 1                                               # the verify step, with entries and snapshots outside theirs
+    pv = to_dev(rand_bf(gen, (B * M, PW), 1.0), dev, BF16)
+    ssv = to_dev((torch.randn((n, M, 16, 128, 128), generator=gen) * 0.05).numpy(), dev)
+    cv = to_dev(rand_bf(gen, (n * 2, M, 3, CD)), dev, BF16)
+    sels, pars = torch.randint(0, M, (B,), generator=gen, dtype=torch.int32), torch.randint(0, 2, (B,), generator=gen, dtype=torch.int32)
+    sels[0] = M
+    good = [b for b in range(1, B) if 0 <= slots[b] <= B]
+    rows = torch.tensor([b * M + j for b in good for j in range(M)], device=dev)
+    c1, s1, c2, s2 = cv.clone(), ssv.clone(), cv.clone(), ssv.clone()
+    want = qt.batch_spec.deltanet_bm(pv[rows], c1, *args, s1, slots[good].to(dev), sels[good].to(dev), pars[good].to(dev), M)
+    got = qt.batch_spec.deltanet_bm(pv, c2, *args, s2, slots.to(dev), sels.to(dev), pars.to(dev), M)
+    check_tensors_equal("verify rows", got[rows], want)
+    check_tensors_equal("verify conv pool", c2, c1)
+    check_tensors_equal("verify ssm pool", s2, s1)
 
 
 def test_a_missing_norm_weight_is_refused(qt, dev):
