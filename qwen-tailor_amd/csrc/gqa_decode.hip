@@ -152,6 +152,9 @@ constexpr int MAX_SEG = 2048;          // segments (2 per sequence) a launch can
 // workgroup whose range crosses a segment border gets fewer tiles to stream.  Layer form, us, with 3 / 5 / 7 positions: 32 sequences of
 // 1000 - 8000 keys 55.4 / 54.9 / 55.7, 64 of 200 - 2000 37.9 / 38.1 / 38.3, 16 of 512 - 32768 92.7 / 90.8 / 91.2, 5 x 3 rows of 90 - 900 17.0 /
 // 16.7 / 16.9.
+// A range that holds nothing but such positions of a segment does not visit it.  (When it did, for the new keys, a workgroup paid a visit, 3.3
+// us, for no tile: 1 of 300 keys 14.0 us, 5 x 3 of 90 - 900 16.2, 16 of 100 - 1000 16.4, 64 of 50 - 200 17.5; without these visits and
+// with a default split of 32 keys instead of 128 9.5 / 12.4 / 12.8 / 15.3.)
 constexpr int VISIT_TILES = 5;
 
 
@@ -253,24 +256,25 @@ __global__ __launch_bounds__(256, 2) void attn_partial_kernel(const bf16_t* __re
         load_rows(base);
         lane_end = seg_start[min(base + lane, nseg - 1) + 1];
     };
-    // A visit is the part of one segment that lies in this workgroup's range: its number (-1: there is none), slot, position of the
-    // pass's first row, pool keys [lo, hi), and whether the range holds the segment's first tile.  All of it is scalar.
+    // A visit is the part of one segment's tiles that lies in this workgroup's range: its number (-1: there is none), slot, position of
+    // the pass's first row, pool keys [lo, hi), and whether the range holds the segment's first tile.  All of it is scalar.  (A range that
+    // holds only empty positions of a segment does not visit it.)
     auto find_visit = [&](int sg, int begin, int& v_sg, int& v_slot, int& v_p0, int& v_lo, int& v_hi, int& v_first) {
         // the first one at or after segment sg, which begins at `begin`
         int end = 0;
-        for (; sg < nseg && begin < wt1; sg++) {
+        for (; sg < nseg && begin + VISIT_TILES < wt1; sg++) {
             if (sg - win >= 64) move_window(sg);
             end = __builtin_amdgcn_readlane(lane_end, sg - win);
             if (end != begin) break;                             // (otherwise a skipped row)
         }
-        const bool found = sg < nseg && begin < wt1;
+        const bool found = sg < nseg && begin + VISIT_TILES < wt1;
         const int at = found ? sg - win : 0;
         v_sg = __builtin_amdgcn_readfirstlane(found ? sg : -1);
         v_slot = __builtin_amdgcn_readlane(lane_slot, at);
         v_p0 = __builtin_amdgcn_readlane(lane_pos, at) + j0;
-        v_first = __builtin_amdgcn_readfirstlane(wt0 <= begin);
-        v_lo = __builtin_amdgcn_readfirstlane(max(0, max(wt0, begin) - begin - VISIT_TILES) * 16);
-        v_hi = __builtin_amdgcn_readfirstlane(min(max(0, min(wt1, end) - begin - VISIT_TILES) * 16, v_p0));
+        v_first = __builtin_amdgcn_readfirstlane(wt0 <= begin + VISIT_TILES);
+        v_lo = __builtin_amdgcn_readfirstlane(max(0, wt0 - begin - VISIT_TILES) * 16);
+        v_hi = __builtin_amdgcn_readfirstlane(min((min(wt1, end) - begin - VISIT_TILES) * 16, v_p0));
     };
     auto end_of = [&](int sg) { return __builtin_amdgcn_readlane(lane_end, sg - win); };
     if (nseg > 64) move_window(sg0);
@@ -581,10 +585,15 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
     const int total = seg_tab[B * AKV], ss = seg_tab[sg], se = seg_tab[sg + 1];   // written by the partial kernel
     if (se == ss) return;                                        // a skipped row
     const int per = tiles_per_wg(total, nwg, min_tiles);
-    const int wg0 = ss / per, ns = (se - 1) / per - wg0 + 1;     // the workgroups that hold tiles of this segment
+    const int wg0 = (ss + VISIT_TILES) / per, ns = (se - 1) / per - wg0 + 1;     // the workgroups that hold tiles of this segment
     const size_t base = (size_t)wg0 + sg;                        // their partials sit in consecutive slots
     const float* ml = part_ml + (base * R + r) * 2;              // slot stride 2 R floats
     const float* po = part_o + (base * R + r) * AD + lane * 4;   // slot stride R * AD floats
+    // this wavefront's first four partials are requested beside the factors' inputs: one memory latency less with few partials (layer form,
+    // 1 of 300 keys 10.4 -> 9.5 us, 16 of 100 - 1000 13.7 -> 12.8)
+    f32x4 first[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) first[i] = *reinterpret_cast<const f32x4*>(po + (size_t)min(w + 4 * i, ns - 1) * R * AD);
     float mx = NEG;
     for (int s = tid; s < ns; s += 256) mx = fmaxf(mx, ml[(size_t)s * 2 * R]);
     mx = wave_max(mx);
@@ -602,7 +611,10 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
     __syncthreads();
     const float l = (red_l[0] + red_l[1]) + (red_l[2] + red_l[3]);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    int s = w;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (w + 4 * i < ns) acc += first[i] * fs_s[w + 4 * i];
+    int s = w + 16;
     for (; s + 12 < ns; s += 16) {
         f32x4 ov[4];
 #pragma unroll

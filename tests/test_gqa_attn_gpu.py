@@ -74,6 +74,16 @@ def test_attn_b_split_invariance_and_single_key(qt, dev):
     check_equal("single key: o == v", outs[0][1], np.repeat(vn[1], 4, axis=0))
 
 
+@pytest.mark.parametrize("B,M,hi,split", [(1, 1, 20, 16), (2, 1, 40, 32), (5, 2, 50, 16), (9, 1, 33, 48), (33, 1, 60, 16), (40, 3, 20, 32), (70, 1, 40, 16)])
+def test_attn_b_ranges_of_empty_positions(qt, dev, B, M, hi, split):
+    """short segments and small splits: many a workgroup's range is, or begins or ends with, the empty positions in front of a segment.  Such a
+    range does not visit it; the new keys belong to the workgroup with the segment's first tile, and the merge counts the same ones."""
+    rng = np.random.default_rng(B * 7 + M)
+    pos = rng.integers(0, hi, B).astype(np.int32)
+    pos[:min(B, 4)] = [0, 16, 1, 15][:min(B, 4)]
+    run_case(qt, dev, rng, B, hi + 48, rng.permutation(B).astype(np.int32), pos, M, split=split)
+
+
 def test_attn_b_out_of_range_rows_are_skipped(qt, dev):
     rng = np.random.default_rng(6)
     Kp = to_dev(bf(rng.standard_normal((3, 2, 64, 256))), dev, BF16)
