@@ -4,7 +4,8 @@
 //
 // attn_prefill_kernel<NH>: one workgroup = 16 NH query rows x the 4 query heads that share a KV head, on eight wavefronts in
 // two roles; NH = heads per pair of wavefronts:
-//   NH = 2   32 rows; every K or V fragment read from LDS feeds two MFMAs (one per head): launches of about 1500 rows and more
+//   NH = 2   32 rows; every K or V fragment read from LDS feeds two MFMAs (one per head): launches of about 1500 rows and more, fewer behind
+//            a long prefix
 //   NH = 1   16 rows: twice the workgroups (and twice the LDS traffic per MFMA), for launches that would leave CUs idle
 // The arithmetic, per 64-key tile and 16 rows of a head:
 //     S^T[keys x rows] = K_tile . Q^T     A = K rows from LDS, B = Q^T resident in registers (16x16x32 bf16 MFMA)
@@ -62,6 +63,15 @@ __device__ __forceinline__ void lds_dma16(const char* base, unsigned voff, unsig
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%4\n\ts_mov_b32 m0, %0"
                  : "=&s"(keep)
                  : "v"(voff), "s"(base), "s"(la), "n"(IMM)
+                 : "memory");
+}
+// ... and from an address of each lane's own
+__device__ __forceinline__ void lds_dma16_from(const char* src, unsigned lds) {
+    const unsigned la = __builtin_amdgcn_readfirstlane(lds);
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(src), "s"(la)
                  : "memory");
 }
 // four such loads, KiB 0 .. 3 behind lds, under one setting of M0 (a wavefront issues one instruction every four clocks, and
@@ -211,8 +221,11 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
     const int ka_row = n * AD;
     // transposing load: within 16 lanes, lane 4q + i receives element i of the 8-byte chunks addressed by lanes q, q+4,
     // q+8, q+12; lane n of group g points at key 4g + n/4, columns 4 (n%4).. of the block and receives keys 4g..4g+3 of column n
+    // Blocks j and j + 1 (j even) share 32 columns: the four lanes of a key take a 16-byte chunk each, and block j the lower half of it in the
+    // even and the upper half in the odd lanes, block j + 1 the other halves.  Afterwards lane group g holds eight adjacent columns in its
+    // two blocks (16-byte stores), and a fragment read still touches every bank twice.
     const int vrow = 4 * g + (n >> 2);                           // row within a 16-key block = its swizzle
-    const int va_row = vrow * AD + 4 * (n & 1), vc0 = (n & 3) >> 1;
+    const int va_row = vrow * AD, vq = n & 3;
     // K fragment kb of sub-tile kt: chunk (4 kb + g) ^ n; n < 16 leaves bit 4 alone, so fragments kb and kb + 4 share an
     // address register
     auto k_frag = [&](const bf16_t* ka, int kt, int kb) {
@@ -221,8 +234,18 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
 
     if (tid < 4) taken_s[tid] = -1, moved_s[tid] = 0;
     if (tid < 4 * NH * 16) (&m_s[0][0][0])[tid] = NEG;
+    bf16_t* const q_s = kv_s + 2 * TILE;                         // Q waits in the V buffers, [pair][head][16 rows][256], swizzled as the tiles
     if (ta < tb) {                                               // (a part past the block's last tile is empty)
         load_four(kg, lds_address(kv_s), ta, ld_off0);
+        // Q goes through LDS as well, whole rows per load: as the score wavefronts' operand it would be asked for 16 bytes of 16 rows at a
+        // time, which a CU takes in at a quarter of the rate (1.2 us of a workgroup with 32 rows).  Rows past the end repeat the last one.
+#pragma unroll
+        for (int i = 0; i < 4 * NH; i++) {
+            const int piece = 4 * NH * w + i, qp = piece / (8 * NH), qh = piece / 8 % NH, rr = 2 * (piece & 7) + (lane >> 5);
+            const int qrow = min(rb * RB + (NH == 2 ? 16 * (qp >> 1) : 0) + rr, S - 1), head = kvh * (AH / AKV) + (NH == 2 ? 2 * (qp & 1) + qh : qp);
+            lds_dma16_from(reinterpret_cast<const char*>(q + (size_t)head * q_head_stride + (size_t)qrow * q_row_stride + 8 * ((lane & 31) ^ rr)),
+                           lds_address(kv_s) + 4 * TILE + 1024 * piece);
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (tb - ta > 1) load_four(kg, lds_address(kv_s) + 2 * TILE, ta + 1, ld_off0);
@@ -234,15 +257,9 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         // Q^T as the B operand of the score MFMA: lane (row n, group g) holds q[row][32 kb + 8 g .. + 8] of each head
         bf16x8 bq[NH][8];
 #pragma unroll
-        for (int hh = 0; hh < NH; hh++) {
-            const u32x4* qr = reinterpret_cast<const u32x4*>(q + (size_t)(h0 + hh) * q_head_stride + (size_t)(row_ok ? row : 0) * q_row_stride);
+        for (int hh = 0; hh < NH; hh++)
 #pragma unroll
-            for (int kb = 0; kb < 8; kb++) {
-                u32x4 v = qr[kb * 4 + g];
-                if (!row_ok) v = u32x4{0, 0, 0, 0};
-                bq[hh][kb] = __builtin_bit_cast(bf16x8, v);
-            }
-        }
+            for (int kb = 0; kb < 8; kb++) bq[hh][kb] = k_frag(q_s + (pr * NH + hh) * 16 * AD + ka_row, 0, kb);
         float m_run[NH];
 #pragma unroll
         for (int hh = 0; hh < NH; hh++) m_run[hh] = NEG;
@@ -436,6 +453,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         return;
     }
     // ---------------------------------------------------------------------------------------------- output wavefront
+    // O^T: block j of lane (n, g) holds row n of the pair's rows, columns col_of(j) .. + 3 (below); every element of Lsum is row n's sum
     f32x4 O[NH][16];
     f32x4 Lsum[NH];                                                  // row sums of P, accumulated by MFMA against a block of ones
 #pragma unroll
@@ -470,17 +488,17 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         for (int hh = 0; hh < NH; hh++)
 #pragma unroll
             for (int pp = 0; pp < 2; pp++) P[hh][pp] = __builtin_bit_cast(s16x8, p_s[pr][hh][pp][lane]);
-        f32x4 c4[NH];
+        float cr[NH];
 #pragma unroll
-        for (int hh = 0; hh < NH; hh++) c4[hh] = mv ? *reinterpret_cast<const f32x4*>(&c_s[pr][hh][4 * g]) : f32x4{1.f, 1.f, 1.f, 1.f};
+        for (int hh = 0; hh < NH; hh++) cr[hh] = mv ? c_s[pr][hh][n] : 1.f;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         *lds_word(&taken_s[pr]) = t;
         asm volatile("" ::: "memory");
         const bf16_t* va = v_cur + va_row;
         auto v_frag = [&](int j, int q4) {
             return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4*)(const_cast<bf16_t*>(va + (16 * q4) * AD + (((2 * (j & 7) + vc0) ^ vrow) << 3) +
-                                                                             128 * (j >> 3))));
+                (__attribute__((address_space(3))) s16x4*)(const_cast<bf16_t*>(va + (16 * q4) * AD + (((4 * ((j >> 1) & 3) + vq) ^ vrow) << 3) +
+                                                                             4 * ((vq ^ j) & 1) + 128 * (j >> 3))));
         };
         s16x4 Bf[V_FRAG_AHEAD + 1][4];
 #pragma unroll
@@ -491,8 +509,8 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
 #pragma unroll
             for (int hh = 0; hh < NH; hh++) {
 #pragma unroll
-                for (int j = 0; j < 16; j++) O[hh][j] *= c4[hh];
-                Lsum[hh] *= c4[hh];
+                for (int j = 0; j < 16; j++) O[hh][j] *= cr[hh];
+                Lsum[hh] *= cr[hh];
             }
         }
         PHASE_FENCE();
@@ -504,8 +522,8 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
             for (int pp = 0; pp < 2; pp++)
 #pragma unroll
                 for (int hh = 0; hh < NH; hh++)
-                    Lsum[hh] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, P[hh][pp]),
-                                                                      __builtin_bit_cast(bf16x8, ones), Lsum[hh], 0, 0, 0);
+                    Lsum[hh] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ones),
+                                                                      __builtin_bit_cast(bf16x8, P[hh][pp]), Lsum[hh], 0, 0, 0);
         }
         const unsigned step_off0 = opaque_off0();
 #pragma unroll
@@ -523,8 +541,8 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
                 const s16x8 B = __builtin_shufflevector(Bf[j % (V_FRAG_AHEAD + 1)][2 * pp], Bf[j % (V_FRAG_AHEAD + 1)][2 * pp + 1], 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
                 for (int hh = 0; hh < NH; hh++)
-                    O[hh][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, P[hh][pp]),
-                                                                      __builtin_bit_cast(bf16x8, B), O[hh][j], 0, 0, 0);
+                    O[hh][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, B),
+                                                                      __builtin_bit_cast(bf16x8, P[hh][pp]), O[hh][j], 0, 0, 0);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -532,41 +550,53 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
     }
     if (ta < tb)
         for (int t = max(tw, ta) + 1; t <= tb; t++) idle_iter(t);
-    // ---- normalise and store: lane (n, g) holds rows 4g .. 4g+3 of column 16 j + n, and of the row sums (any column)
+    // ---- normalise and store: lane (n, g) holds row n, columns 32 jj + 8 g .. + 7 in blocks 2 jj and 2 jj + 1 (odd g: the other way round)
+    auto columns = [&](const f32x4 (&o)[16], int jj, float scale, f32x4& lo, f32x4& hi) {
+        const bool odd = g & 1;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float a = o[2 * jj][i] * scale, b = o[2 * jj + 1][i] * scale;
+            lo[i] = odd ? b : a, hi[i] = odd ? a : b;
+        }
+    };
     if (nparts > 1) {
         // One part of several: leave O / l, m, l of this pair's heads as they are.  A row that sees no key of this part (its
         // last key lies before the part's first) has exponentiated masked scores against a masked maximum: it is written as
         // the neutral element (m = NEG, l = 0, O = 0).
-        const int first_key = ta * KT, lr0 = r0 - rb * RB;
+        const int lr = r0 - rb * RB + n;
+        const bool seen = my_last >= ta * KT;
 #pragma unroll
         for (int hh = 0; hh < NH; hh++) {
             const int hq = hq0 + hh;
-            _Float16* po = part_o + (slot * 4 + hq) * (RB * AD);
+            _Float16* po = part_o + (slot * 4 + hq) * (RB * AD) + lr * AD + 8 * g;
             float* pml = part_ml + (slot * 4 + hq) * (2 * RB);
+            const float inv = 1.0f / Lsum[hh][0];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int lr = lr0 + 4 * g + r;
-                const bool seen = q_pos0 + rb * RB + lr >= first_key;
-                const float inv = seen ? 1.0f / Lsum[hh][r] : 0.f;
+            for (int jj = 0; jj < 8; jj++) {
+                f32x4 lo, hi;
+                columns(O[hh], jj, inv, lo, hi);
+                half8 h;
 #pragma unroll
-                for (int j = 0; j < 16; j++) po[lr * AD + 16 * j + n] = (_Float16)(seen ? O[hh][j][r] * inv : 0.f);
-                if (n == 0) pml[RB + lr] = seen ? Lsum[hh][r] : 0.f;
+                for (int i = 0; i < 4; i++) h[i] = (_Float16)(seen ? lo[i] : 0.f), h[4 + i] = (_Float16)(seen ? hi[i] : 0.f);
+                *reinterpret_cast<half8*>(po + 32 * jj) = h;
             }
-            if (g == 0) pml[lr0 + n] = my_last >= first_key ? m_s[pr][hh][n] : NEG;
+            if (g == 0) {
+                pml[RB + lr] = seen ? Lsum[hh][0] : 0.f;
+                pml[lr] = seen ? m_s[pr][hh][n] : NEG;
+            }
         }
         return;
     }
+    if (!row_ok) return;
 #pragma unroll
     for (int hh = 0; hh < NH; hh++) {
+        const float inv = 1.0f / Lsum[hh][0];
+        bf16_t* dst = out + (size_t)(h0 + hh) * q_head_stride + (size_t)row * q_row_stride + 8 * g;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int orow = r0 + 4 * g + r;
-            if (orow < S) {
-                const float inv = 1.0f / Lsum[hh][r];
-                bf16_t* dst = out + (size_t)(h0 + hh) * q_head_stride + (size_t)orow * q_row_stride + n;
-#pragma unroll
-                for (int j = 0; j < 16; j++) dst[16 * j] = f2bf(O[hh][j][r] * inv);
-            }
+        for (int jj = 0; jj < 8; jj++) {
+            f32x4 lo, hi;
+            columns(O[hh], jj, inv, lo, hi);
+            *reinterpret_cast<u32x4*>(dst + 32 * jj) = u32x4{pack2_bf(lo[0], lo[1]), pack2_bf(lo[2], lo[3]), pack2_bf(hi[0], hi[1]), pack2_bf(hi[2], hi[3])};
         }
     }
 }
@@ -589,23 +619,49 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16*
         if (rb * RB + lr >= S) return;
         const _Float16* po = part_o + (slot0 * 4 + hq) * (RB * AD) + lr * AD + cg * 16;
         const float* pml = part_ml + (slot0 * 4 + hq) * (2 * RB) + lr;
+        // AHEAD parts at a time, all their loads in flight together (an index past the last part loads the last again); the first ones are
+        // requested before the maximum is known
+        constexpr int AHEAD = 4;
+        half8 oh[AHEAD][2];
+        float pm[AHEAD], pl[AHEAD];
+        auto load = [&](int p0) {
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) {
+                const size_t pp = min(p0 + i, np - 1);
+                pm[i] = pml[pp * PML], pl[i] = pml[pp * PML + RB];
+                oh[i][0] = reinterpret_cast<const half8*>(po + pp * PO)[0], oh[i][1] = reinterpret_cast<const half8*>(po + pp * PO)[1];
+            }
+        };
+        load(0);
+        __builtin_amdgcn_sched_barrier(0);
         float m = NEG;
-        for (int pp = 0; pp < np; pp++) m = fmaxf(m, pml[(size_t)pp * PML]);
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) m = fmaxf(m, pm[i]);
+        for (int p0 = AHEAD; p0 < np; p0 += AHEAD) {
+            float mv[AHEAD];
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) mv[i] = pml[(size_t)min(p0 + i, np - 1) * PML];
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) m = fmaxf(m, mv[i]);
+        }
         float l = 0.f;
         f32x4 acc[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-        for (int pp = 0; pp < np; pp++) {
-            half8 oh[2];
+        for (int p0 = 0;;) {
 #pragma unroll
-            for (int i = 0; i < 2; i++) oh[i] = reinterpret_cast<const half8*>(po + (size_t)pp * PO)[i];
-            const float f = __builtin_amdgcn_exp2f(pml[(size_t)pp * PML] - m) * pml[(size_t)pp * PML + RB];
-            l += f;
+            for (int k = 0; k < AHEAD; k++) {
+                if (p0 + k >= np) break;
+                const float f = __builtin_amdgcn_exp2f(pm[k] - m) * pl[k];
+                l += f;
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+                for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) acc[i][e] += f * (float)oh[i >> 1][4 * (i & 1) + e];
+                    for (int e = 0; e < 4; e++) acc[i][e] += f * (float)oh[k][i >> 1][4 * (i & 1) + e];
+            }
+            p0 += AHEAD;
+            if (p0 >= np) break;
+            load(p0);
         }
         const float inv = 1.0f / l;
         uint32_t pk[8];
@@ -628,11 +684,9 @@ inline bool two_heads_per_wave(int S) { return (S + 31) / 32 * AKV >= 288; }   /
 
 // The key split of a launch: tmax = 0 (none) or the tiles per part, parts = grid width, split_blocks = blocks with several parts.
 // Only launches that leave CUs without a workgroup are split (fewer than 2048 query rows: a short continuation of a long
-// prefix, a short prompt), and only as far as the idle CUs go: a part holds the smallest number of tiles (from the launch's
-// average per CU, at least 6) with which all parts are resident at once, and the split must shorten the longest workgroup
-// by six tiles or more to pay for the merge launch.  A workgroup costs
-// about 6 us beyond its tiles (dispatch, Q and first-tile latency, the output stores): measured at S = 2048 (256 workgroups,
-// 57 us unsplit) every part size from 4 to 32 tiles came out between 53 and 61 us before the parts were even merged.
+// prefix, a short prompt), and only as far as the idle CUs go; the split must shorten the longest workgroup by four tiles or more to pay for
+// the merge launch (200 rows on 100 keys, by two: 11.8 us against 10.7; 333 rows, by three: 12.0 against 11.4; 100 rows on 300 keys, by
+// four: 12.0 against 13.1).  A workgroup costs about 6 us beyond its tiles (dispatch, Q and first-tile latency, the output stores).
 struct KeySplit {
     int nh = 1;            // heads per wavefront: row blocks of 16 nh rows
     int tmax = 0;
@@ -652,12 +706,20 @@ KeySplit plan_split_nh(int S, int L, int q_pos0, int nh, int min_gain) {
         total += nt;
         longest = std::max(longest, nt);
     }
-    // the smallest part size (from the average per CU, at least 6 tiles) whose parts are all resident at once: a CU that has
-    // to run a second part pays the per-workgroup cost twice.  (A floor of 6 against 8, us: 768 rows 18.1 / 20.7, 1536 rows
-    // 28.9 / 29.9, one row after 4095 keys 19.6 / 21.1, 64 rows after 8000 keys 29.4 / 27.6; 5 and 7 are worse on more shapes.)
+    // the part size (from the average per CU, at least 3 tiles) with the least time among those whose parts are all resident at once: a CU
+    // that has to run a second part pays the per-workgroup cost twice.  In us, fitted to a sweep of 17 - 1460 rows on 0 - 6000 keys: a tile
+    // 1.25 (32-row blocks 1.8), a part 0.033 in the merge (twice that), and 0.85 for every four parts that the merge takes one after the
+    // other.  (At least 6 tiles always, against this: 17 rows on 700 / 1500 keys 15.1 / 15.3 and 11.5 / 12.7, 100 rows on 700 / 3000 15.4 / 18.8
+    // and 13.1 / 17.8, 333 on 300 / 1500 16.3 / 19.6 and 13.9 / 19.2, 700 rows 17.1 and 15.4.)
     const long p = (q_pos0 + RB - 1) / RB, cpt = KT / RB;
-    int tmax = (int)std::max(6L, (total * AKV + cus - 1) / cus);
-    while (tmax < longest && (parts_upto(p + nb, cpt * tmax) - parts_upto(p, cpt * tmax)) * AKV > cus) tmax++;
+    int tmax = longest;
+    float least = 1e30f;
+    for (int t = (int)std::max(3L, (total * AKV + cus - 1) / cus); t <= longest; t++) {
+        const long parts = (parts_upto(p + nb, cpt * t) - parts_upto(p, cpt * t)) * AKV, most = (p + nb + cpt * t - 1) / (cpt * t);
+        if (parts > cus) continue;
+        const float us = (nh == 1 ? 1.25f : 1.8f) * t + 0.033f * nh * parts + 0.85f * ((most + 3) / 4);
+        if (us < least) least = us, tmax = t;
+    }
     if (longest - tmax < min_gain) return ks;                    // the merge launch has to be earned
     const long c = cpt * tmax;
     ks.tmax = tmax;
@@ -671,10 +733,14 @@ KeySplit plan_split_nh(int S, int L, int q_pos0, int nh, int min_gain) {
 //   from about 4600 rows on     NH = 2, unsplit (enough 32-row blocks to balance themselves);
 //   from about 1500 rows on     NH = 2 with the key split, where the launch leaves room for it and, for a whole prompt, up to
 //                               3200 rows (a tile of a 32-row block costs less than two tiles of 16-row blocks, but its parts
-//                               are twice the size); after a prefix NH = 2 wins by more;
+//                               are twice the size);
+//   fewer rows, split           the form whose parts are shorter in time: a workgroup with 32 rows costs 3.5 us more besides its tiles, and
+//                               a tile 1.8 against 1.25 us.  (NH = 1 / 2, us: 333 rows on 1500 / 6000 / 8000 keys 19.5 / 22.3, 30.2 / 29.7,
+//                               41.9 / 35.4, 700 on 700 / 1500 / 3000 / 6000 21.9 / 25.6, 26.8 / 26.6, 37.6 / 32.2, 77.9 / 49.7, 1300 on 300 / 1500 /
+//                               6000 26.8 / 27.5, 47.5 / 38.2, 153 / 82.6);
 //   everything else             NH = 1, split if CUs would idle.
 KeySplit plan_split(int S, int L, int q_pos0) {
-    if (two_heads_per_wave(S)) {                                 // (two heads: S >= 1472 in every case, so L >= one tile)
+    if (two_heads_per_wave(S)) {                                 // (two heads: S >= 1472, or parts of several tiles, so L >= one tile)
         KeySplit ks;
         ks.nh = 2;
         return ks;
@@ -683,7 +749,12 @@ KeySplit plan_split(int S, int L, int q_pos0) {
         const KeySplit ks = plan_split_nh(S, L, q_pos0, 2, 4);
         if (ks.tmax) return ks;
     }
-    return plan_split_nh(S, L, q_pos0, 1, 6);
+    const KeySplit one = plan_split_nh(S, L, q_pos0, 1, 4);
+    if (one.tmax) {
+        const KeySplit two = plan_split_nh(S, L, q_pos0, 2, 4);
+        if (two.tmax && 1.25f * one.tmax - 1.8f * two.tmax > 3.5f) return two;
+    }
+    return one;
 }
 
 }  // namespace
