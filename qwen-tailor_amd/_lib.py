@@ -93,7 +93,8 @@ class _Host:
     The module is loaded (and built, if it is missing or out of date) when the first of them is asked for."""
 
     FUNCTIONS = ("rms_rows", "fused_gemv", "gated_norm", "decode_step", "decode_step_gnorm", "verify_step", "deltanet", "attn_b", "attn_layer_b",
-                 "sdpa", "qkv_prep", "out_gate", "conv_prep", "phase_a", "phase_b", "phase_b_norm", "gdn_core", "blit_batch", "pools_load")
+                 "sdpa", "qkv_prep", "out_gate", "conv_prep", "phase_a", "phase_b", "phase_b_norm", "gdn_core", "blit_batch", "pools_load",
+                 "cache_restore")
 
     def __getattr__(self, name):
         if name not in self.FUNCTIONS:

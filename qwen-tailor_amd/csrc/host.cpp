@@ -761,32 +761,43 @@ struct Jobs {
     }
     void reserve(size_t n) { held.reserve(2 * n), dst.reserve(n), src.reserve(n), meta.reserve(7 * n); }
     void add(PyObject* dest, PyObject* source, long n, long d0, long s0, long ny, long ds, long ss) {
-        const Tensor &d = gpu_tensor(dest, "dst"), &s = gpu_tensor(source, "src");
-        const std::string who = "blit_batch: job " + std::to_string(dst.size());
+        add(gpu_tensor(dest, "dst"), source, n, d0, s0, ny, ds, ss);
+        Py_INCREF(dest);
+        held.push_back(dest);
+    }
+    // (a destination that the caller keeps)
+    void add(const Tensor& d, PyObject* source, long n, long d0, long s0, long ny, long ds, long ss) {
+        add(d, gpu_tensor(source, "src"), n, d0, s0, ny, ds, ss);
+        Py_INCREF(source);
+        held.push_back(source);
+    }
+    void add(const Tensor& d, const Tensor& s, long n, long d0, long s0, long ny, long ds, long ss) {
+        const auto who = [&] { return "blit_batch: job " + std::to_string(dst.size()); };
         if (d.scalar_type() != s.scalar_type() || (d.scalar_type() != BF16 && d.scalar_type() != F32))
-            type_error(who + ": bf16 or float32 tensors of one dtype expected");
+            type_error(who() + ": bf16 or float32 tensors of one dtype expected");
         check_layout(d, d.scalar_type(), "dst");
         check_layout(s, s.scalar_type(), "src");
-        if (n < 0 || ny < 0 || d0 < 0 || s0 < 0 || ds < 0 || ss < 0) value_error(who + ": negative size, offset or stride");
+        if (n < 0 || ny < 0 || d0 < 0 || s0 < 0 || ds < 0 || ss < 0) value_error(who() + ": negative size, offset or stride");
         // `ny` rows of n elements from `first` on, `stride` apart, end inside t.  By subtraction and division: the sum
         // first + (ny - 1) * stride + n of sizes that no tensor has can pass 2^63
         auto fits = [n, ny](const Tensor& t, long first, long stride) {
             const long numel = t.numel();
             return n <= numel && first <= numel - n && (stride == 0 || ny - 1 <= (numel - n - first) / stride);
         };
-        if (n && ny && !(fits(d, d0, ds) && fits(s, s0, ss))) value_error(who + ": the copy leaves the source or the destination");
-        for (PyObject* o : {dest, source}) {
-            Py_INCREF(o);
-            held.push_back(o);
-        }
+        if (n && ny && !(fits(d, d0, ds) && fits(s, s0, ss))) value_error(who() + ": the copy leaves the source or the destination");
         dst.push_back(d.data_ptr());
         src.push_back(s.data_ptr());
         for (long v : {(long)d.element_size(), n, d0, s0, ny, ds, ss}) meta.push_back(v);
     }
-    void add_zeros(PyObject* d, long n, long d0, long ny, long ds) {       // `ny` rows of `n` zeros
+    void add_zeros(const Tensor& d, long n, long d0, long ny, long ds) {   // `ny` rows of `n` zeros
         add(d, d, n, d0, d0, ny, ds, ds);                        // (the checks of the destination range)
         src.back() = nullptr;
         fills = true;
+    }
+    void add_zeros(PyObject* d, long n, long d0, long ny, long ds) {
+        add_zeros(gpu_tensor(d, "dst"), n, d0, ny, ds);
+        Py_INCREF(d);
+        held.push_back(d);
     }
     bool fills = false;
     void run() const {
@@ -852,6 +863,53 @@ PyObject* pools_load(PyObject* const* a) {
     Py_RETURN_NONE;
 }
 
+// element i of the first dimension of a contiguous tensor as a tensor of its own on the same storage
+Tensor part_of(const Tensor& t, int64_t i) {
+    auto impl = c10::make_intrusive<at::TensorImpl>(c10::Storage(t.storage()), t.key_set(), t.dtype());
+    const auto size = t.sizes().slice(1);
+    impl->set_sizes_contiguous(size);
+    impl->set_storage_offset(t.storage_offset() + i * c10::multiply_integers(size));
+    return Tensor(std::move(impl));
+}
+PyObject* list_of(Py_ssize_t n) {
+    PyObject* o = PyList_New(n);
+    if (!o) throw Raised{};
+    return o;
+}
+// cache_restore(K / V segments of a checkpoint's chain, conv, ssm, pos, max_len) -> [(K, V)], [conv], [ssm]: the segments [2 layers, 1, heads,
+// rows, width] end to end in fresh buffers of max_len rows, rows from pos on zero, and copies of the recurrent state, in one launch
+PyObject* cache_restore(PyObject* const* a) {
+    const Items segs(a[0]);
+    const long pos = integer(a[3]), max_len = integer(a[4]);
+    const Tensor &last = gpu_tensor(segs[segs.size() - 1], "kv"), &conv = gpu_tensor(a[1], "conv"), &ssm = gpu_tensor(a[2], "ssm");
+    if (last.dim() != 5 || conv.dim() < 1 || ssm.dim() < 1) value_error("cache_restore: kv [2 layers, 1, heads, rows, width] expected");
+    const int64_t nb = last.size(0), nkv = last.size(2), D = last.size(4);
+    Tensor bufs, conv_out, ssm_out;
+    unlocked([&] {
+        bufs = empty({nb, 1, nkv, max_len, D}, BF16, last), conv_out = empty(conv.sizes(), conv.scalar_type(), conv), ssm_out = empty(ssm.sizes(), ssm.scalar_type(), ssm);
+    });
+    Jobs j;
+    j.reserve(segs.size() * nb + 3);
+    long at = 0;
+    for (Py_ssize_t k = 0; k < segs.size(); k++) {
+        const Tensor& t = gpu_tensor(segs[k], "kv");
+        if (t.dim() != 5 || t.size(0) != nb || t.size(2) != nkv || t.size(4) != D) value_error("cache_restore: the segments' shapes differ");
+        const long n = t.size(3);
+        for (int64_t i = 0; i < nb; i++) j.add(bufs, segs[k], n * D, i * nkv * max_len * D + at * D, i * nkv * n * D, nkv, max_len * D, n * D);
+        at += n;
+    }
+    if (at != pos) throw Error{PyExc_AssertionError, "cache_restore: " + std::to_string(at) + " rows in the chain, " + std::to_string(pos) + " expected"};
+    j.add(conv_out, a[1], conv.numel(), 0, 0, 1, 0, 0);
+    j.add(ssm_out, a[2], ssm.numel(), 0, 0, 1, 0, 0);
+    if (max_len > pos) j.add_zeros(bufs, (max_len - pos) * D, pos * D, nb * nkv, max_len * D);
+    j.run();
+    const Ref kv(list_of(nb / 2)), cs(list_of(conv.size(0))), ss(list_of(ssm.size(0)));
+    for (int64_t i = 0; i < nb / 2; i++) PyList_SET_ITEM(kv.o, i, wrap({part_of(bufs, 2 * i), part_of(bufs, 2 * i + 1)}));
+    for (int64_t i = 0; i < conv.size(0); i++) PyList_SET_ITEM(cs.o, i, wrap(part_of(conv_out, i)));
+    for (int64_t i = 0; i < ssm.size(0); i++) PyList_SET_ITEM(ss.o, i, wrap(part_of(ssm_out, i)));
+    return PyTuple_Pack(3, kv.o, cs.o, ss.o);
+}
+
 // ---- the module -----------------------------------------------------------------------------------------------------------
 template <PyObject* (*F)(PyObject* const*), int N>
 PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -884,6 +942,7 @@ PyMethodDef methods[] = {
     QT_FN("phase_a", phase_a, 8),         QT_FN("phase_b", phase_b, 5),           QT_FN("phase_b_norm", phase_b_norm, 7),
     QT_FN("gdn_core", gdn_core, 8),
     QT_FN("set_hooks", set_hooks, 3),     QT_FN("blit_batch", blit_batch, 2),     QT_FN("pools_load", pools_load, 12),
+    QT_FN("cache_restore", cache_restore, 5),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_qt_host", "argument checks, allocation and launch of the operators", -1, methods};
 

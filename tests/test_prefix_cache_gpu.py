@@ -100,6 +100,27 @@ def test_restored_tensors_are_contiguous_and_disjoint(qt, dev):
         assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
 
 
+@pytest.mark.parametrize("bad", ["rows", "width", "dtype", "max_len", "none"])
+def test_restore_refuses_a_chain_that_does_not_fit(qt, dev, bad):
+    """segments that do not add up to the checkpoint's rows, that differ in shape or type, a buffer shorter than the checkpoint: errors, and
+    the cache is as good as before"""
+    cfg, st = make_state(qt, dev, 64, 4)
+    pc = qt.prefix_cache.PrefixCache(budget_mb=512)
+    ids = np.arange(64, dtype=np.int32)
+    top = pc.insert(None, ids, 20, st)
+    node = pc.insert(top, ids, 51, st)
+    want, _ = pc.restore(node, 64)
+    kv = top.kv
+    top.kv = {"rows": kv[:, :, :, :19].contiguous(), "width": kv[..., :128].contiguous(), "dtype": kv.float(), "max_len": kv, "none": None}[bad]
+    with pytest.raises((AssertionError, ValueError, TypeError)):
+        pc.restore(node, 40 if bad == "max_len" else 64)
+    top.kv = kv
+    got, _ = pc.restore(node, 64)
+    for (k0, v0), (k1, v1) in zip(want["kv"], got["kv"]):
+        assert torch.equal(k0, k1) and torch.equal(v0, v1)
+    assert all(torch.equal(a, b) for f in ("conv", "ssm") for a, b in zip(want[f], got[f]))
+
+
 def test_cat_rows_pads_with_zeros(qt, dev):
     pc = qt.prefix_cache.PrefixCache
     a, b = torch.ones((1, 3, 4), device=dev), 2 * torch.ones((1, 5, 4), device=dev)
