@@ -169,6 +169,13 @@ int qt_gdn_phase_b_norm(const void* ops, const void* U, const float* gC, void* s
 int qt_gdn_phase_b_report(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out,
                           const void* proj, const float* gw, float eps, void* out, int S, int32_t* host_words, qt_stream_t stream);
 
+/* The whole layer core of a prompt of 1 .. 64 tokens in one launch: qt_gdn_phase_a_conv and qt_gdn_phase_b_report with the gated norm, without
+ * records (snap is used for its status word only).  The same operator, not the same bits: the state's products are taken directly instead
+ * of through half-precision operands that hold part of them.  QT_ERR_UNSUPPORTED for other numbers of tokens (nothing is launched). */
+int qt_gdn_prefill_one(const void* proj, const void* conv_state, const void* conv_w, const void* silu_table, const float* A_log,
+                       const float* dt_bias, void* conv_out, void* snap, const float* state_in, float* state_out, const float* gw, float eps,
+                       void* out, int S, int32_t* host_words, qt_stream_t stream);
+
 /* Causal prefill attention: the mx.fast.scaled_dot_product_attention(..., mask="causal") call of the full-attention layers
  * (qwen35/model.py:160-167, qwen35/prefill.py:468).  q, out [8][S][256] bf16 with head stride q_head_stride (elements);
  * K, V [2][>=L][256] bf16 with head stride kv_head_stride; query i sits at position q_pos0 + i and sees keys 0..q_pos0+i.

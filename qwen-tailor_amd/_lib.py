@@ -34,6 +34,7 @@ _SIGS = {
     "qt_rope_table_build": [_vp, _i, _vp],
     "qt_gdn_phase_b": [_vp] * 7 + [_i, _vp],
     "qt_gdn_phase_b_report": [_vp] * 8 + [_f, _vp, _i, _vp, _vp],
+    "qt_gdn_prefill_one": [_vp] * 11 + [_f, _vp, _i, _vp, _vp],
     "qt_gdn_phase_b_poll_limit": [_i],
     "qt_gdn_phase_b_norm": [_vp] * 8 + [_f, _vp, _i, _vp],
     "qt_gqa_prefill_causal": [_vp] * 5 + [_l, _i, _i, _i, _l, _l, _vp],

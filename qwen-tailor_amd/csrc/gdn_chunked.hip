@@ -374,19 +374,27 @@ __device__ __forceinline__ T load_once(const T* p) {
     return STREAM ? __builtin_nontemporal_load(p) : *p;
 }
 template <bool STREAM>
-__device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c, int h, bf16_t* __restrict__ y,
-                                                           const bf16_t* __restrict__ proj, const float* __restrict__ gw, float eps, int S) {
+__device__ __forceinline__ uint4 z_row(const bf16_t* __restrict__ proj, int c, int h, int row, int cc, int S) {
+    const u32x4 zw = load_once<STREAM>(reinterpret_cast<const u32x4*>(proj + (size_t)min(c * C + row, S - 1) * PW + CD + h * DV) + cc);
+    return make_uint4(zw[0], zw[1], zw[2], zw[3]);
+}
+// by NT = 256 or 512 threads, NT / 16 rows at a time.  Z(it): the z values of row NT / 16 it + tid / 16, eight per thread
+template <int NT, class ZFn>
+__device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c, int h, bf16_t* __restrict__ y, ZFn Z, const float* __restrict__ gw,
+                                                float eps, int S) {
+    constexpr int RP = NT / 16, IT = C / RP;
+    static_assert(IT == 4 || IT == 2, "four or two rows per 16-lane group");
     const int cc = tid & 15;
     float gwv[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) gwv[j] = gw[cc * 8 + j];
-    // the four rows of this 16-lane group: all sums of squares first, then one reciprocal square root per lane
-    uint4 yv4[4];
-    double ss4[4];
-    float inv4[4];
+    // the rows of this 16-lane group: all sums of squares first, then one reciprocal square root per lane
+    uint4 yv4[IT];
+    double ss4[IT];
+    float inv4[IT];
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const int row = it * 16 + (tid >> 4);
+    for (int it = 0; it < IT; it++) {
+        const int row = it * RP + (tid >> 4);
         const u32x4 yw = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(&ys[row * YS_LD + cc * 8]);
         yv4[it] = make_uint4(yw[0], yw[1], yw[2], yw[3]);
         float yy[8];
@@ -398,17 +406,18 @@ __device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c,
     }
     // every z row is requested before the first result is stored: a wavefront's loads and stores share one counter, so a load
     // issued behind a store is waited for together with it, and a store takes microseconds to complete
-    uint4 zv4[4];
+    uint4 zv4[IT];
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const int t = min(c * C + it * 16 + (tid >> 4), S - 1);
-        const u32x4 zw = load_once<STREAM>(reinterpret_cast<const u32x4*>(proj + (size_t)t * PW + CD + h * DV) + cc);
-        zv4[it] = make_uint4(zw[0], zw[1], zw[2], zw[3]);
+    for (int it = 0; it < IT; it++) zv4[it] = Z(it);
+    if constexpr (IT == 4) {
+        rsqrt_rows4(ss4, eps, inv4, cc);
+    } else {
+        const float ss2[2] = {(float)row16_sum_d(ss4[0]), (float)row16_sum_d(ss4[1])};
+        rsqrt_rows<2>(ss2, eps, inv4, cc);
     }
-    rsqrt_rows4(ss4, eps, inv4, cc);
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const int row = it * 16 + (tid >> 4);
+    for (int it = 0; it < IT; it++) {
+        const int row = it * RP + (tid >> 4);
         const int t = c * C + row;
         if (t >= S) continue;                                       // whole 16-lane groups leave together
         float yy[8], zz[8];
@@ -524,7 +533,8 @@ __device__ __forceinline__ void output_item(bf16_t* ys, volatile int* ready, int
                     for (int i = 0; i < 4; i++) dst[i] = src[i];
                 }
             } else {
-                gated_norm_tile<WAIT>((lds_bf16_ptr)ys, tid, c, h, y, proj, gw, eps, S);
+                gated_norm_tile<256>((lds_bf16_ptr)ys, tid, c, h, y, [&](int it) { return z_row<WAIT>(proj, c, h, it * 16 + (tid >> 4), tid & 15, S); }, gw,
+                                eps, S);
             }
         }
         __syncthreads();                                                        // ys is reused by the next round
@@ -660,9 +670,11 @@ __device__ __forceinline__ half4 lds_tr4(const _Float16* p) {
     return __builtin_bit_cast(half4, v);
 }
 // MFMA operand whose contraction index runs over the chunk's tokens, from a row-major [token][ld] tile: lane (n, g) gets
-// column c0 + n of tokens kperm(kb2, g, 0..7) = 32 kb2 + 4 g + {0..3}, 32 kb2 + 16 + 4 g + {0..3}.
+// column c0 + n of tokens kperm(kb2, g, 0..7) = 32 kb2 + 4 g + {0..3}, 32 kb2 + 16 + 4 g + {0..3}.  (Q4: columns between the starts of two
+// fours; with 8 lane n gets column c0 + 8 (n / 4) + n % 4.)
+template <int Q4 = 4>
 __device__ __forceinline__ half8 tokens_operand(const _Float16* base, int ld, int kb2, int c0, int n, int g) {
-    const _Float16* p = base + (32 * kb2 + 4 * g + (n >> 2)) * ld + c0 + 4 * (n & 3);
+    const _Float16* p = base + (32 * kb2 + 4 * g + (n >> 2)) * ld + c0 + Q4 * (n & 3);
     const half4 lo = lds_tr4(p), hi = lds_tr4(p + 16 * ld);
     half8 r;
     r[0] = lo[0]; r[1] = lo[1]; r[2] = lo[2]; r[3] = lo[3];
@@ -816,16 +828,97 @@ __device__ __forceinline__ void inverse_row(PhaseALds& L, const int I, int n, in
 // proj [S,8224] supplies the gate inputs a, b in both forms.  The two forms give the same bits: after the staging of q, k, v
 // every floating-point step is a single instruction chosen in the source (MFMA, multiplication, fused multiply-add), so the
 // compiler has nothing to contract differently in the two instances.
-template <bool from_proj>
-__global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qkv,
-                                                          const bf16_t* __restrict__ proj, bf16_t* qi, bf16_t* ki, bf16_t* vi,
-                                                          const bf16_t* __restrict__ cs, const bf16_t* __restrict__ cw,
-                                                          const bf16_t* __restrict__ silu_tab, bf16_t* __restrict__ conv_out,
-                                                          const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-                                                          _Float16* __restrict__ ops, _Float16* __restrict__ U,
-                                                          float* __restrict__ gates, int S) {
-    __shared__ PhaseALds L;
-    const int c = blockIdx.x / HV, h = blockIdx.x % HV, t0 = c * C;
+//
+// ONE: a prompt of one chunk.  The workgroup of a head goes on to the outputs and the new state by itself (one_chunk below): no records, one
+// launch instead of three.
+struct OneArgs {
+    const float* st_in;
+    float* st_out;
+    bf16_t* y;
+    const float* gw;
+    float eps;
+    int *status, *host_words;
+};
+struct OneLds {
+    __align__(16) _Float16 Tb[NCT * 2 * 512], Am[NCT * 2 * 512];     // operand tiles [row tile][kb2][lane][8]
+    __align__(16) float dec[C];
+    float gC;
+};
+// What remains of a single chunk once K, Q, V, Tb and Am are in LDS; wavefront sl owns the columns 16 sl .. + 15 of the head (dv).  The state
+// never leaves its registers, so that the products are those of the definition, with nothing folded into operands beforehand:
+//     D = Tb (V - gamma * (K S^T)),   Y = gamma * (Q S^T) + Am D,   S' = gamma_C S + K^T (dec * D)
+__device__ __forceinline__ void one_chunk(const PhaseALds& L, const OneLds& L1, bf16_t* ys, const f32x4 (&S0)[8], const uint4 (&zv)[2], const OneArgs& o,
+                                          int h, int sl, int tid, int n, int g, int S) {
+    const int lane = tid & 63;
+    half8 Sb[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) Sb[kb] = pack_half8(S0[2 * kb], S0[2 * kb + 1]);
+    // rows of K or Q with the contraction index (dk) enumerated as the state's operand
+    auto rows = [&](const _Float16* base, int ct, int kb) { return *reinterpret_cast<const half8*>(base + (16 * ct + n) * QS_LD + 32 * kb + 8 * g); };
+    f32x4 R[NCT], Y[NCT];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++) {
+        f32x4 ks = {0.f, 0.f, 0.f, 0.f};
+        Y[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++) {
+            ks = __builtin_amdgcn_mfma_f32_16x16x32_f16(rows(L.Ks, ct, kb), Sb[kb], ks, 0, 0, 0);
+            Y[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Sb[kb], rows(L.Qs, ct, kb), Y[ct], 0, 0, 0);   // (transposed, as in the output kernel)
+        }
+        const f32x4 gm = *reinterpret_cast<const f32x4*>(&L.gam[16 * ct + 4 * g]);
+#pragma unroll
+        for (int r = 0; r < 4; r++) R[ct][r] = __builtin_fmaf(-gm[r], ks[r], (float)L.Vs[(16 * ct + 4 * g + r) * VS_LD + 16 * sl + n]);
+        Y[ct] *= L.gam[16 * ct + n];
+    }
+    const half8 Rb[2] = {pack_half8(R[0], R[1]), pack_half8(R[2], R[3])};
+    f32x4 D[NCT];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++) {
+        D[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb2 = 0; kb2 < (ct < 2 ? 1 : 2); kb2++)             // (lower triangular)
+            D[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const half8*>(&L1.Tb[(ct * 2 + kb2) * 512 + lane * 8]), Rb[kb2], D[ct], 0, 0, 0);
+    }
+    f32x4 Dd[NCT];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++) Dd[ct] = D[ct] * *reinterpret_cast<const f32x4*>(&L1.dec[16 * ct + 4 * g]);
+    const half8 Dn[2] = {pack_half8(D[0], D[1]), pack_half8(D[2], D[3])}, Ds[2] = {pack_half8(Dd[0], Dd[1]), pack_half8(Dd[2], Dd[3])};
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++)
+#pragma unroll
+        for (int kb2 = 0; kb2 < (ct < 2 ? 1 : 2); kb2++)
+            Y[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Dn[kb2], *reinterpret_cast<const half8*>(&L1.Am[(ct * 2 + kb2) * 512 + lane * 8]), Y[ct], 0, 0, 0);
+    bool bad = false;
+    float* so = o.st_out + ((size_t)h * DV + sl * 16 + n) * DK + 8 * g;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {                                    // row 4 g + r of tile i is row 32 (i / 2) + 8 g + 4 (i % 2) + r of the state
+        f32x4 s1 = S0[i] * L1.gC;
+#pragma unroll
+        for (int kb2 = 0; kb2 < 2; kb2++)
+            s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(tokens_operand<8>(L.Ks, QS_LD, kb2, 32 * (i >> 1) + 4 * (i & 1), n, g), Ds[kb2], s1, 0, 0, 0);
+        *reinterpret_cast<f32x4*>(so + 32 * (i >> 1) + 4 * (i & 1)) = s1;
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad |= !(fabsf(s1[r]) <= 3.0e38f);
+    }
+    if (__any(bad) && lane == 0) {                                   // (as in the chain)
+        atomicOr(o.status, ERR_NOT_FINITE);
+        if (o.host_words) o.host_words[1] = 1;
+    }
+    __syncthreads();                                                 // Q has been read: its memory takes the outputs
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++)
+        *reinterpret_cast<uint2*>(&ys[(ct * 16 + n) * YS_LD + sl * 16 + 4 * g]) = make_uint2(pack2_bf(Y[ct][0], Y[ct][1]), pack2_bf(Y[ct][2], Y[ct][3]));
+    __syncthreads();
+    gated_norm_tile<512>((lds_bf16_ptr)ys, tid, 0, h, o.y, [&](int it) { return zv[it]; }, o.gw, o.eps, S);
+}
+
+template <bool from_proj, bool ONE>
+__device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk, const bool write_qkv, const bf16_t* __restrict__ proj, bf16_t* qi,
+                                        bf16_t* ki, bf16_t* vi, const bf16_t* __restrict__ cs, const bf16_t* __restrict__ cw,
+                                        const bf16_t* __restrict__ silu_tab, bf16_t* __restrict__ conv_out,
+                                        const float* __restrict__ A_log, const float* __restrict__ dt_bias, _Float16* __restrict__ ops,
+                                        _Float16* __restrict__ U, float* __restrict__ gates, int S, const OneArgs& o) {
+    const int c = ONE ? 0 : blk / HV, h = blk % HV, t0 = c * C;
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
     // (the wavefront number as a scalar: the branches on it are then real branches, which the barriers inside them need)
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -898,23 +991,10 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
         }
     }
 
-    if (from_proj) {
-        static_assert(TAB_VECS > 512 && TAB_VECS <= 1024, "two vectors of the table per thread");
-        if (silu_tab) {
-            reinterpret_cast<uint4*>(L.tab)[tid] = tab0;
-            if (tid + 512 < TAB_VECS) reinterpret_cast<uint4*>(L.tab)[tid + 512] = tab1;
-        } else {
-            silu_table_fill(L.tab, nullptr, tid, 512);
-        }
-        if (tid >= TAP0) reinterpret_cast<uint4*>(L.taps)[tid - TAP0] = tap;
-    }
-
-    if (tid >= 508) L.staged[tid - 508] = 0;
-    __syncthreads();
-
     // ---- gates of the chunk's tokens (gdn_nax.py:80-104): wavefront 0, one token per lane.  Behind the barrier: nobody needs them before
-    // k is staged, which wavefront 0 announces after them, and group M has the time (it waits for v in the end).
-    if (wv == 0) {
+    // k is staged, which wavefront 0 announces after them, and group M has the time (it waits for v in the end).  With one chunk group M
+    // is what everything waits for, and the gates are computed while the table is on its way.
+    auto chunk_gates = [&] {
         const int t = t0 + lane;
         float lg = 0.f, be = 0.f;
         asm volatile("" : "+v"(ga_raw), "+v"(gb_raw));          // (first used here: moved up to the loads, the use would wait for them there)
@@ -940,11 +1020,43 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
         L.Lc2[lane] = lc * LOG2E;
         L.beta[lane] = be;
         L.gam[lane] = gm;
-        float* gp = gates + rec * GATE_FLOATS;
-        gp[G_GAM + lane] = gm;
-        gp[G_DEC + lane] = dc;
-        if (lane >= 60) gp[G_GC + lane - 60] = lane == 60 ? expf(tot) : 0.f;
+        if constexpr (ONE) {
+            L1->dec[lane] = dc;
+            if (lane == 0) L1->gC = expf(tot);
+        } else {
+            float* gp = gates + rec * GATE_FLOATS;
+            gp[G_GAM + lane] = gm;
+            gp[G_DEC + lane] = dc;
+            if (lane >= 60) gp[G_GC + lane - 60] = lane == 60 ? expf(tot) : 0.f;
+        }
+    };
+    if (ONE && wv == 0) chunk_gates();
+    if (from_proj) {
+        static_assert(TAB_VECS > 512 && TAB_VECS <= 1024, "two vectors of the table per thread");
+        if (silu_tab) {
+            reinterpret_cast<uint4*>(L.tab)[tid] = tab0;
+            if (tid + 512 < TAB_VECS) reinterpret_cast<uint4*>(L.tab)[tid + 512] = tab1;
+        } else {
+            silu_table_fill(L.tab, nullptr, tid, 512);
+        }
+        if (tid >= TAP0) reinterpret_cast<uint4*>(L.taps)[tid - TAP0] = tap;
     }
+
+    // one chunk: this wavefront's columns of the state (lane (n, g): column n, rows 32 kb + 8 g .. + 7 in S0[2 kb], S0[2 kb + 1]) and its rows of z
+    f32x4 S0[ONE ? 8 : 1];
+    uint4 zv[ONE ? 2 : 1];
+    if constexpr (ONE) {
+        const float* sp = o.st_in + ((size_t)h * DV + wv * 16 + n) * DK + 8 * g;
+#pragma unroll
+        for (int i = 0; i < 8; i++) S0[i] = *reinterpret_cast<const f32x4*>(sp + 32 * (i >> 1) + 4 * (i & 1));
+#pragma unroll
+        for (int it = 0; it < 2; it++) zv[it] = z_row<false>(proj, 0, h, it * 32 + (tid >> 4), tid & 15, S);
+    }
+
+    if (tid >= 508) L.staged[tid - 508] = 0;
+    __syncthreads();
+
+    if (!ONE && wv == 0) chunk_gates();
 
     // ---- k (group M) and q (group V): conv + SiLU + L2 norm, staged as half precision
     {
@@ -1009,7 +1121,7 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
         await_part(L, PA_Q);
         await_part(L, PA_K);
         // Kh = K^T (rows dk of tiles 2w, 2w+1), k index permuted: group V has the time for it (group M ends last)
-        for (int mm = 0; mm < 2; mm++) {
+        for (int mm = 0; mm < (ONE ? 0 : 2); mm++) {
             const int mt = 2 * w + mm;
             for (int kb2 = 0; kb2 < 2; kb2++)
                 *reinterpret_cast<half8*>(op + OP_K + (mt * 2 + kb2) * 512 + lane * 8) = tokens_operand(L.Ks, QS_LD, kb2, 16 * mt, n, g);
@@ -1038,7 +1150,15 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
                     }
                 }
             }
-            __builtin_nontemporal_store(pack_half8(part[0], part[1]), reinterpret_cast<half8*>(op + OP_A + (ct * 2 + kb2) * 512 + lane * 8));
+            if constexpr (ONE)
+                *reinterpret_cast<half8*>(&L1->Am[(ct * 2 + kb2) * 512 + lane * 8]) = pack_half8(part[0], part[1]);
+            else
+                __builtin_nontemporal_store(pack_half8(part[0], part[1]), reinterpret_cast<half8*>(op + OP_A + (ct * 2 + kb2) * 512 + lane * 8));
+        }
+        if constexpr (ONE) {
+            __syncthreads();
+            one_chunk(L, *L1, reinterpret_cast<bf16_t*>(L.Qs), S0, zv, o, h, wv, tid, n, g, S);
+            return;
         }
         // Qh = Q (rows of tile ct), k index permuted: two 8-byte pieces of the row
         for (int kb = 0; kb < 4; kb++) {
@@ -1060,6 +1180,14 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
     half8 tbU[2], tbW[2];
     inverse_row(L, w, n, g, tbU, tbW);
     const int ct = w, nkb = ct < 2 ? 1 : 2;              // Tb is lower triangular: columns past the row tile are zero
+    if constexpr (ONE) {
+#pragma unroll
+        for (int kb2 = 0; kb2 < 2; kb2++) *reinterpret_cast<half8*>(&L1->Tb[(ct * 2 + kb2) * 512 + lane * 8]) = tbU[kb2];
+        __builtin_amdgcn_s_setprio(0);
+        __syncthreads();
+        one_chunk(L, *L1, reinterpret_cast<bf16_t*>(L.Qs), S0, zv, o, h, wv, tid, n, g, S);
+        return;
+    }
     for (int kb = 0; kb < 4; kb++) {
         f32x4 acc[2];
 #pragma unroll
@@ -1088,6 +1216,32 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
         uh[0] = (_Float16)acc[0]; uh[1] = (_Float16)acc[1]; uh[2] = (_Float16)acc[2]; uh[3] = (_Float16)acc[3];
         *reinterpret_cast<half4*>(up + ((sl * NCT + ct) * 64 + lane) * 4) = uh;
     }
+}
+
+template <bool from_proj>
+__global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qkv, const bf16_t* __restrict__ proj, bf16_t* qi, bf16_t* ki, bf16_t* vi,
+                                                             const bf16_t* __restrict__ cs, const bf16_t* __restrict__ cw,
+                                                             const bf16_t* __restrict__ silu_tab, bf16_t* __restrict__ conv_out,
+                                                             const float* __restrict__ A_log, const float* __restrict__ dt_bias,
+                                                             _Float16* __restrict__ ops, _Float16* __restrict__ U,
+                                                             float* __restrict__ gates, int S) {
+    __shared__ PhaseALds L;
+    phase_a<from_proj, false>(L, nullptr, blockIdx.x, write_qkv, proj, qi, ki, vi, cs, cw, silu_tab, conv_out, A_log, dt_bias, ops, U, gates, S,
+                              OneArgs{});
+}
+// A prompt of up to 64 tokens: one workgroup per head does everything.  What bounds it is one CU per head: the vector instructions of the conv of
+// k, q and v (until 7.5 us after the first wavefront starts, time stamps) and then the string of dependent products, the norm and the
+// store (5 us).  Records through memory and two more launches cost more than the idle CUs could give: 61 tokens 19.2 us in three launches,
+// 14.9 in one (the chain's products with K and Q in the order of the state's own registers, the gates ahead of the first barrier and the norm
+// on all eight wavefronts; 16.8 without those three).  Errors against float64, one launch / three: state 2.05e-4 / 2.19e-4, outputs 1.50e-3 both.
+__global__ __launch_bounds__(512, 2) void gdn_one_chunk_kernel(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cs,
+                                                               const bf16_t* __restrict__ cw, const bf16_t* __restrict__ silu_tab,
+                                                               bf16_t* __restrict__ conv_out, const float* __restrict__ A_log,
+                                                               const float* __restrict__ dt_bias, int S, OneArgs o) {
+    __shared__ PhaseALds L;
+    __shared__ OneLds L1;
+    static_assert(sizeof(L.Qs) >= sizeof(bf16_t) * C * YS_LD, "the outputs take Q's memory");
+    phase_a<true, true>(L, &L1, blockIdx.x, false, proj, nullptr, nullptr, nullptr, cs, cw, silu_tab, conv_out, A_log, dt_bias, nullptr, nullptr, nullptr, S, o);
 }
 
 }  // namespace
@@ -1199,6 +1353,23 @@ int qt_gdn_phase_a_conv(const void* proj, const void* conv_state, const void* co
     hipLaunchKernelGGL(gdn_phase_a_kernel<true>, dim3(NC * HV), dim3(512), 0, stream, q != nullptr, (const bf16_t*)proj, (bf16_t*)q,
                        (bf16_t*)k, (bf16_t*)v, (const bf16_t*)conv_state, (const bf16_t*)conv_w, (const bf16_t*)silu_table,
                        (bf16_t*)conv_out, A_log, dt_bias, (_Float16*)ops, (_Float16*)U, gC, S);
+    QT_CHECK_LAUNCH();
+    return QT_OK;
+}
+
+// qt_gdn_phase_a_conv and qt_gdn_phase_b_report with the gated norm for a prompt of 1 .. 64 tokens, in one launch without records: snap is
+// used for its status word only.  -4 for more tokens (nothing launched).
+int qt_gdn_prefill_one(const void* proj, const void* conv_state, const void* conv_w, const void* silu_table, const float* A_log,
+                       const float* dt_bias, void* conv_out, void* snap, const float* state_in, float* state_out, const float* gw, float eps,
+                       void* out, int S, int32_t* host_words, hipStream_t stream) {
+    if (!proj || !conv_state || !conv_w || !A_log || !dt_bias || !snap || !state_in || !state_out || !gw || !out || !host_words) return QT_ERR_NULL;
+    if (S < 0) return QT_ERR_DIM;
+    if (S < 1 || S > C || conv_out == conv_state) return QT_ERR_UNSUPPORTED;
+    for (const void* p : {proj, conv_state, conv_w, silu_table, (const void*)conv_out, (const void*)snap, (const void*)state_in, (const void*)state_out, (const void*)out})
+        if (reinterpret_cast<uintptr_t>(p) & 15u) return QT_ERR_ALIGN;
+    hipLaunchKernelGGL(gdn_one_chunk_kernel, dim3(HV), dim3(512), 0, stream, (const bf16_t*)proj, (const bf16_t*)conv_state, (const bf16_t*)conv_w,
+                       (const bf16_t*)silu_table, (bf16_t*)conv_out, A_log, dt_bias, S,
+                       OneArgs{state_in, state_out, (bf16_t*)out, gw, eps, reinterpret_cast<int*>(snap) + FLAG_ERR, (int*)host_words});
     QT_CHECK_LAUNCH();
     return QT_OK;
 }

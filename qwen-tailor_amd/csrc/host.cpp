@@ -740,8 +740,13 @@ PyObject* gdn_core(PyObject* const* a) {
     unlocked([&] {
         if (want)
             for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
-        const Records r = new_records(proj);
         conv_out = empty({1, 3, CD}, BF16, proj), st_out = empty({1, HV, DV, DK}, F32, proj), out = empty({S, HV * DV}, BF16, proj);
+        // a prompt of one chunk: one launch
+        const int rc = qt_gdn_prefill_one(proj.data_ptr(), cs.data_ptr(), w.data_ptr(), silu.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(),
+                                          conv_out.data_ptr(), s.buf.data_ptr(), state.data_ptr<float>(), st_out.data_ptr<float>(),
+                                          gw.data_ptr<float>(), 1e-6f, out.data_ptr(), dim32(S), s.words.data_ptr<int>(), stream());
+        if (rc != -4) return check(rc, "qt_gdn_prefill_one");
+        const Records r = new_records(proj);
         phase_a_conv(proj, cs, w, silu, A, dtb, want ? qkv : nullptr, conv_out.data_ptr(), r);
         phase_b_launch(r, s, state, st_out, &proj, &gw, 1e-6f, out, S);
     });

@@ -271,6 +271,32 @@ def test_status_word_reports_operands_beyond_half_precision(qt, dev, T):
     check_rel("gated output after the reset", to_np(o4), oo, 2e-3, rel_l2)
 
 
+@pytest.mark.parametrize("T", [1, 2, 3, 15, 16, 17, 32, 47, 49, 63, 64])
+def test_prompt_of_one_chunk_in_one_launch(qt, dev, T):
+    """up to 64 tokens the layer core is one launch without records: edges of its 16-row tiles and of the conv window, against the sequential
+    oracle, and against the two phases called one by one.  Both round the operands of their products to half precision (2^-11 each, three
+    products deep): state within 2e-3, as for the longer prompts.  Outputs within one bf16 step, 2^-8: a y that rounds the other way moves an output by that much, and with few tokens a single row can carry the norm
+    (both forms, 8 seeds of 1 - 5 tokens: 0.9e-3 to 3.3e-3)."""
+    proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(700 + T, T, state_scale=0.3)
+    out, conv, st = _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0)
+    qt.gdn_nax.check_status(dev, sync=True)
+    oo, oy, otail, os_ = O.prefill_gdn(proj, cs, cw, A_log, dtb, S0, gw)
+    check_equal("conv window", to_np(conv)[0], np.concatenate([cs, proj[:, :CD]], 0)[-3:])
+    check_rel("final state rel-L2", to_np(st)[0], os_, 2e-3, rel_l2)
+    check_rel("gated output rel-L2", to_np(out), oo, 2.0 ** -8, rel_l2)
+    dproj = to_dev(proj, dev, BF16)
+    records = qt.gdn_nax._phase_a(dproj, to_dev(cs, dev, BF16), to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev), want_qkv=False)[3:]
+    o3, s3 = qt.gdn_nax.phase_b_norm(dproj, *records, to_dev(S0[None], dev), to_dev(gw, dev))
+    check_rel("state against the two phases", to_np(st), to_np(s3).reshape(to_np(st).shape), 2e-3, rel_l2)
+    check_rel("output against the two phases", to_np(out), to_np(o3), 2.0 ** -8, rel_l2)
+
+
+@pytest.mark.parametrize("T", [7, 64])
+def test_one_launch_at_the_edge_of_the_half_precision_range_and_beyond(qt, dev, T):
+    test_chunked_prefill_at_the_edge_of_the_half_precision_range(qt, dev, T)
+    test_status_word_reports_operands_beyond_half_precision(qt, dev, T)
+
+
 def test_give_up_path_ends_the_launch_and_leaves_the_flags_clean(qt, dev):
     """the bounded wait of the one-launch form, forced from the host with a poll limit of one: output workgroups give up on chunks
     the chain has not published yet, leave those rows unwritten and set bit 0 of the status word; every workgroup ends, the
