@@ -78,6 +78,20 @@ __device__ __forceinline__ float max_over_groups(float x) {
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
+// ... and the sum
+__device__ __forceinline__ float sum_over_groups(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    const float s = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+__device__ __forceinline__ float row16_max(float v) {            // over a 16-lane row
+    v = fmaxf(v, dpp_mov<0xB1>(v));
+    v = fmaxf(v, dpp_mov<0x4E>(v));
+    v = fmaxf(v, dpp_mov<0x141>(v));
+    return fmaxf(v, dpp_mov<0x140>(v));
+}
+
 // Online-softmax update of one tile of 16 keys from its transposed scores: lane (row n, group g) holds keys 4g .. 4g+3.
 // Leaves the probabilities of those keys in p (fp32) and returns the row's rescale factor (the same in the row's four lanes).
 __device__ __forceinline__ float softmax_tile(const f32x4& acc, int nvalid, bool causal, float& m_run, float& l_run, float (&p)[4], int lane) {
@@ -524,8 +538,7 @@ __global__ __launch_bounds__(256, 2) void attn_partial_kernel(const bf16_t* __re
     }
 
     // ---- merge the 4 wavefronts (deterministic order); lane (n, g) holds columns 16 j + 4 g .. + 3 of row n
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = sum_over_groups(l_run);
     if (g == 0) {
         m_s[w][n] = m_run;
         l_s[w][n] = l_run;
@@ -594,19 +607,27 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
     f32x4 first[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) first[i] = *reinterpret_cast<const f32x4*>(po + (size_t)min(w + 4 * i, ns - 1) * R * AD);
-    float mx = NEG;
-    for (int s = tid; s < ns; s += 256) mx = fmaxf(mx, ml[(size_t)s * 2 * R]);
-    mx = wave_max(mx);
+    // (a thread's first pair stays in its registers: with up to 256 partials nothing is loaded a second time)
+    float2 own = make_float2(NEG, 0.f);
+    if (tid < ns) own = *reinterpret_cast<const float2*>(ml + (size_t)tid * 2 * R);
+    float mx = own.x;
+    for (int s = tid + 256; s < ns; s += 256) mx = fmaxf(mx, ml[(size_t)s * 2 * R]);
+    mx = max_over_groups(row16_max(mx));
     if (lane == 0) red_m[w] = mx;
     __syncthreads();
     const float mm = fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3]));
     float lp = 0.f;
-    for (int s = tid; s < ns; s += 256) {
+    if (tid < ns) {
+        const float f = __expf(own.x - mm);
+        fs_s[tid] = f;
+        lp = own.y * f;
+    }
+    for (int s = tid + 256; s < ns; s += 256) {
         const float f = __expf(ml[(size_t)s * 2 * R] - mm);
         fs_s[s] = f;
         lp += ml[(size_t)s * 2 * R + 1] * f;
     }
-    lp = wave_sum(lp);
+    lp = sum_over_groups(row16_sum(lp));
     if (lane == 0) red_l[w] = lp;
     __syncthreads();
     const float l = (red_l[0] + red_l[1]) + (red_l[2] + red_l[3]);
