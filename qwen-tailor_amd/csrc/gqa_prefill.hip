@@ -699,25 +699,23 @@ KeySplit plan_split_nh(int S, int L, int q_pos0, int nh, int min_gain) {
     ks.nh = nh;
     const int RB = 16 * nh, nb = (S + RB - 1) / RB, cus = cu_count();
     if (S < 1 || nb * AKV >= cus) return ks;
-    long total = 0;
-    int longest = 0;
-    for (int i = 0; i < nb; i++) {
-        const int kend = std::min(L, q_pos0 + std::min(RB * i + RB - 1, S - 1) + 1), nt = (kend + KT - 1) / KT;
-        total += nt;
-        longest = std::max(longest, nt);
-    }
-    // the part size (from the average per CU, at least 3 tiles) with the least time among those whose parts are all resident at once: a CU
+    const int longest = (std::min(L, q_pos0 + S) + KT - 1) / KT; // (the last block's)
+    // the part size (at least 3 tiles) with the least time among those whose parts are all resident at once: a CU
     // that has to run a second part pays the per-workgroup cost twice.  In us, fitted to a sweep of 17 - 1460 rows on 0 - 6000 keys: a tile
     // 1.25 (32-row blocks 1.8), a part 0.033 in the merge (twice that), and 0.85 for every four parts that the merge takes one after the
     // other.  (At least 6 tiles always, against this: 17 rows on 700 / 1500 keys 15.1 / 15.3 and 11.5 / 12.7, 100 rows on 700 / 3000 15.4 / 18.8
     // and 13.1 / 17.8, 333 on 300 / 1500 16.3 / 19.6 and 13.9 / 19.2, 700 rows 17.1 and 15.4.)
+    // The search begins at a lower bound of the tiles per CU and ends where the tiles alone cost more than the best found: a dozen
+    // divisions, because a launch of 20 us does not hide much of its host.
     const long p = (q_pos0 + RB - 1) / RB, cpt = KT / RB;
+    const float per_tile = nh == 1 ? 1.25f : 1.8f;
+    const long least_tiles = (long)nb * (q_pos0 + 1) / KT + (long)RB * nb * (nb - 1) / (2 * KT);
     int tmax = longest;
     float least = 1e30f;
-    for (int t = (int)std::max(3L, (total * AKV + cus - 1) / cus); t <= longest; t++) {
-        const long parts = (parts_upto(p + nb, cpt * t) - parts_upto(p, cpt * t)) * AKV, most = (p + nb + cpt * t - 1) / (cpt * t);
+    for (int t = (int)std::max(3L, least_tiles * AKV / cus); t <= longest && per_tile * t < least; t++) {
+        const long c = cpt * t, parts = (parts_upto(p + nb, c) - parts_upto(p, c)) * AKV;
         if (parts > cus) continue;
-        const float us = (nh == 1 ? 1.25f : 1.8f) * t + 0.033f * nh * parts + 0.85f * ((most + 3) / 4);
+        const float us = per_tile * t + 0.033f * nh * parts + 0.85f * (((p + nb + c - 1) / c + 3) / 4);
         if (us < least) least = us, tmax = t;
     }
     if (longest - tmax < min_gain) return ks;                    // the merge launch has to be earned
@@ -750,7 +748,7 @@ KeySplit plan_split(int S, int L, int q_pos0) {
         if (ks.tmax) return ks;
     }
     const KeySplit one = plan_split_nh(S, L, q_pos0, 1, 4);
-    if (one.tmax) {
+    if (1.25f * one.tmax > 3.5f + 1.8f * 3) {                    // (parts of 32-row blocks have three tiles or more)
         const KeySplit two = plan_split_nh(S, L, q_pos0, 2, 4);
         if (two.tmax && 1.25f * one.tmax - 1.8f * two.tmax > 3.5f) return two;
     }
