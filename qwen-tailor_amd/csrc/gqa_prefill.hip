@@ -225,7 +225,15 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
     // even and the upper half in the odd lanes, block j + 1 the other halves.  Afterwards lane group g holds eight adjacent columns in its
     // two blocks (16-byte stores), and a fragment read still touches every bank twice.
     const int vrow = 4 * g + (n >> 2);                           // row within a 16-key block = its swizzle
-    const int va_row = vrow * AD, vq = n & 3;
+    const int vq = n & 3;
+    // byte offsets of the lane's reads of blocks j and j + 8 in a tile: one value each, which the compiler would form again in every tile, two
+    // adds and a shift ahead of the first read (0.5 % of a pass over 8192 rows)
+    int va_off[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        va_off[j] = 2 * (vrow * AD + (((4 * (j >> 1) + vq) ^ vrow) << 3) + 4 * ((vq ^ j) & 1));
+        asm("" : "+v"(va_off[j]));
+    }
     // K fragment kb of sub-tile kt: chunk (4 kb + g) ^ n; n < 16 leaves bit 4 alone, so fragments kb and kb + 4 share an
     // address register
     auto k_frag = [&](const bf16_t* ka, int kt, int kb) {
@@ -494,11 +502,9 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         *lds_word(&taken_s[pr]) = t;
         asm volatile("" ::: "memory");
-        const bf16_t* va = v_cur + va_row;
         auto v_frag = [&](int j, int q4) {
-            return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4*)(const_cast<bf16_t*>(va + (16 * q4) * AD + (((4 * ((j >> 1) & 3) + vq) ^ vrow) << 3) +
-                                                                             4 * ((vq ^ j) & 1) + 128 * (j >> 3))));
+            const char* at = reinterpret_cast<const char*>(v_cur) + va_off[j & 7] + 2 * ((16 * q4) * AD + 128 * (j >> 3));
+            return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)const_cast<char*>(at));
         };
         s16x4 Bf[V_FRAG_AHEAD + 1][4];
 #pragma unroll
