@@ -98,6 +98,14 @@ __device__ __forceinline__ float max_over_groups(float x) {
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
+// max(|a|, |b|, c), a NaN among them left out (as one instruction: fmaxf first makes a copy of everything that may be a signalling NaN).
+// The compiler counts no wait states between an MFMA and inline assembly that reads its result: mfma_results_settle() comes before.
+__device__ __forceinline__ void mfma_results_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+__device__ __forceinline__ float max3_abs(float a, float b, float c) {
+    asm volatile("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(c) : "v"(a), "v"(b));
+    return c;
+}
+
 // Key split.  A causal launch with few workgroups is as slow as its longest row block, twice the average.  With tmax > 0 the
 // tiles of a row block (RB = 16 or 32 rows) are cut into parts of tmax tiles, one workgroup per part; a block with more than
 // one part leaves unnormalised partial results (O, reference point m, row sums l) in the workspace and
@@ -109,12 +117,14 @@ __host__ __device__ inline long parts_upto(long n, long c) {      // sum over j 
     const long k = n / c;
     return c * (k * (k + 1) / 2) + (n - k * c) * (k + 1);
 }
-// elements of one part's O, [4 heads][RB rows][256] in half precision (each row divided by its row sum, so that the values are
-// weighted means of V), and floats of its m, l, [4 heads][m | l][RB rows] (RB = rows of a block: 16 or 32)
+// elements of one part's O, [4 heads][RB rows][256] in half precision (each row times the power of two that brings its largest value to
+// 2^14 .. 2^15: a V of any size survives), and floats of its m, l and the inverse of that power u, [4 heads][m | l | u][RB rows] (RB =
+// rows of a block: 16 or 32).  Single precision instead costs 3 - 18 % of a split launch (333 rows on 1500 keys 22.8 us,
+// in halves 19.5; 2048 rows 36.3 and 34.4; halves without the scaling, which V alone can overflow, 18.9 and 33.7).
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-constexpr int part_o_floats(int RB) { return 4 * RB * AD; }
-constexpr long part_bytes(int RB) { return (long)part_o_floats(RB) * 2 + (long)(4 * 2 * RB) * 4; }
-constexpr int part_ml_floats(int RB) { return 4 * 2 * RB; }
+constexpr int part_o_halves(int RB) { return 4 * RB * AD; }
+constexpr int part_ml_floats(int RB) { return 4 * 3 * RB; }
+constexpr long part_bytes(int RB) { return (long)part_o_halves(RB) * 2 + (long)part_ml_floats(RB) * 4; }
 
 // a word of LDS as a volatile object in the LDS address space (through a generic pointer, a volatile access is a flat
 // instruction, which is also counted, and waited for, as an access of global memory)
@@ -566,21 +576,38 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         }
     };
     if (nparts > 1) {
-        // One part of several: leave O / l, m, l of this pair's heads as they are.  A row that sees no key of this part (its
+        // One part of several: leave the scaled O, m, l and u of this pair's heads.  A row that sees no key of this part (its
         // last key lies before the part's first) has exponentiated masked scores against a masked maximum: it is written as
         // the neutral element (m = NEG, l = 0, O = 0).
         const int lr = r0 - rb * RB + n;
         const bool seen = my_last >= ta * KT;
+        mfma_results_settle();
 #pragma unroll
         for (int hh = 0; hh < NH; hh++) {
             const int hq = hq0 + hh;
             _Float16* po = part_o + (slot * 4 + hq) * (RB * AD) + lr * AD + 8 * g;
-            float* pml = part_ml + (slot * 4 + hq) * (2 * RB);
-            const float inv = 1.0f / Lsum[hh][0];
+            float* pml = part_ml + (slot * 4 + hq) * (3 * RB);
+            // the row's largest finite |O|, over this lane's 64 columns and the three lanes with the others
+            constexpr float FINITE = 3.4028234e38f;
+            float tops[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 16; j += 2)
+#pragma unroll
+                for (int i = 0; i < 4; i++) tops[i] = max3_abs(O[hh][j][i], O[hh][j + 1][i], tops[i]);
+            float top = max3_abs(tops[0], tops[1], max3_abs(tops[2], tops[3], 0.f));
+            if (__any(top > FINITE)) {                           // (an infinite V: its columns are infinite, the others keep their values)
+                top = 0.f;
+#pragma unroll
+                for (int j = 0; j < 16; j++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) top = fmaxf(top, fabsf(O[hh][j][i]) <= FINITE ? fabsf(O[hh][j][i]) : 0.f);
+            }
+            const int up_e = min(268 - (int)(__float_as_uint(max_over_groups(top)) >> 23), 253);   // exponent field of the power of two, 14 or more
+            const float up = __uint_as_float((unsigned)up_e << 23);
 #pragma unroll
             for (int jj = 0; jj < 8; jj++) {
                 f32x4 lo, hi;
-                columns(O[hh], jj, inv, lo, hi);
+                columns(O[hh], jj, up, lo, hi);
                 half8 h;
 #pragma unroll
                 for (int i = 0; i < 4; i++) h[i] = (_Float16)(seen ? lo[i] : 0.f), h[4 + i] = (_Float16)(seen ? hi[i] : 0.f);
@@ -589,6 +616,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
             if (g == 0) {
                 pml[RB + lr] = seen ? Lsum[hh][0] : 0.f;
                 pml[lr] = seen ? m_s[pr][hh][n] : NEG;
+                pml[2 * RB + lr] = __uint_as_float((unsigned)(254 - up_e) << 23);      // 1 / up
             }
         }
         return;
@@ -608,13 +636,13 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
 }
 
 // Combines the parts of the row blocks that were split: grid = (split blocks, KV heads, 4 heads of the group x 16-row halves of
-// a block); thread (row, 16-column group) of 16 x 256 outputs.  out = sum_p w_p O_p / sum_p w_p, w_p = 2^(m_p - m) l_p, parts in order; a
+// a block); thread (row, 16-column group) of 16 x 256 outputs.  out = sum_p f_p u_p O_p / sum_p f_p l_p, f_p = 2^(m_p - m), parts in order; a
 // thread's loads of O do not depend on the factors, so all parts are in flight together.
 template <int RB>
 __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                  bf16_t* __restrict__ out, int S, int q_pos0, int tmax, long slots_per_kv,
                                                                  long q_head_stride, int q_row_stride) {
-    constexpr int PO = part_o_floats(RB), PML = part_ml_floats(RB);
+    constexpr int PO = part_o_halves(RB), PML = part_ml_floats(RB);
     const int c = (KT / RB) * tmax, p = (q_pos0 + RB - 1) / RB;
     const int rb = max(0, c - p) + blockIdx.x;                   // the first block with two parts is c - p
     const int np = (p + rb) / c + 1;
@@ -624,17 +652,17 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16*
         const int lr = 16 * (blockIdx.z % (RB / 16)) + (threadIdx.x >> 4);
         if (rb * RB + lr >= S) return;
         const _Float16* po = part_o + (slot0 * 4 + hq) * (RB * AD) + lr * AD + cg * 16;
-        const float* pml = part_ml + (slot0 * 4 + hq) * (2 * RB) + lr;
+        const float* pml = part_ml + (slot0 * 4 + hq) * (3 * RB) + lr;
         // AHEAD parts at a time, all their loads in flight together (an index past the last part loads the last again); the first ones are
         // requested before the maximum is known
         constexpr int AHEAD = 4;
         half8 oh[AHEAD][2];
-        float pm[AHEAD], pl[AHEAD];
+        float pm[AHEAD], pl[AHEAD], pu[AHEAD];
         auto load = [&](int p0) {
 #pragma unroll
             for (int i = 0; i < AHEAD; i++) {
                 const size_t pp = min(p0 + i, np - 1);
-                pm[i] = pml[pp * PML], pl[i] = pml[pp * PML + RB];
+                pm[i] = pml[pp * PML], pl[i] = pml[pp * PML + RB], pu[i] = pml[pp * PML + 2 * RB];
                 oh[i][0] = reinterpret_cast<const half8*>(po + pp * PO)[0], oh[i][1] = reinterpret_cast<const half8*>(po + pp * PO)[1];
             }
         };
@@ -658,12 +686,12 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16*
 #pragma unroll
             for (int k = 0; k < AHEAD; k++) {
                 if (p0 + k >= np) break;
-                const float f = __builtin_amdgcn_exp2f(pm[k] - m) * pl[k];
-                l += f;
+                const float f = __builtin_amdgcn_exp2f(pm[k] - m), fu = f * pu[k];
+                l += f * pl[k];
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc[i][e] += f * (float)oh[k][i >> 1][4 * (i & 1) + e];
+                    for (int e = 0; e < 4; e++) acc[i][e] += fu * (float)oh[k][i >> 1][4 * (i & 1) + e];
             }
             p0 += AHEAD;
             if (p0 >= np) break;
@@ -806,7 +834,7 @@ int qt_gqa_prefill_causal_strided(const void* q, const void* K, const void* V, v
     const int RB = 16 * ks.nh;
     const dim3 grid((ks.tmax ? (unsigned)ks.parts : (unsigned)((S + RB - 1) / RB)) * AKV);
     _Float16* part_o = ks.tmax ? (_Float16*)workspace : nullptr;
-    float* part_ml = ks.tmax ? reinterpret_cast<float*>(part_o + (size_t)ks.parts * AKV * part_o_floats(RB)) : nullptr;
+    float* part_ml = ks.tmax ? reinterpret_cast<float*>(part_o + (size_t)ks.parts * AKV * part_o_halves(RB)) : nullptr;
     if (ks.nh == 2)
         hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(512), 0, stream, (const bf16_t*)q, (const bf16_t*)K, (const bf16_t*)V,
                            (bf16_t*)out, S, L, q_pos0, q_head_stride, q_row_stride, kv_head_stride, ks.tmax, part_o, part_ml);

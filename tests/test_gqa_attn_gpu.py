@@ -365,6 +365,30 @@ def test_prefill_causal_key_split(qt, dev, S, P0, qscale):
         check_attn(f"S={S} P0={P0} row {r}", o[:, r:r + 1], ref)
 
 
+# split launches of 16- and 32-row blocks
+@pytest.mark.parametrize("S,P0", [(17, 700), (800, 0), (333, 1500), (2048, 0), (700, 3000)])
+@pytest.mark.parametrize("k", [100, 17, -30])
+def test_prefill_causal_split_range_of_v(qt, dev, S, P0, k):
+    """V times a power of two: every product, sum and mean scales exactly, so a split launch returns the same significant bits whatever the
+    size of V (parts in half precision as they are were infinite from 2^17 on and lost their bits below 2^-24).  An infinite or
+    undefined value of V goes into its column and leaves the others alone."""
+    from qwen_tailor_amd import _lib as QL
+    L = S + P0
+    assert QL.lib().qt_gqa_prefill_workspace_bytes_for(S, L, P0) > 0, "this case is meant to be split"
+    g = torch.Generator().manual_seed(S + P0)
+    q, K, V = (torch.randn(shape, generator=g).bfloat16().to(dev)[None] for shape in ((8, S, 256), (2, L, 256), (2, L, 256)))
+    run = lambda v: qt.attention.scaled_dot_product_attention(q, K, v, scale=256 ** -0.5, mask="causal")
+    scaled = (V.float() * 2.0 ** k).bfloat16()
+    got, want = run(scaled), (run(V).float() * 2.0 ** k).bfloat16()
+    assert bool(torch.isfinite(got).all())
+    check_tensors_equal(f"V times 2^{k}", got, want)
+    scaled[:, :, 0, 5], scaled[:, :, 0, 200] = float("inf"), float("nan")      # (key 0: every row sees it)
+    got = run(scaled)
+    assert bool((got[..., 5] == float("inf")).all()) and bool(torch.isnan(got[..., 200]).all())
+    got[..., 5], got[..., 200] = want[..., 5], want[..., 200]
+    check_tensors_equal(f"V times 2^{k}, the other columns", got, want)
+
+
 @pytest.mark.parametrize("S,P0", [(1024, 0), (2048, 0), (300, 3000), (5000, 0)])
 def test_prefill_causal_head_strides(qt, dev, S, P0):
     """q / out with a head stride beyond S rows and K / V inside a longer cache, through the C ABI, in every form of the launch
