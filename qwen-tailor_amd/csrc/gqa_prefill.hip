@@ -117,14 +117,22 @@ __host__ __device__ inline long parts_upto(long n, long c) {      // sum over j 
     const long k = n / c;
     return c * (k * (k + 1) / 2) + (n - k * c) * (k + 1);
 }
-// elements of one part's O, [4 heads][RB rows][256] in half precision (each row times the power of two that brings its largest value to
-// 2^14 .. 2^15: a V of any size survives), and floats of its m, l and the inverse of that power u, [4 heads][m | l | u][RB rows] (RB =
-// rows of a block: 16 or 32).  Single precision instead costs 3 - 18 % of a split launch (333 rows on 1500 keys 22.8 us,
-// in halves 19.5; 2048 rows 36.3 and 34.4; halves without the scaling, which V alone can overflow, 18.9 and 33.7).
+// elements of one part's O, [4 heads][RB rows][256] in half precision, and floats of its m, l, [4 heads][m | l][RB rows] (RB = rows of a
+// block: 16 or 32).  So that a V of any size survives, each row of O is stored times the power of two that brings its largest value
+// to 2^13 .. 2^14.  The exponent of that power takes the place of the low eight bits of m (tagged_m); what this adds to m is taken out
+// of O and l again.  Where m is 2^14 or more its low bits count: there O is stored divided by l instead, weighted means of V.
+// (333 rows on 1500 keys 18.8 us, 2048 rows 33.9; without the scaling 18.6 and 33.8; the exponent in an array of its own 19.5 and 34.4; O in
+// single precision 22.8 and 36.3.)
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 constexpr int part_o_halves(int RB) { return 4 * RB * AD; }
-constexpr int part_ml_floats(int RB) { return 4 * 3 * RB; }
+constexpr int part_ml_floats(int RB) { return 4 * 2 * RB; }
 constexpr long part_bytes(int RB) { return (long)part_o_halves(RB) * 2 + (long)part_ml_floats(RB) * 4; }
+constexpr float TAG_BELOW = 16384.f;
+__device__ __forceinline__ float tagged_m(float m, int e) { return __uint_as_float((__float_as_uint(m) & ~255u) | (unsigned)e); }
+// what a part's O is multiplied by in the merge, besides its factor 2^(m - reference)
+__device__ __forceinline__ float part_unit(float m, float l) {
+    return fabsf(m) < TAG_BELOW ? __uint_as_float((254 - (__float_as_uint(m) & 255u)) << 23) : l;
+}
 
 // a word of LDS as a volatile object in the LDS address space (through a generic pointer, a volatile access is a flat
 // instruction, which is also counted, and waited for, as an access of global memory)
@@ -576,7 +584,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         }
     };
     if (nparts > 1) {
-        // One part of several: leave the scaled O, m, l and u of this pair's heads.  A row that sees no key of this part (its
+        // One part of several: leave the scaled O, m, l of this pair's heads.  A row that sees no key of this part (its
         // last key lies before the part's first) has exponentiated masked scores against a masked maximum: it is written as
         // the neutral element (m = NEG, l = 0, O = 0).
         const int lr = r0 - rb * RB + n;
@@ -586,7 +594,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         for (int hh = 0; hh < NH; hh++) {
             const int hq = hq0 + hh;
             _Float16* po = part_o + (slot * 4 + hq) * (RB * AD) + lr * AD + 8 * g;
-            float* pml = part_ml + (slot * 4 + hq) * (3 * RB);
+            float* pml = part_ml + (slot * 4 + hq) * (2 * RB);
             // the row's largest finite |O|, over this lane's 64 columns and the three lanes with the others
             constexpr float FINITE = 3.4028234e38f;
             float tops[4] = {0.f, 0.f, 0.f, 0.f};
@@ -602,8 +610,12 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
 #pragma unroll
                     for (int i = 0; i < 4; i++) top = fmaxf(top, fabsf(O[hh][j][i]) <= FINITE ? fabsf(O[hh][j][i]) : 0.f);
             }
-            const int up_e = min(268 - (int)(__float_as_uint(max_over_groups(top)) >> 23), 253);   // exponent field of the power of two, 14 or more
-            const float up = __uint_as_float((unsigned)up_e << 23);
+            const int up_e = min(267 - (int)(__float_as_uint(max_over_groups(top)) >> 23), 253);   // exponent field of the power of two, 13 or more
+            const float m = m_s[pr][hh][n], l = Lsum[hh][0];
+            const bool tag = fabsf(m) < TAG_BELOW;
+            const float m_part = tag ? tagged_m(m, up_e) : m;
+            const float back = tag ? __builtin_amdgcn_exp2f(m - m_part) : 1.f;              // 2^-1/4 .. 2^1/4
+            const float up = tag ? __uint_as_float((unsigned)up_e << 23) * back : 1.0f / l;
 #pragma unroll
             for (int jj = 0; jj < 8; jj++) {
                 f32x4 lo, hi;
@@ -614,9 +626,8 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
                 *reinterpret_cast<half8*>(po + 32 * jj) = h;
             }
             if (g == 0) {
-                pml[RB + lr] = seen ? Lsum[hh][0] : 0.f;
-                pml[lr] = seen ? m_s[pr][hh][n] : NEG;
-                pml[2 * RB + lr] = __uint_as_float((unsigned)(254 - up_e) << 23);      // 1 / up
+                pml[RB + lr] = seen ? l * back : 0.f;
+                pml[lr] = seen ? m_part : NEG;
             }
         }
         return;
@@ -636,7 +647,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
 }
 
 // Combines the parts of the row blocks that were split: grid = (split blocks, KV heads, 4 heads of the group x 16-row halves of
-// a block); thread (row, 16-column group) of 16 x 256 outputs.  out = sum_p f_p u_p O_p / sum_p f_p l_p, f_p = 2^(m_p - m), parts in order; a
+// a block); thread (row, 16-column group) of 16 x 256 outputs.  out = sum_p f_p u_p O_p / sum_p f_p l_p, f_p = 2^(m_p - m), u_p = part_unit, parts in order; a
 // thread's loads of O do not depend on the factors, so all parts are in flight together.
 template <int RB>
 __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16* __restrict__ part_o, const float* __restrict__ part_ml,
@@ -652,17 +663,17 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16*
         const int lr = 16 * (blockIdx.z % (RB / 16)) + (threadIdx.x >> 4);
         if (rb * RB + lr >= S) return;
         const _Float16* po = part_o + (slot0 * 4 + hq) * (RB * AD) + lr * AD + cg * 16;
-        const float* pml = part_ml + (slot0 * 4 + hq) * (3 * RB) + lr;
+        const float* pml = part_ml + (slot0 * 4 + hq) * (2 * RB) + lr;
         // AHEAD parts at a time, all their loads in flight together (an index past the last part loads the last again); the first ones are
         // requested before the maximum is known
         constexpr int AHEAD = 4;
         half8 oh[AHEAD][2];
-        float pm[AHEAD], pl[AHEAD], pu[AHEAD];
+        float pm[AHEAD], pl[AHEAD];
         auto load = [&](int p0) {
 #pragma unroll
             for (int i = 0; i < AHEAD; i++) {
                 const size_t pp = min(p0 + i, np - 1);
-                pm[i] = pml[pp * PML], pl[i] = pml[pp * PML + RB], pu[i] = pml[pp * PML + 2 * RB];
+                pm[i] = pml[pp * PML], pl[i] = pml[pp * PML + RB];
                 oh[i][0] = reinterpret_cast<const half8*>(po + pp * PO)[0], oh[i][1] = reinterpret_cast<const half8*>(po + pp * PO)[1];
             }
         };
@@ -686,7 +697,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16*
 #pragma unroll
             for (int k = 0; k < AHEAD; k++) {
                 if (p0 + k >= np) break;
-                const float f = __builtin_amdgcn_exp2f(pm[k] - m), fu = f * pu[k];
+                const float f = __builtin_amdgcn_exp2f(pm[k] - m), fu = f * part_unit(pm[k], pl[k]);
                 l += f * pl[k];
 #pragma unroll
                 for (int i = 0; i < 4; i++)

@@ -367,26 +367,30 @@ def test_prefill_causal_key_split(qt, dev, S, P0, qscale):
 
 # split launches of 16- and 32-row blocks
 @pytest.mark.parametrize("S,P0", [(17, 700), (800, 0), (333, 1500), (2048, 0), (700, 3000)])
-@pytest.mark.parametrize("k", [100, 17, -30])
-def test_prefill_causal_split_range_of_v(qt, dev, S, P0, k):
-    """V times a power of two: every product, sum and mean scales exactly, so a split launch returns the same significant bits whatever the
-    size of V (parts in half precision as they are were infinite from 2^17 on and lost their bits below 2^-24).  An infinite or
-    undefined value of V goes into its column and leaves the others alone."""
+@pytest.mark.parametrize("qscale,k", [(1, 100), (1, 17), (1, -30), (200, 100), (3e3, 12), (3e4, 12)])
+def test_prefill_causal_split_range_of_v(qt, dev, S, P0, qscale, k):
+    """V times a power of two scales every product, sum and mean exactly, in a split launch up to the rounding of its parts (parts in
+    half precision as they are were infinite from 2^17 on and lost their bits below 2^-24).  An infinite or undefined value of V goes
+    into its column and leaves the others alone.  qscale: reference points of a few units, of some hundreds, around 2^14 and beyond
+    it, where parts are weighted means of V and hold it up to 65504."""
     from qwen_tailor_amd import _lib as QL
     L = S + P0
     assert QL.lib().qt_gqa_prefill_workspace_bytes_for(S, L, P0) > 0, "this case is meant to be split"
     g = torch.Generator().manual_seed(S + P0)
     q, K, V = (torch.randn(shape, generator=g).bfloat16().to(dev)[None] for shape in ((8, S, 256), (2, L, 256), (2, L, 256)))
-    run = lambda v: qt.attention.scaled_dot_product_attention(q, K, v, scale=256 ** -0.5, mask="causal")
+    q = (q.float() * qscale).bfloat16()
+    run = lambda v: qt.attention.scaled_dot_product_attention(q, K, v, scale=256 ** -0.5, mask="causal").double()
     scaled = (V.float() * 2.0 ** k).bfloat16()
-    got, want = run(scaled), (run(V).float() * 2.0 ** k).bfloat16()
-    assert bool(torch.isfinite(got).all())
-    check_tensors_equal(f"V times 2^{k}", got, want)
+    got, want = run(scaled) * 2.0 ** -k, run(V)
+    # one step of bf16 (2^-7 of a value at most), and two roundings of parts (2^-12 of a part's value, a few times the row's largest output)
+    bound = 2.0 ** -7 * want.abs() + 2.0 ** -9 * want.abs().amax(-1, keepdim=True)
+    assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() / bound).max())
     scaled[:, :, 0, 5], scaled[:, :, 0, 200] = float("inf"), float("nan")      # (key 0: every row sees it)
-    got = run(scaled)
-    assert bool((got[..., 5] == float("inf")).all()) and bool(torch.isnan(got[..., 200]).all())
+    got = run(scaled) * 2.0 ** -k
+    if qscale == 1:                                               # (otherwise key 0 has no weight in most rows)
+        assert bool((got[..., 5] == float("inf")).all()) and bool(torch.isnan(got[..., 200]).all())
     got[..., 5], got[..., 200] = want[..., 5], want[..., 200]
-    check_tensors_equal(f"V times 2^{k}, the other columns", got, want)
+    assert bool(((got - want).abs() <= bound).all()), "a value that is not finite has left its column"
 
 
 @pytest.mark.parametrize("S,P0", [(1024, 0), (2048, 0), (300, 3000), (5000, 0)])
