@@ -117,20 +117,22 @@ __host__ __device__ inline long parts_upto(long n, long c) {      // sum over j 
     const long k = n / c;
     return c * (k * (k + 1) / 2) + (n - k * c) * (k + 1);
 }
-// elements of one part's O, [4 heads][RB rows][256] in half precision, and floats of its m, l, [4 heads][m | l][RB rows] (RB = rows of a
-// block: 16 or 32).  So that a V of any size survives, each row of O is stored times the power of two that brings its largest value
+// elements of one part's O, [4 heads][RB rows][256] in single (`wide`) or half precision, and floats of its m, l, [4 heads][m | l][RB
+// rows] (RB = rows of a block: 16 or 32).  Half precision: so that a V of any size survives, each row of O is stored times the power of two that brings its largest value
 // to 2^13 .. 2^14.  The exponent of that power takes the place of the low eight bits of m (tagged_m); what this adds to m is taken out
 // of O and l again.  Where m is 2^14 or more its low bits count: there O is stored divided by l instead, weighted means of V.
 // (333 rows on 1500 keys 18.8 us, 2048 rows 33.9; without the scaling 18.6 and 33.8; the exponent in an array of its own 19.5 and 34.4; O in
 // single precision 22.8 and 36.3.)
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-constexpr int part_o_halves(int RB) { return 4 * RB * AD; }
+constexpr int part_o_size(int RB) { return 4 * RB * AD; }
 constexpr int part_ml_floats(int RB) { return 4 * 2 * RB; }
-constexpr long part_bytes(int RB) { return (long)part_o_halves(RB) * 2 + (long)part_ml_floats(RB) * 4; }
+constexpr long part_bytes(int RB, bool wide) { return (long)part_o_size(RB) * (wide ? 4 : 2) + (long)part_ml_floats(RB) * 4; }
 constexpr float TAG_BELOW = 16384.f;
 __device__ __forceinline__ float tagged_m(float m, int e) { return __uint_as_float((__float_as_uint(m) & ~255u) | (unsigned)e); }
 // what a part's O is multiplied by in the merge, besides its factor 2^(m - reference)
+template <class PT>
 __device__ __forceinline__ float part_unit(float m, float l) {
+    if (sizeof(PT) == 4) return 1.f;
     return fabsf(m) < TAG_BELOW ? __uint_as_float((254 - (__float_as_uint(m) & 255u)) << 23) : l;
 }
 
@@ -162,11 +164,12 @@ __device__ __forceinline__ volatile __attribute__((address_space(3))) int* lds_w
 // (taken_s[pr] = t), and the score wavefront, which writes the next P a few thousand clocks later, looks at that word first.
 // grid = (row blocks, or parts when tmax > 0) x KV heads in one dimension, the KV head varying fastest: workgroups are
 // dispatched in the order of their index, so both heads' long row blocks come first.
-template <int NH>
+// PT: what O of a part is kept in, _Float16 or float.
+template <int NH, class PT>
 __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ K,
                                                               const bf16_t* __restrict__ V, bf16_t* __restrict__ out, int S, int L,
                                                               int q_pos0, long q_head_stride, int q_row_stride, long kv_head_stride, int tmax,
-                                                              _Float16* __restrict__ part_o, float* __restrict__ part_ml) {
+                                                              PT* __restrict__ part_o, float* __restrict__ part_ml) {
     __shared__ __align__(1024) bf16_t kv_s[4 * TILE];            // K tiles of even / odd iterations, then the V tiles
     __shared__ __align__(16) u32x4 p_s[4][NH][2][64];             // [pair][head][32-key half][lane]: P as the lanes hold it
     __shared__ __align__(16) float c_s[4][NH][16];               // [pair][head][row]: factor of a row whose reference moved
@@ -587,43 +590,54 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         // One part of several: leave the scaled O, m, l of this pair's heads.  A row that sees no key of this part (its
         // last key lies before the part's first) has exponentiated masked scores against a masked maximum: it is written as
         // the neutral element (m = NEG, l = 0, O = 0).
+        constexpr bool HALF = sizeof(PT) == 2;
         const int lr = r0 - rb * RB + n;
         const bool seen = my_last >= ta * KT;
-        mfma_results_settle();
+        if (HALF) mfma_results_settle();
 #pragma unroll
         for (int hh = 0; hh < NH; hh++) {
             const int hq = hq0 + hh;
-            _Float16* po = part_o + (slot * 4 + hq) * (RB * AD) + lr * AD + 8 * g;
+            PT* po = part_o + (slot * 4 + hq) * (RB * AD) + lr * AD + 8 * g;
             float* pml = part_ml + (slot * 4 + hq) * (2 * RB);
-            // the row's largest finite |O|, over this lane's 64 columns and the three lanes with the others
-            constexpr float FINITE = 3.4028234e38f;
-            float tops[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < 16; j += 2)
-#pragma unroll
-                for (int i = 0; i < 4; i++) tops[i] = max3_abs(O[hh][j][i], O[hh][j + 1][i], tops[i]);
-            float top = max3_abs(tops[0], tops[1], max3_abs(tops[2], tops[3], 0.f));
-            if (__any(top > FINITE)) {                           // (an infinite V: its columns are infinite, the others keep their values)
-                top = 0.f;
-#pragma unroll
-                for (int j = 0; j < 16; j++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) top = fmaxf(top, fabsf(O[hh][j][i]) <= FINITE ? fabsf(O[hh][j][i]) : 0.f);
-            }
-            const int up_e = min(267 - (int)(__float_as_uint(max_over_groups(top)) >> 23), 253);   // exponent field of the power of two, 13 or more
             const float m = m_s[pr][hh][n], l = Lsum[hh][0];
-            const bool tag = fabsf(m) < TAG_BELOW;
-            const float m_part = tag ? tagged_m(m, up_e) : m;
-            const float back = tag ? __builtin_amdgcn_exp2f(m - m_part) : 1.f;              // 2^-1/4 .. 2^1/4
-            const float up = tag ? __uint_as_float((unsigned)up_e << 23) * back : 1.0f / l;
+            float m_part = m, back = 1.f, up = 1.f;
+            if constexpr (HALF) {
+                // the row's largest finite |O|, over this lane's 64 columns and the three lanes with the others
+                constexpr float FINITE = 3.4028234e38f;
+                float tops[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < 16; j += 2)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) tops[i] = max3_abs(O[hh][j][i], O[hh][j + 1][i], tops[i]);
+                float top = max3_abs(tops[0], tops[1], max3_abs(tops[2], tops[3], 0.f));
+                if (__any(top > FINITE)) {                       // (an infinite V: its columns are infinite, the others keep their values)
+                    top = 0.f;
+#pragma unroll
+                    for (int j = 0; j < 16; j++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) top = fmaxf(top, fabsf(O[hh][j][i]) <= FINITE ? fabsf(O[hh][j][i]) : 0.f);
+                }
+                const int up_e = min(267 - (int)(__float_as_uint(max_over_groups(top)) >> 23), 253);   // exponent field of the power of two, 13 or more
+                const bool tag = fabsf(m) < TAG_BELOW;
+                m_part = tag ? tagged_m(m, up_e) : m;
+                back = tag ? __builtin_amdgcn_exp2f(m - m_part) : 1.f;                                 // 2^-1/4 .. 2^1/4
+                up = tag ? __uint_as_float((unsigned)up_e << 23) * back : 1.0f / l;
+            }
 #pragma unroll
             for (int jj = 0; jj < 8; jj++) {
                 f32x4 lo, hi;
                 columns(O[hh], jj, up, lo, hi);
-                half8 h;
 #pragma unroll
-                for (int i = 0; i < 4; i++) h[i] = (_Float16)(seen ? lo[i] : 0.f), h[4 + i] = (_Float16)(seen ? hi[i] : 0.f);
-                *reinterpret_cast<half8*>(po + 32 * jj) = h;
+                for (int i = 0; i < 4; i++) lo[i] = seen ? lo[i] : 0.f, hi[i] = seen ? hi[i] : 0.f;
+                if constexpr (HALF) {
+                    half8 h;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) h[i] = (_Float16)lo[i], h[4 + i] = (_Float16)hi[i];
+                    *reinterpret_cast<half8*>(po + 32 * jj) = h;
+                } else {
+                    reinterpret_cast<f32x4*>(po + 32 * jj)[0] = lo;
+                    reinterpret_cast<f32x4*>(po + 32 * jj)[1] = hi;
+                }
             }
             if (g == 0) {
                 pml[RB + lr] = seen ? l * back : 0.f;
@@ -647,13 +661,14 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
 }
 
 // Combines the parts of the row blocks that were split: grid = (split blocks, KV heads, 4 heads of the group x 16-row halves of
-// a block); thread (row, 16-column group) of 16 x 256 outputs.  out = sum_p f_p u_p O_p / sum_p f_p l_p, f_p = 2^(m_p - m), u_p = part_unit, parts in order; a
+// a block); thread (row, lane c of 16) of 16 x 256 outputs has the 16 bytes c of every 256 of
+// a part's row.  out = sum_p f_p u_p O_p / sum_p f_p l_p, f_p = 2^(m_p - m), u_p = part_unit, parts in order; a
 // thread's loads of O do not depend on the factors, so all parts are in flight together.
-template <int RB>
-__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16* __restrict__ part_o, const float* __restrict__ part_ml,
+template <int RB, class PT>
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const PT* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                  bf16_t* __restrict__ out, int S, int q_pos0, int tmax, long slots_per_kv,
                                                                  long q_head_stride, int q_row_stride) {
-    constexpr int PO = part_o_halves(RB), PML = part_ml_floats(RB);
+    constexpr int PO = part_o_size(RB), PML = part_ml_floats(RB);
     const int c = (KT / RB) * tmax, p = (q_pos0 + RB - 1) / RB;
     const int rb = max(0, c - p) + blockIdx.x;                   // the first block with two parts is c - p
     const int np = (p + rb) / c + 1;
@@ -662,19 +677,22 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16*
     {
         const int lr = 16 * (blockIdx.z % (RB / 16)) + (threadIdx.x >> 4);
         if (rb * RB + lr >= S) return;
-        const _Float16* po = part_o + (slot0 * 4 + hq) * (RB * AD) + lr * AD + cg * 16;
+        constexpr int VEC = 16 / sizeof(PT), NV = AD / 16 / VEC;  // values of a load, loads of a part
+        typedef PT vec __attribute__((ext_vector_type(VEC)));
+        const PT* po = part_o + (slot0 * 4 + hq) * (RB * AD) + lr * AD + cg * VEC;
         const float* pml = part_ml + (slot0 * 4 + hq) * (2 * RB) + lr;
         // AHEAD parts at a time, all their loads in flight together (an index past the last part loads the last again); the first ones are
         // requested before the maximum is known
         constexpr int AHEAD = 4;
-        half8 oh[AHEAD][2];
+        vec ov[AHEAD][NV];
         float pm[AHEAD], pl[AHEAD];
         auto load = [&](int p0) {
 #pragma unroll
             for (int i = 0; i < AHEAD; i++) {
                 const size_t pp = min(p0 + i, np - 1);
                 pm[i] = pml[pp * PML], pl[i] = pml[pp * PML + RB];
-                oh[i][0] = reinterpret_cast<const half8*>(po + pp * PO)[0], oh[i][1] = reinterpret_cast<const half8*>(po + pp * PO)[1];
+#pragma unroll
+                for (int j = 0; j < NV; j++) ov[i][j] = *reinterpret_cast<const vec*>(po + pp * PO + 16 * VEC * j);
             }
         };
         load(0);
@@ -690,34 +708,32 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const _Float16*
             for (int i = 0; i < AHEAD; i++) m = fmaxf(m, mv[i]);
         }
         float l = 0.f;
-        f32x4 acc[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float acc[NV][VEC] = {};
         for (int p0 = 0;;) {
 #pragma unroll
             for (int k = 0; k < AHEAD; k++) {
                 if (p0 + k >= np) break;
-                const float f = __builtin_amdgcn_exp2f(pm[k] - m), fu = f * part_unit(pm[k], pl[k]);
+                const float f = __builtin_amdgcn_exp2f(pm[k] - m), fu = f * part_unit<PT>(pm[k], pl[k]);
                 l += f * pl[k];
 #pragma unroll
-                for (int i = 0; i < 4; i++)
+                for (int j = 0; j < NV; j++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc[i][e] += fu * (float)oh[k][i >> 1][4 * (i & 1) + e];
+                    for (int e = 0; e < VEC; e++) acc[j][e] += fu * (float)ov[k][j][e];
             }
             p0 += AHEAD;
             if (p0 >= np) break;
             load(p0);
         }
         const float inv = 1.0f / l;
-        uint32_t pk[8];
+        bf16_t* dst = out + (size_t)(blockIdx.y * (AH / AKV) + hq) * q_head_stride + (size_t)(rb * RB + lr) * q_row_stride + cg * VEC;
+        typedef unsigned words __attribute__((ext_vector_type(VEC / 2)));
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            pk[2 * i] = pack_bf(acc[i][0] * inv, acc[i][1] * inv);
-            pk[2 * i + 1] = pack_bf(acc[i][2] * inv, acc[i][3] * inv);
+        for (int j = 0; j < NV; j++) {
+            words pk;
+#pragma unroll
+            for (int e = 0; e < VEC / 2; e++) pk[e] = pack_bf(acc[j][2 * e] * inv, acc[j][2 * e + 1] * inv);
+            *reinterpret_cast<words*>(dst + 16 * VEC * j) = pk;
         }
-        u32x4* dst = reinterpret_cast<u32x4*>(out + (size_t)(blockIdx.y * (AH / AKV) + hq) * q_head_stride + (size_t)(rb * RB + lr) * q_row_stride + cg * 16);
-        dst[0] = u32x4{pk[0], pk[1], pk[2], pk[3]};
-        dst[1] = u32x4{pk[4], pk[5], pk[6], pk[7]};
     }
 }
 
@@ -729,46 +745,47 @@ inline bool two_heads_per_wave(int S) { return (S + 31) / 32 * AKV >= 288; }   /
 
 // The key split of a launch: tmax = 0 (none) or the tiles per part, parts = grid width, split_blocks = blocks with several parts.
 // Only launches that leave CUs without a workgroup are split (fewer than 2048 query rows: a short continuation of a long
-// prefix, a short prompt), and only as far as the idle CUs go; the split must shorten the longest workgroup by four tiles or more to pay for
-// the merge launch (200 rows on 100 keys, by two: 11.8 us against 10.7; 333 rows, by three: 12.0 against 11.4; 100 rows on 300 keys, by
-// four: 12.0 against 13.1).  A workgroup costs about 6 us beyond its tiles (dispatch, Q and first-tile latency, the output stores).
+// prefix, a short prompt), and only as far as the idle CUs go: all parts are resident at once, because a CU that has to run a second part
+// pays the 6 us that a workgroup costs beyond its tiles (dispatch, Q and first-tile latency, the output stores) twice.
 struct KeySplit {
     int nh = 1;            // heads per wavefront: row blocks of 16 nh rows
     int tmax = 0;
     long parts = 0;
     int split_blocks = 0;
-    long bytes() const { return parts * AKV * part_bytes(16 * nh); }
+    bool wide = false;     // parts in single precision
+    long bytes() const { return parts * AKV * part_bytes(16 * nh, wide); }
 };
-KeySplit plan_split_nh(int S, int L, int q_pos0, int nh, int min_gain) {
-    KeySplit ks;
-    ks.nh = nh;
-    const int RB = 16 * nh, nb = (S + RB - 1) / RB, cus = cu_count();
-    if (S < 1 || nb * AKV >= cus) return ks;
-    const int longest = (std::min(L, q_pos0 + S) + KT - 1) / KT; // (the last block's)
-    // the part size (at least 3 tiles) with the least time among those whose parts are all resident at once: a CU
-    // that has to run a second part pays the per-workgroup cost twice.  In us, fitted to a sweep of 17 - 1460 rows on 0 - 6000 keys: a tile
-    // 1.25 (32-row blocks 1.8), a part 0.033 in the merge (twice that), and 0.85 for every four parts that the merge takes one after the
-    // other.  (At least 6 tiles always, against this: 17 rows on 700 / 1500 keys 15.1 / 15.3 and 11.5 / 12.7, 100 rows on 700 / 3000 15.4 / 18.8
-    // and 13.1 / 17.8, 333 on 300 / 1500 16.3 / 19.6 and 13.9 / 19.2, 700 rows 17.1 and 15.4.)
-    // The search begins at a lower bound of the tiles per CU and ends where the tiles alone cost more than the best found: a dozen
-    // divisions, because a launch of 20 us does not hide much of its host.
+// A form of split launch and its time, us: base + tile * (tiles per part) + part * (parts, both KV heads) + round * (groups of four parts that
+// the merge takes one after the other).  It takes part sizes from min_tiles on that shorten the longest workgroup by min_gain tiles.
+struct SplitForm {
+    int nh, min_tiles, min_gain;
+    bool wide;
+    float base, tile, part, round;
+};
+// Takes the form if its best part size is faster than `us`, the best so far.  parts(t) falls with t: the smallest resident part size is found
+// by bisection, and the few sizes from there on are priced (a launch of 20 us does not hide much of its host).
+void consider(const SplitForm& f, int S, int L, int q_pos0, KeySplit& best, float& us) {
+    const int RB = 16 * f.nh, nb = (S + RB - 1) / RB, cus = cu_count();
+    if (S < 1 || nb * AKV >= cus) return;
+    const int most = (std::min(L, q_pos0 + S) + KT - 1) / KT - f.min_gain;       // (the last block's tiles, less the gain)
     const long p = (q_pos0 + RB - 1) / RB, cpt = KT / RB;
-    const float per_tile = nh == 1 ? 1.25f : 1.8f;
-    const long least_tiles = (long)nb * (q_pos0 + 1) / KT + (long)RB * nb * (nb - 1) / (2 * KT);
-    int tmax = longest;
-    float least = 1e30f;
-    for (int t = (int)std::max(3L, least_tiles * AKV / cus); t <= longest && per_tile * t < least; t++) {
-        const long c = cpt * t, parts = (parts_upto(p + nb, c) - parts_upto(p, c)) * AKV;
-        if (parts > cus) continue;
-        const float us = per_tile * t + 0.033f * nh * parts + 0.85f * (((p + nb + c - 1) / c + 3) / 4);
-        if (us < least) least = us, tmax = t;
+    auto parts = [&](int t) { return parts_upto(p + nb, cpt * t) - parts_upto(p, cpt * t); };
+    int t = f.min_tiles, hi = most + 1;
+    if (t > most) return;
+    if (parts(t) * AKV > cus)
+        while (hi - t > 1) {                                     // parts(t) are too many, parts(hi) are not or hi is out of range
+            const int mid = (t + hi) / 2;
+            if (parts(mid) * AKV > cus) t = mid; else hi = mid;
+        }
+    else
+        hi = t;
+    for (t = hi; t <= std::min(most, hi + 8) && f.base + f.tile * t < us; t++) {
+        const long n = parts(t), c = cpt * t;
+        const float now = f.base + f.tile * t + f.part * AKV * n + f.round * (((p + nb + c - 1) / c + 3) / 4);
+        if (now >= us) continue;
+        us = now;
+        best.nh = f.nh, best.tmax = t, best.parts = n, best.split_blocks = nb - (int)std::max(0L, c - p), best.wide = f.wide;
     }
-    if (longest - tmax < min_gain) return ks;                    // the merge launch has to be earned
-    const long c = cpt * tmax;
-    ks.tmax = tmax;
-    ks.parts = parts_upto(p + nb, c) - parts_upto(p, c);
-    ks.split_blocks = nb - (int)std::max(0L, c - p);
-    return ks;
 }
 // The form of a launch, by measurement (us at q_pos0 = 0, 16-row blocks (NH = 1) in their best form / 32-row blocks (NH = 2) with
 // the split: S = 1280 25.3 / 27.3, 1408 27.7 / 27.7, 1536 32.3 / 30.0, 2048 47.0 / 37.2, 2560 59.9 / 51.4, 2944 68.5 / 63.3,
@@ -776,28 +793,33 @@ KeySplit plan_split_nh(int S, int L, int q_pos0, int nh, int min_gain) {
 //   from about 4600 rows on     NH = 2, unsplit (enough 32-row blocks to balance themselves);
 //   from about 1500 rows on     NH = 2 with the key split, where the launch leaves room for it and, for a whole prompt, up to
 //                               3200 rows (a tile of a 32-row block costs less than two tiles of 16-row blocks, but its parts
-//                               are twice the size);
-//   fewer rows, split           the form whose parts are shorter in time: a workgroup with 32 rows costs 3.5 us more besides its tiles, and
-//                               a tile 1.8 against 1.25 us.  (NH = 1 / 2, us: 333 rows on 1500 / 6000 / 8000 keys 19.5 / 22.3, 30.2 / 29.7,
-//                               41.9 / 35.4, 700 on 700 / 1500 / 3000 / 6000 21.9 / 25.6, 26.8 / 26.6, 37.6 / 32.2, 77.9 / 49.7, 1300 on 300 / 1500 /
-//                               6000 26.8 / 27.5, 47.5 / 38.2, 153 / 82.6);
-//   everything else             NH = 1, split if CUs would idle.
+//                               are twice the size): the smallest resident parts of six tiles or more, if they shorten the longest
+//                               workgroup by four;
+//   fewer rows                  the fastest of no split (NH = 1), NH = 1 with parts of six tiles or more in half precision, NH = 1 with parts
+//                               of three tiles or more and NH = 2, both in single precision.
+// Half precision is for launches that are split in earnest.  A few more tiles side by side, or more rows split for the sake of the
+// larger block, are no reason to give up bits: without the split those rows are summed in single precision to the end.
+// The times are fitted to 15 sizes of 1 - 1400 rows on 11 prefixes of 0 - 32000 keys, each form at up to nine part sizes; the choice is
+// within 0.4 % of the best of these forms on average and 6 % at worst.  With short parts in half precision as well / as chosen: 17 rows on
+// 700 keys 11.7 / 12.7 us, 333 on 300 / 1500 13.5 / 15.9 and 18.9 / 19.4, 600 13.4 / 15.3, 700 on 3000 32.7 / 36.6, 1185 on 1500 36.2 / 38.8.
 KeySplit plan_split(int S, int L, int q_pos0) {
+    KeySplit ks;
     if (two_heads_per_wave(S)) {                                 // (two heads: S >= 1472, or parts of several tiles, so L >= one tile)
-        KeySplit ks;
         ks.nh = 2;
         return ks;
     }
     if (S >= 1472 && (q_pos0 > 0 || S <= 3200)) {
-        const KeySplit ks = plan_split_nh(S, L, q_pos0, 2, 4);
+        float any = 1e30f;
+        consider(SplitForm{2, 6, 4, false, 0.f, 1.f, 0.f, 0.f}, S, L, q_pos0, ks, any);        // (priced by its tiles alone)
         if (ks.tmax) return ks;
     }
-    const KeySplit one = plan_split_nh(S, L, q_pos0, 1, 4);
-    if (1.25f * one.tmax > 3.5f + 1.8f * 3) {                    // (parts of 32-row blocks have three tiles or more)
-        const KeySplit two = plan_split_nh(S, L, q_pos0, 2, 4);
-        if (two.tmax && 1.25f * one.tmax - 1.8f * two.tmax > 3.5f) return two;
+    float us = 4.2f + 1.2f * ((std::min(L, q_pos0 + S) + KT - 1) / KT);         // no split
+    consider(SplitForm{1, 6, 6, false, 6.7f, 1.03f, 0.019f, 1.03f}, S, L, q_pos0, ks, us);
+    if (S < 1472) {
+        consider(SplitForm{1, 3, 1, true, 7.7f, 0.97f, 0.030f, 1.05f}, S, L, q_pos0, ks, us);
+        consider(SplitForm{2, 3, 1, true, 10.4f, 1.51f, 0.037f, 0.61f}, S, L, q_pos0, ks, us);
     }
-    return one;
+    return ks;
 }
 
 }  // namespace
@@ -811,16 +833,9 @@ long qt_gqa_prefill_workspace_bytes_for(int S, int L, int q_pos0) {
     const KeySplit ks = plan_split(S, L, q_pos0);
     return ks.tmax ? ks.bytes() : 0;
 }
-// An upper bound of the above over every launch with at most L keys (S <= L, q_pos0 = L - S or smaller): a part holds at least
-// total / CUs tiles, so there are at most CUs / 2 + 2 * blocks parts per KV head, a split launch has fewer than CUs / 2 blocks,
-// and a part of a 16-row block is half the size of one of a 32-row block.
-long qt_gqa_prefill_workspace_bytes(int L) {
-    if (L < 0) return -1;
-    const long cus = cu_count(), nb16 = std::min((long)(L + 15) / 16, cus / AKV), nb32 = std::min((long)(L + 31) / 32, cus / AKV);
-    const long b16 = (cus + AKV * (2 * nb16 + 2)) * part_bytes(16);
-    const long b32 = (cus + AKV * (2 * nb32 + 2)) * part_bytes(32);
-    return std::max(b16, b32);
-}
+// An upper bound of the above over every launch with at most L keys: a split launch has at most one part per CU, of 32 rows in single
+// precision at most.
+long qt_gqa_prefill_workspace_bytes(int L) { return L < 0 ? -1 : cu_count() * part_bytes(32, true); }
 
 // q, out [8 heads][S rows][256] bf16 with head stride q_head_stride and row stride q_row_stride (elements; head-major rows have row
 // stride 256, the token-major rows of a projection head stride 256 and row stride 2048, so neither has to be copied into the other),
@@ -844,23 +859,23 @@ int qt_gqa_prefill_causal_strided(const void* q, const void* K, const void* V, v
     }
     const int RB = 16 * ks.nh;
     const dim3 grid((ks.tmax ? (unsigned)ks.parts : (unsigned)((S + RB - 1) / RB)) * AKV);
-    _Float16* part_o = ks.tmax ? (_Float16*)workspace : nullptr;
-    float* part_ml = ks.tmax ? reinterpret_cast<float*>(part_o + (size_t)ks.parts * AKV * part_o_halves(RB)) : nullptr;
-    if (ks.nh == 2)
-        hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(512), 0, stream, (const bf16_t*)q, (const bf16_t*)K, (const bf16_t*)V,
+    auto launch = [&](auto nh, auto part_type) {
+        constexpr int NH = decltype(nh)::value;
+        using PT = decltype(part_type);
+        PT* part_o = ks.tmax ? (PT*)workspace : nullptr;
+        float* part_ml = ks.tmax ? reinterpret_cast<float*>(part_o + (size_t)ks.parts * AKV * part_o_size(RB)) : nullptr;
+        hipLaunchKernelGGL((attn_prefill_kernel<NH, PT>), grid, dim3(512), 0, stream, (const bf16_t*)q, (const bf16_t*)K, (const bf16_t*)V,
                            (bf16_t*)out, S, L, q_pos0, q_head_stride, q_row_stride, kv_head_stride, ks.tmax, part_o, part_ml);
-    else
-        hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, dim3(512), 0, stream, (const bf16_t*)q, (const bf16_t*)K, (const bf16_t*)V,
-                           (bf16_t*)out, S, L, q_pos0, q_head_stride, q_row_stride, kv_head_stride, ks.tmax, part_o, part_ml);
-    if (ks.tmax) {
-        const dim3 mgrid((unsigned)ks.split_blocks, AKV, (AH / AKV) * ks.nh);
-        if (ks.nh == 2)
-            hipLaunchKernelGGL(attn_prefill_merge_kernel<32>, mgrid, dim3(256), 0, stream, part_o, part_ml, (bf16_t*)out, S, q_pos0,
-                               ks.tmax, ks.parts, q_head_stride, q_row_stride);
-        else
-            hipLaunchKernelGGL(attn_prefill_merge_kernel<16>, mgrid, dim3(256), 0, stream, part_o, part_ml, (bf16_t*)out, S, q_pos0,
-                               ks.tmax, ks.parts, q_head_stride, q_row_stride);
-    }
+        if (ks.tmax)
+            hipLaunchKernelGGL((attn_prefill_merge_kernel<16 * NH, PT>), dim3((unsigned)ks.split_blocks, AKV, (AH / AKV) * NH), dim3(256), 0, stream,
+                               part_o, part_ml, (bf16_t*)out, S, q_pos0, ks.tmax, ks.parts, q_head_stride, q_row_stride);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    if (ks.nh == 2 && ks.wide) launch(Two{}, float{});
+    else if (ks.nh == 2) launch(Two{}, _Float16{});
+    else if (ks.wide) launch(One{}, float{});
+    else launch(One{}, _Float16{});
     QT_CHECK_LAUNCH();
     return QT_OK;
 }

@@ -136,6 +136,13 @@ def test_prefill_attention_split_plan_on_the_host():
         assert n > 0 and n % (2 * size) == 0, (S, P0, n)                  # whole parts, the same number for both KV heads
         assert n // size <= 256 + 1, (S, P0, n)                           # all parts resident at once (at most one per CU; 256 CUs assumed without a GPU)
         assert n <= bound(S + P0), (S, P0)
+    # half precision is for blocks that are cut into parts of six tiles and more: a launch of up to 704 keys, and 32-row blocks below 1472 rows,
+    # are not split or keep single precision
+    wide = [4 * (rows * 256 * 4 + 2 * rows * 4) for rows in (16, 32)]
+    for S, P0 in ((500, 0), (600, 0), (704, 0), (500, 100), (333, 299), (200, 300), (128, 300), (17, 600), (700, 6000), (1185, 1500), (1400, 6000)):
+        n = need(S, S + P0, P0)
+        assert n == 0 or any(n % (2 * w) == 0 for w in wide), (S, P0, n)
+        assert n <= bound(S + P0), (S, P0)
     # queries past the keys are refused before anything is launched
     assert lib.qt_gqa_prefill_causal(p16, p16, p16, p16, z, 0, 32, 40, 9, 32 * 256, 40 * 256, z) == -1
     assert lib.qt_gqa_prefill_causal(p16, p16, p16, p16, ctypes.c_void_p(8), 0, 32, 40, 8, 32 * 256, 40 * 256, z) == -2
