@@ -870,6 +870,23 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, const OneLds& L1, 
         for (int r = 0; r < 4; r++) R[ct][r] = __builtin_fmaf(-gm[r], ks[r], (float)L.Vs[(16 * ct + 4 * g + r) * VS_LD + 16 * sl + n]);
         Y[ct] *= L.gam[16 * ct + n];
     }
+    // R carries no beta, unlike everything that the chain packs: it may pass the half-precision range where D does not.  A column (a lane's
+    // n) is then multiplied by a power of two first, and its D divided by it.
+    float top = 0.f, back = 1.f;
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++) top = fmaxf(fmaxf(top, fmaxf(fabsf(R[ct][0]), fabsf(R[ct][1]))), fmaxf(fabsf(R[ct][2]), fabsf(R[ct][3])));
+    const bool far = __any(top > 32768.f);
+    if (far) {                                                       // (rare, and the same for the whole wavefront)
+        float a = top, b = top;
+        lanes32_swap(a, b);
+        a = b = fmaxf(a, b);
+        lanes16_swap(a, b);
+        const int e = (int)(__float_as_uint(fmaxf(a, b)) >> 23) - 141;           // the largest below 2^(15 + e)
+        const float down = e > 0 ? __uint_as_float((unsigned)(127 - e) << 23) : 1.f;
+        back = 1.f / down;
+#pragma unroll
+        for (int ct = 0; ct < NCT; ct++) R[ct] *= down;
+    }
     const half8 Rb[2] = {pack_half8(R[0], R[1]), pack_half8(R[2], R[3])};
     f32x4 D[NCT];
 #pragma unroll
@@ -879,6 +896,9 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, const OneLds& L1, 
         for (int kb2 = 0; kb2 < (ct < 2 ? 1 : 2); kb2++)             // (lower triangular)
             D[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const half8*>(&L1.Tb[(ct * 2 + kb2) * 512 + lane * 8]), Rb[kb2], D[ct], 0, 0, 0);
     }
+    if (far)
+#pragma unroll
+        for (int ct = 0; ct < NCT; ct++) D[ct] *= back;
     f32x4 Dd[NCT];
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++) Dd[ct] = D[ct] * *reinterpret_cast<const f32x4*>(&L1.dec[16 * ct + 4 * g]);

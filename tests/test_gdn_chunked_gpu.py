@@ -297,6 +297,25 @@ def test_one_launch_at_the_edge_of_the_half_precision_range_and_beyond(qt, dev, 
     test_status_word_reports_operands_beyond_half_precision(qt, dev, T)
 
 
+@pytest.mark.parametrize("T", [7, 64, 100])
+def test_values_far_from_what_the_state_predicts(qt, dev, T):
+    """v and k.S of opposite signs, each in the documented range, and a small write gate: v - k.S passes 65504 and beta (v - k.S), which is
+    all that the chunked form of longer prompts rounds, stays a thousandth of it"""
+    proj, cs, cw, A_log, dtb, gw, _ = proj_inputs(1100 + T, T)
+    proj[:, 2 * KD:CD] = bf(proj[:, 2 * KD:CD] * 6.0e3)
+    proj[:, CD + KD:CD + KD + HV] = -6.0                                      # b: beta about 0.002
+    proj[:, CD + KD + HV:] = -6.0                                             # a: hardly any decay
+    q, k, v = O.conv_prep(proj, cs, cw)
+    S0 = (-6.0e4 * np.repeat(k[0][:, None, :], 128, axis=1)).astype(np.float32)           # [head, dv, dk]: k_0 . S = -6e4
+    r0 = v[0] + 6.0e4 * O.gates(proj[0, CD + KD + HV:], proj[0, CD + KD:CD + KD + HV], A_log, dtb)[0][:, None]
+    assert np.abs(v).max() < 6.5e4 and np.abs(S0).max() < 6.5e4 and np.abs(r0).max() > 7.0e4
+    out, _, st = _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0)
+    qt.gdn_nax.check_status(dev, sync=True)
+    oo, oy, otail, os_ = O.prefill_gdn(proj, cs, cw, A_log, dtb, S0, gw)
+    check_rel("final state rel-L2", to_np(st)[0], os_, 2e-3, rel_l2)
+    check_rel("gated output rel-L2", to_np(out), oo, 2.0 ** -8, rel_l2)
+
+
 def test_give_up_path_ends_the_launch_and_leaves_the_flags_clean(qt, dev):
     """the bounded wait of the one-launch form, forced from the host with a poll limit of one: output workgroups give up on chunks
     the chain has not published yet, leave those rows unwritten and set bit 0 of the status word; every workgroup ends, the
