@@ -137,8 +137,8 @@ int qt_gqa_attn_layer_decode(const void* qkv, const void* q_norm, const void* k_
  * caller reads it after (or asynchronously behind) the launch and resets it:
  *   bit 0: an output workgroup of the one-launch form polled for its chunk longer than the poll limit (about a second) and
  *          gave up; its rows of y were NOT written.  It cannot happen while the chain workgroups run undisturbed.
- *   bit 1: the final state holds a value that is not finite: an operand left the half-precision range (above) and y is not
- *          to be trusted either.
+ *   bit 1: an operand left the half-precision range (above): the final state holds a value that is not finite, or only y does
+ *          (a head that decays fast forgets it); neither is to be trusted.
  * qt_gdn_phase_b_poll_limit(polls) sets the poll limit of later launches (0 = the default); it exists so that the give-up
  * path can be exercised from the host with a tiny limit.
  * qt_gdn_phase_b_norm is the same with prefill.gated_norm (qwen35/prefill.py:241-244) fused into the output kernel: it

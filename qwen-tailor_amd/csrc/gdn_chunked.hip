@@ -67,7 +67,8 @@ __device__ __forceinline__ half8 pack_half8(const f32x4& a, const f32x4& b) {
 // after its final progress store has been acknowledged), and the last one to do so clears the progress words, the done
 // count and the queue head: they are zero before and after every launch (the caller zeroes them once).  The status word
 // is never cleared by a launch: it is the caller's to read and reset.  Bit 1 of it is set by a chain workgroup whose final
-// state slice holds a value that is not finite: a half-precision operand (the state, D, U or a conv output) has overflowed.
+// state slice holds a value that is not finite, or which has met a D that half precision does not hold: a half-precision operand (the
+// state, D, U or a conv output) has overflowed.
 //
 // Chain role: 5 wavefronts per (head, 16-wide dv slice).  MFMA wavefront w owns rows 16w..16w+15 of D (the chunk's tokens) and
 // rows 32w..32w+31 of S^T (dk): per chunk it pulls only its 8 operand tiles (8 KiB) and keeps PB_DEP chunks of them in flight
@@ -88,6 +89,7 @@ constexpr int FLAG_STRIDE = 64;                  // ints between progress words:
 constexpr int FLAG_WORDS = (N_CHAIN + 1) * FLAG_STRIDE;   // flag area at the head of `snap` (33 KiB): progress [128] | done count, error
 constexpr int FLAG_DONE = N_CHAIN * FLAG_STRIDE, FLAG_ERR = FLAG_DONE + 1, FLAG_NEXT = FLAG_DONE + 2;   // FLAG_ERR: the status word; FLAG_NEXT: head of the item queue
 constexpr int ERR_GAVE_UP = 1, ERR_NOT_FINITE = 2;
+constexpr float HALF_END = 65520.f;              // from here on a value becomes infinite in half precision
 constexpr int FLAG_HALVES = FLAG_WORDS * 2;
 constexpr int SPIN_LIMIT = 1 << 21;              // polls (about a second) before a consumer gives up
 constexpr int MAX_OUT_WGS = 512;                 // output workgroups of the one-launch form: two for every CU (measured: 384 +2 us, 640 +4 us at 8192 tokens)
@@ -253,6 +255,7 @@ __device__ __forceinline__ void chain_role(ChainLds& L, int blk, const _Float16*
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
 
+    float top_d = 0.f;                       // largest |D| of all chunks: the outputs take D itself, the state only what is left after dec
     // One chain step on FIFO entry j (a compile-time index: the steps are unrolled PB_DEP at a time).  Every MFMA is
     // followed by the load that refills its operand for chunk c + PB_DEP and the scheduler is pinned to this order, so
     // loads complete in the order of their use and the waits name exact counts.
@@ -297,6 +300,7 @@ __device__ __forceinline__ void chain_role(ChainLds& L, int blk, const _Float16*
         reinterpret_cast<half4*>(L.dn_x)[((w >> 1) * 64 + lane) * 2 + (w & 1)] = dh;
         ST[0] *= gct[j];
         ST[1] *= gct[j];
+        top_d = fmaxf(fmaxf(top_d, fmaxf(fabsf(D[0]), fabsf(D[1]))), fmaxf(fabsf(D[2]), fabsf(D[3])));
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();                                           // E2
         asm volatile("" ::: "memory");
@@ -341,8 +345,9 @@ __device__ __forceinline__ void chain_role(ChainLds& L, int blk, const _Float16*
         float* sp = st_out + ((size_t)h * DV + sl * 16 + n) * DK + w * 32 + 4 * g;
         *reinterpret_cast<f32x4*>(sp) = ST[0];
         *reinterpret_cast<f32x4*>(sp + 16) = ST[1];
-        // an overflow of a half-precision operand anywhere in the chain (state, D, U, conv outputs) ends here as inf or NaN
-        bool bad = false;
+        // an overflow of a half-precision operand anywhere in the chain (state, U, conv outputs) ends here as inf or NaN; a D that
+        // overflows may be gone by then, where the head decays fast
+        bool bad = top_d >= HALF_END;
 #pragma unroll
         for (int i = 0; i < 4; i++) bad |= !(fabsf(ST[0][i]) <= 3.0e38f) | !(fabsf(ST[1][i]) <= 3.0e38f);
         if (__any(bad) && lane == 0) {
@@ -909,6 +914,10 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, const OneLds& L1, 
         for (int kb2 = 0; kb2 < (ct < 2 ? 1 : 2); kb2++)
             Y[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Dn[kb2], *reinterpret_cast<const half8*>(&L1.Am[(ct * 2 + kb2) * 512 + lane * 8]), Y[ct], 0, 0, 0);
     bool bad = false;
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad |= fabsf(D[ct][r]) >= HALF_END;
     float* so = o.st_out + ((size_t)h * DV + sl * 16 + n) * DK + 8 * g;
 #pragma unroll
     for (int i = 0; i < 8; i++) {                                    // row 4 g + r of tile i is row 32 (i / 2) + 8 g + 4 (i % 2) + r of the state
@@ -922,7 +931,7 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, const OneLds& L1, 
     }
     if (__any(bad) && lane == 0) {                                   // (as in the chain)
         atomicOr(o.status, ERR_NOT_FINITE);
-        if (o.host_words) o.host_words[1] = 1;
+        o.host_words[1] = 1;
     }
     __syncthreads();                                                 // Q has been read: its memory takes the outputs
 #pragma unroll

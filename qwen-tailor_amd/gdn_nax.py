@@ -41,7 +41,7 @@ def gdn_chunked(q, k, v, proj, A_log, dt_bias, state, relaxed=True, flags=DEFAUL
 
 _SNAP = {}            # (device index, stream handle) -> float16 tensor: flag area + chain snapshots
 _SNAP_RETIRED = []    # outgrown buffers stay alive: a captured HIP graph may hold their address
-_STATUS = {}          # (device index, stream handle) -> pinned int32[2]: set to 1 by a launch that gave up / whose state is not finite
+_STATUS = {}          # (device index, stream handle) -> pinned int32[2]: set to 1 by a launch that gave up / whose values are not finite
 
 GAVE_UP, NOT_FINITE = 1, 2        # bits of the status word
 
@@ -93,7 +93,7 @@ def _describe(v):
     if v & GAVE_UP:
         what.append("an output workgroup waited for its chunk for too long and gave up (its rows were not written)")
     if v & NOT_FINITE:
-        what.append("the final state is not finite: a half-precision operand overflowed (|state|, |v| or an intermediate above 65504)")
+        what.append("a value is not finite: a half-precision operand overflowed (|state|, |v| or an intermediate above 65504)")
     return "; ".join(what) or f"status {v}"
 
 

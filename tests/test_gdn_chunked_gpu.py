@@ -316,6 +316,26 @@ def test_values_far_from_what_the_state_predicts(qt, dev, T):
     check_rel("gated output rel-L2", to_np(out), oo, 2.0 ** -8, rel_l2)
 
 
+@pytest.mark.parametrize("T", [7, 64, 300, 4100])
+def test_status_word_reports_outputs_that_overflow_alone(qt, dev, T):
+    """a first token that writes beta (v - k.S) beyond 65504, which its output takes as a half-precision operand, into heads that then decay so
+    fast that nothing of it is left in the state: the outputs are not finite, the state is, and the launch is reported in every form"""
+    proj, cs, cw, A_log, dtb, gw, _ = proj_inputs(1200 + T, T)
+    proj[:, 2 * KD:CD] = bf(proj[:, 2 * KD:CD] * 6.0e3)
+    proj[0, CD + KD:CD + KD + HV] = 8.0                                       # b: beta about 1
+    proj[0, CD + KD + HV:], proj[1:, CD + KD + HV:] = -6.0, 20.0              # a: no decay, then exp(-20) and less a token
+    q, k, v = O.conv_prep(proj, cs, cw)
+    S0 = (-6.0e4 * np.repeat(k[0][:, None, :], 128, axis=1)).astype(np.float32)
+    d0 = v[0] + 6.0e4 * O.gates(proj[0, CD + KD + HV:], proj[0, CD + KD:CD + KD + HV], A_log, dtb)[0][:, None]
+    assert np.abs(v).max() < 6.5e4 and np.abs(S0).max() < 6.5e4 and np.abs(d0).max() > 7.0e4
+    out, _, st = _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0)
+    with pytest.raises(qt.gdn_nax.ChunkedPrefillError, match="not finite"):
+        qt.gdn_nax.check_status(dev, sync=True)
+    assert np.isfinite(to_np(st)).all() and not np.isfinite(to_np(out)).all()
+    _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0 * 1e-3)
+    qt.gdn_nax.check_status(dev, sync=True)
+
+
 def test_give_up_path_ends_the_launch_and_leaves_the_flags_clean(qt, dev):
     """the bounded wait of the one-launch form, forced from the host with a poll limit of one: output workgroups give up on chunks
     the chain has not published yet, leave those rows unwritten and set bit 0 of the status word; every workgroup ends, the
