@@ -41,6 +41,7 @@ __device__ __forceinline__ void load_raw_window(RawIn& r, const bf16_t* __restri
 }
 // (a value that is converted in the block that loads it is waited for there: what is read again behind this is converted behind it)
 __device__ __forceinline__ void pin(RawIn& r) { asm volatile("" : "+v"(r.w0), "+v"(r.w1), "+v"(r.w2), "+v"(r.x)); }
+__device__ __forceinline__ void drop(const RawIn& r) { asm volatile("" ::"v"(r.x), "v"(r.c.x), "v"(r.c.y)); }
 __device__ __forceinline__ float conv_raw(const RawIn& r) {
     return conv_silu(bf2f((bf16_t)r.w0), bf2f((bf16_t)r.w1), bf2f((bf16_t)r.w2), bf2f((bf16_t)r.x), r.c);
 }
@@ -50,10 +51,10 @@ __device__ __forceinline__ void store_window(bf16_t* __restrict__ cs_out, const 
     cs_out[2 * CD + ch] = (bf16_t)r.x;
 }
 // where a sequence's window and state lie; snapshot j of the state goes to st_out + j*st_stride and of the conv window to cs_out +
-// j*cs_stride (strides 0 = update in place).  ok = false: the row is skipped; its places are then others inside the pools, from which
-// is read but nothing is written
+// j*cs_stride (strides 0 = update in place).  ok = false: the row is skipped, and the places are none
 struct Place {
     bool ok;
+    int par;                            // which of two windows is read (looked up with the slot)
     const bf16_t* cs_in;
     bf16_t* cs_out;
     size_t cs_stride;
@@ -71,7 +72,7 @@ __device__ __forceinline__ float lane_value(float v, int i) { return __uint_as_f
 // Order of the loads: what depends on neither slot nor position first, while those two are looked up, then the window, then the state;
 // nothing is waited for before the state has been requested.  (Slot, position and the inputs one after the other, and the inputs
 // converted where they are loaded, the state's requests left about two memory latencies late.  Fused norm, us in a HIP graph at 1 / 8 / 16 /
-// 20 / 64 rows 4.7 / 5.8 / 7.6 / 9.2 / 24.6, now 4.4 / 5.4 / 7.2 / 8.9 / 24.4; verify of 16 x 4 17.9, now 17.5.)
+// 20 / 64 rows 4.7 / 5.8 / 7.6 / 9.2 / 24.6, now 4.4 / 5.4 / 7.2 / 8.9 / 24.4; verify of 16 x 4 17.9, now 17.3.)
 // WPH: four wavefronts share q, k, v and the gates; with more, q and k, v, and the gates have wavefronts of their own, and the state is in
 // more hands: a little faster while most CUs have nothing to do.
 template <int RS, int HPW = 1, bool NORM = false, int WPH = 4, class PlaceFn>
@@ -120,6 +121,14 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
     }
     __builtin_amdgcn_sched_barrier(0);
     const Place at = place();
+    // A skipped row costs its slot's lookup and these few loads (64 of them 2.7 us, 64 rows 21; with the state's loads and the conv 5.5).
+    if (__builtin_expect(!at.ok, 0)) {
+        // (they count as used on this way out as well: otherwise they would be moved below the branch, and wait for it)
+        drop(rq);
+        drop(rv);
+        asm volatile("" ::"v"(gx), "v"(nz), "v"(ngw), "s"(gA), "s"(gdt), "s"(at.par));
+        __builtin_amdgcn_endpgm();                               // (a return would join the way out of the whole step: two more branches for every row)
+    }
     if (is_qk) load_raw_window(rq, at.cs_in, proj, 0, ch_qk);
     if (WPH == 4 || has_v) load_raw_window(rv, at.cs_in, proj, 0, ch_v_ld);
     __builtin_amdgcn_sched_barrier(0);           // keep the small loads ahead of the state loads in issue order
@@ -165,7 +174,6 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
             beta = lane_value(sigmoid_bf16(gv), 2);
         }
         __syncthreads();
-        if (!at.ok) return;                                      // (before the first barrier the loads would be sunk below this branch, and wait for it)
         if (is_qk) {
             if (split == 0) store_window(cso, rq, ch_qk);
             const float ss = (float)(red[which * 2] + red[which * 2 + 1]);
@@ -246,9 +254,8 @@ __device__ __forceinline__ void split_id(int& b, int& h, int& split) {
 __device__ __forceinline__ Place decode_place(bf16_t* conv_pool, float* ssm_pool, int slot, int p, int n_slots) {
     const int par = p & 1;                                       // batch.py:49-52: read buffer pos&1, write the other
     const bool ok = (unsigned)slot < (unsigned)n_slots;
-    slot = ok ? slot : 0;
     float* st = ssm_pool + (size_t)slot * HV * DV * DK;
-    return {ok, conv_pool + (size_t)(slot * 2 + par) * 3 * CD, conv_pool + (size_t)(slot * 2 + (par ^ 1)) * 3 * CD, 0, st, st, 0};
+    return {ok, par, conv_pool + (size_t)(slot * 2 + par) * 3 * CD, conv_pool + (size_t)(slot * 2 + (par ^ 1)) * 3 * CD, 0, st, st, 0};
 }
 
 // batch.deltanet_b (qwen35/batch.py:128-135): one token per row, pools updated in place
@@ -291,13 +298,12 @@ __global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restric
                                                          int n_entries) {
     int b, h, split;
     split_id<RS>(b, h, split);
-    const int s_in = sslots[b], sl_in = sels[b], pr = pars[b];
+    const int ss = sslots[b], sl = sels[b], pr = pars[b];
     gdn_tokens<RS>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, [&] {
         const int par = pr & 1;
         const size_t hs = (size_t)HV * DV * DK;
-        const bool ok = (unsigned)s_in < (unsigned)n_entries && (unsigned)sl_in < (unsigned)M;
-        const int ss = ok ? s_in : 0, sl = ok ? sl_in : 0;
-        return Place{ok, conv_pool + ((size_t)(ss * 2 + par) * M + sl) * 3 * CD,
+        const bool ok = (unsigned)ss < (unsigned)n_entries && (unsigned)sl < (unsigned)M;
+        return Place{ok, par, conv_pool + ((size_t)(ss * 2 + par) * M + sl) * 3 * CD,
                      conv_pool + (size_t)(ss * 2 + (par ^ 1)) * M * 3 * CD, (size_t)3 * CD, ssm_pool + ((size_t)ss * M + sl) * hs,
                      ssm_pool + (size_t)ss * M * hs, hs};
     });
@@ -313,12 +319,11 @@ __global__ __launch_bounds__(256) void gdn_solo_kernel(const bf16_t* __restrict_
                                                        int n_snap) {
     int b, h, split;
     split_id<RS>(b, h, split);
-    const int sl_in = sel[0];
+    const int sl = sel[0];
     gdn_tokens<RS>(proj, cw, A_log, dt_bias, y, M, h, split, [&] {
         const size_t hs = (size_t)HV * DV * DK;
-        const bool ok = (unsigned)sl_in < (unsigned)n_snap;
-        const int sl = ok ? sl_in : 0;
-        return Place{ok, cs_snap + (size_t)sl * 3 * CD, cs_out, (size_t)3 * CD, st_snap + sl * hs, st_out, hs};
+        const bool ok = (unsigned)sl < (unsigned)n_snap;
+        return Place{ok, 0, cs_snap + (size_t)sl * 3 * CD, cs_out, (size_t)3 * CD, st_snap + sl * hs, st_out, hs};
     });
 }
 
