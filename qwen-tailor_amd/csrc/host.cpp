@@ -723,7 +723,7 @@ PyObject* phase_b_norm(PyObject* const* a) {
     return wrap({out, st_out});
 }
 
-// gdn_core(proj, conv_state, ssm_state, conv_w, A_log, dt_bias, gw, want_qkv): both phases with the gated norm
+// gdn_core(proj, conv_state, ssm_state, conv_w, A_log, dt_bias, gw): both phases with the gated norm
 PyObject* gdn_core(PyObject* const* a) {
     const Tensor& proj = dev(a[0], BF16, "proj", {ANY, PW});
     const int64_t S = proj.size(0);
@@ -732,14 +732,10 @@ PyObject* gdn_core(PyObject* const* a) {
     const Tensor& w = flat_conv_w(a[3]);
     const Tensor A = f32(a[4], "A_log", HV), dtb = f32(a[5], "dt_bias", HV), gw = f32(a[6], "gw", DV);
     const Tensor state = dev(a[2], F32, "state").reshape({1, HV, DV, DK});
-    Tensor qkv[3];
-    const bool want = truth(a[7]);
     const Snap s = snap_buffer(proj, S);
     const Tensor silu = silu_table(proj);
     Tensor conv_out, st_out, out;
     unlocked([&] {
-        if (want)
-            for (Tensor& t : qkv) t = empty({S, HV, DK}, BF16, proj);
         conv_out = empty({1, 3, CD}, BF16, proj), st_out = empty({1, HV, DV, DK}, F32, proj), out = empty({S, HV * DV}, BF16, proj);
         // a prompt of one chunk: one launch
         const int rc = qt_gdn_prefill_one(proj.data_ptr(), cs.data_ptr(), w.data_ptr(), silu.data_ptr(), A.data_ptr<float>(), dtb.data_ptr<float>(),
@@ -747,7 +743,7 @@ PyObject* gdn_core(PyObject* const* a) {
                                           gw.data_ptr<float>(), 1e-6f, out.data_ptr(), dim32(S), s.words.data_ptr<int>(), stream());
         if (rc != -4) return check(rc, "qt_gdn_prefill_one");
         const Records r = new_records(proj);
-        phase_a_conv(proj, cs, w, silu, A, dtb, want ? qkv : nullptr, conv_out.data_ptr(), r);
+        phase_a_conv(proj, cs, w, silu, A, dtb, nullptr, conv_out.data_ptr(), r);
         phase_b_launch(r, s, state, st_out, &proj, &gw, 1e-6f, out, S);
     });
     return wrap({out, conv_out, st_out});
@@ -945,7 +941,7 @@ PyMethodDef methods[] = {
     QT_FN("attn_b", attn_b, 10),          QT_FN("attn_layer_b", attn_layer_b, 11), QT_FN("sdpa", sdpa, 3),
     QT_FN("qkv_prep", qkv_prep, 7),       QT_FN("out_gate", out_gate, 2),         QT_FN("conv_prep", conv_prep, 3),
     QT_FN("phase_a", phase_a, 8),         QT_FN("phase_b", phase_b, 5),           QT_FN("phase_b_norm", phase_b_norm, 7),
-    QT_FN("gdn_core", gdn_core, 8),
+    QT_FN("gdn_core", gdn_core, 7),
     QT_FN("set_hooks", set_hooks, 3),     QT_FN("blit_batch", blit_batch, 2),     QT_FN("pools_load", pools_load, 12),
     QT_FN("cache_restore", cache_restore, 5),
     {nullptr, nullptr, 0, nullptr}};

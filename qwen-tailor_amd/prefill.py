@@ -22,9 +22,10 @@ GDN_IMPL = os.environ.get("QWEN35_GDN", "nax")
 def gdn_core(proj, conv_state, ssm_state, conv_w, A_log, dt_bias, gnorm, want_qkv=False):
     """The GatedDeltaNet layer core over S tokens, between the in_proj and out_proj GEMMs of prefill._linear_attn
     (qwen35/prefill.py:247-265): proj [S,8224] bf16, conv_state [1,3,6144] bf16, ssm_state [1,16,128,128] f32 ->
-    (gated-norm output [S,2048] bf16, new conv state [1,3,6144], new ssm state [1,16,128,128])."""
+    (gated-norm output [S,2048] bf16, new conv state [1,3,6144], new ssm state [1,16,128,128]).  want_qkv is accepted and changes
+    nothing: q, k and v are not among the results (gdn_nax.prep_a returns them)."""
     if GDN_IMPL == "nax":
-        return L.host.gdn_core(proj, conv_state, ssm_state, conv_w, A_log, dt_bias, gnorm, want_qkv)
+        return L.host.gdn_core(proj, conv_state, ssm_state, conv_w, A_log, dt_bias, gnorm)
     S = proj.shape[0]
     cs = conv_state.reshape(3, CD)
     q, k, v = conv_prep(proj, cs, conv_w)

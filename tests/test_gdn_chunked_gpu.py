@@ -297,6 +297,25 @@ def test_one_launch_at_the_edge_of_the_half_precision_range_and_beyond(qt, dev, 
     test_status_word_reports_operands_beyond_half_precision(qt, dev, T)
 
 
+@pytest.mark.parametrize("T", [40, 300])
+def test_want_qkv_changes_nothing(qt, dev, T):
+    """q, k and v are not among the results of the layer core, whatever is asked for: no memory is taken for them"""
+    proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(1300 + T, T)
+    args = [to_dev(proj, dev, BF16), to_dev(cs[None], dev, BF16), to_dev(S0[None], dev), to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev),
+            to_dev(gw, dev)]
+    taken = lambda: torch.cuda.memory_stats(dev)["allocation.all.allocated"]
+    qt.prefill.gdn_core(*args)
+    n = [taken()]
+    want = qt.prefill.gdn_core(*args)
+    n.append(taken())
+    got = qt.prefill.gdn_core(*args, want_qkv=True)
+    n.append(taken())
+    assert n[2] - n[1] == n[1] - n[0], n
+    assert len(got) == len(want) == 3
+    for a, b in zip(got, want):
+        check_tensors_equal("result", a, b)
+
+
 @pytest.mark.parametrize("T", [7, 64, 100])
 def test_values_far_from_what_the_state_predicts(qt, dev, T):
     """v and k.S of opposite signs, each in the documented range, and a small write gate: v - k.S passes 65504 and beta (v - k.S), which is
