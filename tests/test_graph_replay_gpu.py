@@ -76,7 +76,7 @@ def test_decode_step_and_layer_half_under_graph(qt, dev):
     _replays(dev, run, lambda: [out, ssm, conv], restore)
 
 
-@pytest.mark.parametrize("T", [300, 4100])
+@pytest.mark.parametrize("T", [1, 61, 300, 4100])
 def test_chunked_prefill_under_graph(qt, dev, T):
     """both launch forms of phase B; the one-launch form's flag area must be back to zero after every replay"""
     gen = torch.Generator().manual_seed(6 + T)
@@ -152,7 +152,7 @@ def _prefill_inputs(dev, T, seed):
             to_dev(dtb, dev), to_dev(gw, dev)]
 
 
-@pytest.mark.parametrize("T", [300, 4033, 4100])
+@pytest.mark.parametrize("T", [7, 64, 300, 4033, 4100])
 def test_a_replayed_prefill_reports_to_the_stream_it_is_replayed_on(qt, dev, T):
     """captured on a side stream that has seen no prefill, replayed on the current one: its failure (a state beyond the half-precision
     range) is found by check_status there, and the next replay, with a good state, has the eager bits (4033 tokens are the first

@@ -100,6 +100,28 @@ def test_restored_tensors_are_contiguous_and_disjoint(qt, dev):
         assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
 
 
+@pytest.mark.parametrize("inference", [False, True])
+def test_restored_tensors_are_tensors_of_their_own(qt, dev, inference):
+    """not views of their block: no base, a version counter each, no gradient, and inference tensors where they are made under that mode; a
+    change to one is seen in no other"""
+    cfg, st = make_state(qt, dev, 64, 5)
+    pc = qt.prefix_cache.PrefixCache(budget_mb=512)
+    node = pc.insert(None, np.arange(64, dtype=np.int32), 51, st)
+    with torch.inference_mode(inference):
+        got, _ = pc.restore(node, 64)
+        parts = [*(t for pair in got["kv"] for t in pair), *got["conv"], *got["ssm"]]
+        want = [t.clone() for t in parts]
+        assert all(t._base is None and not t._is_view() and not t.requires_grad and t.is_inference() == inference for t in parts)
+        if not inference:                                         # (inference tensors count no versions)
+            assert all(t._version == 0 for t in parts)
+        parts[0].add_(1)
+        if not inference:
+            assert [t._version for t in parts] == [1] + [0] * (len(parts) - 1)
+        check_tensors_equal("the changed tensor", parts[0], want[0] + 1)
+        for a, b in zip(parts[1:], want[1:]):
+            check_tensors_equal("another tensor", a, b)
+
+
 @pytest.mark.parametrize("bad", ["rows", "width", "dtype", "max_len", "none"])
 def test_restore_refuses_a_chain_that_does_not_fit(qt, dev, bad):
     """segments that do not add up to the checkpoint's rows, that differ in shape or type, a buffer shorter than the checkpoint: errors, and
