@@ -33,7 +33,9 @@ def deltanet_b_gnorm(proj, conv_pool, conv_w, A_log, dt_bias, ssm_pool, slots, p
 def split_size(Lmax: int, B: int = 16) -> int:
     """Smallest number of pool keys a split-K workgroup takes.  The kernel spreads the batch's key tiles evenly over one
     workgroup per CU whatever the mix of lengths; this lower bound only matters for small batches of short sequences (layer form, us,
-    with 32 / 64 / 128 keys: one of 300 10.4 / 12.0 / 14.0, 5 x 3 of 90 - 900 12.4 / 12.5 / 14.6, 16 of 100 - 1000 13.7 / 13.7 / 15.0)."""
+    with 32 / 64 / 128 keys: 5 x 3 of 90 - 900 12.4 / 12.5 / 14.6, 16 of 100 - 1000 13.7 / 13.7 / 15.0, one sequence of 300 9.3 / 9.6 / 10.3, of 1000
+    9.7 / 9.7 / 10.8, of 2000 10.9 / 10.2 / 13.4, of 4000 12.8 / 12.1 / 11.8, of 8000 13.6 / 13.5 / 14.3, of 16000 16.1 / 15.9 / 15.7, and with four rows 11.0 /
+    11.1 / 11.4, 11.4 / 11.2 / 12.3, 12.8 / 11.6 / 15.5, 15.1 / 14.1 / 13.2, 15.7 / 15.6 / 16.7, 18.3 / 18.2 / 18.1)."""
     return 32
 
 

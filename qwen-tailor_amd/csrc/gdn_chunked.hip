@@ -1387,7 +1387,7 @@ int qt_gdn_phase_a_conv(const void* proj, const void* conv_state, const void* co
 }
 
 // qt_gdn_phase_a_conv and qt_gdn_phase_b_report with the gated norm for a prompt of 1 .. 64 tokens, in one launch without records: snap is
-// used for its status word only.  -4 for more tokens (nothing launched).
+// used for its status word only.  -4 for other numbers of tokens and for a window written in place (nothing launched).
 int qt_gdn_prefill_one(const void* proj, const void* conv_state, const void* conv_w, const void* silu_table, const float* A_log,
                        const float* dt_bias, void* conv_out, void* snap, const float* state_in, float* state_out, const float* gw, float eps,
                        void* out, int S, int32_t* host_words, hipStream_t stream) {

@@ -10,10 +10,11 @@
 // The arithmetic, per 64-key tile and 16 rows of a head:
 //     S^T[keys x rows] = K_tile . Q^T     A = K rows from LDS, B = Q^T resident in registers (16x16x32 bf16 MFMA)
 //     online softmax in the accumulator layout: lane (row n, group g) holds keys 4g..4g+3 of each 16-key sub-tile
-//     O[rows x 256]   += P . V            A = two exponentiated S^T accumulators packed to bf16 (they ARE the A operand
-//                                         when a 32-key block is enumerated as 16 (j >> 2) + 4 g + (j & 3)),
-//                                         B = V through the transposing LDS load (4 consecutive keys of one column);
-//                                         the row sums are one more column block, P . 1
+//     O^T[256 x rows] += V^T . P^T        A = V^T through the transposing LDS load (4 consecutive keys of one column),
+//                                         B = two exponentiated S^T accumulators packed to bf16 (they ARE the B operand
+//                                         when a 32-key block is enumerated as 16 (j >> 2) + 4 g + (j & 3));
+//                                         the row sums are one more product, 1 . P^T: every element is the row's sum.
+//                                         A lane then holds one row, eight adjacent columns in two blocks: 16-byte stores
 // K / V tiles travel HBM -> LDS directly (global_load_lds_dwordx4: 64 lanes x 16 bytes land as one contiguous KiB, no
 // registers in between) into double-buffered tiles.  The LDS rows are unpadded (a direct load cannot pad); instead the
 // 16-byte chunks of row r are stored XOR-swizzled by r & 15 (the loading lane picks the matching global chunk), which keeps
@@ -156,7 +157,7 @@ __device__ __forceinline__ volatile __attribute__((address_space(3))) int* lds_w
 // two tiles of scores (64), the output side O (128).
 //     iteration t (after barrier X(t): K(t + 1) and V(t - 1) are in LDS):
 //         score wavefront:  softmax of tile t (its scores are in registers since iteration t - 1) and the score MFMAs of
-//                           tile t + 1; then P(t), as packed A operands, and the rows' rescale factors go to LDS
+//                           tile t + 1; then P(t), as packed B operands, and the rows' rescale factors go to LDS
 //         output wavefront: takes P(t - 1) and the factors from LDS, rescales O and the row sums if any row's reference
 //                           moved, O += P(t - 1) V(t - 1)
 //         all eight:        direct-to-LDS loads of K(t + 2) into K(t)'s buffer and of V(t) into V(t - 2)'s
@@ -482,7 +483,8 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         return;
     }
     // ---------------------------------------------------------------------------------------------- output wavefront
-    // O^T: block j of lane (n, g) holds row n of the pair's rows, columns col_of(j) .. + 3 (below); every element of Lsum is row n's sum
+    // O^T: lane (n, g) holds row n of the pair's rows, columns 32 jj + 8 g .. + 7 in blocks 2 jj and 2 jj + 1 (odd g: the halves change places);
+    // every element of Lsum is row n's sum
     f32x4 O[NH][16];
     f32x4 Lsum[NH];                                                  // row sums of P, accumulated by MFMA against a block of ones
 #pragma unroll
@@ -541,7 +543,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
             }
         }
         PHASE_FENCE();
-        {                                                            // the row sums: P . 1, the sum of exactly the rounded values
+        {                                                            // the row sums: 1 . P^T, the sum of exactly the rounded values
             s16x8 ones;
 #pragma unroll
             for (int e = 0; e < 8; e++) ones[e] = (short)0x3f80;

@@ -225,7 +225,8 @@ __device__ __forceinline__ void quad_transpose(u32x4& a, u32x4& b, u32x4& c, u32
 // address, and need no transpose; with a whole block of 16 more for two workgroups those two ended the launch 0.5 us late.
 // A workgroup's time at one row (in-kernel time stamps): rows in LDS after 1.9 us, W there after 3.0, product 0.65, the quarters' sum and
 // the store 0.6.  Hence the order: the rows' loads ahead of all W (0.2 us from 16 rows on), the row fragments read before W is waited
-// for and the partial sums beside the rows in LDS, without a barrier between (0.4 us; 16 rows only: beyond, registers and LDS are short).
+// for and the partial sums beside the rows in LDS, without a barrier between (0.4 us; 16 rows only: with more, the
+// fragments do not fit a wavefront's registers, and the sums take the rows' memory).
 // Tile sizes (us in a HIP graph, rms prologue included, N = 8224 / 7168 swiglu / 5120; before these: 6.2 / 5.7 / 5.0 at one row, 6.2 / 5.9 / 5.1
 // at 16, 7.1 / 6.7 / 5.9, 8.9 / 8.3 / 7.6, 10.4 / 9.6 / 7.6): 1 row 5.5 / 5.2 / 4.6, 16 rows 5.8 / 5.2 / 4.6, 32 rows 7.1 / 6.3 / 5.7, 64 rows 8.6 / 7.9 /
 // 7.3, 80 rows 10.1 / 9.5 / 7.4.  An empty kernel takes 1.8 us there, a bare read of the 16.8 MB 4.1; what is left at 64 rows is the 64 KiB of rows

@@ -355,21 +355,6 @@ __device__ __forceinline__ double groups_sum_d(double v) {
 }
 // total over the whole 64-lane wavefront (every lane gets it)
 __device__ __forceinline__ double wave_sum_d(double v) { return groups_sum_d(row16_sum_d(v)); }
-__device__ __forceinline__ float wave_sum(float v) {
-    v = row16_sum(v);
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-    v = fmaxf(v, dpp_mov<0xB1>(v));
-    v = fmaxf(v, dpp_mov<0x4E>(v));
-    v = fmaxf(v, dpp_mov<0x141>(v));
-    v = fmaxf(v, dpp_mov<0x140>(v));
-    v = fmaxf(v, __shfl_xor(v, 16, 64));
-    v = fmaxf(v, __shfl_xor(v, 32, 64));
-    return v;
-}
 
 // One value row of the gated delta rule, this lane's 8 of the 128 columns (kernels.py:518-530):
 //   kv = g (S_r . k);  delta = (v - kv) beta;  y = g (S_r . q) + delta (k . q);  S_r <- g S_r + delta k
