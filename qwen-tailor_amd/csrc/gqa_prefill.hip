@@ -766,9 +766,9 @@ struct SplitForm {
 };
 // Takes the form if its best part size is faster than `us`, the best so far.  parts(t) falls with t: the smallest resident part size is found
 // by bisection, and the few sizes from there on are priced (a launch of 20 us does not hide much of its host).
-void consider(const SplitForm& f, int S, int L, int q_pos0, KeySplit& best, float& us) {
-    const int RB = 16 * f.nh, nb = (S + RB - 1) / RB, cus = cu_count();
-    if (S < 1 || nb * AKV >= cus) return;
+void consider(const SplitForm& f, int cus, int S, int L, int q_pos0, KeySplit& best, float& us) {
+    const int RB = 16 * f.nh, nb = (S + RB - 1) / RB;
+    if (S < 1 || nb * AKV >= cus || f.base + f.tile * f.min_tiles >= us) return;
     const int most = (std::min(L, q_pos0 + S) + KT - 1) / KT - f.min_gain;       // (the last block's tiles, less the gain)
     const long p = (q_pos0 + RB - 1) / RB, cpt = KT / RB;
     auto parts = [&](int t) { return parts_upto(p + nb, cpt * t) - parts_upto(p, cpt * t); };
@@ -810,16 +810,17 @@ KeySplit plan_split(int S, int L, int q_pos0) {
         ks.nh = 2;
         return ks;
     }
+    const int cus = cu_count();
     if (S >= 1472 && (q_pos0 > 0 || S <= 3200)) {
         float any = 1e30f;
-        consider(SplitForm{2, 6, 4, false, 0.f, 1.f, 0.f, 0.f}, S, L, q_pos0, ks, any);        // (priced by its tiles alone)
+        consider(SplitForm{2, 6, 4, false, 0.f, 1.f, 0.f, 0.f}, cus, S, L, q_pos0, ks, any);        // (priced by its tiles alone)
         if (ks.tmax) return ks;
     }
     float us = 4.2f + 1.2f * ((std::min(L, q_pos0 + S) + KT - 1) / KT);         // no split
-    consider(SplitForm{1, 6, 6, false, 6.7f, 1.03f, 0.019f, 1.03f}, S, L, q_pos0, ks, us);
+    consider(SplitForm{1, 6, 6, false, 6.7f, 1.03f, 0.019f, 1.03f}, cus, S, L, q_pos0, ks, us);
     if (S < 1472) {
-        consider(SplitForm{1, 3, 1, true, 7.7f, 0.97f, 0.030f, 1.05f}, S, L, q_pos0, ks, us);
-        consider(SplitForm{2, 3, 1, true, 10.4f, 1.51f, 0.037f, 0.61f}, S, L, q_pos0, ks, us);
+        consider(SplitForm{1, 3, 1, true, 7.7f, 0.97f, 0.030f, 1.05f}, cus, S, L, q_pos0, ks, us);
+        consider(SplitForm{2, 3, 1, true, 10.4f, 1.51f, 0.037f, 0.61f}, cus, S, L, q_pos0, ks, us);
     }
     return ks;
 }
