@@ -816,7 +816,7 @@ struct Items {                                                   // the items of
     ~Items() { Py_DECREF(seq); }
     Py_ssize_t size() const { return PySequence_Fast_GET_SIZE(seq); }
     PyObject* operator[](Py_ssize_t i) const {
-        if (i >= size()) throw Error{PyExc_IndexError, "list index out of range"};
+        if (i < 0 || i >= size()) throw Error{PyExc_IndexError, "list index out of range"};
         return PySequence_Fast_GET_ITEM(seq, i);
     }
 };

@@ -46,6 +46,8 @@ def test_host_rejects_bad_arguments_without_a_gpu():
         qt.kernels.fused_gemv(x, x)
     with pytest.raises(TypeError):
         qt.batch.rms_rows(x, x[0])
+    with pytest.raises(IndexError):                # a chain of no checkpoints
+        qt._lib.host.cache_restore([], x, x, 0, 16)
 
 
 def test_null_and_dimension_errors_from_the_c_abi():
