@@ -121,7 +121,8 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
     }
     __builtin_amdgcn_sched_barrier(0);
     const Place at = place();
-    // A skipped row costs its slot's lookup and these few loads (64 of them 2.7 us, 64 rows 21; with the state's loads and the conv 5.5).
+    // A skipped row costs its slot's lookup and these few loads (us: 64 of them 2.3, with the state's loads and the conv 7.5, without a load 1.8; 32 rows
+    // and 32 skipped 16.6 / 17.9 / 17.1, 64 and 64 30.5 / 35.4 / 30.3).
     if (__builtin_expect(!at.ok, 0)) {
         // (they count as used on this way out as well: otherwise they would be moved below the branch, and wait for it)
         drop(rq);

@@ -483,11 +483,11 @@ def test_skipped_rows_between_others(qt, dev, B):
 
 
 def test_skipped_rows_cost_no_state(qt, dev):
-    """a batch padded with skipped rows pays for their slots' lookup, not for their state: 64 of them take an eighth of 64 rows' time
-    (2.7 of 21 us; a quarter to a third if they read a state and run the conv)"""
+    """a batch padded with skipped rows pays for their slots' lookup, not for their state: 256 of them take 4.4 us where 256
+    rows take 97 (13 if they read a state and run the conv); the bound lies between the two, at the same factor from both"""
     gen = torch.Generator().manual_seed(77)
     cw, A_log, dtb, gw = layer_params(77)
-    B = 64
+    B = 256                                                       # (many rows: the launch itself hardly counts)
     args = [to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev)]
     proj, dgw = to_dev(rand_bf(gen, (B, PW), 1.0), dev, BF16), to_dev(gw, dev)
     ssm, conv = torch.zeros((B + 1, 16, 128, 128), device=dev), torch.zeros(((B + 1) * 2, 3, CD), dtype=BF16, device=dev)
@@ -513,7 +513,7 @@ def test_skipped_rows_cost_no_state(qt, dev):
         return min(times)
 
     real, skipped = time_of(torch.arange(B, dtype=torch.int32, device=dev)), time_of(torch.full((B,), -1, dtype=torch.int32, device=dev))
-    assert skipped < 0.19 * real, (skipped, real)
+    assert skipped < 0.08 * real, (skipped, real)
 
 
 def test_a_missing_norm_weight_is_refused(qt, dev):
