@@ -648,7 +648,9 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         }
         return;
     }
-    if (!row_ok) return;
+    // Sixteen-row blocks compute the rows past the end too and leave out their stores alone: with the lanes of one or two rows these instructions
+    // took 1.2 us instead of 0.4 (time stamps).
+    if (NH == 2 && !row_ok) return;
 #pragma unroll
     for (int hh = 0; hh < NH; hh++) {
         const float inv = 1.0f / Lsum[hh][0];
@@ -657,7 +659,9 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(const bf16_t* __restr
         for (int jj = 0; jj < 8; jj++) {
             f32x4 lo, hi;
             columns(O[hh], jj, inv, lo, hi);
-            *reinterpret_cast<u32x4*>(dst + 32 * jj) = u32x4{pack2_bf(lo[0], lo[1]), pack2_bf(lo[2], lo[3]), pack2_bf(hi[0], hi[1]), pack2_bf(hi[2], hi[3])};
+            u32x4 pk = u32x4{pack2_bf(lo[0], lo[1]), pack2_bf(lo[2], lo[3]), pack2_bf(hi[0], hi[1]), pack2_bf(hi[2], hi[3])};
+            if (NH == 1) asm volatile("" : "+v"(pk));            // (otherwise formed below the branch)
+            if (NH == 2 || row_ok) *reinterpret_cast<u32x4*>(dst + 32 * jj) = pk;
         }
     }
 }

@@ -393,6 +393,15 @@ def test_prefill_causal_split_range_of_v(qt, dev, S, P0, qscale, k):
     assert bool(((got - want).abs() <= bound).all()), "a value that is not finite has left its column"
 
 
+def test_prefill_of_one_row_costs_no_more_than_of_sixteen(qt, dev):
+    """a row block with one row: its outputs are formed by whole wavefronts (5.4 us, sixteen rows 6.0; by the lanes of that row alone 6.3)"""
+    def time_of(S):
+        q, K, V = (torch.randn(shape, device=dev).bfloat16()[None] for shape in ((8, S, 256), (2, S, 256), (2, S, 256)))
+        return graph_us(lambda: qt.attention.scaled_dot_product_attention(q, K, V, scale=256 ** -0.5, mask="causal"))
+    one, sixteen = time_of(1), time_of(16)
+    assert one < 0.97 * sixteen, (one, sixteen)
+
+
 @pytest.mark.parametrize("S,P0", [(1024, 0), (2048, 0), (300, 3000), (5000, 0)])
 def test_prefill_causal_head_strides(qt, dev, S, P0):
     """q / out with a head stride beyond S rows and K / V inside a longer cache, through the C ABI, in every form of the launch

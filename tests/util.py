@@ -98,3 +98,23 @@ def check_tensors_equal(name, a, b):
     n = int((a != b).sum().item())
     if n:
         raise AssertionError(f"{name}: {n} of {a.numel()} elements differ")
+
+
+def graph_us(run, calls=50, replays=5):
+    """time of a call on the GPU, us: the fastest of a few replays of a HIP graph of `calls` of them"""
+    side, g, times = torch.cuda.Stream(), torch.cuda.CUDAGraph(), []
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+        side.synchronize()
+        with torch.cuda.graph(g, stream=side):
+            for _ in range(calls):
+                run()
+        for _ in range(replays):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record(side)
+            g.replay()
+            b.record(side)
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 1e3 / calls)
+    return min(times)
