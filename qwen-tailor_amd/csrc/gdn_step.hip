@@ -29,9 +29,11 @@ __device__ __forceinline__ unsigned inp(const bf16_t* __restrict__ cs_in, const 
     return t < 0 ? cs_in[(t + 3) * CD + ch] : proj[(size_t)t * PW + ch];
 }
 // what does not depend on the sequence's slot ...
+__device__ __forceinline__ void load_taps(RawIn& r, const bf16_t* __restrict__ cw, int ch) { r.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch * 4); }
+template <bool TAPS = true>
 __device__ __forceinline__ void load_raw_proj(RawIn& r, const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cw, int j, int ch) {
     r.x = proj[(size_t)j * PW + ch];
-    r.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch * 4);
+    if (TAPS) load_taps(r, cw, ch);
 }
 // ... and what does
 __device__ __forceinline__ void load_raw_window(RawIn& r, const bf16_t* __restrict__ cs_in, const bf16_t* __restrict__ proj, int j, int ch) {
@@ -73,9 +75,10 @@ __device__ __forceinline__ float lane_value(float v, int i) { return __uint_as_f
 // nothing is waited for before the state has been requested.  (Slot, position and the inputs one after the other, and the inputs
 // converted where they are loaded, the state's requests left about two memory latencies late.  Fused norm, us in a HIP graph at 1 / 8 / 16 /
 // 20 / 64 rows 4.7 / 5.8 / 7.6 / 9.2 / 24.6, now 4.4 / 5.4 / 7.2 / 8.9 / 24.4; verify of 16 x 4 17.9, now 17.3.)
+// TAPS_LATE: the taps behind the state, which the conv then waits for (the rule is at the launch of the verify step).
 // WPH: four wavefronts share q, k, v and the gates; with more, q and k, v, and the gates have wavefronts of their own, and the state is in
 // more hands: a little faster while most CUs have nothing to do.
-template <int RS, int HPW = 1, bool NORM = false, int WPH = 4, class PlaceFn>
+template <int RS, int HPW = 1, bool NORM = false, int WPH = 4, bool TAPS_LATE = false, class PlaceFn>
 __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
                                            const float* __restrict__ dt_bias, bf16_t* __restrict__ y, int M, int h, int split,
                                            PlaceFn place, const float* __restrict__ gw = nullptr, float eps = 0.f) {
@@ -104,8 +107,8 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
     const int ch_v_ld = has_v ? ch_v : ch_qk;                    // (four wavefronts: every load is unconditional)
 
     RawIn rq = {0, 0, 0, 0, {0, 0}}, rv = {0, 0, 0, 0, {0, 0}};
-    if (is_qk) load_raw_proj(rq, proj, cw, 0, ch_qk);
-    if (WPH == 4 || has_v) load_raw_proj(rv, proj, cw, 0, ch_v_ld);
+    if (is_qk) load_raw_proj<!TAPS_LATE>(rq, proj, cw, 0, ch_qk);
+    if (WPH == 4 || has_v) load_raw_proj<!TAPS_LATE>(rv, proj, cw, 0, ch_v_ld);
     // gates: lane 1 the decay gate (reads a), lane 2 beta (reads b)
     const int g_at = CD + KD + HV * (lane == 1 ? 1 : 0) + h;
     unsigned gx = 0;
@@ -145,6 +148,7 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
         }
     }
     __builtin_amdgcn_sched_barrier(0);
+    if (TAPS_LATE) load_taps(rq, cw, ch_qk), load_taps(rv, cw, ch_v_ld);
     pin(rq);
     pin(rv);
     asm volatile("" : "+v"(gx), "+v"(nz));
@@ -290,7 +294,7 @@ __global__ __launch_bounds__(64 * WPH * HPW) void gdn_decode_wide_kernel(const b
 }
 
 // batch_spec.deltanet_bm (qwen35/batch_spec.py:142-150): M chained tokens per sequence, snapshot pools in place
-template <int RS>
+template <int RS, bool TAPS_LATE = false>
 __global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
                                                          const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
                                                          const float* __restrict__ dt_bias, float* ssm_pool,
@@ -300,7 +304,7 @@ __global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restric
     int b, h, split;
     split_id<RS>(b, h, split);
     const int ss = sslots[b], sl = sels[b], pr = pars[b];
-    gdn_tokens<RS>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, [&] {
+    gdn_tokens<RS, 1, false, 4, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, [&] {
         const int par = pr & 1;
         const size_t hs = (size_t)HV * DV * DK;
         const bool ok = (unsigned)ss < (unsigned)n_entries && (unsigned)sl < (unsigned)M;
@@ -424,8 +428,21 @@ int qt_gdn_verify_step(const void* proj, void* conv_pool, const void* conv_w, co
     if (B == 0) return QT_OK;
     if (!aligned16(ssm_pool) || (reinterpret_cast<uintptr_t>(conv_w) & 7u)) return QT_ERR_ALIGN;
     const int rs = pick_rs(B, rows_per_wg);
-    QT_DISPATCH_RS(rs, gdn_verify_kernel, B, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log,
-                   dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
+    // More than a head per CU, in workgroups of half a head or more: the taps behind the state, so that a workgroup waits for its whole state before
+    // it computes and stores: fewer stores of one between the loads of another (us, taps late / ahead: 24 x 4 23.9 / 25.1, 18 x 4 19.6 / 20.8, 32 x
+    // 2 17.9 / 18.7).  With less the conv beside the state's loads wins (8 x 4 11.4 / 10.4, 12 x 4 14.1 / 13.9, 16 x 8 33.0 / 31.2).
+    if (rs >= 4 && (long)B * HV > cu_count()) {
+        const dim3 grid(B * HV * (8 / rs));
+        if (rs == 8)
+            hipLaunchKernelGGL((gdn_verify_kernel<8, true>), grid, dim3(256), 0, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w,
+                               A_log, dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
+        else
+            hipLaunchKernelGGL((gdn_verify_kernel<4, true>), grid, dim3(256), 0, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w,
+                               A_log, dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
+    } else {
+        QT_DISPATCH_RS(rs, gdn_verify_kernel, B, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log,
+                       dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
+    }
     QT_CHECK_LAUNCH();
     return QT_OK;
 }

@@ -493,27 +493,33 @@ def test_skipped_rows_cost_no_state(qt, dev):
     ssm, conv = torch.zeros((B + 1, 16, 128, 128), device=dev), torch.zeros(((B + 1) * 2, 3, CD), dtype=BF16, device=dev)
     pos = torch.zeros(B, dtype=torch.int32, device=dev)
 
-    def time_of(slots):
-        run = lambda: qt.batch.deltanet_b_gnorm(proj, conv, *args, ssm, slots, pos, dgw)
-        side, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
-        times = []
-        with torch.cuda.stream(side):
-            run()
-            side.synchronize()
-            with torch.cuda.graph(g, stream=side):
-                for _ in range(50):
-                    run()
-            for _ in range(5):
-                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                a.record(side)
-                g.replay()
-                b.record(side)
-                b.synchronize()
-                times.append(a.elapsed_time(b))
-        return min(times)
-
+    time_of = lambda slots: graph_us(lambda: qt.batch.deltanet_b_gnorm(proj, conv, *args, ssm, slots, pos, dgw))
     real, skipped = time_of(torch.arange(B, dtype=torch.int32, device=dev)), time_of(torch.full((B,), -1, dtype=torch.int32, device=dev))
     assert skipped < 0.08 * real, (skipped, real)
+
+
+@pytest.mark.parametrize("B,M,rows", [(16, 2, 64), (17, 1, 0), (24, 4, 0), (33, 2, 0), (17, 3, 128)])
+def test_verify_with_more_than_a_head_per_cu(qt, dev, B, M, rows):
+    """the form that asks for the conv's taps behind the state (more than 16 sequences, half a head or more per workgroup) gives the bits of the
+    other one, skipped rows among the rows"""
+    gen = torch.Generator().manual_seed(500 + B + M)
+    cw, A_log, dtb, gw = layer_params(50 + B)
+    args = [to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev)]
+    proj = to_dev(rand_bf(gen, (B * M, PW), 1.5), dev, BF16)
+    ssm = to_dev((torch.randn((B + 1, M, 16, 128, 128), generator=gen) * 0.1).numpy(), dev)
+    conv = to_dev(rand_bf(gen, ((B + 1) * 2, M, 3, CD)), dev, BF16)
+    slots = torch.randperm(B, generator=gen).to(torch.int32)
+    slots[B // 2], slots[B - 1] = -1, B + 1
+    ints = lambda hi: torch.randint(0, hi, (B,), generator=gen).to(torch.int32).to(dev)
+    slots, sels, pars = slots.to(dev), ints(M), ints(2)
+    taken = [b for b in range(B) if b not in (B // 2, B - 1)]
+    got, want = [], []
+    for r, res in ((rows, got), (32, want)):
+        c, s = conv.clone(), ssm.clone()
+        y = qt.batch_spec.deltanet_bm(proj, c, args[0], *args[1:], s, slots, sels, pars, M, r)
+        res += [y.reshape(B, M, -1)[taken], c, s]
+    for name, a, b in zip(("y", "conv pool", "ssm pool"), got, want):
+        check_tensors_equal(name, a, b)
 
 
 def test_a_missing_norm_weight_is_refused(qt, dev):
