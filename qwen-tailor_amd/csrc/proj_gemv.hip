@@ -386,11 +386,14 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
 // (row n >> 2, k slice n & 3), and of the 16 x 16 results those whose k slices agree are partial sums: element i of lane (n, g)
 // belongs to feature g and row n >> 2 if i = n & 3.  Three of four MFMA results are thrown away; the matrix cores have nothing
 // else to do here (8 x 8 tile, K = 3584: 28 steps x 4 MFMAs per CU).
+// ONE: K of up to 128 NWV KS, a single trip for every wavefront (one past the end loads the last step and multiplies nothing): the residual behind the
+// operands, as with PEEL (4 rows, K = 1024, N = 1024 / 2048 / 3072
+// 2.8 / 3.0 / 3.6 us; in a loop and with the residual ahead of the operands 3.25 / 3.75 / 4.05).
 // PEEL: the first trip is taken out of the loop (by the residual's load, which only that trip makes): 0.2 - 0.6 us less, for a tenth more
 // registers, which costs where several workgroups share a CU (80 rows 7.2 / 10.8 us against 6.4 / 10.3).
 // Measured in a HIP graph with the residual epilogue, K = 2048 / 3584 (before: residual loaded behind the last barrier, no trip peeled): 1 row
 // 3.0 / 3.5 us (3.3 / 3.8), 16 rows 3.4 / 4.4 (3.7 / 4.8), 32 rows 3.8 / 5.2 (4.2 / 5.6), 64 rows 5.2 / 6.2 (5.4 / 6.9).
-template <int NWV, int KS, int FG, int MG, int EPI, bool PEEL>
+template <int NWV, int KS, int FG, int MG, int EPI, bool PEEL, bool ONE>
 __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
                                                              const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N, int K,
                                                              int groups) {
@@ -410,13 +413,13 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
     const bool e_mine = er < R && m0 + er < M && n0 + ef < N;
     const size_t eo = (size_t)(m0 + er) * N + n0 + ef;
     unsigned res_raw = 0;
-    if (EPI == EPI_ADD && !PEEL && e_mine) res_raw = res[eo];
+    if (EPI == EPI_ADD && !PEEL && !ONE && e_mine) res_raw = res[eo];
     f32x4 acc[FG][MG];
 #pragma unroll
     for (int f = 0; f < FG; f++)
 #pragma unroll
         for (int m = 0; m < MG; m++) acc[f][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int base = w; base < steps; base += NWV * KS) {
+    for (int base = w; ONE ? base == w : base < steps; base += NWV * KS) {
         u32x4 a[KS][FG], b[KS][MG];
 #pragma unroll
         for (int c = 0; c < KS; c++) {
@@ -427,7 +430,7 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
             for (int m = 0; m < MG; m++) b[c][m] = *reinterpret_cast<const u32x4*>(xp[m] + k0);
         }
         // (what only the first trip does makes the compiler take that trip out of the loop)
-        if (EPI == EPI_ADD && PEEL && base == w && e_mine) res_raw = res[eo];
+        if (EPI == EPI_ADD && (PEEL || ONE) && base == w && e_mine) res_raw = res[eo];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c = 0; c < KS; c++)
@@ -566,22 +569,22 @@ bool launch_rows_any(const gemv_args& p, int cus) {
     return false;
 }
 
-template <int NWV, int KS, int FG, int MG, bool PEEL>
+template <int NWV, int KS, int FG, int MG, bool PEEL, bool ONE = false>
 void launch_quad_tile(const gemv_args& p) {
     const int groups = (p.M + 4 * MG - 1) / (4 * MG), tiles = (p.N + 4 * FG - 1) / (4 * FG);
     const dim3 grid((tiles + 7) / 8 * 8 * groups), block(64 * NWV);
     if (p.epi == EPI_NONE)
-        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_NONE, PEEL>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_NONE, PEEL, ONE>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
     else if (p.epi == EPI_ADD)
-        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_ADD, PEEL>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_ADD, PEEL, ONE>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
     else
-        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_SWIGLU, PEEL>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL((quad_gemm_kernel<NWV, KS, FG, MG, EPI_SWIGLU, PEEL, ONE>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
 }
 // wavefronts and steps at a time by K: all of K in flight at once up to 4096.  PEEL_: the first trip taken out of the loop
 template <int FG, int MG, bool PEEL_ = true>
 void launch_quad(const gemv_args& p) {
     if (p.K <= 1024)
-        launch_quad_tile<4, 2, FG, MG, false>(p);
+        launch_quad_tile<4, 2, FG, MG, false, true>(p);
     else if (p.K <= 2048)
         launch_quad_tile<8, 2, FG, MG, PEEL_>(p);
     else
