@@ -184,11 +184,12 @@ def test_narrow_projection_of_one_trip(qt, dev, M, N, K):
 
 
 def test_the_residual_costs_a_narrow_projection_nothing(qt, dev):
-    """it is requested behind the operands: 0.99 - 1.01 of the time without it (1.18 - 1.23 when it stood ahead of them; the bound lies between)"""
+    """it is requested behind the operands: 0.987 - 0.998 of the time without it (1.057 - 1.074 when it stood ahead of them; the bound
+    lies between)"""
     g = torch.Generator().manual_seed(5)
     W, x, res = (to_dev(rand_bf(g, s, 0.03), dev, BF16) for s in ((2048, 768), (4, 768), (4, 2048)))
     without, with_res = graph_us(lambda: qt.kernels.fused_gemv(W, x)), graph_us(lambda: qt.kernels.fused_gemv(W, x, res=res))
-    assert with_res < 1.09 * without, (with_res, without)
+    assert with_res < 1.03 * without, (with_res, without)
 
 
 def test_fused_gemv_prologues_and_leading_dims(qt, dev):

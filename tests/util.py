@@ -100,8 +100,8 @@ def check_tensors_equal(name, a, b):
         raise AssertionError(f"{name}: {n} of {a.numel()} elements differ")
 
 
-def graph_us(run, calls=50, replays=5):
-    """time of a call on the GPU, us: the fastest of a few replays of a HIP graph of `calls` of them"""
+def graph_us(run, calls=50, replays=60):
+    """time of a call on the GPU, us: the fastest of many replays of a HIP graph of `calls` of them (the first ones meet a slow clock)"""
     side, g, times = torch.cuda.Stream(), torch.cuda.CUDAGraph(), []
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
