@@ -192,27 +192,27 @@ __device__ __forceinline__ void rows_inv(const double (&ss)[NR], float eps, int 
 }
 
 // 4 x 4 transpose of 16-byte items between four registers and the four lanes of a quad: 48 vector instructions
-__device__ __forceinline__ void quad_transpose(u32x4& a, u32x4& b, u32x4& c, u32x4& d, bool odd, bool high) {
+__device__ __forceinline__ void quad_transpose(u32x4 (&v)[4], bool odd, bool high) {
     auto swz = [](unsigned v, auto ctrl) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl.value, 0xF, 0xF, true); };
     constexpr std::integral_constant<int, 0xB1> by1{};            // quad_perm [1,0,3,2]
     constexpr std::integral_constant<int, 0x4E> by2{};            // quad_perm [2,3,0,1]
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        unsigned x0 = a[i], x1 = b[i], x2 = c[i], x3 = d[i];
+        unsigned x0 = v[0][i], x1 = v[1][i], x2 = v[2][i], x3 = v[3][i];
         unsigned t = swz(odd ? x0 : x1, by1), u = swz(odd ? x2 : x3, by1);
         x0 = odd ? t : x0, x1 = odd ? x1 : t, x2 = odd ? u : x2, x3 = odd ? x3 : u;
         t = swz(high ? x0 : x2, by2), u = swz(high ? x1 : x3, by2);
-        a[i] = high ? t : x0, c[i] = high ? x2 : t, b[i] = high ? u : x1, d[i] = high ? x3 : u;
+        v[0][i] = high ? t : x0, v[2][i] = high ? x2 : t, v[1][i] = high ? u : x1, v[3][i] = high ? x3 : u;
     }
 }
 
 // K = 1024, wide outputs.  A workgroup of eight wavefronts owns NB = 2 FB blocks of 16 features and 16 RB rows; wavefront (half,
 // q) multiplies FB of the blocks over the quarter q of K (two of the eight 128-wide steps of a row), and the quarters meet in
 // LDS in a fixed order.
-// Rows: every wavefront brings in 2 RB of them, a row per two loads of 1 KiB, asks for its W right after, and applies the rms
-// prologue (RMS) while W is on its way from HBM; the rows then go to LDS, their 16-byte chunks XOR-swizzled by the row number
+// Rows: every wavefront brings in 2 RB of them, a row per two loads of 1 KiB, asks for the W of its first block right after, and applies the
+// rms prologue (RMS) while that is on its way from HBM; the rows then go to LDS, their 16-byte chunks XOR-swizzled by the row number
 // so that the fragment reads of 16 rows fall on distinct banks.  Every workgroup normalises its rows itself: 0.1 us (16 rows)
-// to 1.2 us (32 rows x 64 features) instead of a launch of its own at 2.6 us.
+// to 0.7 us (32 rows x 64 features) instead of a launch of its own at 2.6 us.
 // W: a load takes 256 contiguous bytes of four features, 64 of them in each quad of lanes (register j of lane (g, h, c): feature
 // 4 h + j, elements 32 g + 8 c ..), and quad_transpose turns four such loads into the MFMA layout: feature n in lane (n, g),
 // elements 32 g + 8 r .. in register r.  The x fragments are read from LDS in the same enumeration of k.  Which wavefront takes
@@ -223,22 +223,30 @@ __device__ __forceinline__ void quad_transpose(u32x4& a, u32x4& b, u32x4& c, u32
 // N need not divide: with `extra` > 0 the first `extra` tiles take four features more each, from the end of N (N = 8224 is 256 tiles of 32
 // and eight times four; a 257th workgroup would take a CU twice as long as the others).  They come in MFMA layout, four lanes to an
 // address, and need no transpose; with a whole block of 16 more for two workgroups those two ended the launch 0.5 us late.
-// A workgroup's time at one row (in-kernel time stamps): rows in LDS after 1.9 us, W there after 3.0, product 0.65, the quarters' sum and
-// the store 0.6.  Hence the order: the rows' loads ahead of all W (0.2 us from 16 rows on), the row fragments read before W is waited
-// for and the partial sums beside the rows in LDS, without a barrier between (0.4 us; 16 rows only: with more, the
-// fragments do not fit a wavefront's registers, and the sums take the rows' memory).
-// Tile sizes (us in a HIP graph, rms prologue included, N = 8224 / 7168 swiglu / 5120; before these: 6.2 / 5.7 / 5.0 at one row, 6.2 / 5.9 / 5.1
-// at 16, 7.1 / 6.7 / 5.9, 8.9 / 8.3 / 7.6, 10.4 / 9.6 / 7.6): 1 row 5.5 / 5.2 / 4.6, 16 rows 5.8 / 5.2 / 4.6, 32 rows 7.1 / 6.3 / 5.7, 64 rows 8.6 / 7.9 /
-// 7.3, 80 rows 10.1 / 9.5 / 7.4.  An empty kernel takes 1.8 us there, a bare read of the 16.8 MB 4.1; what is left at 64 rows is the 64 KiB of rows
-// and 128 KiB of W a CU pulls and the vector instructions of the prologue and the transposes.
-template <int RB, int FB, bool RMS, int EPI>
+// A workgroup's time (in-kernel time stamps).  At one row: rows in LDS after 1.9 us, W there after 3.0, product 0.65, the quarters' sum and
+// the store 0.6.  With 32 rows x 64 features: a CU takes a load of 1 KiB every 16 clocks and a wavefront waits at a load that is not taken yet, so
+// that 26 loads a wavefront ahead of the prologue held it up for 2.1 - 2.9 us, with the rows long there.  Hence the order: the rows' loads
+// ahead of all W (0.2 us from 16 rows on); of W what 8 loads a wavefront bring before the prologue, and the second block's behind the rows'
+// barrier (0.7 us at 64 rows; 4 or 6 loads ahead 0.2 - 0.4 more, all ahead as before; interleaved with the prologue 0.1 - 0.5 more); the row
+// fragments read before W is waited for and each block multiplied as it comes (0.3 us at 32 - 48 rows); the partial sums beside the rows in
+// LDS, without a barrier between (0.4 us).
+// Transposing through LDS (4 KiB a wavefront, 8 accesses instead of 64 vector instructions) takes as long: what follows the arrival
+// of W is serial either way.
+// Tile sizes (us in a HIP graph, rms prologue included, N = 8224 / 7168 swiglu / 5120; in brackets the build before this order): 1 row 5.4 / 5.15 /
+// 4.5 (5.45 / 5.2 / 4.6), 16 rows 5.45 / 5.1 / 4.5 (5.5 / 5.2 / 4.6), 32 rows 6.1 / 5.95 / 5.4 (6.6 / 6.2 / 5.7), 48 and 64 rows 7.1 / 6.7 / 6.2 (8.0 - 8.2 / 7.4 - 7.9 / 7.0 -
+// 7.4), 80 rows 8.2 / 8.0 / 6.2 (9.8 / 9.4 / 7.4).  An empty kernel takes 1.8 us there; one that only loads takes 4.05 for the 16.8 MB, 5.2
+// with the loads of 32 rows x 64 features: what is left is the prologue and what follows the last of W.
+template <int RB, int FB, bool RMS, int EPI, bool ALONE>
 __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
                                                                          const bf16_t* __restrict__ nw, float eps,
                                                                          const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N,
                                                                          int tiles, int extra) {
     constexpr int NB = 2 * FB, R = 16 * RB, RW = R / 8;
-    __shared__ __align__(1024) bf16_t x_s[R * XK];                // later (16 rows: beside them): the partial sums [NB + 1][4 quarters][R][16 features]
-    __shared__ __align__(16) float red_s[RB == 1 ? (NB + 1) * 4 * R * 16 : 4];
+    // row fragments in registers before W is there, partial sums beside the rows: not where the registers (64 rows) or the LDS (two workgroups
+    // of 32 rows x 32 features on a CU) do not hold them
+    constexpr bool PRE = RB == 1 || (RB <= 3 && ALONE);
+    __shared__ __align__(1024) bf16_t x_s[R * XK];
+    __shared__ __align__(16) float red_s[PRE ? (NB + 1) * 4 * R * 16 : 4];     // the partial sums [NB + 1][4 quarters][R][16 features], or in the rows' place
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
     // the row groups of a tile sit on one XCD (workgroups are dealt to the eight XCDs in turn) and share its W through the L2, also though
     // it is loaded nontemporally (N = 8224, two groups: 18.1 MB fetched, W is 16.8 and the rows on eight XCDs 1.0)
@@ -261,18 +269,21 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    u32x4 a[FB][8], ax[8];
+    u32x4 a[FB][2][4], ax[8];
+    auto load_w = [&](int f, int i) {
+        a[f][i >> 2][i & 3] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+            W + (size_t)min(nb0 + 16 * (half * FB + f) + (n & 12) + (i & 3), N - 1) * XK + 128 * (2 * q + (i >> 2)) + 32 * g + 8 * (n & 3)));
+    };
+    auto load_extra = [&] {
+        if (has_x)
 #pragma unroll
-    for (int f = 0; f < FB; f++)
+            for (int i = 0; i < 8; i++)
+                ax[i] = *reinterpret_cast<const u32x4*>(W + (size_t)(nx + (n & 3)) * XK + 128 * (2 * q + (i >> 2)) + 32 * g + 8 * (i & 3));
+    };
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            a[f][i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
-                W + (size_t)min(nb0 + 16 * (half * FB + f) + (n & 12) + (i & 3), N - 1) * XK + 128 * (2 * q + (i >> 2)) + 32 * g + 8 * (n & 3)));
-    if (has_x)
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            ax[i] = *reinterpret_cast<const u32x4*>(W + (size_t)(nx + (n & 3)) * XK + 128 * (2 * q + (i >> 2)) + 32 * g + 8 * (i & 3));
-    __builtin_amdgcn_sched_barrier(0);                            // everything is in flight before the first row is looked at
+    for (int i = 0; i < 8; i++) load_w(0, i);
+    if (FB == 1) load_extra();
+    __builtin_amdgcn_sched_barrier(0);                            // all this is in flight before the first row is looked at
     if (RMS) {
         double ss[RW];
 #pragma unroll
@@ -294,7 +305,7 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
             for (int c = 0; c < 2; c++)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    xr[i][c][j] = pack_bf(lo_bf(wn[c][j]) * (lo_bf(xr[i][c][j]) * inv[i]), hi_bf(wn[c][j]) * (hi_bf(xr[i][c][j]) * inv[i]));
+                    xr[i][c][j] = pack2_bf(lo_bf(wn[c][j]) * (lo_bf(xr[i][c][j]) * inv[i]), hi_bf(wn[c][j]) * (hi_bf(xr[i][c][j]) * inv[i]));
     }
 #pragma unroll
     for (int i = 0; i < RW; i++) {
@@ -303,6 +314,11 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
         for (int c = 0; c < 2; c++) *reinterpret_cast<u32x4*>(x_s + r * XK + 8 * ((lane + 64 * c) ^ (r & 15))) = xr[i][c];
     }
     lds_barrier();
+    if (FB == 2) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) load_w(1, i);
+        load_extra();
+    }
     f32x4 acc[FB][RB], acc_x[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) acc_x[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -317,35 +333,46 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
     auto mma = [](const u32x4& av, const u32x4& bv, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv), c, 0, 0, 0);
     };
-    u32x4 xf[RB == 1 ? 8 : 1];                                    // (one row block: read while the last of W is still on its way)
-    if constexpr (RB == 1) {
+    u32x4 xf[PRE ? 8 : 1][PRE ? RB : 1];                          // (read while W is still on its way)
+    if constexpr (PRE) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) xf[i] = x_frag(i, 0);
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) xf[i][rb] = x_frag(i, rb);
         __builtin_amdgcn_sched_barrier(0);
     }
+    auto x_at = [&](int i, int rb) { return PRE ? xf[PRE ? i : 0][PRE ? rb : 0] : x_frag(i, rb); };
+    // block by block, so that one is multiplied while the next one's W arrives; where the fragments are read for each use, all blocks at once
 #pragma unroll
-    for (int f = 0; f < FB; f++)
+    for (int f = 0; f < FB; f++) {
 #pragma unroll
-        for (int t = 0; t < 8; t += 4) quad_transpose(a[f][t], a[f][t + 1], a[f][t + 2], a[f][t + 3], odd, high);
+        for (int t = 0; t < 2; t++) quad_transpose(a[f][t], odd, high);
+        if (PRE)
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        u32x4 b[RB];
+            for (int i = 0; i < 8; i++)
 #pragma unroll
-        for (int rb = 0; rb < RB; rb++) b[rb] = RB == 1 ? xf[RB == 1 ? i : 0] : x_frag(i, rb);
-#pragma unroll
-        for (int f = 0; f < FB; f++)
-#pragma unroll
-            for (int rb = 0; rb < RB; rb++) acc[f][rb] = mma(a[f][i], b[rb], acc[f][rb]);
+                for (int rb = 0; rb < RB; rb++) acc[f][rb] = mma(a[f][i >> 2][i & 3], x_at(i, rb), acc[f][rb]);
     }
+    if (!PRE)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            u32x4 b[RB];
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) b[rb] = x_frag(i, rb);
+#pragma unroll
+            for (int f = 0; f < FB; f++)
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++) acc[f][rb] = mma(a[f][i >> 2][i & 3], b[rb], acc[f][rb]);
+        }
     if (has_x) {
 #pragma unroll
         for (int i = 0; i < 8; i++)
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++) acc_x[rb] = mma(ax[i], RB == 1 ? xf[RB == 1 ? i : 0] : x_frag(i, rb), acc_x[rb]);
+            for (int rb = 0; rb < RB; rb++) acc_x[rb] = mma(ax[i], x_at(i, rb), acc_x[rb]);
     }
-    if (RB > 1) lds_barrier();                                    // the rows have been read: their memory takes the partial sums
+    if (!PRE) lds_barrier();                                      // the rows have been read: their memory takes the partial sums
     // accumulator element i of lane (n, g) is feature 4 g + i of row 16 rb + n
-    float* red = RB == 1 ? red_s : reinterpret_cast<float*>(x_s);
+    float* red = PRE ? red_s : reinterpret_cast<float*>(x_s);
     auto put = [&](int blk, const f32x4 (&v)[RB]) {
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) *reinterpret_cast<f32x4*>(red + ((blk * 4 + q) * R + 16 * rb + n) * 16 + 4 * g) = v[rb];
@@ -499,7 +526,7 @@ struct RowsGrid {
     bool one_round(int cus) const { return (long)tiles * groups <= cus; }        // a workgroup per CU at most
 };
 constexpr int MAX_GROUPS = 65535;      // of a launch (second dimension of a grid)
-template <int RB, int FB, bool RMS>
+template <int RB, int FB, bool RMS, bool ALONE = true>
 void launch_rows(const gemv_args& p, int cus) {
     const RowsGrid r(p, cus, RB, FB);
     const dim3 block(512);
@@ -510,11 +537,11 @@ void launch_rows(const gemv_args& p, int cus) {
         bf16_t* y = p.y + row0 * (p.epi == EPI_SWIGLU ? p.N / 2 : p.N);
         const int M = p.M - (int)row0;
         if (p.epi == EPI_NONE)
-            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_NONE>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
+            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_NONE, ALONE>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
         else if (p.epi == EPI_ADD)
-            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_ADD>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
+            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_ADD, ALONE>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
         else
-            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_SWIGLU>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
+            hipLaunchKernelGGL((rows_gemm_kernel<RB, FB, RMS, EPI_SWIGLU, ALONE>), grid, block, 0, p.stream, p.W, x, p.nw, p.eps, res, y, M, p.N, r.tiles, r.extra);
     }
 }
 // the shapes rows_gemm_kernel takes (its 8-byte stores and residual loads want y and res aligned to 8 bytes)
@@ -523,9 +550,10 @@ inline bool rows_shape(const gemv_args& p) {
 }
 constexpr int RMS_ROWS_MAX = 96;       // most rows with the prologue fused in: beyond, the rows are normalised too often
 // Tile by rows.  Up to 96 rows: the smallest tile that leaves at most one workgroup per CU (32 features as long as one row
-// group holds the batch, then 64).  Where none does, W is what costs, and one row group is better than two that read it twice:
-// 64 features x 48 or 64 rows (N = 9216 / 32768 / 151936 at 48 rows 8.5 / 19.2 / 82 us, 11.3 / 24.4 / 102 with 32 features; at 64 rows 9.1 /
-// 20.8 / 88, 11.9 / 25.7 / 108 with two groups of 32 rows); up to 32 rows 32 features again, whose two workgroups per CU overlap (N =
+// group holds the batch, then 64; at 33 - 48 rows with the prologue 32 rows x 64 features, which normalise fewer rows each: 7.1 / 6.7 / 6.2 us against
+// 7.3 / 7.0 / 6.5 with 48 x 32, without it 6.5 against 6.0).  Where none does, W is what costs, and one row group is better than two that read it twice:
+// 64 features x 48 or 64 rows (N = 9216 / 32768 / 151936 at 48 rows 6.6 / 15.9 / 70 us; with an earlier build 8.5 / 19.2 / 82, 11.3 / 24.4 / 102 with 32
+// features, at 64 rows 9.1 / 20.8 / 88, 11.9 / 25.7 / 108 with two groups of 32 rows); up to 32 rows 32 features again, whose two workgroups per CU overlap (N =
 // 32768 / 151936 16 / 61 us at 17 rows, 17.3 / 68 with 64).  Beyond 96 rows 64 x 64 up to 128 rows, then 32 x 32 (N = 8224 / 7168 / 5120 at
 // 128 rows 13.1 / 12.5 / 11.6 us with the rms launch, 256 23 / 21.4 / 16.8, 4096 351 / 301 / 221; 23.7 / 22.6 / 14.7, 33.8 / 31.5 / 24.7 and 429 / 325 / 274
 // with the 64-row tiles of general loads before).
@@ -541,18 +569,20 @@ bool launch_rows_any(const gemv_args& p, int cus) {
     if (p.M <= 32) {
         if (!one_round(2, 1) && one_round(2, 2))
             launch_rows<2, 2, RMS>(p, cus);
-        else if (!RMS || one_round(2, 1))
+        else if (one_round(2, 1))
             launch_rows<2, 1, RMS>(p, cus);
+        else if constexpr (!RMS)
+            launch_rows<2, 1, false, false>(p, cus);
         else
             return false;
         return true;
     }
-    if (p.M <= 48 && one_round(3, 1)) {
-        launch_rows<3, 1, RMS>(p, cus);
+    if (p.M <= 96 && (RMS || p.M > 48) && one_round(2, 2)) {
+        launch_rows<2, 2, RMS>(p, cus);
         return true;
     }
-    if (p.M > 48 && p.M <= 96 && one_round(2, 2)) {
-        launch_rows<2, 2, RMS>(p, cus);
+    if (p.M <= 48 && one_round(3, 1)) {
+        launch_rows<3, 1, RMS>(p, cus);
         return true;
     }
     if ((p.M <= 48 || (p.M > 64 && p.M <= 96)) && (!RMS || one_round(3, 2))) {
@@ -563,7 +593,7 @@ bool launch_rows_any(const gemv_args& p, int cus) {
         if (p.M <= 128)
             launch_rows<4, 2, false>(p, cus);
         else
-            launch_rows<2, 1, false>(p, cus);
+            launch_rows<2, 1, false, false>(p, cus);
         return true;
     }
     return false;
