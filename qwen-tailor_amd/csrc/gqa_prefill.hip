@@ -66,15 +66,6 @@ __device__ __forceinline__ void lds_dma16(const char* base, unsigned voff, unsig
                  : "v"(voff), "s"(base), "s"(la), "n"(IMM)
                  : "memory");
 }
-// ... and from an address of each lane's own
-__device__ __forceinline__ void lds_dma16_from(const char* src, unsigned lds) {
-    const unsigned la = __builtin_amdgcn_readfirstlane(lds);
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep)
-                 : "v"(src), "s"(la)
-                 : "memory");
-}
 // four such loads, KiB 0 .. 3 behind lds, under one setting of M0 (a wavefront issues one instruction every four clocks, and
 // the tile loop is bound by exactly that, so the five scalar instructions around a single load count)
 __device__ __forceinline__ void lds_dma16x4(const char* base, unsigned v0, unsigned v1, unsigned v2, unsigned v3, unsigned lds) {

@@ -7,10 +7,11 @@
 //               add:    y = bf16(BF(s) + res)                                                           (kernels.py:161-169)
 //               swiglu: y[m][p] = bf16(silu_bf16(BF(s[m][2p])) * BF(s[m][2p+1]))   interleaved rows     (kernels.py:170-182)
 // The batch is small, so the product is bound by what ONE CU has to pull in (its share of W and of x) and by the launch itself.
-// Three kernels by shape:
+// Four kernels by shape:
 //   rows_gemm_kernel  the wide projections of a decode / verify batch (K = 1024, N >= 4096): the rows live in LDS, the rms
 //                     prologue is applied on the way there, a workgroup owns 32 or 64 output features (and up to four more)
 //   quad_gemm_kernel  narrow outputs: small tiles (4 x 4 .. 16 x 16 outputs) so that every CU has one
+//   tile_gemm_kernel  narrow outputs where one tile of 16 x 16 per CU does: operands through LDS
 //   skinny_gemm_kernel  everything else: 16 features x up to 64 rows per workgroup
 // What decides the first two is how a load maps to lanes.  An MFMA operand wants 16 different rows in 16 neighbouring lanes; a
 // load shaped like that asks for 16 bytes of 16 different rows per quarter-wavefront, and a CU then takes in 16 bytes per clock
@@ -419,7 +420,7 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
 // PEEL: the first trip is taken out of the loop (by the residual's load, which only that trip makes): 0.2 - 0.6 us less, for a tenth more
 // registers, which costs where several workgroups share a CU (80 rows 7.2 / 10.8 us against 6.4 / 10.3).
 // Measured in a HIP graph with the residual epilogue, K = 2048 / 3584 (before: residual loaded behind the last barrier, no trip peeled): 1 row
-// 3.0 / 3.5 us (3.3 / 3.8), 16 rows 3.4 / 4.4 (3.7 / 4.8), 32 rows 3.8 / 5.2 (4.2 / 5.6), 64 rows 5.2 / 6.2 (5.4 / 6.9).
+// 3.0 / 3.5 us (3.3 / 3.8), 16 rows 3.4 / 4.4 (3.7 / 4.8), 32 rows 3.8 / 5.2 (4.2 / 5.6), 64 rows - / 6.2 (5.4 / 6.9).
 template <int NWV, int KS, int FG, int MG, int EPI, bool PEEL, bool ONE>
 __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
                                                              const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N, int K,
@@ -502,6 +503,90 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
             const float v = total(er, ef);
             y[eo] = EPI == EPI_ADD ? f2bf(BF(v) + bf2f((bf16_t)res_raw)) : f2bf(v);
         }
+    }
+}
+
+// Narrow outputs of 1024 < K <= 2048 whose 16 x 16 tiles leave at most one workgroup per CU and whose 8 x 16 tiles do not.  A CU takes a load of
+// 1 KiB every 16 clocks, so what counts is the bytes of its tiles: 128 KiB for one of 16 x 16 at K = 2048, 192 for two of 8 x 16.  The wavefronts
+// deal the 128-wide steps of K among themselves as quad_gemm_kernel's do; the operands go straight to LDS, into 16 KiB that belong to the
+// wavefront (no barrier, no registers: a wavefront waits for its own loads), the 16-byte chunks of a row XOR-swizzled by the row number, so
+// that an MFMA takes 16 rows of each and none of its results is thrown away (16 MFMAs a step there, 4 here).
+// MFMA j of a step takes k slice j (elements 32 g + 8 j ..), each slice has an accumulator of its own and the four are added as there: the
+// same bits.
+// us in a graph with the residual, quad_gemm_kernel / here: N = 1024, K = 2048 at 33 / 48 / 64 rows 4.8 / 5.05 / 5.1 -> 3.8 / 4.2 / 4.25, N = 2048 at 24 / 32
+// rows 5.2 / 5.4 -> 4.2 / 4.6, N = 4096 at 16 rows 6.0 -> 5.3, N = 520 at 96 rows 4.7 -> 4.2, K = 1280 0.5 less.  A kernel that only loads these
+// bytes takes 3.6 (N = 1024, 64 rows).  Longer K (224 KiB at K = 3584) with the steps beyond 128 KiB held in registers: 6.4, 6.1 there.
+template <int EPI>
+__global__ __launch_bounds__(512) void tile_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
+                                                        bf16_t* __restrict__ y, int M, int N, int K, int groups) {
+    __shared__ __align__(1024) char own_s[8 * 16384];
+    __shared__ __align__(16) float red[8][16][16];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int s = blockIdx.x >> 3, grp = s % groups, tile = (s / groups) * 8 + (blockIdx.x & 7);      // row groups of a tile: one XCD
+    const int n0 = tile * 16, m0 = grp * 16, steps = K / 128;
+    if (n0 >= N) return;
+    const char *wsrc[4], *xsrc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int r = 4 * i + g, off = (n ^ r) * 16;
+        wsrc[i] = reinterpret_cast<const char*>(W + (size_t)min(n0 + r, N - 1) * K) + off;
+        xsrc[i] = reinterpret_cast<const char*>(x + (size_t)min(m0 + r, M - 1) * K) + off;
+    }
+    const char* own = own_s + w * 16384;
+    const unsigned own_a = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)own_s + w * 16384;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const int k0 = min(w + 8 * c, steps - 1) * 256;           // (a step past the end loads the last one and is not multiplied)
+#pragma unroll
+        for (int i = 0; i < 4; i++) lds_dma16_from(wsrc[i] + k0, own_a + c * 8192 + i * 1024);
+#pragma unroll
+        for (int i = 0; i < 4; i++) lds_dma16_from(xsrc[i] + k0, own_a + c * 8192 + 4096 + i * 1024);
+    }
+    // the thread's output in the epilogue; its residual is requested behind the operands
+    const int er = threadIdx.x >> 4, ef = threadIdx.x & 15;
+    const bool e_mine = er < 16 && m0 + er < M && n0 + ef < N;
+    const size_t eo = (size_t)(m0 + er) * N + n0 + ef;
+    unsigned res_raw = 0;
+    if (EPI == EPI_ADD && e_mine) res_raw = res[eo];
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](int c) {
+        u32x4 a[4], b[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const char* q = own + c * 8192 + n * 256 + ((4 * g + j) ^ n) * 16;
+            a[j] = *reinterpret_cast<const u32x4*>(q);
+            b[j] = *reinterpret_cast<const u32x4*>(q + 4096);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[j]), __builtin_bit_cast(bf16x8, b[j]), acc[j], 0, 0, 0);
+    };
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");              // (the second step's loads; the residual's may be one more)
+    multiply(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (w + 8 < steps) multiply(1);
+    *reinterpret_cast<f32x4*>(&red[w][n][4 * g]) = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    lds_barrier();
+    auto total = [&](int r, int f) {                              // fixed order: pairs, then pairs of pairs, ...
+        float t[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) t[k] = red[k][r][f];
+#pragma unroll
+        for (int st = 1; st < 8; st *= 2)
+#pragma unroll
+            for (int k = 0; k < 8; k += 2 * st) t[k] += t[k + st];
+        return t[0];
+    };
+    if (EPI == EPI_SWIGLU) {
+        const int r = threadIdx.x / 8, p = threadIdx.x % 8, m = m0 + r;
+        if (r < 16 && m < M && n0 + 2 * p + 1 < N)
+            y[(size_t)m * (N / 2) + n0 / 2 + p] = f2bf(silu_bf16(BF(total(r, 2 * p))) * BF(total(r, 2 * p + 1)));
+    } else if (e_mine) {
+        const float v = total(er, ef);
+        y[eo] = EPI == EPI_ADD ? f2bf(BF(v) + bf2f((bf16_t)res_raw)) : f2bf(v);
     }
 }
 
@@ -620,6 +705,16 @@ void launch_quad(const gemv_args& p) {
     else
         launch_quad_tile<8, 4, FG, MG, PEEL_>(p);
 }
+void launch_tile(const gemv_args& p) {
+    const int groups = (p.M + 15) / 16, tiles = (p.N + 15) / 16;
+    const dim3 grid((tiles + 7) / 8 * 8 * groups), block(512);
+    if (p.epi == EPI_NONE)
+        hipLaunchKernelGGL(tile_gemm_kernel<EPI_NONE>, grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+    else if (p.epi == EPI_ADD)
+        hipLaunchKernelGGL(tile_gemm_kernel<EPI_ADD>, grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+    else
+        hipLaunchKernelGGL(tile_gemm_kernel<EPI_SWIGLU>, grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+}
 // The smallest tile that leaves at most one workgroup per CU; beyond, small tiles still win with several workgroups per CU (measured
 // against skinny_gemm_kernel over N = 264 .. 3072, K = 512 .. 4096, 16 .. 192 rows, us: three workgroups of 8 x 16 per CU N = 1024, K = 2048 / 3584 at 80
 // rows 6.4 / 10.3 against 9.5 / 16.1, N = 3072, K = 2048 at 32 rows 7.3 against 10.1; N = 8192, K = 2048, 8 rows, four of 8 x 8 8.3 against 9.4; two
@@ -633,6 +728,8 @@ inline bool launch_quad_any(const gemv_args& p, int cus) {
         launch_quad<2, 2>(p);
     else if (wgs(8, 16) <= cus)
         launch_quad<2, 4>(p);
+    else if (p.K > 1024 && p.K <= 2048 && wgs(16, 16) <= cus)
+        launch_tile(p);
     else if (p.K > 2048 && wgs(16, 16) <= cus)
         launch_quad<4, 4>(p);
     else if (wgs(8, 16) <= 3 * cus)

@@ -382,6 +382,17 @@ __device__ __forceinline__ float dot8_row16(const float (&a)[8], const float (&b
     return row16_sum(t);
 }
 
+// One direct-to-LDS load of 16 bytes per lane (global_load_lds_dwordx4) from an address of each lane's own: the 64 pieces land at lds + 16 l.
+// Inline assembly, so that the compiler does not count it: it is waited for by hand.  lds is wavefront-uniform.
+__device__ __forceinline__ void lds_dma16_from(const char* src, unsigned lds) {
+    const unsigned la = __builtin_amdgcn_readfirstlane(lds);
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(src), "s"(la)
+                 : "memory");
+}
+
 // workgroup id remapped so that consecutive logical ids share an XCD (8 XCDs, hardware deals workgroups round-robin)
 __device__ __forceinline__ unsigned xcd_remap(unsigned id, unsigned n) {
     return (n % 8u == 0u) ? (id % 8u) * (n / 8u) + id / 8u : id;

@@ -175,6 +175,20 @@ def test_narrow_projection_tiles_exact_on_small_integers(qt, dev, M, N, K, epi):
         check_equal("integer product", to_np(got), want)
 
 
+# 16 x 16 tiles through LDS (one per CU where 8 x 16 would take two): outputs and rows that end inside a tile, wavefronts with one and with two
+# steps of K (1280: two of ten wavefronts' steps; 1792), the fewest and the most tiles of the rule
+@pytest.mark.parametrize("M,N,K", [(33, 1024, 2048), (64, 1023, 2048), (49, 1030, 1280), (96, 520, 1792), (17, 2047, 1536), (32, 2050, 2048), (9, 4095, 1280), (16, 4096, 2048),
+                                   (130, 260, 2048), (257, 130, 1280)])
+def test_narrow_projection_one_tile_per_cu(qt, dev, M, N, K):
+    """exact on small integers, and on real values the bits of the same rows in batches of up to 16 (which smaller tiles take)"""
+    for epi in (0, 1) + ((2,) if N % 2 == 0 else ()):
+        test_narrow_projection_tiles_exact_on_small_integers(qt, dev, M, N, K, epi)
+    g = torch.Generator().manual_seed(M + N + K)
+    W, x = (torch.randn((N, K), generator=g) * K ** -0.5).to(BF16).to(dev), torch.randn((M, K), generator=g).to(BF16).to(dev)
+    few = 16 if N <= 1024 else 8 if N <= 2050 else 4
+    check_tensors_equal("rows", qt.kernels.fused_gemv(W, x), torch.cat([qt.kernels.fused_gemv(W, x[i:i + few]) for i in range(0, M, few)]))
+
+
 # K of one trip (up to 1024): every wavefront with two steps, with one, with one of two, and none for some
 @pytest.mark.parametrize("K", [1024, 512, 768, 256])
 @pytest.mark.parametrize("M,N", [(1, 2048), (3, 1027), (17, 2050), (80, 520)])
