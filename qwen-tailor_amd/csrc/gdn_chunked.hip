@@ -383,12 +383,12 @@ __device__ __forceinline__ uint4 z_row(const bf16_t* __restrict__ proj, int c, i
     const u32x4 zw = load_once<STREAM>(reinterpret_cast<const u32x4*>(proj + (size_t)min(c * C + row, S - 1) * PW + CD + h * DV) + cc);
     return make_uint4(zw[0], zw[1], zw[2], zw[3]);
 }
-// by NT = 256 or 512 threads, NT / 16 rows at a time.  Z(it): the z values of row NT / 16 it + tid / 16, eight per thread
-template <int NT, class ZFn>
-__device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c, int h, bf16_t* __restrict__ y, ZFn Z, const float* __restrict__ gw,
+// of the 16 IT rows from token t0 on, by 256 threads, 16 rows at a time.  Z(it): the z values of row 16 it + tid / 16, eight per thread
+template <int IT, class ZFn>
+__device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int t0, int h, bf16_t* __restrict__ y, ZFn Z, const float* __restrict__ gw,
                                                 float eps, int S) {
-    constexpr int RP = NT / 16, IT = C / RP;
-    static_assert(IT == 4 || IT == 2, "four or two rows per 16-lane group");
+    constexpr int RP = 16;
+    static_assert(IT == 4 || IT == 1, "four rows or one per 16-lane group");
     const int cc = tid & 15;
     float gwv[8];
 #pragma unroll
@@ -417,13 +417,12 @@ __device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int c,
     if constexpr (IT == 4) {
         rsqrt_rows4(ss4, eps, inv4, cc);
     } else {
-        const float ss2[2] = {(float)row16_sum_d(ss4[0]), (float)row16_sum_d(ss4[1])};
-        rsqrt_rows<2>(ss2, eps, inv4, cc);
+        inv4[0] = rsqrt_rn((float)row16_sum_d(ss4[0]) / 128.0f + eps);
     }
 #pragma unroll
     for (int it = 0; it < IT; it++) {
         const int row = it * RP + (tid >> 4);
-        const int t = c * C + row;
+        const int t = t0 + row;
         if (t >= S) continue;                                       // whole 16-lane groups leave together
         float yy[8], zz[8];
         unpack8(yv4[it], yy);
@@ -538,8 +537,8 @@ __device__ __forceinline__ void output_item(bf16_t* ys, volatile int* ready, int
                     for (int i = 0; i < 4; i++) dst[i] = src[i];
                 }
             } else {
-                gated_norm_tile<256>((lds_bf16_ptr)ys, tid, c, h, y, [&](int it) { return z_row<WAIT>(proj, c, h, it * 16 + (tid >> 4), tid & 15, S); }, gw,
-                                eps, S);
+                gated_norm_tile<4>((lds_bf16_ptr)ys, tid, c * C, h, y, [&](int it) { return z_row<WAIT>(proj, c, h, it * 16 + (tid >> 4), tid & 15, S); }, gw,
+                                   eps, S);
             }
         }
         __syncthreads();                                                        // ys is reused by the next round
@@ -639,10 +638,10 @@ struct PhaseALds {                       // 73 KiB: two workgroups per CU
     __align__(16) bf16_t taps[3 * DK * 4];       // fused conv only: this head's conv taps
     __align__(16) float Td[4 * ND_BLK];          // their inverses: [block][column][row]
     float Lc2[C], beta[C], gam[C];               // Lc2 = log2(e) * cumsum(log g)
-    int staged[4];                               // wavefronts that have staged their part of k, q, v (PA_K, PA_Q, PA_V)
+    int staged[4];                               // wavefronts that have staged their part of k, q, v, the gates (PA_K ..)
 };
 static_assert(sizeof(PhaseALds) >= 65536 && __builtin_offsetof(PhaseALds, tab) == 0, "an unclamped lookup reads up to 64 KiB from tab on");
-constexpr int PA_K = 0, PA_Q = 1, PA_V = 2;
+constexpr int PA_K = 0, PA_Q = 1, PA_V = 2, PA_GATES = 3;     // (the gates: one producer, a prompt of one chunk only)
 
 // A wavefront announces that its LDS stores of a part are done; a consumer waits until all four producers have.  (The parts
 // are produced and consumed by different wavefronts at different times: a workgroup barrier would hold up seven wavefronts
@@ -651,8 +650,8 @@ __device__ __forceinline__ void part_staged(PhaseALds& L, int part, int lane) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     if (lane == 0) __hip_atomic_fetch_add(&L.staged[part], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ __forceinline__ void await_part(PhaseALds& L, int part) {
-    while (__hip_atomic_load(&L.staged[part], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < 4) __builtin_amdgcn_s_sleep(1);
+__device__ __forceinline__ void await_part(PhaseALds& L, int part, int producers = 4) {
+    while (__hip_atomic_load(&L.staged[part], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < producers) __builtin_amdgcn_s_sleep(1);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
@@ -694,6 +693,27 @@ __device__ __forceinline__ f32x4 kk_block(const _Float16* Ks, int I, int J, int 
         const half8 a = *reinterpret_cast<const half8*>(&Ks[(16 * I + n) * QS_LD + 32 * kb + 8 * g]);
         const half8 b = *reinterpret_cast<const half8*>(&Ks[(16 * J + n) * QS_LD + 32 * kb + 8 * g]);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+// lower_incl(G * K Q^T), block of tokens 16 tj .. (rows) and queries 16 ct .. (columns): lane (n, g) gets query 16 ct + n, tokens 16 tj + 4 g + r;
+// G_ij = exp2(Lc2_i - Lc2_j)
+__device__ __forceinline__ f32x4 qk_block(const PhaseALds& L, int tj, int ct, int n, int g) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) {
+        const half8 a = *reinterpret_cast<const half8*>(&L.Ks[(16 * tj + n) * QS_LD + 32 * kb + 8 * g]);
+        const half8 b = *reinterpret_cast<const half8*>(&L.Qs[(16 * ct + n) * QS_LD + 32 * kb + 8 * g]);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc, 0, 0, 0);
+    }
+    const float lco = L.Lc2[16 * ct + n];
+    const f32x4 lcj = *reinterpret_cast<const f32x4*>(&L.Lc2[16 * tj + 4 * g]);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        float v = __builtin_amdgcn_exp2f(lco - lcj[r]) * acc[r];
+        asm("" : "+v"(v));                               // (the product is rounded to float before it is converted to half precision, in every instance)
+        acc[r] = (tj < ct || 4 * g + r <= n) ? v : 0.f;
     }
     return acc;
 }
@@ -834,8 +854,11 @@ __device__ __forceinline__ void inverse_row(PhaseALds& L, const int I, int n, in
 // every floating-point step is a single instruction chosen in the source (MFMA, multiplication, fused multiply-add), so the
 // compiler has nothing to contract differently in the two instances.
 //
-// ONE: a prompt of one chunk.  The workgroup of a head goes on to the outputs and the new state by itself (one_chunk below): no records, one
-// launch instead of three.
+// ONE: a prompt of one chunk.  The workgroups of a head go on to the outputs and the new state by themselves (one_chunk below): no records, one
+// launch instead of three.  A head has a workgroup per 16 rows of outputs and two for the state (half of the columns each).  Each convolves
+// what it needs: k and v of all tokens up to its own (`nt` tiles of 16, wavefront w of either group takes tile w), q of its own rows.  A ninth
+// wavefront computes the gates.
+constexpr int ONE_STATE_WGS = 2, ONE_THREADS = 576;
 struct OneArgs {
     const float* st_in;
     float* st_out;
@@ -845,35 +868,39 @@ struct OneArgs {
     int *status, *host_words;
 };
 struct OneLds {
-    __align__(16) _Float16 Tb[NCT * 2 * 512], Am[NCT * 2 * 512];     // operand tiles [row tile][kb2][lane][8]
+    __align__(16) _Float16 Tb[NCT * 2 * 512], Am[2 * 512];           // operand tiles [row tile][kb2][lane][8]
     __align__(16) float dec[C];
+    __align__(16) bf16_t ys[16 * YS_LD];                             // outputs
     float gC;
 };
 // What remains of a single chunk once K, Q, V, Tb and Am are in LDS; wavefront sl owns the columns 16 sl .. + 15 of the head (dv).  The state
 // never leaves its registers, so that the products are those of the definition, with nothing folded into operands beforehand:
 //     D = Tb (V - gamma * (K S^T)),   Y = gamma * (Q S^T) + Am D,   S' = gamma_C S + K^T (dec * D)
-__device__ __forceinline__ void one_chunk(const PhaseALds& L, const OneLds& L1, bf16_t* ys, const f32x4 (&S0)[8], const uint4 (&zv)[2], const OneArgs& o,
-                                          int h, int sl, int tid, int n, int g, int S) {
+// ot: the row tile whose outputs this workgroup forms; negative for the state, of which the wavefront then writes half of the rows (dk).
+__device__ __forceinline__ void one_chunk(const PhaseALds& L, OneLds& L1, const f32x4 (&S0)[8], const uint4& zv, const OneArgs& o, int h, int ot,
+                                          int nt, int sl, int half, int tid, int n, int g, int S) {
     const int lane = tid & 63;
     half8 Sb[4];
 #pragma unroll
     for (int kb = 0; kb < 4; kb++) Sb[kb] = pack_half8(S0[2 * kb], S0[2 * kb + 1]);
     // rows of K or Q with the contraction index (dk) enumerated as the state's operand
     auto rows = [&](const _Float16* base, int ct, int kb) { return *reinterpret_cast<const half8*>(base + (16 * ct + n) * QS_LD + 32 * kb + 8 * g); };
-    f32x4 R[NCT], Y[NCT];
+    f32x4 R[NCT], Y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++) {
+        R[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (ct >= nt) continue;                                      // (the same for the whole workgroup)
         f32x4 ks = {0.f, 0.f, 0.f, 0.f};
-        Y[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kb = 0; kb < 4; kb++) {
-            ks = __builtin_amdgcn_mfma_f32_16x16x32_f16(rows(L.Ks, ct, kb), Sb[kb], ks, 0, 0, 0);
-            Y[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Sb[kb], rows(L.Qs, ct, kb), Y[ct], 0, 0, 0);   // (transposed, as in the output kernel)
-        }
+        for (int kb = 0; kb < 4; kb++) ks = __builtin_amdgcn_mfma_f32_16x16x32_f16(rows(L.Ks, ct, kb), Sb[kb], ks, 0, 0, 0);
         const f32x4 gm = *reinterpret_cast<const f32x4*>(&L.gam[16 * ct + 4 * g]);
 #pragma unroll
         for (int r = 0; r < 4; r++) R[ct][r] = __builtin_fmaf(-gm[r], ks[r], (float)L.Vs[(16 * ct + 4 * g + r) * VS_LD + 16 * sl + n]);
-        Y[ct] *= L.gam[16 * ct + n];
+    }
+    if (ot >= 0) {
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++) Y = __builtin_amdgcn_mfma_f32_16x16x32_f16(Sb[kb], rows(L.Qs, ot, kb), Y, 0, 0, 0);   // (transposed, as in the output kernel)
+        Y *= L.gam[16 * ot + n];
     }
     // R carries no beta, unlike everything that the chain packs: it may pass the half-precision range where D does not.  A column (a lane's
     // n) is then multiplied by a power of two first, and its D divided by it.
@@ -897,6 +924,7 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, const OneLds& L1, 
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++) {
         D[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (ct >= nt) continue;
 #pragma unroll
         for (int kb2 = 0; kb2 < (ct < 2 ? 1 : 2); kb2++)             // (lower triangular)
             D[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const half8*>(&L1.Tb[(ct * 2 + kb2) * 512 + lane * 8]), Rb[kb2], D[ct], 0, 0, 0);
@@ -904,41 +932,43 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, const OneLds& L1, 
     if (far)
 #pragma unroll
         for (int ct = 0; ct < NCT; ct++) D[ct] *= back;
-    f32x4 Dd[NCT];
-#pragma unroll
-    for (int ct = 0; ct < NCT; ct++) Dd[ct] = D[ct] * *reinterpret_cast<const f32x4*>(&L1.dec[16 * ct + 4 * g]);
-    const half8 Dn[2] = {pack_half8(D[0], D[1]), pack_half8(D[2], D[3])}, Ds[2] = {pack_half8(Dd[0], Dd[1]), pack_half8(Dd[2], Dd[3])};
-#pragma unroll
-    for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-        for (int kb2 = 0; kb2 < (ct < 2 ? 1 : 2); kb2++)
-            Y[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Dn[kb2], *reinterpret_cast<const half8*>(&L1.Am[(ct * 2 + kb2) * 512 + lane * 8]), Y[ct], 0, 0, 0);
     bool bad = false;
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++)
 #pragma unroll
         for (int r = 0; r < 4; r++) bad |= fabsf(D[ct][r]) >= HALF_END;
-    float* so = o.st_out + ((size_t)h * DV + sl * 16 + n) * DK + 8 * g;
+    if (ot < 0) {
+        f32x4 Dd[NCT];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {                                    // row 4 g + r of tile i is row 32 (i / 2) + 8 g + 4 (i % 2) + r of the state
-        f32x4 s1 = S0[i] * L1.gC;
+        for (int ct = 0; ct < NCT; ct++) Dd[ct] = D[ct] * *reinterpret_cast<const f32x4*>(&L1.dec[16 * ct + 4 * g]);
+        const half8 Ds[2] = {pack_half8(Dd[0], Dd[1]), pack_half8(Dd[2], Dd[3])};
+        float* so = o.st_out + ((size_t)h * DV + sl * 16 + n) * DK + 8 * g;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {                                // row 4 g + r of tile i is row 32 (i / 2) + 8 g + 4 (i % 2) + r of the state
+            if ((i >> 2) != half) continue;
+            f32x4 s1 = S0[i] * L1.gC;
+#pragma unroll
+            for (int kb2 = 0; kb2 < 2; kb2++)
+                s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(tokens_operand<8>(L.Ks, QS_LD, kb2, 32 * (i >> 1) + 4 * (i & 1), n, g), Ds[kb2], s1, 0, 0, 0);
+            *reinterpret_cast<f32x4*>(so + 32 * (i >> 1) + 4 * (i & 1)) = s1;
+#pragma unroll
+            for (int r = 0; r < 4; r++) bad |= !(fabsf(s1[r]) <= 3.0e38f);
+        }
+    } else {
+        const half8 Dn[2] = {pack_half8(D[0], D[1]), pack_half8(D[2], D[3])};
 #pragma unroll
         for (int kb2 = 0; kb2 < 2; kb2++)
-            s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(tokens_operand<8>(L.Ks, QS_LD, kb2, 32 * (i >> 1) + 4 * (i & 1), n, g), Ds[kb2], s1, 0, 0, 0);
-        *reinterpret_cast<f32x4*>(so + 32 * (i >> 1) + 4 * (i & 1)) = s1;
-#pragma unroll
-        for (int r = 0; r < 4; r++) bad |= !(fabsf(s1[r]) <= 3.0e38f);
+            if (kb2 == 0 || ot >= 2)
+                Y = __builtin_amdgcn_mfma_f32_16x16x32_f16(Dn[kb2], *reinterpret_cast<const half8*>(&L1.Am[kb2 * 512 + lane * 8]), Y, 0, 0, 0);
     }
     if (__any(bad) && lane == 0) {                                   // (as in the chain)
         atomicOr(o.status, ERR_NOT_FINITE);
         o.host_words[1] = 1;
     }
-    __syncthreads();                                                 // Q has been read: its memory takes the outputs
-#pragma unroll
-    for (int ct = 0; ct < NCT; ct++)
-        *reinterpret_cast<uint2*>(&ys[(ct * 16 + n) * YS_LD + sl * 16 + 4 * g]) = make_uint2(pack2_bf(Y[ct][0], Y[ct][1]), pack2_bf(Y[ct][2], Y[ct][3]));
+    if (ot < 0) return;
+    *reinterpret_cast<uint2*>(&L1.ys[n * YS_LD + sl * 16 + 4 * g]) = make_uint2(pack2_bf(Y[0], Y[1]), pack2_bf(Y[2], Y[3]));
     __syncthreads();
-    gated_norm_tile<512>((lds_bf16_ptr)ys, tid, 0, h, o.y, [&](int it) { return zv[it]; }, o.gw, o.eps, S);
+    if (tid < 256) gated_norm_tile<1>((lds_bf16_ptr)L1.ys, tid, 16 * ot, h, o.y, [&](int) { return zv; }, o.gw, o.eps, S);
 }
 
 template <bool from_proj, bool ONE>
@@ -948,6 +978,8 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
                                         const float* __restrict__ A_log, const float* __restrict__ dt_bias, _Float16* __restrict__ ops,
                                         _Float16* __restrict__ U, float* __restrict__ gates, int S, const OneArgs& o) {
     const int c = ONE ? 0 : blk / HV, h = blk % HV, t0 = c * C;
+    const int ot = ONE ? blk / HV - ONE_STATE_WGS : 0;  // ONE: the row tile of the outputs, or the state (-2: the lower columns, -1)
+    const int nt = ONE && ot >= 0 ? ot + 1 : (S - t0 + 15) / 16;
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
     // (the wavefront number as a scalar: the branches on it are then real branches, which the barriers inside them need)
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -959,70 +991,17 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
     bf16_t* const outA = grpV ? qi : ki;                // group M convolves k, group V q and then v
     const int partA = grpV ? 0 : 1;
 
-    // ---- the chunk's rows: every load is issued before anything else; rows past the end are zero (gdn_nax.py:172-174)
-    // one register array per part for both forms.  !from_proj: rw[rr] = token rr * 16 + gi, a lane 8 consecutive columns;
-    // from_proj: rw[d] = input row 4 gi - 3 + d of 8 channels of the part
-    uint4 rwA[7], rwB[7];
-    // input rows 4 gi - 3 .. + 3 of this thread's channels of a part; rows before the sequence come from the conv state (first chunk
-    // only), rows past the end repeat the last.  Elsewhere an address is one multiply-add on a scalar base: with the choice
-    // made row by row the 21 addresses of a thread were 200 instructions, and the first loads left that much later.
-    auto conv_rows = [&](uint4 (&rw)[7], int part) {
-        const int ch = part * KD + h * DK;
-        if (c > 0) {
-            const char* base = reinterpret_cast<const char*>(proj + (size_t)(t0 - 3) * PW + ch);
-            const unsigned last = (unsigned)(S + 2 - t0);
-#pragma unroll
-            for (int d = 0; d < 7; d++)
-                rw[d] = *reinterpret_cast<const uint4*>(base + (__umul24(min((unsigned)(4 * gi + d), last), PW * 2) + 16u * (unsigned)cc));
-        } else {
-#pragma unroll
-            for (int d = 0; d < 7; d++) {
-                const int tt = min(4 * gi - 3 + d, S - 1);
-                rw[d] = *reinterpret_cast<const uint4*>((tt < 0 ? cs + (tt + 3) * CD : proj + tt * PW) + ch + 8 * cc);
-            }
-        }
-    };
-    // (wavefront 0 asks for its gate inputs first: loads return in order)
+    // (the wavefront of the gates asks for its inputs first: loads return in order)
+    constexpr int GATES_WV = ONE ? 8 : 0;
     unsigned ga_raw = 0, gb_raw = 0;
-    if (wv == 0) {
+    if (wv == GATES_WV) {
         const bf16_t* row = proj + (size_t)min(t0 + lane, S - 1) * PW + CD + KD + h;
         ga_raw = row[HV];
         gb_raw = row[0];
     }
-    // the SiLU table and the head's conv taps (3 x 128 channels x 4 taps: every token group needs the same 3 KiB) go to LDS.  Both
-    // are asked for ahead of the rows: a load behind them returns behind them, and a copy loop waits once per trip.
-    constexpr int TAB_VECS = SILU_TAB_SIZE / 8, TAP0 = 512 - 3 * 64;
-    uint4 tab0 = make_uint4(0, 0, 0, 0), tab1 = tab0, tap = tab0;
-    if (from_proj) {
-        const int i3 = max(tid - TAP0, 0);
-        if (silu_tab) {
-            tab0 = reinterpret_cast<const uint4*>(silu_tab)[tid];
-            tab1 = reinterpret_cast<const uint4*>(silu_tab)[min(tid + 512, TAB_VECS - 1)];
-        }
-        tap = reinterpret_cast<const uint4*>(cw + (size_t)((i3 >> 6) * KD + h * DK) * 4)[i3 & 63];
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (!from_proj) {
-#pragma unroll
-        for (int rr = 0; rr < 4; rr++) {
-            const int t = t0 + rr * 16 + gi;
-            const size_t o = ((size_t)min(t, S - 1) * HV + h) * DK + cc * 8;
-            rwA[rr] = *reinterpret_cast<const uint4*>(outA + o);
-            if (t >= S) rwA[rr] = make_uint4(0, 0, 0, 0);
-        }
-    } else {
-        conv_rows(rwA, partA);
-        if (conv_out && c == (S - 1) / C && tid >= 64 && tid < 64 + 3 * 48) {   // new conv window: input rows S-3 .. S-1 of this head's channels
-            const int i3 = tid - 64;
-            const int r = i3 / 48, part = (i3 % 48) >> 4, ch0 = part * KD + h * DK + (i3 & 15) * 8, tt = S - 3 + r;
-            *reinterpret_cast<uint4*>(conv_out + r * CD + ch0) =
-                *reinterpret_cast<const uint4*>(tt < 0 ? cs + (tt + 3) * CD + ch0 : proj + (size_t)tt * PW + ch0);
-        }
-    }
-
-    // ---- gates of the chunk's tokens (gdn_nax.py:80-104): wavefront 0, one token per lane.  Behind the barrier: nobody needs them before
-    // k is staged, which wavefront 0 announces after them, and group M has the time (it waits for v in the end).  With one chunk group M
-    // is what everything waits for, and the gates are computed while the table is on its way.
+    // ---- gates of the chunk's tokens (gdn_nax.py:80-104), one token per lane.  Behind the barrier: nobody needs them before k is staged, which
+    // wavefront 0 announces after them, and group M has the time (it waits for v in the end).  With one chunk group M is what everything waits
+    // for, and they have a wavefront of their own (0.3 - 0.6 us against a wavefront of either group; ahead of the barrier 0.5 slower).
     auto chunk_gates = [&] {
         const int t = t0 + lane;
         float lg = 0.f, be = 0.f;
@@ -1059,7 +1038,76 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
             if (lane >= 60) gp[G_GC + lane - 60] = lane == 60 ? expf(tot) : 0.f;
         }
     };
-    if (ONE && wv == 0) chunk_gates();
+    if (ONE && wv == GATES_WV) {                         // (ended, it is no party to the barriers that follow)
+        __syncthreads();
+        chunk_gates();
+        part_staged(L, PA_GATES, lane);
+        return;
+    }
+    // ---- the chunk's rows: every load is issued before anything else; rows past the end are zero (gdn_nax.py:172-174)
+    // one register array per part for both forms.  !from_proj: rw[rr] = token rr * 16 + gi, a lane 8 consecutive columns;
+    // from_proj: rw[d] = input row 4 gi - 3 + d of 8 channels of the part
+    uint4 rwA[7], rwB[7];
+    // input rows 4 gi - 3 .. + 3 of this thread's channels of a part; rows before the sequence come from the conv state (first chunk
+    // only), rows past the end repeat the last.  Elsewhere an address is one multiply-add on a scalar base: with the choice
+    // made row by row the 21 addresses of a thread were 200 instructions, and the first loads left that much later.
+    auto conv_rows = [&](uint4 (&rw)[7], int part) {
+        const int ch = part * KD + h * DK;
+        if (c > 0) {
+            const char* base = reinterpret_cast<const char*>(proj + (size_t)(t0 - 3) * PW + ch);
+            const unsigned last = (unsigned)(S + 2 - t0);
+#pragma unroll
+            for (int d = 0; d < 7; d++)
+                rw[d] = *reinterpret_cast<const uint4*>(base + (__umul24(min((unsigned)(4 * gi + d), last), PW * 2) + 16u * (unsigned)cc));
+        } else {
+#pragma unroll
+            for (int d = 0; d < 7; d++) {
+                const int tt = min(4 * gi - 3 + d, S - 1);
+                rw[d] = *reinterpret_cast<const uint4*>((tt < 0 ? cs + (tt + 3) * CD : proj + tt * PW) + ch + 8 * cc);
+            }
+        }
+    };
+    // the SiLU table and the head's conv taps (3 x 128 channels x 4 taps: every token group needs the same 3 KiB) go to LDS.  Both
+    // are asked for ahead of the rows: a load behind them returns behind them, and a copy loop waits once per trip.
+    constexpr int TAB_VECS = SILU_TAB_SIZE / 8, TAP0 = 512 - 3 * 64;
+    uint4 tab0 = make_uint4(0, 0, 0, 0), tab1 = tab0, tap = tab0;
+    if (from_proj) {
+        const int i3 = max(tid - TAP0, 0);
+        if (silu_tab) {
+            tab0 = reinterpret_cast<const uint4*>(silu_tab)[tid];
+            tab1 = reinterpret_cast<const uint4*>(silu_tab)[min(tid + 512, TAB_VECS - 1)];
+        }
+        tap = reinterpret_cast<const uint4*>(cw + (size_t)((i3 >> 6) * KD + h * DK) * 4)[i3 & 63];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!from_proj) {
+#pragma unroll
+        for (int rr = 0; rr < 4; rr++) {
+            const int t = t0 + rr * 16 + gi;
+            const size_t o = ((size_t)min(t, S - 1) * HV + h) * DK + cc * 8;
+            rwA[rr] = *reinterpret_cast<const uint4*>(outA + o);
+            if (t >= S) rwA[rr] = make_uint4(0, 0, 0, 0);
+        }
+    } else {
+        if constexpr (ONE) {                                    // k or v of the wavefront's token tile, q of one row a 16-lane group
+            if (grpV && ot >= 0)
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const int tt = min(16 * ot + 4 * w + g - 3 + d, S - 1);
+                    rwB[d] = *reinterpret_cast<const uint4*>((tt < 0 ? cs + (tt + 3) * CD : proj + (size_t)tt * PW) + h * DK + 8 * cc);
+                }
+            if (w < nt) conv_rows(rwA, grpV ? 2 : 1);
+        } else {
+            conv_rows(rwA, partA);
+        }
+        if (conv_out && (!ONE || ot == -1) && c == (S - 1) / C && tid >= 64 && tid < 64 + 3 * 48) {   // new conv window: input rows S-3 .. S-1 of this head's channels
+            const int i3 = tid - 64;
+            const int r = i3 / 48, part = (i3 % 48) >> 4, ch0 = part * KD + h * DK + (i3 & 15) * 8, tt = S - 3 + r;
+            *reinterpret_cast<uint4*>(conv_out + r * CD + ch0) =
+                *reinterpret_cast<const uint4*>(tt < 0 ? cs + (tt + 3) * CD + ch0 : proj + (size_t)tt * PW + ch0);
+        }
+    }
+
     if (from_proj) {
         static_assert(TAB_VECS > 512 && TAB_VECS <= 1024, "two vectors of the table per thread");
         if (silu_tab) {
@@ -1071,24 +1119,41 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
         if (tid >= TAP0) reinterpret_cast<uint4*>(L.taps)[tid - TAP0] = tap;
     }
 
-    // one chunk: this wavefront's columns of the state (lane (n, g): column n, rows 32 kb + 8 g .. + 7 in S0[2 kb], S0[2 kb + 1]) and its rows of z
+    // one chunk: this wavefront's columns of the state (lane (n, g): column n, rows 32 kb + 8 g .. + 7 in S0[2 kb], S0[2 kb + 1]) and its row of z.
+    // Asked for when the first part has been staged: ahead of the barrier they hold up the rows and the table (0.6 - 1 us).
+    const int sl = ONE && ot < 0 ? 4 * (ot + ONE_STATE_WGS) + w : wv;
     f32x4 S0[ONE ? 8 : 1];
-    uint4 zv[ONE ? 2 : 1];
+    uint4 zv = make_uint4(0, 0, 0, 0);
+    auto ask_state = [&] {
     if constexpr (ONE) {
-        const float* sp = o.st_in + ((size_t)h * DV + wv * 16 + n) * DK + 8 * g;
+        const float* sp = o.st_in + ((size_t)h * DV + sl * 16 + n) * DK + 8 * g;
 #pragma unroll
         for (int i = 0; i < 8; i++) S0[i] = *reinterpret_cast<const f32x4*>(sp + 32 * (i >> 1) + 4 * (i & 1));
-#pragma unroll
-        for (int it = 0; it < 2; it++) zv[it] = z_row<false>(proj, 0, h, it * 32 + (tid >> 4), tid & 15, S);
+        if (ot >= 0 && !grpV) zv = z_row<false>(proj, 0, h, 16 * ot + gi, tid & 15, S);
     }
-
+    };
     if (tid >= 508) L.staged[tid - 508] = 0;
     __syncthreads();
 
-    if (!ONE && wv == 0) chunk_gates();
+    if (ONE && !grpV) __builtin_amdgcn_s_setprio(1);
+    if (!ONE && wv == GATES_WV) chunk_gates();
 
     // ---- k (group M) and q (group V): conv + SiLU + L2 norm, staged as half precision
-    {
+    if (ONE && grpV) {
+        if (ot >= 0) {                                           // one row of q
+            const int tl = 16 * ot + 4 * w + g;
+            uint4 wt[4], pk;
+#pragma unroll
+            for (int e = 0; e < 4; e++) wt[e] = *reinterpret_cast<const uint4*>(&L.taps[(cc * 8 + 2 * e) * 4]);
+            const double ss = row16_sum_d(conv8_silu_packed<true>(L.tab, rwB[0], rwB[1], rwB[2], rwB[3], wt, pk));
+            uint4 p = scale8_packed(pk, rsqrt_rn((float)ss / 128.0f + qk_eps()), BF(INV_SCALE * INV_SCALE));
+            if (tl >= S) p = make_uint4(0, 0, 0, 0);
+            *reinterpret_cast<half8*>(&L.Qs[tl * QS_LD + cc * 8]) = bf8_to_half8(p);
+        }
+    } else if (ONE && w >= nt) {                                 // (no such tokens, or nobody asks: the state's products meet zeros)
+#pragma unroll
+        for (int j = 0; j < 4; j++) *reinterpret_cast<uint4*>(&L.Ks[(4 * gi + j) * QS_LD + cc * 8]) = make_uint4(0, 0, 0, 0);
+    } else {
         _Float16* dst = grpV ? L.Qs : L.Ks;
         if (!from_proj) {
 #pragma unroll
@@ -1111,9 +1176,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
 #pragma unroll
             for (int j = 0; j < 4; j++) ss[j] = conv8_silu_packed<true>(L.tab, rwA[j], rwA[j + 1], rwA[j + 2], rwA[j + 3], wt, pk[j]);
             __builtin_amdgcn_sched_barrier(0);           // (the loads below must not be moved up: there is no room for them before)
-            if (grpV) {                                  // v's rows: requested once q's are consumed (the register file holds one set)
-                conv_rows(rwB, 2);
-            }
+            if (grpV && !ONE) conv_rows(rwB, 2);         // v's rows: requested once q's are consumed (the register file holds one set)
             rsqrt_rows4(ss, qk_eps(), rr, cc);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -1126,13 +1189,15 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
         }
     }
     part_staged(L, grpV ? PA_Q : PA_K, lane);
+    if (ONE) ask_state();
 
     if (grpV) {
         // ---- v: conv + SiLU, staged
         if (!from_proj) {
 #pragma unroll
             for (int rr = 0; rr < 4; rr++) *reinterpret_cast<half8*>(&L.Vs[(rr * 16 + gi) * VS_LD + cc * 8]) = bf8_to_half8(rwB[rr]);
-        } else {
+        } else if (!ONE || w < nt) {
+            const uint4 (&rw)[7] = ONE ? rwA : rwB;
             uint4 wt[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) wt[e] = *reinterpret_cast<const uint4*>(&L.taps[(2 * DK + cc * 8 + 2 * e) * 4]);
@@ -1140,7 +1205,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
             for (int j = 0; j < 4; j++) {
                 const int tl = 4 * gi + j, t = t0 + tl;
                 uint4 p;
-                (void)conv8_silu_packed<true>(L.tab, rwB[j], rwB[j + 1], rwB[j + 2], rwB[j + 3], wt, p);
+                (void)conv8_silu_packed<true>(L.tab, rw[j], rw[j + 1], rw[j + 2], rw[j + 3], wt, p);
                 if (t >= S) p = make_uint4(0, 0, 0, 0);
                 if (write_qkv && t < S) *reinterpret_cast<uint4*>(vi + ((size_t)t * HV + h) * DK + cc * 8) = p;
                 *reinterpret_cast<half8*>(&L.Vs[tl * VS_LD + cc * 8]) = bf8_to_half8(p);
@@ -1149,45 +1214,36 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
         part_staged(L, PA_V, lane);
         await_part(L, PA_Q);
         await_part(L, PA_K);
+        if constexpr (ONE) {
+            // Am of the workgroup's row tile: wavefront w forms the block of token tile w
+            if (ot >= 0) {
+                await_part(L, PA_GATES, 1);
+                f32x4 part = {0.f, 0.f, 0.f, 0.f};
+                if (w <= ot) part = qk_block(L, w, ot, n, g);
+                const half4 ph = {(_Float16)part[0], (_Float16)part[1], (_Float16)part[2], (_Float16)part[3]};
+                *reinterpret_cast<half4*>(&L1->Am[(w >> 1) * 512 + lane * 8 + (w & 1) * 4]) = ph;
+            }
+            __syncthreads();
+            one_chunk(L, *L1, S0, zv, o, h, ot, nt, sl, wv >> 2, tid, n, g, S);
+            return;
+        }
         // Kh = K^T (rows dk of tiles 2w, 2w+1), k index permuted: group V has the time for it (group M ends last)
-        for (int mm = 0; mm < (ONE ? 0 : 2); mm++) {
+        for (int mm = 0; mm < 2; mm++) {
             const int mt = 2 * w + mm;
             for (int kb2 = 0; kb2 < 2; kb2++)
                 *reinterpret_cast<half8*>(op + OP_K + (mt * 2 + kb2) * 512 + lane * 8) = tokens_operand(L.Ks, QS_LD, kb2, 16 * mt, n, g);
         }
-        // ---- Am = lower_incl(G * Q K^T) transposed, rows c_out = 16 ct + n, k = c_in (permuted); G_ij = exp2(Lc2_i - Lc2_j)
-        const int ct = w, co = 16 * ct + n;
-        const float lco = L.Lc2[co];
+        // ---- Am = lower_incl(G * Q K^T) transposed, rows c_out = 16 ct + n, k = c_in (permuted)
+        const int ct = w;
         for (int kb2 = 0; kb2 < 2; kb2++) {
             f32x4 part[2];
 #pragma unroll
             for (int hf = 0; hf < 2; hf++) {
                 const int tj = 2 * kb2 + hf;
                 part[hf] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (tj <= ct) {
-#pragma unroll
-                    for (int kb = 0; kb < 4; kb++) {
-                        const half8 a = *reinterpret_cast<const half8*>(&L.Ks[(16 * tj + n) * QS_LD + 32 * kb + 8 * g]);
-                        const half8 b = *reinterpret_cast<const half8*>(&L.Qs[(16 * ct + n) * QS_LD + 32 * kb + 8 * g]);
-                        part[hf] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, part[hf], 0, 0, 0);
-                    }
-                    const f32x4 lcj = *reinterpret_cast<const f32x4*>(&L.Lc2[16 * tj + 4 * g]);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const float v = __builtin_amdgcn_exp2f(lco - lcj[r]) * part[hf][r];
-                        part[hf][r] = (tj < ct || 4 * g + r <= n) ? v : 0.f;
-                    }
-                }
+                if (tj <= ct) part[hf] = qk_block(L, tj, ct, n, g);
             }
-            if constexpr (ONE)
-                *reinterpret_cast<half8*>(&L1->Am[(ct * 2 + kb2) * 512 + lane * 8]) = pack_half8(part[0], part[1]);
-            else
-                __builtin_nontemporal_store(pack_half8(part[0], part[1]), reinterpret_cast<half8*>(op + OP_A + (ct * 2 + kb2) * 512 + lane * 8));
-        }
-        if constexpr (ONE) {
-            __syncthreads();
-            one_chunk(L, *L1, reinterpret_cast<bf16_t*>(L.Qs), S0, zv, o, h, wv, tid, n, g, S);
-            return;
+            __builtin_nontemporal_store(pack_half8(part[0], part[1]), reinterpret_cast<half8*>(op + OP_A + (ct * 2 + kb2) * 512 + lane * 8));
         }
         // Qh = Q (rows of tile ct), k index permuted: two 8-byte pieces of the row
         for (int kb = 0; kb < 4; kb++) {
@@ -1205,16 +1261,18 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
     // chunk rows of tile ct = w.  Both Tb operands hold Tb[16 ct + n][kperm(kb2, g, 0..7)]: as the A operand of U, and (columns
     // scaled by -gamma) as the B operand of Wn^T.
     await_part(L, PA_K);
+    if (ONE) await_part(L, PA_GATES, 1);
     __builtin_amdgcn_s_setprio(2);                       // few instructions, all of them on the critical path
     half8 tbU[2], tbW[2];
-    inverse_row(L, w, n, g, tbU, tbW);
+    if (!ONE || w < nt) inverse_row(L, w, n, g, tbU, tbW);
     const int ct = w, nkb = ct < 2 ? 1 : 2;              // Tb is lower triangular: columns past the row tile are zero
     if constexpr (ONE) {
+        if (w < nt)
 #pragma unroll
-        for (int kb2 = 0; kb2 < 2; kb2++) *reinterpret_cast<half8*>(&L1->Tb[(ct * 2 + kb2) * 512 + lane * 8]) = tbU[kb2];
+            for (int kb2 = 0; kb2 < 2; kb2++) *reinterpret_cast<half8*>(&L1->Tb[(ct * 2 + kb2) * 512 + lane * 8]) = tbU[kb2];
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
-        one_chunk(L, *L1, reinterpret_cast<bf16_t*>(L.Qs), S0, zv, o, h, wv, tid, n, g, S);
+        one_chunk(L, *L1, S0, zv, o, h, ot, nt, sl, wv >> 2, tid, n, g, S);
         return;
     }
     for (int kb = 0; kb < 4; kb++) {
@@ -1258,19 +1316,20 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
     phase_a<from_proj, false>(L, nullptr, blockIdx.x, write_qkv, proj, qi, ki, vi, cs, cw, silu_tab, conv_out, A_log, dt_bias, ops, U, gates, S,
                               OneArgs{});
 }
-// A prompt of up to 64 tokens: one workgroup per head does everything.  What bounds it is one CU per head: the vector instructions of the conv of
-// k, q and v (until 7.5 us after the first wavefront starts, time stamps) and then the string of dependent products, the norm and the
-// store (5 us).  Records through memory and two more launches cost more than the idle CUs could give: 61 tokens 19.2 us in three launches,
-// 14.9 in one (the chain's products with K and Q in the order of the state's own registers, the gates ahead of the first barrier and the norm
-// on all eight wavefronts; 16.8 without those three).  Errors against float64, one launch / three: state 2.05e-4 / 2.19e-4, outputs 1.50e-3 both.
-__global__ __launch_bounds__(512, 2) void gdn_one_chunk_kernel(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cs,
-                                                               const bf16_t* __restrict__ cw, const bf16_t* __restrict__ silu_tab,
-                                                               bf16_t* __restrict__ conv_out, const float* __restrict__ A_log,
-                                                               const float* __restrict__ dt_bias, int S, OneArgs o) {
+// A prompt of up to 64 tokens: 3 - 6 workgroups per head, which share nothing but their inputs.  What bounds it is one CU's vector instructions
+// for the conv of k, q and v and the string of dependent products behind them; records through memory and more launches cost more than the
+// idle CUs could give, a conv done several times over costs nothing there.  us in a graph at 5 / 17 / 33 / 49 / 61 tokens: three launches - / - / - / -
+// / 19.2, one workgroup per head for everything 14.2 / 14.5 / 15.2 / 15.7 / 15.4, now 8.8 / 9.2 / 10.1 / 11.2 / 11.5 (time stamps at 61: barrier 2.2 us,
+// k staged 4.2, inverse 7.3, v 6.5 - 7.5, products 9.3, norm and store 10.2).  Errors against float64, one launch / three: state 2.05e-4 / 2.19e-4,
+// outputs 1.50e-3 both.
+// first: of the workgroups, where a launch holds the outputs' or the state's alone.
+__global__ __launch_bounds__(ONE_THREADS) void gdn_one_chunk_kernel(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cs,
+                                                                    const bf16_t* __restrict__ cw, const bf16_t* __restrict__ silu_tab,
+                                                                    bf16_t* __restrict__ conv_out, const float* __restrict__ A_log,
+                                                                    const float* __restrict__ dt_bias, int S, int first, OneArgs o) {
     __shared__ PhaseALds L;
     __shared__ OneLds L1;
-    static_assert(sizeof(L.Qs) >= sizeof(bf16_t) * C * YS_LD, "the outputs take Q's memory");
-    phase_a<true, true>(L, &L1, blockIdx.x, false, proj, nullptr, nullptr, nullptr, cs, cw, silu_tab, conv_out, A_log, dt_bias, nullptr, nullptr, nullptr, S, o);
+    phase_a<true, true>(L, &L1, blockIdx.x + first, false, proj, nullptr, nullptr, nullptr, cs, cw, silu_tab, conv_out, A_log, dt_bias, nullptr, nullptr, nullptr, S, o);
 }
 
 }  // namespace
@@ -1396,9 +1455,18 @@ int qt_gdn_prefill_one(const void* proj, const void* conv_state, const void* con
     if (S < 1 || S > C || conv_out == conv_state) return QT_ERR_UNSUPPORTED;
     for (const void* p : {proj, conv_state, conv_w, silu_table, (const void*)conv_out, (const void*)snap, (const void*)state_in, (const void*)state_out, (const void*)out})
         if (reinterpret_cast<uintptr_t>(p) & 15u) return QT_ERR_ALIGN;
-    hipLaunchKernelGGL(gdn_one_chunk_kernel, dim3(HV), dim3(512), 0, stream, (const bf16_t*)proj, (const bf16_t*)conv_state, (const bf16_t*)conv_w,
-                       (const bf16_t*)silu_table, (bf16_t*)conv_out, A_log, dt_bias, S,
-                       OneArgs{state_in, state_out, (bf16_t*)out, gw, eps, reinterpret_cast<int*>(snap) + FLAG_ERR, (int*)host_words});
+    const int state_wgs = HV * ONE_STATE_WGS, out_wgs = HV * ((S + 15) / 16);
+    auto launch = [&](int first, int n) {
+        hipLaunchKernelGGL(gdn_one_chunk_kernel, dim3(n), dim3(ONE_THREADS), 0, stream, (const bf16_t*)proj, (const bf16_t*)conv_state, (const bf16_t*)conv_w,
+                           (const bf16_t*)silu_table, (bf16_t*)conv_out, A_log, dt_bias, S, first,
+                           OneArgs{state_in, state_out, (bf16_t*)out, gw, eps, reinterpret_cast<int*>(snap) + FLAG_ERR, (int*)host_words});
+    };
+    if (state_out == state_in) {                                  // every workgroup reads the old state: it is replaced when all outputs are formed
+        launch(state_wgs, out_wgs);
+        launch(0, state_wgs);
+    } else {
+        launch(0, state_wgs + out_wgs);
+    }
     QT_CHECK_LAUNCH();
     return QT_OK;
 }

@@ -291,6 +291,26 @@ def test_prompt_of_one_chunk_in_one_launch(qt, dev, T):
     check_rel("output against the two phases", to_np(out), to_np(o3), 2.0 ** -8, rel_l2)
 
 
+@pytest.mark.parametrize("T", [1, 33, 64])
+def test_one_launch_with_the_state_in_place(qt, dev, T):
+    """through the C ABI with state_out = state_in: every workgroup of a head reads the old state, which is replaced when all outputs are
+    formed; the bits of the call with a state of its own"""
+    import ctypes
+    proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(750 + T, T, state_scale=0.3)
+    want, conv, s_want = _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0)
+    t = dict(proj=to_dev(proj, dev, BF16), cs=to_dev(cs, dev, BF16), cw=to_dev(cw, dev, BF16), A=to_dev(A_log, dev), dtb=to_dev(dtb, dev), gw=to_dev(gw, dev),
+             st=to_dev(S0, dev), out=torch.empty((T, 2048), dtype=BF16, device=dev), conv=torch.empty((3, CD), dtype=BF16, device=dev))
+    lib, p = qt._lib.lib(), lambda x: ctypes.c_void_p(x.data_ptr())
+    snap, words = torch.zeros(lib.qt_gdn_chunk_snap_bytes(T), dtype=torch.uint8, device=dev), torch.zeros(2, dtype=torch.int32, pin_memory=True)
+    rc = lib.qt_gdn_prefill_one(p(t["proj"]), p(t["cs"]), p(t["cw"]), None, p(t["A"]), p(t["dtb"]), p(t["conv"]), p(snap), p(t["st"]), p(t["st"]), p(t["gw"]), 1e-6,
+                                p(t["out"]), T, p(words), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert rc == 0 and words.tolist() == [0, 0]
+    check_tensors_equal("outputs", t["out"], want)
+    check_tensors_equal("state", t["st"].reshape(s_want.shape), s_want)
+    check_tensors_equal("conv window", t["conv"].reshape(conv.shape), conv)
+
+
 @pytest.mark.parametrize("T", [7, 64])
 def test_one_launch_at_the_edge_of_the_half_precision_range_and_beyond(qt, dev, T):
     test_chunked_prefill_at_the_edge_of_the_half_precision_range(qt, dev, T)
