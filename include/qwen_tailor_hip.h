@@ -128,8 +128,8 @@ int qt_gqa_attn_layer_decode(const void* qkv, const void* q_norm, const void* k_
  * Intermediate operands are half precision (fp16: 11 significant bits, largest finite value 65504): conv outputs |v| and
  * states |S| beyond that are not representable and are not supported; values below 6e-5 lose precision gracefully.
  * Phase B: state_in / state_out [16,128,128] f32, y [S,16,128] bf16.  128 workgroups run the serial state chain over the chunks
- * and leave the per-chunk B operands in `snap`; others compute the outputs of a chunk from them: as a second launch up to 63
- * chunks (4032 tokens), from 64 chunks on in the same launch, as soon as the chain has published the chunk.  `snap`: qt_gdn_chunk_snap_bytes(S) bytes, caller-owned, 16-byte aligned; its
+ * and leave the per-chunk B operands in `snap`; others compute the outputs of a chunk from them: as a second launch up to 111
+ * chunks (7104 tokens), from 112 chunks on in the same launch, as soon as the chain has published the chunk.  `snap`: qt_gdn_chunk_snap_bytes(S) bytes, caller-owned, 16-byte aligned; its
  * first 33 KiB (qt_gdn_chunk_snap_bytes(0) bytes) are the flag area of the launch and MUST BE ZERO when a launch starts (memory that
  * was merely allocated will not do: the one-launch form reads its queue head and progress words from it).  A launch leaves
  * them zero, so the caller zeroes them once; launches that use the same `snap` must not overlap.  The one word a launch may

@@ -93,7 +93,9 @@ constexpr float HALF_END = 65520.f;              // from here on a value becomes
 constexpr int FLAG_HALVES = FLAG_WORDS * 2;
 constexpr int SPIN_LIMIT = 1 << 21;              // polls (about a second) before a consumer gives up
 constexpr int MAX_OUT_WGS = 512;                 // output workgroups of the one-launch form: two for every CU (measured: 384 +2 us, 640 +4 us at 8192 tokens)
-constexpr int FUSED_MIN_CHUNKS = 64;              // from 4096 tokens on the one-launch form wins (measured: 2048 tokens 37 / 35 us, 8192 134 / 155 us)
+// from here on (7105 tokens) the one-launch form wins: whole core, one launch / two, 4033 tokens 102 / 98 us, 6000 143 / 138, 7000 163.5 / 160, 7500 174 / 173, 8000
+// 181 / 183, 8192 185 / 188
+constexpr int FUSED_MIN_CHUNKS = 112;
 typedef unsigned long long u64;
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));

@@ -644,7 +644,7 @@ struct Snap {
     Tensor buf, words;
     std::mutex* busy;                                            // see Scratch
 };
-constexpr int64_t ONE_LAUNCH_TOKENS = 64 * 64 - 63;              // (FUSED_MIN_CHUNKS of gdn_chunked.hip) from here on the flag area is read
+constexpr int64_t ONE_LAUNCH_TOKENS = 64 * 112 - 63;             // (FUSED_MIN_CHUNKS of gdn_chunked.hip) from here on the flag area is read
 Snap snap_buffer(const Tensor& like, int64_t S) {
     const long bytes = qt_gdn_chunk_snap_bytes(dim32(S));
     const int device = like.device().index();

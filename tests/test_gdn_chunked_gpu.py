@@ -407,6 +407,15 @@ def test_give_up_path_ends_the_launch_and_leaves_the_flags_clean(qt, dev):
     check_tensors_equal("state of the launch after a give-up", s_got, s_want)
 
 
+# the two lengths either side of the switch from two launches to one (112 chunks), and one with several chunks more
+@pytest.mark.parametrize("T", [7104, 7105, 7350])
+def test_either_side_of_the_one_launch_form(qt, dev, T):
+    """against the sequential oracle, the report of operands beyond half precision, and two launches in a row through the C ABI"""
+    test_config2_long_prefill(qt, dev, T)
+    test_status_word_reports_operands_beyond_half_precision(qt, dev, T)
+    test_phase_b_through_the_c_abi_with_a_caller_owned_snap(qt, dev, T)
+
+
 def test_report_words_outlive_an_outgrown_buffer(qt, dev):
     """launches (those of a captured HIP graph among them) keep the address of their stream's report words: a longer prompt that
     outgrows the snapshot buffer must not replace the words"""

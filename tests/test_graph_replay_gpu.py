@@ -216,3 +216,10 @@ def test_graphs_captured_on_one_stream_may_overlap(qt, dev):
         for i, (x, y) in enumerate(zip(got, w)):
             check_tensors_equal(f"program {k}, result {i}", x, y)
     qt.gdn_nax.check_status(dev, sync=True)
+
+
+@pytest.mark.parametrize("T", [7105, 7200])
+def test_the_one_launch_prefill_under_graph(qt, dev, T):
+    """from 112 chunks on phase B is one launch with a flag area, which its replays have to find and leave at zero"""
+    test_chunked_prefill_under_graph(qt, dev, T)
+    test_a_replayed_prefill_reports_to_the_stream_it_is_replayed_on(qt, dev, T)
