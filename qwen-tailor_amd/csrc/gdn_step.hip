@@ -246,6 +246,168 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
     }
 }
 
+// The same for a verify step whose workgroups have half a head or less: TOKENS tokens share one prologue.  Token by token, the inputs of each
+// token but the first were asked for behind the stores of the one before (a wavefront's loads and stores share a counter, so such a load is
+// waited for together with microseconds of stores), and two barriers and the string conv - sum - root stood in every token.  Here the
+// inputs of a group come ahead of the state, convs, norms and gates of all its tokens are formed at once, the next group's inputs are asked for
+// ahead of this group's stores, and the windows are stored behind the state.  The same bits.
+// us in a HIP graph, token by token / here: 1 x 4 7.7 / 6.1, 5 x 3 8.2 / 7.0, 5 x 5 11.6 / 9.9, 8 x 4 10.4 / 9.9, 12 x 4 13.9 / 13.2, 16 x 4 16.5 / 16.1, 16 x 5 19.4 / 19.5,
+// 20 x 4 21.7 / 20.9, 3 x 8 16.1 / 12.8, 2 x 16 24.8 / 19.0; groups of two 6.5 / 7.6 / 10.1 / 9.6 / 13.6 / 17.3 at 1 x 4 .. 16 x 4.  With whole heads (from 32
+// sequences on) the registers cost more than that gives (32 x 2 18.9 / 19.5).
+constexpr int TOKENS = 4;
+struct GroupIn {                        // one channel's raw input rows t0 - 3 .. t0 + TOKENS - 1, and its taps
+    unsigned in[TOKENS + 3];
+    uint2 c;
+};
+__device__ __forceinline__ float conv_raw(const GroupIn& r, int t) {
+    return conv_silu(bf2f((bf16_t)r.in[t]), bf2f((bf16_t)r.in[t + 1]), bf2f((bf16_t)r.in[t + 2]), bf2f((bf16_t)r.in[t + 3]), r.c);
+}
+__device__ __forceinline__ void store_window(bf16_t* __restrict__ cs_out, const GroupIn& r, int t, int ch) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) cs_out[i * CD + ch] = (bf16_t)r.in[t + 1 + i];     // kernels.py:531
+}
+template <int RS, bool TAPS_LATE, class PlaceFn>
+__device__ __forceinline__ void gdn_token_groups(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
+                                                 const float* __restrict__ dt_bias, bf16_t* __restrict__ y, int M, int h, int split, PlaceFn place) {
+    constexpr int GRPS = 16, ROWS = RS * GRPS;
+    __shared__ double red[TOKENS][4];
+    __shared__ __align__(16) float qk_s[TOKENS][2][DK];
+    __shared__ float v_s[TOKENS][ROWS];
+    __shared__ float gb_s[TOKENS][2];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, c = lane & 15;
+    const int row0 = split * ROWS;
+    // wavefronts 0, 1: q channels, 2, 3: k channels; v channels: the first ROWS threads (every load is unconditional); gates: wavefront 3
+    const bool has_v = tid < ROWS, is_g = w == 3;
+    const int which = w >> 1;                                    // 0: a q channel, 1: a k channel
+    const int ch_qk = which * KD + h * DK + (tid & 127), ch_v = has_v ? 2 * KD + h * DV + row0 + tid : ch_qk;
+    // gates: lane 2 t the decay gate of token t (reads a), lane 2 t + 1 its beta (reads b)
+    const int g_at = CD + KD + HV * ((lane & 1) ^ 1) + h, g_tok = min(lane >> 1, TOKENS - 1);
+    GroupIn rq, rv;
+    unsigned gx;
+    auto ask = [&](int t0) {                                     // a group's own rows (past the last token: the last one)
+#pragma unroll
+        for (int t = 0; t < TOKENS; t++) {
+            const size_t at = (size_t)min(t0 + t, M - 1) * PW;
+            rq.in[3 + t] = proj[at + ch_qk];
+            rv.in[3 + t] = proj[at + ch_v];
+        }
+        gx = proj[(size_t)min(t0 + g_tok, M - 1) * PW + g_at];
+    };
+    auto ask_taps = [&] {
+        rq.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch_qk * 4);
+        rv.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch_v * 4);
+    };
+    ask(0);
+    if (!TAPS_LATE) ask_taps();
+    const float gA = A_log[h], gdt = dt_bias[h];
+    __builtin_amdgcn_sched_barrier(0);
+    const Place at = place();
+    if (__builtin_expect(!at.ok, 0)) {                           // (a skipped row, see above)
+#pragma unroll
+        for (int t = 0; t < TOKENS; t++) asm volatile("" ::"v"(rq.in[3 + t]), "v"(rv.in[3 + t]));
+        if (!TAPS_LATE) asm volatile("" ::"v"(rq.c.x), "v"(rq.c.y), "v"(rv.c.x), "v"(rv.c.y));
+        asm volatile("" ::"v"(gx), "s"(gA), "s"(gdt), "s"(at.par));
+        __builtin_amdgcn_endpgm();
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        rq.in[i] = at.cs_in[i * CD + ch_qk];
+        rv.in[i] = at.cs_in[i * CD + ch_v];
+    }
+    __builtin_amdgcn_sched_barrier(0);           // keep the small loads ahead of the state loads in issue order
+    f4 s[RS][2];
+    {
+        const f4* sin4 = reinterpret_cast<const f4*>(at.st_in + ((size_t)h * DV + row0) * DK);
+#pragma unroll
+        for (int i = 0; i < RS; i++) {
+            const int row = i * GRPS + w * 4 + grp;
+            s[i][0] = __builtin_nontemporal_load(sin4 + row * (DK / 4) + c);
+            s[i][1] = __builtin_nontemporal_load(sin4 + row * (DK / 4) + 16 + c);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (TAPS_LATE) ask_taps();
+    // (nothing is converted, and so waited for, before the state has been requested)
+#pragma unroll
+    for (int i = 0; i < TOKENS + 3; i++) asm volatile("" : "+v"(rq.in[i]), "+v"(rv.in[i]));
+    asm volatile("" : "+v"(gx));
+
+    const float sc = which == 0 ? BF(INV_SCALE * INV_SCALE) : BF(INV_SCALE);       // kernels.py:492
+    // groups of one length: five tokens are three and two (16 x 5 19.4 us; 20.0 as four and one, whose last token waits for four tokens' stores)
+    const int groups = (M + TOKENS - 1) / TOKENS, step = (M + groups - 1) / groups;         // (3 or 4 where there are several)
+    for (int t0 = 0; t0 < M; t0 += step) {
+        const int n = min(step, M - t0);                                         // (the same for the whole workgroup)
+        // conv + silu, exact sums of squares over the head's 128 q (waves 0, 1) / k (waves 2, 3) channels
+        float u[TOKENS], vv[TOKENS], gate = 0.f;
+#pragma unroll
+        for (int t = 0; t < TOKENS; t++) {
+            u[t] = vv[t] = 0.f;
+            if (t >= n) continue;
+            u[t] = conv_raw(rq, t);
+            const double tot = wave_sum_d((double)u[t] * (double)u[t]);
+            if (lane == 0) red[t][w] = tot;
+            if (has_v) vv[t] = conv_raw(rv, t);
+        }
+        if (is_g) {                                                              // kernels.py:511-515
+            const float gv = bf2f((bf16_t)gx);
+            const float g = decay_gate(gA, BF(gv + gdt)), beta = sigmoid_bf16(gv);
+            gate = (lane & 1) ? beta : g;
+        }
+        __syncthreads();
+        if (is_g && lane < 2 * TOKENS) gb_s[g_tok][lane & 1] = gate;
+#pragma unroll
+        for (int t = 0; t < TOKENS; t++) {
+            if (t >= n) continue;
+            const float ss = (float)(red[t][which * 2] + red[t][which * 2 + 1]);
+            const float r = rsqrt_rn(ss / (float)DK + qk_eps());
+            qk_s[t][which][tid & 127] = BF(BF(u[t] * r) * sc);                   // kernels.py:507-510
+            if (has_v) v_s[t][tid] = vv[t];
+        }
+        __syncthreads();
+        const GroupIn oq = rq, ov = rv;
+        if (t0 + step < M) {                                                     // the next group's inputs, ahead of this one's stores
+            const bool full = step == TOKENS;
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                rq.in[i] = full ? rq.in[TOKENS + i] : rq.in[TOKENS - 1 + i];
+                rv.in[i] = full ? rv.in[TOKENS + i] : rv.in[TOKENS - 1 + i];
+            }
+            ask(t0 + step);
+        }
+#pragma unroll
+        for (int t = 0; t < TOKENS; t++) {
+            if (t >= n) break;
+            const int j = t0 + t;
+            // ---- the recurrence over this thread's 8 columns of RS rows
+            float q8[8], k8[8];
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const f4 a = reinterpret_cast<const f4*>(qk_s[t][0])[4 * e + c], b = reinterpret_cast<const f4*>(qk_s[t][1])[4 * e + c];
+#pragma unroll
+                for (int i = 0; i < 4; i++) q8[e + i] = a[i], k8[e + i] = b[i];
+            }
+            const float gg = gb_s[t][0], bb = gb_s[t][1];
+            const float kq = dot8_row16(k8, q8);
+            f4* so4 = reinterpret_cast<f4*>(at.st_out + (size_t)j * at.st_stride + ((size_t)h * DV + row0) * DK);
+            bf16_t* yo = y + (size_t)j * KD + h * DV + row0;
+#pragma unroll
+            for (int i = 0; i < RS; i++) {
+                const int row = i * GRPS + w * 4 + grp;
+                float sv[8] = {s[i][0].x, s[i][0].y, s[i][0].z, s[i][0].w, s[i][1].x, s[i][1].y, s[i][1].z, s[i][1].w};
+                const float yv = gdn_row_step(sv, k8, q8, v_s[t][row], gg, bb, kq);
+                s[i][0] = f4{sv[0], sv[1], sv[2], sv[3]};
+                s[i][1] = f4{sv[4], sv[5], sv[6], sv[7]};
+                __builtin_nontemporal_store(s[i][0], so4 + row * (DK / 4) + c);
+                __builtin_nontemporal_store(s[i][1], so4 + row * (DK / 4) + 16 + c);
+                if (c == 0) yo[row] = f2bf(yv);
+            }
+            bf16_t* cso = at.cs_out + (size_t)j * at.cs_stride;
+            if (split == 0) store_window(cso, oq, t, ch_qk);
+            if (has_v) store_window(cso, ov, t, ch_v);
+        }
+    }
+}
+
 template <int RS>
 __device__ __forceinline__ void split_id(int& b, int& h, int& split) {
     constexpr int NSPLIT = 8 / RS;
@@ -293,9 +455,10 @@ __global__ __launch_bounds__(64 * WPH * HPW) void gdn_decode_wide_kernel(const b
                                          [&] { return decode_place(conv_pool, ssm_pool, slot, p, n_slots); }, gw, eps);
 }
 
-// batch_spec.deltanet_bm (qwen35/batch_spec.py:142-150): M chained tokens per sequence, snapshot pools in place
+// batch_spec.deltanet_bm (qwen35/batch_spec.py:142-150): M chained tokens per sequence, snapshot pools in place.  (Half a head: three workgroups on
+// a CU, 168 registers; at 172 and two a CU 20 x 4 took 24.3 us instead of 21.3.)
 template <int RS, bool TAPS_LATE = false>
-__global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
+__global__ __launch_bounds__(256, RS == 4 ? 3 : 1) void gdn_verify_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
                                                          const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
                                                          const float* __restrict__ dt_bias, float* ssm_pool,
                                                          const int* __restrict__ sslots, const int* __restrict__ sels,
@@ -304,14 +467,18 @@ __global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restric
     int b, h, split;
     split_id<RS>(b, h, split);
     const int ss = sslots[b], sl = sels[b], pr = pars[b];
-    gdn_tokens<RS, 1, false, 4, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, [&] {
+    auto place = [&] {
         const int par = pr & 1;
         const size_t hs = (size_t)HV * DV * DK;
         const bool ok = (unsigned)ss < (unsigned)n_entries && (unsigned)sl < (unsigned)M;
         return Place{ok, par, conv_pool + ((size_t)(ss * 2 + par) * M + sl) * 3 * CD,
                      conv_pool + (size_t)(ss * 2 + (par ^ 1)) * M * 3 * CD, (size_t)3 * CD, ssm_pool + ((size_t)ss * M + sl) * hs,
                      ssm_pool + (size_t)ss * M * hs, hs};
-    });
+    };
+    if constexpr (RS == 8)
+        gdn_tokens<RS, 1, false, 4, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
+    else
+        gdn_token_groups<RS, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
 }
 
 // kernels.deltanet (qwen35/kernels.py:555-567): one sequence, starts from snapshot sel[0], writes M fresh snapshots
@@ -325,11 +492,15 @@ __global__ __launch_bounds__(256) void gdn_solo_kernel(const bf16_t* __restrict_
     int b, h, split;
     split_id<RS>(b, h, split);
     const int sl = sel[0];
-    gdn_tokens<RS>(proj, cw, A_log, dt_bias, y, M, h, split, [&] {
+    auto place = [&] {
         const size_t hs = (size_t)HV * DV * DK;
         const bool ok = (unsigned)sl < (unsigned)n_snap;
         return Place{ok, 0, cs_snap + (size_t)sl * 3 * CD, cs_out, (size_t)3 * CD, st_snap + sl * hs, st_out, hs};
-    });
+    };
+    if constexpr (RS == 8)
+        gdn_tokens<RS>(proj, cw, A_log, dt_bias, y, M, h, split, place);
+    else
+        gdn_token_groups<RS, false>(proj, cw, A_log, dt_bias, y, M, h, split, place);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -535,3 +535,18 @@ def test_a_missing_norm_weight_is_refused(qt, dev):
         qt.gdn_nax.phase_b_norm(proj, *records, ssm[:1], None)
     with pytest.raises(TypeError, match="gw"):
         qt.prefill.gdn_core(proj, conv[:1], ssm[:1], cw, A, A, None)
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 6, 8, 9, 13, 16])
+def test_tokens_in_groups_give_the_bits_of_tokens_one_by_one(qt, dev, M):
+    """parts of a head take a group of up to four tokens through one prologue (groups of one length: five are three and two), whole heads one
+    token after the other: outputs, windows and states alike, bit for bit"""
+    gen = torch.Generator().manual_seed(900 + M)
+    cw, A_log, dtb, _ = layer_params(900 + M)
+    proj, conv = to_dev(rand_bf(gen, (M, PW), 1.0), dev, BF16), to_dev(rand_bf(gen, (3, 3, CD)), dev, BF16)
+    ssm, sel = (torch.randn((3, 16, 128, 128), generator=gen) * 0.1).to(dev), torch.tensor([1], dtype=torch.int32, device=dev)
+    args = (proj, conv, to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev), ssm, sel)
+    want = qt.kernels.deltanet(*args, rows_per_wg=128)
+    for rows in (16, 32, 64):
+        for name, got, w in zip(("y", "windows", "states"), qt.kernels.deltanet(*args, rows_per_wg=rows), want):
+            check_tensors_equal(f"{rows} rows a workgroup: {name}", got, w)
