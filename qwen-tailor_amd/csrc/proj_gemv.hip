@@ -420,7 +420,7 @@ __global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void rows_gemm_kernel(const b
 // PEEL: the first trip is taken out of the loop (by the residual's load, which only that trip makes): 0.2 - 0.6 us less, for a tenth more
 // registers, which costs where several workgroups share a CU (80 rows 7.2 / 10.8 us against 6.4 / 10.3).
 // Measured in a HIP graph with the residual epilogue, K = 2048 / 3584 (before: residual loaded behind the last barrier, no trip peeled): 1 row
-// 3.0 / 3.5 us (3.3 / 3.8), 16 rows 3.4 / 4.4 (3.7 / 4.8), 32 rows 3.8 / 5.2 (4.2 / 5.6).
+// 3.0 / 3.5 us (3.3 / 3.8), 16 rows 3.4 / 4.4 (3.7 / 4.8), 32 rows 3.8 / 5.2 (4.2 / 5.6), 64 rows - / 6.2 (5.4 / 6.9).
 template <int NWV, int KS, int FG, int MG, int EPI, bool PEEL, bool ONE>
 __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x,
                                                              const bf16_t* __restrict__ res, bf16_t* __restrict__ y, int M, int N, int K,
@@ -506,7 +506,7 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
     }
 }
 
-// Narrow outputs of 1024 < K <= 4096 whose 16 x 16 tiles leave at most one workgroup per CU and whose 8 x 16 tiles do not.  A CU takes a load of
+// Narrow outputs of 1024 < K <= 2048 whose 16 x 16 tiles leave at most one workgroup per CU and whose 8 x 16 tiles do not.  A CU takes a load of
 // 1 KiB every 16 clocks, so what counts is the bytes of its tiles: 128 KiB for one of 16 x 16 at K = 2048, 192 for two of 8 x 16.  The wavefronts
 // deal the 128-wide steps of K among themselves as quad_gemm_kernel's do; the operands go straight to LDS, into 16 KiB that belong to the
 // wavefront (no barrier, no registers: a wavefront waits for its own loads), the 16-byte chunks of a row XOR-swizzled by the row number, so
@@ -515,11 +515,8 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
 // same bits.
 // us in a graph with the residual, quad_gemm_kernel / here: N = 1024, K = 2048 at 33 / 48 / 64 rows 4.8 / 5.05 / 5.1 -> 3.8 / 4.2 / 4.25, N = 2048 at 24 / 32
 // rows 5.2 / 5.4 -> 4.2 / 4.6, N = 4096 at 16 rows 6.0 -> 5.3, N = 520 at 96 rows 4.7 -> 4.2, K = 1280 0.5 less.  A kernel that only loads these
-// bytes takes 3.6 (N = 1024, 64 rows).
-// LONG: K of up to four steps a wavefront, the third and the fourth asked for when the first and the second have been read.  N = 1024, K = 3584 at 33 /
-// 48 / 64 rows 5.85 / 6.1 / 6.05 -> 5.3 / 5.9 / 5.9, N = 2048 at 32 rows 6 % less (with one or two steps in registers and then through LDS 6.1 - 6.4 at 64
-// rows).  Not for one row group, whose W nobody else reads: it streams faster past the caches (N = 4096, K = 4096, 16 rows 8.0 us there, 8.5 here).
-template <int EPI, bool LONG>
+// bytes takes 3.6 (N = 1024, 64 rows).  Longer K (224 KiB at K = 3584) with the steps beyond 128 KiB held in registers: 6.4, 6.1 there.
+template <int EPI>
 __global__ __launch_bounds__(512) void tile_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                         bf16_t* __restrict__ y, int M, int N, int K, int groups) {
     __shared__ __align__(1024) char own_s[8 * 16384];
@@ -537,20 +534,20 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(const bf16_t* __restrict
     }
     const char* own = own_s + w * 16384;
     const unsigned own_a = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)own_s + w * 16384;
-    auto ask = [&](int c) {
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
         const int k0 = min(w + 8 * c, steps - 1) * 256;           // (a step past the end loads the last one and is not multiplied)
 #pragma unroll
-        for (int i = 0; i < 4; i++) lds_dma16_from(wsrc[i] + k0, own_a + (c & 1) * 8192 + i * 1024);
+        for (int i = 0; i < 4; i++) lds_dma16_from(wsrc[i] + k0, own_a + c * 8192 + i * 1024);
 #pragma unroll
-        for (int i = 0; i < 4; i++) lds_dma16_from(xsrc[i] + k0, own_a + (c & 1) * 8192 + 4096 + i * 1024);
-    };
-    ask(0);
-    ask(1);
+        for (int i = 0; i < 4; i++) lds_dma16_from(xsrc[i] + k0, own_a + c * 8192 + 4096 + i * 1024);
+    }
     // the thread's output in the epilogue; its residual is requested behind the operands
     const int er = threadIdx.x >> 4, ef = threadIdx.x & 15;
     const bool e_mine = er < 16 && m0 + er < M && n0 + ef < N;
     const size_t eo = (size_t)(m0 + er) * N + n0 + ef;
     unsigned res_raw = 0;
+    if (EPI == EPI_ADD && e_mine) res_raw = res[eo];
     __builtin_amdgcn_sched_barrier(0);
     f32x4 acc[4];
 #pragma unroll
@@ -567,21 +564,10 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(const bf16_t* __restrict
         for (int j = 0; j < 4; j++)
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[j]), __builtin_bit_cast(bf16x8, b[j]), acc[j], 0, 0, 0);
     };
-    constexpr int STEPS = LONG ? 4 : 2;
-    if (EPI == EPI_ADD && !LONG && e_mine) res_raw = res[eo];
-#pragma unroll
-    for (int c = 0; c < STEPS; c++) {
-        if (c < STEPS - 1)
-            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");      // (the next step's loads; the residual's may be one more)
-        else
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (w + 8 * c < steps) multiply(c & 1);
-        if (c + 2 < STEPS) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // read: the step after the next takes its place
-            ask(c + 2);
-            if (c + 3 == STEPS && EPI == EPI_ADD && e_mine) res_raw = res[eo];
-        }
-    }
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");              // (the second step's loads; the residual's may be one more)
+    multiply(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (w + 8 < steps) multiply(1);
     *reinterpret_cast<f32x4*>(&red[w][n][4 * g]) = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     lds_barrier();
     auto total = [&](int r, int f) {                              // fixed order: pairs, then pairs of pairs, ...
@@ -719,16 +705,15 @@ void launch_quad(const gemv_args& p) {
     else
         launch_quad_tile<8, 4, FG, MG, PEEL_>(p);
 }
-template <bool LONG>
 void launch_tile(const gemv_args& p) {
     const int groups = (p.M + 15) / 16, tiles = (p.N + 15) / 16;
     const dim3 grid((tiles + 7) / 8 * 8 * groups), block(512);
     if (p.epi == EPI_NONE)
-        hipLaunchKernelGGL((tile_gemm_kernel<EPI_NONE, LONG>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL(tile_gemm_kernel<EPI_NONE>, grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
     else if (p.epi == EPI_ADD)
-        hipLaunchKernelGGL((tile_gemm_kernel<EPI_ADD, LONG>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL(tile_gemm_kernel<EPI_ADD>, grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
     else
-        hipLaunchKernelGGL((tile_gemm_kernel<EPI_SWIGLU, LONG>), grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
+        hipLaunchKernelGGL(tile_gemm_kernel<EPI_SWIGLU>, grid, block, 0, p.stream, p.W, p.x, p.res, p.y, p.M, p.N, p.K, groups);
 }
 // The smallest tile that leaves at most one workgroup per CU; beyond, small tiles still win with several workgroups per CU (measured
 // against skinny_gemm_kernel over N = 264 .. 3072, K = 512 .. 4096, 16 .. 192 rows, us: three workgroups of 8 x 16 per CU N = 1024, K = 2048 / 3584 at 80
@@ -744,9 +729,7 @@ inline bool launch_quad_any(const gemv_args& p, int cus) {
     else if (wgs(8, 16) <= cus)
         launch_quad<2, 4>(p);
     else if (p.K > 1024 && p.K <= 2048 && wgs(16, 16) <= cus)
-        launch_tile<false>(p);
-    else if (p.K > 2048 && p.K <= 4096 && p.M > 16 && wgs(16, 16) <= cus)
-        launch_tile<true>(p);
+        launch_tile(p);
     else if (p.K > 2048 && wgs(16, 16) <= cus)
         launch_quad<4, 4>(p);
     else if (wgs(8, 16) <= 3 * cus)
