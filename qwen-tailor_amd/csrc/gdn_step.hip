@@ -246,14 +246,14 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
     }
 }
 
-// The same for a verify step whose workgroups have half a head or less: TOKENS tokens share one prologue.  Token by token, the inputs of each
-// token but the first were asked for behind the stores of the one before (a wavefront's loads and stores share a counter, so such a load is
+// The same for a verify step whose workgroups have a quarter of a head or less: TOKENS tokens share one prologue.  Token by token, the inputs of
+// each token but the first were asked for behind the stores of the one before (a wavefront's loads and stores share a counter, so such a load is
 // waited for together with microseconds of stores), and two barriers and the string conv - sum - root stood in every token.  Here the
 // inputs of a group come ahead of the state, convs, norms and gates of all its tokens are formed at once, the next group's inputs are asked for
 // ahead of this group's stores, and the windows are stored behind the state.  The same bits.
-// us in a HIP graph, token by token / here: 1 x 4 7.7 / 6.1, 5 x 3 8.2 / 7.0, 5 x 5 11.6 / 9.9, 8 x 4 10.4 / 9.9, 12 x 4 13.9 / 13.2, 16 x 4 16.5 / 16.1, 16 x 5 19.4 / 19.5,
-// 20 x 4 21.7 / 20.9, 3 x 8 16.1 / 12.8, 2 x 16 24.8 / 19.0; groups of two 6.5 / 7.6 / 10.1 / 9.6 / 13.6 / 17.3 at 1 x 4 .. 16 x 4.  With whole heads (from 32
-// sequences on) the registers cost more than that gives (32 x 2 18.9 / 19.5).
+// us in a HIP graph, token by token / here: 1 x 4 7.7 / 6.1, 5 x 3 8.2 / 7.0, 5 x 5 11.6 / 9.9, 3 x 8 16.1 / 12.8, 2 x 16 24.8 / 19.0; groups of two 6.5 / 7.6 /
+// 10.1 at 1 x 4 .. 5 x 5.  With half a head the launch alone gains, too (16 x 4 16.5 / 16.1), but a step of eight layers of 16 x 4 rows takes 382.2 us
+// against 378.9, and with whole heads the registers cost more than it gives (32 x 2 18.9 / 19.5): both go token by token.
 constexpr int TOKENS = 4;
 struct GroupIn {                        // one channel's raw input rows t0 - 3 .. t0 + TOKENS - 1, and its taps
     unsigned in[TOKENS + 3];
@@ -266,7 +266,7 @@ __device__ __forceinline__ void store_window(bf16_t* __restrict__ cs_out, const 
 #pragma unroll
     for (int i = 0; i < 3; i++) cs_out[i * CD + ch] = (bf16_t)r.in[t + 1 + i];     // kernels.py:531
 }
-template <int RS, bool TAPS_LATE, class PlaceFn>
+template <int RS, class PlaceFn>
 __device__ __forceinline__ void gdn_token_groups(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
                                                  const float* __restrict__ dt_bias, bf16_t* __restrict__ y, int M, int h, int split, PlaceFn place) {
     constexpr int GRPS = 16, ROWS = RS * GRPS;
@@ -293,19 +293,16 @@ __device__ __forceinline__ void gdn_token_groups(const bf16_t* __restrict__ proj
         }
         gx = proj[(size_t)min(t0 + g_tok, M - 1) * PW + g_at];
     };
-    auto ask_taps = [&] {
-        rq.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch_qk * 4);
-        rv.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch_v * 4);
-    };
     ask(0);
-    if (!TAPS_LATE) ask_taps();
+    rq.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch_qk * 4);
+    rv.c = *reinterpret_cast<const uint2*>(cw + (size_t)ch_v * 4);
     const float gA = A_log[h], gdt = dt_bias[h];
     __builtin_amdgcn_sched_barrier(0);
     const Place at = place();
     if (__builtin_expect(!at.ok, 0)) {                           // (a skipped row, see above)
 #pragma unroll
         for (int t = 0; t < TOKENS; t++) asm volatile("" ::"v"(rq.in[3 + t]), "v"(rv.in[3 + t]));
-        if (!TAPS_LATE) asm volatile("" ::"v"(rq.c.x), "v"(rq.c.y), "v"(rv.c.x), "v"(rv.c.y));
+        asm volatile("" ::"v"(rq.c.x), "v"(rq.c.y), "v"(rv.c.x), "v"(rv.c.y));
         asm volatile("" ::"v"(gx), "s"(gA), "s"(gdt), "s"(at.par));
         __builtin_amdgcn_endpgm();
     }
@@ -326,14 +323,13 @@ __device__ __forceinline__ void gdn_token_groups(const bf16_t* __restrict__ proj
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (TAPS_LATE) ask_taps();
     // (nothing is converted, and so waited for, before the state has been requested)
 #pragma unroll
     for (int i = 0; i < TOKENS + 3; i++) asm volatile("" : "+v"(rq.in[i]), "+v"(rv.in[i]));
     asm volatile("" : "+v"(gx));
 
     const float sc = which == 0 ? BF(INV_SCALE * INV_SCALE) : BF(INV_SCALE);       // kernels.py:492
-    // groups of one length: five tokens are three and two (16 x 5 19.4 us; 20.0 as four and one, whose last token waits for four tokens' stores)
+    // groups of one length: five tokens are three and two (as four and one the last token waits for four tokens' stores)
     const int groups = (M + TOKENS - 1) / TOKENS, step = (M + groups - 1) / groups;         // (3 or 4 where there are several)
     for (int t0 = 0; t0 < M; t0 += step) {
         const int n = min(step, M - t0);                                         // (the same for the whole workgroup)
@@ -455,10 +451,9 @@ __global__ __launch_bounds__(64 * WPH * HPW) void gdn_decode_wide_kernel(const b
                                          [&] { return decode_place(conv_pool, ssm_pool, slot, p, n_slots); }, gw, eps);
 }
 
-// batch_spec.deltanet_bm (qwen35/batch_spec.py:142-150): M chained tokens per sequence, snapshot pools in place.  (Half a head: three workgroups on
-// a CU, 168 registers; at 172 and two a CU 20 x 4 took 24.3 us instead of 21.3.)
+// batch_spec.deltanet_bm (qwen35/batch_spec.py:142-150): M chained tokens per sequence, snapshot pools in place
 template <int RS, bool TAPS_LATE = false>
-__global__ __launch_bounds__(256, RS == 4 ? 3 : 1) void gdn_verify_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
+__global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
                                                          const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
                                                          const float* __restrict__ dt_bias, float* ssm_pool,
                                                          const int* __restrict__ sslots, const int* __restrict__ sels,
@@ -475,10 +470,10 @@ __global__ __launch_bounds__(256, RS == 4 ? 3 : 1) void gdn_verify_kernel(const 
                      conv_pool + (size_t)(ss * 2 + (par ^ 1)) * M * 3 * CD, (size_t)3 * CD, ssm_pool + ((size_t)ss * M + sl) * hs,
                      ssm_pool + (size_t)ss * M * hs, hs};
     };
-    if constexpr (RS == 8)
+    if constexpr (RS >= 4)
         gdn_tokens<RS, 1, false, 4, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
     else
-        gdn_token_groups<RS, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
+        gdn_token_groups<RS>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
 }
 
 // kernels.deltanet (qwen35/kernels.py:555-567): one sequence, starts from snapshot sel[0], writes M fresh snapshots
@@ -497,10 +492,10 @@ __global__ __launch_bounds__(256) void gdn_solo_kernel(const bf16_t* __restrict_
         const bool ok = (unsigned)sl < (unsigned)n_snap;
         return Place{ok, 0, cs_snap + (size_t)sl * 3 * CD, cs_out, (size_t)3 * CD, st_snap + sl * hs, st_out, hs};
     };
-    if constexpr (RS == 8)
+    if constexpr (RS >= 4)
         gdn_tokens<RS>(proj, cw, A_log, dt_bias, y, M, h, split, place);
     else
-        gdn_token_groups<RS, false>(proj, cw, A_log, dt_bias, y, M, h, split, place);
+        gdn_token_groups<RS>(proj, cw, A_log, dt_bias, y, M, h, split, place);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -539,8 +539,8 @@ def test_a_missing_norm_weight_is_refused(qt, dev):
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 6, 8, 9, 13, 16])
 def test_tokens_in_groups_give_the_bits_of_tokens_one_by_one(qt, dev, M):
-    """parts of a head take a group of up to four tokens through one prologue (groups of one length: five are three and two), whole heads one
-    token after the other: outputs, windows and states alike, bit for bit"""
+    """quarters of a head and less take a group of up to four tokens through one prologue (groups of one length: five are three and two), halves
+    and whole heads one token after the other: outputs, windows and states alike, bit for bit"""
     gen = torch.Generator().manual_seed(900 + M)
     cw, A_log, dtb, _ = layer_params(900 + M)
     proj, conv = to_dev(rand_bf(gen, (M, PW), 1.0), dev, BF16), to_dev(rand_bf(gen, (3, 3, CD)), dev, BF16)
