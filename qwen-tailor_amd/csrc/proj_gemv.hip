@@ -515,7 +515,9 @@ __global__ __launch_bounds__(64 * NWV) void quad_gemm_kernel(const bf16_t* __res
 // same bits.
 // us in a graph with the residual, quad_gemm_kernel / here: N = 1024, K = 2048 at 33 / 48 / 64 rows 4.8 / 5.05 / 5.1 -> 3.8 / 4.2 / 4.25, N = 2048 at 24 / 32
 // rows 5.2 / 5.4 -> 4.2 / 4.6, N = 4096 at 16 rows 6.0 -> 5.3, N = 520 at 96 rows 4.7 -> 4.2, K = 1280 0.5 less.  A kernel that only loads these
-// bytes takes 3.6 (N = 1024, 64 rows).  Longer K (224 KiB at K = 3584) with the steps beyond 128 KiB held in registers: 6.4, 6.1 there.
+// bytes takes 3.6 (N = 1024, 64 rows).  Longer K (224 KiB at K = 3584) with the steps beyond 128 KiB held in registers: 6.4, 6.1 there.  Through a ring in LDS it is
+// 5.9 alone, but slower inside a step of eight layers (64 x 1 rows 415.3 us against 408.3), or no faster with nontemporal W (407.3 against 407.5).
+// W is loaded plainly here: nontemporal, that step takes 415 us against 410.8.
 template <int EPI>
 __global__ __launch_bounds__(512) void tile_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                         bf16_t* __restrict__ y, int M, int N, int K, int groups) {
