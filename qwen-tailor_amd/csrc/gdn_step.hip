@@ -251,8 +251,9 @@ __device__ __forceinline__ void gdn_tokens(const bf16_t* __restrict__ proj, cons
 // waited for together with microseconds of stores), and two barriers and the string conv - sum - root stood in every token.  Here the
 // inputs of a group come ahead of the state, convs, norms and gates of all its tokens are formed at once, the next group's inputs are asked for
 // ahead of this group's stores, and the windows are stored behind the state.  The same bits.
-// us in a HIP graph, token by token / here: 1 x 4 7.7 / 6.1, 5 x 3 8.2 / 7.0, 5 x 5 11.6 / 9.9, 3 x 8 16.1 / 12.8, 2 x 16 24.8 / 19.0; groups of two 6.5 / 7.6 /
-// 10.1 at 1 x 4 .. 5 x 5.  With half a head the launch alone gains, too (16 x 4 16.5 / 16.1), but a step of eight layers of 16 x 4 rows takes 382.2 us
+// us in a HIP graph, token by token / here: 1 x 2 4.6 / 4.45, 7 x 2 6.75 / 6.55, 1 x 4 7.7 / 6.1, 5 x 3 8.2 / 7.0, 5 x 5 11.6 / 9.9, 3 x 8 16.1 / 12.8, 2 x 16 24.8 / 19.0;
+// groups of two 6.5 / 7.6 / 10.1 at 1 x 4 .. 5 x 5.  A single token has no other to share with and would only load and keep the rows of three more: 1 x 1
+// 3.3 / 3.8, 4 x 1 4.0 / 4.5, 7 x 1 4.65 / 5.4: gdn_tokens takes it.  With half a head the launch alone gains, too (16 x 4 16.5 / 16.1), but a step of eight layers of 16 x 4 rows takes 382.2 us
 // against 378.9, and with whole heads the registers cost more than it gives (32 x 2 18.9 / 19.5): both go token by token.
 constexpr int TOKENS = 4;
 struct GroupIn {                        // one channel's raw input rows t0 - 3 .. t0 + TOKENS - 1, and its taps
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(64 * WPH * HPW) void gdn_decode_wide_kernel(const b
 }
 
 // batch_spec.deltanet_bm (qwen35/batch_spec.py:142-150): M chained tokens per sequence, snapshot pools in place
-template <int RS, bool TAPS_LATE = false>
+template <int RS, bool TAPS_LATE = false, bool GROUPS = (RS < 4)>
 __global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restrict__ proj, bf16_t* conv_pool,
                                                          const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
                                                          const float* __restrict__ dt_bias, float* ssm_pool,
@@ -470,14 +471,16 @@ __global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restric
                      conv_pool + (size_t)(ss * 2 + (par ^ 1)) * M * 3 * CD, (size_t)3 * CD, ssm_pool + ((size_t)ss * M + sl) * hs,
                      ssm_pool + (size_t)ss * M * hs, hs};
     };
-    if constexpr (RS >= 4)
-        gdn_tokens<RS, 1, false, 4, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
-    else
+    if constexpr (GROUPS)
         gdn_token_groups<RS>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
+    else
+        gdn_tokens<RS, 1, false, 4, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
 }
+template <int RS>
+constexpr auto gdn_verify_one_kernel = gdn_verify_kernel<RS, false, false>;      // a single token (see gdn_token_groups)
 
 // kernels.deltanet (qwen35/kernels.py:555-567): one sequence, starts from snapshot sel[0], writes M fresh snapshots
-template <int RS>
+template <int RS, bool GROUPS = (RS < 4)>
 __global__ __launch_bounds__(256) void gdn_solo_kernel(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cs_snap,
                                                        const bf16_t* __restrict__ cw, const float* __restrict__ A_log,
                                                        const float* __restrict__ dt_bias, const float* __restrict__ st_snap,
@@ -492,11 +495,13 @@ __global__ __launch_bounds__(256) void gdn_solo_kernel(const bf16_t* __restrict_
         const bool ok = (unsigned)sl < (unsigned)n_snap;
         return Place{ok, 0, cs_snap + (size_t)sl * 3 * CD, cs_out, (size_t)3 * CD, st_snap + sl * hs, st_out, hs};
     };
-    if constexpr (RS >= 4)
-        gdn_tokens<RS>(proj, cw, A_log, dt_bias, y, M, h, split, place);
-    else
+    if constexpr (GROUPS)
         gdn_token_groups<RS>(proj, cw, A_log, dt_bias, y, M, h, split, place);
+    else
+        gdn_tokens<RS>(proj, cw, A_log, dt_bias, y, M, h, split, place);
 }
+template <int RS>
+constexpr auto gdn_solo_one_kernel = gdn_solo_kernel<RS, false>;
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -605,6 +610,9 @@ int qt_gdn_verify_step(const void* proj, void* conv_pool, const void* conv_w, co
         else
             hipLaunchKernelGGL((gdn_verify_kernel<4, true>), grid, dim3(256), 0, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w,
                                A_log, dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
+    } else if (M == 1) {
+        QT_DISPATCH_RS(rs, gdn_verify_one_kernel, B, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log,
+                       dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
     } else {
         QT_DISPATCH_RS(rs, gdn_verify_kernel, B, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log,
                        dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
@@ -621,8 +629,13 @@ int qt_gdn_deltanet(const void* proj, const void* conv_snap, const void* conv_w,
     if (M < 1 || M > 16) return QT_ERR_UNSUPPORTED;
     if (!aligned16(ssm_snap) || !aligned16(st_out) || (reinterpret_cast<uintptr_t>(conv_w) & 7u)) return QT_ERR_ALIGN;
     const int rs = pick_rs(1, rows_per_wg);
-    QT_DISPATCH_RS(rs, gdn_solo_kernel, 1, stream, (const bf16_t*)proj, (const bf16_t*)conv_snap, (const bf16_t*)conv_w, A_log,
-                   dt_bias, ssm_snap, sel, (bf16_t*)y, (bf16_t*)cs_out, st_out, M, n_snap);
+    if (M == 1) {
+        QT_DISPATCH_RS(rs, gdn_solo_one_kernel, 1, stream, (const bf16_t*)proj, (const bf16_t*)conv_snap, (const bf16_t*)conv_w, A_log,
+                       dt_bias, ssm_snap, sel, (bf16_t*)y, (bf16_t*)cs_out, st_out, M, n_snap);
+    } else {
+        QT_DISPATCH_RS(rs, gdn_solo_kernel, 1, stream, (const bf16_t*)proj, (const bf16_t*)conv_snap, (const bf16_t*)conv_w, A_log,
+                       dt_bias, ssm_snap, sel, (bf16_t*)y, (bf16_t*)cs_out, st_out, M, n_snap);
+    }
     QT_CHECK_LAUNCH();
     return QT_OK;
 }

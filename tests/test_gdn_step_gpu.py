@@ -550,3 +550,18 @@ def test_tokens_in_groups_give_the_bits_of_tokens_one_by_one(qt, dev, M):
     for rows in (16, 32, 64):
         for name, got, w in zip(("y", "windows", "states"), qt.kernels.deltanet(*args, rows_per_wg=rows), want):
             check_tensors_equal(f"{rows} rows a workgroup: {name}", got, w)
+
+
+@pytest.mark.parametrize("B", [1, 4, 7])
+def test_a_verify_step_of_one_token_takes_what_a_decode_step_takes(qt, dev, B):
+    """by the same workgroups (a quarter of a head or less each): the prologue that a verify step's tokens share loads the rows of four, 14 - 16 %
+    more here.  The two are the same work but for a lookup of snapshots (1 - 2 %); the bound lies between"""
+    gen = torch.Generator().manual_seed(70 + B)
+    cw, A_log, dtb, _ = layer_params(70)
+    args = [to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev)]
+    proj, rows = to_dev(rand_bf(gen, (B, PW), 1.0), dev, BF16), 16 if B == 1 else 32
+    ssm, conv = torch.zeros((B + 1, 16, 128, 128), device=dev), torch.zeros(((B + 1) * 2, 3, CD), dtype=BF16, device=dev)
+    slots, zeros = torch.arange(B, dtype=torch.int32, device=dev), torch.zeros(B, dtype=torch.int32, device=dev)
+    decode = graph_us(lambda: qt.batch.deltanet_b(proj, conv, *args, ssm, slots, zeros, rows))
+    verify = graph_us(lambda: qt.batch_spec.deltanet_bm(proj, conv.view((B + 1) * 2, 1, 3, CD), *args, ssm.view(B + 1, 1, 16, 128, 128), slots, zeros, zeros, 1, rows))
+    assert verify < 1.07 * decode, (verify, decode)
