@@ -477,7 +477,7 @@ __global__ __launch_bounds__(256) void gdn_verify_kernel(const bf16_t* __restric
         gdn_tokens<RS, 1, false, 4, TAPS_LATE>(proj + (size_t)b * M * PW, cw, A_log, dt_bias, y + (size_t)b * M * KD, M, h, split, place);
 }
 template <int RS>
-constexpr auto gdn_verify_one_kernel = gdn_verify_kernel<RS, false, false>;      // a single token (see gdn_token_groups)
+constexpr auto gdn_verify_single_kernel = gdn_verify_kernel<RS, false, false>;   // token by token
 
 // kernels.deltanet (qwen35/kernels.py:555-567): one sequence, starts from snapshot sel[0], writes M fresh snapshots
 template <int RS, bool GROUPS = (RS < 4)>
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(256) void gdn_solo_kernel(const bf16_t* __restrict_
         gdn_tokens<RS>(proj, cw, A_log, dt_bias, y, M, h, split, place);
 }
 template <int RS>
-constexpr auto gdn_solo_one_kernel = gdn_solo_kernel<RS, false>;
+constexpr auto gdn_solo_single_kernel = gdn_solo_kernel<RS, false>;
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -610,8 +610,15 @@ int qt_gdn_verify_step(const void* proj, void* conv_pool, const void* conv_w, co
         else
             hipLaunchKernelGGL((gdn_verify_kernel<4, true>), grid, dim3(256), 0, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w,
                                A_log, dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
-    } else if (M == 1) {
-        QT_DISPATCH_RS(rs, gdn_verify_one_kernel, B, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log,
+        QT_CHECK_LAUNCH();
+        return QT_OK;
+    }
+    // Quarters of a head in groups of tokens take 142 registers, so that three workgroups fit a CU, token by token 120 and four.  With that they go where it
+    // makes a round of workgroups less (us, groups / token by token, rows_per_wg = 32: 13 x 4 17.4 / 15.1, 16 x 2 11.4 / 10.4, 16 x 4 21.9 / 17.2, 30 x 4
+    // 35.1 / 32.8, 32 x 2 23.4 / 21.7; with as many rounds 12 x 4 12.6 / 12.8, 17 x 4 21.6 / 22.4, 24 x 4 24.6 / 26.4).
+    auto rounds = [&](long per_cu) { return ((long)B * HV * 4 + per_cu * cu_count() - 1) / (per_cu * cu_count()); };
+    if (M == 1 || (rs == 2 && rounds(3) > rounds(4))) {
+        QT_DISPATCH_RS(rs, gdn_verify_single_kernel, B, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log,
                        dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
     } else {
         QT_DISPATCH_RS(rs, gdn_verify_kernel, B, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log,
@@ -630,7 +637,7 @@ int qt_gdn_deltanet(const void* proj, const void* conv_snap, const void* conv_w,
     if (!aligned16(ssm_snap) || !aligned16(st_out) || (reinterpret_cast<uintptr_t>(conv_w) & 7u)) return QT_ERR_ALIGN;
     const int rs = pick_rs(1, rows_per_wg);
     if (M == 1) {
-        QT_DISPATCH_RS(rs, gdn_solo_one_kernel, 1, stream, (const bf16_t*)proj, (const bf16_t*)conv_snap, (const bf16_t*)conv_w, A_log,
+        QT_DISPATCH_RS(rs, gdn_solo_single_kernel, 1, stream, (const bf16_t*)proj, (const bf16_t*)conv_snap, (const bf16_t*)conv_w, A_log,
                        dt_bias, ssm_snap, sel, (bf16_t*)y, (bf16_t*)cs_out, st_out, M, n_snap);
     } else {
         QT_DISPATCH_RS(rs, gdn_solo_kernel, 1, stream, (const bf16_t*)proj, (const bf16_t*)conv_snap, (const bf16_t*)conv_w, A_log,

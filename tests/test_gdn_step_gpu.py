@@ -565,3 +565,17 @@ def test_a_verify_step_of_one_token_takes_what_a_decode_step_takes(qt, dev, B):
     decode = graph_us(lambda: qt.batch.deltanet_b(proj, conv, *args, ssm, slots, zeros, rows))
     verify = graph_us(lambda: qt.batch_spec.deltanet_bm(proj, conv.view((B + 1) * 2, 1, 3, CD), *args, ssm.view(B + 1, 1, 16, 128, 128), slots, zeros, zeros, 1, rows))
     assert verify < 1.07 * decode, (verify, decode)
+
+
+@pytest.mark.parametrize("B,M", [(16, 4), (14, 4)])
+def test_quarters_of_a_head_stay_one_round_of_workgroups(qt, dev, B, M):
+    """asked for by the caller (rows_per_wg), they took as long as halves of a head, 17 us at 16 x 4, and 22 in groups of tokens, of which one
+    workgroup less fits a CU"""
+    gen = torch.Generator().manual_seed(80 + B)
+    cw, A_log, dtb, _ = layer_params(80)
+    args = [to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev)]
+    proj = to_dev(rand_bf(gen, (B * M, PW), 1.0), dev, BF16)
+    ssm, conv = torch.zeros((B + 1, M, 16, 128, 128), device=dev), torch.zeros(((B + 1) * 2, M, 3, CD), dtype=BF16, device=dev)
+    slots, zeros = torch.arange(B, dtype=torch.int32, device=dev), torch.zeros(B, dtype=torch.int32, device=dev)
+    halves, quarters = (graph_us(lambda: qt.batch_spec.deltanet_bm(proj, conv, *args, ssm, slots, zeros, zeros, M, rows)) for rows in (64, 32))
+    assert quarters < 1.1 * halves, (quarters, halves)
