@@ -169,7 +169,7 @@ int qt_gdn_phase_b_norm(const void* ops, const void* U, const float* gC, void* s
 int qt_gdn_phase_b_report(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out,
                           const void* proj, const float* gw, float eps, void* out, int S, int32_t* host_words, qt_stream_t stream);
 
-/* The whole layer core of a prompt of 1 .. 64 tokens in one launch (two where state_out is state_in): qt_gdn_phase_a_conv and
+/* The whole layer core of a prompt of 1 .. 64 tokens in one launch: qt_gdn_phase_a_conv and
  * qt_gdn_phase_b_report with the gated norm, without records (snap is used for its status word only).  The same operator, not the same
  * bits: the state's products are taken directly instead of through half-precision operands that hold part of them.
  * QT_ERR_UNSUPPORTED, with nothing launched, for other numbers of tokens and where conv_out is conv_state (the window is still being

@@ -390,7 +390,7 @@ template <int IT, class ZFn>
 __device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int t0, int h, bf16_t* __restrict__ y, ZFn Z, const float* __restrict__ gw,
                                                 float eps, int S) {
     constexpr int RP = 16;
-    static_assert(IT == 4 || IT == 1, "four rows or one per 16-lane group");
+    static_assert(IT == 4 || IT == 2 || IT == 1, "four rows, two or one per 16-lane group");
     const int cc = tid & 15;
     float gwv[8];
 #pragma unroll
@@ -419,7 +419,8 @@ __device__ __forceinline__ void gated_norm_tile(lds_bf16_ptr ys, int tid, int t0
     if constexpr (IT == 4) {
         rsqrt_rows4(ss4, eps, inv4, cc);
     } else {
-        inv4[0] = rsqrt_rn((float)row16_sum_d(ss4[0]) / 128.0f + eps);
+#pragma unroll
+        for (int it = 0; it < IT; it++) inv4[it] = rsqrt_rn((float)row16_sum_d(ss4[it]) / 128.0f + eps);
     }
 #pragma unroll
     for (int it = 0; it < IT; it++) {
@@ -856,11 +857,13 @@ __device__ __forceinline__ void inverse_row(PhaseALds& L, const int I, int n, in
 // every floating-point step is a single instruction chosen in the source (MFMA, multiplication, fused multiply-add), so the
 // compiler has nothing to contract differently in the two instances.
 //
-// ONE: a prompt of one chunk.  The workgroups of a head go on to the outputs and the new state by themselves (one_chunk below): no records, one
+// ONE_SPLIT: a prompt of one chunk.  The workgroups of a head go on to the outputs and the new state by themselves (one_chunk below): no records, one
 // launch instead of three.  A head has a workgroup per 16 rows of outputs and two for the state (half of the columns each).  Each convolves
 // what it needs: k and v of all tokens up to its own (`nt` tiles of 16, wavefront w of either group takes tile w), q of its own rows.  A ninth
 // wavefront computes the gates.
-constexpr int ONE_STATE_WGS = 2, ONE_THREADS = 576;
+// ONE_WHOLE: the same by one workgroup per head, for a state that is updated in place: every wavefront replaces the columns that it alone has read.
+enum Form { RECORDS, ONE_SPLIT, ONE_WHOLE };
+constexpr int ONE_STATE_WGS = 2, ONE_THREADS = 576, WHOLE_THREADS = 512;
 struct OneArgs {
     const float* st_in;
     float* st_out;
@@ -869,25 +872,30 @@ struct OneArgs {
     float eps;
     int *status, *host_words;
 };
+template <bool WHOLE>
 struct OneLds {
-    __align__(16) _Float16 Tb[NCT * 2 * 512], Am[2 * 512];           // operand tiles [row tile][kb2][lane][8]
+    static constexpr int OT = WHOLE ? NCT : 1;                       // row tiles of outputs
+    __align__(16) _Float16 Tb[NCT * 2 * 512], Am[OT * 2 * 512];      // operand tiles [row tile][kb2][lane][8]
     __align__(16) float dec[C];
-    __align__(16) bf16_t ys[16 * YS_LD];                             // outputs
+    __align__(16) bf16_t ys[16 * OT * YS_LD];                        // outputs
     float gC;
 };
 // What remains of a single chunk once K, Q, V, Tb and Am are in LDS; wavefront sl owns the columns 16 sl .. + 15 of the head (dv).  The state
 // never leaves its registers, so that the products are those of the definition, with nothing folded into operands beforehand:
 //     D = Tb (V - gamma * (K S^T)),   Y = gamma * (Q S^T) + Am D,   S' = gamma_C S + K^T (dec * D)
-// ot: the row tile whose outputs this workgroup forms; negative for the state, of which the wavefront then writes half of the rows (dk).
-__device__ __forceinline__ void one_chunk(const PhaseALds& L, OneLds& L1, const f32x4 (&S0)[8], const uint4& zv, const OneArgs& o, int h, int ot,
-                                          int nt, int sl, int half, int tid, int n, int g, int S) {
+// ot: the row tile whose outputs this workgroup forms; negative for the state, of which the wavefront then writes half of the rows (dk).  WHOLE: both,
+// all tiles and all rows.
+template <bool WHOLE>
+__device__ __forceinline__ void one_chunk(const PhaseALds& L, OneLds<WHOLE>& L1, const f32x4 (&S0)[8], const uint4 (&zv)[WHOLE ? 2 : 1], const OneArgs& o,
+                                          int h, int ot, int nt, int sl, int half, int tid, int n, int g, int S) {
+    constexpr int OT = OneLds<WHOLE>::OT;
     const int lane = tid & 63;
     half8 Sb[4];
 #pragma unroll
     for (int kb = 0; kb < 4; kb++) Sb[kb] = pack_half8(S0[2 * kb], S0[2 * kb + 1]);
     // rows of K or Q with the contraction index (dk) enumerated as the state's operand
     auto rows = [&](const _Float16* base, int ct, int kb) { return *reinterpret_cast<const half8*>(base + (16 * ct + n) * QS_LD + 32 * kb + 8 * g); };
-    f32x4 R[NCT], Y = {0.f, 0.f, 0.f, 0.f};
+    f32x4 R[NCT], Y[OT];
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++) {
         R[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -899,10 +907,14 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, OneLds& L1, const 
 #pragma unroll
         for (int r = 0; r < 4; r++) R[ct][r] = __builtin_fmaf(-gm[r], ks[r], (float)L.Vs[(16 * ct + 4 * g + r) * VS_LD + 16 * sl + n]);
     }
-    if (ot >= 0) {
 #pragma unroll
-        for (int kb = 0; kb < 4; kb++) Y = __builtin_amdgcn_mfma_f32_16x16x32_f16(Sb[kb], rows(L.Qs, ot, kb), Y, 0, 0, 0);   // (transposed, as in the output kernel)
-        Y *= L.gam[16 * ot + n];
+    for (int i = 0; i < OT; i++) {
+        const int yt = WHOLE ? i : ot;
+        Y[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (yt < 0 || yt >= nt) continue;
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++) Y[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Sb[kb], rows(L.Qs, yt, kb), Y[i], 0, 0, 0);   // (transposed, as in the output kernel)
+        Y[i] *= L.gam[16 * yt + n];
     }
     // R carries no beta, unlike everything that the chain packs: it may pass the half-precision range where D does not.  A column (a lane's
     // n) is then multiplied by a power of two first, and its D divided by it.
@@ -939,7 +951,18 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, OneLds& L1, const 
     for (int ct = 0; ct < NCT; ct++)
 #pragma unroll
         for (int r = 0; r < 4; r++) bad |= fabsf(D[ct][r]) >= HALF_END;
-    if (ot < 0) {
+    if (WHOLE || ot >= 0) {
+        const half8 Dn[2] = {pack_half8(D[0], D[1]), pack_half8(D[2], D[3])};
+#pragma unroll
+        for (int i = 0; i < OT; i++) {
+            const int yt = WHOLE ? i : ot;
+#pragma unroll
+            for (int kb2 = 0; kb2 < 2; kb2++)
+                if (yt < nt && (kb2 == 0 || yt >= 2))
+                    Y[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Dn[kb2], *reinterpret_cast<const half8*>(&L1.Am[(i * 2 + kb2) * 512 + lane * 8]), Y[i], 0, 0, 0);
+        }
+    }
+    if (WHOLE || ot < 0) {
         f32x4 Dd[NCT];
 #pragma unroll
         for (int ct = 0; ct < NCT; ct++) Dd[ct] = D[ct] * *reinterpret_cast<const f32x4*>(&L1.dec[16 * ct + 4 * g]);
@@ -947,7 +970,7 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, OneLds& L1, const 
         float* so = o.st_out + ((size_t)h * DV + sl * 16 + n) * DK + 8 * g;
 #pragma unroll
         for (int i = 0; i < 8; i++) {                                // row 4 g + r of tile i is row 32 (i / 2) + 8 g + 4 (i % 2) + r of the state
-            if ((i >> 2) != half) continue;
+            if (!WHOLE && (i >> 2) != half) continue;
             f32x4 s1 = S0[i] * L1.gC;
 #pragma unroll
             for (int kb2 = 0; kb2 < 2; kb2++)
@@ -956,32 +979,33 @@ __device__ __forceinline__ void one_chunk(const PhaseALds& L, OneLds& L1, const 
 #pragma unroll
             for (int r = 0; r < 4; r++) bad |= !(fabsf(s1[r]) <= 3.0e38f);
         }
-    } else {
-        const half8 Dn[2] = {pack_half8(D[0], D[1]), pack_half8(D[2], D[3])};
-#pragma unroll
-        for (int kb2 = 0; kb2 < 2; kb2++)
-            if (kb2 == 0 || ot >= 2)
-                Y = __builtin_amdgcn_mfma_f32_16x16x32_f16(Dn[kb2], *reinterpret_cast<const half8*>(&L1.Am[kb2 * 512 + lane * 8]), Y, 0, 0, 0);
     }
     if (__any(bad) && lane == 0) {                                   // (as in the chain)
         atomicOr(o.status, ERR_NOT_FINITE);
         o.host_words[1] = 1;
     }
-    if (ot < 0) return;
-    *reinterpret_cast<uint2*>(&L1.ys[n * YS_LD + sl * 16 + 4 * g]) = make_uint2(pack2_bf(Y[0], Y[1]), pack2_bf(Y[2], Y[3]));
+    if (!WHOLE && ot < 0) return;
+#pragma unroll
+    for (int i = 0; i < OT; i++)
+        *reinterpret_cast<uint2*>(&L1.ys[(16 * i + n) * YS_LD + sl * 16 + 4 * g]) = make_uint2(pack2_bf(Y[i][0], Y[i][1]), pack2_bf(Y[i][2], Y[i][3]));
     __syncthreads();
-    if (tid < 256) gated_norm_tile<1>((lds_bf16_ptr)L1.ys, tid, 16 * ot, h, o.y, [&](int) { return zv; }, o.gw, o.eps, S);
+    auto z = [&](int it) { return zv[it]; };
+    if constexpr (WHOLE)                                             // (either half of the wavefronts takes half of the rows)
+        gated_norm_tile<2>((lds_bf16_ptr)L1.ys + (tid >> 8) * 32 * YS_LD, tid & 255, 32 * (tid >> 8), h, o.y, z, o.gw, o.eps, S);
+    else if (tid < 256)
+        gated_norm_tile<1>((lds_bf16_ptr)L1.ys, tid, 16 * ot, h, o.y, z, o.gw, o.eps, S);
 }
 
-template <bool from_proj, bool ONE>
-__device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk, const bool write_qkv, const bf16_t* __restrict__ proj, bf16_t* qi,
+template <bool from_proj, Form FORM>
+__device__ __forceinline__ void phase_a(PhaseALds& L, OneLds<FORM == ONE_WHOLE>* L1, const int blk, const bool write_qkv, const bf16_t* __restrict__ proj, bf16_t* qi,
                                         bf16_t* ki, bf16_t* vi, const bf16_t* __restrict__ cs, const bf16_t* __restrict__ cw,
                                         const bf16_t* __restrict__ silu_tab, bf16_t* __restrict__ conv_out,
                                         const float* __restrict__ A_log, const float* __restrict__ dt_bias, _Float16* __restrict__ ops,
                                         _Float16* __restrict__ U, float* __restrict__ gates, int S, const OneArgs& o) {
+    constexpr bool ONE = FORM != RECORDS, SPLIT = FORM == ONE_SPLIT, WHOLE = FORM == ONE_WHOLE;
     const int c = ONE ? 0 : blk / HV, h = blk % HV, t0 = c * C;
-    const int ot = ONE ? blk / HV - ONE_STATE_WGS : 0;  // ONE: the row tile of the outputs, or the state (-2: the lower columns, -1)
-    const int nt = ONE && ot >= 0 ? ot + 1 : (S - t0 + 15) / 16;
+    const int ot = SPLIT ? blk / HV - ONE_STATE_WGS : 0;  // SPLIT: the row tile of the outputs, or the state (-2: the lower columns, -1)
+    const int nt = WHOLE ? NCT : SPLIT && ot >= 0 ? ot + 1 : (S - t0 + 15) / 16;
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
     // (the wavefront number as a scalar: the branches on it are then real branches, which the barriers inside them need)
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -994,7 +1018,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
     const int partA = grpV ? 0 : 1;
 
     // (the wavefront of the gates asks for its inputs first: loads return in order)
-    constexpr int GATES_WV = ONE ? 8 : 0;
+    constexpr int GATES_WV = SPLIT ? 8 : 0;
     unsigned ga_raw = 0, gb_raw = 0;
     if (wv == GATES_WV) {
         const bf16_t* row = proj + (size_t)min(t0 + lane, S - 1) * PW + CD + KD + h;
@@ -1040,7 +1064,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
             if (lane >= 60) gp[G_GC + lane - 60] = lane == 60 ? expf(tot) : 0.f;
         }
     };
-    if (ONE && wv == GATES_WV) {                         // (ended, it is no party to the barriers that follow)
+    if (SPLIT && wv == GATES_WV) {                         // (ended, it is no party to the barriers that follow)
         __syncthreads();
         chunk_gates();
         part_staged(L, PA_GATES, lane);
@@ -1091,7 +1115,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
             if (t >= S) rwA[rr] = make_uint4(0, 0, 0, 0);
         }
     } else {
-        if constexpr (ONE) {                                    // k or v of the wavefront's token tile, q of one row a 16-lane group
+        if constexpr (SPLIT) {                                  // k or v of the wavefront's token tile, q of one row a 16-lane group
             if (grpV && ot >= 0)
 #pragma unroll
                 for (int d = 0; d < 4; d++) {
@@ -1102,7 +1126,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
         } else {
             conv_rows(rwA, partA);
         }
-        if (conv_out && (!ONE || ot == -1) && c == (S - 1) / C && tid >= 64 && tid < 64 + 3 * 48) {   // new conv window: input rows S-3 .. S-1 of this head's channels
+        if (conv_out && (!SPLIT || ot == -1) && c == (S - 1) / C && tid >= 64 && tid < 64 + 3 * 48) {   // new conv window: input rows S-3 .. S-1 of this head's channels
             const int i3 = tid - 64;
             const int r = i3 / 48, part = (i3 % 48) >> 4, ch0 = part * KD + h * DK + (i3 & 15) * 8, tt = S - 3 + r;
             *reinterpret_cast<uint4*>(conv_out + r * CD + ch0) =
@@ -1121,27 +1145,34 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
         if (tid >= TAP0) reinterpret_cast<uint4*>(L.taps)[tid - TAP0] = tap;
     }
 
-    // one chunk: this wavefront's columns of the state (lane (n, g): column n, rows 32 kb + 8 g .. + 7 in S0[2 kb], S0[2 kb + 1]) and its row of z.
-    // Asked for when the first part has been staged: ahead of the barrier they hold up the rows and the table (0.6 - 1 us).
-    const int sl = ONE && ot < 0 ? 4 * (ot + ONE_STATE_WGS) + w : wv;
+    // one chunk: this wavefront's columns of the state (lane (n, g): column n, rows 32 kb + 8 g .. + 7 in S0[2 kb], S0[2 kb + 1]) and its rows of z.
+    // Asked for when the first part has been staged: ahead of the barrier they hold up the rows and the table (0.6 - 1 us).  Not so where one workgroup
+    // has all three parts to convolve: ahead of it 0.3 - 0.6 us less.
+    const int sl = SPLIT && ot < 0 ? 4 * (ot + ONE_STATE_WGS) + w : wv;
     f32x4 S0[ONE ? 8 : 1];
-    uint4 zv = make_uint4(0, 0, 0, 0);
+    uint4 zv[WHOLE ? 2 : 1] = {};
     auto ask_state = [&] {
-    if constexpr (ONE) {
-        const float* sp = o.st_in + ((size_t)h * DV + sl * 16 + n) * DK + 8 * g;
+        if constexpr (ONE) {
+            const float* sp = o.st_in + ((size_t)h * DV + sl * 16 + n) * DK + 8 * g;
 #pragma unroll
-        for (int i = 0; i < 8; i++) S0[i] = *reinterpret_cast<const f32x4*>(sp + 32 * (i >> 1) + 4 * (i & 1));
-        if (ot >= 0 && !grpV) zv = z_row<false>(proj, 0, h, 16 * ot + gi, tid & 15, S);
-    }
+            for (int i = 0; i < 8; i++) S0[i] = *reinterpret_cast<const f32x4*>(sp + 32 * (i >> 1) + 4 * (i & 1));
+        }
+        if constexpr (SPLIT) {
+            if (ot >= 0 && !grpV) zv[0] = z_row<false>(proj, 0, h, 16 * ot + gi, cc, S);
+        } else if constexpr (WHOLE) {
+#pragma unroll
+            for (int it = 0; it < 2; it++) zv[it] = z_row<false>(proj, 0, h, (grpV ? 32 : 0) + 16 * it + gi, cc, S);
+        }
     };
+    if (WHOLE) ask_state();
     if (tid >= 508) L.staged[tid - 508] = 0;
     __syncthreads();
 
-    if (ONE && !grpV) __builtin_amdgcn_s_setprio(1);
-    if (!ONE && wv == GATES_WV) chunk_gates();
+    if (SPLIT && !grpV) __builtin_amdgcn_s_setprio(1);
+    if (!SPLIT && wv == GATES_WV) chunk_gates();
 
     // ---- k (group M) and q (group V): conv + SiLU + L2 norm, staged as half precision
-    if (ONE && grpV) {
+    if (SPLIT && grpV) {
         if (ot >= 0) {                                           // one row of q
             const int tl = 16 * ot + 4 * w + g;
             uint4 wt[4], pk;
@@ -1152,7 +1183,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
             if (tl >= S) p = make_uint4(0, 0, 0, 0);
             *reinterpret_cast<half8*>(&L.Qs[tl * QS_LD + cc * 8]) = bf8_to_half8(p);
         }
-    } else if (ONE && w >= nt) {                                 // (no such tokens, or nobody asks: the state's products meet zeros)
+    } else if (SPLIT && w >= nt) {                                 // (no such tokens, or nobody asks: the state's products meet zeros)
 #pragma unroll
         for (int j = 0; j < 4; j++) *reinterpret_cast<uint4*>(&L.Ks[(4 * gi + j) * QS_LD + cc * 8]) = make_uint4(0, 0, 0, 0);
     } else {
@@ -1178,7 +1209,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
 #pragma unroll
             for (int j = 0; j < 4; j++) ss[j] = conv8_silu_packed<true>(L.tab, rwA[j], rwA[j + 1], rwA[j + 2], rwA[j + 3], wt, pk[j]);
             __builtin_amdgcn_sched_barrier(0);           // (the loads below must not be moved up: there is no room for them before)
-            if (grpV && !ONE) conv_rows(rwB, 2);         // v's rows: requested once q's are consumed (the register file holds one set)
+            if (grpV && !SPLIT) conv_rows(rwB, 2);       // v's rows: requested once q's are consumed (the register file holds one set)
             rsqrt_rows4(ss, qk_eps(), rr, cc);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -1191,15 +1222,15 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
         }
     }
     part_staged(L, grpV ? PA_Q : PA_K, lane);
-    if (ONE) ask_state();
+    if (SPLIT) ask_state();
 
     if (grpV) {
         // ---- v: conv + SiLU, staged
         if (!from_proj) {
 #pragma unroll
             for (int rr = 0; rr < 4; rr++) *reinterpret_cast<half8*>(&L.Vs[(rr * 16 + gi) * VS_LD + cc * 8]) = bf8_to_half8(rwB[rr]);
-        } else if (!ONE || w < nt) {
-            const uint4 (&rw)[7] = ONE ? rwA : rwB;
+        } else if (!SPLIT || w < nt) {
+            const uint4 (&rw)[7] = SPLIT ? rwA : rwB;
             uint4 wt[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) wt[e] = *reinterpret_cast<const uint4*>(&L.taps[(2 * DK + cc * 8 + 2 * e) * 4]);
@@ -1216,7 +1247,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
         part_staged(L, PA_V, lane);
         await_part(L, PA_Q);
         await_part(L, PA_K);
-        if constexpr (ONE) {
+        if constexpr (SPLIT) {
             // Am of the workgroup's row tile: wavefront w forms the block of token tile w
             if (ot >= 0) {
                 await_part(L, PA_GATES, 1);
@@ -1226,11 +1257,11 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
                 *reinterpret_cast<half4*>(&L1->Am[(w >> 1) * 512 + lane * 8 + (w & 1) * 4]) = ph;
             }
             __syncthreads();
-            one_chunk(L, *L1, S0, zv, o, h, ot, nt, sl, wv >> 2, tid, n, g, S);
+            one_chunk<false>(L, *L1, S0, zv, o, h, ot, nt, sl, wv >> 2, tid, n, g, S);
             return;
         }
         // Kh = K^T (rows dk of tiles 2w, 2w+1), k index permuted: group V has the time for it (group M ends last)
-        for (int mm = 0; mm < 2; mm++) {
+        for (int mm = 0; mm < (WHOLE ? 0 : 2); mm++) {
             const int mt = 2 * w + mm;
             for (int kb2 = 0; kb2 < 2; kb2++)
                 *reinterpret_cast<half8*>(op + OP_K + (mt * 2 + kb2) * 512 + lane * 8) = tokens_operand(L.Ks, QS_LD, kb2, 16 * mt, n, g);
@@ -1245,7 +1276,15 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
                 part[hf] = f32x4{0.f, 0.f, 0.f, 0.f};
                 if (tj <= ct) part[hf] = qk_block(L, tj, ct, n, g);
             }
-            __builtin_nontemporal_store(pack_half8(part[0], part[1]), reinterpret_cast<half8*>(op + OP_A + (ct * 2 + kb2) * 512 + lane * 8));
+            if constexpr (WHOLE)
+                *reinterpret_cast<half8*>(&L1->Am[(ct * 2 + kb2) * 512 + lane * 8]) = pack_half8(part[0], part[1]);
+            else
+                __builtin_nontemporal_store(pack_half8(part[0], part[1]), reinterpret_cast<half8*>(op + OP_A + (ct * 2 + kb2) * 512 + lane * 8));
+        }
+        if constexpr (WHOLE) {
+            __syncthreads();
+            one_chunk<true>(L, *L1, S0, zv, o, h, ot, nt, sl, 0, tid, n, g, S);
+            return;
         }
         // Qh = Q (rows of tile ct), k index permuted: two 8-byte pieces of the row
         for (int kb = 0; kb < 4; kb++) {
@@ -1263,7 +1302,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
     // chunk rows of tile ct = w.  Both Tb operands hold Tb[16 ct + n][kperm(kb2, g, 0..7)]: as the A operand of U, and (columns
     // scaled by -gamma) as the B operand of Wn^T.
     await_part(L, PA_K);
-    if (ONE) await_part(L, PA_GATES, 1);
+    if (SPLIT) await_part(L, PA_GATES, 1);
     __builtin_amdgcn_s_setprio(2);                       // few instructions, all of them on the critical path
     half8 tbU[2], tbW[2];
     if (!ONE || w < nt) inverse_row(L, w, n, g, tbU, tbW);
@@ -1274,7 +1313,7 @@ __device__ __forceinline__ void phase_a(PhaseALds& L, OneLds* L1, const int blk,
             for (int kb2 = 0; kb2 < 2; kb2++) *reinterpret_cast<half8*>(&L1->Tb[(ct * 2 + kb2) * 512 + lane * 8]) = tbU[kb2];
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
-        one_chunk(L, *L1, S0, zv, o, h, ot, nt, sl, wv >> 2, tid, n, g, S);
+        one_chunk<WHOLE>(L, *L1, S0, zv, o, h, ot, nt, sl, wv >> 2, tid, n, g, S);
         return;
     }
     for (int kb = 0; kb < 4; kb++) {
@@ -1315,7 +1354,7 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
                                                              _Float16* __restrict__ ops, _Float16* __restrict__ U,
                                                              float* __restrict__ gates, int S) {
     __shared__ PhaseALds L;
-    phase_a<from_proj, false>(L, nullptr, blockIdx.x, write_qkv, proj, qi, ki, vi, cs, cw, silu_tab, conv_out, A_log, dt_bias, ops, U, gates, S,
+    phase_a<from_proj, RECORDS>(L, nullptr, blockIdx.x, write_qkv, proj, qi, ki, vi, cs, cw, silu_tab, conv_out, A_log, dt_bias, ops, U, gates, S,
                               OneArgs{});
 }
 // A prompt of up to 64 tokens: 3 - 6 workgroups per head, which share nothing but their inputs.  What bounds it is one CU's vector instructions
@@ -1324,14 +1363,17 @@ __global__ __launch_bounds__(512, 4) void gdn_phase_a_kernel(const bool write_qk
 // / 19.2, one workgroup per head for everything 14.2 / 14.5 / 15.2 / 15.7 / 15.4, now 8.8 / 9.2 / 10.1 / 11.2 / 11.5 (time stamps at 61: barrier 2.2 us,
 // k staged 4.2, inverse 7.3, v 6.5 - 7.5, products 9.3, norm and store 10.2).  Errors against float64, one launch / three: state 2.05e-4 / 2.19e-4,
 // outputs 1.50e-3 both.
-// first: of the workgroups, where a launch holds the outputs' or the state's alone.
-__global__ __launch_bounds__(ONE_THREADS) void gdn_one_chunk_kernel(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cs,
+// With the state in place (WHOLE), whatever reads the old state has to be done before it is replaced: one workgroup per head instead, 1 / 17 / 33 / 64
+// tokens 15.5 / 16.1 / 16.3 / 17.0 (other weights and rows each time; 10.7 / 11.2 / 12.2 / 13.5 with a state of its own).  As two launches of the above,
+// outputs and then state, it took 20.4 / 21.3 / 23.4 / 25.9.
+template <bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? WHOLE_THREADS : ONE_THREADS) void gdn_one_chunk_kernel(const bf16_t* __restrict__ proj, const bf16_t* __restrict__ cs,
                                                                     const bf16_t* __restrict__ cw, const bf16_t* __restrict__ silu_tab,
                                                                     bf16_t* __restrict__ conv_out, const float* __restrict__ A_log,
-                                                                    const float* __restrict__ dt_bias, int S, int first, OneArgs o) {
+                                                                    const float* __restrict__ dt_bias, int S, OneArgs o) {
     __shared__ PhaseALds L;
-    __shared__ OneLds L1;
-    phase_a<true, true>(L, &L1, blockIdx.x + first, false, proj, nullptr, nullptr, nullptr, cs, cw, silu_tab, conv_out, A_log, dt_bias, nullptr, nullptr, nullptr, S, o);
+    __shared__ OneLds<WHOLE> L1;
+    phase_a<true, WHOLE ? ONE_WHOLE : ONE_SPLIT>(L, &L1, blockIdx.x, false, proj, nullptr, nullptr, nullptr, cs, cw, silu_tab, conv_out, A_log, dt_bias, nullptr, nullptr, nullptr, S, o);
 }
 
 }  // namespace
@@ -1457,18 +1499,13 @@ int qt_gdn_prefill_one(const void* proj, const void* conv_state, const void* con
     if (S < 1 || S > C || conv_out == conv_state) return QT_ERR_UNSUPPORTED;
     for (const void* p : {proj, conv_state, conv_w, silu_table, (const void*)conv_out, (const void*)snap, (const void*)state_in, (const void*)state_out, (const void*)out})
         if (reinterpret_cast<uintptr_t>(p) & 15u) return QT_ERR_ALIGN;
-    const int state_wgs = HV * ONE_STATE_WGS, out_wgs = HV * ((S + 15) / 16);
-    auto launch = [&](int first, int n) {
-        hipLaunchKernelGGL(gdn_one_chunk_kernel, dim3(n), dim3(ONE_THREADS), 0, stream, (const bf16_t*)proj, (const bf16_t*)conv_state, (const bf16_t*)conv_w,
-                           (const bf16_t*)silu_table, (bf16_t*)conv_out, A_log, dt_bias, S, first,
-                           OneArgs{state_in, state_out, (bf16_t*)out, gw, eps, reinterpret_cast<int*>(snap) + FLAG_ERR, (int*)host_words});
-    };
-    if (state_out == state_in) {                                  // every workgroup reads the old state: it is replaced when all outputs are formed
-        launch(state_wgs, out_wgs);
-        launch(0, state_wgs);
-    } else {
-        launch(0, state_wgs + out_wgs);
-    }
+    const OneArgs args{state_in, state_out, (bf16_t*)out, gw, eps, reinterpret_cast<int*>(snap) + FLAG_ERR, (int*)host_words};
+    if (state_out == state_in)
+        hipLaunchKernelGGL(gdn_one_chunk_kernel<true>, dim3(HV), dim3(WHOLE_THREADS), 0, stream, (const bf16_t*)proj, (const bf16_t*)conv_state,
+                           (const bf16_t*)conv_w, (const bf16_t*)silu_table, (bf16_t*)conv_out, A_log, dt_bias, S, args);
+    else
+        hipLaunchKernelGGL(gdn_one_chunk_kernel<false>, dim3(HV * (ONE_STATE_WGS + (S + 15) / 16)), dim3(ONE_THREADS), 0, stream, (const bf16_t*)proj,
+                           (const bf16_t*)conv_state, (const bf16_t*)conv_w, (const bf16_t*)silu_table, (bf16_t*)conv_out, A_log, dt_bias, S, args);
     QT_CHECK_LAUNCH();
     return QT_OK;
 }
