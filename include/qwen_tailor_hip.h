@@ -147,6 +147,8 @@ long qt_gdn_chunk_ops_bytes(int S);
 long qt_gdn_chunk_u_bytes(int S);
 long qt_gdn_chunk_gc_bytes(int S);
 long qt_gdn_chunk_snap_bytes(int S);
+/* bytes of the flag area that a launch of S tokens reads and needs zero: qt_gdn_chunk_snap_bytes(0) in the one-launch form, 0 otherwise */
+long qt_gdn_chunk_flag_bytes(int S);
 long qt_gdn_chunk_status_offset(void);
 int qt_gdn_phase_b_poll_limit(int polls);
 int qt_gdn_phase_a(const void* proj, const void* q, const void* k, const void* v, const float* A_log, const float* dt_bias,

@@ -1388,6 +1388,9 @@ long qt_gdn_chunk_gc_bytes(int S) { return S < 0 ? -1 : (long)((S + C - 1) / C) 
 // polls before an output workgroup of the one-launch form gives up on its chunk (0 = the default, about a second)
 static std::atomic<int> poll_limit{0};
 
+// whether phase B is one launch; only then does it read the flag area
+static bool one_launch(int S) { return S > (FUSED_MIN_CHUNKS - 1) * C; }
+
 static int phase_b_launch(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out,
                           void* y, const void* proj, const float* gw, float eps, bool norm, int S, int32_t* host_words,
                           hipStream_t stream) {
@@ -1403,7 +1406,7 @@ static int phase_b_launch(const void* ops, const void* U, const float* gC, void*
             return QT_ERR_LAUNCH;
         return QT_OK;
     }
-    if (NC >= FUSED_MIN_CHUNKS) {
+    if (one_launch(S)) {
         const dim3 grid(N_CHAIN + min(MAX_OUT_WGS, NC * HV)), block(384);
         const int pl = poll_limit.load(std::memory_order_relaxed), spin = pl > 0 ? pl : SPIN_LIMIT;
         if (norm)
@@ -1435,6 +1438,8 @@ int qt_gdn_phase_b_poll_limit(int polls) {
 long qt_gdn_chunk_status_offset(void) { return (long)FLAG_ERR * 4; }
 
 long qt_gdn_chunk_snap_bytes(int S) { return S < 0 ? -1 : (long)FLAG_WORDS * 4 + (long)((S + C - 1) / C) * HV * 8 * SNAP_HALVES * 2; }
+
+long qt_gdn_chunk_flag_bytes(int S) { return S < 0 ? -1 : one_launch(S) ? (long)FLAG_WORDS * 4 : 0; }
 
 int qt_gdn_phase_b(const void* ops, const void* U, const float* gC, void* snap, const float* state_in, float* state_out, void* y,
                    int S, hipStream_t stream) {

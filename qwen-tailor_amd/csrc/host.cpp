@@ -644,7 +644,6 @@ struct Snap {
     Tensor buf, words;
     std::mutex* busy;                                            // see Scratch
 };
-constexpr int64_t ONE_LAUNCH_TOKENS = 64 * 112 - 63;             // (FUSED_MIN_CHUNKS of gdn_chunked.hip) from here on the flag area is read
 Snap snap_buffer(const Tensor& like, int64_t S) {
     const long bytes = qt_gdn_chunk_snap_bytes(dim32(S));
     const int device = like.device().index();
@@ -653,7 +652,7 @@ Snap snap_buffer(const Tensor& like, int64_t S) {
         const Ref words(PyObject_CallFunction(words_provider, "i", device));
         return {unlocked([&] {
                     Tensor buf = empty({bytes / 2}, F16, like);
-                    if (S >= ONE_LAUNCH_TOKENS) buf.narrow(0, 0, qt_gdn_chunk_snap_bytes(0) / 2).zero_();
+                    if (const long flags = qt_gdn_chunk_flag_bytes(dim32(S))) buf.narrow(0, 0, flags / 2).zero_();
                     return buf;
                 }), THPVariable_Unpack(words.o), nullptr};
     }

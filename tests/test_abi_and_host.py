@@ -121,6 +121,20 @@ def test_batched_copy_refuses_sizes_that_overflow(e, n, d0, s0, ny, ds, ss):
     assert lib.qt_blit_fill_batch(p, p, meta, 1, ctypes.c_void_p(0)) == -1
 
 
+def test_the_flag_area_of_phase_b_has_one_rule():
+    """which lengths read it is known where the launch form is chosen, and the host module, which clears it under capture, asks there: it holds no
+    number of tokens of its own"""
+    import os
+    import qwen_tailor_amd as qt
+    lib = qt._lib.lib()
+    need = [lib.qt_gdn_chunk_flag_bytes(S) for S in range(0, 20000)]
+    first = next(S for S, n in enumerate(need) if n)
+    assert need == [0] * first + [lib.qt_gdn_chunk_snap_bytes(0)] * (20000 - first) and first % 64 == 1 and lib.qt_gdn_chunk_flag_bytes(-1) == -1
+    with open(os.path.join(qt._build.CSRC, "host.cpp")) as f:
+        src = f.read()
+    assert "qt_gdn_chunk_flag_bytes(" in src and "ONE_LAUNCH_TOKENS" not in src
+
+
 def test_prefill_attention_split_plan_on_the_host():
     """The key split of the causal prefill attention is planned on the host (no GPU call computes anything here): which launches
     are split, how much workspace they use, and that the bound for a key count covers every launch below it."""

@@ -221,5 +221,7 @@ def test_graphs_captured_on_one_stream_may_overlap(qt, dev):
 @pytest.mark.parametrize("T", [7105, 7200])
 def test_the_one_launch_prefill_under_graph(qt, dev, T):
     """from 112 chunks on phase B is one launch with a flag area, which its replays have to find and leave at zero"""
+    flag_bytes = qt._lib.lib().qt_gdn_chunk_flag_bytes
+    assert flag_bytes(T) and (T > 7105 or not flag_bytes(T - 1))
     test_chunked_prefill_under_graph(qt, dev, T)
     test_a_replayed_prefill_reports_to_the_stream_it_is_replayed_on(qt, dev, T)
