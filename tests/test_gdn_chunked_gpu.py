@@ -128,10 +128,9 @@ def test_config2_chunked_prefill(qt, dev, T):
 @pytest.mark.parametrize("T", [8192, 8131, 4100, 4033, 4032])
 def test_config2_long_prefill(qt, dev, T):
     """config 2's longest sweep point (T = 8192: a chain of 128 chunks, each step rounding its operands to half precision), the
-    same with a partial last chunk, 65 chunks (the output units of the one-launch form of phase B, which these lengths
-    take, then run different numbers of rounds), and the two lengths either side of the switch between the forms (64 chunks,
-    the last one of a single token: one launch; 63 chunks: two), from a nonzero state, through the layer core (reference entry
-    qwen35/gdn_nax.py:413-426).  Run twice on the same buffers: the second launch finds the progress words the first one left.
+    same with a partial last chunk, and 63 - 65 chunks, from a nonzero state, through the layer core (reference entry
+    qwen35/gdn_nax.py:413-426).  From 112 chunks on phase B is one launch, below two (the lengths either side:
+    test_either_side_of_the_one_launch_form).  Run twice on the same buffers: the second launch finds the progress words the first one left.
     The per-head errors are checked too: a head whose state decays fast must not hide behind the slow ones."""
     proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(2002 + T, T)
     o4, conv4, s4 = qt.prefill.gdn_core(to_dev(proj, dev, BF16), to_dev(cs[None], dev, BF16), to_dev(S0[None], dev), to_dev(cw, dev, BF16),
@@ -238,7 +237,7 @@ def _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0):
 @pytest.mark.parametrize("T", [300, 4100])
 def test_chunked_prefill_at_the_edge_of_the_half_precision_range(qt, dev, T):
     """the documented operand range (|v|, |S| up to 65504): a state of N(0, 1e4) (largest element ~4.8e4) and conv outputs of a few
-    thousand keep the 2e-3 tolerance, in both launch forms of phase B, and leave the status word clear"""
+    thousand keep the 2e-3 tolerance, and leave the status word clear (two launches of phase B; one: test_either_side_of_the_one_launch_form)"""
     proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(900 + T, T, state_scale=1.0e4)
     proj[:, 4096:6144] = bf(proj[:, 4096:6144] * 2000.0)
     assert np.abs(S0).max() < 6.0e4
@@ -399,7 +398,8 @@ def test_status_word_reports_outputs_that_overflow_alone(qt, dev, T):
     """a first token that writes beta (v - k.S) beyond 65504, which its output takes as a half-precision operand, into heads that then decay so
     fast that nothing of it is left in the state: the outputs are not finite, the state is, and the launch is reported in every form"""
     proj, cs, cw, A_log, dtb, gw, _ = proj_inputs(1200 + T, T)
-    proj[:, 2 * KD:CD] = bf(proj[:, 2 * KD:CD] * 6.0e3)
+    # (the bound on v is 65504, and the largest of more draws lies further out: 6.8e4 of 7105 rows at 6e3, 5.7e4 at 5e3; the assertion below holds it)
+    proj[:, 2 * KD:CD] = bf(proj[:, 2 * KD:CD] * (6.0e3 if T <= 4100 else 5.0e3))
     proj[0, CD + KD:CD + KD + HV] = 8.0                                       # b: beta about 1
     proj[0, CD + KD + HV:], proj[1:, CD + KD + HV:] = -6.0, 20.0              # a: no decay, then exp(-20) and less a token
     q, k, v = O.conv_prep(proj, cs, cw)
@@ -433,11 +433,11 @@ def test_give_up_path_ends_the_launch_and_leaves_the_flags_clean(qt, dev):
     check_tensors_equal("the chain is not affected by output workgroups that gave up", s_gave_up, s_want)
     flag_halves = lib.qt_gdn_chunk_snap_bytes(0) // 2
     off = lib.qt_gdn_chunk_status_offset() // 4
-    for snap in qt.gdn_nax._SNAP.values():
-        words = snap[:flag_halves].view(torch.int32).clone()
-        assert int(words[off].item()) & qt.gdn_nax.GAVE_UP
-        words[off] = 0
-        assert int(words.ne(0).sum().item()) == 0, "progress words, done count or queue head left set"
+    snap = qt.gdn_nax._SNAP[qt.gdn_nax._key(torch.device("cuda", torch.cuda.current_device()))]      # (this stream's: others may have theirs)
+    words = snap[:flag_halves].view(torch.int32).clone()
+    assert int(words[off].item()) & qt.gdn_nax.GAVE_UP
+    words[off] = 0
+    assert int(words.ne(0).sum().item()) == 0, "progress words, done count or queue head left set"
     with pytest.raises(qt.gdn_nax.ChunkedPrefillError, match="gave up"):
         qt.gdn_nax.check_status(dev, sync=True)
     got, _, s_got = _core(qt, dev, proj, cs, cw, A_log, dtb, gw, S0)
@@ -449,10 +449,27 @@ def test_give_up_path_ends_the_launch_and_leaves_the_flags_clean(qt, dev):
 # the two lengths either side of the switch from two launches to one (112 chunks), and one with several chunks more
 @pytest.mark.parametrize("T", [7104, 7105, 7350])
 def test_either_side_of_the_one_launch_form(qt, dev, T):
-    """against the sequential oracle, the report of operands beyond half precision, and two launches in a row through the C ABI"""
+    """against the sequential oracle, the edge of the half-precision range, the reports of operands and of outputs beyond it, and two launches in
+    a row through the C ABI"""
+    assert (qt._lib.lib().qt_gdn_chunk_flag_bytes(T) > 0) == (T > 7104)
     test_config2_long_prefill(qt, dev, T)
+    test_chunked_prefill_at_the_edge_of_the_half_precision_range(qt, dev, T)
     test_status_word_reports_operands_beyond_half_precision(qt, dev, T)
+    test_status_word_reports_outputs_that_overflow_alone(qt, dev, T)
     test_phase_b_through_the_c_abi_with_a_caller_owned_snap(qt, dev, T)
+
+
+@pytest.mark.parametrize("T", [300, 7104, 7105, 8131])
+def test_phase_b_without_the_norm_in_either_form(qt, dev, T):
+    """its outputs through the gated norm of their own are the bits of phase B with the norm in it, and so is the state"""
+    proj, cs, cw, A_log, dtb, gw, S0 = proj_inputs(3100 + T, T)
+    dproj, dgw, dS0 = to_dev(proj, dev, BF16), to_dev(gw, dev), to_dev(S0[None], dev)
+    q, k, v, ops, U, gC = qt.gdn_nax._phase_a(dproj, to_dev(cs, dev, BF16), to_dev(cw, dev, BF16), to_dev(A_log, dev), to_dev(dtb, dev))
+    want, s_want = qt.gdn_nax.phase_b_norm(dproj, ops, U, gC, dS0, dgw)
+    y, s = qt.gdn_nax.phase_b(q, k, v, ops, U, gC, dS0)
+    check_tensors_equal("outputs", qt.prefill.gated_norm(y.reshape(T, 2048), dproj, dgw), want)
+    check_tensors_equal("state", s, s_want)
+    qt.gdn_nax.check_status(dev, sync=True)
 
 
 def test_report_words_outlive_an_outgrown_buffer(qt, dev):

@@ -78,7 +78,8 @@ def test_decode_step_and_layer_half_under_graph(qt, dev):
 
 @pytest.mark.parametrize("T", [1, 61, 300, 4100])
 def test_chunked_prefill_under_graph(qt, dev, T):
-    """both launch forms of phase B; the one-launch form's flag area must be back to zero after every replay"""
+    """a prompt of one chunk, phase B as two launches, and (test_the_one_launch_prefill_under_graph) as one, whose flag area must be back to zero after
+    every replay"""
     gen = torch.Generator().manual_seed(6 + T)
     cw, A_log, dtb, gw = layer_params(32)
     proj = to_dev(rand_bf(gen, (T, PW)), dev, BF16)
@@ -155,8 +156,8 @@ def _prefill_inputs(dev, T, seed):
 @pytest.mark.parametrize("T", [7, 64, 300, 4033, 4100])
 def test_a_replayed_prefill_reports_to_the_stream_it_is_replayed_on(qt, dev, T):
     """captured on a side stream that has seen no prefill, replayed on the current one: its failure (a state beyond the half-precision
-    range) is found by check_status there, and the next replay, with a good state, has the eager bits (4033 tokens are the first
-    that read the flag area, which the replays have to clear)"""
+    range) is found by check_status there, and the next replay, with a good state, has the eager bits (7105 tokens are the first
+    that read the flag area, which the replays have to clear: test_the_one_launch_prefill_under_graph)"""
     ins = _prefill_inputs(dev, T, 70 + T)
     good = ins[2].clone()
     want = qt.prefill.gdn_core(*ins)

@@ -177,10 +177,12 @@ def test_narrow_projection_tiles_exact_on_small_integers(qt, dev, M, N, K, epi):
 
 # 16 x 16 tiles through LDS (one per CU where 8 x 16 would take two): outputs and rows that end inside a tile, wavefronts with one and with two
 # steps of K (1280: two of ten wavefronts' steps; 1792), the fewest and the most tiles of the rule
-@pytest.mark.parametrize("M,N,K", [(33, 1024, 2048), (64, 1023, 2048), (49, 1030, 1280), (96, 520, 1792), (17, 2047, 1536), (32, 2050, 2048), (9, 4095, 1280), (16, 4096, 2048),
+@pytest.mark.parametrize("M,N,K", [(33, 1024, 2048), (64, 1023, 2048), (48, 1030, 1280), (96, 520, 1792), (17, 2047, 1536), (32, 2034, 2048), (9, 4095, 1280), (16, 4096, 2048),
                                    (130, 260, 2048), (257, 130, 1280)])
 def test_narrow_projection_one_tile_per_cu(qt, dev, M, N, K):
     """exact on small integers, and on real values the bits of the same rows in batches of up to 16 (which smaller tiles take)"""
+    cus, wgs = torch.cuda.get_device_properties(dev).multi_processor_count, lambda f: ((N + f - 1) // f) * ((M + 15) // 16)
+    assert M > 8 and 1024 < K <= 2048 and wgs(16) <= cus < wgs(8), "not a case of this kernel"
     for epi in (0, 1) + ((2,) if N % 2 == 0 else ()):
         test_narrow_projection_tiles_exact_on_small_integers(qt, dev, M, N, K, epi)
     g = torch.Generator().manual_seed(M + N + K)
