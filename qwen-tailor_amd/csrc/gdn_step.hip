@@ -602,7 +602,8 @@ int qt_gdn_verify_step(const void* proj, void* conv_pool, const void* conv_w, co
     // More than a head per CU, in workgroups of half a head or more: the taps behind the state, so that a workgroup waits for its whole state before
     // it computes and stores: fewer stores of one between the loads of another (us, taps late / ahead: 24 x 4 23.9 / 25.1, 18 x 4 19.6 / 20.8, 32 x
     // 2 17.9 / 18.7).  With less the conv beside the state's loads wins (8 x 4 11.4 / 10.4, 12 x 4 14.1 / 13.9, 16 x 8 33.0 / 31.2).
-    if (rs >= 4 && (long)B * HV > cu_count()) {
+    const long cus = cu_count();
+    if (rs >= 4 && (long)B * HV > cus) {
         const dim3 grid(B * HV * (8 / rs));
         if (rs == 8)
             hipLaunchKernelGGL((gdn_verify_kernel<8, true>), grid, dim3(256), 0, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w,
@@ -616,7 +617,7 @@ int qt_gdn_verify_step(const void* proj, void* conv_pool, const void* conv_w, co
     // Quarters of a head in groups of tokens take 142 registers, so that three workgroups fit a CU, token by token 120 and four.  With that they go where it
     // makes a round of workgroups less (us, groups / token by token, rows_per_wg = 32: 13 x 4 17.4 / 15.1, 16 x 2 11.4 / 10.4, 16 x 4 21.9 / 17.2, 30 x 4
     // 35.1 / 32.8, 32 x 2 23.4 / 21.7; with as many rounds 12 x 4 12.6 / 12.8, 17 x 4 21.6 / 22.4, 24 x 4 24.6 / 26.4).
-    auto rounds = [&](long per_cu) { return ((long)B * HV * 4 + per_cu * cu_count() - 1) / (per_cu * cu_count()); };
+    auto rounds = [&](long per_cu) { return ((long)B * HV * 4 + per_cu * cus - 1) / (per_cu * cus); };
     if (M == 1 || (rs == 2 && rounds(3) > rounds(4))) {
         QT_DISPATCH_RS(rs, gdn_verify_single_kernel, B, stream, (const bf16_t*)proj, (bf16_t*)conv_pool, (const bf16_t*)conv_w, A_log,
                        dt_bias, ssm_pool, sslots, sels, pars, (bf16_t*)y, M, n_entries);
