@@ -93,8 +93,10 @@ constexpr float HALF_END = 65520.f;              // from here on a value becomes
 constexpr int FLAG_HALVES = FLAG_WORDS * 2;
 constexpr int SPIN_LIMIT = 1 << 21;              // polls (about a second) before a consumer gives up
 constexpr int MAX_OUT_WGS = 512;                 // output workgroups of the one-launch form: two for every CU (measured: 384 +2 us, 640 +4 us at 8192 tokens)
-// from here on (7105 tokens) the one-launch form wins: whole core, one launch / two, 4033 tokens 102 / 98 us, 6000 143 / 138, 7000 163.5 / 160, 7500 174 / 173, 8000
-// 181 / 183, 8192 185 / 188
+// from here on (7105 tokens) phase B is one launch.  Where the two forms cross depends on what the caches hold: at about 6700 tokens with records and inputs
+// warm (the same call again), at about 7700 with four sets of inputs in turn in a graph; the line lies between.  Whole core, us, one launch / two, warm 6000
+// tokens 129.7 / 125.6, 6900 146.6 / 148.0, 7168 149.8 / 153.6, 8192 168.0 / 177.2, in turn 6000 139.8 / 133.4, 6900 157.7 / 152.9, 7168 161.0 / 160.5, 7800
+// 177.0 / 174.2, 8192 179.9 / 183.4
 constexpr int FUSED_MIN_CHUNKS = 112;
 typedef unsigned long long u64;
 
@@ -601,8 +603,8 @@ __global__ __launch_bounds__(384, 3) void gdn_phase_b_kernel(const _Float16* ops
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Phase A: one workgroup of 512 threads per (chunk, head), two workgroups per CU.  Bound by its vector-ALU instructions (half of the time)
-// and by the latencies at either end of a workgroup.  Whole prefill at 61 / 2048 / 8192 tokens 20.5 / 51.5 / 170.1 us with row addresses
+// Phase A: one workgroup of 512 threads per (chunk, head), two workgroups per CU.  Bound by its vector-ALU instructions (half of the time),
+// by the latencies at either end of a workgroup and, with many chunks, by its bytes (8192 tokens: 287 MB, 56 us at a copy's rate, of 67).  Whole prefill at 61 / 2048 / 8192 tokens 20.5 / 51.5 / 170.1 us with row addresses
 // chosen per row, the table behind the rows and the gates ahead of the barrier; 19.7 / 50.0 / 166.9 us now.
 //
 // A (chunk, head) costs about 10^5 vector-ALU instructions of conv + SiLU + normalisation and a chain of dependent matrix

@@ -212,8 +212,10 @@ __device__ __forceinline__ void quad_transpose(u32x4 (&v)[4], bool odd, bool hig
 // LDS in a fixed order.
 // Rows: every wavefront brings in 2 RB of them, a row per two loads of 1 KiB, asks for the W of its first block right after, and applies the
 // rms prologue (RMS) while that is on its way from HBM; the rows then go to LDS, their 16-byte chunks XOR-swizzled by the row number
-// so that the fragment reads of 16 rows fall on distinct banks.  Every workgroup normalises its rows itself: 0.1 us (16 rows)
-// to 0.7 us (32 rows x 64 features) instead of a launch of its own at 2.6 us.
+// so that the 16 rows of one k group fall on distinct banks.  (Not yet those of a whole read: 16 bytes a lane are read for lanes 0 - 3, 12 - 15 and 20 - 27
+// together, then 4 - 11, 16 - 19 and 28 - 31, which are rows of two k groups, and the XOR puts the one on the other's banks.  Such a read takes eight
+// cycles instead of four: the conflicts in half of the LDS's active cycles that the counters show here and in tile_gemm_kernel.)
+// Every workgroup normalises its rows itself: 0.1 us (16 rows) to 0.7 us (32 rows x 64 features) instead of a launch of its own at 2.6 us.
 // W: a load takes 256 contiguous bytes of four features, 64 of them in each quad of lanes (register j of lane (g, h, c): feature
 // 4 h + j, elements 32 g + 8 c ..), and quad_transpose turns four such loads into the MFMA layout: feature n in lane (n, g),
 // elements 32 g + 8 r .. in register r.  The x fragments are read from LDS in the same enumeration of k.  Which wavefront takes
@@ -638,7 +640,8 @@ inline bool rows_shape(const gemv_args& p) {
 constexpr int RMS_ROWS_MAX = 96;       // most rows with the prologue fused in: beyond, the rows are normalised too often
 // Tile by rows.  Up to 96 rows: the smallest tile that leaves at most one workgroup per CU (32 features as long as one row
 // group holds the batch, then 64; at 33 - 48 rows with the prologue 32 rows x 64 features, which normalise fewer rows each: 7.1 / 6.7 / 6.2 us against
-// 7.3 / 7.0 / 6.5 with 48 x 32, without it 6.5 against 6.0).  Where none does, W is what costs, and one row group is better than two that read it twice:
+// 7.3 / 7.0 / 6.5 with 48 x 32, without it 6.5 against 6.0; where 64 features leave no room for the extra fours, N = 8324 .. 8448, 48 x 32 takes 7.9 and
+// 8.1 with swiglu, 48 x 64 8.05 and 8.4).  Where none does, W is what costs, and one row group is better than two that read it twice:
 // 64 features x 48 or 64 rows (N = 9216 / 32768 / 151936 at 48 rows 6.6 / 15.9 / 70 us; with an earlier build 8.5 / 19.2 / 82, 11.3 / 24.4 / 102 with 32
 // features, at 64 rows 9.1 / 20.8 / 88, 11.9 / 25.7 / 108 with two groups of 32 rows); up to 32 rows 32 features again, whose two workgroups per CU overlap (N =
 // 32768 / 151936 16 / 61 us at 17 rows, 17.3 / 68 with 64).  Beyond 96 rows 64 x 64 up to 128 rows, then 32 x 32 (N = 8224 / 7168 / 5120 at
