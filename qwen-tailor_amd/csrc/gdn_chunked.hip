@@ -96,7 +96,8 @@ constexpr int MAX_OUT_WGS = 512;                 // output workgroups of the one
 // from here on (7105 tokens) phase B is one launch.  Where the two forms cross depends on what the caches hold: at about 6700 tokens with records and inputs
 // warm (the same call again), at about 7700 with four sets of inputs in turn in a graph; the line lies between.  Whole core, us, one launch / two, warm 6000
 // tokens 129.7 / 125.6, 6900 146.6 / 148.0, 7168 149.8 / 153.6, 8192 168.0 / 177.2, in turn 6000 139.8 / 133.4, 6900 157.7 / 152.9, 7168 161.0 / 160.5, 7800
-// 177.0 / 174.2, 8192 179.9 / 183.4
+// 177.0 / 174.2, 8192 179.9 / 183.4.  That is with records that phase A has just written, as every prefill has them; phase B with the norm by itself on
+// records and z that have left the caches would rather have one launch (4500 tokens 66.9 / 80.1, 6000 94.7 / 101.5), without the norm it hardly matters (74.0 / 75.3)
 constexpr int FUSED_MIN_CHUNKS = 112;
 typedef unsigned long long u64;
 
