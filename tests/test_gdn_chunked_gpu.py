@@ -341,12 +341,12 @@ def test_state_in_place_at_the_edge_of_the_half_precision_range_and_beyond(qt, d
 
 @pytest.mark.parametrize("T", [1, 64])
 def test_state_in_place_costs_no_second_launch(qt, dev, T):
-    """one workgroup per head instead of three to six takes 1.2 - 1.45 times as long as with a state of its own; outputs and state as two launches one
-    after the other took 1.8 - 1.9 times"""
+    """one workgroup per head instead of three to six takes 1.48 (one token) and 1.30 (64) times as long as with a state of its own; outputs and state as two
+    launches one after the other 1.96 and 1.87; the bound lies between"""
     launch, t, _ = _in_place(qt, dev, *proj_inputs(770 + T, T))
     other = torch.empty_like(t["st"])
     in_place, own = graph_us(launch), graph_us(lambda: launch(other))
-    assert in_place < 1.62 * own, (in_place, own)
+    assert in_place < 1.68 * own, (in_place, own)
 
 
 @pytest.mark.parametrize("T", [7, 64])
